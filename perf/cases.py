@@ -200,9 +200,10 @@ def _weight(name, shape, dtype, seed, spec):
     elif leaf == "ff_coef":
         w = torch.tensor([0.6, 0.3, 0.2, 0.0], device="cuda") + rnd(0.05)
     elif "router" in (leaf, owner):
-        w = rnd(2.0 / math.sqrt(shape[-1]))
+        # a trained router is sharp: the choice it nearly made weighs little
+        w = rnd((4.0 if uniform else 2.0) / math.sqrt(shape[-1]))
     elif owner in ("embed_tokens", "bigram"):
-        w = rnd(0.2 if uniform else 1.0 / math.sqrt(shape[1])
+        w = rnd((2.0 if spec.arch == "qwen3_moe" else 0.2) if uniform else 1.0 / math.sqrt(shape[1])
                 if spec.tie_embeddings and owner == "embed_tokens" else 1.0)
     else:
         w = rnd(1.0 / math.sqrt(shape[-1]))
@@ -608,8 +609,8 @@ def _cost(case):
 # measured: about four times the distance to `exact` over the listed and some
 # drawn cases. Routed models are further off than dense ones because a token
 # near a tie between two experts goes to the other one when its router input is
-# rounded differently; fp8 pages round keys and values to 4 bits
-_REL = {"qwen3": 0.04, "qwen3moe": 0.3, "vodinex": 0.03, "ruludra": 0.015,
+# rounded differently
+_REL = {"qwen3": 0.03, "qwen3moe": 0.03, "vodinex": 0.03, "ruludra": 0.015,
         "nosalorn": 0.03, "vanulorn": 0.015}
 
 
@@ -620,8 +621,9 @@ def tolerance(case):
         return {"rel": 1e-5, "differ": 0.002}
     if case["path"] == "embed":
         return {"rel": 0.03}
-    rel = _REL[case["model"]]
-    return {"rel": rel + 0.04 if case["kv"] == "fp8_e4m3" else rel}
+    # a token that goes to another expert moves its own row further
+    moved = case["model"] in ("qwen3moe", "nosalorn")
+    return {"rel": _REL[case["model"]], "max": 0.9 if moved else 0.5}
 
 
 # ---- the same in 64 bits -------------------------------------------------
