@@ -364,26 +364,23 @@ static void launch_decode(long blocks, int wpb, void* out, const void* q,
 extern "C" void sutro_attn_decode_mfma(void*, const void*, const void*,
                                        const void*, const int*, const int*,
                                        int, int, int, int, int, float, int,
-                                       int, hipStream_t);
+                                       int, int, float*, float*, hipStream_t);
 
 extern "C" void sutro_attn_decode(void* out, const void* q, const void* k_cache,
                                   const void* v_cache, const int* block_tables,
                                   const int* seq_lens, int bt_stride, int n_dec,
                                   int Hq, int Hk, int head_dim, int kv_fp8,
-                                  int seq_offset, float scale, hipStream_t s) {
+                                  int seq_offset, float scale, int nsplit,
+                                  float* part_o, float* part_ml,
+                                  hipStream_t s) {
   if (n_dec == 0) return;
-  // MFMA variant is the measured default at head_dim 128, bf16 AND e4m3 KV
-  // (bf16: 10654 vs 10134 tok/s at batch 1024 / ctx 128; attention slope
-  // halves at ctx 512; fp8 dequants with the native pk converts at the K/V
-  // fragment loads). head_dim 64 routes to MFMA too since the DB-bounded
-  // alpha-rescale fix (attn_decode_mfma.hip:202) — verified against the fp32
-  // reference by test_attn_head_dim_64 on hardware.
+  // the matrix-core kernel covers head sizes 64 and 128, bf16 and e4m3 pages;
   // SUTRO_DECODE_VALU=1 falls back to the VALU kernel for A/B.
   if ((head_dim == 128 || head_dim == 64) && Hq / Hk <= 8 &&
       getenv("SUTRO_DECODE_VALU") == nullptr) {
     sutro_attn_decode_mfma(out, q, k_cache, v_cache, block_tables, seq_lens,
                            bt_stride, n_dec, Hq, Hk, seq_offset, scale, kv_fp8,
-                           head_dim, s);
+                           head_dim, nsplit, part_o, part_ml, s);
     return;
   }
   const int wpb = 4;

@@ -31,7 +31,8 @@ void sutro_mean_pool_normalize(float*, const void*, const int*, int, int,
                                hipStream_t);
 void sutro_attn_decode(void*, const void*, const void*, const void*,
                        const int*, const int*, int, int, int, int, int, int,
-                       int, float, hipStream_t);
+                       int, float, int, float*, float*, hipStream_t);
+int sutro_attn_decode_splits(int, int, int);
 void sutro_attn_prefill(void*, const void*, const void*, const void*,
                         const int*, const int*, const int*, const int*,
                         const int*, int, int, int, int, int, int, float,
@@ -139,12 +140,21 @@ void paged_attention(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
     const int seq_offset = S - (int)num_decodes;
     const u_int16_t* qp = (const u_int16_t*)q.data_ptr();
     u_int16_t* op = (u_int16_t*)out.data_ptr();
+    // partial results of contexts that are cut into runs of pages
+    const int ns = sutro_attn_decode_splits((int)num_decodes, Hk, bt_stride);
+    torch::Tensor po, pml;
+    if (ns > 1) {
+      auto o = q.options().dtype(at::kFloat);
+      po = torch::empty({num_decodes * Hq * ns, D}, o);
+      pml = torch::empty({num_decodes * Hq * ns, 2}, o);
+    }
     sutro_attn_decode(op + dec_off * Hq * D, qp + dec_off * Hq * D,
                       k_cache.data_ptr(), v_cache.data_ptr(),
                       block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(),
                       bt_stride, (int)num_decodes, Hq, Hk, D,
-                      is_fp8(k_cache) ? 1 : 0, seq_offset, (float)scale,
-                      cur_stream());
+                      is_fp8(k_cache) ? 1 : 0, seq_offset, (float)scale, ns,
+                      ns > 1 ? po.data_ptr<float>() : nullptr,
+                      ns > 1 ? pml.data_ptr<float>() : nullptr, cur_stream());
   }
 }
 

@@ -1,0 +1,61 @@
+"""The paged attention kernels at the sizes where their splits change: run
+borders of the decode kernel, tile and workgroup borders of the prompt
+kernel."""
+
+import math
+
+import pytest
+import torch
+
+from sutro_amd import ops
+from sutro_amd.ops import torch_ref as R
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _paged(lens, new, Hq, Hk, D, fp8, spare=0, seed=0):
+    """Random queries and shuffled pages; block tables `spare` columns wider
+    than the longest sequence needs."""
+    g = torch.Generator().manual_seed(seed)
+    pages = [(n + 31) // 32 for n in lens]
+    perm = torch.randperm(sum(pages) + 3, generator=g).tolist()
+    bt = torch.zeros(len(lens), max(pages) + spare, dtype=torch.int32)
+    at = 0
+    for s, n in enumerate(pages):
+        bt[s, :n] = torch.tensor(perm[at:at + n])
+        at += n
+    shape = (len(perm), Hk, 32, D)
+    kc, vc = (torch.randn(shape, generator=g).bfloat16() for _ in range(2))
+    if fp8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    q = torch.randn(sum(new), Hq, D, generator=g).bfloat16()
+    ql = torch.tensor([0] + new).cumsum(0).to(torch.int32)
+    return q, kc, vc, bt, torch.tensor(lens, dtype=torch.int32), ql
+
+
+def _check(args, got):
+    q, kc, vc, bt, sl, ql = args
+    ref = R.paged_attention(q.float(), kc.float(), vc.float(), bt, sl, ql,
+                            1.0 / math.sqrt(q.shape[2]))
+    # weights and results are rounded to bf16 once each (2^-9 of a convex sum
+    # of values, which is at most the largest value)
+    bound = 2.0 ** -8 * vc.float().abs().max().item() + 1e-3
+    err = (got.float().cpu() - ref).abs().max().item()
+    assert err < bound, (err, bound)
+
+
+@pytest.mark.parametrize("Hq,Hk,D,fp8", [
+    (16, 4, 128, False), (5, 1, 128, False), (8, 1, 64, False),
+    (8, 8, 128, True), (14, 2, 64, True)])
+@pytest.mark.parametrize("lens,spare", [
+    ([1, 32, 33], 0),              # one run each
+    ([255, 256, 257, 3], 40),      # 8 pages = one run; wide tables
+    ([2049, 40, 8191], 5),         # many runs beside a single one
+])
+def test_decode_runs(Hq, Hk, D, fp8, lens, spare):
+    args = _paged(lens, [1] * len(lens), Hq, Hk, D, fp8, spare, seed=D + Hq)
+    q, kc, vc, bt, sl, ql = (x.to(DEV) for x in args)
+    got = ops.paged_attention(q, kc, vc, bt, sl, ql, 1.0 / math.sqrt(D),
+                              num_decodes_tail=len(lens))
+    _check(args, got)
