@@ -84,10 +84,9 @@ __device__ __forceinline__ pa_frag pa_pack8(pa_f32x8 v) {
 __device__ __forceinline__ u32x2 pa_pack4(f32x4 v) {
   return __builtin_bit_cast(u32x2, __builtin_convertvector(v, pa_bf16x4));
 }
-__device__ __forceinline__ void pa_glds16(const void* g, void* lds) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) u32*)g,
-      (__attribute__((address_space(3))) u32*)lds, 16, 0, 0);
+// an entry of the block table, through the scalar cache (no kernel writes it)
+__device__ __forceinline__ int pa_entry(const int* p, int i) {
+  return ((const __attribute__((address_space(4))) int*)p)[i];
 }
 // transposed reads of rows base..base+3 and base+8.. (or +16..) of a V tile
 __device__ __forceinline__ pa_frag pa_tr(const char* a, const char* b) {
@@ -97,13 +96,28 @@ __device__ __forceinline__ pa_frag pa_tr(const char* a, const char* b) {
       (__attribute__((address_space(3))) pa_s16x4*)b);
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
-// 8 cached elements as bf16
+// Issue order of a run of LDS reads feeding matrix products: AHEAD reads first,
+// then EACH reads behind every product (left alone, the compiler waits for
+// every fragment in front of its product).
+template <int READS, int MFMAS, int AHEAD, int EACH>
+__device__ __forceinline__ void pa_order() {
+  constexpr int STEPS = (READS - AHEAD) / EACH;
+  __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x8, MFMAS - STEPS, 0);
+}
+// 8 cached elements as they are stored, and as bf16
+template <bool KV8> struct PaRaw { typedef u16x8 type; };
+template <> struct PaRaw<true> { typedef u32x2 type; };
 template <bool KV8>
-__device__ __forceinline__ u16x8 pa_cached8(const u8* p) {
+__device__ __forceinline__ u16x8 pa_widen(typename PaRaw<KV8>::type raw) {
   if constexpr (!KV8) {
-    return *(const u16x8*)p;
+    return raw;
   } else {
-    const u32x2 raw = *(const u32x2*)p;
     float f[8];
     fp8x4_to_f32(raw[0], f);
     fp8x4_to_f32(raw[1], f + 4);
@@ -126,6 +140,286 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
   kept = lo;              // kept first keys: [kept, keep_first)
   if (A.window > 0) lo = max(lo, p - A.window + 1);
   return lo;
+}
+
+// ---------------------------------------------------------------------------
+// Prompt pieces. A workgroup owns hpb query heads of one kv head times rpb
+// blocks of 32 rows, one wave each (hpb * rpb = 4), and walks the visible keys
+// 64 at a time: K and V of the next step are on their way in registers while
+// this step is computed and then go to the other half of a double-buffered LDS
+// tile, one barrier a step. (Straight copies into LDS are no use here: the
+// transposed reads wait for every one of them in flight.)
+//
+// Bound by LDS reads (every wave reads the whole K and V tile for its 32 rows:
+// as many cycles as its products take) and by the exponentials beside them. The
+// form before, 32 keys a step, two barriers, V scattered into a transposed tile
+// two bytes at a time and weights passed through LDS, ran at 337 TFLOP/s on a
+// 32 k prompt (16 heads, 4 kv heads, 128; useful flops) and 250 on prompts of
+// 2 k; this one at 860 and 640 (13.1 -> 5.1 ms, 1.10 -> 0.43 ms), 0.78 instead
+// of 1.61 ms on 7 prompts of 3 k with 32 heads over e4m3 pages, 0.11 instead of
+// 0.22 ms on 160 short ones (24 k tokens). Two workgroups a CU (64 KB of LDS,
+// up to 256 registers a lane) are what both limits allow.
+//
+// Entries of the tile map that continue each other (same sequence, 32 rows on)
+// share a workgroup; the entry at a multiple of rpb, or one that continues
+// nothing, leads.
+// ---------------------------------------------------------------------------
+template <int D, bool KV8, bool LOCAL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+paged_prefill_kernel(PagedArgs A) {
+  constexpr int CPR = D / 8;                // 16-byte chunks per row
+  constexpr int TILE = PA_KEYS * D * 2;     // bytes of a K or V tile
+  constexpr int PER = TILE / 1024;          // 1 KB pieces per tile
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 31, hi = lane >> 5;
+  // heads vary fastest: workgroup id i runs on XCD i % 8, so an XCD works on
+  // few kv heads and the tiles that share their pages meet in its L2; long
+  // contexts first
+  const int hgroups = A.Hq / A.hpb;
+  const int hg = blockIdx.x % hgroups;
+  const int e = A.n_tiles - 1 - blockIdx.x / hgroups;
+  const int s = A.tile_seq[e], q0 = A.tile_q0[e];
+  const int k0 = (q0 >> 5) % A.rpb;
+  if (k0 > 0 && e > 0 && A.tile_seq[e - 1] == s && A.tile_q0[e - 1] == q0 - 32)
+    return;
+  int cnt = 1;
+  while (k0 + cnt < A.rpb && e + cnt < A.n_tiles && A.tile_seq[e + cnt] == s &&
+         A.tile_q0[e + cnt] == q0 + 32 * cnt)
+    ++cnt;
+  const int hq = hg * A.hpb + w % A.hpb, rb = w / A.hpb;
+  const int kh = hg * A.hpb / (A.Hq / A.Hk);
+
+  const int nq_total = A.qlocs[s + 1] - A.qlocs[s];
+  const int rows = min(cnt * 32, nq_total - q0);   // of the workgroup
+  if (rows <= 0) return;                    // a padding entry
+  const int row_base = A.qlocs[s] + q0;
+  const int L = A.seq_lens[s];
+  const int p0 = L - nq_total + q0;         // position of the first row
+  const int kv_end = p0 + rows;             // causal bound (exclusive)
+  const int my_r = rb * 32 + ln;            // this lane's row of the workgroup
+  const int my_p = p0 + my_r;
+  const bool live = rb * 32 < rows;         // this wave has rows
+  const int w_end = min(kv_end, p0 + rb * 32 + 32);
+
+  extern __shared__ __attribute__((aligned(16))) char pa_smem[];
+
+  pa_frag qb[D / 16];
+  {
+    const u16* qp =
+        A.q + ((long)(row_base + min(my_r, rows - 1)) * A.Hq + hq) * D + hi * 8;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk) {
+      qb[kk] = *(const s16x8*)(qp + kk * 16);
+      // scores are compared before they are scaled: by a positive number
+      if (A.scale < 0.f) qb[kk] ^= (short)0x8000;
+    }
+  }
+  const float scale = fabsf(A.scale);
+  f32x16 acc[D / 32];
+#pragma unroll
+  for (int b = 0; b < D / 32; ++b) acc[b] = (f32x16)(0.f);
+  float m_run = PA_NONE, l_run = 0.f;
+  if (LOCAL && A.sink) {
+    m_run = A.sink_w ? A.sink_w[hq] * PA_LOG2E : 0.f;
+    l_run = hi == 0 ? 1.f : 0.f;            // the lane pair's sums are added
+  }
+  const float r1 = LOCAL && A.r1 ? A.r1[hq] : 0.f;
+  const float r2 = LOCAL && A.r1 ? A.r2[hq] : 0.f;
+  // lower key bounds: of this lane's row, of the workgroup's first row, and of
+  // this wave's last row (above which a step needs no mask)
+  int lo_row = 0, c_row = 0, kt0 = 0, kf0 = 0, n_kept = 0, lo_last = 0;
+  if (LOCAL) {
+    int c_first, c_last;
+    lo_row = pa_lower(A, my_p, c_row);
+    const int lo_first = pa_lower(A, p0, c_first);
+    lo_last = pa_lower(A, w_end - 1, c_last);
+    kt0 = lo_first / PA_KEYS;
+    kf0 = c_first / PA_KEYS;
+    n_kept = max(min(kt0, (A.keep_first + PA_KEYS - 1) / PA_KEYS) - kf0, 0);
+  }
+  const int kt1 = (kv_end + PA_KEYS - 1) / PA_KEYS;
+  const int steps = n_kept + kt1 - kt0;
+  const int last_page = (kv_end - 1) / PA_PG;
+  const int* table = A.bt + (long)s * A.bt_stride;
+
+  auto step_tile = [&](int it) {
+    return it < n_kept ? kf0 + it : kt0 + (it - n_kept);
+  };
+  // A step is 2 * PER pieces of 1 KB of LDS, of K and then of V, piece c on wave
+  // c % 4; all of its addresses but the lane's own offset are wave-uniform
+  // (made per lane they cost more than the step's products). The second page of
+  // the last step may lie past the context and is then fetched from the last
+  // one (masked).
+  constexpr int ES = KV8 ? 1 : 2;
+  constexpr int RPP = 64 / CPR;             // rows per piece
+  const int st_row = lane / CPR;
+  const u32 koff = (st_row * D + pa_kchunk(st_row, lane % CPR) * 8) * ES;
+  const u32 voff = (st_row * D + pa_vchunk(st_row, lane % CPR) * 8) * ES;
+  typename PaRaw<KV8>::type st[PER / 2];
+  int pa = 0, pb = 0;    // pages of the next step to load
+  auto pages = [&](int kt) {
+    pa = pa_entry(table, min(2 * kt, last_page));
+    pb = pa_entry(table, min(2 * kt + 1, last_page));
+  };
+  auto load = [&]() {
+#pragma unroll
+    for (int j = 0; j < PER / 2; ++j) {
+      const bool isv = j >= PER / 4;
+      const int piece = (isv ? j - PER / 4 : j) * 4 + w;
+      const long blk = j % (PER / 4) >= PER / 8 ? pb : pa;
+      const u8* base = (isv ? A.vc : A.kc) +
+                       ((blk * A.Hk + kh) * PA_PG + piece % (PER / 2) * RPP) *
+                           (D * ES);
+      // rows of odd pieces of 4 rows swizzle keys with row bit 2 set
+      const u32 off =
+          isv ? voff : (RPP == 4 && (w & 1) ? koff ^ (4 * 8 * ES) : koff);
+      st[j] = *(const typename PaRaw<KV8>::type*)(base + off);
+    }
+  };
+  auto store = [&](char* buf) {
+#pragma unroll
+    for (int j = 0; j < PER / 2; ++j)
+      *(u16x8*)(buf + (j * 4 + w) * 1024 + lane * 16) = pa_widen<KV8>(st[j]);
+  };
+
+  // fragment addresses: keys row ln (+32), chunk kk*2 + hi; values rows
+  // 4*hi + ti/4 (+8), columns of 32-block b
+  int kad[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    kad[j] = ln * (2 * D) + pa_kchunk(ln, j * 2 + hi) * 16;
+  const int ti = lane & 15;
+  int vad[2];
+#pragma unroll
+  for (int o = 0; o < 2; ++o)
+    vad[o] = (4 * hi + (ti >> 2)) * (2 * D) +
+             pa_vchunk(ti >> 2,
+                       o * 4 + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) * 16 +
+             (ti & 1) * 8;
+
+  pages(step_tile(0));
+  load();
+  if (steps > 1) pages(step_tile(1));
+  store(pa_smem);
+  for (int it = 0; it < steps; ++it) {
+    __syncthreads();
+    const int kv0 = step_tile(it) * PA_KEYS;
+    const bool more = it + 1 < steps;
+    if (more) load();
+    if (it + 2 < steps) pages(step_tile(it + 2));
+    if (live && kv0 < w_end) {
+    const char* kb = pa_smem + (it & 1) * 2 * TILE;
+    const char* vb = kb + TILE;
+
+    f32x16 d[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) d[h] = (f32x16)(0.f);
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        d[h] = pa_mfma32(*(const s16x8*)(kb + kad[kk & 3] + (kk >> 2) * 128 +
+                                         h * 32 * 2 * D),
+                         qb[kk], d[h]);
+    pa_order<D / 8, D / 8, 6, 1>();
+    // ---- scores: this lane's row, keys kv0 + h*32 + (r&3) + 8*(r>>2) + 4*hi;
+    // without a distance bias they stay unscaled until the exponential
+    float tmax = PA_NONE;
+    const bool whole = kv0 + PA_KEYS <= p0 + rb * 32 + 1 &&
+                       (!LOCAL || kv0 >= lo_last);
+    const bool biased = (LOCAL && A.r1) || scale < 1e-20f;
+    if (biased) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kp = kv0 + h * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+          d[h][r] = d[h][r] * scale -
+                    r1 * __builtin_amdgcn_logf(
+                             1.f + r2 * (float)max(my_p - kp, 0));
+        }
+    }
+    const float mul = biased ? 1.f : scale;
+    if (!whole) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kp = kv0 + h * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+          bool vis = kp <= my_p;
+          if (LOCAL)
+            vis = vis && (kp >= lo_row || (kp < A.keep_first && kp >= c_row));
+          d[h][r] = vis ? d[h][r] : -INFINITY;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, fmaxf(d[0][r], d[1][r]));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * mul;
+    const bool up = tmax > m_run + PA_SLACK;
+    if (__any(up)) {
+      const float m_new = up ? tmax : m_run;
+      const float al = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= al;
+#pragma unroll
+      for (int b = 0; b < D / 32; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[b][r] *= al;
+    }
+    // a row that has seen no key yet: every weight is exp2(-inf) = 0
+    const float m_sub = LOCAL && m_run < 0.1f * PA_NONE ? 0.f : m_run;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      pa_f32x8 p;
+      const int h = ks >> 1;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        p[j] = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(d[h][(ks & 1) * 8 + j], mul, -m_sub));
+        l_run += p[j];
+      }
+      const pa_frag pb = pa_pack8(p);
+#pragma unroll
+      for (int b = 0; b < D / 32; ++b) {
+        const char* at = vb + ks * 16 * 2 * D + vad[b & 1] + (b >> 1) * 128;
+        acc[b] = pa_mfma32(pa_tr(at, at + 8 * 2 * D), pb, acc[b]);
+      }
+    }
+    pa_order<D / 4, D / 8, 8, 2>();
+    }
+    if (more) store(pa_smem + ((it + 1) & 1) * 2 * TILE);
+  }
+
+  if (!live) return;
+  const float l = l_run + __shfl_xor(l_run, 32, 64);
+  float f = l > 0.f ? 1.0f / l : 0.f;
+  const long row = row_base + my_r;
+  if (my_r >= rows) return;
+  const u16* gp = nullptr;
+  if (LOCAL) {
+    f *= A.out_scale;
+    if (A.gate_off >= 0) {
+      gp = A.proj + row * A.ld + A.gate_off + (long)hq * A.gate_n;
+      if (A.gate_n == 1) f *= 1.f / (1.f + expf(-bf2f(gp[0])));
+    }
+  }
+  u16* op = A.out + row * A.ldo + A.out_off + (long)hq * D;
+#pragma unroll
+  for (int b = 0; b < D / 32; ++b)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int col = b * 32 + 8 * g + 4 * hi;
+      f32x4 o;
+#pragma unroll
+      for (int e2 = 0; e2 < 4; ++e2) o[e2] = acc[b][4 * g + e2] * f;
+      if (LOCAL && gp && A.gate_n > 1) {
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2)
+          o[e2] *= 1.f / (1.f + expf(-bf2f(gp[col + e2])));
+      }
+      *(u32x2*)(op + col) = pa_pack4(o);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -197,7 +491,8 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
   constexpr int DB = D / 16;                 // 16-column blocks of O
   constexpr int VL = PA_PG * D / (64 * 8);   // 8-element pieces a lane stages
   constexpr int VT = PA_PG * D * 2;          // bytes of a V page in LDS
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lo16 = lane & 15, g4 = lane >> 4;
   const int G = A.Hq / A.Hk;
   const int kh = blockIdx.x % A.Hk;
@@ -234,19 +529,20 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
   auto page_of = [&](int x) {
     return x < v.n_kept ? v.kf0 + x : v.pg0 + (x - v.n_kept);
   };
-  u16x8 kx[2 * KK], vx[VL];
-  auto load = [&](int x) {
-    const long base =
-        (((long)table[page_of(x)] * A.Hk + kh) * PA_PG) * D;
+  typedef typename PaRaw<KV8>::type Raw;
+  Raw kx[2 * KK], vx[VL];
+  int next = 0;      // page to load next
+  auto load = [&]() {
+    const long base = (((long)next * A.Hk + kh) * PA_PG) * D;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk)
-        kx[h * KK + kk] = pa_cached8<KV8>(
+        kx[h * KK + kk] = *(const Raw*)(
             A.kc + (base + (h * 16 + lo16) * D + kk * 32 + g4 * 8) * ES);
 #pragma unroll
     for (int j = 0; j < VL; ++j)
-      vx[j] = pa_cached8<KV8>(A.vc + (base + (j * 64 + lane) * 8) * ES);
+      vx[j] = *(const Raw*)(A.vc + (base + (j * 64 + lane) * 8) * ES);
   };
   // V fragment addresses: rows 4*g4 + ti/4 (+16), columns of 16-block b
   int vad[4];
@@ -257,13 +553,18 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
              (lo16 & 1) * 8;
 
   int x = begin + w;
-  if (x < end) load(x);
+  if (x < end) {
+    next = pa_entry(table, page_of(x));
+    load();
+    if (x + 4 < end) next = pa_entry(table, page_of(x + 4));
+  }
   for (; x < end; x += 4) {
     // this page's V into the wave's tile, then the next page's loads
 #pragma unroll
     for (int j = 0; j < VL; ++j) {
       const int row = (j * 64 + lane) / (D / 8), c = (j * 64 + lane) % (D / 8);
-      *(u16x8*)(vt + row * (2 * D) + pa_vchunk(row, c) * 16) = vx[j];
+      *(u16x8*)(vt + row * (2 * D) + pa_vchunk(row, c) * 16) =
+          pa_widen<KV8>(vx[j]);
     }
     f32x4 sc[2];
 #pragma unroll
@@ -271,11 +572,13 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
       sc[h] = (f32x4)(0.f);
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk)
-        sc[h] = pa_mfma16(__builtin_bit_cast(pa_frag, kx[h * KK + kk]), qb[kk],
-                          sc[h]);
+        sc[h] = pa_mfma16(
+            __builtin_bit_cast(pa_frag, pa_widen<KV8>(kx[h * KK + kk])), qb[kk],
+            sc[h]);
     }
     const int kv0 = page_of(x) * PA_PG;
-    if (x + 4 < end) load(x + 4);
+    if (x + 4 < end) load();
+    if (x + 8 < end) next = pa_entry(table, page_of(x + 8));
     // ---- this lane: head lo16, keys kv0 + h*16 + g4*4 + r
     float tmax = PA_NONE;
 #pragma unroll
@@ -309,11 +612,26 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
       l_run += p[j];
     }
     const pa_frag pb = pa_pack8(p);
+    // LOCAL keeps the weights' 24 bits: three bf16 terms (the products are
+    // idle here), the other form rounds them to one
+    pa_frag pb2, pb3;
+    if (LOCAL) {
+      p -= __builtin_convertvector(__builtin_bit_cast(pa_bf16x8, pb), pa_f32x8);
+      pb2 = pa_pack8(p);
+      p -= __builtin_convertvector(__builtin_bit_cast(pa_bf16x8, pb2),
+                                   pa_f32x8);
+      pb3 = pa_pack8(p);
+    }
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
       const char* at = vt + vad[b & 3] + (b >> 2) * 128;
+      const pa_frag va = pa_tr(at, at + 16 * 2 * D);
       f32x4 a = acc[b] * al;
-      acc[b] = pa_mfma16(pa_tr(at, at + 16 * 2 * D), pb, a);
+      if (LOCAL) {
+        a = pa_mfma16(va, pb3, a);
+        a = pa_mfma16(va, pb2, a);
+      }
+      acc[b] = pa_mfma16(va, pb, a);
     }
   }
   l_run += __shfl_xor(l_run, 16, 64);
@@ -419,6 +737,19 @@ static inline int pa_splits(long rows, int Hk, int max_pages) {
   long n = want < most ? want : most;
   if (n > PA_MOST_RUNS) n = PA_MOST_RUNS;
   return n < 1 ? 1 : (int)n;
+}
+
+template <int D, bool KV8, bool LOCAL>
+static inline void pa_launch_prefill(PagedArgs A, hipStream_t s) {
+  // K and V are read once for 128 rows: 4, 2 or 1 query heads (what divides
+  // their group) times 1, 2 or 4 row blocks
+  const int G = A.Hq / A.Hk;
+  A.hpb = G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
+  A.rpb = 4 / A.hpb;
+  const size_t smem = 2 * 2 * (size_t)PA_KEYS * D * 2;
+  hipLaunchKernelGGL((paged_prefill_kernel<D, KV8, LOCAL>),
+                     dim3((unsigned)A.n_tiles * (A.Hq / A.hpb)),
+                     dim3(256), smem, s, A);
 }
 
 template <int D, bool KV8, bool LOCAL>

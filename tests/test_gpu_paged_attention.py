@@ -59,3 +59,47 @@ def test_decode_runs(Hq, Hk, D, fp8, lens, spare):
     got = ops.paged_attention(q, kc, vc, bt, sl, ql, 1.0 / math.sqrt(D),
                               num_decodes_tail=len(lens))
     _check(args, got)
+
+
+def _tiles(new):
+    return ([s for s, c in enumerate(new) for _ in range(0, c, 32)],
+            [j for c in new for j in range(0, c, 32)])
+
+
+def _prefill(args, D, tiles):
+    q, kc, vc, bt, sl, ql = (x.to(DEV) for x in args)
+    ts, tq = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in tiles)
+    return ops.paged_attention(q, kc, vc, bt, sl, ql, 1.0 / math.sqrt(D),
+                               num_decodes_tail=0, tile_seq=ts, tile_q0=tq,
+                               prefill_token_count=q.shape[0])
+
+
+# every split of query heads and row blocks over the waves of a workgroup
+@pytest.mark.parametrize("Hq,Hk", [(3, 3), (4, 2), (6, 2), (8, 2), (10, 2),
+                                   (6, 1), (7, 1), (8, 1)])
+@pytest.mark.parametrize("D,fp8", [(128, False), (64, True)])
+def test_prompt_tiles(Hq, Hk, D, fp8):
+    # whole prompts and continued ones around borders of pages, key steps
+    # and row blocks
+    new = [1, 31, 32, 33, 64, 65, 128, 129, 40, 96]
+    ctx = [0, 0, 0, 0, 0, 0, 0, 0, 25, 352]
+    lens = [a + b for a, b in zip(new, ctx)]
+    args = _paged(lens, new, Hq, Hk, D, fp8, seed=Hq)
+    _check(args, _prefill(args, D, _tiles(new)))
+
+
+@pytest.mark.parametrize("Hq,Hk", [(2, 2), (4, 2), (4, 1)])
+def test_prompt_tiles_in_any_order(Hq, Hk):
+    # a tile map need not list a sequence's tiles in order, nor at all
+    new = [200, 130]
+    args = _paged(new, new, Hq, Hk, 128, False, seed=9)
+    ts, tq = _tiles(new)
+    whole = _prefill(args, 128, (ts, tq))
+    _check(args, whole)
+    for order in (list(range(len(ts)))[::-1], [3, 0, 9, 1, 4, 5, 7]):
+        part = _prefill(args, 128, ([ts[i] for i in order],
+                                    [tq[i] for i in order]))
+        for i in order:
+            a = (0 if ts[i] == 0 else 200) + tq[i]
+            b = min(a + 32, 200 if ts[i] == 0 else 330)
+            assert torch.equal(part[a:b], whole[a:b])
