@@ -238,6 +238,7 @@ paged_prefill_kernel(PagedArgs A) {
     kf0 = c_first / PA_KEYS;
     n_kept = max(min(kt0, (A.keep_first + PA_KEYS - 1) / PA_KEYS) - kf0, 0);
   }
+  const u32 kept_n = max(A.keep_first - c_row, 0);
   const int kt1 = (kv_end + PA_KEYS - 1) / PA_KEYS;
   const int steps = n_kept + kt1 - kt0;
   const int last_page = (kv_end - 1) / PA_PG;
@@ -348,8 +349,8 @@ paged_prefill_kernel(PagedArgs A) {
         for (int r = 0; r < 16; ++r) {
           const int kp = kv0 + h * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
           bool vis = kp <= my_p;
-          if (LOCAL)
-            vis = vis && (kp >= lo_row || (kp < A.keep_first && kp >= c_row));
+          if (LOCAL)  // no short circuits: 32 selects, not 32 branches
+            vis &= (kp >= lo_row) | ((u32)(kp - c_row) < kept_n);
           d[h][r] = vis ? d[h][r] : -INFINITY;
         }
     }
@@ -524,6 +525,7 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
 #pragma unroll
   for (int b = 0; b < DB; ++b) acc[b] = (f32x4)(0.f);
   float m_run = PA_NONE, l_run = 0.f;
+  const u32 kept_n = max(A.keep_first - v.c_lo, 0);
 
   const int* table = A.bt + (long)v.s * A.bt_stride;
   auto page_of = [&](int x) {
@@ -592,7 +594,7 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
           if (A.r1)
             z -= r1 * __builtin_amdgcn_logf(1.f +
                                             r2 * (float)max(v.p - kp, 0));
-          vis = vis && (kp >= v.lo || (kp < A.keep_first && kp >= v.c_lo));
+          vis &= (kp >= v.lo) | ((u32)(kp - v.c_lo) < kept_n);
         }
         sc[h][r] = vis ? z : PA_NONE;
         tmax = fmaxf(tmax, sc[h][r]);

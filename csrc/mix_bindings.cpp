@@ -59,6 +59,13 @@ int mix_local_attention_mfma(void*, long, int, const void*, const void*,
                              int, int, const void*, long, int, int, float,
                              const float*, const float*, int, const float*,
                              int, int, int, int, int, int, int, hipStream_t);
+int mix_paged_splits(long, int, int, int, int, int);
+void mix_paged_attention(void*, long, int, const void*, const void*,
+                         const void*, const int*, int, const int*, const int*,
+                         const int*, const int*, int, const int*, long, int,
+                         int, float*, float*, float, int, int, const void*,
+                         long, int, int, float, const float*, const float*,
+                         int, const float*, int, int, int, int, hipStream_t);
 int mix_latent_splits(long, int, int, int, int, int, int);
 int mix_latent_attention(void*, long, int, const void*, const void*,
                          const int*, int, const int*, const int*, const int*,
@@ -365,15 +372,50 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
     if (ok) return;
   }
   // prompt pieces (the first `prefill_rows` rows, tiled 32 rows a tile by
-  // tile_seq / tile_q0) go to the MFMA kernel when the shape allows it;
-  // single-token rows and every other shape go to the generic kernel
+  // tile_seq / tile_q0) go to a matrix-core kernel when the shape allows it,
+  // single-token rows too where keys and values are equally long; every other
+  // shape goes to the generic kernel. The paged kernels read 16 bytes of
+  // queries and pages and write 8 bytes at a time.
+  const bool paged =
+      act_kind(q) == 0 && page == 32 && dk == dv && ldv == dv &&
+      (dk == 64 || dk == 128) && out_off % 4 == 0 && out.stride(0) % 4 == 0 &&
+      (size_t)out.data_ptr() % 8 == 0 && (size_t)q.data_ptr() % 16 == 0 &&
+      (size_t)k_cache.data_ptr() % 16 == 0 &&
+      (size_t)v_cache.data_ptr() % 16 == 0;
+  auto run_paged = [&](int tiles, const int* ts, const int* tq, long first,
+                       long n) {
+    const int ns = n > 0 ? mix_paged_splits(n, (int)G, (int)bt.size(1),
+                                            (int)chunk, (int)window,
+                                            (int)keep_first)
+                         : 1;
+    torch::Tensor po, pml;
+    if (ns > 1) {
+      auto o = q.options().dtype(at::kFloat);
+      po = torch::empty({n * H * ns, dv}, o);
+      pml = torch::empty({n * H * ns, 2}, o);
+    }
+    mix_paged_attention(
+        out.data_ptr(), out.stride(0), (int)out_off, q.data_ptr(),
+        k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr<int>(),
+        (int)bt.size(1), seq_lens.data_ptr<int>(), qlocs.data_ptr<int>(), ts,
+        tq, tiles, token_seq.data_ptr<int>(), first, (int)n, ns,
+        ns > 1 ? po.data_ptr<float>() : nullptr,
+        ns > 1 ? pml.data_ptr<float>() : nullptr, (float)scale, (int)chunk,
+        (int)window, proj.data_ptr(), proj.stride(0), (int)gate_off,
+        (int)gate_n, (float)out_scale, r1, r2, sink ? 1 : 0, sw,
+        (int)keep_first, (int)H, (int)G, (int)dk, cur_stream());
+  };
   long t0 = 0;
   if (act_kind(q) == 0 && tile_seq.has_value() && tile_q0.has_value() &&
       prefill_rows > 0) {
     CHECK_I32(*tile_seq); CHECK_I32(*tile_q0);
     TORCH_CHECK(tile_seq->numel() == tile_q0->numel() && prefill_rows <= T,
                 "tile map sizes");
-    if (mix_local_attention_mfma(
+    if (paged) {
+      run_paged((int)tile_seq->numel(), tile_seq->data_ptr<int>(),
+                tile_q0->data_ptr<int>(), 0, 0);
+      t0 = prefill_rows;
+    } else if (mix_local_attention_mfma(
             out.data_ptr(), out.stride(0), (int)out_off, q.data_ptr(),
             k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr<int>(),
             (int)bt.size(1), seq_lens.data_ptr<int>(), qlocs.data_ptr<int>(),
@@ -384,7 +426,9 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
             (int)G, (int)dk, (int)dv, (int)ldv, (int)page, cur_stream()))
       t0 = prefill_rows;
   }
-  if (t0 < T)
+  if (t0 < T && paged && H / G <= 16)
+    run_paged(0, nullptr, nullptr, t0, T - t0);
+  else if (t0 < T)
     mix_local_attention(out.data_ptr(), out.stride(0), (int)out_off,
                         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                         bt.data_ptr<int>(), (int)bt.size(1),

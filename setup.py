@@ -33,6 +33,7 @@ MIX_SOURCES = [
     "csrc/mix_norm.hip",
     "csrc/mix_attn.hip",
     "csrc/mix_attn_mfma.hip",
+    "csrc/mix_attn_paged.hip",
     "csrc/mix_attn_latent.hip",
     "csrc/mix_delta.hip",
     "csrc/mix_stream.hip",
