@@ -52,8 +52,14 @@ void sutro_sampler_fused(const void*, int, const float*, const float*,
 void sutro_grouped_gemm(void*, const void*, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
                         int, hipStream_t);
-void sutro_moe_combine(void*, const void*, const long*, const float*, int,
+void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
                        int, int, hipStream_t);
+void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
+                    hipStream_t);
+long mix_moe_dispatch_scratch(long, int);
+void mix_moe_dispatch(int*, int*, int*, int*, const int*, const long*, long,
+                      int, int, int, long, int*, const float*, float*,
+                      hipStream_t);
 }
 
 void rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor w, double eps) {
@@ -271,12 +277,53 @@ void moe_combine(torch::Tensor out, torch::Tensor rows, torch::Tensor padpos,
   CHECK_CONTIG(out); CHECK_BF16(out);
   const long T = out.size(0), h = out.size(1), k = padpos.size(1);
   TORCH_CHECK(h % 8 == 0, "h must be a multiple of 8");
-  TORCH_CHECK(padpos.scalar_type() == at::kLong, "padpos must be int64");
+  const bool pos64 = padpos.scalar_type() == at::kLong;
+  TORCH_CHECK(pos64 || padpos.scalar_type() == at::kInt,
+              "padpos must be int64 or int32");
   TORCH_CHECK(w.scalar_type() == at::kFloat, "w must be f32");
   TORCH_CHECK(padpos.is_contiguous() && w.is_contiguous(), "contig");
   sutro_moe_combine(out.data_ptr(), rows.data_ptr(),
-                    padpos.data_ptr<long>(), w.data_ptr<float>(), (int)T,
-                    (int)h, (int)k, cur_stream());
+                    padpos.data_ptr(), pos64 ? 1 : 0, w.data_ptr<float>(),
+                    (int)T, (int)h, (int)k, cur_stream());
+}
+
+// router logits bf16 [T, E] -> the top k experts of every token and their
+// layout in segments of `bm` rows: weights fp32 [T, k], tile_off int32
+// [segs + 1], counts int32 [segs], padpos int32 [T, k]; row_tok int32 (given)
+// names the token of every row. This rank holds experts base..base+n_local-1;
+// with fewer than E of them, one more segment takes the other choices.
+std::vector<torch::Tensor> moe_layout(torch::Tensor logits, long k, long base,
+                                      long n_local, long bm,
+                                      torch::Tensor row_tok) {
+  CHECK_CUDA(logits); CHECK_CONTIG(logits); CHECK_BF16(logits);
+  CHECK_CUDA(row_tok); CHECK_CONTIG(row_tok);
+  TORCH_CHECK(row_tok.scalar_type() == at::kInt, "row_tok int32");
+  const long T = logits.size(0), E = logits.size(1);
+  TORCH_CHECK(k >= 1 && k <= 64 && k <= E && E <= 1024,
+              "router: up to 64 of up to 1024 experts");
+  TORCH_CHECK(base >= 0 && n_local >= 1 && base + n_local <= E, "local experts");
+  TORCH_CHECK(bm == 64 || bm == 128, "bm must be 64 or 128");
+  const long segs = n_local + (n_local < E ? 1 : 0);
+  TORCH_CHECK(row_tok.numel() >= T * k + segs * (bm - 1), "row_tok too short");
+  TORCH_CHECK(T * k + segs * bm < (1l << 31), "too many rows");
+  auto i32 = row_tok.options();
+  auto idx = torch::empty({T, k}, i32);
+  auto wts = torch::empty({T, k}, i32.dtype(at::kFloat));
+  auto tile_off = torch::empty({segs + 1}, i32);
+  auto counts = torch::empty({segs}, i32);
+  auto padpos = torch::empty({T, k}, i32);
+  torch::Tensor scratch;
+  if (const long n = mix_moe_dispatch_scratch(T * k, (int)segs))
+    scratch = torch::empty({n}, i32);
+  sutro_moe_topk(idx.data_ptr<int>(), wts.data_ptr<float>(), logits.data_ptr(),
+                 T, (int)E, (int)k, (int)base, (int)n_local, cur_stream());
+  mix_moe_dispatch(row_tok.data_ptr<int>(), tile_off.data_ptr<int>(),
+                   counts.data_ptr<int>(), padpos.data_ptr<int>(),
+                   idx.data_ptr<int>(), nullptr, T * k, (int)k, (int)segs,
+                   (int)bm, row_tok.numel(),
+                   scratch.defined() ? scratch.data_ptr<int>() : nullptr,
+                   nullptr, nullptr, cur_stream());
+  return {wts, tile_off, counts, padpos};
 }
 
 void sampler_fused(torch::Tensor logits, torch::Tensor temps,
@@ -323,6 +370,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma16_probe", &mfma16_probe, "16x16 MFMA fragment-layout probe");
   m.def("hd64_stage_probe", &hd64_stage_probe, "D=64 decode stage dump probe");
   m.def("moe_combine", &moe_combine, "fused MoE weighted gather-combine");
+  m.def("moe_layout", &moe_layout, "softmax top-k router + expert segments");
   m.def("grouped_gemm", &grouped_gemm,
         "dropless MoE grouped GEMM (padded segments, static grid)");
   m.def("sampler_fused", &sampler_fused,

@@ -321,12 +321,13 @@ extern "C" void sutro_grouped_gemm_weighted(
 
 // ---- fused MoE combine: out[t] = sum_j w[t,j] * rows[padpos[t,j]] ----
 // One thread per (token, 8-element h-chunk); k reads + 1 write per thread,
-// f32 accumulate, bf16 store. Replaces a k-long index_select/addcmul loop
-// (8x3 kernels per layer inside the decode graph).
+// f32 accumulate, bf16 store. In the int32 layout pairs of weight 0 (experts of
+// another rank) have no row to read.
+template <typename P>
 __global__ void __launch_bounds__(256) moe_combine_kernel(
     u16* __restrict__ out,          // [T, h] bf16
     const u16* __restrict__ rows,   // [rows_max, h] bf16
-    const long* __restrict__ padpos,  // [T, k]
+    const P* __restrict__ padpos,   // [T, k]
     const float* __restrict__ w,    // [T, k]
     int T, int h, int k) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -337,6 +338,7 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   for (int j = 0; j < k; ++j) {
     const float wj = w[(long)t * k + j];
+    if (sizeof(P) == 4 && wj == 0.f) continue;
     const long r = padpos[(long)t * k + j];
     const u16x8 v = *(const u16x8*)(rows + r * h + h0);
 #pragma unroll
@@ -349,13 +351,19 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(
 }
 
 extern "C" void sutro_moe_combine(void* out, const void* rows,
-                                  const long* padpos, const float* w, int T,
-                                  int h, int k, hipStream_t stream) {
+                                  const void* padpos, int pos64, const float* w,
+                                  int T, int h, int k, hipStream_t stream) {
   const long total = (long)T * (h / 8);
   if (total == 0) return;
   const long blocks = (total + 255) / 256;
   // no hipGetLastError here: error-state queries are rejected while a
   // stream is capturing (decode steps replay this inside hipGraphs)
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     stream, (u16*)out, (const u16*)rows, padpos, w, T, h, k);
+  if (pos64)
+    hipLaunchKernelGGL(moe_combine_kernel<long>, dim3((unsigned)blocks),
+                       dim3(256), 0, stream, (u16*)out, (const u16*)rows,
+                       (const long*)padpos, w, T, h, k);
+  else
+    hipLaunchKernelGGL(moe_combine_kernel<int>, dim3((unsigned)blocks),
+                       dim3(256), 0, stream, (u16*)out, (const u16*)rows,
+                       (const int*)padpos, w, T, h, k);
 }

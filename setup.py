@@ -23,6 +23,8 @@ SOURCES = [
     "csrc/gemm_tn.hip",
     "csrc/sampler.hip",
     "csrc/grouped_gemm.hip",
+    "csrc/moe_topk.hip",
+    "csrc/moe_dispatch.hip",
 ]
 
 # kernels of layer-list decoders (local attention, gated delta rule, gated
@@ -43,8 +45,9 @@ MIX_SOURCES = [
     "csrc/mix_prenorm.hip",
     "csrc/mix_hyper.hip",
     "csrc/mix_decay.hip",
-    # the matrix-core expert GEMM serves both extensions
+    # the matrix-core expert GEMM and the expert layout serve both extensions
     "csrc/grouped_gemm.hip",
+    "csrc/moe_dispatch.hip",
 ]
 
 # hipcc's automatic packed-fp32 forms are switched off for all device code

@@ -310,7 +310,7 @@ class Qwen3MoE(nn.Module):
     def _workspace(self, T: int, dev) -> dict:
         h = self.down.shape[1]
         m_l = self.gate_up.shape[1] // 2
-        rows_max = T * self.top_k + self.experts_per_rank * self._GG_BM
+        rows_max = T * self.top_k + (self.experts_per_rank + 1) * self._GG_BM
         key = (str(dev), self.gate_up.dtype, h, m_l, self.experts_per_rank)
         ws = _MOE_WS.get(key)
         if ws is None or ws["rows"] < rows_max or ws["max_T"] < T:
@@ -396,11 +396,9 @@ class Qwen3MoE(nn.Module):
     def _forward_grouped(self, x: torch.Tensor) -> torch.Tensor:
         """EXACT dropless top-k execution on the GPU hot path.
 
-        Assignments are sorted by expert into per-expert segments padded to
-        the 64-row kernel tile, so the grouped-GEMM grid is a static upper
-        bound (hipGraph-capturable) and NO assignment is ever dropped —
-        replaces the round-1 capacity-factor bmm path that silently dropped
-        over-capacity tokens. All shaping tensors stay
+        Assignments are laid out in per-expert segments padded to the kernel
+        tile, so the grouped-GEMM grid is a static upper bound (hipGraph-
+        capturable) and NO assignment is ever dropped. All shaping tensors stay
         on device (no host sync); the large transients live in the shared
         prealloc'd workspace (see prealloc_workspace)."""
         T, h = x.shape
@@ -409,9 +407,42 @@ class Qwen3MoE(nn.Module):
         # big batches pad segments to 128 (8-wave 128-row tiles run ~4x the
         # MFMA work per barrier); small batches keep 64 to bound padding
         BM = 128 if T * k >= E_l * 256 else 64
-        dev = x.device
-        ws = self._workspace(T, dev)
-        weights, idx = torch_ref.topk_softmax_router(self.router(x), k)
+        ws = self._workspace(T, x.device)
+        rows_max = T * k + (E_l + 1) * BM                 # static bound
+        row_tok = ws["row_tok"][:rows_max]
+        logits = self.router(x)
+        if x.is_cuda and self.num_experts <= 1024 and k <= 64:
+            w, tile_off, counts, padpos = ops.moe_layout(
+                logits, k, base, E_l, BM, row_tok)
+            tile_off, counts = tile_off[:E_l + 1], counts[:E_l]
+        else:
+            w, tile_off, counts, padpos = self._layout(logits, BM, row_tok)
+        # the GEMMs visit local segments only, which end below this
+        rows = T * k + E_l * BM
+        max_tiles = rows // BM
+        act = ws["act"][:rows]
+        ops.grouped_gemm(act, x, self.gate_up, row_tok, tile_off, counts,
+                         max_tiles, True, bm=BM)
+        out_sorted = ws["out_sorted"][:rows]
+        ops.grouped_gemm(out_sorted, act, self.down, None, tile_off, counts,
+                         max_tiles, False, bm=BM)
+        # deterministic combine in fixed k-order (no float atomics)
+        if x.is_cuda:
+            # fused weighted gather-combine into the workspace (no allocs
+            # inside captured decode steps)
+            out = ws["out"][:T]
+            ops.moe_combine(out, out_sorted, padpos, w)
+            return out
+        contrib = out_sorted[padpos].float()
+        return (contrib * w.view(T, k, 1)).sum(dim=1).to(x.dtype)
+
+    def _layout(self, logits: torch.Tensor, BM: int, row_tok: torch.Tensor):
+        """The expert layout in torch ops (CPU tensors, and more experts or
+        choices than the kernel takes)."""
+        T, k = logits.shape[0], self.top_k
+        E_l, base = self.experts_per_rank, self.expert_base
+        dev = logits.device
+        weights, idx = torch_ref.topk_softmax_router(logits, k)
         flat_e = idx.reshape(-1)                          # [T*k]
         flat_tok = torch.arange(T, device=dev).repeat_interleave(k)
         order = torch.argsort(flat_e, stable=True)
@@ -420,58 +451,33 @@ class Qwen3MoE(nn.Module):
         e_loc = sorted_e - base
         valid = (e_loc >= 0) & (e_loc < E_l)              # EP: local only
         # capture-clean counting: bincount and boolean-mask indexing host-
-        # sync (output size), which silently broke hipGraph capture of MoE
-        # decode steps — every shaping op below is static-shaped
+        # sync (output size); every shaping op below is static-shaped
         counts = torch.zeros(E_l, dtype=torch.int32, device=dev)
         counts.index_add_(0, e_loc.clamp(0, E_l - 1),
                           valid.to(torch.int32))
         padded = (counts + (BM - 1)) // BM * BM
         pad_off = torch.zeros(E_l + 1, dtype=torch.int32, device=dev)
         pad_off[1:] = torch.cumsum(padded, 0)
-        tile_off = pad_off // BM
         # rank of each assignment within its expert segment
         first = torch.searchsorted(sorted_e, sorted_e, side="left")
         pos = torch.arange(T * k, device=dev) - first
-        rows_max = T * k + E_l * BM                       # static bound
-        row_tok = ws["row_tok"][:rows_max]
         row_tok.fill_(-1)
         padpos_sorted = (pad_off[e_loc.clamp(0, E_l - 1).long()].long()
                          + pos)
-        # invalid (non-local EP) assignments redirect to the last slot,
-        # which lies beyond every padded segment (padded_total < rows_max)
-        # so no tile ever reads it — scatter_ keeps shapes static
+        # invalid (non-local EP) assignments redirect to a slot beyond every
+        # padded segment, so no tile ever reads it
         padpos_sorted = torch.where(valid, padpos_sorted,
                                     torch.full_like(padpos_sorted,
-                                                    rows_max - 1))
+                                                    T * k + E_l * BM - 1))
         row_tok.scatter_(0, padpos_sorted, sorted_tok.to(torch.int32))
-        max_tiles = rows_max // BM
-
-        m_l = self.gate_up.shape[1] // 2
-        act = ws["act"][:rows_max]
-        ops.grouped_gemm(act, x, self.gate_up, row_tok, tile_off, counts,
-                         max_tiles, True, bm=BM)
-        out_sorted = ws["out_sorted"][:rows_max]
-        ops.grouped_gemm(out_sorted, act, self.down, None, tile_off, counts,
-                         max_tiles, False, bm=BM)
-        # deterministic combine in fixed k-order (no float atomics): map each
-        # original (token, j) assignment back to its padded row
+        # map each original (token, j) assignment back to its padded row
         padpos = torch.empty(T * k, dtype=torch.long, device=dev)
         padpos[order] = padpos_sorted
-        w_flat = weights.reshape(-1).clone()
         inv_valid = torch.zeros(T * k, dtype=torch.bool, device=dev)
         inv_valid[order] = valid
-        w_flat = torch.where(inv_valid, w_flat,
-                             torch.zeros_like(w_flat)).view(T, k)
-        pp = padpos.view(T, k)
-        if x.is_cuda:
-            # fused weighted gather-combine into the workspace (no allocs
-            # inside captured decode steps)
-            out = ws["out"][:T]
-            ops.moe_combine(out, out_sorted, pp.contiguous(),
-                            w_flat.contiguous())
-            return out
-        contrib = out_sorted[pp].float()
-        return (contrib * w_flat.view(T, k, 1)).sum(dim=1).to(x.dtype)
+        w_flat = weights.reshape(-1)
+        w_flat = torch.where(inv_valid, w_flat, torch.zeros_like(w_flat))
+        return (w_flat.view(T, k), pad_off // BM, counts, padpos.view(T, k))
 
 
 class Qwen3Block(nn.Module):

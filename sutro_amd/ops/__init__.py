@@ -182,6 +182,15 @@ def grouped_gemm(out, a, w, row_tok, tile_off, counts, max_tiles, gate_silu,
                                   max_tiles, gate_silu, bm)
 
 
+def moe_layout(logits, k: int, base: int, n_local: int, bm: int, row_tok):
+    """Softmax top-k router and expert layout of one rank (csrc/moe_topk.hip,
+    csrc/moe_dispatch.hip), GPU only: bf16 logits [T, E] -> (weights fp32
+    [T, k], tile_off, counts, padpos int32 [T, k]); `row_tok` (int32) receives
+    the token of every padded row. The rank holds the experts base .. base +
+    n_local - 1; other choices share one more segment, with weight 0."""
+    return _require_hip().moe_layout(logits, k, base, n_local, bm, row_tok)
+
+
 def moe_combine(out, rows, padpos, w):
     """out[t] = sum_j w[t,j] * rows[padpos[t,j]]: fused bf16 gather-combine
     (csrc/grouped_gemm.hip) on GPU, deterministic torch gather on CPU."""
