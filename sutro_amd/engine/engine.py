@@ -65,6 +65,35 @@ def _setup_tunableop(cfg: EngineConfig) -> None:
     tunable.tuning_enable(_os.environ.get("SUTRO_AMD_TUNABLEOP_TUNE", "0") == "1")
 
 
+class _HostPack:
+    """Integer arrays of one step in one buffer, which reaches the device in
+    one copy: pinned there, so the host goes on while earlier GPU work runs
+    (the pinned allocator does not hand the buffer out again before the copy
+    has been made). 64-bit arrays come first, every array starts on 16
+    bytes."""
+
+    def __init__(self, device: str, fields):
+        self.cuda = str(device).startswith("cuda")
+        self.device = device
+        self.at = []
+        size = 0
+        for name, shape, dtype in fields:
+            n = int(np.prod(shape)) * np.dtype(dtype).itemsize
+            self.at.append((name, shape, dtype, size, n))
+            size += (n + 15) // 16 * 16
+        self.buf = torch.empty(max(size, 16), dtype=torch.uint8,
+                               pin_memory=self.cuda)
+        raw = self.buf.numpy()
+        self.host = {name: raw[o:o + n].view(dtype).reshape(shape)
+                     for name, shape, dtype, o, n in self.at}
+
+    def to_device(self) -> Dict[str, torch.Tensor]:
+        dev = self.buf.to(self.device, non_blocking=True)
+        kinds = {np.int64: torch.int64, np.int32: torch.int32}
+        return {name: dev[o:o + n].view(kinds[dtype]).view(shape)
+                for name, shape, dtype, o, n in self.at}
+
+
 class LLMEngine:
     def __init__(self, cfg: EngineConfig, model: Optional[torch.nn.Module] = None):
         self.cfg = cfg
@@ -253,87 +282,103 @@ class LLMEngine:
     # ---- the step ----
 
     def _build_forward_batch(self, sb: ScheduledBatch) -> ForwardBatch:
+        """The batch's device tensors: filled array by array on the host (a
+        Python loop over 32 k prompt tokens took 27 ms, this takes 2) and sent
+        as one copy."""
         S = len(sb.reqs)
         T = sb.total_tokens
-        input_ids = np.empty(T, dtype=np.int64)
-        positions = np.empty(T, dtype=np.int64)
-        slots = np.empty(T, dtype=np.int64)
-        want_prev = getattr(self.model, "uses_prev_ids", False)
-        prev_ids = np.full(T, -1, dtype=np.int64) if want_prev else None
-        qlocs = np.zeros(S + 1, dtype=np.int32)
-        seq_lens = np.empty(S, dtype=np.int32)
         bs = self.kv.block_size
-        max_blocks = 1
+        tables = self.kv.block_tables
+        counts = np.asarray(sb.num_new_tokens, dtype=np.int64)
+        starts = np.fromiter((r.num_computed_tokens for r in sb.reqs),
+                             np.int64, S)
+        ends = np.cumsum(counts)
+        max_blocks = max([1] + [len(tables[r.req_id]) for r in sb.reqs])
+        want_prev = getattr(self.model, "uses_prev_ids", False)
+
+        # rows that need logits: completing prefills + all decodes
+        ends_prompt = np.fromiter((r.num_prompt_tokens for r in sb.reqs),
+                                  np.int64, S) == starts + counts
+        ends_prompt[sb.num_prefills:] = True
+        logits_rows = ends[ends_prompt] - 1
+        # prefill q-tile map (32 rows per tile) for the GPU flash kernel
+        npf = sb.num_prefills
+        n_tiles = (counts[:npf] + 31) // 32
+        total_tiles = int(n_tiles.sum())
+
+        has_state = self.kv.state is not None
+        pack = _HostPack(self.device, [
+            ("input_ids", (T,), np.int64), ("positions", (T,), np.int64),
+            ("slot_mapping", (T,), np.int64),
+            ("prev_ids", (T if want_prev else 0,), np.int64),
+            ("logits_idx", (len(logits_rows),), np.int64),
+            ("block_tables", (S, max_blocks), np.int32),
+            ("seq_lens", (S,), np.int32),
+            ("query_start_locs", (S + 1,), np.int32),
+            ("token_seq", (T,), np.int32), ("tile_seq", (total_tiles,), np.int32),
+            ("tile_q0", (total_tiles,), np.int32),
+            ("state_slots", (S if has_state else 0,), np.int32)])
+        h = pack.host
+
+        ids, bt = h["input_ids"], h["block_tables"]
+        bt.fill(0)
         cursor = 0
         for s, (req, c) in enumerate(zip(sb.reqs, sb.num_new_tokens)):
             start = req.num_computed_tokens
-            table = self.kv.block_tables[req.req_id]
-            max_blocks = max(max_blocks, len(table))
-            for j in range(c):
-                pos = start + j
+            n = req.num_prompt_tokens
+            if start + c <= n:
+                ids[cursor:cursor + c] = req.prompt_token_ids[start:start + c]
+            else:
                 # async decode: the row's last token is still in flight
                 # (pending tensor overrides fb.input_ids); placeholder here
-                input_ids[cursor] = (req.token_at(pos)
-                                     if pos < req.total_len else 0)
-                positions[cursor] = pos
-                slots[cursor] = table[pos // bs] * bs + pos % bs
-                if want_prev and pos > 0:
-                    prev_ids[cursor] = (input_ids[cursor - 1] if j > 0
-                                        else req.token_at(pos - 1))
-                cursor += 1
-            qlocs[s + 1] = cursor
-            seq_lens[s] = start + c
-        block_tables = np.zeros((S, max_blocks), dtype=np.int32)
-        for s, req in enumerate(sb.reqs):
-            t = self.kv.block_tables[req.req_id]
-            block_tables[s, : len(t)] = t
-
-        # rows that need logits: completing prefills + all decodes
-        logits_rows: List[int] = []
-        for s in range(sb.num_prefills):
-            req, c = sb.reqs[s], sb.num_new_tokens[s]
-            if req.num_computed_tokens + c == req.num_prompt_tokens:
-                logits_rows.append(int(qlocs[s + 1]) - 1)
-        for s in range(sb.num_prefills, S):
-            logits_rows.append(int(qlocs[s + 1]) - 1)
-
-        # prefill q-tile map (32 rows per tile) for the GPU flash kernel
-        tiles_s: List[int] = []
-        tiles_q0: List[int] = []
-        for s in range(sb.num_prefills):
-            c = sb.num_new_tokens[s]
-            for j in range(0, c, 32):
-                tiles_s.append(s)
-                tiles_q0.append(j)
-        prefill_token_count = int(qlocs[sb.num_prefills])
-
-        dev = self.device
-        state_slots = None
-        if self.kv.state is not None:
+                have = min(start + c, req.total_len)
+                row = [req.token_at(i) for i in range(start, have)]
+                ids[cursor:cursor + c] = row + [0] * (c - len(row))
+            if want_prev:
+                h["prev_ids"][cursor] = req.token_at(start - 1) if start else -1
+            table = tables[req.req_id]
+            bt[s, :len(table)] = table
+            cursor += c
+        if want_prev:
+            firsts = np.zeros(T, dtype=bool)
+            firsts[ends - counts] = True
+            rest = np.flatnonzero(~firsts)
+            h["prev_ids"][rest] = ids[rest - 1]
+        seq = np.repeat(np.arange(S, dtype=np.int32), counts)
+        h["token_seq"][:] = seq
+        pos = np.arange(T, dtype=np.int64) + np.repeat(
+            starts - (ends - counts), counts)
+        h["positions"][:] = pos
+        h["slot_mapping"][:] = bt[seq, pos // bs].astype(np.int64) * bs + pos % bs
+        h["query_start_locs"][0] = 0
+        h["query_start_locs"][1:] = ends
+        seq_lens = starts + counts
+        h["seq_lens"][:] = seq_lens
+        h["logits_idx"][:] = logits_rows
+        h["tile_seq"][:] = np.repeat(np.arange(npf, dtype=np.int32), n_tiles)
+        h["tile_q0"][:] = 32 * (np.arange(total_tiles) - np.repeat(
+            np.cumsum(n_tiles) - n_tiles, n_tiles))
+        if has_state:
             slots_of = self.kv.state.slots
-            state_slots = torch.tensor([slots_of[r.req_id] for r in sb.reqs],
-                                       dtype=torch.int32, device=dev)
-        token_seq = torch.from_numpy(np.repeat(
-            np.arange(S, dtype=np.int32),
-            np.asarray(sb.num_new_tokens, dtype=np.int64))).to(dev)
+            h["state_slots"][:] = [slots_of[r.req_id] for r in sb.reqs]
+        d = pack.to_device()
         return ForwardBatch(
-            state_slots=state_slots,
-            token_seq=token_seq,
-            prev_ids=(torch.from_numpy(prev_ids).to(dev) if want_prev
-                      else None),
-            input_ids=torch.from_numpy(input_ids).to(dev),
-            positions=torch.from_numpy(positions).to(dev),
-            slot_mapping=torch.from_numpy(slots).to(dev),
-            block_tables=torch.from_numpy(block_tables).to(dev),
-            seq_lens=torch.from_numpy(seq_lens).to(dev),
-            query_start_locs=torch.from_numpy(qlocs).to(dev),
+            state_slots=d["state_slots"] if has_state else None,
+            token_seq=d["token_seq"],
+            prev_ids=d["prev_ids"] if want_prev else None,
+            input_ids=d["input_ids"],
+            positions=d["positions"],
+            slot_mapping=d["slot_mapping"],
+            block_tables=d["block_tables"],
+            seq_lens=d["seq_lens"],
+            query_start_locs=d["query_start_locs"],
             num_decodes_tail=sb.num_decodes,
-            logits_idx=torch.tensor(logits_rows, dtype=torch.long, device=dev),
+            logits_idx=d["logits_idx"],
             max_seq_len=int(seq_lens.max()) if S else 0,
-            max_query_len=int(max(sb.num_new_tokens)) if S else 0,
-            tile_seq=torch.tensor(tiles_s, dtype=torch.int32, device=dev),
-            tile_q0=torch.tensor(tiles_q0, dtype=torch.int32, device=dev),
-            prefill_token_count=prefill_token_count,
+            max_query_len=int(counts.max()) if S else 0,
+            tile_seq=d["tile_seq"],
+            tile_q0=d["tile_q0"],
+            prefill_token_count=int(ends[npf - 1]) if npf else 0,
         )
 
     def _sampling_reqs(self, sb: ScheduledBatch) -> List[Request]:
@@ -463,9 +508,8 @@ class LLMEngine:
                         cum += c
                         if req.num_computed_tokens + c == req.num_prompt_tokens:
                             rows.append(cum - 1)
-                    idx = torch.tensor(rows, dtype=torch.long,
-                                       device=hidden.device)
-                    logits = self.model.compute_logits(hidden[idx])
+                    logits = self.model.compute_logits(
+                        hidden[self._index(rows)])
                 else:
                     logits = None
             else:
@@ -513,7 +557,7 @@ class LLMEngine:
         Returns fp32 logits [wanted, vocab] in entry order, or None."""
         want_of: Dict[int, List[int]] = {}
         for req, toks, want in entries:
-            req.prompt_token_ids.extend(int(t) for t in toks)
+            req.prompt_token_ids.extend(map(int, toks))
             want_of[id(req)] = list(want)
         sb = self.scheduler.schedule_explicit(
             [(req, len(toks)) for req, toks, _ in entries])
@@ -540,18 +584,17 @@ class LLMEngine:
                     owners.append(req)
                 cum += c
             if self.graph_runner is not None and self.graph_runner.can_run(sub):
+                # (the graph's own buffer: what follows copies out of it)
                 logits = self.graph_runner.run(sub)
-                if rows:
-                    logits = logits[torch.tensor(rows, dtype=torch.long,
-                                                 device=logits.device)]
+                if rows and rows != list(range(len(sub.reqs))):
+                    logits = logits[self._index(rows)]
             else:
                 fb = self._build_forward_batch(sub)
                 hidden = self.model(fb, self.kv)
                 logits = None
                 if rows:
-                    idx = torch.tensor(rows, dtype=torch.long,
-                                       device=hidden.device)
-                    logits = self.model.compute_logits(hidden[idx])
+                    logits = self.model.compute_logits(
+                        hidden[self._index(rows)])
             self._advance_computed(sub)
             if rows:
                 logits = logits.float()
@@ -563,6 +606,11 @@ class LLMEngine:
                         k += n
         parts = [got[id(req)] for req, _, want in entries if len(want)]
         return torch.cat(parts, dim=0) if parts else None
+
+    def _index(self, rows) -> torch.Tensor:
+        pack = _HostPack(self.device, [("rows", (len(rows),), np.int64)])
+        pack.host["rows"][:] = rows
+        return pack.to_device()["rows"]
 
     def finish_replay_request(self, req: Request) -> None:
         self.scheduler.finish(req, FinishReason.STOP)
@@ -676,13 +724,14 @@ class LLMEngine:
                 done_rows.append(s)
                 done_reqs.append(req)
         if done_reqs:
-            vecs = []
             for s, req in zip(done_rows, done_reqs):
                 v = self._emb_sums.pop(req.req_id, None)
-                if v is None:
-                    v = sums[s]
-                vecs.append(v / max(1, req.num_prompt_tokens))
-            mat = torch.stack(vecs)
+                if v is not None:
+                    sums[s] = v
+            rows = self._index(done_rows + [max(1, r.num_prompt_tokens)
+                                            for r in done_reqs])
+            n = len(done_rows)
+            mat = sums[rows[:n]] / rows[n:].unsqueeze(1)
             mat = mat / (mat.norm(dim=-1, keepdim=True) + 1e-12)
             mat_cpu = mat.cpu().numpy()  # ONE sync for the whole step
             for i, req in enumerate(done_reqs):

@@ -42,33 +42,32 @@ class DecodeGraphRunner:
         B = self.max_bucket
         W = self.bt_width
         # static device buffers (shared across buckets; graphs capture views)
-        self.d_ids = torch.zeros(B, dtype=torch.long, device=dev)
-        self.d_pos = torch.zeros(B, dtype=torch.long, device=dev)
-        self.d_slots = torch.zeros(B, dtype=torch.long, device=dev)
-        self.d_bt = torch.zeros(B, W, dtype=torch.int32, device=dev)
-        self.d_sl = torch.ones(B, dtype=torch.int32, device=dev)
+        # and their pinned host staging. What changes every step lies in one
+        # buffer, sent in one copy: ids, positions, slots, the token before
+        # each row's token (models whose embedding looks at token pairs; -1 =
+        # none, padding rows), lengths, and the state slot per row
+        # (recurrent-state models; padding rows use the state cache's scratch
+        # slot and start from position 0 = zero state).
+        self._d_step, (self.d_ids, self.d_pos, self.d_slots, self.d_prev,
+                       self.d_sl, self.d_state) = self._step_fields(B, dev)
+        self._h_step, (self.h_ids, self.h_pos, self.h_slots, self.h_prev,
+                       self.h_sl, self.h_state) = self._step_fields(B, None)
+        for sl, prev in ((self.d_sl, self.d_prev), (self.h_sl, self.h_prev)):
+            sl.fill_(1)
+            prev.fill_(-1)
+        self.d_bt = torch.full((B, W), engine.scratch_block, dtype=torch.int32,
+                               device=dev)
+        self.h_bt = torch.full((B, W), engine.scratch_block, dtype=torch.int32,
+                               pin_memory=True)
         self.d_qlocs = torch.arange(B + 1, dtype=torch.int32, device=dev)
         self.d_tiles = torch.empty(0, dtype=torch.int32, device=dev)
-        # recurrent-state models: state slot per row (padding rows use the
-        # state cache's scratch slot and start from position 0 = zero state)
         self.has_state = engine.kv.state is not None
-        self.d_state = torch.zeros(B, dtype=torch.int32, device=dev)
-        self.h_state = torch.zeros(B, dtype=torch.int32, pin_memory=True)
-        # models whose embedding looks at token pairs: the token before each
-        # row's token (-1 = none; padding rows)
         self.has_prev = getattr(engine.model, "uses_prev_ids", False)
-        self.d_prev = torch.full((B,), -1, dtype=torch.long, device=dev)
-        self.h_prev = torch.full((B,), -1, dtype=torch.long, pin_memory=True)
-        # pinned host staging
-        self.h_ids = torch.zeros(B, dtype=torch.long, pin_memory=True)
-        self.h_pos = torch.zeros(B, dtype=torch.long, pin_memory=True)
-        self.h_slots = torch.zeros(B, dtype=torch.long, pin_memory=True)
-        self.h_bt = torch.zeros(B, W, dtype=torch.int32, pin_memory=True)
-        self.h_sl = torch.ones(B, dtype=torch.int32, pin_memory=True)
         # incremental block-table state: which request's table row i holds, how
         # many blocks of it are written, and its alloc_gen (preemption counter)
         # — at steady decode a row's table only gains one block every
-        # kv_block_size steps, so per-step work is a compare, not a copy
+        # kv_block_size steps, so per-step work is a compare, not a copy (and
+        # the device keeps its rows in steps that change none)
         self._row_req = np.full(B, -1, dtype=np.int64)
         self._row_nb = np.zeros(B, dtype=np.int32)
         self._row_gen = np.zeros(B, dtype=np.int64)
@@ -82,6 +81,17 @@ class DecodeGraphRunner:
         self.logits_out: Dict[int, torch.Tensor] = {}
         self._pool = None
         self._capture_all()
+
+    @staticmethod
+    def _step_fields(B: int, device):
+        """(buffer, its fields): four of B int64 and two of B int32, pinned on
+        the host without a device."""
+        kw = dict(dtype=torch.int64)
+        buf = (torch.zeros(5 * B, pin_memory=True, **kw) if device is None
+               else torch.zeros(5 * B, device=device, **kw))
+        tail = buf[4 * B:].view(torch.int32)
+        return buf, (buf[:B], buf[B:2 * B], buf[2 * B:3 * B], buf[3 * B:4 * B],
+                     tail[:B], tail[B:])
 
     def _fb(self, n: int) -> ForwardBatch:
         return ForwardBatch(
@@ -156,20 +166,14 @@ class DecodeGraphRunner:
         bucket = next(b for b in self.buckets if b >= n)
         if self._h2d_done is not None:
             self._h2d_done.synchronize()
-        self._fill_host(sb, bucket)
-        self.d_ids[:bucket].copy_(self.h_ids[:bucket], non_blocking=True)
-        self.d_pos[:bucket].copy_(self.h_pos[:bucket], non_blocking=True)
-        self.d_slots[:bucket].copy_(self.h_slots[:bucket], non_blocking=True)
-        self.d_bt[:bucket].copy_(self.h_bt[:bucket], non_blocking=True)
-        self.d_sl[:bucket].copy_(self.h_sl[:bucket], non_blocking=True)
-        if self.has_state:
-            self.d_state[:bucket].copy_(self.h_state[:bucket],
-                                        non_blocking=True)
-        if self.has_prev:
+        changed = self._fill_host(sb, bucket)
+        self._d_step.copy_(self._h_step, non_blocking=True)
+        if changed:
+            self.d_bt[:bucket].copy_(self.h_bt[:bucket], non_blocking=True)
+        if self.has_prev and ids_override is not None:
             # with lagged ids (async decode) the host-staged ids ARE the
             # tokens before the overriding ones
-            src = self.h_ids if ids_override is not None else self.h_prev
-            self.d_prev[:bucket].copy_(src[:bucket], non_blocking=True)
+            self.d_prev[:bucket].copy_(self.h_ids[:bucket], non_blocking=True)
         if ids_override is not None:
             self.d_ids[:n].copy_(ids_override, non_blocking=True)
         if self._h2d_done is not None:
@@ -177,8 +181,9 @@ class DecodeGraphRunner:
         self.graphs[bucket].replay()
         return self.logits_out[bucket][:n]
 
-    def _fill_host(self, sb: ScheduledBatch, bucket: int) -> None:
-        """Fill the pinned host staging buffers for a decode batch."""
+    def _fill_host(self, sb: ScheduledBatch, bucket: int) -> bool:
+        """Fill the pinned host staging buffers for a decode batch. Returns
+        whether a block-table row changed."""
         eng = self.engine
         n = len(sb.reqs)
         kv = eng.kv
@@ -207,7 +212,8 @@ class DecodeGraphRunner:
         # and the already-written blocks cover the token being written
         stale = ((row_req[:n] != rid) | (row_gen[:n] != gen)
                  | (row_nb[:n] < p // bs + 1))
-        for i in np.nonzero(stale)[0]:
+        stale = np.nonzero(stale)[0]
+        for i in stale:
             req = sb.reqs[i]
             table = tables[req.req_id]
             tl = len(table)
@@ -235,10 +241,13 @@ class DecodeGraphRunner:
                   if r.num_computed_tokens > 0 else -1) for r in sb.reqs),
                 np.int64, n)
             pv[n:bucket] = -1
+        changed = len(stale) > 0
         if n < bucket:  # padding rows target the reserved scratch block
             ids[n:bucket] = 0
             pos[n:bucket] = 0
             sl[n:bucket] = 1
             bt[n:bucket, 0] = scratch
             slots[n:bucket] = scratch * bs
+            changed = changed or bool((row_req[n:bucket] != -1).any())
             row_req[n:bucket] = -1
+        return changed

@@ -44,9 +44,11 @@ class FinishReason(str, Enum):
     ABORT = "abort"        # cancelled
 
 
-@dataclass
+@dataclass(eq=False)
 class Request:
-    """One row of a batch job as the engine sees it."""
+    """One row of a batch job as the engine sees it. A request is itself, not
+    its fields: comparing those made every look into the running list walk the
+    token lists of its neighbours (105 of 160 ms in a job of 256 rows)."""
 
     req_id: int
     prompt_token_ids: List[int]

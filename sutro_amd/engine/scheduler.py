@@ -94,10 +94,11 @@ class Scheduler:
         rows, everything else is a prefill chunk; prefills come first."""
         prefill: List[tuple] = []
         decode: List[Request] = []
+        live = set(self.running)
         for req, n in plan:
             if n <= 0:
                 continue
-            if req not in self.running:
+            if req not in live:
                 if len(self.running) >= self.cfg.max_num_seqs:
                     raise MemoryError("no free sequence slot for the plan")
                 for q in (self.waiting_p0, self.waiting_p1):
@@ -107,6 +108,7 @@ class Scheduler:
                         pass
                 self.priorities.setdefault(req.req_id, 0)
                 self.running.append(req)
+                live.add(req)
             self.kv.grow(req.req_id, req.num_computed_tokens + n)
             if n == 1 and req.num_computed_tokens > 0:
                 decode.append(req)
