@@ -242,11 +242,15 @@ torch::Tensor mfma16_probe(torch::Tensor a, torch::Tensor b) {
   return c;
 }
 
+static bool tile_rows_ok(long bm) {
+  return bm == 64 || bm == 128 || bm == 256;
+}
+
 void grouped_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
                   c10::optional<torch::Tensor> row_tok, torch::Tensor tile_off,
                   torch::Tensor counts, long max_tiles, bool gate_silu,
                   long bm) {
-  TORCH_CHECK(bm == 64 || bm == 128, "bm must be 64 or 128");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
   CHECK_CUDA(a); CHECK_CONTIG(a); CHECK_BF16(a);
   CHECK_CUDA(w); CHECK_CONTIG(w); CHECK_BF16(w);
   CHECK_CONTIG(out); CHECK_BF16(out);
@@ -255,6 +259,8 @@ void grouped_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
   TORCH_CHECK(K % 64 == 0 && n_cols % 64 == 0,
               "grouped_gemm needs K, n_cols multiples of 64 (K=", K,
               ", n_cols=", n_cols, ")");
+  TORCH_CHECK(bm != 256 || n_cols % (gate_silu ? 128 : 256) == 0,
+              "tiles of 256 rows need n_cols a multiple of 256 (gated: 128)");
   TORCH_CHECK(a.size(1) == K, "A K mismatch");
   TORCH_CHECK(out.size(1) == n_cols, "out width mismatch");
   TORCH_CHECK(tile_off.scalar_type() == at::kInt
@@ -302,7 +308,7 @@ std::vector<torch::Tensor> moe_layout(torch::Tensor logits, long k, long base,
   TORCH_CHECK(k >= 1 && k <= 64 && k <= E && E <= 1024,
               "router: up to 64 of up to 1024 experts");
   TORCH_CHECK(base >= 0 && n_local >= 1 && base + n_local <= E, "local experts");
-  TORCH_CHECK(bm == 64 || bm == 128, "bm must be 64 or 128");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
   const long segs = n_local + (n_local < E ? 1 : 0);
   TORCH_CHECK(row_tok.numel() >= T * k + segs * (bm - 1), "row_tok too short");
   TORCH_CHECK(T * k + segs * bm < (1l << 31), "too many rows");

@@ -24,6 +24,10 @@
 // mode 2), mfma_f32_16x16x32_bf16, fp32 accumulate. 4 waves as 2(M)x2(N),
 // 64x64 macro-tile (expert segments average T*k/E rows — large gemm_tn
 // tiles would mostly be padding).
+//
+// Two kernels by the height of the segments' tiles (the caller pads with the
+// height it passes): tiles of 256 rows for prompts, tiles of 64 and 128 rows for
+// fewer rows an expert and for widths the other does not take.
 #include "common.h"
 
 typedef s16x8 bf16x8;
@@ -89,6 +93,38 @@ __device__ __forceinline__ const bf16x8* gg_frag(const u16* lds, int row,
   return (const bf16x8*)((const char*)lds + gswz(lb));
 }
 
+// the unit between the two expert matrices, on fp32 products
+template <int MODE>
+__device__ __forceinline__ float gg_unit(float v, float u, float limit,
+                                         float rw) {
+  if (MODE == 4) {
+    v *= rw;
+    u *= rw;
+  }
+  if (MODE == 1 || MODE == 4) return v / (1.0f + __expf(-v)) * u;
+  if (MODE == 3) {
+    const float g = fminf(v, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g / (1.0f + __expf(-1.702f * g)) * (u + 1.0f);
+  }
+  if (MODE == 2) {
+    v = fmaxf(v, 0.f);
+    return v * v;
+  }
+  return v;
+}
+
+// expert e with tile_off[e] <= t < tile_off[e + 1]
+__device__ __forceinline__ int gg_expert(const int* tile_off, int n, int t) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (tile_off[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
 // MODE=1: rows gathered, B has two streams (gate/up at N-offset 0 and n_cols), output
 // n_cols wide with silu(g)*u. MODE=0: plain A, plain B, plain store.
 // MODE=2: rows gathered, one B stream, relu(x)^2 in the epilogue.
@@ -117,14 +153,7 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   const int t = blockIdx.x;
   const int n0 = blockIdx.y * BN;
   if (t >= tile_off[n_experts]) return;
-  // binary search: expert e with tile_off[e] <= t < tile_off[e+1]
-  int lo = 0, hi = n_experts - 1;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (tile_off[mid] <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  const int e = lo;
+  const int e = gg_expert(tile_off, n_experts, t);
   const int m0 = (t - tile_off[e]) * BM;              // within-segment row
   const int seg0 = tile_off[e] * BM;                  // segment global base
   const int rows_valid = counts[e] - m0;              // live rows this tile
@@ -222,29 +251,149 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
       for (int r = 0; r < 4; ++r) {
         const int grow = grow0 + r;
         const long o = (long)(seg0 + m0 + grow) * n_cols + gn;
-        float v = accg[i][j][r];
-        if (MODE == 1) {
-          const float g = v;
-          v = g / (1.0f + __expf(-g)) * accu[i][j][r];
-        }
-        if (MODE == 4) {
-          const float rw = row_w[seg0 + m0 + grow];
-          const float g = v * rw;
-          v = g / (1.0f + __expf(-g)) * (accu[i][j][r] * rw);
-        }
-        if (MODE == 3) {
-          const float g = fminf(v, limit);
-          const float u = fminf(fmaxf(accu[i][j][r], -limit), limit);
-          v = g / (1.0f + __expf(-1.702f * g)) * (u + 1.0f);
-        }
-        if (MODE == 2) {
-          v = fmaxf(v, 0.f);
-          v *= v;
-        }
+        const float v = gg_unit<MODE>(
+            accg[i][j][r], GATED ? accu[GATED ? i : 0][GATED ? j : 0][r] : 0.f,
+            limit, MODE == 4 ? row_w[seg0 + m0 + grow] : 1.f);
         out[o] = f2bf(v);
       }
     }
   }
+}
+
+// ---- tiles of 256 rows ----------------------------------------------------
+// 256 rows x 256 weight rows (gated: 128 gate and 128 up rows) a workgroup, 8
+// waves as 2 x 4, each 128 x 64 on mfma_f32_32x32x16_bf16; 64 of k a step, both
+// operands copied straight into a double-buffered LDS tile (128 KB), one
+// barrier a step. Bound by LDS reads and the products together: a wave reads
+// 24 KB a step for 1.05 MFLOP, half of what the 64 x 32 wave tiles of the
+// 128-row kernel need. At 32 experts of 2048 x 2048, gate and up / down:
+// 4096 rows an expert 3187 / 2188 -> 2081 / 1086 us (690 / 502 -> 1057 / 1013
+// TFLOP/s), 375 rows 422 / 249 -> 277 / 145, 187 rows 224 / 163 -> 154 / 89,
+// 96 rows 142 / 67 -> 154 / 89 (the padding: the other kernel's).
+//
+// Row tables are looked up once, not every step. Workgroup id i runs on XCD
+// i % 8: an XCD takes four neighbouring row tiles and goes through all column
+// blocks with them, so what its L2 holds is used by many workgroups at a time.
+#define GW_ROWS 4
+template <int MODE>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gg_wide_kernel(u16* __restrict__ out, const u16* __restrict__ a,
+               const u16* __restrict__ w, const int* __restrict__ row_tok,
+               const int* __restrict__ tile_off, const int* __restrict__ counts,
+               int n_experts, int n_cols, long K, float limit,
+               const float* __restrict__ row_w) {
+  constexpr bool GATED = MODE == 1 || MODE >= 3;
+  constexpr bool GATHER = MODE != 0;
+  constexpr int BN = GATED ? 128 : 256;   // output columns
+  constexpr int TILE = 256 * 128;         // bytes of an operand tile
+  const int nb = n_cols / BN;
+  const int xcd = blockIdx.x & 7, j8 = blockIdx.x >> 3;
+  const int r8 = j8 % (GW_ROWS * nb);
+  const int t = ((j8 / (GW_ROWS * nb)) * 8 + xcd) * GW_ROWS + r8 % GW_ROWS;
+  const int n0 = r8 / GW_ROWS * BN;
+  if (t >= tile_off[n_experts]) return;
+  const int e = gg_expert(tile_off, n_experts, t);
+  const int m0 = (t - tile_off[e]) * 256;
+  const long seg = (long)tile_off[e] * 256 + m0;   // first row of the tile
+  const int live = counts[e] - m0;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 31, hi = lane >> 5;
+  const int wm = wave >> 2, wn = wave & 3;
+  extern __shared__ __attribute__((aligned(16))) char gw_smem[];
+
+  // copies: 1 KB (8 rows of 128 bytes) an instruction, pieces wave*4 + j of
+  // either operand; 16-byte chunks are XOR-swizzled by the row
+  const int pr = lane >> 3, pc = ((lane & 7) ^ pr) * 8;
+  const u16* pa[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = (wave * 4 + j) * 8 + pr;
+    long row;
+    if (GATHER) {
+      row = row_tok[seg + min(r, live - 1)];   // padding rows repeat the last
+      if (row < 0) row = 0;
+    } else {
+      row = seg + r;
+    }
+    pa[j] = a + row * K + pc;
+  }
+  const int br = wave * 32;                    // first of this wave's B rows
+  const long brow = (GATED && br >= 128) ? n_cols + n0 + br - 128 : n0 + br;
+  const u16* pb = w + ((long)e * (GATED ? 2 : 1) * n_cols + brow) * K;
+  const u32 boff = (u32)(pr * K + pc);
+  auto stage = [&](int buf, long k) {
+    char* dst = gw_smem + buf * 2 * TILE + wave * 4096;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      glds16g((const u32*)(pa[j] + k), (u32*)(dst + j * 1024));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      glds16g((const u32*)(pb + k + j * 8 * K + boff),
+              (u32*)(dst + TILE + j * 1024));
+  };
+
+  int kad[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    kad[kk] = ln * 128 + (((kk * 2 + hi) ^ (ln & 7)) << 4);
+  const int arow = wm * 128 * 128;
+  const int brow0 = (GATED ? wn * 32 : wn * 64) * 128 + TILE;
+  const int brow1 = (GATED ? 128 + wn * 32 : wn * 64 + 32) * 128 + TILE;
+
+  f32x16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x16)(0.f);
+
+  const int KT = (int)(K >> 6);
+  stage(0, 0);
+  for (int kt = 0; kt < KT; ++kt) {
+    __syncthreads();
+    if (kt + 1 < KT) stage((kt + 1) & 1, (long)(kt + 1) * 64);
+    const char* at = gw_smem + (kt & 1) * 2 * TILE;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const bf16x8 b0 = *(const bf16x8*)(at + brow0 + kad[kk]);
+      const bf16x8 b1 = *(const bf16x8*)(at + brow1 + kad[kk]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bf16x8 af = *(const bf16x8*)(at + arow + i * 4096 + kad[kk]);
+        acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, b0, acc[i][0],
+                                                            0, 0, 0);
+        acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, b1, acc[i][1],
+                                                            0, 0, 0);
+      }
+    }
+    // ten fragments ahead of the products, then one behind each
+    __builtin_amdgcn_sched_group_barrier(0x100, 10, 0);
+#pragma unroll
+    for (int i = 0; i < 14; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x8, 18, 0);
+  }
+
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const long row =
+          seg + wm * 128 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+      u16* o = out + row * n_cols + n0;
+      const float rw = MODE == 4 ? row_w[row] : 1.f;
+      if (GATED) {
+        o[wn * 32 + ln] = f2bf(
+            gg_unit<MODE>(acc[i][0][r], acc[i][1][r], limit, rw));
+      } else {
+        o[wn * 64 + ln] = f2bf(gg_unit<MODE>(acc[i][0][r], 0.f, limit, rw));
+        o[wn * 64 + 32 + ln] =
+            f2bf(gg_unit<MODE>(acc[i][1][r], 0.f, limit, rw));
+      }
+    }
 }
 
 static void grouped_gemm_launch(void* out, const void* a, const void* w,
@@ -263,6 +412,38 @@ static void grouped_gemm_launch(void* out, const void* a, const void* w,
                        (const u16*)w, row_tok, tile_off, counts, n_experts, \
                        n_cols, K, limit, row_w);                            \
     return;                                                                 \
+  }
+#define GG_MODES(CALL)                                                      \
+  {                                                                         \
+    if (gate_silu == 1) CALL(1)                                             \
+    else if (gate_silu == 3) CALL(3)                                        \
+    else if (gate_silu == 4) CALL(4)                                        \
+    else if (gate_silu == 2) CALL(2)                                        \
+    else CALL(0)                                                            \
+  }
+#define GG_ARGS                                                             \
+  (u16*)out, (const u16*)a, (const u16*)w, row_tok, tile_off, counts,       \
+      n_experts, n_cols, K, limit, row_w
+  const bool gated = gate_silu == 1 || gate_silu >= 3;
+  if (bm == 256) {
+    const int nb = n_cols / (gated ? 128 : 256);
+    const unsigned groups = (unsigned)((max_tiles + 8 * GW_ROWS - 1) /
+                                       (8 * GW_ROWS));
+    const dim3 grid(groups * 8 * GW_ROWS * nb);
+#define GG_WIDE(M)                                                          \
+  {                                                                         \
+    static bool once = [] {                                                 \
+      (void)hipFuncSetAttribute((const void*)gg_wide_kernel<M>,             \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                4 * 256 * 128);                             \
+      return true;                                                          \
+    }();                                                                    \
+    (void)once;                                                             \
+    hipLaunchKernelGGL(gg_wide_kernel<M>, grid, dim3(512), 4 * 256 * 128,   \
+                       stream, GG_ARGS);                                    \
+  }
+    GG_MODES(GG_WIDE)
+    return;
   }
   /* no hipGetLastError in this launcher: error-state queries are rejected
      while a stream is capturing (decode steps replay under hipGraphs) */

@@ -887,6 +887,10 @@ void moe_route(torch::Tensor idx, torch::Tensor wts, torch::Tensor logits,
                 (int)keep, (int)rank, renorm ? 1 : 0, cur_stream());
 }
 
+static bool tile_rows_ok(long bm) {
+  return bm == 64 || bm == 128 || bm == 256;
+}
+
 void moe_dispatch(torch::Tensor row_tok, torch::Tensor tile_off,
                   torch::Tensor counts, torch::Tensor padpos,
                   torch::Tensor idx, long bm,
@@ -899,7 +903,7 @@ void moe_dispatch(torch::Tensor row_tok, torch::Tensor tile_off,
   CHECK_GPU(padpos); CHECK_I32(padpos); CHECK_CONTIG(padpos);
   TORCH_CHECK(idx.dim() == 2 && padpos.sizes() == idx.sizes(), "pair shapes");
   const long T = idx.size(0), k = idx.size(1), E = counts.numel();
-  TORCH_CHECK(bm == 64 || bm == 128, "bm must be 64 or 128");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
   TORCH_CHECK(tile_off.numel() == E + 1 && row_tok.numel() % bm == 0 &&
               row_tok.numel() >= T * k + E * (bm - 1), "segment table sizes");
   TORCH_CHECK((2 * E + 1) * 4 <= 64 * 1024 && T * k < (1L << 31),
@@ -941,7 +945,7 @@ void moe_dispatch_table(torch::Tensor row_tok, torch::Tensor tile_off,
   const long T = ids.size(0), k = table.size(1), E = counts.numel();
   TORCH_CHECK(padpos.dim() == 2 && padpos.size(0) == T && padpos.size(1) == k,
               "pair shapes");
-  TORCH_CHECK(bm == 64 || bm == 128, "bm must be 64 or 128");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
   TORCH_CHECK(tile_off.numel() == E + 1 && row_tok.numel() % bm == 0 &&
               row_tok.numel() >= T * k + E * (bm - 1), "segment table sizes");
   TORCH_CHECK((2 * E + 1) * 4 <= 64 * 1024 && T * k < (1L << 31),
@@ -973,7 +977,7 @@ void expert_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
   const long E = w.size(0), K = w.size(2);
   const long N = glu ? w.size(1) / 2 : w.size(1);
   const long n_rows = out.size(0);
-  TORCH_CHECK(bm == 64 || bm == 128, "bm must be 64 or 128");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
   TORCH_CHECK(act >= 0 && act <= 3, "activation: 0 (none), 1 (silu gate), 2 "
               "(relu squared) or 3 (clamped unit)");
   TORCH_CHECK(!glu || (w.size(1) % 2 == 0 && (act == 1 || limit > 0)),
@@ -1001,7 +1005,11 @@ void expert_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
     rw = row_w->data_ptr<float>();
   }
   // weighted rows: the matrix-core kernel has the silu unit only
-  if (kind == 0 && K % 64 == 0 && N % 64 == 0 && (!rw || act == 1)) {
+  const bool mfma = kind == 0 && K % 64 == 0 && N % 64 == 0 &&
+                    (!rw || act == 1);
+  TORCH_CHECK(bm != 256 || !mfma || N % (glu ? 128 : 256) == 0,
+              "tiles of 256 rows need a multiple of 256 columns (gated: 128)");
+  if (mfma) {
     if (rw)
       sutro_grouped_gemm_weighted(
           out.data_ptr(), a.data_ptr(), w.data_ptr(), rt,

@@ -864,7 +864,7 @@ class RoutedExperts(nn.Module):
         T = h.shape[0]
         w1 = self.gate_up.view(s.experts, 2 * s.ff, self.width) if self.glu \
             else self.up
-        bm = hops.expert_gemm_tile(h, w1, T * s.top)
+        bm = hops.expert_gemm_tile(h, w1, T * s.top, self.glu)
         row_w = None
         if s.router == "table":
             wts, idw = 1.0 / s.top, None

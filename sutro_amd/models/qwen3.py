@@ -290,9 +290,8 @@ class Qwen3MoE(nn.Module):
         out.index_add_(0, flat_tok[order], back_rows.float() * w_sorted)
         return out.to(x_local.dtype)
 
-    _GG_BM = 128  # MAX grouped-gemm tile height (workspace sizing); the
-    # per-call tile is 128 when average segments fill it (big batches),
-    # else 64 (csrc/grouped_gemm.hip tile configurations)
+    _GG_BM = 256  # MAX grouped-gemm tile height (workspace sizing; the
+    # per-call tile is ops.expert_tile's)
 
     def prealloc_workspace(self, max_tokens: int) -> None:
         """Size the shared grouped-MoE workspace BEFORE hipGraph capture.
@@ -404,9 +403,9 @@ class Qwen3MoE(nn.Module):
         T, h = x.shape
         k = self.top_k
         E_l, base = self.experts_per_rank, self.expert_base
-        # big batches pad segments to 128 (8-wave 128-row tiles run ~4x the
-        # MFMA work per barrier); small batches keep 64 to bound padding
-        BM = 128 if T * k >= E_l * 256 else 64
+        m_l = self.gate_up.shape[1] // 2
+        BM = (ops.expert_tile(T * k, self.num_experts, m_l, h)
+              if x.is_cuda else 64)
         ws = self._workspace(T, x.device)
         rows_max = T * k + (E_l + 1) * BM                 # static bound
         row_tok = ws["row_tok"][:rows_max]

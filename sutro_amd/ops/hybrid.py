@@ -25,7 +25,7 @@ from typing import Optional
 
 import torch
 
-from . import torch_ref
+from . import expert_tile, torch_ref
 
 _M = None
 _M_ERR: Optional[str] = None
@@ -387,14 +387,16 @@ def moe_dispatch(idx, experts: int, bm: int, wts=None):
     return layout + (row_w,)
 
 
-def expert_gemm_tile(a, w, n_rows: int) -> int:
-    """Segment padding (rows) the expert GEMM of these operands wants: the
-    matrix-core kernel takes bf16 with K and N multiples of 64 and pads to
-    128 rows when segments are long; everything else runs the plain kernel on
-    64-row tiles."""
-    E = w.shape[0]
-    if a.is_cuda and a.dtype == torch.bfloat16 and n_rows >= E * 256:
-        return 128
+def expert_gemm_tile(a, w, n_rows: int, gated: bool = True) -> int:
+    """Segment padding (rows) the expert GEMMs want whose first one has these
+    operands: the matrix-core kernels take bf16 with K and N multiples of 64
+    and tiles by the rows an expert gets; everything else runs the plain kernel
+    on 64-row tiles."""
+    E, N, K = w.shape
+    inner = N // 2 if gated else N
+    if a.is_cuda and a.dtype == torch.bfloat16 and K % 64 == 0 \
+            and inner % 64 == 0:
+        return expert_tile(n_rows, E, inner, K, gated)
     return 64
 
 
