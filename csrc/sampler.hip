@@ -18,8 +18,9 @@
 // by a 4-level radix descent over the monotonic u32 transform of s_i
 // (256-bucket count+mass histograms per level; boundary bucket recursed).
 //
-// Throughput notes (r2 rocprof: first version ran 2.33 ms per 2048x151,936
-// bf16 call ~ 5x the pass-count HBM bound):
+// Throughput notes (a first version ran 2.33 ms per 2048x151,936 bf16 call,
+// about 5x the pass-count HBM bound; bf16 rows count values instead, see
+// sampler_count_kernel):
 //  - all full-vocab passes consume u16x8 (16 B) per lane per step — the
 //    scalar-u16 version dispatched 8x the instructions for the same bytes;
 //  - the level-0 histogram is 8-way lane-replicated (hist[lane&7][bucket]):
@@ -35,8 +36,20 @@
 #include "common.h"
 
 #define SMP_THREADS 256
-#define SMP_WAVES (SMP_THREADS / 64)
 #define HREP 8  // level-0 histogram replicas
+
+struct SmpArgs {
+  const void* logits;
+  const float* temps;
+  const float* topps;
+  const int* topks;
+  const float* us;
+  const u32* mask;
+  long v_row;
+  int vl, w_words;
+  int* out_tok;
+  float* out_lp;
+};
 
 // monotonic u32 key: key(a) < key(b)  <=>  a < b (floats, no NaN)
 __device__ __forceinline__ u32 f32key(float s) {
@@ -53,6 +66,7 @@ struct Boundary {
   int active;
 };
 
+template <int SMP_WAVES>
 struct SmpShared {
   float wmax[SMP_WAVES];
   int warg[SMP_WAVES];
@@ -74,6 +88,9 @@ struct SmpShared {
   int last_kept[SMP_WAVES];
   int token;
   int done;
+  int chunk;   // of the crossing
+  u64 base;
+  int lastk;
 };
 
 template <bool BF16>
@@ -112,8 +129,9 @@ __device__ __forceinline__ u32 alive_bits8(const u32* mrow, int i0) {
 }
 
 // deterministic block max+argmax (lowest index wins ties)
-__device__ __forceinline__ void block_argmax(SmpShared* sm, float v, int idx,
-                                             int tid) {
+template <int SMP_WAVES>
+__device__ __forceinline__ void block_argmax(SmpShared<SMP_WAVES>* sm, float v,
+                                             int idx, int tid) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     float ov = __shfl_xor(v, off, 64);
@@ -169,20 +187,17 @@ __device__ __forceinline__ void scan_level(const u32* cnt, const u64* mass,
   b->active = 0;  // never crossed: threshold keeps everything
 }
 
-template <bool BF16>
-__global__ void __launch_bounds__(SMP_THREADS)
-sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
-               const float* __restrict__ topps, const int* __restrict__ topks,
-               const float* __restrict__ us, const u32* __restrict__ mask,
-               long v_row, int vl, int w_words, int* __restrict__ out_tok,
-               float* __restrict__ out_lp) {
-  __shared__ SmpShared sm;
-  const int row = blockIdx.x;
-  const int tid = threadIdx.x;
-  const void* lrow = BF16 ? (const void*)((const u16*)logits + (long)row * v_row)
-                          : (const void*)((const float*)logits + (long)row * v_row);
-  const u32* mrow = mask ? mask + (long)row * w_words : nullptr;
-  const float T = temps[row];
+// any logits, any row: one workgroup of THREADS
+template <bool BF16, int THREADS>
+__device__ __forceinline__ void sample_row(const SmpArgs& A, int row, int tid,
+                                           SmpShared<THREADS / 64>& sm) {
+  constexpr int SMP_WAVES = THREADS / 64;
+  const void* lrow =
+      BF16 ? (const void*)((const u16*)A.logits + (long)row * A.v_row)
+           : (const void*)((const float*)A.logits + (long)row * A.v_row);
+  const u32* mrow = A.mask ? A.mask + (long)row * A.w_words : nullptr;
+  const int vl = A.vl;
+  const float T = A.temps[row];
   const bool greedy = T < 1e-5f;
   const float inv_t = greedy ? 1.0f : 1.0f / T;
   const int vl8 = vl & ~7;
@@ -190,7 +205,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
   // ---- pass A: max + argmax over alive (vectorized) ----
   float lmax = -INFINITY;
   int larg = -1;
-  for (int i0 = tid * 8; i0 < vl8; i0 += SMP_THREADS * 8) {
+  for (int i0 = tid * 8; i0 < vl8; i0 += THREADS * 8) {
     const u32 ab = alive_bits8(mrow, i0);
     if (ab == 0) continue;
     float v[8];
@@ -202,7 +217,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
         larg = i0 + j;
       }
   }
-  for (int i = vl8 + tid; i < vl; i += SMP_THREADS)
+  for (int i = vl8 + tid; i < vl; i += THREADS)
     if (alive_bit(mrow, i)) {
       float v = load_logit<BF16>(lrow, i);
       if (v > lmax) {
@@ -214,14 +229,14 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
   const float m = (sm.argmax >= 0) ? sm.m : 0.0f;
   if (sm.argmax < 0) {  // no alive token (should not happen): emit 0
     if (tid == 0) {
-      out_tok[row] = 0;
-      out_lp[row] = -INFINITY;
+      A.out_tok[row] = 0;
+      A.out_lp[row] = -INFINITY;
     }
     return;
   }
 
   // ---- pass B: Z (float + fixed) and 8-way replicated level-0 hist ----
-  for (int i = tid; i < HREP * 256; i += SMP_THREADS) {
+  for (int i = tid; i < HREP * 256; i += THREADS) {
     ((u32*)sm.hist_cnt)[i] = 0;
     ((u64*)sm.hist_mass)[i] = 0;
   }
@@ -229,7 +244,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
   const int rep = tid & (HREP - 1);
   float zf_part = 0.0f;
   u64 zx_part = 0;
-  for (int i0 = tid * 8; i0 < vl8; i0 += SMP_THREADS * 8) {
+  for (int i0 = tid * 8; i0 < vl8; i0 += THREADS * 8) {
     const u32 ab = alive_bits8(mrow, i0);
     if (ab == 0) continue;
     float v[8];
@@ -250,7 +265,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
       }
     }
   }
-  for (int i = vl8 + tid; i < vl; i += SMP_THREADS) {
+  for (int i = vl8 + tid; i < vl; i += THREADS) {
     if (!alive_bit(mrow, i)) continue;
     const float s = (load_logit<BF16>(lrow, i) - m) * inv_t;
     const float p = __expf(s);
@@ -277,7 +292,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
   __syncthreads();
   // reduce histogram replicas into replica 0 (integers: order-free)
   if (!greedy) {
-    for (int b = tid; b < 256; b += SMP_THREADS) {
+    for (int b = tid; b < 256; b += THREADS) {
       u32 c = 0;
       u64 q = 0;
 #pragma unroll
@@ -303,16 +318,16 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
 
   if (greedy) {
     if (tid == 0) {
-      out_tok[row] = sm.argmax;
-      out_lp[row] = -logf(sm.zf);  // s_argmax == 0 at T=1
+      A.out_tok[row] = sm.argmax;
+      A.out_lp[row] = -logf(sm.zf);  // s_argmax == 0 at T=1
     }
     return;
   }
 
   // ---- radix descent: resolve tau_k (count) and tau_p (mass) ----
-  const u32 k_thr = (u32)max(1, topks[row]);
+  const u32 k_thr = (u32)max(1, A.topks[row]);
   if (tid == 0) {
-    double pd = (double)topps[row] * (double)sm.zfix;
+    double pd = (double)A.topps[row] * (double)sm.zfix;
     u64 p_thr = (pd >= (double)sm.zfix) ? sm.zfix : (u64)pd;
     if (p_thr == 0) p_thr = 1;  // top_p ~ 0: keep at least the max token
     sm.bk = Boundary{0u, 0, 0, 0, 0, 1};
@@ -326,7 +341,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
   for (int level = 1; level < 4 && !sm.done; ++level) {
     const int shift_prev = 32 - 8 * level;
     const int shift_cur = shift_prev - 8;
-    for (int i = tid; i < 256; i += SMP_THREADS) {
+    for (int i = tid; i < 256; i += THREADS) {
       sm.hist_cnt[0][i] = 0;
       sm.hist_mass[0][i] = 0;
       sm.hist_cnt[1][i] = 0;
@@ -335,7 +350,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
     __syncthreads();
     const int ka = sm.bk.active, pa = sm.bp.active;
     const u32 kpref = sm.bk.pref, ppref = sm.bp.pref;
-    for (int i0 = tid * 8; i0 < vl8; i0 += SMP_THREADS * 8) {
+    for (int i0 = tid * 8; i0 < vl8; i0 += THREADS * 8) {
       const u32 ab = alive_bits8(mrow, i0);
       if (ab == 0) continue;
       float v[8];
@@ -361,7 +376,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
         }
       }
     }
-    for (int i = vl8 + tid; i < vl; i += SMP_THREADS) {
+    for (int i = vl8 + tid; i < vl; i += THREADS) {
       if (!alive_bit(mrow, i)) continue;
       const float s = (load_logit<BF16>(lrow, i) - m) * inv_t;
       const u32 key = f32key(s);
@@ -382,7 +397,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
     }
     __syncthreads();
     if (tid == 0) {
-      double pd = (double)topps[row] * (double)sm.zfix;
+      double pd = (double)A.topps[row] * (double)sm.zfix;
       u64 p_thr = (pd >= (double)sm.zfix) ? sm.zfix : (u64)pd;
       if (p_thr == 0) p_thr = 1;
       if (sm.bk.active)
@@ -406,7 +421,7 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
       sm.tau = tp;
       sm.kept_mass = sm.bp.above_mass + sm.bp.eq_mass;
     }
-    sm.target = (u64)((double)us[row] * (double)sm.kept_mass);
+    sm.target = (u64)((double)A.us[row] * (double)sm.kept_mass);
     sm.token = -1;
   }
   __syncthreads();
@@ -459,9 +474,6 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
   }
   __syncthreads();
   // phase 1b: pick the crossing chunk (thread 0)
-  __shared__ int s_chunk;
-  __shared__ u64 s_base;
-  __shared__ int s_lastk;
   if (tid == 0) {
     u64 acc = 0;
     int pick = -1, lastk = -1;
@@ -469,21 +481,21 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
       if (sm.last_kept[w2] >= 0) lastk = sm.last_kept[w2];
       if (pick < 0 && acc + sm.chunk_sum[w2] > target) {
         pick = w2;
-        s_base = acc;
+        sm.base = acc;
       }
       acc += sm.chunk_sum[w2];
     }
-    s_chunk = pick;
-    s_lastk = lastk;
+    sm.chunk = pick;
+    sm.lastk = lastk;
     if (pick < 0) sm.token = lastk;  // float-edge fallback: last kept
   }
   __syncthreads();
 
-  if (sm.token < 0 && wv == 0 && s_chunk >= 0) {
+  if (sm.token < 0 && wv == 0 && sm.chunk >= 0) {
     // phase 2: wave 0 streams the chosen chunk with a whole-wave u64 scan
     // (cache-hot after phase 1); ballot early-exit at the crossing
-    const int p0 = min(vl, s_chunk * chunk), p1 = min(vl, p0 + chunk);
-    const u64 rem = target - s_base;
+    const int p0 = min(vl, sm.chunk * chunk), p1 = min(vl, p0 + chunk);
+    const u64 rem = target - sm.base;
     u64 running = 0;
     for (int j = p0; j < p1; j += 64) {
       const int i = j + lane;
@@ -509,14 +521,501 @@ sampler_kernel(const void* __restrict__ logits, const float* __restrict__ temps,
       }
       running += total;
     }
-    if (lane == 0 && sm.token < 0) sm.token = s_lastk;
+    if (lane == 0 && sm.token < 0) sm.token = sm.lastk;
   }
   __syncthreads();
   if (tid == 0) {
     int tok = sm.token >= 0 ? sm.token : sm.argmax;
     float s = (load_logit<BF16>(lrow, tok) - m) * inv_t;
-    out_tok[row] = tok;
-    out_lp[row] = s - logf(sm.zf);
+    A.out_tok[row] = tok;
+    A.out_lp[row] = s - logf(sm.zf);
+  }
+}
+
+template <bool BF16>
+__global__ void __launch_bounds__(SMP_THREADS) sampler_kernel(SmpArgs A) {
+  __shared__ SmpShared<SMP_THREADS / 64> sm;
+  sample_row<BF16, SMP_THREADS>(A, blockIdx.x, threadIdx.x, sm);
+}
+
+// ---- bf16 rows: count the values ----
+//
+// A bf16 logit has one of 65,536 values, and everything above (p, q, the
+// sampling key) is a function of the value alone. So one pass over the row
+// counts the values in LDS, and masses, thresholds and Z come from the counts:
+// the exponential is taken once per value present (about 2,500 of 151,936
+// logits) instead of five times per logit, the sums are the same integers, and
+// the thresholds are found by one scan in order of value. The row stays in
+// registers (1,024 threads, up to 155,648 logits), so that the selection in
+// order of index reads no memory; longer rows are read twice.
+//
+// Counters are 16 bits wide, those of v and -v share a word (128 KB). A row
+// with a value that occurs 65,536 times overflows one; every overflow lowers
+// the sum of the counters, so comparing it with the number of alive tokens
+// finds all of them, and such a row is sampled by the general code.
+//
+// Bound by instruction issue: four to count and sixteen to select per logit.
+// 1024 x 151,936 by the general kernel and here: 1382 -> 197 us (top_p 0.95 at
+// temperature 0.8), 1393 -> 151 with top_k 20, 148 -> 139 greedy, 1338 -> 250
+// with a mask; one row 636 -> 41 us. Of the 50 us that a row takes its
+// workgroup 16 are fixed, clearing and scanning 128 KB of counters.
+#define CNT_MIN 2048
+#define CNT_THREADS 1024
+#define CNT_WAVES (CNT_THREADS / 64)
+#define CNT_CHUNKS 19                          // of 8 logits a thread
+#define CNT_CHUNK (CNT_THREADS * 8)
+#define CNT_TILE (CNT_CHUNKS * CNT_CHUNK)
+#define CNT_SEGS 512                           // of 64 magnitudes
+
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+
+struct CountShared {
+  u32 words[CNT_SEGS * 64];     // [magnitude]: low half of v, high half of -v
+  u64 seg_mass[2 * CNT_SEGS];   // in descending order of value
+  u32 seg_cnt[2 * CNT_SEGS];
+  u64 blk[CNT_CHUNKS];          // of the wave's part that u falls into
+  u64 wave_mass[CNT_WAVES];
+  u32 wave_cnt[CNT_WAVES];
+  u32 wave_alive[CNT_WAVES];
+  float wave_z[CNT_WAVES];
+  int max_pos, min_neg;         // magnitudes of the extremes
+  int seg[2];                   // where the count / the mass crosses
+  u64 above[2];
+  u32 tau[2];
+  int tcode;                    // lowest kept value, as an ordered code
+  int one;                      // and lowest value with p = 1
+  u64 kept;
+  int last, token;
+  u64 base;
+};
+
+// order of the values: as signed 16-bit numbers
+__device__ __forceinline__ s16x2 ordered2(u32 w) {
+  const s16x2 v = __builtin_bit_cast(s16x2, w);
+  const s16x2 m = {0x7fff, 0x7fff};
+  return v ^ ((v >> (short)15) & m);
+}
+
+template <class T>
+__device__ __forceinline__ T wave_sum(T v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+template <class T>
+__device__ __forceinline__ T wave_scan(T v, int lane) {  // inclusive
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const T t = __shfl_up(v, off, 64);
+    if (lane >= off) v += t;
+  }
+  return v;
+}
+
+template <bool MASKED>
+__global__ void __launch_bounds__(CNT_THREADS)
+sampler_count_kernel(SmpArgs A) {
+  extern __shared__ __attribute__((aligned(16))) char cnt_lds[];
+  CountShared& sm = *(CountShared*)cnt_lds;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const u16* lrow = (const u16*)A.logits + (long)row * A.v_row;
+  const u8* mrow = MASKED ? (const u8*)(A.mask + (long)row * A.w_words)
+                          : nullptr;
+  const int vl = A.vl;
+  const int tiles = (vl + CNT_TILE - 1) / CNT_TILE;
+  const int last8 = (vl - 1) & ~7;   // rows are whole eights: readable
+  const float T = A.temps[row];
+  const bool greedy = T < 1e-5f;
+  const float inv_t = greedy ? 1.0f : 1.0f / T;
+
+  // a wave's part of a tile is contiguous: `part` chunks of 512 logits
+  auto part_of = [&](int tile) {
+    return (min(vl - tile * CNT_TILE, CNT_TILE) + CNT_CHUNK - 1) / CNT_CHUNK;
+  };
+  auto eight = [&](int i0) {
+    return *(const u32x4*)((const char*)lrow + 2 * (u32)min(i0, last8));
+  };
+  auto bits8 = [&](int i0) -> u32 {
+    return MASKED ? mrow[min(i0, last8) >> 3] : 0xffu;
+  };
+  // logits that are not alive become 0xffff, the lowest of all values (and, as
+  // a NaN, nobody's logit)
+  auto patch = [&](u32x4& w, u32 bits, int i0) {
+    const int left = vl - i0;
+    if (!MASKED && left >= 8) return;
+    u32 dead = ~bits;
+    if (left < 8) dead |= left > 0 ? 0xffu << left : 0xffu;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      w[j] |= ((dead >> (2 * j)) & 1u) * 0xffffu |
+              ((dead >> (2 * j + 1)) & 1u) * 0xffff0000u;
+  };
+  u32x4 r[CNT_CHUNKS];
+  auto load = [&](int tile) {
+    const int part = part_of(tile);
+    const int t0 = tile * CNT_TILE + wave * part * 512 + lane * 8;
+    u32 bits[CNT_CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c)
+      if (c < part) bits[c] = bits8(t0 + c * 512);
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c)
+      if (c < part) r[c] = eight(t0 + c * 512);
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c)
+      if (c < part) patch(r[c], bits[c], t0 + c * 512);
+  };
+
+  {
+    u32x4* z = (u32x4*)sm.words;
+#pragma unroll
+    for (int i = 0; i < CNT_SEGS * 16 / CNT_THREADS; ++i)
+      z[i * CNT_THREADS + tid] = (u32x4)(0u);
+    sm.seg_mass[tid] = 0;
+    sm.seg_cnt[tid] = 0;
+    if (tid == 0) {
+      sm.max_pos = -1;
+      sm.min_neg = 0x8000;
+      sm.seg[0] = sm.seg[1] = -1;
+      sm.tau[0] = sm.tau[1] = 0;
+      sm.tcode = sm.one = 0x7fff;
+      sm.kept = 0;
+      sm.last = sm.token = -1;
+      sm.base = 0;
+    }
+  }
+  __syncthreads();
+
+  // ---- count the values ----
+  for (int tile = 0; tile < tiles; ++tile) {
+    load(tile);
+    const int part = part_of(tile);
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c) {
+      // lanes without a live logit would all add to one counter
+      if (c < part && (MASKED || r[c][0] != ~0u))
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const u32 w = r[c][j];
+        const u32 lo = w & 0x7fffu, hi = (w >> 16) & 0x7fffu;
+        if (!MASKED || (w & 0xffffu) != 0xffffu)
+          atomicAdd(&sm.words[lo], (w & 0x8000u) ? 0x10000u : 1u);
+        if (!MASKED || w < 0xffff0000u)
+          atomicAdd(&sm.words[hi], (int)w < 0 ? 0x10000u : 1u);
+      }
+    }
+  }
+  // alive tokens, for the check of the counters
+  u32 n_alive = 0;
+  if (MASKED)
+    for (int i = tid; i * 32 < vl; i += CNT_THREADS) {
+      u32 w = ((const u32*)mrow)[i];
+      if (vl - i * 32 < 32) w &= (1u << (vl - i * 32)) - 1;
+      n_alive += __popc(w);
+    }
+  else if (tid == 0)
+    n_alive = vl;
+  __syncthreads();
+  if (tid == 0) sm.words[0x7fff] &= 0xffffu;   // 0xffff: not alive
+  __syncthreads();
+
+  // ---- segments that hold a value, and the largest value ----
+  // segment j * CNT_WAVES + wave is this wave's, so that neighbours spread
+  u32 present = 0;
+  int max_pos = -1, min_neg = 0x8000;
+#pragma unroll 4
+  for (int j = 0; j < CNT_SEGS / CNT_WAVES; ++j) {
+    const int mag0 = (j * CNT_WAVES + wave) * 64;
+    const u32 w = sm.words[mag0 + lane];
+    if (__ballot(w != 0) == 0) continue;
+    present |= 1u << j;
+    const bool number = mag0 + lane <= 0x7f80;   // not a NaN
+    const u64 p = __ballot(number && (w & 0xffffu) != 0);
+    const u64 n = __ballot(number && (w >> 16) != 0);
+    if (p) max_pos = mag0 + 63 - __clzll(p);
+    if (n) min_neg = min(min_neg, mag0 + __ffsll((unsigned long long)n) - 1);
+  }
+  if (lane == 0) {
+    atomicMax(&sm.max_pos, max_pos);
+    atomicMin(&sm.min_neg, min_neg);
+  }
+  __syncthreads();
+  const bool pos = sm.max_pos >= 0;
+  // nothing above -inf counted: none alive, or a counter overflowed
+  const bool none = !pos && sm.min_neg >= 0x7f80;
+  float m = bf2f((u16)(pos ? sm.max_pos : 0x8000 | sm.min_neg));
+
+  // ---- Z, and counts and masses by segment ----
+  float z = 0.f;
+  int one = 0x7fff;
+  for (u32 left = present; left; left &= left - 1) {
+    const int seg = (__ffs(left) - 1) * CNT_WAVES + wave;
+    const int mag = seg * 64 + lane;
+    const u32 w = sm.words[mag];
+    const u32 cp = w & 0xffffu, cn = w >> 16;
+    const float v = bf2f((u16)mag);
+    if (__ballot(cp != 0)) {
+      const float p = __expf((v - m) * inv_t);
+      if (cp) z += (float)cp * p;
+      if (cp && p >= 1.f) one = min(one, mag);
+      const u64 q = (u64)(p * 4294967296.0f);
+      const u64 ms = wave_sum(cp ? q * cp : (u64)0);
+      const u32 cs = wave_sum(cp);
+      if (lane == 0) {
+        sm.seg_mass[CNT_SEGS - 1 - seg] = ms;
+        sm.seg_cnt[CNT_SEGS - 1 - seg] = cs;
+      }
+    }
+    if (__ballot(cn != 0)) {
+      const float p = __expf((-v - m) * inv_t);
+      if (cn) z += (float)cn * p;
+      if (cn && p >= 1.f) one = min(one, -1 - mag);
+      const u64 q = (u64)(p * 4294967296.0f);
+      const u64 ms = wave_sum(cn ? q * cn : (u64)0);
+      const u32 cs = wave_sum(cn);
+      if (lane == 0) {
+        sm.seg_mass[CNT_SEGS + seg] = ms;
+        sm.seg_cnt[CNT_SEGS + seg] = cs;
+      }
+    }
+  }
+  if (one != 0x7fff) atomicMin(&sm.one, one);
+  z = wave_sum(z);
+  n_alive = wave_sum(n_alive);
+  if (lane == 0) {
+    sm.wave_z[wave] = z;
+    sm.wave_alive[wave] = n_alive;
+  }
+  __syncthreads();
+
+  // ---- running count and mass, from the largest value down ----
+  const u64 my_mass = sm.seg_mass[tid];
+  const u32 my_cnt = sm.seg_cnt[tid];
+  u64 mass = wave_scan(my_mass, lane);
+  u32 cnt = wave_scan(my_cnt, lane);
+  if (lane == 63) {
+    sm.wave_mass[wave] = mass;
+    sm.wave_cnt[wave] = cnt;
+  }
+  __syncthreads();
+  // every wave scans the sixteen sums
+  const int l16 = lane & (CNT_WAVES - 1);
+  u64 wm = sm.wave_mass[l16];
+  u32 wc = sm.wave_cnt[l16], want = sm.wave_alive[l16];
+  float zf = sm.wave_z[l16];
+#pragma unroll
+  for (int off = 1; off < CNT_WAVES; off <<= 1) {
+    const u64 tm = __shfl_up(wm, off, CNT_WAVES);
+    const u32 tc = __shfl_up(wc, off, CNT_WAVES);
+    wm += l16 >= off ? tm : 0;
+    wc += l16 >= off ? tc : 0;
+    want += __shfl_xor(want, off, CNT_WAVES);
+    zf += __shfl_xor(zf, off, CNT_WAVES);
+  }
+  const u64 zfix = __shfl(wm, CNT_WAVES - 1, 64);
+  const u32 counted = __shfl(wc, CNT_WAVES - 1, 64);
+  const u64 mass0 = wave ? __shfl(wm, wave - 1, 64) : 0;
+  const u32 cnt0 = wave ? __shfl(wc, wave - 1, 64) : 0;
+  // ... or zeros of both signs on top, of which the first is the maximum and
+  // decides whether the other sign ranks below
+  const bool zeros = pos && sm.max_pos == 0 && sm.min_neg == 0;
+  if (none || counted != want || (zeros && !greedy)) {
+    __syncthreads();
+    sample_row<true, CNT_THREADS>(A, row, tid,
+                                  *(SmpShared<CNT_WAVES>*)cnt_lds);
+    return;
+  }
+  // a greedy row: the first of the tokens of the largest value
+  u64 target = 0;
+  int tcode = m > 0.f ? sm.max_pos : (m < 0.f ? -1 - sm.min_neg : -1);
+  if (!greedy) {
+    mass += mass0;
+    cnt += cnt0;
+    const u32 k_thr = (u32)max(1, A.topks[row]);
+    const double pd = (double)A.topps[row] * (double)zfix;
+    u64 p_thr = (pd >= (double)zfix) ? zfix : (u64)pd;
+    if (p_thr == 0) p_thr = 1;   // top_p ~ 0: keep at least the max token
+    if (cnt >= k_thr && cnt - my_cnt < k_thr) {
+      sm.seg[0] = tid;
+      sm.above[0] = cnt - my_cnt;
+    }
+    if (mass >= p_thr && mass - my_mass < p_thr) {
+      sm.seg[1] = tid;
+      sm.above[1] = mass - my_mass;
+    }
+    __syncthreads();
+    // the crossing value within its segment: wave 0 the count's, wave 1 the
+    // mass's
+    if (wave < 2 && sm.seg[wave] >= 0) {
+      const int e = sm.seg[wave];
+      const bool up = e < CNT_SEGS;
+      const int mag = up ? (CNT_SEGS - 1 - e) * 64 + 63 - lane
+                         : (e - CNT_SEGS) * 64 + lane;
+      const u32 w = sm.words[mag];
+      const u32 cv = up ? w & 0xffffu : w >> 16;
+      const float v = bf2f((u16)(up ? mag : 0x8000 | mag));
+      const float s = (v - m) * inv_t;
+      u64 own = cv;
+      if (wave == 1) own = cv ? (u64)(__expf(s) * 4294967296.0f) * cv : 0;
+      const u64 sum = wave_scan(own, lane) + sm.above[wave];
+      const u64 thr = wave == 0 ? (u64)k_thr : p_thr;
+      if (sum >= thr && sum - own < thr) sm.tau[wave] = f32key(s);
+    }
+    __syncthreads();
+
+    // ---- kept mass, and the lowest kept value ----
+    // different values can have one key (v - m rounds): all of them are kept
+    const u32 tau = max(sm.tau[0], sm.tau[1]);
+    u64 kept = 0;
+    tcode = 0x7fff;
+    for (u32 left = present; left; left &= left - 1) {
+      const int mag = ((__ffs(left) - 1) * CNT_WAVES + wave) * 64 + lane;
+      const u32 w = sm.words[mag];
+      const u32 cp = w & 0xffffu, cn = w >> 16;
+      const float v = bf2f((u16)mag);
+      const float sp = (v - m) * inv_t, sn = (-v - m) * inv_t;
+      if (cp && f32key(sp) >= tau) {
+        kept += (u64)(__expf(sp) * 4294967296.0f) * cp;
+        tcode = min(tcode, mag);
+      }
+      if (cn && f32key(sn) >= tau) {
+        kept += (u64)(__expf(sn) * 4294967296.0f) * cn;
+        tcode = min(tcode, -1 - mag);
+      }
+    }
+    kept = wave_sum(kept);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      tcode = min(tcode, __shfl_xor(tcode, off, 64));
+    if (lane == 0 && tcode != 0x7fff) {
+      atomicAdd((unsigned long long*)&sm.kept, (unsigned long long)kept);
+      atomicMin(&sm.tcode, tcode);
+    }
+    __syncthreads();
+    target = (u64)((double)A.us[row] * (double)sm.kept);
+    tcode = sm.tcode;
+  }
+
+  // ---- selection in order of index ----
+  // by float order: apart from the zeros (see above) that of the codes
+  const float low = bf2f((u16)(tcode >= 0 ? tcode : 0x7fff ^ tcode));
+  // floor(p 2**32) of one logit; the conversion stops at 2**32 - 1, so that
+  // values of p = 1 lack one
+  auto q32 = [&](float v) -> u32 {
+    return v >= low ? (u32)(__expf((v - m) * inv_t) * 4294967296.0f) : 0u;
+  };
+  auto mass8 = [&](const u32x4& w) {
+    u64 sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sum += q32(__uint_as_float(w[j] << 16));
+      sum += q32(__uint_as_float(w[j] & 0xffff0000u));
+    }
+    return sum;
+  };
+  const int top_code = sm.one;
+  const float top = bf2f((u16)(top_code >= 0 ? top_code : 0x7fff ^ top_code));
+  auto ones8 = [&](const u32x4& w) {
+    u32 n = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      n += (__uint_as_float(w[j] << 16) >= top) +
+           (__uint_as_float(w[j] & 0xffff0000u) >= top);
+    return n;
+  };
+  auto best8 = [&](const u32x4& w) {
+    s16x2 t = ordered2(w[0]);
+#pragma unroll
+    for (int j = 1; j < 4; ++j) t = __builtin_elementwise_max(t, ordered2(w[j]));
+    return max((int)t[0], (int)t[1]);
+  };
+  auto mass_of = [&](const u32x4& w) -> u64 {   // a wave together
+    const int best = best8(w);
+    if (!__ballot(best >= tcode)) return 0;
+    u64 sum = mass8(w);
+    if (__ballot(best >= top_code)) sum += ones8(w);
+    return sum;
+  };
+  for (int tile = 0; tile < tiles; ++tile) {
+    if (tiles > 1) load(tile);
+    const int part = part_of(tile), t0 = tile * CNT_TILE;
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c) asm volatile("" : "+v"(r[c]));
+    u64 sum = 0;
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c) {
+      if (c < part) sum += mass_of(r[c]);
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) sm.wave_mass[wave] = sum;
+    __syncthreads();
+    // the wave's part that holds u (every wave finds it), its chunks again
+    u64 at = sm.base, next = at;
+    int own = -1;
+    for (int w2 = 0; w2 < CNT_WAVES; ++w2) {
+      next = at + sm.wave_mass[w2];
+      if (next > target) {
+        own = w2;
+        break;
+      }
+      at = next;
+    }
+    if (own >= 0) {
+      const int p0 = t0 + own * part * 512 + lane * 8;
+      for (int c = wave; c < part; c += CNT_WAVES) {
+        u32x4 w = eight(p0 + c * 512);
+        patch(w, bits8(p0 + c * 512), p0 + c * 512);
+        const u64 s8 = wave_sum(mass_of(w));
+        if (lane == 0) sm.blk[c] = s8;
+      }
+      __syncthreads();
+      if (wave == 0) {
+        int c = 0;
+        while (c < part - 1 && at + sm.blk[c] <= target) at += sm.blk[c++];
+        const int i0 = p0 + c * 512;
+        u32x4 w = eight(i0);
+        patch(w, bits8(i0), i0);
+        u64 q[8], mine = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float v = __uint_as_float(j & 1 ? w[j >> 1] & 0xffff0000u
+                                                : w[j >> 1] << 16);
+          q[j] = (u64)q32(v) + (v >= top);
+          mine += q[j];
+        }
+        const u64 to = wave_scan(mine, lane) + at;
+        u64 from = to - mine;
+        if (to > target && from <= target) {
+          int tok = i0;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            if (from <= target) tok = i0 + j;
+            from += q[j];
+          }
+          sm.token = tok;
+        }
+      }
+      __syncthreads();
+      break;
+    }
+    __syncthreads();   // all have read base
+    if (tid == 0) sm.base = next;
+  }
+  if (sm.token < 0) {   // u at the upper edge: the last kept token
+    for (int i = tid; i < vl; i += CNT_THREADS)
+      if ((!MASKED || ((mrow[i >> 3] >> (i & 7)) & 1u)) &&
+          ordered2((u32)lrow[i])[0] >= tcode)
+        atomicMax(&sm.last, i);
+    __syncthreads();
+    if (tid == 0) sm.token = sm.last;
+    __syncthreads();
+  }
+  if (tid == 0) {
+    const int tok = sm.token;
+    A.out_tok[row] = tok;
+    A.out_lp[row] = (bf2f(lrow[tok]) - m) * inv_t - logf(zf);
   }
 }
 
@@ -528,14 +1027,27 @@ extern "C" void sutro_sampler_fused(const void* logits, int logits_f32,
                                     int* out_tok, float* out_lp,
                                     hipStream_t stream) {
   if (n == 0) return;
+  const SmpArgs A = {logits, temps, topps, topks, us, mask, v_row, vl, w_words,
+                     out_tok, out_lp};
   dim3 grid((unsigned)n), block(SMP_THREADS);
-  if (logits_f32)
-    hipLaunchKernelGGL((sampler_kernel<false>), grid, block, 0, stream, logits,
-                       temps, topps, topks, us, mask, v_row, vl, w_words,
-                       out_tok, out_lp);
-  else
-    hipLaunchKernelGGL((sampler_kernel<true>), grid, block, 0, stream, logits,
-                       temps, topps, topks, us, mask, v_row, vl, w_words,
-                       out_tok, out_lp);
+  // counting: rows of whole, aligned 16-byte pieces, from 2048 logits on (there
+  // 124 -> 67 us for 1024 rows and 91 -> 17 us for one; below that no
+  // vocabulary in use, and the general kernel has no 128 KB to clear)
+  if (!logits_f32 && vl >= CNT_MIN && v_row % 8 == 0 &&
+      (size_t)logits % 16 == 0) {
+    const auto fn = mask ? sampler_count_kernel<true>
+                         : sampler_count_kernel<false>;
+    constexpr int lds = sizeof(CountShared) > sizeof(SmpShared<CNT_WAVES>)
+                            ? sizeof(CountShared)
+                            : sizeof(SmpShared<CNT_WAVES>);
+    (void)hipFuncSetAttribute((const void*)fn,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(fn, grid, dim3(CNT_THREADS), lds, stream, A);
+  } else if (logits_f32) {
+    hipLaunchKernelGGL((sampler_kernel<false>), grid, block, 0,
+                       stream, A);
+  } else {
+    hipLaunchKernelGGL((sampler_kernel<true>), grid, block, 0, stream, A);
+  }
   HIP_CHECK_LAUNCH();
 }

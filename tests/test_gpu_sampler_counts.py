@@ -1,0 +1,134 @@
+"""The sampler's counting kernel (bf16 rows) at the rows where its bookkeeping
+can go wrong, against the same arithmetic in whole numbers: q = floor(p 2**32)
+of float32 exponentials, whose sums are exact. The kernel's exponential takes
+exp2 of a rounded product, so p is off by up to (1 + |s|) 2**-24 of itself;
+weighted with p that is below 2**-22 of a sum, of the sum up to a token and of
+the whole: a token must hold u within 2**-21. Logprobs: 1e-5, which is 40 ulp
+of a sum of float32 exponentials in another order."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from sutro_amd import ops
+
+DEV = "cuda"
+
+
+def pack(keep):
+    n, v = keep.shape
+    words = (v + 31) // 32
+    bits = torch.zeros(n, words * 32, dtype=torch.int64)
+    bits[:, :v] = keep.long().cpu()
+    w = (bits.view(n, words, 32) << torch.arange(32)).sum(-1)
+    return torch.where(w >= 2**31, w - 2**32, w).to(torch.int32).to(DEV)
+
+
+def check(logits, vl, temp, top_p, top_k, u, keep=None):
+    n = logits.shape[0]
+    temps = torch.full((n,), temp, device=DEV)
+    top_ps = torch.full((n,), top_p, device=DEV)
+    top_ks = torch.full((n,), top_k or vl, dtype=torch.int32, device=DEV)
+    us = torch.full((n,), u, device=DEV)
+    tok = torch.empty(n, dtype=torch.int32, device=DEV)
+    lp = torch.empty(n, device=DEV)
+    ops.sampler_fused(logits, temps, top_ps, top_ks, us,
+                      pack(keep) if keep is not None else None, vl, tok, lp)
+    tok, lp = tok.long().cpu(), lp.cpu()
+    for r in range(n):
+        v = logits[r, :vl].cpu().float()
+        alive = torch.ones(vl, dtype=torch.bool) if keep is None \
+            else keep[r, :vl].cpu()
+        m = v[(alive & (v == v[alive].max())).nonzero()[0, 0]]   # its sign too
+        t = int(tok[r])
+        s = (v - m) * (1.0 if temp == 0 else 1.0 / torch.tensor(temp))
+        p = torch.where(alive, s.exp(), 0.0)
+        want = s[t] - p.double().sum().log()
+        assert abs(float(lp[r]) - float(want)) < 1e-5, (r, temp)
+        if temp == 0:
+            assert t == int(torch.where(alive & (v == m))[0][0])
+            continue
+        q = (p.double() * 2**32).floor().long()
+        s = torch.where(alive, s, -torch.inf)
+        # scaled logits rank by their bits: -0.0 below 0.0
+        s = torch.where((s == 0) & s.signbit(), -1e-45, s)
+        order = s.argsort(descending=True, stable=True)
+        ss, above = s[order], q[order].cumsum(0) - q[order]
+        first = torch.searchsorted(-ss, -ss)        # of the values that tie
+        ok = (first < (top_k or vl)) & \
+            (above[first].double() < max(1.0, top_p * float(q.sum())))
+        kept = torch.zeros(vl, dtype=torch.bool)
+        kept[order] = ok
+        kept &= alive
+        c = torch.where(kept, q, 0).cumsum(0).double() / \
+            float(q[kept].sum())
+        eps = 2.0**-21
+        assert kept[t], (r, temp, top_p, top_k)
+        assert u < c[t] + eps and u >= (c[t - 1] if t else 0.0) - eps, \
+            (r, temp, top_p, top_k, t)
+    return tok, lp
+
+
+# one chunk, tails of a chunk, a full tile (19 chunks of 8192) and more
+@pytest.mark.parametrize("row,vl", [(2048, 2048), (8192, 8191), (8200, 8193),
+                                    (16384, 9001), (155648, 155648),
+                                    (155656, 155649), (200000, 199999)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_sizes(row, vl, masked):
+    g = torch.Generator().manual_seed(row + masked)
+    n = 3
+    # nine values, spread so that every boundary is far from any u here
+    lg = (torch.randint(-4, 5, (n, row), generator=g) * 0.75)
+    lg = lg.to(torch.bfloat16).to(DEV)
+    keep = torch.rand(n, row, generator=g) < 0.4 if masked else None
+    for temp, top_p, top_k, u in ((0.7, 0.83, 0, 0.313), (1.3, 1.0, 0, 0.777),
+                                  (1.0, 1.0, 40, 0.5), (0.0, 1.0, 0, 0.5),
+                                  (1.0, 1e-9, 0, 0.9)):
+        check(lg, vl, temp, top_p, top_k, u, keep)
+    # the last token alone alive
+    if masked:
+        keep = torch.zeros(n, row, dtype=torch.bool)
+        keep[:, vl - 1] = True
+        tok, lp = check(lg, vl, 0.9, 0.9, 3, 0.99, keep)
+        assert (tok == vl - 1).all() and lp.abs().max() == 0
+
+
+def test_values_that_repeat_beyond_a_counter():
+    """65,535 to 131,072 tokens of one value: the 16-bit counters overflow and
+    the rows are sampled all the same."""
+    v = 140000
+    for value in (0.0, -2.5, 3.0):
+        for reps in (65535, 65536, 65537, 131072):
+            lg = torch.full((1, v), value - 1.0)
+            lg[0, 500:500 + reps] = value
+            lg[0, 500 + reps:] = float("-inf")
+            lg = lg.to(torch.bfloat16).to(DEV)
+            for temp, top_k, u in ((1.0, 0, 0.37), (0.8, 7, 0.99), (0.0, 0, 0.)):
+                check(lg, v, temp, 1.0, top_k, u)
+
+
+def test_extreme_rows():
+    v = 4096
+    ninf = float("-inf")
+    base = torch.full((8, v), ninf)
+    base[1, 77] = 1.0                                  # one finite logit
+    base[2, :] = torch.linspace(-1.5e38, 1.5e38, v)    # the whole range
+    base[3, 10], base[3, 20] = -0.0, 0.0               # zeros, -0 first
+    base[4, 10], base[4, 20] = 0.0, -0.0               # zeros, +0 first
+    base[5, :] = torch.arange(v) * 1e-20               # keys that coincide:
+    base[5, 7] = 9.0                                   # all but one at -9
+    base[6, 100:200] = -torch.logspace(-38, 1, 100)    # subnormal steps
+    base[7, :] = -1.0
+    lg = base.to(torch.bfloat16).to(DEV)
+    for temp, top_p, top_k, u in ((1.0, 1.0, 0, 0.4), (0.5, 0.9, 2, 0.9),
+                                  (0.0, 1.0, 0, 0.0), (2.0, 1.0, 1, 0.6)):
+        check(lg[1:], v, temp, top_p, top_k, u)
+    # nothing alive, by the logits or by the mask: token 0, logprob -inf
+    one = torch.ones(1, device=DEV)
+    for row, mask in ((0, None), (1, torch.zeros(1, v, dtype=torch.bool))):
+        tok = torch.full((1,), 9, dtype=torch.int32, device=DEV)
+        lp = torch.zeros(1, device=DEV)
+        ops.sampler_fused(lg[row:row + 1], one, one, (one * v).int(), one * 0.5,
+                          None if mask is None else pack(mask), v, tok, lp)
+        assert tok.item() == 0 and lp.item() == ninf
