@@ -56,6 +56,8 @@ void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
                        int, int, hipStream_t);
 void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
                     hipStream_t);
+void sutro_linear_skinny(void*, long, const void*, long, const void*,
+                         const void*, int, int, int, int, hipStream_t);
 long mix_moe_dispatch_scratch(long, int);
 void mix_moe_dispatch(int*, int*, int*, int*, const int*, const long*, long,
                       int, int, int, long, int*, const float*, float*,
@@ -332,6 +334,36 @@ std::vector<torch::Tensor> moe_layout(torch::Tensor logits, long k, long base,
   return {wts, tile_off, counts, padpos};
 }
 
+// out [M, N] = x [M, K] @ w [N, K]^T (+ bias), or, `gated`, silu of the first
+// N rows of w [2 N, K] times the other N; bf16, up to 32 rows
+torch::Tensor linear_skinny(torch::Tensor x, torch::Tensor w,
+                            c10::optional<torch::Tensor> bias, bool gated) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device(),
+              "operands on one GPU");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16, "bf16 operands");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.is_contiguous() &&
+              x.stride(1) == 1, "matrix operands, rows contiguous");
+  const long M = x.size(0), K = x.size(1), rows = w.size(0);
+  const long N = gated ? rows / 2 : rows;
+  TORCH_CHECK(w.size(1) == K && K >= 32 && K % 32 == 0 && N % 4 == 0 &&
+              (!gated || rows == 2 * N) && M >= 1 && M <= 32 &&
+              rows < (1l << 31) && K < (1l << 31), "unsupported sizes");
+  TORCH_CHECK(x.stride(0) % 8 == 0 && (size_t)x.data_ptr() % 16 == 0 &&
+              (size_t)w.data_ptr() % 16 == 0, "16-byte rows");
+  const void* b = nullptr;
+  if (bias.has_value()) {
+    TORCH_CHECK(bias->is_cuda() && bias->scalar_type() == at::kBFloat16 &&
+                bias->is_contiguous() && bias->numel() == rows, "bias");
+    b = bias->data_ptr();
+  }
+  auto out = torch::empty({M, N}, x.options());
+  sutro_linear_skinny(out.data_ptr(), N, x.data_ptr(), x.stride(0),
+                      w.data_ptr(), b, (int)M, (int)N, (int)K, gated ? 1 : 0,
+                      cur_stream());
+  return out;
+}
+
 void sampler_fused(torch::Tensor logits, torch::Tensor temps,
                    torch::Tensor topps, torch::Tensor topks, torch::Tensor us,
                    c10::optional<torch::Tensor> mask, long vl,
@@ -376,6 +408,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma16_probe", &mfma16_probe, "16x16 MFMA fragment-layout probe");
   m.def("hd64_stage_probe", &hd64_stage_probe, "D=64 decode stage dump probe");
   m.def("moe_combine", &moe_combine, "fused MoE weighted gather-combine");
+  m.def("linear_skinny", &linear_skinny, "linear layer over few rows");
   m.def("moe_layout", &moe_layout, "softmax top-k router + expert segments");
   m.def("grouped_gemm", &grouped_gemm,
         "dropless MoE grouped GEMM (padded segments, static grid)");

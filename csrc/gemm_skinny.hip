@@ -1,0 +1,228 @@
+// Linear layers over few rows (decode steps): out[M, N] = x[M, K] W[N, K]^T (+
+// bias), bf16 with fp32 sums, M up to 32, optionally with the gated unit of a
+// feed-forward behind it (W: N gate rows, then N up rows).
+//
+// Bound by the weights, which are read once, and for the small matrices of a
+// step by the time to get enough loads in flight. A workgroup owns 16 or 32
+// rows of W (gated: 16 and 16) and its waves split k, each with a batch of
+// fragments ahead of its products (gemm_stream.h); their sums meet in LDS. The
+// split is as fine as leaves every wave four k-steps, so that also a 2048 x
+// 2048 matrix keeps 2000 waves of loads in flight. Against the library: 2048 x
+// 2048 at 16 rows 11.0 -> 6.5 us, 4096 x 4096 15.5 -> 12.5; at more rows or
+// longer k the waves read too much of x, which nothing shares.
+#include "common.h"
+#include "gemm_stream.h"
+
+struct SkinnyArgs {
+  u16* out;
+  const u16* x;
+  const u16* w;
+  const u16* bias;   // [N] or null
+  long ldx, ldo;
+  int M, N, K;
+  int act;           // 0 none, 1 silu(gate) up (W has 2 N rows)
+};
+
+template <int NF, int MB, int WAVES, bool GATED>
+__global__ void __launch_bounds__(WAVES * 64) skinny_kernel(SkinnyArgs A) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, g = lane >> 4;
+  constexpr int COLS = GATED ? 16 : NF * 16;
+  const int n0 = blockIdx.x * COLS;
+  const int steps = A.K / GS_STEP;
+  const int s0 = steps * wave / WAVES, s1 = steps * (wave + 1) / WAVES;
+  const long k0 = (long)s0 * GS_STEP + g * 8;
+
+  const u16* wp[NF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+    const int r = GATED ? min(n0 + lr, A.N - 1) + i * A.N
+                        : min(n0 + i * 16 + lr, A.N - 1);
+    wp[i] = A.w + (long)r * A.K + k0;
+  }
+  const u16* ap[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+    ap[m] = A.x + (long)min(m * 16 + lr, A.M - 1) * A.ldx + k0;
+  f32x4 acc[NF][MB];
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) acc[i][m] = (f32x4)(0.f);
+  if (s1 > s0) gs_dot<NF, MB>(wp, ap, s1 - s0, acc);
+
+  __shared__ f32x4 red[WAVES][NF][MB][64];
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) red[wave][i][m][lane] = acc[i][m];
+  __syncthreads();
+  // one thread four neighbouring columns of a row
+  constexpr int OUTS = (GATED ? 1 : NF) * MB;
+  for (int z = threadIdx.x; z < OUTS * 64; z += WAVES * 64) {
+    const int l = z & 63, m = (z >> 6) % MB, i = (z >> 6) / MB;
+    const int row = m * 16 + (l & 15);
+    const int col = n0 + i * 16 + (l >> 4) * 4;
+    f32x4 y = red[0][i][m][l], u;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) y += red[w][i][m][l];
+    if (row >= A.M || col >= A.N) continue;
+    if (GATED) {
+      u = red[0][NF - 1][m][l];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) u += red[w][NF - 1][m][l];
+    }
+    if (A.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        y[e] += bf2f(A.bias[col + e]);
+        if (GATED) u[e] += bf2f(A.bias[A.N + col + e]);
+      }
+    }
+    if (GATED) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = y[e] / (1.f + __expf(-y[e])) * u[e];
+    }
+    *(u32x2*)(A.out + (long)row * A.ldo + col) = gs_pack4(y);
+  }
+}
+
+// One or two rows: no matrix core, its blocks of 16 rows would be mostly empty
+// and reading the fragments holds a workgroup to 16 neighbouring weight rows.
+// Here a workgroup owns four (gated: two and two), the lanes of its waves lie
+// along k, 1 KB of a weight row per load, and all of a wave's loads of two
+// steps are in flight together. Against the library, one row: 2048 x 2048 10.9
+// -> 4.8 us, 32768 x 4096 61.5 -> 48.8 (5.5 TB/s); 2 x 8192 x 2048 with the unit
+// behind it 19.6 -> 14.0.
+template <int MR, int WAVES, bool GATED>
+__global__ void __launch_bounds__(WAVES * 64) gemv_kernel(SkinnyArgs A) {
+  constexpr int R = 4, V = R * MR;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int COLS = GATED ? R / 2 : R;
+  const int n0 = blockIdx.x * COLS;
+  const u16* wp[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    wp[i] = A.w + (long)(GATED ? n0 + (i & 1) + (i >> 1) * A.N : n0 + i) * A.K;
+  float acc[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) acc[v] = 0.f;
+  const int step = WAVES * 512;
+  for (int k0 = threadIdx.x * 8; k0 < A.K; k0 += 2 * step) {
+    u16x8 w[2][R], x[2][MR];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int k = min(k0 + b * step, A.K - 8);
+#pragma unroll
+      for (int i = 0; i < R; ++i) w[b][i] = *(const u16x8*)(wp[i] + k);
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+        x[b][m] = *(const u16x8*)(A.x + (long)min(m, A.M - 1) * A.ldx + k);
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (k0 + b * step >= A.K) break;
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int m = 0; m < MR; ++m)
+            acc[i * MR + m] = fmaf(bf2f(w[b][i][e]), bf2f(x[b][m][e]),
+                                   acc[i * MR + m]);
+    }
+  }
+  // the lanes of 64 / V neighbours end with the sum of one value: half the
+  // values go to the other half of the lanes at each step
+  int v0 = 0;
+#pragma unroll
+  for (int half = V / 2, bit = 32; half >= 1; half /= 2, bit /= 2) {
+    const bool up = lane & bit;
+#pragma unroll
+    for (int v = 0; v < V / 2; ++v)
+      if (v < half) {
+        const float give = up ? acc[v] : acc[v + half];
+        const float keep = up ? acc[v + half] : acc[v];
+        acc[v] = keep + __shfl_xor(give, bit, 64);
+      }
+    v0 += up ? half : 0;
+  }
+#pragma unroll
+  for (int bit = 32 / V; bit >= 1; bit /= 2)
+    acc[0] += __shfl_xor(acc[0], bit, 64);
+  __shared__ float red[WAVES][V];
+  if ((lane & (64 / V - 1)) == 0) red[wave][v0] = acc[0];
+  __syncthreads();
+  const int m = threadIdx.x % MR, c = threadIdx.x / MR;
+  if (c >= COLS || m >= A.M) return;
+  auto total = [&](int i) {
+    float y = red[0][i * MR + m];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) y += red[w][i * MR + m];
+    const int col = GATED ? n0 + (i & 1) + (i >> 1) * A.N : n0 + i;
+    return A.bias ? y + bf2f(A.bias[col]) : y;
+  };
+  float y = total(c);
+  if (GATED) y = y / (1.f + __expf(-y)) * total(c + 2);
+  A.out[(long)m * A.ldo + n0 + c] = f2bf(y);
+}
+
+template <int MR, bool GATED>
+static void gemv_launch(const SkinnyArgs& A, hipStream_t s) {
+  const unsigned blocks = A.N / (GATED ? 2 : 4);
+#define LAUNCH_GV(WW)                                                        \
+  hipLaunchKernelGGL((gemv_kernel<MR, WW, GATED>), dim3(blocks),             \
+                     dim3(WW * 64), 0, s, A)
+  if (A.K <= 1024) LAUNCH_GV(1);
+  else if (A.K <= 2048 || blocks >= 2048) LAUNCH_GV(2);
+  else if (A.K <= 4096) LAUNCH_GV(4);
+  else LAUNCH_GV(8);
+#undef LAUNCH_GV
+}
+
+template <int NF, int MB, bool GATED>
+static void skinny_launch(const SkinnyArgs& A, hipStream_t s) {
+  const unsigned blocks = (A.N + (GATED ? 16 : NF * 16) - 1) /
+                          (GATED ? 16 : NF * 16);
+  const int steps = A.K / GS_STEP;
+#define LAUNCH_SK(WW)                                                        \
+  hipLaunchKernelGGL((skinny_kernel<NF, MB, WW, GATED>), dim3(blocks),       \
+                     dim3(WW * 64), 0, s, A)
+  // waves that split k: toward 2048 in all, at least four k-steps each
+  if (blocks >= 1024 || steps < 16) LAUNCH_SK(2);
+  else if (blocks >= 512 || steps < 32) LAUNCH_SK(4);
+  else if (blocks >= 256 || steps < 64) LAUNCH_SK(8);
+  else LAUNCH_SK(16);
+#undef LAUNCH_SK
+}
+
+// K % 32 == 0, N % 4 == 0, 1 <= M <= 32, 16-byte rows of x and w, 8-byte rows
+// of out
+extern "C" void sutro_linear_skinny(void* out, long ldo, const void* x,
+                                    long ldx, const void* w, const void* bias,
+                                    int M, int N, int K, int act,
+                                    hipStream_t s) {
+  SkinnyArgs A = {(u16*)out, (const u16*)x, (const u16*)w, (const u16*)bias,
+                  ldx, ldo, M, N, K, act};
+  const int mb = (M + 15) / 16;
+#define SK_GEMV(MR)                                                          \
+  do {                                                                       \
+    if (act == 1) gemv_launch<MR, true>(A, s);                               \
+    else gemv_launch<MR, false>(A, s);                                       \
+    return;                                                                  \
+  } while (0)
+  if (M == 1) SK_GEMV(1);
+  if (M == 2) SK_GEMV(2);
+#undef SK_GEMV
+#define SK_MB(NF, GG)                                                        \
+  do {                                                                       \
+    if (mb == 1) skinny_launch<NF, 1, GG>(A, s);                             \
+    else skinny_launch<NF, 2, GG>(A, s);                                     \
+  } while (0)
+  if (act == 1) SK_MB(2, true);
+  else if (N >= 8192) SK_MB(2, false);
+  else SK_MB(1, false);
+#undef SK_MB
+}

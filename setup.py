@@ -24,6 +24,7 @@ SOURCES = [
     "csrc/sampler.hip",
     "csrc/grouped_gemm.hip",
     "csrc/moe_topk.hip",
+    "csrc/gemm_skinny.hip",
     "csrc/moe_dispatch.hip",
 ]
 

@@ -15,12 +15,14 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import ops
 from ..engine.batch import ForwardBatch
 from ..engine.kv_cache import PagedKVCache
 from ..ops import hybrid as hops
 from .hybrid_spec import (AttnMixerSpec, DecayAttnMixerSpec, DeltaMixerSpec,
                           LatentAttnMixerSpec, MLSTMMixerSpec,
                           RoutedExpertsSpec, SSDMixerSpec, TiedAttnMixerSpec)
+from .linear import Linear
 
 _ALIGN = 8  # section starts are multiples of 8 columns (16 B in bf16)
 
@@ -66,7 +68,7 @@ class SectionedLinear(nn.Module):
                      if self.biased else None)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
 
     def section_targets(self, prefix: str, names: Dict[str, str]):
         """Checkpoint tensor -> (parameter, dim, start, length, scale) for the
@@ -464,7 +466,7 @@ class LatentAttention(nn.Module):
             cq = torch.empty((T, s.q_rank), dtype=dt, device=dev)
             hops.section_rmsnorm(proj, off[tag + "dq"], s.q_rank, self.dq_norm,
                                  self.eps, cq)
-            q = F.linear(cq, self.uq)              # [T, H*(dk+rd)]
+            q = ops.linear(cq, self.uq)            # [T, H*(dk+rd)]
         else:
             q = proj[:, off[tag + "q"]:off[tag + "q"] + self.q_cols]
         q = q.unflatten(1, (H, dk + rd))
@@ -800,7 +802,7 @@ class RoutedExperts(nn.Module):
                 width, [("gate", spec.shared_ff, False),
                         ("up", spec.shared_ff, False)]
                 + ([("sg", 1, False)] if spec.shared_gate else []), dtype)
-            self.shared_down = nn.Linear(spec.shared_ff, width, bias=False,
+            self.shared_down = Linear(spec.shared_ff, width, bias=False,
                                          dtype=dtype)
 
     def param_targets(self, prefix: str, ck: str):

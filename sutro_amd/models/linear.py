@@ -1,0 +1,21 @@
+"""The decoders' linear layer: torch's, with the product of ops.linear."""
+
+from __future__ import annotations
+
+import torch
+import torch.nn as nn
+
+from .. import ops
+
+
+class Linear(nn.Linear):
+    def forward(self, input: torch.Tensor) -> torch.Tensor:
+        return ops.linear(input, self.weight, self.bias)
+
+
+def bare(layer: nn.Module) -> bool:
+    """Whether a caller may fuse this layer's product with what follows it: a
+    Linear without bias, hooks or a forward of its own."""
+    return (type(layer) is Linear and layer.bias is None
+            and not layer._forward_hooks and not layer._forward_pre_hooks
+            and "forward" not in layer.__dict__)

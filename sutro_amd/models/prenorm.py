@@ -32,6 +32,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import ops
 from ..engine.batch import ForwardBatch
 from ..engine.kv_cache import PagedKVCache
 from ..ops import hybrid as hops
@@ -42,6 +43,7 @@ from .hybrid_spec import (AttnMixerSpec, DecayAttnMixerSpec, DeltaMixerSpec,
 from .layers import (DecayAttention, GatedDeltaRule, HyperConnection,
                      LatentAttention, LocalAttention, RoutedExperts,
                      SectionedLinear, SSDMixer, _pad)
+from .linear import Linear
 
 
 class PreNormBlock(nn.Module):
@@ -73,7 +75,7 @@ class PreNormBlock(nn.Module):
         self.in_proj = SectionedLinear(W, self.mixer.in_sections(""), dtype)
         k = _pad(self.mixer.out_width)
         self.out_padded = k != self.mixer.out_width
-        self.out_proj = nn.Linear(k, W, bias=False, dtype=dtype)
+        self.out_proj = Linear(k, W, bias=False, dtype=dtype)
         self.ff = layer.ff
         self.relu2 = layer.ff_kind == "relu2"
         self.experts: Optional[RoutedExperts] = None
@@ -83,7 +85,7 @@ class PreNormBlock(nn.Module):
             self.ff_in = SectionedLinear(
                 W, [("up", layer.ff, False)] if self.relu2 else
                 [("gate", layer.ff, False), ("up", layer.ff, False)], dtype)
-            self.ff_out = nn.Linear(layer.ff, W, bias=False, dtype=dtype)
+            self.ff_out = Linear(layer.ff, W, bias=False, dtype=dtype)
         if layer.moe is not None:
             self.experts = RoutedExperts(layer.moe, W, dtype)
         self.streams = spec.streams
@@ -238,7 +240,7 @@ class PreNormModel(nn.Module):
             self.register_buffer("sum_in", torch.ones(spec.streams),
                                  persistent=False)
         if not spec.tie_embeddings:
-            self.lm_head = nn.Linear(W, spec.vocab_size, bias=False, dtype=dtype)
+            self.lm_head = Linear(W, spec.vocab_size, bias=False, dtype=dtype)
         self.act_dtype = dtype
         # debugging aid: when set to a list, the fp32 residual stream after
         # every layer run is appended to it
@@ -331,7 +333,7 @@ class PreNormModel(nn.Module):
 
     @torch.no_grad()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        logits = F.linear(hidden, self.embed_tokens.weight
+        logits = ops.linear(hidden, self.embed_tokens.weight
                           if self.spec.tie_embeddings
                           else self.lm_head.weight).float()
         if self.spec.logit_scale != 1.0:

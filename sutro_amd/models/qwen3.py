@@ -2,8 +2,9 @@
 
 One architecture covers the whole registry: RMSNorm + RoPE-NeoX + GQA paged
 attention + SwiGLU MLP (dense) or top-k routed SwiGLU experts (MoE).
-GEMMs go through F.linear (hipBLASLt on ROCm); everything between GEMMs is a
-hand-written HIP kernel on GPU (see sutro_amd/ops).
+GEMMs go through ops.linear (hipBLASLt on ROCm, a kernel of its own for decode
+steps of few rows); everything between GEMMs is a hand-written HIP kernel on GPU
+(see sutro_amd/ops).
 """
 
 from __future__ import annotations
@@ -21,6 +22,7 @@ from ..engine.batch import ForwardBatch
 from ..engine.kv_cache import PagedKVCache
 from ..ops import torch_ref
 from ..parallel.tp import TPContext
+from .linear import Linear, bare
 from .registry import ModelSpec
 
 
@@ -74,13 +76,13 @@ class Qwen3Attention(nn.Module):
         qs_full = spec.num_heads * spec.head_dim
         kv_full = spec.num_kv_heads * spec.head_dim
         # merged qkv projection, column-parallel per q/k/v section
-        self.qkv_proj = nn.Linear(h, self.q_size + 2 * self.kv_size, bias=False,
+        self.qkv_proj = Linear(h, self.q_size + 2 * self.kv_size, bias=False,
                                   dtype=dtype)
         _mark_shard(self.qkv_proj.weight, (qs_full + 2 * kv_full, h), 0, tp,
                     row_sections=[(0, qs_full), (qs_full, kv_full),
                                   (qs_full + kv_full, kv_full)])
         # output projection, row-parallel (one all-reduce per attention block)
-        self.o_proj = nn.Linear(self.q_size, h, bias=False, dtype=dtype)
+        self.o_proj = Linear(self.q_size, h, bias=False, dtype=dtype)
         _mark_shard(self.o_proj.weight, (h, qs_full), 1, tp)
         self.qk_norm = spec.qk_norm
         if spec.qk_norm:
@@ -115,14 +117,18 @@ class Qwen3MLP(nn.Module):
         self.tp = tp
         assert intermediate % tp.size == 0
         inter_l = intermediate // tp.size
-        self.gate_up_proj = nn.Linear(hidden, 2 * inter_l, bias=False, dtype=dtype)
+        self.gate_up_proj = Linear(hidden, 2 * inter_l, bias=False, dtype=dtype)
         _mark_shard(self.gate_up_proj.weight, (2 * intermediate, hidden), 0, tp,
                     row_sections=[(0, intermediate), (intermediate, intermediate)])
-        self.down_proj = nn.Linear(inter_l, hidden, bias=False, dtype=dtype)
+        self.down_proj = Linear(inter_l, hidden, bias=False, dtype=dtype)
         _mark_shard(self.down_proj.weight, (hidden, intermediate), 1, tp)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.tp.all_reduce(self.down_proj(ops.silu_mul(self.gate_up_proj(x))))
+        if bare(self.gate_up_proj):
+            act = ops.linear_silu_mul(x, self.gate_up_proj.weight)
+        else:
+            act = ops.silu_mul(self.gate_up_proj(x))
+        return self.tp.all_reduce(self.down_proj(act))
 
 
 class Qwen3MoE(nn.Module):
@@ -148,7 +154,7 @@ class Qwen3MoE(nn.Module):
         self.num_experts = spec.num_experts
         self.top_k = spec.experts_per_token
         h, m = spec.hidden_size, spec.moe_intermediate_size
-        self.router = nn.Linear(h, spec.num_experts, bias=False, dtype=dtype)
+        self.router = Linear(h, spec.num_experts, bias=False, dtype=dtype)
         # weights are [E, N, K] K-contiguous — per-expert torch-Linear
         # layout: direct MFMA K-fragments in the grouped kernel AND direct
         # per-expert copies from HF checkpoints (experts.N.gate_proj etc.)
@@ -526,7 +532,7 @@ class Qwen3Model(nn.Module):
             if spec.tie_embeddings:
                 self.lm_head = None
             else:
-                self.lm_head = nn.Linear(spec.hidden_size, spec.vocab_size,
+                self.lm_head = Linear(spec.hidden_size, spec.vocab_size,
                                          bias=False, dtype=dtype)
         cos_sin = torch_ref.rope_cos_sin(max_len, spec.head_dim, spec.rope_theta)
         self.register_buffer("cos_sin", cos_sin, persistent=False)
@@ -544,7 +550,7 @@ class Qwen3Model(nn.Module):
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         if self.lm_head is not None:
             return self.lm_head(hidden)
-        return F.linear(hidden, self.embed_tokens.weight)
+        return ops.linear(hidden, self.embed_tokens.weight)
 
     @torch.no_grad()
     def init_random_weights(self, seed: int = 0) -> None:

@@ -32,6 +32,7 @@ from .hybrid_spec import (HybridLayerSpec, HybridSpec, LatentAttnMixerSpec,
                           MLSTMMixerSpec, TiedAttnMixerSpec)
 from .layers import (MLSTM, LatentAttention, SectionedLinear,
                      TiedWindowAttention, _pad)
+from .linear import Linear
 
 
 class SandwichBlock(nn.Module):
@@ -57,7 +58,7 @@ class SandwichBlock(nn.Module):
         self.in_proj = SectionedLinear(W, self.mixer.in_sections(""), dtype)
         k = _pad(self.mixer.out_width)
         self.out_padded = k != self.mixer.out_width
-        self.out_proj = nn.Linear(k, W, bias=False, dtype=dtype)
+        self.out_proj = Linear(k, W, bias=False, dtype=dtype)
         f32 = torch.float32
         self.norm1 = nn.Parameter(torch.ones(W, dtype=f32))
         self.norm1b = nn.Parameter(torch.ones(W, dtype=f32))
@@ -66,8 +67,8 @@ class SandwichBlock(nn.Module):
         if layer.ff:
             self.norm2 = nn.Parameter(torch.ones(W, dtype=f32))
             self.norm2b = nn.Parameter(torch.ones(W, dtype=f32))
-            self.ff_up = nn.Linear(W, layer.ff, bias=False, dtype=dtype)
-            self.ff_down = nn.Linear(layer.ff, W, bias=False, dtype=dtype)
+            self.ff_up = Linear(W, layer.ff, bias=False, dtype=dtype)
+            self.ff_down = Linear(layer.ff, W, bias=False, dtype=dtype)
             self.ff_coef = nn.Parameter(torch.zeros(4, dtype=f32))
 
     def checkpoint_targets(self, prefix: str) -> Dict[str, tuple]:
@@ -150,7 +151,7 @@ class RuludraModel(nn.Module):
             [SandwichBlock(spec, layer, i, dtype)
              for i, layer in enumerate(spec.layers)])
         self.final_norm = nn.Parameter(torch.ones(W, dtype=torch.float32))
-        self.lm_head = nn.Linear(W, spec.vocab_size, bias=False, dtype=dtype)
+        self.lm_head = Linear(W, spec.vocab_size, bias=False, dtype=dtype)
         self.act_dtype = dtype
         # debugging aid: when set to a list, every layer's outgoing stream
         # (the next layer's input, fp32) is appended to it

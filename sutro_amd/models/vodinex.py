@@ -31,6 +31,7 @@ from ..parallel.tp import TPContext
 from .hybrid_spec import (AttnMixerSpec, DeltaMixerSpec, HybridLayerSpec,
                           HybridSpec, ParallelMixerSpec)
 from .layers import GatedDeltaRule, LocalAttention, SectionedLinear, _pad
+from .linear import Linear
 
 
 class HybridBlock(nn.Module):
@@ -69,14 +70,14 @@ class HybridBlock(nn.Module):
                               for _, mod, _, _ in mixers)
         has_bias = any(isinstance(mod, LocalAttention) and mod.spec.bias
                        for _, mod, _, _ in mixers)
-        self.out_proj = nn.Linear(k_total, W, bias=has_bias, dtype=dtype)
+        self.out_proj = Linear(k_total, W, bias=has_bias, dtype=dtype)
         self.norm1 = nn.Parameter(torch.ones((), dtype=torch.float32))
         self.ff = layer.ff
         if layer.ff:
             self.ff_in = SectionedLinear(
                 W, [("gate", layer.ff, False), ("up", layer.ff, False),
                     ("rg", W, True)], dtype)
-            self.ff_out = nn.Linear(layer.ff, W, bias=False, dtype=dtype)
+            self.ff_out = Linear(layer.ff, W, bias=False, dtype=dtype)
             self.norm2 = nn.Parameter(torch.ones((), dtype=torch.float32))
 
     # ---- cache layout ----
@@ -176,7 +177,7 @@ class VodinexModel(nn.Module):
             [HybridBlock(spec, layer, i, dtype)
              for i, layer in enumerate(spec.layers)])
         self.final_norm = nn.Parameter(torch.ones((), dtype=torch.float32))
-        self.lm_head = nn.Linear(spec.hidden_size, spec.vocab_size, bias=False,
+        self.lm_head = Linear(spec.hidden_size, spec.vocab_size, bias=False,
                                  dtype=dtype)
         self.act_dtype = dtype
         # debugging aid: when set to a list, the fp32 residual stream after

@@ -30,12 +30,14 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import ops
 from ..engine.batch import ForwardBatch
 from ..engine.kv_cache import PagedKVCache
 from ..ops import hybrid as hops
 from ..parallel.tp import TPContext
 from .hybrid_spec import AttnMixerSpec, HybridLayerSpec, HybridSpec
 from .layers import LocalAttention, RoutedExperts, SectionedLinear, _pad
+from .linear import Linear
 
 
 class DynamicTanh(nn.Module):
@@ -76,7 +78,7 @@ class ParallelBlock(nn.Module):
         self.in_proj = SectionedLinear(W, self.mixer.in_sections(""), dtype)
         k = _pad(self.mixer.out_width)
         self.out_padded = k != self.mixer.out_width
-        self.out_proj = nn.Linear(k, W, bias=False, dtype=dtype)
+        self.out_proj = Linear(k, W, bias=False, dtype=dtype)
         self.ls1 = nn.Parameter(torch.ones(W, dtype=torch.float32))
         self.experts: Optional[RoutedExperts] = None
         if layer.moe is not None:
@@ -199,7 +201,7 @@ class VukotarModel(nn.Module):
 
     @torch.no_grad()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        logits = F.linear(hidden, self.embed_tokens.weight)
+        logits = ops.linear(hidden, self.embed_tokens.weight)
         if self.spec.logit_softcap:
             return hops.softcap(logits, self.spec.logit_softcap)
         return logits.float()

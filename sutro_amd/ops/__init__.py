@@ -12,6 +12,7 @@ import os
 from typing import Optional
 
 import torch
+import torch.nn.functional as F
 
 from . import torch_ref
 
@@ -167,6 +168,54 @@ def sampler_fused(logits, temps, top_ps, top_ks, u, packed_mask, vocab_limit,
     GPU-only: logits must be CUDA; raises if the extension is missing."""
     _require_hip().sampler_fused(logits, temps, top_ps, top_ks, u,
                                  packed_mask, vocab_limit, out_tok, out_lp)
+
+
+def _few_rows(x, w, gated: bool = False) -> bool:
+    """Whether csrc/gemm_skinny.hip is the faster one for x [M, K] w^T. The
+    library takes 11 us or more for any product; us by it and by the kernel,
+    weights from memory:
+      rows of w x K    M = 1          3             16            32
+      2048 x 2048      10.9 /  4.8    11.0 /  5.3   11.0 /  6.5   11.2 /  8.7
+      3072 x 2048      11.3 /  5.1    11.3 /  5.5   11.2 /  6.7   11.5 /  8.9
+      2048 x 3072      12.1 /  5.2    12.1 /  7.0   12.1 /  9.3   10.2 / 13.8
+      4096 x 4096      15.4 /  7.7    15.5 /  9.6   15.5 / 12.5   13.1 / 17.4
+      2048 x 8192      12.7 /  8.1    12.6 / 15.5   13.0 / 22.0
+      6144 x 4096      15.6 / 10.7    14.6 / 15.8   14.2 / 22.3
+      32768 x 4096     61.5 / 48.8    61.7 / 65.6   62.0 / 70.5
+    and with silu_mul behind it 16384 x 2048: 19.6 / 14.0 for one row."""
+    if x.dim() != 2 or not 1 <= x.shape[0] <= 32 or not _use_hip(x):
+        return False
+    M, K = x.shape
+    rows = w.shape[0]
+    fits = (M <= 2 or (M <= 16 and K <= 4096 and rows * K <= 1 << 24)
+            or (K <= 2048 and rows * K <= 1 << 23))
+    return (fits and type(x) is torch.Tensor and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and w.device == x.device
+            and w.dim() == 2 and w.shape[1] == K and K % 32 == 0 and K > 0
+            and rows % (8 if gated else 4) == 0 and rows > 0
+            and w.is_contiguous() and x.stride(1) == 1
+            and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
+def linear(x, w, bias=None):
+    """x w^T (+ bias): the library's product, or over few rows (decode steps)
+    csrc/gemm_skinny.hip."""
+    if _few_rows(x, w) and (bias is None or (
+            bias.dtype == torch.bfloat16 and bias.device == x.device
+            and bias.shape == w.shape[:1] and bias.is_contiguous()
+            and not (torch.is_grad_enabled() and bias.requires_grad))):
+        return _require_hip().linear_skinny(x, w, bias, False)
+    return F.linear(x, w, bias)
+
+
+def linear_silu_mul(x, w):
+    """silu_mul(x w^T), w the gate's rows and then the up's."""
+    if _few_rows(x, w, gated=True):
+        return _require_hip().linear_skinny(x, w, None, True)
+    return silu_mul(F.linear(x, w))
 
 
 def expert_tile(n_rows: int, experts: int, inner: int, width: int,
