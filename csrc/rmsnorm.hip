@@ -1,74 +1,78 @@
 // RMSNorm + fused residual-add RMSNorm, bf16 I/O, fp32 accumulation.
 // Memory-bound: vectorized u16x8 loads (G13: scalar bf16 loads cost ~2x).
 // Two shapes:
-//  - wide rows (hidden_size 1k..16k): one 256-thread block per row, row kept
-//    in registers between the sum-of-squares pass and the normalize pass.
+//  - wide rows (hidden_size 1k..16k): one or four waves per row, row kept in
+//    registers between the sum-of-squares pass and the normalize pass.
 //  - small rows (head_dim 64/128, q/k norm): one wave per row.
 #include "common.h"
 
 // ---------------- wide rows ----------------
 
-template <bool FUSED_ADD>
-__global__ void rmsnorm_wide_kernel(u16* __restrict__ out,       // [rows, C]
-                                    u16* __restrict__ residual,  // [rows, C] or null
-                                    const u16* __restrict__ in,  // [rows, C]
-                                    const u16* __restrict__ w,   // [C]
-                                    float eps, int rows, int C) {
-  const int tid = threadIdx.x;
-  const int nthreads = blockDim.x;
-  const int vec_per_row = C / 8;
-  // up to 8 chunks of 8 -> hidden up to 8*8*256 = 16384
-  float xf[8][8];
-
-  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const u16* rin = in + (long)row * C;
-    u16* rout = out + (long)row * C;
-    float ssq = 0.f;
-    int nchunk = 0;
-    for (int v = tid; v < vec_per_row; v += nthreads, ++nchunk) {
-      u16x8 x = *(const u16x8*)(rin + v * 8);
-      if (FUSED_ADD) {
-        u16x8 r = *(const u16x8*)(residual + (long)row * C + v * 8);
+// WAVES waves hold a row in registers, NV pieces of 8 a lane. Bound by memory.
+// Where rows are many, one wave a row: no barrier, no LDS, and a row's loads
+// all in flight at once. With a workgroup a row half of it had nothing to do at
+// 1024 columns: 24,000 such rows with the residual 59 -> 32 us (6.2 TB/s, some of
+// it from the caches). Few rows take four waves each, for the latency.
+template <bool FUSED_ADD, int NV, int WAVES>
+__global__ void __launch_bounds__(256)
+rmsnorm_wide_kernel(u16* __restrict__ out,       // [rows, C]
+                    u16* __restrict__ residual,  // [rows, C] or null
+                    const u16* __restrict__ in,  // [rows, C]
+                    const u16* __restrict__ w,   // [C]
+                    float eps, long rows, int C) {
+  constexpr int LANES = WAVES * (int)WAVE;
+  const int l = threadIdx.x % LANES;
+  const long row = (long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+  if (WAVES == 1 && row >= rows) return;
+  const int pieces = C / 8;
+  const long base = row * C;
+  u16x8 x[NV], r[NV];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float s = bf2f(x[j]) + bf2f(r[j]);
-          xf[nchunk][j] = s;
-          ssq += s * s;
-        }
-        // write the new residual back (residual += x)
+  for (int i = 0; i < NV; ++i) {
+    const int v = l + i * LANES;
+    if (v < pieces) {
+      x[i] = *(const u16x8*)(in + base + v * 8);
+      if (FUSED_ADD) r[i] = *(const u16x8*)(residual + base + v * 8);
+    }
+  }
+  float xf[NV][8], ssq = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = l + i * LANES;
+    if (v < pieces) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        xf[i][j] = bf2f(x[i][j]) + (FUSED_ADD ? bf2f(r[i][j]) : 0.f);
+        ssq += xf[i][j] * xf[i][j];
+      }
+      if (FUSED_ADD) {   // residual += x
         u16x8 nr;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) nr[j] = f2bf(xf[nchunk][j]);
-        *(u16x8*)(residual + (long)row * C + v * 8) = nr;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float f = bf2f(x[j]);
-          xf[nchunk][j] = f;
-          ssq += f * f;
-        }
+        for (int j = 0; j < 8; ++j) nr[j] = f2bf(xf[i][j]);
+        *(u16x8*)(residual + base + v * 8) = nr;
       }
     }
-    // block reduction
-    ssq = wave_sum_f32(ssq);
-    __shared__ float red[16];
-    const int wid = tid / WAVE, nw = nthreads / WAVE;
-    if ((tid & (WAVE - 1)) == 0) red[wid] = ssq;
+  }
+  ssq = wave_sum_f32(ssq);
+  if (WAVES > 1) {
+    __shared__ float red[WAVES];
+    if ((l & (WAVE - 1)) == 0) red[l / WAVE] = ssq;
     __syncthreads();
-    float total = 0.f;
-#pragma unroll 4
-    for (int i = 0; i < nw; ++i) total += red[i];
-    float inv = rsqrtf(total / (float)C + eps);
-    nchunk = 0;
-    for (int v = tid; v < vec_per_row; v += nthreads, ++nchunk) {
-      u16x8 wv = *(const u16x8*)(w + v * 8);
+    ssq = red[0];
+#pragma unroll
+    for (int i = 1; i < WAVES; ++i) ssq += red[i];
+  }
+  const float inv = rsqrtf(ssq / (float)C + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int v = l + i * LANES;
+    if (v < pieces) {
+      const u16x8 wv = *(const u16x8*)(w + v * 8);
       u16x8 o;
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        o[j] = f2bf(xf[nchunk][j] * inv * bf2f(wv[j]));
-      *(u16x8*)(rout + v * 8) = o;
+      for (int j = 0; j < 8; ++j) o[j] = f2bf(xf[i][j] * inv * bf2f(wv[j]));
+      *(u16x8*)(out + base + v * 8) = o;
     }
-    __syncthreads();  // red[] reuse across grid-stride rows
   }
 }
 
@@ -98,6 +102,25 @@ __global__ void rmsnorm_small_kernel(u16* __restrict__ out,
 
 // ---------------- launchers ----------------
 
+template <bool FUSED_ADD>
+static void wide_launch(u16* out, u16* residual, const u16* in, const u16* w,
+                        float eps, long rows, int C, hipStream_t s) {
+  if (rows == 0) return;
+#define LAUNCH_WIDE(NV, WAVES)                                              \
+  hipLaunchKernelGGL((rmsnorm_wide_kernel<FUSED_ADD, NV, WAVES>),           \
+                     dim3((unsigned)((rows * WAVES + 3) / 4)), dim3(256), 0, \
+                     s, out, residual, in, w, eps, rows, C)
+  if (rows >= 2048 && C <= 4096) {   // eight waves on every CU
+    if (C <= 1024) LAUNCH_WIDE(2, 1);
+    else if (C <= 2048) LAUNCH_WIDE(4, 1);
+    else LAUNCH_WIDE(8, 1);
+  } else if (C <= 2048) LAUNCH_WIDE(1, 4);
+  else if (C <= 4096) LAUNCH_WIDE(2, 4);
+  else if (C <= 8192) LAUNCH_WIDE(4, 4);
+  else LAUNCH_WIDE(8, 4);
+#undef LAUNCH_WIDE
+}
+
 extern "C" void sutro_rmsnorm(void* out, const void* in, const void* w,
                               float eps, long rows, int C, hipStream_t s) {
   if (C % (int)WAVE == 0 && C <= 256 && C / (int)WAVE <= 4) {
@@ -108,17 +131,13 @@ extern "C" void sutro_rmsnorm(void* out, const void* in, const void* w,
                        (const u16*)in, (const u16*)w, eps, rows, C);
     return;
   }
-  int grid = rows < 2048 ? (int)rows : 2048;
-  hipLaunchKernelGGL((rmsnorm_wide_kernel<false>), dim3(grid), dim3(256), 0, s,
-                     (u16*)out, (u16*)nullptr, (const u16*)in, (const u16*)w,
-                     eps, (int)rows, C);
+  wide_launch<false>((u16*)out, nullptr, (const u16*)in, (const u16*)w, eps,
+                     rows, C, s);
 }
 
 extern "C" void sutro_fused_add_rmsnorm(void* x, void* residual, const void* w,
                                         float eps, long rows, int C,
                                         hipStream_t s) {
-  int grid = rows < 2048 ? (int)rows : 2048;
-  hipLaunchKernelGGL((rmsnorm_wide_kernel<true>), dim3(grid), dim3(256), 0, s,
-                     (u16*)x, (u16*)residual, (const u16*)x, (const u16*)w, eps,
-                     (int)rows, C);
+  wide_launch<true>((u16*)x, (u16*)residual, (const u16*)x, (const u16*)w, eps,
+                    rows, C, s);
 }
