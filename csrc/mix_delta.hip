@@ -519,6 +519,154 @@ __global__ void delta_out_kernel(A* __restrict__ out, long ldo, int out_off,
   }
 }
 
+// ---- low-rank gates on the matrix cores ----
+// bf16 projections of rank up to 32 and heads of whole tiles: W2 x is a product
+// of [16 channels x 32] by [32 x 16 tokens] tiles. W2 is fp32: it is split into
+// three bf16 terms (24 bits: exact), held as fragments in registers across the
+// wave's tokens, and the three products are summed in fp32 from the smallest
+// term up, so that nothing is rounded that the FMA chain did not round. A lane
+// ends with four neighbouring channels of one token (16-byte loads and stores).
+// The chain spent 64 instructions an output on readlane and FMA; 32,768 tokens
+// of 16 heads x 128 channels, rank 32: gates 516 -> 227 us
+// (what is left is exp and log1p), read-out 442 -> 140 us (2.9 TB/s).
+#define LR_TOK 128   // tokens per wave
+
+__device__ __forceinline__ f32x4 lr_mfma(s16x8 a, s16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// the fragments of 16 channels: this lane's is channel `col`, k = k0 .. k0 + 7
+__device__ __forceinline__ void lr_split(s16x8 (&w)[3],
+                                         const float* __restrict__ w2t,
+                                         long stride, long col, int k0,
+                                         int rank) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    float v = k0 + j < rank ? w2t[(long)(k0 + j) * stride + col] : 0.f;
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const u16 b = f2bf(v);
+      w[n][j] = (short)b;
+      const float f = bf2f(b);
+      v = fabsf(f) <= 3.4e38f ? v - f : 0.f;   // nothing below an infinity
+    }
+  }
+}
+
+// eight inputs of a token; infinities become the largest numbers, because a
+// term of W2 that is zero must not make them NaN
+__device__ __forceinline__ s16x8 lr_input(const u16* p, bool in) {
+  s16x8 x = (s16x8)(short)0;
+  if (in) x = *(const s16x8*)p;
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if ((x[j] & 0x7fff) == 0x7f80) x[j] = x[j] - 1;
+  return x;
+}
+
+__device__ __forceinline__ f32x4 lr_dot(const s16x8 (&w)[3], s16x8 x,
+                                        f32x4 acc) {
+#pragma unroll
+  for (int n = 2; n >= 0; --n) acc = lr_mfma(w[n], x, acc);
+  return acc;
+}
+
+// grid (token groups, H, channel groups of 64); block of four waves, each with
+// its own LR_TOK tokens
+__global__ void __launch_bounds__(WPB * WAVE) delta_gates_mfma_kernel(
+    float* __restrict__ decay, float* __restrict__ beta,
+    const u16* __restrict__ proj, long ld, int b_off, int a1_off,
+    const float* __restrict__ a2t, int rank, const float* __restrict__ dt_bias,
+    const float* __restrict__ a_log, long T, int H, int dk) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int h = blockIdx.y, c0 = blockIdx.z * 64;
+  const int lr = lane & 15, g = lane >> 4;
+  const long t_end0 = ((long)blockIdx.x * WPB + wid) * LR_TOK;
+  if (t_end0 >= T) return;
+  const long t_end = t_end0 + LR_TOK < T ? t_end0 + LR_TOK : T;
+  const float rate = expf(a_log[h]);
+  s16x8 w[4][3];
+  f32x4 bias[4];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    lr_split(w[n], a2t, (long)H * dk, (long)h * dk + c0 + n * 16 + lr, g * 8,
+             rank);
+    bias[n] = *(const f32x4*)(dt_bias + (long)h * dk + c0 + n * 16 + g * 4);
+  }
+  for (long t0 = t_end0; t0 < t_end; t0 += 16) {
+    const long t = t0 + lr < t_end ? t0 + lr : t_end - 1;
+    const s16x8 x = lr_input(proj + t * ld + a1_off + g * 8, g * 8 < rank);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const f32x4 a = lr_dot(w[n], x, bias[n]);
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = expf(-rate * softplus_f(a[e]));
+      if (t0 + lr < t_end)
+        *(f32x4*)(decay + (t * H + h) * (long)dk + c0 + n * 16 + g * 4) = y;
+    }
+    if (blockIdx.z == 0 && g == 0 && t0 + lr < t_end)
+      beta[t * H + h] = sigmoid_f(bf2f(proj[t * ld + b_off + h]));
+  }
+}
+
+// grid (token groups, H); a wave owns all dv = 16 NT channels of a head
+template <int NT>
+__global__ void __launch_bounds__(WPB * WAVE) delta_out_mfma_kernel(
+    u16* __restrict__ out, long ldo, int out_off, const float* __restrict__ o,
+    const float* __restrict__ norm_w, const u16* __restrict__ proj, long ld,
+    int g1_off, const float* __restrict__ g2t, int rank, float eps,
+    float out_scale, long T, int H) {
+  constexpr int dv = NT * 16;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int h = blockIdx.y;
+  const int lr = lane & 15, g = lane >> 4;
+  const long t_end0 = ((long)blockIdx.x * WPB + wid) * LR_TOK;
+  if (t_end0 >= T) return;
+  const long t_end = t_end0 + LR_TOK < T ? t_end0 + LR_TOK : T;
+  s16x8 w[NT][3];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+    lr_split(w[n], g2t, (long)H * dv, (long)h * dv + n * 16 + lr, g * 8, rank);
+  for (long t0 = t_end0; t0 < t_end; t0 += 16) {
+    const long t = t0 + lr < t_end ? t0 + lr : t_end - 1;
+    const float* orow = o + (t * H + h) * (long)dv + g * 4;
+    f32x4 v[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) v[n] = *(const f32x4*)(orow + n * 16);
+    const s16x8 x = lr_input(proj + t * ld + g1_off + g * 8, g * 8 < rank);
+    float ssq = 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ssq += v[n][e] * v[n][e];
+    ssq += __shfl_xor(ssq, 16, 64);
+    ssq += __shfl_xor(ssq, 32, 64);
+    const float inv = out_scale / sqrtf(ssq / (float)dv + eps);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const f32x4 a = lr_dot(w[n], x, (f32x4)(0.f));
+      const f32x4 wn = *(const f32x4*)(norm_w + n * 16 + g * 4);
+      u16x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = f2bf(v[n][e] * inv * wn[e] * sigmoid_f(a[e]));
+      if (t0 + lr < t_end)
+        *(u16x4*)(out + t * ldo + out_off + (long)h * dv + n * 16 + g * 4) = y;
+    }
+  }
+}
+
+// 16-byte pieces of the rank inputs, whole tiles of channels
+static bool lr_fits(const void* proj, long ld, int off, int rank,
+                    const void* w2, const void* vec) {
+  return rank > 0 && rank <= 32 && rank % 8 == 0 && ld % 8 == 0 &&
+         off % 8 == 0 && (size_t)proj % 16 == 0 && (size_t)vec % 16 == 0 &&
+         (size_t)w2 % 4 == 0;
+}
+
 extern "C" void mix_delta_prep(
     float* qn, float* kn, float* vv, float* decay, float* beta,
     const void* proj, long ld, int q_off, int k_off, int v_off, int b_off,
@@ -537,6 +685,14 @@ extern "C" void mix_delta_prep(
   const int grid = (int)((units + WPB - 1) / WPB);
   if (grid == 0) return;
   const dim3 ggrid((unsigned)((T + WPB * GT - 1) / (WPB * GT)), (unsigned)H);
+  const bool lr = !f32 && a2 && dk % 64 == 0 && (size_t)decay % 16 == 0 &&
+                  lr_fits(proj, ld, a1_off, rank, a2, dt_bias);
+  if (lr)
+    hipLaunchKernelGGL(delta_gates_mfma_kernel,
+                       dim3((unsigned)((T + WPB * LR_TOK - 1) / (WPB * LR_TOK)),
+                            (unsigned)H, (unsigned)(dk / 64)),
+                       dim3(WPB * WAVE), 0, s, decay, beta, (const u16*)proj,
+                       ld, b_off, a1_off, a2, rank, dt_bias, a_log, T, H, dk);
   const int Cq = G * dk, C = 2 * Cq + H * dv;
   const long su = (long)S * C;
   const int sgrid = (int)((su + 255) / 256);
@@ -560,7 +716,7 @@ extern "C" void mix_delta_prep(
     else if (GS == 16) LAUNCH_DV(16);
     else LAUNCH_DV(32);
 #undef LAUNCH_DV
-    if (a2)
+    if (a2 && !lr)
     hipLaunchKernelGGL(delta_gates_kernel<u16>, ggrid, dim3(WPB * WAVE), 0, s,
                        decay, beta, (const u16*)proj, ld, b_off, a1_off, a2,
                        rank, dt_bias, a_log, T, H, dk);
@@ -575,7 +731,7 @@ extern "C" void mix_delta_prep(
                        0, s, qn, kn, vv, hg, (const float*)proj, ld, q_off, k_off,
                        v_off, conv_w, taps, conv_state, state_slots, qlocs,
                        seq_lens, token_seq, T, H, G, dk, dv);
-    if (a2)
+    if (a2 && !lr)
     hipLaunchKernelGGL(delta_gates_kernel<float>, ggrid, dim3(WPB * WAVE), 0, s,
                        decay, beta, (const float*)proj, ld, b_off, a1_off, a2,
                        rank, dt_bias, a_log, T, H, dk);
@@ -589,7 +745,7 @@ extern "C" void mix_delta_prep(
                        s, qn, kn, vv, hg, (const u16*)proj, ld, q_off, k_off, v_off,
                        conv_w, taps, conv_state, state_slots, qlocs, seq_lens,
                        token_seq, T, H, G, dk, dv);
-    if (a2)
+    if (a2 && !lr)
     hipLaunchKernelGGL(delta_gates_kernel<u16>, ggrid, dim3(WPB * WAVE), 0, s,
                        decay, beta, (const u16*)proj, ld, b_off, a1_off, a2,
                        rank, dt_bias, a_log, T, H, dk);
@@ -653,7 +809,18 @@ extern "C" void mix_delta_out(void* out, long ldo, int out_off, const float* o,
                               hipStream_t s) {
   if (T == 0) return;
   const dim3 grid((unsigned)((T + WPB * GT - 1) / (WPB * GT)), (unsigned)H);
-  if (f32)
+  if (!f32 && (dv == 64 || dv == 128) && ldo % 4 == 0 && out_off % 4 == 0 &&
+      (size_t)out % 8 == 0 && (size_t)o % 16 == 0 &&
+      lr_fits(proj, ld, g1_off, rank, g2, norm_w)) {
+    const auto fn = dv == 128 ? delta_out_mfma_kernel<8>
+                              : delta_out_mfma_kernel<4>;
+    hipLaunchKernelGGL(fn,
+                       dim3((unsigned)((T + WPB * LR_TOK - 1) / (WPB * LR_TOK)),
+                            (unsigned)H),
+                       dim3(WPB * WAVE), 0, s, (u16*)out, ldo, out_off, o,
+                       norm_w, (const u16*)proj, ld, g1_off, g2, rank, eps,
+                       out_scale, T, H);
+  } else if (f32)
     hipLaunchKernelGGL(delta_out_kernel<float>, grid, dim3(WPB * WAVE),
                        0, s, (float*)out, ldo, out_off, o, norm_w,
                        (const float*)proj, ld, g1_off, g2, rank, eps,
