@@ -304,8 +304,11 @@ gg_wide_kernel(u16* __restrict__ out, const u16* __restrict__ a,
   extern __shared__ __attribute__((aligned(16))) char gw_smem[];
 
   // copies: 1 KB (8 rows of 128 bytes) an instruction, pieces wave*4 + j of
-  // either operand; 16-byte chunks are XOR-swizzled by the row
-  const int pr = lane >> 3, pc = ((lane & 7) ^ pr) * 8;
+  // either operand; 16-byte chunks are XOR-swizzled by bits 1 to 3 of the row, so
+  // that the 16 rows read in a cycle cover all 64 banks (by bits 0 to 2, eight of
+  // them did: down product at 4096 rows an expert 1089 -> 1058 us, the gated one
+  // 2155 -> 2125)
+  const int pr = lane >> 3;
   const u16* pa[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -317,12 +320,13 @@ gg_wide_kernel(u16* __restrict__ out, const u16* __restrict__ a,
     } else {
       row = seg + r;
     }
-    pa[j] = a + row * K + pc;
+    pa[j] = a + row * K + ((lane & 7) ^ (((j & 1) * 8 + pr) >> 1)) * 8;
   }
   const int br = wave * 32;                    // first of this wave's B rows
   const long brow = (GATED && br >= 128) ? n_cols + n0 + br - 128 : n0 + br;
   const u16* pb = w + ((long)e * (GATED ? 2 : 1) * n_cols + brow) * K;
-  const u32 boff = (u32)(pr * K + pc);
+  const u32 boff[2] = {(u32)(pr * K + ((lane & 7) ^ (pr >> 1)) * 8),
+                       (u32)(pr * K + ((lane & 7) ^ ((8 + pr) >> 1)) * 8)};
   auto stage = [&](int buf, long k) {
     char* dst = gw_smem + buf * 2 * TILE + wave * 4096;
 #pragma unroll
@@ -330,14 +334,14 @@ gg_wide_kernel(u16* __restrict__ out, const u16* __restrict__ a,
       glds16g((const u32*)(pa[j] + k), (u32*)(dst + j * 1024));
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      glds16g((const u32*)(pb + k + j * 8 * K + boff),
+      glds16g((const u32*)(pb + k + j * 8 * K + boff[j & 1]),
               (u32*)(dst + TILE + j * 1024));
   };
 
   int kad[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk)
-    kad[kk] = ln * 128 + (((kk * 2 + hi) ^ (ln & 7)) << 4);
+    kad[kk] = ln * 128 + (((kk * 2 + hi) ^ ((ln >> 1) & 7)) << 4);
   const int arow = wm * 128 * 128;
   const int brow0 = (GATED ? wn * 32 : wn * 64) * 128 + TILE;
   const int brow1 = (GATED ? 128 + wn * 32 : wn * 64 + 32) * 128 + TILE;
