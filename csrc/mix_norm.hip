@@ -83,6 +83,68 @@ __global__ void gated_norm_residual_kernel(
   }
 }
 
+// The same for bf16 rows of whole 16-byte pieces, up to 512 NV WAVES columns:
+// WAVES waves hold a row in registers, so that everything is read once, the
+// gate's exponential is taken once and all of a row's loads are in flight
+// together. Many rows take one wave each, few rows four (as rmsnorm does).
+// 32,768 rows of 2048: 268 -> 155 us (5.9 TB/s with what the caches hold).
+template <int NV, int WAVES>
+__global__ void __launch_bounds__(256) gated_norm_residual_vec_kernel(
+    float* __restrict__ x, const u16* __restrict__ y,
+    const u16* __restrict__ proj, long ld, int gate_off,
+    const float* __restrict__ gain, float eps, float mult,
+    u16* __restrict__ h_out, long T, int W) {
+  constexpr int LANES = WAVES * (int)WAVE;
+  const int l = threadIdx.x % LANES;
+  const long row = (long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+  if (WAVES == 1 && row >= T) return;
+  const int pieces = W / 8;
+  const long base = row * W;
+  const u16* gr = proj + row * ld + gate_off;
+  u16x8 yv[NV], gv[NV];
+  f32x4 xv[NV][2];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (l + i * LANES) * 8;
+    if (l + i * LANES < pieces) {
+      yv[i] = *(const u16x8*)(y + base + c);
+      gv[i] = *(const u16x8*)(gr + c);
+      xv[i][0] = *(const f32x4*)(x + base + c);
+      xv[i][1] = *(const f32x4*)(x + base + c + 4);
+    }
+  }
+  float z[NV][8], ssq = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+    if (l + i * LANES < pieces) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        z[i][e] = bf2f(yv[i][e]) * sigmoid_f(bf2f(gv[i][e]));
+        ssq += z[i][e] * z[i][e];
+      }
+    }
+  __shared__ float red[4];
+  if (WAVES > 1) ssq = block_sum_256(ssq, red);
+  else ssq = wave_sum_f32(ssq);
+  const float inv = gain[0] * mult / sqrtf(ssq / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (l + i * LANES) * 8;
+    if (l + i * LANES < pieces) {
+      u16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float nx = xv[i][e >> 2][e & 3] + z[i][e] * inv;
+        xv[i][e >> 2][e & 3] = nx;
+        h[e] = f2bf(nx);
+      }
+      *(f32x4*)(x + base + c) = xv[i][0];
+      *(f32x4*)(x + base + c + 4) = xv[i][1];
+      if (h_out) *(u16x8*)(h_out + base + c) = h;
+    }
+  }
+}
+
 template <typename A>
 __global__ void scalar_rmsnorm_kernel(A* __restrict__ out,
                                       const float* __restrict__ x,
@@ -141,7 +203,19 @@ extern "C" void mix_gated_norm_residual(float* x, const void* y,
                                         float eps, float mult, void* h_out,
                                         long T, int W, int f32,
                                         hipStream_t s) {
-  if (f32)
+  if (!f32 && T > 0 && W <= 8192 && (W | gate_off | (int)(ld & 7)) % 8 == 0 &&
+      ((size_t)x | (size_t)y | (size_t)proj | (size_t)h_out) % 16 == 0) {
+#define LAUNCH_GN(NV, WAVES)                                                  \
+  hipLaunchKernelGGL((gated_norm_residual_vec_kernel<NV, WAVES>),             \
+                     dim3((unsigned)((T * WAVES + 3) / 4)), dim3(256), 0, s,  \
+                     x, (const u16*)y, (const u16*)proj, ld, gate_off, gain,  \
+                     eps, mult, (u16*)h_out, T, W)
+    if (T >= 2048 && W <= 2048) LAUNCH_GN(4, 1);
+    else if (W <= 2048) LAUNCH_GN(1, 4);
+    else if (W <= 4096) LAUNCH_GN(2, 4);
+    else LAUNCH_GN(4, 4);
+#undef LAUNCH_GN
+  } else if (f32)
     hipLaunchKernelGGL(gated_norm_residual_kernel<float>, dim3(row_grid(T)),
                        dim3(256), 0, s, x, (const float*)y, (const float*)proj,
                        ld, gate_off, gain, eps, mult, (float*)h_out, T, W);
