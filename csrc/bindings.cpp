@@ -245,14 +245,14 @@ torch::Tensor mfma16_probe(torch::Tensor a, torch::Tensor b) {
 }
 
 static bool tile_rows_ok(long bm) {
-  return bm == 64 || bm == 128 || bm == 256;
+  return bm == 32 || bm == 64 || bm == 128 || bm == 256;
 }
 
 void grouped_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
                   c10::optional<torch::Tensor> row_tok, torch::Tensor tile_off,
                   torch::Tensor counts, long max_tiles, bool gate_silu,
                   long bm) {
-  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 32, 64, 128 or 256");
   CHECK_CUDA(a); CHECK_CONTIG(a); CHECK_BF16(a);
   CHECK_CUDA(w); CHECK_CONTIG(w); CHECK_BF16(w);
   CHECK_CONTIG(out); CHECK_BF16(out);
@@ -310,7 +310,7 @@ std::vector<torch::Tensor> moe_layout(torch::Tensor logits, long k, long base,
   TORCH_CHECK(k >= 1 && k <= 64 && k <= E && E <= 1024,
               "router: up to 64 of up to 1024 experts");
   TORCH_CHECK(base >= 0 && n_local >= 1 && base + n_local <= E, "local experts");
-  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 32, 64, 128 or 256");
   const long segs = n_local + (n_local < E ? 1 : 0);
   TORCH_CHECK(row_tok.numel() >= T * k + segs * (bm - 1), "row_tok too short");
   TORCH_CHECK(T * k + segs * bm < (1l << 31), "too many rows");

@@ -26,7 +26,7 @@
 // tiles would mostly be padding).
 //
 // Two kernels by the height of the segments' tiles (the caller pads with the
-// height it passes): tiles of 256 rows for prompts, tiles of 64 and 128 rows for
+// height it passes): tiles of 256 rows for prompts, tiles of 32 to 128 rows for
 // fewer rows an expert and for widths the other does not take.
 #include "common.h"
 
@@ -48,6 +48,8 @@ __device__ __forceinline__ u32 gswz(u32 byte) {
 }
 
 // Tile configurations (all reuse the verified gemm_tn staging recipe):
+//   BM=32,  BN=64,  4 waves 2x2  — decode steps: 40 KB of LDS for the gated
+//                                  product, four workgroups a CU (64: three)
 //   BM=64,  BN=64,  4 waves 2x2  — small batches (avg segment < 256 rows):
 //                                  least padding waste
 //   BM=128, BN=128, 8 waves 2x4  — big batches: 4x the MFMA work per
@@ -464,6 +466,13 @@ static void grouped_gemm_launch(void* out, const void* a, const void* w,
     else if (gate_silu == 4) GG_LAUNCH(4, 128, 64, 4, 2)
     else if (gate_silu == 2) GG_LAUNCH(2, 128, 64, 4, 2)
     else GG_LAUNCH(0, 128, 64, 4, 2)
+  }
+  if (bm == 32) {
+    if (gate_silu == 1) GG_LAUNCH(1, 32, 64, 2, 2)
+    else if (gate_silu == 3) GG_LAUNCH(3, 32, 64, 2, 2)
+    else if (gate_silu == 4) GG_LAUNCH(4, 32, 64, 2, 2)
+    else if (gate_silu == 2) GG_LAUNCH(2, 32, 64, 2, 2)
+    else GG_LAUNCH(0, 32, 64, 2, 2)
   }
   if (gate_silu == 1) GG_LAUNCH(1, 64, 64, 2, 2)
   else if (gate_silu == 3) GG_LAUNCH(3, 64, 64, 2, 2)

@@ -888,7 +888,7 @@ void moe_route(torch::Tensor idx, torch::Tensor wts, torch::Tensor logits,
 }
 
 static bool tile_rows_ok(long bm) {
-  return bm == 64 || bm == 128 || bm == 256;
+  return bm == 32 || bm == 64 || bm == 128 || bm == 256;
 }
 
 void moe_dispatch(torch::Tensor row_tok, torch::Tensor tile_off,
@@ -903,7 +903,7 @@ void moe_dispatch(torch::Tensor row_tok, torch::Tensor tile_off,
   CHECK_GPU(padpos); CHECK_I32(padpos); CHECK_CONTIG(padpos);
   TORCH_CHECK(idx.dim() == 2 && padpos.sizes() == idx.sizes(), "pair shapes");
   const long T = idx.size(0), k = idx.size(1), E = counts.numel();
-  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 32, 64, 128 or 256");
   TORCH_CHECK(tile_off.numel() == E + 1 && row_tok.numel() % bm == 0 &&
               row_tok.numel() >= T * k + E * (bm - 1), "segment table sizes");
   TORCH_CHECK((2 * E + 1) * 4 <= 64 * 1024 && T * k < (1L << 31),
@@ -945,7 +945,7 @@ void moe_dispatch_table(torch::Tensor row_tok, torch::Tensor tile_off,
   const long T = ids.size(0), k = table.size(1), E = counts.numel();
   TORCH_CHECK(padpos.dim() == 2 && padpos.size(0) == T && padpos.size(1) == k,
               "pair shapes");
-  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 32, 64, 128 or 256");
   TORCH_CHECK(tile_off.numel() == E + 1 && row_tok.numel() % bm == 0 &&
               row_tok.numel() >= T * k + E * (bm - 1), "segment table sizes");
   TORCH_CHECK((2 * E + 1) * 4 <= 64 * 1024 && T * k < (1L << 31),
@@ -977,7 +977,7 @@ void expert_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
   const long E = w.size(0), K = w.size(2);
   const long N = glu ? w.size(1) / 2 : w.size(1);
   const long n_rows = out.size(0);
-  TORCH_CHECK(tile_rows_ok(bm), "bm must be 64, 128 or 256");
+  TORCH_CHECK(tile_rows_ok(bm), "bm must be 32, 64, 128 or 256");
   TORCH_CHECK(act >= 0 && act <= 3, "activation: 0 (none), 1 (silu gate), 2 "
               "(relu squared) or 3 (clamped unit)");
   TORCH_CHECK(!glu || (w.size(1) % 2 == 0 && (act == 1 || limit > 0)),
@@ -1007,6 +1007,7 @@ void expert_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
   // weighted rows: the matrix-core kernel has the silu unit only
   const bool mfma = kind == 0 && K % 64 == 0 && N % 64 == 0 &&
                     (!rw || act == 1);
+  TORCH_CHECK(bm != 32 || mfma, "tiles of 32 rows: matrix-core kernel only");
   TORCH_CHECK(bm != 256 || !mfma || N % (glu ? 128 : 256) == 0,
               "tiles of 256 rows need a multiple of 256 columns (gated: 128)");
   if (mfma) {

@@ -225,8 +225,17 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
     multiples of 64), by the rows an expert gets on average. Taller tiles do
     more work per byte but pad more; both products together, at 32 experts of
     2048 x 2048: at 96 rows 290 / 209 / 243 us on tiles of 64 / 128 / 256, at
-    187 rows 561 / 387 / 243, at 375 rows 1074 / 671 / 422."""
+    187 rows 561 / 387 / 243, at 375 rows 1074 / 671 / 422.
+
+    Up to 16 rows, where the weights are all there is to read, tiles of 32: four
+    workgroups of the gated product fit a CU instead of three. They are taken
+    unless their number then fills the rounds worse: 1024 workgroups (2048 wide)
+    222 -> 200 us, 1536 (3072 wide, K 4096) 431 -> 445."""
     avg = n_rows / experts
+    if avg <= 16:
+        blocks = min(experts, n_rows) * (inner // 64)
+        if blocks <= 768 or -(-blocks // 1024) * 4 <= -(-blocks // 768) * 3:
+            return 32
     if avg >= 144 and inner % (128 if gated else 256) == 0 and width % 256 == 0:
         return 256
     return 128 if avg >= 72 else 64

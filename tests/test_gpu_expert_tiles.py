@@ -1,4 +1,4 @@
-"""The expert GEMMs on tiles of 64 and 256 rows against the torch
+"""The expert GEMMs on tiles of 32, 64 and 256 rows against the torch
 reference: empty experts, segments one row short of, at and past a tile, one
 and several steps of k, every unit between the two matrices."""
 
@@ -20,7 +20,7 @@ def _segments(counts, bm):
 
 @pytest.mark.parametrize("K", [64, 320, 1024])   # 64: a single step
 @pytest.mark.parametrize("bm,counts", [
-    (64, [1, 63, 0, 64, 65, 130]), (256, [1, 255, 0, 256, 257, 600])])
+    (32, [1, 31, 0, 32, 33, 70]), (64, [1, 63, 0, 64, 65, 130]), (256, [1, 255, 0, 256, 257, 600])])
 @pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE,
                                  hops.ACT_RELU2, hops.ACT_GLU_CLAMPED,
                                  "weighted"])
@@ -67,7 +67,7 @@ def test_tiles(K, bm, counts, act):
 
 
 @pytest.mark.parametrize("n_rows,want", [
-    (1, 64), (575, 64), (576, 128), (1151, 128), (1152, 256), (99999, 256)])
+    (1, 32), (128, 32), (129, 64), (575, 64), (576, 128), (1151, 128), (1152, 256), (99999, 256)])
 def test_tile_rule(n_rows, want):
     from sutro_amd.ops import expert_tile
 
@@ -76,3 +76,5 @@ def test_tile_rule(n_rows, want):
     assert expert_tile(n_rows, 8, 192, 256) <= 128
     assert expert_tile(n_rows, 8, 128, 320) <= 128
     assert expert_tile(n_rows, 8, 128, 256, gated=False) <= 128
+    # 1536 workgroups: two rounds of three a CU, but one and a half of four
+    assert expert_tile(512, 32, 3072, 4096) == 64
