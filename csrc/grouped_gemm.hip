@@ -1,9 +1,9 @@
 // Grouped (per-expert) bf16 GEMM for dropless MoE on MI355X.
 //
 // Exact top-k routing with NO capacity dropping: token assignments are
-// sorted by expert and laid out in per-expert segments padded to the BM=64
-// tile height, so every workgroup tile belongs to exactly one expert and the
-// grid is a STATIC upper bound (ceil(T*k/64) + E tiles) — decode steps stay
+// sorted by expert and laid out in per-expert segments padded to the tile
+// height BM, so every workgroup tile belongs to exactly one expert and the
+// grid is a STATIC upper bound (ceil(T*k/BM) + E tiles) — decode steps stay
 // hipGraph-capturable; tiles past the live padded total exit early by
 // reading the device-side tile-offset table.
 //
@@ -21,9 +21,7 @@
 // expert), so MFMA fragments are 8 consecutive bf16 along K for both
 // operands — same verified recipe as csrc/gemm_tn.hip: BK=64 double-
 // buffered direct global->LDS staging (global_load_lds dwordx4, swizzle
-// mode 2), mfma_f32_16x16x32_bf16, fp32 accumulate. 4 waves as 2(M)x2(N),
-// 64x64 macro-tile (expert segments average T*k/E rows — large gemm_tn
-// tiles would mostly be padding).
+// mode 2), mfma_f32_16x16x32_bf16, fp32 accumulate.
 //
 // Two kernels by the height of the segments' tiles (the caller pads with the
 // height it passes): tiles of 256 rows for prompts, tiles of 32 to 128 rows for
@@ -50,16 +48,12 @@ __device__ __forceinline__ u32 gswz(u32 byte) {
 // Tile configurations (all reuse the verified gemm_tn staging recipe):
 //   BM=32,  BN=64,  4 waves 2x2  — decode steps: 40 KB of LDS for the gated
 //                                  product, four workgroups a CU (64: three)
-//   BM=64,  BN=64,  4 waves 2x2  — small batches (avg segment < 256 rows):
-//                                  least padding waste
-//   BM=128, BN=128, 8 waves 2x4  — big batches: 4x the MFMA work per
-//                                  barrier, B tiles shared across 4 M-rows
-//                                  of waves (measured 3-5x kernel speedup
-//                                  at the b8192 operating point)
-//   BM=128, BN=64,  8 waves 4x2  — big batches whose n_cols % 128 != 0
-//                                  (gpt-oss m=2880)
-// The segment padding (and tile_off table) is computed host-side with the
-// SAME BM the kernel is launched with.
+//   BM=64,  BN=64,  4 waves 2x2  — up to 72 rows an expert
+//   BM=128, BN=128, 8 waves 2x4  — more rows: 4x the MFMA work per barrier, B
+//                                  tiles shared across 4 M-rows of waves
+//   BM=128, BN=64,  8 waves 4x2  — the same where n_cols % 128 != 0
+// The segment padding (and tile_off table) is computed with the SAME BM the
+// kernel is launched with; ops.expert_tile chooses it, with both sides measured.
 
 // Stage a ROWS x 64 bf16 tile (ROWS rows of 128B) with WAVES waves; each
 // wave issues ROWS/(8*WAVES) x 1KB chunks.
