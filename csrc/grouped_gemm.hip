@@ -27,6 +27,7 @@
 // height it passes): tiles of 256 rows for prompts, tiles of 32 to 128 rows for
 // fewer rows an expert and for widths the other does not take.
 #include "common.h"
+#include "lds_limit.h"
 
 typedef s16x8 bf16x8;
 
@@ -432,13 +433,8 @@ static void grouped_gemm_launch(void* out, const void* a, const void* w,
     const dim3 grid(groups * 8 * GW_ROWS * nb);
 #define GG_WIDE(M)                                                          \
   {                                                                         \
-    static bool once = [] {                                                 \
-      (void)hipFuncSetAttribute((const void*)gg_wide_kernel<M>,             \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                4 * 256 * 128);                             \
-      return true;                                                          \
-    }();                                                                    \
-    (void)once;                                                             \
+    static std::atomic<unsigned long long> asked{0};                        \
+    lds_limit((const void*)gg_wide_kernel<M>, 4 * 256 * 128, asked);        \
     hipLaunchKernelGGL(gg_wide_kernel<M>, grid, dim3(512), 4 * 256 * 128,   \
                        stream, GG_ARGS);                                    \
   }

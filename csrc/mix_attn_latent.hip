@@ -32,6 +32,7 @@
 // ds_read_tr16_b64: in a group of 16 lanes lane i addresses 4 consecutive
 // columns (i%4)*4.. of row i/4; it receives column i of those 4 rows.
 #include "mix_common.h"
+#include "lds_limit.h"
 
 #define LT_ROWS 64   // query rows per tile
 #define LT_KEYS 64   // keys per step (two pages)
@@ -458,13 +459,9 @@ extern "C" int mix_latent_attention(
                       3 * LT_ROWS * sizeof(float);
 #define LAUNCH_LT(KK, VV)                                                     \
   do {                                                                        \
-    static bool once = [&] {  /* more LDS than the default limit of a block */ \
-      (void)hipFuncSetAttribute(                                              \
-          (const void*)latent_attention_kernel<KK, VV>,                       \
-          hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);             \
-      return true;                                                            \
-    }();                                                                      \
-    (void)once;                                                               \
+    static std::atomic<unsigned long long> asked{0};                          \
+    lds_limit((const void*)latent_attention_kernel<KK, VV>, (int)smem,        \
+              asked);                                                         \
     hipLaunchKernelGGL((latent_attention_kernel<KK, VV>), grid, dim3(256),    \
                        smem, s, A);                                           \
   } while (0)
