@@ -24,6 +24,8 @@
 //     (i%4)*4.. of row i/4 and receives column i of those 4 rows.
 #pragma once
 
+#include "lds_limit.h"
+
 #define PA_PG 32       // page size
 #define PA_KEYS 64     // keys per prefill step (two pages)
 #define PA_SLACK 8.f   // log2 of the largest weight against a stale maximum
@@ -157,7 +159,7 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 // 32 k prompt (16 heads, 4 kv heads, 128; useful flops) and 250 on prompts of
 // 2 k; this one at 860 and 640 (13.1 -> 5.1 ms, 1.10 -> 0.43 ms), 0.78 instead
 // of 1.61 ms on 7 prompts of 3 k with 32 heads over e4m3 pages, 0.11 instead of
-// 0.22 ms on 160 short ones (24 k tokens). Two workgroups a CU (64 KB of LDS,
+// 0.22 ms on 160 short ones (24 k tokens). Two workgroups a CU (68 KB of LDS,
 // up to 256 registers a lane) are what both limits allow.
 //
 // Entries of the tile map that continue each other (same sequence, 32 rows on)
@@ -229,11 +231,13 @@ paged_prefill_kernel(PagedArgs A) {
   // lower key bounds: of this lane's row, of the workgroup's first row, and of
   // this wave's last row (above which a step needs no mask)
   int lo_row = 0, c_row = 0, kt0 = 0, kf0 = 0, n_kept = 0, lo_last = 0;
+  int lo_first = 0, c_first = 0, w_lo = 0, w_c = 0;  // w: this wave's first row
   if (LOCAL) {
-    int c_first, c_last;
+    int c_last;
     lo_row = pa_lower(A, my_p, c_row);
-    const int lo_first = pa_lower(A, p0, c_first);
+    lo_first = pa_lower(A, p0, c_first);
     lo_last = pa_lower(A, w_end - 1, c_last);
+    w_lo = pa_lower(A, p0 + rb * 32, w_c);
     kt0 = lo_first / PA_KEYS;
     kf0 = c_first / PA_KEYS;
     n_kept = max(min(kt0, (A.keep_first + PA_KEYS - 1) / PA_KEYS) - kf0, 0);
@@ -278,7 +282,22 @@ paged_prefill_kernel(PagedArgs A) {
       st[j] = *(const typename PaRaw<KV8>::type*)(base + off);
     }
   };
-  auto store = [&](char* buf) {
+  // Keys that a row does not see have weight 0, but their values may be infinite
+  // or NaN (behind the context lies what an earlier request left there), which
+  // 0 does not take away: values of keys that no row of the workgroup sees are
+  // stored as zeros, and a wave takes 16 keys that none of its own rows see from
+  // a tile of zeros.
+  const u32 g_kept = max(A.keep_first - c_first, 0);
+  auto store = [&](char* buf, int kv) {
+    const bool edge = kv + PA_KEYS > kv_end || (LOCAL && kv < lo_first);
+    if (edge)
+#pragma unroll
+      for (int j = PER / 4; j < PER / 2; ++j) {
+        const int kp = kv + ((j - PER / 4) * 4 + w) * RPP + st_row;
+        bool any = kp < kv_end;
+        if (LOCAL) any &= (kp >= lo_first) | ((u32)(kp - c_first) < g_kept);
+        if (!any) st[j] = typename PaRaw<KV8>::type(0);
+      }
 #pragma unroll
     for (int j = 0; j < PER / 2; ++j)
       *(u16x8*)(buf + (j * 4 + w) * 1024 + lane * 16) = pa_widen<KV8>(st[j]);
@@ -302,7 +321,10 @@ paged_prefill_kernel(PagedArgs A) {
   pages(step_tile(0));
   load();
   if (steps > 1) pages(step_tile(1));
-  store(pa_smem);
+  store(pa_smem, step_tile(0) * PA_KEYS);
+  *(u32x2*)(pa_smem + 4 * TILE + threadIdx.x * (D / 8)) = u32x2{0u, 0u};
+  if (D == 128)
+    *(u32x2*)(pa_smem + 4 * TILE + threadIdx.x * (D / 8) + 8) = u32x2{0u, 0u};
   for (int it = 0; it < steps; ++it) {
     __syncthreads();
     const int kv0 = step_tile(it) * PA_KEYS;
@@ -381,15 +403,23 @@ paged_prefill_kernel(PagedArgs A) {
         l_run += p[j];
       }
       const pa_frag pb = pa_pack8(p);
+      // 16 keys that no row of this wave sees: zeros for values
+      const int key0 = kv0 + ks * 16;
+      bool blind = key0 >= w_end;
+      if (LOCAL)
+        blind |= (key0 + 16 <= w_lo) &
+                 ((key0 >= A.keep_first) | (key0 + 16 <= w_c));
+      const char* vk = blind ? pa_smem + 4 * TILE : vb + ks * 16 * 2 * D;
 #pragma unroll
       for (int b = 0; b < D / 32; ++b) {
-        const char* at = vb + ks * 16 * 2 * D + vad[b & 1] + (b >> 1) * 128;
+        const char* at = vk + vad[b & 1] + (b >> 1) * 128;
         acc[b] = pa_mfma32(pa_tr(at, at + 8 * 2 * D), pb, acc[b]);
       }
     }
     pa_order<D / 4, D / 8, 8, 2>();
     }
-    if (more) store(pa_smem + ((it + 1) & 1) * 2 * TILE);
+    if (more)
+      store(pa_smem + ((it + 1) & 1) * 2 * TILE, step_tile(it + 1) * PA_KEYS);
   }
 
   if (!live) return;
@@ -486,7 +516,9 @@ __device__ __forceinline__ void pa_store(const PagedArgs& A, long t, int hq,
 }
 
 template <int D, bool KV8, bool LOCAL>
-__global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
+paged_decode_kernel(PagedArgs A) {
   constexpr int ES = KV8 ? 1 : 2;
   constexpr int KK = D / 32;                 // k-steps of the scores
   constexpr int DB = D / 16;                 // 16-column blocks of O
@@ -561,7 +593,19 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
     if (x + 4 < end) next = pa_entry(table, page_of(x + 4));
   }
   for (; x < end; x += 4) {
-    // this page's V into the wave's tile, then the next page's loads
+    const int kv0 = page_of(x) * PA_PG;
+    auto visible = [&](int kp) {
+      bool vis = kp <= v.p;
+      if (LOCAL) vis &= (kp >= v.lo) | ((u32)(kp - v.c_lo) < kept_n);
+      return vis;
+    };
+    // this page's V into the wave's tile, then the next page's loads; rows of
+    // keys that are not visible as zeros (their weight is 0, but what lies there
+    // may be infinite or NaN, which 0 does not take away)
+    if (kv0 + PA_PG - 1 > v.p || (LOCAL && kv0 < v.lo))
+#pragma unroll
+      for (int j = 0; j < VL; ++j)
+        if (!visible(kv0 + (j * 64 + lane) / (D / 8))) vx[j] = Raw(0);
 #pragma unroll
     for (int j = 0; j < VL; ++j) {
       const int row = (j * 64 + lane) / (D / 8), c = (j * 64 + lane) % (D / 8);
@@ -578,7 +622,6 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
             __builtin_bit_cast(pa_frag, pa_widen<KV8>(kx[h * KK + kk])), qb[kk],
             sc[h]);
     }
-    const int kv0 = page_of(x) * PA_PG;
     if (x + 4 < end) load();
     if (x + 8 < end) next = pa_entry(table, page_of(x + 8));
     // ---- this lane: head lo16, keys kv0 + h*16 + g4*4 + r
@@ -589,14 +632,10 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(PagedArgs A) {
       for (int r = 0; r < 4; ++r) {
         const int kp = kv0 + h * 16 + g4 * 4 + r;
         float z = sc[h][r] * A.scale;
-        bool vis = kp <= v.p;
-        if (LOCAL) {
-          if (A.r1)
-            z -= r1 * __builtin_amdgcn_logf(1.f +
-                                            r2 * (float)max(v.p - kp, 0));
-          vis &= (kp >= v.lo) | ((u32)(kp - v.c_lo) < kept_n);
-        }
-        sc[h][r] = vis ? z : PA_NONE;
+        if (LOCAL && A.r1)
+          z -= r1 * __builtin_amdgcn_logf(1.f +
+                                          r2 * (float)max(v.p - kp, 0));
+        sc[h][r] = visible(kp) ? z : PA_NONE;
         tmax = fmaxf(tmax, sc[h][r]);
       }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
@@ -748,7 +787,11 @@ static inline void pa_launch_prefill(PagedArgs A, hipStream_t s) {
   const int G = A.Hq / A.Hk;
   A.hpb = G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
   A.rpb = 4 / A.hpb;
-  const size_t smem = 2 * 2 * (size_t)PA_KEYS * D * 2;
+  const size_t smem = 2 * 2 * (size_t)PA_KEYS * D * 2 + 16 * D * 2;
+  static std::atomic<unsigned long long> asked{0};
+  if (smem > 65536)
+    lds_limit((const void*)paged_prefill_kernel<D, KV8, LOCAL>, (int)smem,
+              asked);
   hipLaunchKernelGGL((paged_prefill_kernel<D, KV8, LOCAL>),
                      dim3((unsigned)A.n_tiles * (A.Hq / A.hpb)),
                      dim3(256), smem, s, A);
