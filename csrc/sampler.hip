@@ -596,6 +596,13 @@ __device__ __forceinline__ s16x2 ordered2(u32 w) {
   return v ^ ((v >> (short)15) & m);
 }
 
+// whole part, 2**32 - 1 for 2**32 (which a C++ conversion leaves undefined)
+__device__ __forceinline__ u32 to_u32(float v) {
+  u32 r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
 template <class T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
@@ -904,7 +911,7 @@ sampler_count_kernel(SmpArgs A) {
   // floor(p 2**32) of one logit; the conversion stops at 2**32 - 1, so that
   // values of p = 1 lack one
   auto q32 = [&](float v) -> u32 {
-    return v >= low ? (u32)(__expf((v - m) * inv_t) * 4294967296.0f) : 0u;
+    return v >= low ? to_u32(__expf((v - m) * inv_t) * 4294967296.0f) : 0u;
   };
   auto mass8 = [&](const u32x4& w) {
     u64 sum = 0;
@@ -915,7 +922,9 @@ sampler_count_kernel(SmpArgs A) {
     }
     return sum;
   };
-  const int top_code = sm.one;
+  // kept values of p = 1 (a value just below the maximum may round to it and
+  // still be cut off)
+  const int top_code = max(sm.one, tcode);
   const float top = bf2f((u16)(top_code >= 0 ? top_code : 0x7fff ^ top_code));
   auto ones8 = [&](const u32x4& w) {
     u32 n = 0;

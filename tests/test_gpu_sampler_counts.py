@@ -132,3 +132,42 @@ def test_extreme_rows():
         ops.sampler_fused(lg[row:row + 1], one, one, (one * v).int(), one * 0.5,
                           None if mask is None else pack(mask), v, tok, lp)
         assert tok.item() == 0 and lp.item() == ninf
+
+
+def same_as_general(logits, temp, top_p, top_k, us):
+    """bf16 rows against the same values in float32, which the kernel without
+    counters samples: the tokens are equal, as both sum whole numbers."""
+    v = logits.shape[1]
+    for u in us:
+        res = []
+        for lg in (logits, logits.float()):
+            n = lg.shape[0]
+            tok = torch.full((n,), -7, dtype=torch.int32, device=DEV)
+            lp = torch.zeros(n, device=DEV)
+            ops.sampler_fused(
+                lg, torch.full((n,), temp, device=DEV),
+                torch.full((n,), top_p, device=DEV),
+                torch.full((n,), top_k or v, dtype=torch.int32, device=DEV),
+                torch.full((n,), u, device=DEV), None, v, tok, lp)
+            res.append((tok.cpu(), lp.cpu()))
+        assert torch.equal(res[0][0], res[1][0]), (temp, top_p, top_k, u)
+        torch.testing.assert_close(res[0][1], res[1][1], rtol=0, atol=1e-5,
+                                   equal_nan=True)
+
+
+@pytest.mark.parametrize("temp,top_p,top_k", [
+    (0.0, 1.0, 0), (1.0, 1.0, 1), (0.7, 1.0, 2), (1.0, 1e-9, 0), (3.0, 0.9, 0)])
+def test_values_that_round_to_the_maximum(temp, top_p, top_k):
+    """Values whose exponential is 1 although they are not the largest: only
+    those that are kept have a mass."""
+    v = 4096
+    rows = torch.full((6, v), -1.0)
+    rows[0, 10], rows[0, 20] = -1e-9, 0.0
+    rows[1, 5:205] = -torch.logspace(-6, -30, 200)       # rising towards zero
+    rows[2, 5:205] = torch.logspace(-30, -9, 200)        # rising from zero
+    rows[3, 700:900] = torch.logspace(-30, -9, 200)
+    rows[3, 3000:3200] = -torch.logspace(-9, -30, 200)
+    rows[4, :] = torch.linspace(1e-12, 1e-9, v)
+    rows[5, 600], rows[5, 601], rows[5, 4000] = 1e-9, 2e-9, 3e-9
+    same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
+                    (0.0, 0.3, 0.999))
