@@ -552,7 +552,8 @@ __global__ void __launch_bounds__(SMP_THREADS) sampler_kernel(SmpArgs A) {
 // Counters are 16 bits wide, those of v and -v share a word (128 KB). A row
 // with a value that occurs 65,536 times overflows one; every overflow lowers
 // the sum of the counters, so comparing it with the number of alive tokens
-// finds all of them, and such a row is sampled by the general code.
+// finds all of them, and such a row is sampled by the general code. So is a row
+// with a NaN or +inf.
 //
 // Bound by instruction issue: four to count and sixteen to select per logit.
 // 1024 x 151,936 by the general kernel and here: 1382 -> 197 us (top_p 0.95 at
@@ -579,6 +580,7 @@ struct CountShared {
   u32 wave_alive[CNT_WAVES];
   float wave_z[CNT_WAVES];
   int max_pos, min_neg;         // magnitudes of the extremes
+  int odd;                      // a NaN or +inf was counted
   int seg[2];                   // where the count / the mass crosses
   u64 above[2];
   u32 tau[2];
@@ -685,6 +687,7 @@ sampler_count_kernel(SmpArgs A) {
     if (tid == 0) {
       sm.max_pos = -1;
       sm.min_neg = 0x8000;
+      sm.odd = 0;
       sm.seg[0] = sm.seg[1] = -1;
       sm.tau[0] = sm.tau[1] = 0;
       sm.tcode = sm.one = 0x7fff;
@@ -732,6 +735,10 @@ sampler_count_kernel(SmpArgs A) {
   // segment j * CNT_WAVES + wave is this wave's, so that neighbours spread
   u32 present = 0;
   int max_pos = -1, min_neg = 0x8000;
+  if (tid < 0x80) {
+    const u32 w = sm.words[0x7f80 + tid];
+    if (tid ? w : w & 0xffffu) sm.odd = 1;
+  }
 #pragma unroll 4
   for (int j = 0; j < CNT_SEGS / CNT_WAVES; ++j) {
     const int mag0 = (j * CNT_WAVES + wave) * 64;
@@ -828,7 +835,8 @@ sampler_count_kernel(SmpArgs A) {
   // ... or zeros of both signs on top, of which the first is the maximum and
   // decides whether the other sign ranks below
   const bool zeros = pos && sm.max_pos == 0 && sm.min_neg == 0;
-  if (none || counted != want || (zeros && !greedy)) {
+  // ... or NaN or +inf, whose differences have no order
+  if (none || counted != want || (zeros && !greedy) || sm.odd) {
     __syncthreads();
     sample_row<true, CNT_THREADS>(A, row, tid,
                                   *(SmpShared<CNT_WAVES>*)cnt_lds);

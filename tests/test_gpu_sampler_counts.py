@@ -171,3 +171,25 @@ def test_values_that_round_to_the_maximum(temp, top_p, top_k):
     rows[5, 600], rows[5, 601], rows[5, 4000] = 1e-9, 2e-9, 3e-9
     same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
                     (0.0, 0.3, 0.999))
+
+
+@pytest.mark.parametrize("temp,top_p,top_k", [
+    (0.0, 1.0, 0), (1.0, 1.0, 0), (0.7, 0.9, 0), (1.0, 1.0, 3)])
+def test_infinities_and_nans(temp, top_p, top_k):
+    v = 4096
+    inf, nan = float("inf"), float("nan")
+    rows = torch.randn(8, v, generator=torch.Generator().manual_seed(5))
+    rows[0, 70], rows[0, 3000] = inf, inf         # greedy: the first of them
+    rows[1, 9] = inf
+    rows[2, 70:90] = -inf
+    rows[3, 5], rows[3, 4000] = nan, nan
+    rows[4, 5], rows[4, 4000], rows[4, 6] = nan, inf, -inf
+    rows[5, :] = inf
+    rows[6, :] = nan
+    rows[7, 1:] = nan
+    same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
+                    (0.0, 0.4, 0.999))
+    bits = rows.to(torch.bfloat16).view(torch.int16)
+    bits[3, 5], bits[3, 4000] = -1, -1            # the NaN of all bits
+    same_as_general(bits.view(torch.bfloat16).to(DEV), temp, top_p, top_k,
+                    (0.0, 0.4, 0.999))
