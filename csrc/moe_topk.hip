@@ -9,6 +9,8 @@
 //
 // Ranks that hold the experts [base, base + n_local) get local numbers; other
 // choices come back as n_local with weight 0 (a segment that no GEMM visits).
+#include <cfloat>
+
 #include "common.h"
 
 template <int NP>
@@ -20,15 +22,16 @@ __global__ void __launch_bounds__(256) moe_topk_kernel(
   const int lane = threadIdx.x & 63;
   const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T) return;
-  // cmp orders the choice: NaN and -inf logits below every finite one, chosen
-  // and missing experts below those
+  // cmp orders the choice: NaN and -inf logits below every finite one (the
+  // lowest float lies below the lowest bf16), chosen and missing experts below
+  // those
   float x[NP], cmp[NP];
   float m = -INFINITY;
 #pragma unroll
   for (int n = 0; n < NP; ++n) {
     const int e = n * 64 + lane;
     x[n] = e < E ? bf2f(logits[t * E + e]) : -INFINITY;
-    cmp[n] = e < E ? (x[n] >= -3e38f ? x[n] : -3e38f) : -INFINITY;
+    cmp[n] = e < E ? (x[n] > -INFINITY ? x[n] : -FLT_MAX) : -INFINITY;
     m = fmaxf(m, x[n]);
   }
   m = wave_max_f32(m);

@@ -75,3 +75,21 @@ def test_ties_and_non_finite():
     # as the torch router: a row with inf or NaN has NaN weights
     assert w[2].isnan().any() and w[3].isnan().all()
     assert ((seg >= 0) & (seg < 4)).all()
+
+
+@pytest.mark.parametrize("E,k", [(8, 2), (70, 8)])
+def test_masks_of_the_lowest_value(E, k):
+    """Logits masked with the type's lowest value are ordinary numbers: a token
+    with nothing else shares its weight among them, and beside others they
+    weigh nothing."""
+    lowest = torch.finfo(torch.bfloat16).min
+    logits = torch.full((4, E), lowest)
+    logits[1, 3] = 0.0
+    logits[2, 3:3 + k] = 1.0
+    logits[3, 5] = lowest * (1 - 2.0 ** -7)       # the next number above it
+    logits = logits.bfloat16()
+    row_tok, w, off, cnt, pos = _layout(logits, k, 0, E, 64)
+    want, _ = R.topk_softmax_router(logits, k)
+    assert torch.isfinite(w).all()
+    torch.testing.assert_close(w.sort(1)[0], want.sort(1)[0])
+    assert int(cnt.sum()) == 4 * k
