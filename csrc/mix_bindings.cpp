@@ -1007,7 +1007,6 @@ void expert_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
   // weighted rows: the matrix-core kernel has the silu unit only
   const bool mfma = kind == 0 && K % 64 == 0 && N % 64 == 0 &&
                     (!rw || act == 1);
-  TORCH_CHECK(bm != 32 || mfma, "tiles of 32 rows: matrix-core kernel only");
   TORCH_CHECK(bm != 256 || !mfma || N % (glu ? 128 : 256) == 0,
               "tiles of 256 rows need a multiple of 256 columns (gated: 128)");
   if (mfma) {

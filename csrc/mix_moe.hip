@@ -211,7 +211,7 @@ extern "C" void mix_moe_route(int* idx, float* wts, const float* logits, long T,
 
 // ---- expert_gemm (plain) ---------------------------------------------------
 // out[r, n] = act(sum_k a[tok(r), k] * w[e, n, k]) over 64-row tiles of the
-// padded segments; 256 threads as 16 x 16, 4 x 4 outputs a thread, K staged
+// padded segments (32 rows where these are padded to 32); 256 threads as 16 x 16, 4 x 4 outputs a thread, K staged
 // 16 at a time through LDS. Rows past a segment's live count are not stored.
 // act 1: relu(x)^2. act 2: w holds N gate rows then N up rows per expert and
 // out[r, n] = g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up).
@@ -227,8 +227,9 @@ __global__ void __launch_bounds__(256) expert_gemm_plain_kernel(
   __shared__ float Bs[16][65];
   __shared__ float Us[16][65];
   const bool glu = act >= 2;
-  const int tiles_per = bm / 64;
-  const int t64 = blockIdx.x;              // 64-row tile over all segments
+  const int rows = min(bm, 64);
+  const int tiles_per = bm / rows;
+  const int t64 = blockIdx.x;              // tile of `rows` over all segments
   const int t = t64 / tiles_per;           // bm-row tile
   if (t >= tile_off[E]) return;
   int lo = 0, hi = E - 1;
@@ -237,8 +238,8 @@ __global__ void __launch_bounds__(256) expert_gemm_plain_kernel(
     if (tile_off[mid] <= t) lo = mid; else hi = mid - 1;
   }
   const int e = lo;
-  const int m0 = (t - tile_off[e]) * bm + (t64 % tiles_per) * 64;
-  const int live = counts[e] - m0;         // live rows of this tile
+  const int m0 = (t - tile_off[e]) * bm + (t64 % tiles_per) * rows;
+  const int live = min(counts[e] - m0, rows);  // live rows of this tile
   if (live <= 0) return;
   const long seg = (long)tile_off[e] * bm + m0;
   const int n0 = blockIdx.y * 64;
@@ -320,7 +321,7 @@ extern "C" void mix_expert_gemm_plain(void* out, const void* a, const void* w,
                                       int bm, long n_rows, int act, float limit,
                                       const float* row_w, int f32,
                                       hipStream_t s) {
-  const long tiles = n_rows / 64;
+  const long tiles = n_rows / (bm < 64 ? bm : 64);
   if (tiles == 0) return;
   const dim3 grid((unsigned)tiles, (unsigned)((N + 63) / 64));
   if (f32)

@@ -78,3 +78,48 @@ def test_tile_rule(n_rows, want):
     assert expert_tile(n_rows, 8, 128, 256, gated=False) <= 128
     # 1536 workgroups: two rounds of three a CU, but one and a half of four
     assert expert_tile(512, 32, 3072, 4096) == 64
+
+
+@pytest.mark.parametrize("act,weighted,dtype", [
+    (hops.ACT_GLU_CLAMPED, True, torch.bfloat16),
+    (hops.ACT_RELU2, True, torch.bfloat16),
+    (hops.ACT_SILU_GATE, False, torch.float32)])
+def test_plain_kernel_takes_every_tile(act, weighted, dtype):
+    """Units that the matrix-core kernel does not have over weighted rows, and
+    float32, on the tile that `expert_gemm_tile` names for a few tokens and on
+    the others."""
+    g = torch.Generator().manual_seed(11)
+    E, K, ff, T, k = 8, 128, 64, 9, 2
+    gated = act in (hops.ACT_SILU_GATE, hops.ACT_GLU_CLAMPED)
+    w = (torch.randn(E, ff * (2 if gated else 1), K, generator=g)
+         * K ** -0.5).to(dtype)
+    x = torch.randn(T, K, generator=g).to(dtype)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k]
+                       for _ in range(T)]).int()
+    wts = torch.rand(T, k, generator=g)
+    xd, wd = x.to(DEV), w.to(DEV)
+    for bm in {hops.expert_gemm_tile(xd, wd, T * k, gated), 32, 64, 128, 256}:
+        rt, off, cnt, pos, rw = hops.moe_dispatch(idx.to(DEV), E, bm,
+                                                  wts.to(DEV))
+        out = torch.zeros(rt.shape[0], ff, dtype=dtype, device=DEV)
+        hops.expert_gemm(out, xd, wd, rt, off, cnt, act, bm, 1.5,
+                         rw if weighted else None)
+        got = out[pos.long()].float().cpu()
+        for t in range(T):
+            for j in range(k):
+                y = x[t].double() @ w[idx[t, j]].double().T
+                if weighted:
+                    y = y * float(wts[t, j])
+                if act == hops.ACT_RELU2:
+                    y = y.clamp(min=0) ** 2
+                else:
+                    a, u = y[:ff], y[ff:]
+                    if act == hops.ACT_GLU_CLAMPED:
+                        a, u = a.clamp(max=1.5), u.clamp(-1.5, 1.5)
+                        y = a * torch.sigmoid(1.702 * a) * (u + 1)
+                    else:
+                        y = a * torch.sigmoid(a) * u
+                # one rounding to the type over sums of 128 products
+                tol = 2 ** -8 if dtype == torch.bfloat16 else 1e-5
+                torch.testing.assert_close(got[t, j].double(), y, rtol=tol,
+                                           atol=tol)
