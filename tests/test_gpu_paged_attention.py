@@ -103,3 +103,37 @@ def test_prompt_tiles_in_any_order(Hq, Hk):
             a = (0 if ts[i] == 0 else 200) + tq[i]
             b = min(a + 32, 200 if ts[i] == 0 else 330)
             assert torch.equal(part[a:b], whole[a:b])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("delta", [0.375, 0.6, 0.65, 0.9, 1.05, 1.25])
+def test_sum_of_many_weights(D, delta):
+    """The denominator of a prompt's row over 40,000 keys, a first one above all
+    others and the rest alike, so that results are (rounded weights x values) /
+    (weights). Every page holds the same 32 values a column. The roundings of
+    the results to bf16 (up to 2^-8 of a value between 1 and 2) are 0 on
+    average: the mean of 64 D of them is within 4 * 2^-8 / sqrt(3 * 64 D)."""
+    n, H, new = 40000, 64, 32
+    pages = (n + 31) // 32
+    g = torch.Generator().manual_seed(2)
+    u = torch.randn(D, generator=g).sign().to(DEV)
+    v = (1 + torch.rand(H, 32, D, generator=g)).bfloat16().to(DEV)
+    vc = v.expand(pages, H, 32, D).contiguous()
+    top = torch.tensor(8.0 / D).bfloat16().item()
+    low = torch.tensor((8.0 - delta) / D).bfloat16().item()
+    kc = (u * low).bfloat16().expand(pages, H, 32, D).contiguous()
+    kc[0, :, 0] = (u * top).bfloat16()
+    q = u.bfloat16().expand(new, H, D).contiguous()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    one = torch.zeros(1, **i32)
+    out = ops.paged_attention(
+        q, kc, vc, torch.arange(pages, **i32)[None], torch.tensor([n], **i32),
+        torch.tensor([0, new], **i32), 1.0, num_decodes_tail=0, tile_seq=one,
+        tile_q0=one, prefill_token_count=new)
+    p = math.exp(D * low - D * top)
+    b = torch.tensor(p).bfloat16().item()
+    last = new - 1                                   # its row sees every key
+    total = v.double().sum(1) * pages - v[:, 0].double()
+    want = (v[:, 0].double() + b * total) / (1 + (n - 1) * p)
+    ratio = (out[last].double() / want).mean().item()
+    assert abs(ratio - 1) < 4 * 2.0 ** -8 / math.sqrt(3 * H * D)
