@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module
 
 from .. import ops
 
@@ -15,7 +16,9 @@ class Linear(nn.Linear):
 
 def bare(layer: nn.Module) -> bool:
     """Whether a caller may fuse this layer's product with what follows it: a
-    Linear without bias, hooks or a forward of its own."""
+    Linear without bias, hooks (its own or every module's) or a forward of its
+    own."""
     return (type(layer) is Linear and layer.bias is None
             and not layer._forward_hooks and not layer._forward_pre_hooks
+            and not module._has_any_global_hook()
             and "forward" not in layer.__dict__)

@@ -1,0 +1,137 @@
+"""Where a linear layer may leave torch's product for the kernel over few rows:
+never where something of torch's has to see the product."""
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from sutro_amd import ops
+from sutro_amd.models import linear as L
+from sutro_amd.models.qwen3 import Qwen3MLP
+from sutro_amd.parallel.tp import TPContext
+
+
+class _Kernels:
+    """Stands in for the extension: counts the calls that reach it."""
+
+    def __init__(self):
+        self.calls = 0
+
+    def linear_skinny(self, x, w, bias, gated):
+        self.calls += 1
+        y = F.linear(x, w, bias)
+        if gated:
+            a, b = y.chunk(2, -1)
+            y = F.silu(a) * b
+        return y
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    k = _Kernels()
+    monkeypatch.setattr(ops, "_use_hip", lambda t: True)
+    monkeypatch.setattr(ops, "_require_hip", lambda: k)
+    return k
+
+
+def _operands(rows=4, n=8, k=32):
+    g = torch.Generator().manual_seed(1)
+    return (torch.randn(rows, k, generator=g).bfloat16(),
+            torch.randn(n, k, generator=g).bfloat16())
+
+
+def test_plain_call_takes_the_kernel(kernels):
+    x, w = _operands()
+    with torch.no_grad():
+        ops.linear(x, w)
+    assert kernels.calls == 1
+
+
+def test_gradients(kernels):
+    x, w = _operands()
+    w.requires_grad_()
+    ops.linear(x, w).sum().backward()
+    assert kernels.calls == 0 and w.grad is not None
+
+
+def test_forward_mode(kernels):
+    x, w = _operands()
+    t = torch.ones_like(x)
+    with torch.no_grad(), forward_ad.dual_level():
+        y = ops.linear(forward_ad.make_dual(x, t), w)
+        tangent = forward_ad.unpack_dual(y).tangent
+    assert kernels.calls == 0
+    torch.testing.assert_close(tangent, F.linear(t, w))
+
+
+def test_vmap(kernels):
+    x, w = _operands()
+    xs = torch.stack([x, 2 * x])
+    with torch.no_grad():
+        y = torch.func.vmap(lambda v: ops.linear(v, w))(xs)
+    assert kernels.calls == 0
+    torch.testing.assert_close(y, F.linear(xs, w))
+
+
+def test_modes_see_the_product(kernels):
+    x, w = _operands()
+    seen = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with torch.no_grad():
+        with Functions():
+            ops.linear(x, w)
+        assert "linear" in seen
+        del seen[:]
+        with Dispatch():
+            ops.linear(x, w)
+        assert seen
+    assert kernels.calls == 0
+
+
+def test_trace(kernels):
+    x, w = _operands()
+    with torch.no_grad():
+        f = torch.jit.trace(lambda v: ops.linear(v, w), (x,),
+                            check_trace=False)
+        assert kernels.calls == 0
+        torch.testing.assert_close(f(3 * x), F.linear(3 * x, w))
+
+
+def test_autocast(kernels):
+    x, w = _operands()
+    with torch.no_grad(), torch.autocast("cpu", dtype=torch.float16):
+        y = ops.linear(x, w)
+    assert kernels.calls == 0 and y.dtype == torch.float16
+
+
+def test_hooks_on_every_module():
+    mlp = Qwen3MLP(32, 16, torch.bfloat16, TPContext())
+    called = []
+    handles = [
+        nn.modules.module.register_module_forward_hook(
+            lambda m, a, y: called.append(m)),
+        nn.modules.module.register_module_forward_pre_hook(
+            lambda m, a: called.append(m))]
+    try:
+        assert not L.bare(mlp.gate_up_proj)
+        with torch.no_grad():
+            mlp(torch.zeros(2, 32, dtype=torch.bfloat16))
+        assert called.count(mlp.gate_up_proj) == 2
+    finally:
+        for h in handles:
+            h.remove()
+    assert L.bare(mlp.gate_up_proj)
