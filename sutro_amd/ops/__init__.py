@@ -173,20 +173,23 @@ def sampler_fused(logits, temps, top_ps, top_ks, u, packed_mask, vocab_limit,
                                  packed_mask, vocab_limit, out_tok, out_lp)
 
 
-def _unwatched(device: str) -> bool:
+_functions, _dispatches = (torch._C._len_torch_function_stack,
+                           torch._C._len_torch_dispatch_stack)
+_transforms = torch._C._functorch.peek_interpreter_stack
+_tracing, _autocast = torch._C._is_tracing, torch._C._is_any_autocast_enabled
+
+
+def _unwatched() -> bool:
     """Whether nothing of torch's has to see an operation on plain tensors:
     function and dispatch modes (counters, fake tensors, graph recorders),
     vmap and the other transforms, forward-mode derivatives, a compiler,
     autocast. (A default device is a function mode too, and minds nothing.)"""
-    if torch._C._len_torch_function_stack() and not all(
-            isinstance(m, DeviceContext)
-            for m in _get_current_function_mode_stack()):
+    if _functions() and not all(isinstance(m, DeviceContext)
+                                for m in _get_current_function_mode_stack()):
         return False
-    return not (torch._C._len_torch_dispatch_stack()
-                or torch._C._functorch.peek_interpreter_stack() is not None
+    return not (_dispatches() or _transforms() is not None or _autocast()
                 or forward_ad._current_level >= 0
-                or torch.compiler.is_compiling()
-                or torch.is_autocast_enabled(device))
+                or torch.compiler.is_compiling())
 
 
 def _few_rows(x, w, gated: bool = False) -> bool:
@@ -202,7 +205,7 @@ def _few_rows(x, w, gated: bool = False) -> bool:
       6144 x 4096      15.6 / 10.7    14.6 / 15.8   14.2 / 22.3
       32768 x 4096     61.5 / 48.8    61.7 / 65.6   62.0 / 70.5
     and with silu_mul behind it 16384 x 2048: 19.6 / 14.0 for one row."""
-    if (type(x) is not torch.Tensor or torch.jit.is_tracing()
+    if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False
     if x.dim() != 2 or not 1 <= x.shape[0] <= 32 or not _use_hip(x):
@@ -211,7 +214,7 @@ def _few_rows(x, w, gated: bool = False) -> bool:
     rows = w.shape[0]
     fits = (M <= 2 or (M <= 16 and K <= 4096 and rows * K <= 1 << 24)
             or (K <= 2048 and rows * K <= 1 << 23))
-    return (fits and _unwatched(x.device.type) and x.dtype == torch.bfloat16
+    return (fits and _unwatched() and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.device == x.device
             and w.dim() == 2 and w.shape[1] == K and K % 32 == 0 and K > 0
             and rows % (8 if gated else 4) == 0 and rows > 0
