@@ -77,11 +77,11 @@ extern "C" void sutro_attn_decode_mfma(void* out, const void* q,
   A.part_o = part_o;
   A.part_ml = part_ml;
   if (head_dim == 128) {
-    if (kv_fp8) pa_launch_decode<128, true, false>(A, s);
-    else pa_launch_decode<128, false, false>(A, s);
+    if (kv_fp8) pa_launch_decode<128, true, false>(A, bt_stride, s);
+    else pa_launch_decode<128, false, false>(A, bt_stride, s);
   } else {
-    if (kv_fp8) pa_launch_decode<64, true, false>(A, s);
-    else pa_launch_decode<64, false, false>(A, s);
+    if (kv_fp8) pa_launch_decode<64, true, false>(A, bt_stride, s);
+    else pa_launch_decode<64, false, false>(A, bt_stride, s);
   }
 }
 

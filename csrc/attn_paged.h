@@ -59,6 +59,7 @@ struct PagedArgs {
   // seq_offset + t - t0
   const int* token_seq;
   int seq_offset, n_rows, nsplit;
+  int quad;             // pages up to which a wave takes an item (0: none)
   long t0;
   float* part_o;        // [n_rows * Hq][nsplit][D]
   float* part_ml;       // [n_rows * Hq][nsplit][2]
@@ -458,14 +459,15 @@ paged_prefill_kernel(PagedArgs A) {
 }
 
 // ---------------------------------------------------------------------------
-// Single tokens. One workgroup of 4 waves per (row, kv head, run of pages); the
-// G <= 16 query heads of the kv head are the 16 columns of the products. The
-// waves take the run's pages in turn, each with the next page's K and V on the
-// way in registers while this one is computed (V passes through the wave's own
-// LDS tile to be read transposed), and their partial results meet in LDS. Few
-// rows over long contexts would leave most of the chip idle: their pages are
-// cut into up to nsplit runs of at least PA_RUN pages, whose partial results
-// paged_join_kernel joins. A context of one run is finished here.
+// Single tokens. One workgroup of 4 waves per item (row and kv head) and run of
+// pages; the G <= 16 query heads of the kv head are the 16 columns of the
+// products. The waves take the run's pages in turn, each with the next page's K
+// and V on the way in registers while this one is computed (V passes through the
+// wave's own LDS tile to be read transposed), and their partial results meet in
+// LDS. Few rows over long contexts would leave most of the chip idle: their pages
+// are cut into up to nsplit runs of at least PA_RUN pages, whose partial results
+// a second kernel joins. A context of one run is finished here, one of a single
+// page by one wave.
 //
 // Bound by memory: K and V of a row are read once. One wave a row, each page
 // loaded and then computed, took 1.9 us a page; a call now takes (with the
@@ -475,8 +477,20 @@ paged_prefill_kernel(PagedArgs A) {
 // 256 rows of 130 keys and 8 heads (138 MB, 3.7 TB/s, one run each). Runs of 8
 // pages give every wave two pages, the fewest that hide one load behind
 // another's work.
+//
+// Many rows over short contexts are bound by the workgroups themselves: two of
+// them fit a CU, and one that has a page or two leaves most of its waves idle.
+// From PA_QUAD_ITEMS items on a first layer of workgroups takes four neighbouring
+// items each, a wave one, where none has more than PA_QUAD_PAGES pages; four more
+// layers take the other items one by one as above (no layer where the table or
+// the window bounds all of them). 4 kv heads, 1024 rows of 20 / 60 / 130 / 400
+// keys: 30 / 35 / 68 / 153 us a workgroup an item, 20 / 28 / 62 / 153 this way; 2048
+// rows of 20 keys 55 -> 35. (A wave alone with a long context beside short ones
+// would take as long as four together: therefore the layers, not more pages.)
 // ---------------------------------------------------------------------------
 #define PA_RUN 8
+#define PA_QUAD_ITEMS 1024  // items from which a wave takes a short one alone,
+#define PA_QUAD_PAGES 6     // short: up to so many pages
 
 // runs of a context of n pages: (pages per run, number of runs)
 __device__ __forceinline__ int pa_run_pages(int n, int nsplit) {
@@ -519,6 +533,26 @@ __device__ __forceinline__ void pa_store(const PagedArgs& A, long t, int hq,
   A.out[t * A.ldo + A.out_off + (long)hq * D + c] = f2bf(o * f);
 }
 
+// the same for columns c .. c + 3
+template <bool LOCAL>
+__device__ __forceinline__ void pa_store4(const PagedArgs& A, long t, int hq,
+                                          int D, int c, f32x4 o, float l) {
+  float f = l > 0.f ? 1.0f / l : 0.f;
+  if (LOCAL) {
+    f *= A.out_scale;
+    if (A.gate_off >= 0) {
+      const u16* gp = A.proj + t * A.ld + A.gate_off + (long)hq * A.gate_n;
+      if (A.gate_n > 1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] *= 1.f / (1.f + expf(-bf2f(gp[c + e])));
+      } else {
+        f *= 1.f / (1.f + expf(-bf2f(gp[0])));
+      }
+    }
+  }
+  *(u32x2*)(A.out + t * A.ldo + A.out_off + (long)hq * D + c) = pa_pack4(o * f);
+}
+
 template <int D, bool KV8, bool LOCAL>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
@@ -532,14 +566,37 @@ paged_decode_kernel(PagedArgs A) {
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lo16 = lane & 15, g4 = lane >> 4;
   const int G = A.Hq / A.Hk;
-  const int kh = blockIdx.x % A.Hk;
-  const int i = blockIdx.x / A.Hk;
+  const int items = A.n_rows * A.Hk;   // (row, kv head)
+  // with A.quad: the first layer of workgroups (y = 0) takes four items each,
+  // one a wave, where all four are short; the other four layers take the items
+  // of the rest one by one, neighbours side by side
+  int item = blockIdx.x;
+  bool solo = false;
+  if (A.quad) {
+    if (blockIdx.y) item += (blockIdx.y - 1) * gridDim.x;
+    const int first = blockIdx.y ? item & ~3 : item * 4;
+    if (first >= items) return;
+    int longest = 0;
+    for (int r = first / A.Hk; r <= min(first + 3, items - 1) / A.Hk; ++r)
+      longest = max(longest, pa_span<LOCAL>(A, r).total);
+    solo = blockIdx.y == 0;
+    if (solo != (longest <= A.quad)) return;
+    if (solo) item = first + w;
+    if (item >= items) return;
+  }
+  const int kh = item % A.Hk;
+  const int i = item / A.Hk;
   const PagedSpan v = pa_span<LOCAL>(A, i);
   const int run = pa_run_pages(v.total, A.nsplit);
-  const int begin = blockIdx.y * run;
+  const int begin = A.quad ? 0 : blockIdx.y * run;
   if (begin >= v.total) return;
   const int end = min(v.total, begin + run);
   const bool alone = run >= v.total;
+  if (!A.quad && v.total == 1) {
+    solo = true;
+    if (w) return;
+  }
+  const int step = solo ? 1 : 4;
   const long t = A.t0 + i;
 
   // V tiles of the waves, then (behind a barrier) their results [4][16][D]
@@ -590,13 +647,13 @@ paged_decode_kernel(PagedArgs A) {
              pa_vchunk(lo16 >> 2, o * 2 + ((lo16 & 3) >> 1)) * 16 +
              (lo16 & 1) * 8;
 
-  int x = begin + w;
+  int x = solo ? begin : begin + w;
   if (x < end) {
     next = pa_entry(table, page_of(x));
     load();
-    if (x + 4 < end) next = pa_entry(table, page_of(x + 4));
+    if (x + step < end) next = pa_entry(table, page_of(x + step));
   }
-  for (; x < end; x += 4) {
+  for (; x < end; x += step) {
     const int kv0 = page_of(x) * PA_PG;
     auto visible = [&](int kp) {
       bool vis = kp <= v.p;
@@ -626,8 +683,8 @@ paged_decode_kernel(PagedArgs A) {
             __builtin_bit_cast(pa_frag, pa_widen<KV8>(kx[h * KK + kk])), qb[kk],
             sc[h]);
     }
-    if (x + 4 < end) load();
-    if (x + 8 < end) next = pa_entry(table, page_of(x + 8));
+    if (x + step < end) load();
+    if (x + 2 * step < end) next = pa_entry(table, page_of(x + 2 * step));
     // ---- this lane: head lo16, keys kv0 + h*16 + g4*4 + r
     float tmax = PA_NONE;
 #pragma unroll
@@ -683,6 +740,20 @@ paged_decode_kernel(PagedArgs A) {
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
 
+  if (solo) {
+    if (lo16 >= G) return;
+    float m = m_run, l = l_run, f = 1.f;
+    if (LOCAL && A.sink) {
+      const float sk = A.sink_w ? A.sink_w[hq] * PA_LOG2E : 0.f;
+      m = fmaxf(m_run, sk);
+      f = __builtin_amdgcn_exp2f(m_run - m);
+      l = f * l_run + __builtin_amdgcn_exp2f(sk - m);
+    }
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+      pa_store4<LOCAL>(A, t, hq, D, b * 16 + g4 * 4, acc[b] * f, l);
+    return;
+  }
   __syncthreads();   // the V tiles are done with
   float* res = (float*)smem;
   if (g4 == 0) {
@@ -725,7 +796,7 @@ paged_decode_kernel(PagedArgs A) {
   }
 }
 
-// Joins the runs of one (row, head). The threads of a column share its runs:
+// Joins the runs of a (row, head). The threads of a column share its runs:
 // one thread a column walked up to 157 of them one after the other, 48 us at
 // 40 k keys against 20 us for the kernel above.
 #define PA_JOIN 512
@@ -774,10 +845,55 @@ __global__ void __launch_bounds__(PA_JOIN) paged_join_kernel(PagedArgs A) {
   pa_store<LOCAL>(A, A.t0 + i, hq, D, c, o, l);
 }
 
-// runs to cut contexts of up to max_pages pages into: as many as give every CU
-// four workgroups, none shorter than PA_RUN pages
+// The same for few runs (then rows are many): a thread a column, nothing shared,
+// and as few workgroups as that leaves, since rows of one run have nothing to
+// join. 32 rows of 64 heads over 20 keys 8.8 -> 6.0 us
+// for the call, over 400 keys 20.7 -> 17.1.
+#define PA_FEW_RUNS 8
+template <int D, bool LOCAL>
+__global__ void __launch_bounds__(PA_JOIN) paged_join_few_kernel(PagedArgs A) {
+  const int idx = blockIdx.x * (PA_JOIN / D) + threadIdx.x / D;
+  if (idx >= A.n_rows * A.Hq) return;
+  const int i = idx / A.Hq, hq = idx % A.Hq, c = threadIdx.x % D;
+  const PagedSpan v = pa_span<LOCAL>(A, i);
+  const int run = pa_run_pages(v.total, A.nsplit);
+  const int n = (v.total + run - 1) / run;
+  if (n <= 1) return;
+  const long at = (long)idx * A.nsplit;
+  float po[PA_FEW_RUNS], pm[PA_FEW_RUNS], pl[PA_FEW_RUNS];
+#pragma unroll
+  for (int y = 0; y < PA_FEW_RUNS; ++y)
+    if (y < n) {
+      po[y] = A.part_o[(at + y) * D + c];
+      pm[y] = A.part_ml[(at + y) * 2];
+      pl[y] = A.part_ml[(at + y) * 2 + 1];
+    }
+  float m = PA_NONE, sk = 0.f;
+#pragma unroll
+  for (int y = 0; y < PA_FEW_RUNS; ++y)
+    if (y < n) m = fmaxf(m, pm[y]);
+  if (LOCAL && A.sink) {
+    sk = A.sink_w ? A.sink_w[hq] * PA_LOG2E : 0.f;
+    m = fmaxf(m, sk);
+  }
+  float l = LOCAL && A.sink ? __builtin_amdgcn_exp2f(sk - m) : 0.f, o = 0.f;
+#pragma unroll
+  for (int y = 0; y < PA_FEW_RUNS; ++y)
+    if (y < n) {
+      const float f = __builtin_amdgcn_exp2f(pm[y] - m);
+      l += f * pl[y];
+      o += f * po[y];
+    }
+  pa_store<LOCAL>(A, A.t0 + i, hq, D, c, o, l);
+}
+
+// Runs to cut contexts of up to max_pages pages into: as many as give every CU
+// four workgroups, none shorter than PA_RUN pages. From 512 items (row, kv head)
+// on contexts stay whole: 128 rows of 400 keys, 4 heads, 28 us in two runs and
+// 21 in one, 2500 keys 127 and 116.
 static inline int pa_splits(long rows, int Hk, int max_pages) {
   const long items = rows * Hk;
+  if (items >= 512) return 1;
   const long want = (1024 + items - 1) / (items > 0 ? items : 1);
   const long most = (max_pages + PA_RUN - 1) / PA_RUN;
   long n = want < most ? want : most;
@@ -802,13 +918,24 @@ static inline void pa_launch_prefill(PagedArgs A, hipStream_t s) {
                      dim3(256), smem, s, A);
 }
 
+// max_pages: of a row at most (by the table, the window or the chunk)
 template <int D, bool KV8, bool LOCAL>
-static inline void pa_launch_decode(const PagedArgs& A, hipStream_t s) {
-  hipLaunchKernelGGL((paged_decode_kernel<D, KV8, LOCAL>),
-                     dim3((unsigned)(A.n_rows * A.Hk), (unsigned)A.nsplit),
-                     dim3(256), 0, s, A);
-  if (A.nsplit > 1)
+static inline void pa_launch_decode(PagedArgs A, int max_pages, hipStream_t s) {
+  const long items = (long)A.n_rows * A.Hk;
+  dim3 grid((unsigned)items, (unsigned)A.nsplit);
+  if (A.nsplit == 1 && items >= PA_QUAD_ITEMS) {
+    A.quad = PA_QUAD_PAGES;
+    grid = dim3((unsigned)((items + 3) / 4), max_pages <= A.quad ? 1u : 5u);
+  }
+  hipLaunchKernelGGL((paged_decode_kernel<D, KV8, LOCAL>), grid, dim3(256), 0,
+                     s, A);
+  if (A.nsplit > PA_FEW_RUNS)
     hipLaunchKernelGGL((paged_join_kernel<D, LOCAL>),
                        dim3((unsigned)(A.n_rows * A.Hq)), dim3(PA_JOIN), 0, s,
                        A);
+  else if (A.nsplit > 1)
+    hipLaunchKernelGGL((paged_join_few_kernel<D, LOCAL>),
+                       dim3((unsigned)((A.n_rows * A.Hq + PA_JOIN / D - 1) /
+                                       (PA_JOIN / D))),
+                       dim3(PA_JOIN), 0, s, A);
 }

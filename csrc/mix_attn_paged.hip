@@ -13,16 +13,21 @@
 #include "mix_common.h"
 #include "attn_paged.h"
 
-// runs the pages of a single token are cut into (see attn_paged.h): its
-// window, chunk and block table bound their number
-extern "C" int mix_paged_splits(long rows, int Hk, int bt_stride, int chunk,
-                                int window, int keep_first) {
+// pages that a single token sees at most
+static int most_pages(int bt_stride, int chunk, int window, int keep_first) {
   long pages = bt_stride;
   if (chunk > 0) pages = min(pages, (long)(chunk + PA_PG - 1) / PA_PG + 1);
   if (window > 0)
     pages = min(pages, (long)(window + PA_PG - 1) / PA_PG + 1 +
                            (keep_first + PA_PG - 1) / PA_PG);
-  return pa_splits(rows, Hk, (int)pages);
+  return (int)pages;
+}
+
+// runs these are cut into (see attn_paged.h)
+extern "C" int mix_paged_splits(long rows, int Hk, int bt_stride, int chunk,
+                                int window, int keep_first) {
+  return pa_splits(rows, Hk,
+                   most_pages(bt_stride, chunk, window, keep_first));
 }
 
 // prompt pieces of n_tiles entries of the tile map, then the n_rows single
@@ -76,7 +81,8 @@ extern "C" void mix_paged_attention(
     else pa_launch_prefill<64, false, true>(A, s);
   }
   if (n_rows > 0) {
-    if (D == 128) pa_launch_decode<128, false, true>(A, s);
-    else pa_launch_decode<64, false, true>(A, s);
+    const int most = most_pages(bt_stride, chunk, window, keep_first);
+    if (D == 128) pa_launch_decode<128, false, true>(A, most, s);
+    else pa_launch_decode<64, false, true>(A, most, s);
   }
 }

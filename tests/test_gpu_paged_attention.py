@@ -137,3 +137,22 @@ def test_sum_of_many_weights(D, delta):
     want = (v[:, 0].double() + b * total) / (1 + (n - 1) * p)
     ratio = (out[last].double() / want).mean().item()
     assert abs(ratio - 1) < 4 * 2.0 ** -8 / math.sqrt(3 * H * D)
+
+
+@pytest.mark.parametrize("Hq,Hk,rows", [(2, 1, 1026), (6, 3, 343), (16, 8, 129)])
+@pytest.mark.parametrize("D,fp8", [(128, False), (64, True)])
+@pytest.mark.parametrize("longest", [192, 420])
+def test_decode_many_rows(Hq, Hk, rows, D, fp8, longest):
+    """1026 to 1032 (row, kv head) pairs: four of them share a workgroup where
+    none has more than six pages; the last four are not whole, and fours of
+    one and of three heads a row span rows of different lengths."""
+    g = torch.Generator().manual_seed(rows)
+    choice = torch.tensor([1, 20, 32, 33, 100, 160, 192, 193, 260, 420])
+    choice = choice[choice <= longest]
+    lens = choice[torch.randint(len(choice), (rows,), generator=g)]
+    lens[:40] = torch.where(lens[:40] > 192, 192, lens[:40])
+    lens[-1] = longest
+    args = _paged(lens.tolist(), [1] * rows, Hq, Hk, D, fp8, seed=rows)
+    got = ops.paged_attention(*(x.to(DEV) for x in args), 1.0 / math.sqrt(D),
+                              num_decodes_tail=rows)
+    _check(args, got)
