@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(SMP_THREADS) sampler_kernel(SmpArgs A) {
 //
 // Bound by instruction issue: four to count and sixteen to select per logit.
 // 1024 x 151,936 by the general kernel and here: 1382 -> 197 us (top_p 0.95 at
-// temperature 0.8), 1393 -> 151 with top_k 20, 148 -> 139 greedy, 1338 -> 250
+// temperature 0.8), 1393 -> 151 with top_k 20, 1338 -> 250
 // with a mask; one row 636 -> 41 us. Of the 50 us that a row takes its
 // workgroup 16 are fixed, clearing and scanning 128 KB of counters.
 #define CNT_MIN 2048
@@ -580,7 +580,6 @@ struct CountShared {
   u32 wave_alive[CNT_WAVES];
   float wave_z[CNT_WAVES];
   int max_pos, min_neg;         // magnitudes of the extremes
-  int odd;                      // a NaN or +inf was counted
   int seg[2];                   // where the count / the mass crosses
   u64 above[2];
   u32 tau[2];
@@ -677,6 +676,88 @@ sampler_count_kernel(SmpArgs A) {
       if (c < part) patch(r[c], bits[c], t0 + c * 512);
   };
 
+  // ---- greedy rows: the first of the largest, and Z, from the registers ----
+  // Nothing is counted. 1024 rows of 151,936 / 65,536 / 32,000 / 2048 logits: with
+  // counts 139 / 91 / 75 / 60 us, now 111 / 51 / 34 / 20 (the general kernel, of which
+  // more rows fit a CU, 153 / 53 / 30 / 8; one row 73 / 34 / 20 / 8 and here 24 / 13
+  // / 10 / 8).
+  if (greedy && tiles == 1) {
+    const int part = part_of(0), t0 = wave * part * 512 + lane * 8;
+    load(0);
+    float best = -INFINITY;
+    int ones = 0;      // logits that look like one that is not alive
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c)
+      if (c < part) {
+        int dead = 0;
+        if (MASKED || t0 + c * 512 + 8 > vl) {
+          u32 bits = bits8(t0 + c * 512);
+          const int left = vl - (t0 + c * 512);
+          if (left < 8) bits &= left > 0 ? (1u << left) - 1 : 0u;
+          dead = 8 - __popc(bits);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u32 w = r[c][j];
+          ones += ((w & 0xffffu) == 0xffffu) + (w >= 0xffff0000u);
+          best = fmaxf(best, fmaxf(__uint_as_float(w << 16),
+                                   __uint_as_float(w & 0xffff0000u)));
+        }
+        ones -= dead;
+      }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      best = fmaxf(best, __shfl_xor(best, off, 64));
+    if (lane == 0) sm.wave_z[wave] = best;
+    const bool odd = __ballot(ones != 0) != 0;
+    if (lane == 0) sm.wave_cnt[wave] = odd;
+    __syncthreads();
+    const int l16 = lane & (CNT_WAVES - 1);
+    best = sm.wave_z[l16];
+    u32 any = sm.wave_cnt[l16];
+#pragma unroll
+    for (int off = 1; off < CNT_WAVES; off <<= 1) {
+      best = fmaxf(best, __shfl_xor(best, off, CNT_WAVES));
+      any |= __shfl_xor(any, off, CNT_WAVES);
+    }
+    if (!any) {
+      float z = 0.f;
+      int first = 0x7fffffff;
+#pragma unroll
+      for (int c = 0; c < CNT_CHUNKS; ++c)
+        if (c < part)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const u32 w = r[c][j >> 1];
+            const u32 h = j & 1 ? w & 0xffff0000u : w << 16;
+            const float v = __uint_as_float(h);
+            z += h == 0xffff0000u ? 0.f : __expf(v - best);
+            if (v == best) first = min(first, t0 + c * 512 + j);
+          }
+      z = wave_sum(z);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1)
+        first = min(first, __shfl_xor(first, off, 64));
+      if (lane == 0) {
+        sm.seg_cnt[wave] = (u32)first;
+        sm.seg_cnt[CNT_WAVES + wave] = __float_as_uint(z);
+      }
+      __syncthreads();
+      if (tid == 0) {
+        z = 0.f;
+        for (int w = 0; w < CNT_WAVES; ++w) {
+          first = min(first, (int)sm.seg_cnt[w]);
+          z += __uint_as_float(sm.seg_cnt[CNT_WAVES + w]);
+        }
+        const bool none = best == -INFINITY;
+        A.out_tok[row] = none ? 0 : first;
+        A.out_lp[row] = none ? -INFINITY : -logf(z);
+      }
+      return;
+    }
+    __syncthreads();
+  }
+
   {
     u32x4* z = (u32x4*)sm.words;
 #pragma unroll
@@ -687,7 +768,6 @@ sampler_count_kernel(SmpArgs A) {
     if (tid == 0) {
       sm.max_pos = -1;
       sm.min_neg = 0x8000;
-      sm.odd = 0;
       sm.seg[0] = sm.seg[1] = -1;
       sm.tau[0] = sm.tau[1] = 0;
       sm.tcode = sm.one = 0x7fff;
@@ -735,10 +815,6 @@ sampler_count_kernel(SmpArgs A) {
   // segment j * CNT_WAVES + wave is this wave's, so that neighbours spread
   u32 present = 0;
   int max_pos = -1, min_neg = 0x8000;
-  if (tid < 0x80) {
-    const u32 w = sm.words[0x7f80 + tid];
-    if (tid ? w : w & 0xffffu) sm.odd = 1;
-  }
 #pragma unroll 4
   for (int j = 0; j < CNT_SEGS / CNT_WAVES; ++j) {
     const int mag0 = (j * CNT_WAVES + wave) * 64;
@@ -835,8 +911,8 @@ sampler_count_kernel(SmpArgs A) {
   // ... or zeros of both signs on top, of which the first is the maximum and
   // decides whether the other sign ranks below
   const bool zeros = pos && sm.max_pos == 0 && sm.min_neg == 0;
-  // ... or NaN or +inf, whose differences have no order
-  if (none || counted != want || (zeros && !greedy) || sm.odd) {
+  // ... or NaN or +inf (then Z is NaN), whose differences have no order
+  if (none || counted != want || (zeros && !greedy) || zf != zf) {
     __syncthreads();
     sample_row<true, CNT_THREADS>(A, row, tid,
                                   *(SmpShared<CNT_WAVES>*)cnt_lds);
