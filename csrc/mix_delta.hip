@@ -651,7 +651,7 @@ __global__ void delta_out_kernel(A* __restrict__ out, long ldo, int out_off,
 // The chain spent 64 instructions an output on readlane and FMA; 32,768 tokens
 // of 16 heads x 128 channels, rank 32: gates 516 -> 227 us
 // (what is left is exp and log1p), read-out 442 -> 140 us (2.9 TB/s).
-#define LR_TOK 128   // tokens per wave
+#define LR_TOK 128   // tokens per wave, at most
 
 __device__ __forceinline__ f32x4 lr_mfma(s16x8 a, s16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -694,19 +694,19 @@ __device__ __forceinline__ f32x4 lr_dot(const s16x8 (&w)[3], s16x8 x,
 }
 
 // grid (token groups, H, channel groups of 64); block of four waves, each with
-// its own LR_TOK tokens
+// its own `per` tokens
 __global__ void __launch_bounds__(WPB * WAVE) delta_gates_mfma_kernel(
     float* __restrict__ decay, float* __restrict__ beta,
     const u16* __restrict__ proj, long ld, int b_off, int a1_off,
     const float* __restrict__ a2t, int rank, const float* __restrict__ dt_bias,
-    const float* __restrict__ a_log, long T, int H, int dk) {
+    const float* __restrict__ a_log, long T, int H, int dk, int per) {
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int h = blockIdx.y, c0 = blockIdx.z * 64;
   const int lr = lane & 15, g = lane >> 4;
-  const long t_end0 = ((long)blockIdx.x * WPB + wid) * LR_TOK;
+  const long t_end0 = ((long)blockIdx.x * WPB + wid) * per;
   if (t_end0 >= T) return;
-  const long t_end = t_end0 + LR_TOK < T ? t_end0 + LR_TOK : T;
+  const long t_end = t_end0 + per < T ? t_end0 + per : T;
   const float rate = expf(a_log[h]);
   s16x8 w[4][3];
   f32x4 bias[4];
@@ -739,15 +739,15 @@ __global__ void __launch_bounds__(WPB * WAVE) delta_out_mfma_kernel(
     u16* __restrict__ out, long ldo, int out_off, const float* __restrict__ o,
     const float* __restrict__ norm_w, const u16* __restrict__ proj, long ld,
     int g1_off, const float* __restrict__ g2t, int rank, float eps,
-    float out_scale, long T, int H) {
+    float out_scale, long T, int H, int per) {
   constexpr int dv = NT * 16;
   const int lane = threadIdx.x & (WAVE - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int h = blockIdx.y;
   const int lr = lane & 15, g = lane >> 4;
-  const long t_end0 = ((long)blockIdx.x * WPB + wid) * LR_TOK;
+  const long t_end0 = ((long)blockIdx.x * WPB + wid) * per;
   if (t_end0 >= T) return;
-  const long t_end = t_end0 + LR_TOK < T ? t_end0 + LR_TOK : T;
+  const long t_end = t_end0 + per < T ? t_end0 + per : T;
   s16x8 w[NT][3];
 #pragma unroll
   for (int n = 0; n < NT; ++n)
@@ -789,6 +789,15 @@ static bool lr_fits(const void* proj, long ld, int off, int rank,
          (size_t)w2 % 4 == 0;
 }
 
+// Tokens a wave: 128 to read W2 seldom, fewer (whole tiles of 16) where that
+// leaves less than 4096 waves. With 128 always, 200 tokens of 16 heads x 128 took
+// 53 us for the inputs with their gates and 30 for the read-out (the readlane
+// chain 26 and 19), now 18 and 10; 8192 tokens of 8 heads 84 and 40, now 68 and 24.
+static int lr_tokens(long T, long groups) {
+  const long per = (T * groups + 4096 * 16 - 1) / (4096 * 16) * 16;
+  return per < 16 ? 16 : (per > LR_TOK ? LR_TOK : (int)per);
+}
+
 extern "C" void mix_delta_prep(
     float* qn, float* kn, float* vv, float* decay, float* beta,
     const void* proj, long ld, int q_off, int k_off, int v_off, int b_off,
@@ -809,12 +818,15 @@ extern "C" void mix_delta_prep(
   const dim3 ggrid((unsigned)((T + WPB * GT - 1) / (WPB * GT)), (unsigned)H);
   const bool lr = !f32 && a2 && dk % 64 == 0 && (size_t)decay % 16 == 0 &&
                   lr_fits(proj, ld, a1_off, rank, a2, dt_bias);
-  if (lr)
+  if (lr) {
+    const int per = lr_tokens(T, H * (dk / 64));
     hipLaunchKernelGGL(delta_gates_mfma_kernel,
-                       dim3((unsigned)((T + WPB * LR_TOK - 1) / (WPB * LR_TOK)),
+                       dim3((unsigned)((T + WPB * per - 1) / (WPB * per)),
                             (unsigned)H, (unsigned)(dk / 64)),
                        dim3(WPB * WAVE), 0, s, decay, beta, (const u16*)proj,
-                       ld, b_off, a1_off, a2, rank, dt_bias, a_log, T, H, dk);
+                       ld, b_off, a1_off, a2, rank, dt_bias, a_log, T, H, dk,
+                       per);
+  }
   const int Cq = G * dk, C = 2 * Cq + H * dv;
   const long su = (long)S * C;
   const int sgrid = (int)((su + 255) / 256);
@@ -953,12 +965,13 @@ extern "C" void mix_delta_out(void* out, long ldo, int out_off, const float* o,
       lr_fits(proj, ld, g1_off, rank, g2, norm_w)) {
     const auto fn = dv == 128 ? delta_out_mfma_kernel<8>
                               : delta_out_mfma_kernel<4>;
+    const int per = lr_tokens(T, H);
     hipLaunchKernelGGL(fn,
-                       dim3((unsigned)((T + WPB * LR_TOK - 1) / (WPB * LR_TOK)),
+                       dim3((unsigned)((T + WPB * per - 1) / (WPB * per)),
                             (unsigned)H),
                        dim3(WPB * WAVE), 0, s, (u16*)out, ldo, out_off, o,
                        norm_w, (const u16*)proj, ld, g1_off, g2, rank, eps,
-                       out_scale, T, H);
+                       out_scale, T, H, per);
   } else if (f32)
     hipLaunchKernelGGL(delta_out_kernel<float>, grid, dim3(WPB * WAVE),
                        0, s, (float*)out, ldo, out_off, o, norm_w,

@@ -69,3 +69,26 @@ def test_low_rank_gates(T, rank, dk, dv):
     got = got[:, 8:8 + H * dv].view(T, H, dv)
     ok = (got - want).abs() <= bound
     assert ok[:-1].all() and (got[-1] == 0).all()
+
+
+@pytest.mark.parametrize("T", [1400, 8191, 60000])   # 16, 32, 128 tokens a wave
+def test_tokens_of_a_wave(T):
+    """A token's gate does not depend on how many tokens its wave takes."""
+    H, dv, rank = 16, 64, 16
+    g = torch.Generator(device="cuda").manual_seed(T)
+    o = torch.randn(T, H, dv, generator=g, device="cuda")
+    proj = torch.randn(T, rank, generator=g, device="cuda").bfloat16()
+    g2 = torch.randn(H * dv, rank, generator=g, device="cuda")
+    norm_w = torch.randn(dv, generator=g, device="cuda")
+
+    def gate(rows):
+        out = torch.full((rows.stop - rows.start, H * dv), 7.0, device="cuda",
+                         dtype=torch.bfloat16)
+        hops.delta_out(o[rows], norm_w, proj[rows], 0, g2, 1e-5, out, 0, 1.0)
+        return out
+
+    whole = gate(slice(0, T))
+    for a in (0, 100, T // 2, T - 90):
+        rows = slice(a, min(a + 90, T))
+        assert torch.equal(whole[rows], gate(rows))
+    assert (whole != 7.0).any(1).all()
