@@ -410,7 +410,7 @@ class Qwen3MoE(nn.Module):
         k = self.top_k
         E_l, base = self.experts_per_rank, self.expert_base
         m_l = self.gate_up.shape[1] // 2
-        BM = (ops.expert_tile(T * k, self.num_experts, m_l, h)
+        BM = (ops.expert_tile(T * k, self.num_experts, m_l, h, local=E_l)
               if x.is_cuda else 64)
         ws = self._workspace(T, x.device)
         rows_max = T * k + (E_l + 1) * BM                 # static bound

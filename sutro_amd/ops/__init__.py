@@ -244,26 +244,40 @@ def linear_silu_mul(x, w):
 
 
 def expert_tile(n_rows: int, experts: int, inner: int, width: int,
-                gated: bool = True) -> int:
+                gated: bool = True, local: Optional[int] = None) -> int:
     """Rows that the segments of both expert GEMMs of a layer are padded to,
     for `n_rows` (token, expert) pairs in bf16 on the matrix cores (K and N
     multiples of 64), by the rows an expert gets on average. Taller tiles do
     more work per byte but pad more; both products together, at 32 experts of
-    2048 x 2048: at 96 rows 290 / 209 / 243 us on tiles of 64 / 128 / 256, at
-    187 rows 561 / 387 / 243, at 375 rows 1074 / 671 / 422.
+    2048 x 2048: at 96 rows 302 / 230 / 249 us on tiles of 64 / 128 / 256, at
+    192 rows 523 / 373 / 258, at 384 rows 1050 / 650 / 415.
+
+    They also leave fewer workgroups: 256 rows are one for 128 columns of the
+    gated product, and below about 320 the chip idles. 8 experts of 1024 x 512,
+    192 / 512 / 2048 rows an expert (24 / 64 / 256 workgroups of 256 rows) 35 /
+    52 / 115 us on 64, 41 / 47 / 113 on 128, 55 / 56 / 107 on 256; 8 of 2048 x
+    2048 at 384 rows (192) 223 / 147 / 180, 8 of 4096 x 3072 at 384 (288) 637 /
+    450 / 493 and at 512 (384) 800 / 561 / 499. Tiles of 128 want 128.
 
     Up to 16 rows, where the weights are all there is to read, tiles of 32: four
     workgroups of the gated product fit a CU instead of three. They are taken
     unless their number then fills the rounds worse: 1024 workgroups (2048 wide)
-    222 -> 200 us, 1536 (3072 wide, K 4096) 431 -> 445."""
+    222 -> 200 us, 1536 (3072 wide, K 4096) 431 -> 445.
+
+    `local`: the experts whose products this rank makes (all by default); its
+    workgroups are counted."""
+    local = experts if local is None else local
     avg = n_rows / experts
+    rows = avg * local
     if avg <= 16:
-        blocks = min(experts, n_rows) * (inner // 64)
+        blocks = min(local, max(1, round(rows))) * (inner // 64)
         if blocks <= 768 or -(-blocks // 1024) * 4 <= -(-blocks // 768) * 3:
             return 32
-    if avg >= 144 and inner % (128 if gated else 256) == 0 and width % 256 == 0:
+    cols = 128 if gated else 256
+    if (avg >= 144 and inner % cols == 0 and width % 256 == 0
+            and rows / 256 * (inner // cols) >= 320):
         return 256
-    return 128 if avg >= 72 else 64
+    return 128 if avg >= 72 and rows / 128 * (inner // 128) >= 128 else 64
 
 
 def grouped_gemm(out, a, w, row_tok, tile_off, counts, max_tiles, gate_silu,
