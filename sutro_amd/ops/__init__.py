@@ -252,12 +252,12 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
     2048 x 2048: at 96 rows 302 / 230 / 249 us on tiles of 64 / 128 / 256, at
     192 rows 523 / 373 / 258, at 384 rows 1050 / 650 / 415.
 
-    They also leave fewer workgroups: 256 rows are one for 128 columns of the
-    gated product, and below about 320 the chip idles. 8 experts of 1024 x 512,
-    192 / 512 / 2048 rows an expert (24 / 64 / 256 workgroups of 256 rows) 35 /
-    52 / 115 us on 64, 41 / 47 / 113 on 128, 55 / 56 / 107 on 256; 8 of 2048 x
-    2048 at 384 rows (192) 223 / 147 / 180, 8 of 4096 x 3072 at 384 (288) 637 /
-    450 / 493 and at 512 (384) 800 / 561 / 499. Tiles of 128 want 128.
+    They also leave fewer workgroups: one of 256 rows takes 128 columns of the
+    gated product or 256 of the other, and below 128 of them in either product
+    the chip idles. 8 experts of 1024 x 512, 192 / 512 / 1024 rows an expert (24 /
+    64 / 128 of either) 35 / 52 / 76 us on 64, 41 / 47 / 78 on 128, 55 / 56 / 61 on
+    256; 8 of 2048 x 2048 at 384 / 512 rows (96 / 128 of the second) 223 / 263 on
+    64, 147 / 208 on 128, 180 / 183 on 256. Tiles of 128 want 96.
 
     Up to 16 rows, where the weights are all there is to read, tiles of 32: four
     workgroups of the gated product fit a CU instead of three. They are taken
@@ -275,9 +275,9 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
             return 32
     cols = 128 if gated else 256
     if (avg >= 144 and inner % cols == 0 and width % 256 == 0
-            and rows / 256 * (inner // cols) >= 320):
+            and rows / 256 * min(inner // cols, width // 256) >= 128):
         return 256
-    return 128 if avg >= 72 and rows / 128 * (inner // 128) >= 128 else 64
+    return 128 if avg >= 72 and rows / 128 * (inner // 128) >= 96 else 64
 
 
 def grouped_gemm(out, a, w, row_tok, tile_off, counts, max_tiles, gate_silu,

@@ -72,20 +72,20 @@ def test_tile_rule(n_rows, want):
     from sutro_amd.ops import expert_tile
 
     # wide enough that every tile leaves enough workgroups
-    assert expert_tile(n_rows, 8, 16384, 256) == want
+    assert expert_tile(n_rows, 8, 16384, 16384) == want
     # widths the wide kernel does not take
-    assert expert_tile(n_rows, 8, 16384 + 64, 256) <= 128
-    assert expert_tile(n_rows, 8, 16384, 320) <= 128
-    assert expert_tile(n_rows, 8, 16384 + 128, 256, gated=False) <= 128
+    assert expert_tile(n_rows, 8, 16384 + 64, 16384) <= 128
+    assert expert_tile(n_rows, 8, 16384, 16384 + 64) <= 128
+    assert expert_tile(n_rows, 8, 16384 + 128, 16384, gated=False) <= 128
     # 1536 workgroups: two rounds of three a CU, but one and a half of four
     assert expert_tile(512, 32, 3072, 4096) == 64
 
 
 @pytest.mark.parametrize("experts,inner,width,avg,want", [
     (8, 512, 1024, 128, 64), (8, 512, 1024, 192, 64), (8, 512, 1024, 512, 128),
-    (8, 512, 1024, 2560, 256), (8, 2048, 2048, 192, 128),
-    (8, 2048, 2048, 384, 128), (8, 2048, 2048, 640, 256),
-    (8, 3072, 4096, 384, 128), (8, 3072, 4096, 512, 256),
+    (8, 512, 1024, 1024, 256), (8, 2048, 2048, 96, 128),
+    (8, 2048, 2048, 192, 128), (8, 2048, 2048, 384, 128),
+    (8, 2048, 2048, 512, 256), (8, 1024, 512, 1024, 128),
     (4, 512, 512, 768, 64), (32, 2048, 2048, 192, 256)])
 def test_tiles_that_leave_the_chip_busy(experts, inner, width, avg, want):
     """Few experts of small matrices: the tile that was measured as the faster
