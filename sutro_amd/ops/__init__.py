@@ -192,19 +192,35 @@ def _unwatched() -> bool:
                 or torch.compiler.is_compiling())
 
 
+def _two_rows(rows: int, K: int, gated: bool) -> bool:
+    return (rows * K <= (64 if gated else 24) << 20 or rows >= 16384
+            or (rows > 8192 and K <= 5120) or (rows < 8192 and K >= 16384))
+
+
 def _few_rows(x, w, gated: bool = False) -> bool:
     """Whether csrc/gemm_skinny.hip is the faster one for x [M, K] w^T. The
     library takes 11 us or more for any product; us by it and by the kernel,
     weights from memory:
-      rows of w x K    M = 1          3             16            32
-      2048 x 2048      10.9 /  4.8    11.0 /  5.3   11.0 /  6.5   11.2 /  8.7
-      3072 x 2048      11.3 /  5.1    11.3 /  5.5   11.2 /  6.7   11.5 /  8.9
-      2048 x 3072      12.1 /  5.2    12.1 /  7.0   12.1 /  9.3   10.2 / 13.8
-      4096 x 4096      15.4 /  7.7    15.5 /  9.6   15.5 / 12.5   13.1 / 17.4
-      2048 x 8192      12.7 /  8.1    12.6 / 15.5   13.0 / 22.0
-      6144 x 4096      15.6 / 10.7    14.6 / 15.8   14.2 / 22.3
-      32768 x 4096     61.5 / 48.8    61.7 / 65.6   62.0 / 70.5
-    and with silu_mul behind it 16384 x 2048: 19.6 / 14.0 for one row."""
+      rows of w x K    M = 1          2             3             16            32
+      2048 x 2048      11.0 /  4.8    10.7 /  5.9   10.7 /  5.2   10.7 /  6.4   10.9 /  8.6
+      3072 x 2048      11.5 /  5.1    11.1 /  6.5   11.1 /  5.6   11.0 /  6.7   11.2 /  9.0
+      2048 x 3072      12.1 /  5.2    11.9 /  6.3   11.9 /  7.1   11.8 /  9.3   10.1 / 13.9
+      4096 x 4096      15.4 /  7.8    15.2 / 10.0   15.2 /  9.7   15.4 / 12.4   13.0 / 17.3
+      2048 x 8192      12.6 /  8.2    12.5 / 10.2   12.4 / 15.4   13.0 / 21.8
+      6144 x 4096      15.6 / 10.9    15.3 / 13.0   14.3 / 16.0   14.3 / 22.1
+      5120 x 5120      13.6 / 12.0    13.9 / 14.8   13.7 / 17.4   15.2 / 24.9
+      8192 x 4096      17.1 / 14.7    16.5 / 18.3
+      12288 x 5120     26.8 / 23.9    25.9 / 25.7
+      12288 x 12288    61.0 / 60.6    60.7 / 64.9
+      5120 x 25600      135 / 51       136 / 57      136 / 79      139 / 116
+      32768 x 4096     63.2 / 49.5    62.9 / 56.1   63.1 / 67.0   60.9 / 69.1
+    and with silu_mul behind it (rows of both halves)
+      4096 x 2048      13.8 /  5.6    13.6 /  7.0   13.6 /  8.4   13.9 /  9.7   13.9 / 13.4
+      16384 x 2048     20.8 / 14.0    20.3 / 17.6   20.4 / 17.5   20.6 / 21.1   19.3 / 24.1
+      12288 x 8192     43.9 / 42.4    43.8 / 47.5
+      51200 x 5120     98.8 / 92.3    99.1 / 95.9   99.3 / 143
+    Two rows lose where the library has a good tile (24 to 64 M weights of long
+    rows) and one load a weight row is no longer the whole cost."""
     if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False
@@ -212,7 +228,8 @@ def _few_rows(x, w, gated: bool = False) -> bool:
         return False
     M, K = x.shape
     rows = w.shape[0]
-    fits = (M <= 2 or (M <= 16 and K <= 4096 and rows * K <= 1 << 24)
+    fits = (M == 1 or (M == 2 and _two_rows(rows, K, gated))
+            or (M <= 16 and K <= 4096 and rows * K <= 1 << 24)
             or (K <= 2048 and rows * K <= 1 << 23))
     return (fits and _unwatched() and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.device == x.device

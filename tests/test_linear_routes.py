@@ -135,3 +135,15 @@ def test_hooks_on_every_module():
         for h in handles:
             h.remove()
     assert L.bare(mlp.gate_up_proj)
+
+
+@pytest.mark.parametrize("rows,k,n,gated,kernel", [
+    (1, 5120, 5120, False, 1), (2, 5120, 5120, False, 0),
+    (2, 4096, 6144, False, 1), (2, 4096, 8192, False, 0),
+    (2, 5120, 10240, False, 1), (2, 16384, 4096, False, 1),
+    (2, 8192, 6144, True, 1), (2, 8192, 12288, True, 0)])
+def test_one_and_two_rows(kernels, rows, k, n, gated, kernel):
+    """Two rows over matrices where the library is the faster one."""
+    w = torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
+    assert ops._few_rows(torch.empty(rows, k, dtype=torch.bfloat16), w,
+                         gated) == bool(kernel)
