@@ -87,6 +87,9 @@ __device__ __forceinline__ pa_frag pa_pack8(pa_f32x8 v) {
 __device__ __forceinline__ u32x2 pa_pack4(f32x4 v) {
   return __builtin_bit_cast(u32x2, __builtin_convertvector(v, pa_bf16x4));
 }
+__device__ __forceinline__ int pa_same(int v) {
+  return __builtin_amdgcn_readfirstlane(v);
+}
 // an entry of the block table, through the scalar cache (no kernel writes it)
 __device__ __forceinline__ int pa_entry(const int* p, int i) {
   return ((const __attribute__((address_space(4))) int*)p)[i];
@@ -160,15 +163,18 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 // 32 k prompt (16 heads, 4 kv heads, 128; useful flops) and 250 on prompts of
 // 2 k; this one at 860 and 640 (13.1 -> 5.1 ms, 1.10 -> 0.43 ms), 0.78 instead
 // of 1.61 ms on 7 prompts of 3 k with 32 heads over e4m3 pages, 0.11 instead of
-// 0.22 ms on 160 short ones (24 k tokens). Two workgroups a CU (68 KB of LDS,
+// 0.22 ms on 160 short ones (24 k tokens). Two workgroups a CU (64 KB of LDS,
 // up to 256 registers a lane) are what both limits allow.
+//
+// BLOCKS: more than one block of rows in a workgroup.
 //
 // Entries of the tile map that continue each other (same sequence, 32 rows on)
 // share a workgroup; the entry at a multiple of rpb, or one that continues
 // nothing, leads.
 // ---------------------------------------------------------------------------
-template <int D, bool KV8, bool LOCAL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int D, bool KV8, bool LOCAL, bool BLOCKS, int WAVES_PER_SIMD>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(WAVES_PER_SIMD, WAVES_PER_SIMD)))
 paged_prefill_kernel(PagedArgs A) {
   constexpr int CPR = D / 8;                // 16-byte chunks per row
   constexpr int TILE = PA_KEYS * D * 2;     // bytes of a K or V tile
@@ -182,7 +188,8 @@ paged_prefill_kernel(PagedArgs A) {
   const int hgroups = A.Hq / A.hpb;
   const int hg = blockIdx.x % hgroups;
   const int e = A.n_tiles - 1 - blockIdx.x / hgroups;
-  const int s = A.tile_seq[e], q0 = A.tile_q0[e];
+  // (the same for all lanes: kept in scalar registers)
+  const int s = pa_same(A.tile_seq[e]), q0 = pa_same(A.tile_q0[e]);
   const int k0 = (q0 >> 5) % A.rpb;
   if (k0 > 0 && e > 0 && A.tile_seq[e - 1] == s && A.tile_q0[e - 1] == q0 - 32)
     return;
@@ -193,11 +200,12 @@ paged_prefill_kernel(PagedArgs A) {
   const int hq = hg * A.hpb + w % A.hpb, rb = w / A.hpb;
   const int kh = hg * A.hpb / (A.Hq / A.Hk);
 
-  const int nq_total = A.qlocs[s + 1] - A.qlocs[s];
+  const int q_first = pa_same(A.qlocs[s]);
+  const int nq_total = pa_same(A.qlocs[s + 1]) - q_first;
   const int rows = min(cnt * 32, nq_total - q0);   // of the workgroup
   if (rows <= 0) return;                    // a padding entry
-  const int row_base = A.qlocs[s] + q0;
-  const int L = A.seq_lens[s];
+  const int row_base = q_first + q0;
+  const int L = pa_same(A.seq_lens[s]);
   const int p0 = L - nq_total + q0;         // position of the first row
   const int kv_end = p0 + rows;             // causal bound (exclusive)
   const int my_r = rb * 32 + ln;            // this lane's row of the workgroup
@@ -323,16 +331,30 @@ paged_prefill_kernel(PagedArgs A) {
   load();
   if (steps > 1) pages(step_tile(1));
   store(pa_smem, step_tile(0) * PA_KEYS);
-  *(u32x2*)(pa_smem + 4 * TILE + threadIdx.x * (D / 8)) = u32x2{0u, 0u};
-  if (D == 128)
-    *(u32x2*)(pa_smem + 4 * TILE + threadIdx.x * (D / 8) + 8) = u32x2{0u, 0u};
+  if (BLOCKS)
+#pragma unroll
+    for (int z = 0; z < D / 64; ++z)
+      *(u32x2*)(pa_smem + 4 * TILE + threadIdx.x * (D / 8) + z * 8) =
+          u32x2{0u, 0u};
   for (int it = 0; it < steps; ++it) {
     __syncthreads();
     const int kv0 = step_tile(it) * PA_KEYS;
     const bool more = it + 1 < steps;
     if (more) load();
     if (it + 2 < steps) pages(step_tile(it + 2));
-    if (live && kv0 < w_end) {
+    // With several row blocks in the workgroup a step may be for the rows of
+    // others: which of its four times 16 keys does a row of this wave see?
+    u32 seen = 15;
+    if (BLOCKS) {
+      auto below = [&](int key) {       // the sixteens that begin before `key`
+        return (1u << min(max((key - kv0 + 15) >> 4, 0), 4)) - 1;
+      };
+      seen = below(w_end);
+      if (LOCAL)
+        seen &= ~below(w_lo - 15) | (below(A.keep_first) & ~below(w_c - 15));
+    }
+    const bool mine = live && seen;
+    if (mine) {
     const char* kb = pa_smem + (it & 1) * 2 * TILE;
     const char* vb = kb + TILE;
 
@@ -407,13 +429,8 @@ paged_prefill_kernel(PagedArgs A) {
         sum += p[j];
       }
       const pa_frag pb = pa_pack8(p);
-      // 16 keys that no row of this wave sees: zeros for values
-      const int key0 = kv0 + ks * 16;
-      bool blind = key0 >= w_end;
-      if (LOCAL)
-        blind |= (key0 + 16 <= w_lo) &
-                 ((key0 >= A.keep_first) | (key0 + 16 <= w_c));
-      const char* vk = blind ? pa_smem + 4 * TILE : vb + ks * 16 * 2 * D;
+      const char* vk = vb + ks * 16 * 2 * D;
+      if (BLOCKS) vk = seen & (1u << ks) ? vk : pa_smem + 4 * TILE;
 #pragma unroll
       for (int b = 0; b < D / 32; ++b) {
         const char* at = vk + vad[b & 1] + (b >> 1) * 128;
@@ -901,21 +918,40 @@ static inline int pa_splits(long rows, int Hk, int max_pages) {
   return n < 1 ? 1 : (int)n;
 }
 
+template <int D, bool KV8, bool LOCAL, bool BLOCKS, int WAVES_PER_SIMD>
+static inline void pa_start_prefill(const PagedArgs& A, hipStream_t s) {
+  // K and V twice, and zeros for 16 keys
+  const size_t smem =
+      2 * 2 * (size_t)PA_KEYS * D * 2 + (BLOCKS ? 16 * D * 2 : 0);
+  const auto kernel =
+      paged_prefill_kernel<D, KV8, LOCAL, BLOCKS, WAVES_PER_SIMD>;
+  static std::atomic<unsigned long long> asked{0};
+  if (smem > 65536) lds_limit((const void*)kernel, (int)smem, asked);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)A.n_tiles * (A.Hq / A.hpb)),
+                     dim3(256), smem, s, A);
+}
+
+// n_seqs: prompts that the tile map is of
 template <int D, bool KV8, bool LOCAL>
-static inline void pa_launch_prefill(PagedArgs A, hipStream_t s) {
+static inline void pa_launch_prefill(PagedArgs A, int n_seqs, hipStream_t s) {
   // K and V are read once for 128 rows: 4, 2 or 1 query heads (what divides
   // their group) times 1, 2 or 4 row blocks
   const int G = A.Hq / A.Hk;
   A.hpb = G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
   A.rpb = 4 / A.hpb;
-  const size_t smem = 2 * 2 * (size_t)PA_KEYS * D * 2 + 16 * D * 2;
-  static std::atomic<unsigned long long> asked{0};
-  if (smem > 65536)
-    lds_limit((const void*)paged_prefill_kernel<D, KV8, LOCAL>, (int)smem,
-              asked);
-  hipLaunchKernelGGL((paged_prefill_kernel<D, KV8, LOCAL>),
-                     dim3((unsigned)A.n_tiles * (A.Hq / A.hpb)),
-                     dim3(256), smem, s, A);
+  // Heads of 64 leave room for four workgroups a CU in 128 registers. Many short
+  // prompts, a few steps each with nothing to overlap them, are faster that way:
+  // 128 of 100 tokens, 8 heads and kv heads 50 -> 37 us, 160 of 150, 14 and 2
+  // heads, 63 -> 45; long ones (2000 tokens 38 -> 40) and few are not.
+  if constexpr (D == 64 && !LOCAL) {
+    if ((long)A.n_tiles * (A.Hq / A.hpb) >= 512 && A.n_tiles <= 8 * n_seqs) {
+      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 4>(A, s);
+      else pa_start_prefill<D, KV8, LOCAL, true, 4>(A, s);
+      return;
+    }
+  }
+  if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 2>(A, s);
+  else pa_start_prefill<D, KV8, LOCAL, true, 2>(A, s);
 }
 
 // max_pages: of a row at most (by the table, the window or the chunk)

@@ -8,9 +8,9 @@ extern "C" void sutro_attn_prefill(void* out, const void* q,
                                    const int* block_tables,
                                    const int* seq_lens, const int* qlocs,
                                    const int* tile_seq, const int* tile_q0,
-                                   int n_tiles, int bt_stride, int Hq, int Hk,
-                                   int head_dim, int kv_fp8, float scale,
-                                   hipStream_t s) {
+                                   int n_tiles, int n_seqs, int bt_stride, int Hq,
+                                   int Hk, int head_dim, int kv_fp8,
+                                   float scale, hipStream_t s) {
   if (n_tiles == 0) return;
   PagedArgs A = {};
   A.out = (u16*)out;
@@ -29,11 +29,11 @@ extern "C" void sutro_attn_prefill(void* out, const void* q,
   A.tile_q0 = tile_q0;
   A.n_tiles = n_tiles;
   if (head_dim == 128) {
-    if (kv_fp8) pa_launch_prefill<128, true, false>(A, s);
-    else pa_launch_prefill<128, false, false>(A, s);
+    if (kv_fp8) pa_launch_prefill<128, true, false>(A, n_seqs, s);
+    else pa_launch_prefill<128, false, false>(A, n_seqs, s);
   } else {
-    if (kv_fp8) pa_launch_prefill<64, true, false>(A, s);
-    else pa_launch_prefill<64, false, false>(A, s);
+    if (kv_fp8) pa_launch_prefill<64, true, false>(A, n_seqs, s);
+    else pa_launch_prefill<64, false, false>(A, n_seqs, s);
   }
 }
 

@@ -35,7 +35,7 @@ void sutro_attn_decode(void*, const void*, const void*, const void*,
 int sutro_attn_decode_splits(int, int, int);
 void sutro_attn_prefill(void*, const void*, const void*, const void*,
                         const int*, const int*, const int*, const int*,
-                        const int*, int, int, int, int, int, int, float,
+                        const int*, int, int, int, int, int, int, int, float,
                         hipStream_t);
 void sutro_mfma32_probe(float*, const void*, const void*, hipStream_t);
 void sutro_gemm_tn_launch(void*, const void*, const void*, const void*, int,
@@ -140,7 +140,7 @@ void paged_attention(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                        v_cache.data_ptr(), block_tables.data_ptr<int>(),
                        seq_lens.data_ptr<int>(), qlocs.data_ptr<int>(),
                        tile_seq.data_ptr<int>(), tile_q0.data_ptr<int>(),
-                       n_tiles, bt_stride, Hq, Hk, D,
+                       n_tiles, S - (int)num_decodes, bt_stride, Hq, Hk, D,
                        is_fp8(k_cache) ? 1 : 0, (float)scale, cur_stream());
   }
   if (num_decodes > 0) {

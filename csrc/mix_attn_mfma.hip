@@ -134,9 +134,13 @@ local_attention_mfma_kernel(
         *(u16x8*)((char*)ktile + kswz<DKP>(row, slot * 16)) = kx;
       }
       for (int it = tid; it < PG * VS; it += nthr) {
-        const int kv = it % PG, d0 = (it / PG) * 8;
+        const int kv = it % PG, d0 = (it / PG) * 8, key = kv0 + kv;
+        // zeros for keys that no row of the tile sees: their weight is 0, but
+        // what lies there may be infinite or NaN
+        const bool seen = key < kv_end && (key >= lo_tile ||
+                                           (key < keep_first && key >= clo_tile));
         u16x8 vx = (u16x8)(0);
-        if (d0 < dv) vx = *(const u16x8*)(vp + kv * ldv + d0);
+        if (d0 < dv && seen) vx = *(const u16x8*)(vp + kv * ldv + d0);
 #pragma unroll
         for (int j = 0; j < 8; ++j) vt[(d0 + j) * VPAD + kv] = vx[j];
       }

@@ -77,8 +77,8 @@ extern "C" void mix_paged_attention(
   A.gate_n = gate_n;
   A.out_scale = out_scale;
   if (n_tiles > 0) {
-    if (D == 128) pa_launch_prefill<128, false, true>(A, s);
-    else pa_launch_prefill<64, false, true>(A, s);
+    if (D == 128) pa_launch_prefill<128, false, true>(A, 0, s);
+    else pa_launch_prefill<64, false, true>(A, 0, s);
   }
   if (n_rows > 0) {
     const int most = most_pages(bt_stride, chunk, window, keep_first);

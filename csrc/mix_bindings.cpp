@@ -3,6 +3,7 @@
 // stream go to the extern "C" launchers in mix_*.hip. Activation tensors are
 // bf16 or fp32 (all of one call the same); recurrence inputs, norm weights
 // and the residual stream are fp32.
+#include <algorithm>
 #include <torch/extension.h>
 
 #include <hip/hip_runtime.h>
@@ -382,6 +383,22 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
       (size_t)out.data_ptr() % 8 == 0 && (size_t)q.data_ptr() % 16 == 0 &&
       (size_t)k_cache.data_ptr() % 16 == 0 &&
       (size_t)v_cache.data_ptr() % 16 == 0;
+  // Prompts with heads of 64 and a chunk or window of a few of the 32-row blocks
+  // that a workgroup of the paged kernel has (1, 2 or 4 by the group's heads):
+  // many of its steps are for the rows of one block only, and where there are
+  // enough tiles to fill the chip the other kernel, a workgroup a block, is the
+  // faster one. 128 prompts of 100 tokens, 8 heads and kv heads: chunk 32 / 64 /
+  // 128 23 / 31 / 46 us against 60 / 60 / 57 (4 and 2 heads 11 / 14 / 18 against 17
+  // / 17 / 16), window 32 / 64 31 / 40 against 59 / 59; 3 heads, window 64, 21
+  // against 15.
+  const long group = H / G;
+  const long blocks = group % 4 == 0 ? 1 : (group % 2 == 0 ? 2 : 4);
+  const long reach = std::max(32l, 16 * blocks);
+  const long entries =
+      (tile_seq.has_value() ? tile_seq->numel() : 0) * H * blocks / 4;
+  const bool narrow = dk == 64 &&
+                      ((chunk > 0 && chunk <= reach && entries >= 1024) ||
+                       (window > 0 && window <= reach && entries >= 2048));
   auto run_paged = [&](int tiles, const int* ts, const int* tq, long first,
                        long n) {
     const int ns = n > 0 ? mix_paged_splits(n, (int)G, (int)bt.size(1),
@@ -411,7 +428,7 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
     CHECK_I32(*tile_seq); CHECK_I32(*tile_q0);
     TORCH_CHECK(tile_seq->numel() == tile_q0->numel() && prefill_rows <= T,
                 "tile map sizes");
-    if (paged) {
+    if (paged && !narrow) {
       run_paged((int)tile_seq->numel(), tile_seq->data_ptr<int>(),
                 tile_q0->data_ptr<int>(), 0, 0);
       t0 = prefill_rows;

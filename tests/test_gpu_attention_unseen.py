@@ -154,3 +154,61 @@ def test_layer_list_attention(Hq, Hk, D, chunk, window, keep, prompt):
         return out
 
     _same(run, pg, unseen)
+
+
+@pytest.mark.parametrize("Hq,Hk,chunk,window,keep", [
+    (8, 8, 32, 0, 0), (8, 8, 0, 40, 9), (6, 2, 64, 0, 0), (4, 1, 32, 0, 0)])
+def test_many_narrow_prompts(Hq, Hk, chunk, window, keep):
+    """Enough prompts with heads of 64 and a narrow chunk or window to leave the
+    kernel of 128 rows a workgroup: against the reference, and with what no
+    32-row block sees poisoned."""
+    from sutro_amd.ops import torch_ref as R
+
+    D, S = 64, 140
+    g = torch.Generator().manual_seed(Hq)
+    new = torch.randint(33, 97, (S,), generator=g).tolist()
+    lens = [n + int(c) for n, c in
+            zip(new, torch.randint(0, 40, (S,), generator=g))]
+    if keep:
+        lens[3] = new[3] + 200
+    pg = Pages(lens, Hk, D, seed=1)
+    T = sum(new)
+    q = torch.randn(T, Hq, D, generator=g).bfloat16()
+    proj = torch.randn(T, 16, generator=g).bfloat16()
+    sl = torch.tensor(lens, dtype=torch.int32)
+    ql = torch.tensor([0] + new).cumsum(0).int()
+    ts = torch.tensor([s for s in range(S) for _ in range(0, new[s], 32)]).int()
+    tq = torch.tensor([j for c in new for j in range(0, c, 32)]).int()
+    seq = torch.repeat_interleave(torch.arange(S), torch.tensor(new)).int()
+    hpb = 4 if Hq // Hk % 4 == 0 else (2 if Hq // Hk % 2 == 0 else 1)
+    assert ts.numel() * Hq // hpb >= (2048 if window else 1024) or Hq // Hk == 4
+    unseen = []
+    for s, n in enumerate(lens):
+        seen = torch.zeros((n // 32 + 2) * 32, dtype=torch.bool)
+        for p in range(n - new[s], n):
+            lo = p // chunk * chunk if chunk else 0
+            kept = lo
+            if window:
+                lo = max(lo, p - window + 1)
+            seen[lo:p + 1] = True
+            seen[kept:max(kept, min(keep, p + 1))] = True
+        unseen += [(s, p) for p in range(seen.numel()) if not seen[p]]
+    d = [x.to(DEV) for x in (q, pg.bt, sl, ql, proj, seq, ts, tq)]
+
+    def run(k, v):
+        out = torch.zeros(T, Hq * D, dtype=torch.bfloat16, device=DEV)
+        hops.local_attention(d[0], k, v, d[1], d[2], d[3], D ** -0.5, chunk,
+                             window, d[4], -1, out, 0, 1.0, token_seq=d[5],
+                             tile_seq=d[6], tile_q0=d[7], prefill_rows=T,
+                             keep_first=keep)
+        return out
+
+    _same(run, pg, unseen)
+    k, v = (x.cpu().float() for x in pg.with_unseen([], 0.0))
+    want = torch.zeros(T, Hq * D)
+    R.local_attention(q.float(), k, v, pg.bt, sl, ql, D ** -0.5, chunk, window,
+                      proj, -1, want, 0, 1.0, keep_first=keep)
+    got = run(*pg.with_unseen([], 0.0)).float().cpu()
+    # weights and results are rounded to bf16 once each
+    bound = 2.0 ** -8 * v.abs().max().item() + 1e-3
+    assert (got - want).abs().max().item() < bound
