@@ -35,14 +35,57 @@ def _paged(lens, new, Hq, Hk, D, fp8, spare=0, seed=0):
 
 
 def _check(args, got):
+    """Weights p and results are rounded to bf16 once each, 2^-8 of sum(p |v|)
+    at most, element by element; 2^-12 is for scores of up to 20 in 32 bits."""
     q, kc, vc, bt, sl, ql = args
-    ref = R.paged_attention(q.float(), kc.float(), vc.float(), bt, sl, ql,
-                            1.0 / math.sqrt(q.shape[2]))
-    # weights and results are rounded to bf16 once each (2^-9 of a convex sum
-    # of values, which is at most the largest value)
-    bound = 2.0 ** -8 * vc.float().abs().max().item() + 1e-3
-    err = (got.float().cpu() - ref).abs().max().item()
-    assert err < bound, (err, bound)
+    ref, size = (R.paged_attention(q.float(), kc.float(), v, bt, sl, ql,
+                                   1.0 / math.sqrt(q.shape[2]))
+                 for v in (vc.float(), vc.float().abs()))
+    bound = (2.0 ** -7 + 2.0 ** -12) * size
+    err = (got.float().cpu() - ref).abs()
+    assert (err <= bound).all(), (err / bound).max().item()
+    return ref, bound
+
+
+RUN = 256    # keys of a run
+
+
+def _plant(args):
+    """A key of weight exp(14) in every run of every sequence (single tokens),
+    for one head of each group that has another, so that no run can be left out
+    or counted twice unseen."""
+    q, kc, vc, bt, sl, ql = args
+    Hk, D = kc.shape[1], kc.shape[3]
+    G = q.shape[1] // Hk
+    for s, n in enumerate(sl.tolist()):
+        runs = (n + RUN - 1) // RUN
+        for r in range(runs):
+            p = min(r * RUN + 37 * r % RUN, n - 1)
+            head = q[s].view(Hk, G, D)[:, r % max(min(G, runs // 2), 1)].float()
+            key = head * (14 * math.sqrt(D) / head.square().sum(-1, keepdim=True))
+            kc[int(bt[s, p // 32]), :, p % 32] = key.to(kc.dtype)
+
+
+def _assert_runs_show(args, ref, bound):
+    """Leaving out or doubling any run moves the reference past the bound."""
+    q, kc, vc, bt, sl, ql = args
+    Hk, D = kc.shape[1], kc.shape[3]
+    G = q.shape[1] // Hk
+    for s, n in enumerate(sl.tolist()):
+        runs = (n + RUN - 1) // RUN
+        if runs < 2:
+            continue
+        pages = bt[s, :(n + 31) // 32].long()
+        k, v = (x[pages].float().transpose(0, 1).reshape(Hk, -1, D)[:, :n]
+                for x in (kc, vc))
+        z = q[s].float().view(Hk, G, D) @ k.transpose(1, 2) / math.sqrt(D)
+        p = (z - z.amax(-1, keepdim=True)).exp()
+        for r in range(runs):
+            for times in (0.0, 2.0):
+                w = p.clone()
+                w[:, :, r * RUN:(r + 1) * RUN] *= times
+                o = (w @ v / w.sum(-1, keepdim=True)).view(Hk * G, D)
+                assert ((o - ref[s]).abs() > 2 * bound[s]).any(), (s, r, times)
 
 
 @pytest.mark.parametrize("Hq,Hk,D,fp8", [
@@ -53,12 +96,17 @@ def _check(args, got):
     ([255, 256, 257, 3], 40),      # 8 pages = one run; wide tables
     ([2049, 40, 8191], 5),         # many runs beside a single one
 ])
-def test_decode_runs(Hq, Hk, D, fp8, lens, spare):
+@pytest.mark.parametrize("planted", [False, True])
+def test_decode_runs(Hq, Hk, D, fp8, lens, spare, planted):
     args = _paged(lens, [1] * len(lens), Hq, Hk, D, fp8, spare, seed=D + Hq)
+    if planted:
+        _plant(args)
     q, kc, vc, bt, sl, ql = (x.to(DEV) for x in args)
     got = ops.paged_attention(q, kc, vc, bt, sl, ql, 1.0 / math.sqrt(D),
                               num_decodes_tail=len(lens))
-    _check(args, got)
+    ref, bound = _check(args, got)
+    if planted:
+        _assert_runs_show(args, ref, bound)
 
 
 def _tiles(new):
