@@ -220,9 +220,10 @@ def test_delta_rule_ops(dtype, H, G, dk, dv, taps, rank):
     (16, 1, 64, 64, 0, 0),
 ])
 def test_local_attention_matrix_core_path(H, G, dk, dv, chunk, window):
-    """bf16, page 32: prompt pieces run on the MFMA kernel (tile map given),
-    trailing single-token rows on the generic kernel; both against the fp32
-    reference. Pieces start inside pages and inside chunks."""
+    """bf16, page 32, a tile map: equal key and value sizes of 64 or 128 run on the
+    paged kernels; the others run prompt pieces on the MFMA kernel and trailing
+    single-token rows on the generic one. All against the fp32 reference. Pieces
+    start inside pages and inside chunks."""
     dtype = torch.bfloat16
     page, n_blocks = 32, 41
     g = torch.Generator().manual_seed(13)
