@@ -490,10 +490,10 @@ paged_prefill_kernel(PagedArgs A) {
 // loaded and then computed, took 1.9 us a page; a call now takes (with the
 // join) 28 us instead of 2390 for one row of 40 k keys and 4 kv heads (82 MB,
 // 3 TB/s), 24 instead of 314 for 7 rows of 3 k e4m3 keys and 8 heads, 24
-// instead of 128 for 16 rows of 2 k keys and 4 heads, and 37 instead of 41 for
-// 256 rows of 130 keys and 8 heads (138 MB, 3.7 TB/s, one run each). Runs of 8
-// pages give every wave two pages, the fewest that hide one load behind
-// another's work.
+// instead of 128 for 16 rows of 2 k keys and 4 heads, and 33 instead of 41 for
+// 256 rows of 130 keys and 8 heads (138 MB, 4.1 TB/s; a wave each, see below).
+// Runs of 8 pages give every wave two pages, the fewest that hide one load
+// behind another's work.
 //
 // Many rows over short contexts are bound by the workgroups themselves: two of
 // them fit a CU, and one that has a page or two leaves most of its waves idle.
