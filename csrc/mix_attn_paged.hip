@@ -30,13 +30,13 @@ extern "C" int mix_paged_splits(long rows, int Hk, int bt_stride, int chunk,
                    most_pages(bt_stride, chunk, window, keep_first));
 }
 
-// prompt pieces of n_tiles entries of the tile map, then the n_rows single
+// prompt pieces of n_tiles entries of the tile map (n_prompts of them), then the n_rows single
 // tokens from row t0 on (either may be none)
 extern "C" void mix_paged_attention(
     void* out, long ldo, int out_off, const void* q, const void* k_cache,
     const void* v_cache, const int* bt, int bt_stride, const int* seq_lens,
     const int* qlocs, const int* tile_seq, const int* tile_q0, int n_tiles,
-    const int* token_seq, long t0, int n_rows, int nsplit, float* part_o,
+    int n_prompts, const int* token_seq, long t0, int n_rows, int nsplit, float* part_o,
     float* part_ml, float scale, int chunk, int window, const void* proj,
     long ld, int gate_off, int gate_n, float out_scale, const float* bias_r1,
     const float* bias_r2, int sink, const float* sink_w, int keep_first, int H,
@@ -77,8 +77,8 @@ extern "C" void mix_paged_attention(
   A.gate_n = gate_n;
   A.out_scale = out_scale;
   if (n_tiles > 0) {
-    if (D == 128) pa_launch_prefill<128, false, true>(A, 0, s);
-    else pa_launch_prefill<64, false, true>(A, 0, s);
+    if (D == 128) pa_launch_prefill<128, false, true>(A, n_prompts, s);
+    else pa_launch_prefill<64, false, true>(A, n_prompts, s);
   }
   if (n_rows > 0) {
     const int most = most_pages(bt_stride, chunk, window, keep_first);

@@ -63,9 +63,9 @@ int mix_local_attention_mfma(void*, long, int, const void*, const void*,
 int mix_paged_splits(long, int, int, int, int, int);
 void mix_paged_attention(void*, long, int, const void*, const void*,
                          const void*, const int*, int, const int*, const int*,
-                         const int*, const int*, int, const int*, long, int,
-                         int, float*, float*, float, int, int, const void*,
-                         long, int, int, float, const float*, const float*,
+                         const int*, const int*, int, int, const int*, long,
+                         int, int, float*, float*, float, int, int,
+                         const void*, long, int, int, float, const float*, const float*,
                          int, const float*, int, int, int, int, hipStream_t);
 int mix_latent_splits(long, int, int, int, int, int, int);
 int mix_latent_attention(void*, long, int, const void*, const void*,
@@ -394,6 +394,7 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
   const long group = H / G;
   const long blocks = group % 4 == 0 ? 1 : (group % 2 == 0 ? 2 : 4);
   const long reach = std::max(32l, 16 * blocks);
+  const long n_prompts = std::max(0l, seq_lens.numel() - (T - prefill_rows));
   const long entries =
       (tile_seq.has_value() ? tile_seq->numel() : 0) * H * blocks / 4;
   const bool narrow = dk == 64 &&
@@ -415,7 +416,7 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
         out.data_ptr(), out.stride(0), (int)out_off, q.data_ptr(),
         k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr<int>(),
         (int)bt.size(1), seq_lens.data_ptr<int>(), qlocs.data_ptr<int>(), ts,
-        tq, tiles, token_seq.data_ptr<int>(), first, (int)n, ns,
+        tq, tiles, (int)n_prompts, token_seq.data_ptr<int>(), first, (int)n, ns,
         ns > 1 ? po.data_ptr<float>() : nullptr,
         ns > 1 ? pml.data_ptr<float>() : nullptr, (float)scale, (int)chunk,
         (int)window, proj.data_ptr(), proj.stride(0), (int)gate_off,

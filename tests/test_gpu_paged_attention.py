@@ -136,6 +136,20 @@ def test_prompt_tiles(Hq, Hk, D, fp8):
     _check(args, _prefill(args, D, _tiles(new)))
 
 
+# enough prompts of one and of two blocks for workgroups of four and of two heads
+# of any group
+@pytest.mark.parametrize("Hq,Hk", [(3, 1), (14, 2), (5, 1), (6, 1)])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("longest", [32, 64])
+def test_many_short_prompts(Hq, Hk, D, longest):
+    n = 1600 // Hq
+    g = torch.Generator().manual_seed(Hq)
+    new = torch.randint(longest - 31, longest + 1, (n,), generator=g).tolist()
+    ctx = torch.randint(0, 70, (n,), generator=g).tolist()
+    args = _paged([a + b for a, b in zip(new, ctx)], new, Hq, Hk, D, False, seed=D)
+    _check(args, _prefill(args, D, _tiles(new)))
+
+
 @pytest.mark.parametrize("Hq,Hk", [(2, 2), (4, 2), (4, 1)])
 def test_prompt_tiles_in_any_order(Hq, Hk):
     # a tile map need not list a sequence's tiles in order, nor at all
