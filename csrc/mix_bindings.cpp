@@ -383,23 +383,25 @@ void local_attention(torch::Tensor out, long out_off, torch::Tensor q,
       (size_t)out.data_ptr() % 8 == 0 && (size_t)q.data_ptr() % 16 == 0 &&
       (size_t)k_cache.data_ptr() % 16 == 0 &&
       (size_t)v_cache.data_ptr() % 16 == 0;
-  // Prompts with heads of 64 and a chunk or window of a few of the 32-row blocks
-  // that a workgroup of the paged kernel has (1, 2 or 4 by the group's heads):
-  // many of its steps are for the rows of one block only, and where there are
-  // enough tiles to fill the chip the other kernel, a workgroup a block, is the
-  // faster one. 128 prompts of 100 tokens, 8 heads and kv heads: chunk 32 / 64 /
-  // 128 23 / 31 / 46 us against 60 / 60 / 57 (4 and 2 heads 11 / 14 / 18 against 17
-  // / 17 / 16), window 32 / 64 31 / 40 against 59 / 59; 3 heads, window 64, 21
-  // against 15.
+  // Prompts with heads of 64 that the other kernel, a workgroup for every 32 rows,
+  // is faster on, where there are enough of them to fill the chip: prompts of one
+  // such block, and chunks or windows of one, which leave most steps of a paged
+  // workgroup (1, 2 or 4 blocks by the group's heads) to the rows of one block.
+  // Paged against the other, us:
+  //   heads        256 x 30 tokens   16 x 2000, chunk 32 / 64   window 32 / 64
+  //   8 and 8      21.6 / 13.1       41 / 40      42 / 46       50 / 54   51 / 68
+  //   14 and 2     17.7 / 15.7       67 / 51      68 / 61       81 / 71   83 / 89
+  //   32 and 8     31.5 / 27.9       109 / 95     107 / 112     130 / 124 135 / 157
+  // (64 x 30 tokens: 7.8 / 9.3, 7.9 / 9.7 and 10.5 / 10.8.)
   const long group = H / G;
   const long blocks = group % 4 == 0 ? 1 : (group % 2 == 0 ? 2 : 4);
-  const long reach = std::max(32l, 16 * blocks);
   const long n_prompts = std::max(0l, seq_lens.numel() - (T - prefill_rows));
-  const long entries =
-      (tile_seq.has_value() ? tile_seq->numel() : 0) * H * blocks / 4;
-  const bool narrow = dk == 64 &&
-                      ((chunk > 0 && chunk <= reach && entries >= 1024) ||
-                       (window > 0 && window <= reach && entries >= 2048));
+  const long tiles = tile_seq.has_value() ? tile_seq->numel() : 0;
+  const bool narrow =
+      dk == 64 &&
+      ((tiles <= n_prompts && tiles * H >= 1000 * std::min(group, 3l)) ||
+       (chunk > 0 && chunk <= 32 && tiles * H * blocks >= 4096) ||
+       (window > 0 && window <= 32 && group > 1 && tiles * H * blocks >= 8192));
   auto run_paged = [&](int tiles, const int* ts, const int* tq, long first,
                        long n) {
     const int ns = n > 0 ? mix_paged_splits(n, (int)G, (int)bt.size(1),
