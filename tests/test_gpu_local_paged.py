@@ -190,3 +190,17 @@ def test_beside_the_paged_kernels(H, G, D, out_off, kind):
     new = [70, 33, 1, 1]
     lens = [270, 33, 400, 65]
     _run(kind, H, G, D, 0, 150, 20, lens, new, 2, seed=H, out_off=out_off)
+
+
+@pytest.mark.parametrize("H,G,D,prompts", [
+    (8, 8, 64, 126), (16, 8, 64, 126),    # fill the chip: the other kernel
+    (3, 1, 128, 175), (14, 2, 64, 40)])   # four heads of an odd group a workgroup
+@pytest.mark.parametrize("kind", ["plain", "all"])
+@pytest.mark.parametrize("window,keep", [(0, 0), (24, 3)])
+def test_many_prompts_of_one_block(H, G, D, prompts, kind, window, keep):
+    g = torch.Generator().manual_seed(H)
+    new = torch.randint(1, 7, (prompts,), generator=g).tolist()
+    new[0] = 32
+    lens = [n + int(c) for n, c in
+            zip(new, torch.randint(0, 50, (prompts,), generator=g))]
+    _run(kind, H, G, D, 0, window, keep, lens, new, prompts, seed=H)
