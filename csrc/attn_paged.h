@@ -957,8 +957,10 @@ static inline void pa_launch_prefill(PagedArgs A, int n_seqs, hipStream_t s) {
   A.leads = (A.n_tiles + A.rpb - 1) / A.rpb;
   // Heads of 64 leave room for four workgroups a CU in 128 registers. Many short
   // prompts, a few steps each with nothing to overlap them, are faster that way:
-  // 128 of 100 tokens, 8 heads and kv heads 50 -> 37 us, 160 of 150, 14 and 2
-  // heads, 63 -> 45; long ones (2000 tokens 38 -> 40) and few are not.
+  // 128 of 100 tokens, 8 heads and kv heads 19 -> 16 us, 160 of 150, 14 and 2
+  // heads, 60 -> 45, 500 of 30, 16 and 8, 38 -> 26; long ones (2000 tokens 38 ->
+  // 40) and few are not. (Layer lists would spill registers: 32 prompts of 200
+  // tokens, 8 heads and kv heads, 19 -> 24 us.)
   if constexpr (D == 64 && !LOCAL) {
     if ((long)A.n_tiles * A.groups >= 512 && A.n_tiles <= 8 * n_seqs) {
       if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 4>(A, s);
