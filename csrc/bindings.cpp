@@ -47,7 +47,7 @@ void sutro_qkv_prep(const void*, void*, void*, void*, const long*, const long*,
 void sutro_sampler_fused(const void*, int, const float*, const float*,
                          const int*, const float*, const unsigned int*, int,
                          long, int, int, int*, float*, hipStream_t);
-void sutro_grouped_gemm(void*, const void*, const void*, const int*,
+void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
                         int, hipStream_t);
 void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
@@ -257,7 +257,7 @@ void grouped_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
     TORCH_CHECK(row_tok->scalar_type() == at::kInt, "row_tok int32");
     rt = row_tok->data_ptr<int>();
   }
-  sutro_grouped_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(), rt,
+  sutro_grouped_gemm(out.data_ptr(), a.data_ptr(), a.size(0), w.data_ptr(), rt,
                      tile_off.data_ptr<int>(), counts.data_ptr<int>(), (int)E,
                      (int)max_tiles, (int)n_cols, K, gate_silu ? 1 : 0,
                      (int)bm, cur_stream());

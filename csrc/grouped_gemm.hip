@@ -258,146 +258,367 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
 }
 
 // ---- tiles of 256 rows ----------------------------------------------------
-// 256 rows x 256 weight rows (gated: 128 gate and 128 up rows) a workgroup, 8
-// waves as 2 x 4, each 128 x 64 on mfma_f32_32x32x16_bf16; 64 of k a step, both
-// operands copied straight into a double-buffered LDS tile (128 KB), one
-// barrier a step. Bound by LDS reads and the products together: a wave reads
-// 24 KB a step for 1.05 MFLOP, half of what the 64 x 32 wave tiles of the
-// 128-row kernel need. At 32 experts of 2048 x 2048, gate and up / down:
-// 4096 rows an expert 3187 / 2188 -> 2081 / 1086 us (690 / 502 -> 1057 / 1013
-// TFLOP/s), 375 rows 422 / 249 -> 277 / 145, 187 rows 224 / 163 -> 154 / 89,
-// 96 rows 142 / 67 -> 154 / 89 (the padding: the other kernel's).
+// 256 rows x 256 weight rows (gated: 128 gate and 128 up rows) a tile, four waves
+// of 128 x 128, one on a SIMD with all of its registers: 256 of them hold the
+// sums, and a wave reads 32 KB of LDS for 2.1 MFLOP. One workgroup a CU stays for
+// the whole launch and goes from tile to tile; its copies run across the tiles.
 //
-// Row tables are looked up once, not every step. Workgroup id i runs on XCD
-// i % 8: an XCD takes four neighbouring row tiles and goes through all column
-// blocks with them, so what its L2 holds is used by many workgroups at a time.
+// Bound by the power limit and by the copies' share of the LDS: the matrix cores
+// are busy 65 to 77 % at 1.75 to 1.85 GHz. What that took:
+// - mfma 16x16x32 instead of 32x32x16. Both do as much a cycle, but a sum is read
+//   and written half as often, and the clock the power limit leaves is higher:
+//   8192^3 785 -> 727 us, the rest alike.
+// - Operands of the next 32 of k are read while the products of these run (two
+//   register sets), so no wave waits for the LDS behind a barrier.
+// - Copies go straight to LDS by buffer loads (one address register, the step in a
+//   scalar) into a ring of five units of 32 KB: three of A rows and B rows ahead
+//   of those in use, A two steps and B one step before they are needed.
+// At 32 experts of 2048 x 2048, gate and up / down, against eight waves of 128 x
+// 64 with two buffers: 4096 rows an expert 2081 / 1086 -> 1604 / 835 us (1057 /
+// 1013 -> 1371 / 1317 TFLOP/s), 384 rows 277 / 145 -> 242 / 118. A large product of
+// the library reaches 1.6 PFLOP/s on the same card (8192^3: 675 us).
+//
+// An XCD (workgroup id % 8) takes GW_ROWS neighbouring row tiles and goes through
+// all column blocks with them: its 32 workgroups share 4 row tiles and 8 column
+// blocks at a time, so that four of five copies hit its L2.
 #define GW_ROWS 4
-template <int MODE>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-gg_wide_kernel(u16* __restrict__ out, const u16* __restrict__ a,
-               const u16* __restrict__ w, const int* __restrict__ row_tok,
-               const int* __restrict__ tile_off, const int* __restrict__ counts,
-               int n_experts, int n_cols, long K, float limit,
-               const float* __restrict__ row_w) {
+#define GW_CUS 256
+#define GW_UNIT (256 * 128)       // bytes of 256 rows x 64 of k
+#define GW_LDS (5 * GW_UNIT)
+
+template <int V>
+struct GwFlag {
+  static constexpr bool v = V != 0;
+};
+
+// an output tile: first row, first column, expert, live rows from the first on
+struct GwTile {
+  long seg;
+  int n0, e, live;
+};
+
+// where a workgroup is: first row tile of its XCD's group, place in the group
+struct GwWalk {
+  int t0, r8;
+};
+
+// next tile of the walk; lanes hold tile_off and counts where experts are few
+template <int BN>
+__device__ __forceinline__ bool gw_next(GwWalk& k, int nb, int total,
+                                        int n_experts, int loff, int lcnt,
+                                        const int* tile_off, const int* counts,
+                                        GwTile& g) {
+  for (; k.t0 < total; k.r8 += gridDim.x >> 3) {
+    while (k.r8 >= GW_ROWS * nb) {
+      k.r8 -= GW_ROWS * nb;
+      k.t0 += 8 * GW_ROWS;
+    }
+    const int t = k.t0 + k.r8 % GW_ROWS;
+    if (t >= total) continue;
+    int first, rows;
+    if (n_experts < 64) {
+      g.e = __builtin_popcountll(__ballot(loff <= t)) - 1;
+      first = __builtin_amdgcn_readlane(loff, g.e);
+      rows = __builtin_amdgcn_readlane(lcnt, g.e);
+    } else {
+      g.e = gg_expert(tile_off, n_experts, t);
+      first = tile_off[g.e];
+      rows = counts[g.e];
+    }
+    g.n0 = k.r8 / GW_ROWS * BN;
+    g.seg = (long)t * 256;
+    g.live = rows - (t - first) * 256;
+    k.r8 += gridDim.x >> 3;
+    return true;
+  }
+  return false;
+}
+
+// two floats to bf16 (round to nearest even), the first in the low half
+typedef __bf16 gw_bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32 gw_pack(float x, float y) {
+  gw_bf16x2 p;
+  p[0] = (__bf16)x;
+  p[1] = (__bf16)y;
+  return __builtin_bit_cast(u32, p);
+}
+
+// ANY: gathered rows of 4 GB or more in all, or operands that do not begin at
+// multiples of 16 bytes; 64-bit addresses and narrow stores then.
+template <int MODE, bool ANY>
+__device__ __forceinline__ void gw_body(
+    u16* __restrict__ out, const u16* __restrict__ a,
+    const u16* __restrict__ w, const int* __restrict__ row_tok,
+    const int* __restrict__ tile_off, const int* __restrict__ counts,
+    int n_experts, int n_cols, long K, float limit,
+    const float* __restrict__ row_w) {
   constexpr bool GATED = MODE == 1 || MODE >= 3;
   constexpr bool GATHER = MODE != 0;
   constexpr int BN = GATED ? 128 : 256;   // output columns
-  constexpr int TILE = 256 * 128;         // bytes of an operand tile
   const int nb = n_cols / BN;
-  const int xcd = blockIdx.x & 7, j8 = blockIdx.x >> 3;
-  const int r8 = j8 % (GW_ROWS * nb);
-  const int t = ((j8 / (GW_ROWS * nb)) * 8 + xcd) * GW_ROWS + r8 % GW_ROWS;
-  const int n0 = r8 / GW_ROWS * BN;
-  if (t >= tile_off[n_experts]) return;
-  const int e = gg_expert(tile_off, n_experts, t);
-  const int m0 = (t - tile_off[e]) * 256;
-  const long seg = (long)tile_off[e] * 256 + m0;   // first row of the tile
-  const int live = counts[e] - m0;
-
+  const int total = tile_off[n_experts];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ln = lane & 31, hi = lane >> 5;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int ln = lane & 15, quad = lane >> 4;
+  const int wm = wave >> 1, wn = wave & 1;
   extern __shared__ __attribute__((aligned(16))) char gw_smem[];
 
-  // copies: 1 KB (8 rows of 128 bytes) an instruction, pieces wave*4 + j of
+  const int loff = lane <= n_experts ? tile_off[lane] : 0x7fffffff;
+  const int lcnt = lane < n_experts ? counts[lane] : 0;
+  GwWalk walk = {(int)(blockIdx.x & 7) * GW_ROWS, (int)(blockIdx.x >> 3)};
+  GwTile cur;
+  auto next = [&](GwTile& g) {
+    return gw_next<BN>(walk, nb, total, n_experts, loff, lcnt, tile_off, counts,
+                       g);
+  };
+  if (!next(cur)) return;
+
+  // copies: 1 KB (8 rows of 128 bytes) an instruction, pieces wave * 8 + j of
   // either operand; 16-byte chunks are XOR-swizzled by bits 1 to 3 of the row, so
-  // that the 16 rows read in a cycle cover all 64 banks (by bits 0 to 2, eight of
-  // them did: down product at 4096 rows an expert 1089 -> 1058 us, the gated one
-  // 2155 -> 2125)
+  // that the 16 rows read in a cycle cover all 64 banks
   const int pr = lane >> 3;
-  const u16* pa[4];
+  const int ch[2] = {((lane & 7) ^ (pr >> 1)) * 8,
+                     ((lane & 7) ^ ((8 + pr) >> 1)) * 8};
+  struct Source {
+    __amdgpu_buffer_rsrc_t ra, rb;
+    u32 va[ANY ? 1 : 8];
+    const u16* pa[ANY ? 8 : 1];
+    const u16* pb;
+  };
+  auto point = [&](const GwTile& g, Source& s) {
+    const u16* base = GATHER ? a : a + g.seg * K;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = (wave * 4 + j) * 8 + pr;
-    long row;
-    if (GATHER) {
-      row = row_tok[seg + min(r, live - 1)];   // padding rows repeat the last
-      if (row < 0) row = 0;
-    } else {
-      row = seg + r;
+    for (int j = 0; j < 8; ++j) {
+      const int r = (wave * 8 + j) * 8 + pr;
+      int row = r;
+      if (GATHER)        // padding rows repeat the last
+        row = max(row_tok[g.seg + min(r, g.live - 1)], 0);
+      if (ANY)
+        s.pa[ANY ? j : 0] = base + row * K + ch[j & 1];
+      else
+        s.va[ANY ? 0 : j] = (u32)row * (u32)(K * 2) + ch[j & 1] * 2;
     }
-    pa[j] = a + row * K + ((lane & 7) ^ (((j & 1) * 8 + pr) >> 1)) * 8;
-  }
-  const int br = wave * 32;                    // first of this wave's B rows
-  const long brow = (GATED && br >= 128) ? n_cols + n0 + br - 128 : n0 + br;
-  const u16* pb = w + ((long)e * (GATED ? 2 : 1) * n_cols + brow) * K;
-  const u32 boff[2] = {(u32)(pr * K + ((lane & 7) ^ (pr >> 1)) * 8),
-                       (u32)(pr * K + ((lane & 7) ^ ((8 + pr) >> 1)) * 8)};
-  auto stage = [&](int buf, long k) {
-    char* dst = gw_smem + buf * 2 * TILE + wave * 4096;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      glds16g((const u32*)(pa[j] + k), (u32*)(dst + j * 1024));
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      glds16g((const u32*)(pb + k + j * 8 * K + boff[j & 1]),
-              (u32*)(dst + TILE + j * 1024));
+    const int br = wave * 64;                  // first of this wave's B rows
+    const long brow =
+        (GATED && br >= 128) ? n_cols + g.n0 + br - 128 : g.n0 + br;
+    s.pb = w + ((long)g.e * (GATED ? 2 : 1) * n_cols + brow) * K;
+    s.ra = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu,
+                                             0x00027000);
+    s.rb = __builtin_amdgcn_make_buffer_rsrc((void*)s.pb, 0, 0xffffffffu,
+                                             0x00027000);
+  };
+  const u32 vb[2] = {(u32)(pr * K + ch[0]), (u32)(pr * K + ch[1])};
+  char* const mine = gw_smem + wave * 8192;
+  Source src;
+  auto copy_a = [&](int slot, int j, int k) {
+    char* d = mine + slot + j * 1024;
+    if (ANY)
+      glds16g((const u32*)(src.pa[ANY ? j : 0] + k), (u32*)d);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src.ra, (__attribute__((address_space(3))) void*)d, 16,
+          src.va[ANY ? 0 : j], (u32)k * 2, 0, 0);
+  };
+  auto copy_b = [&](int slot, int j, int k) {
+    char* d = mine + slot + j * 1024;
+    if (ANY)
+      glds16g((const u32*)(src.pb + k + j * 8 * K + vb[j & 1]), (u32*)d);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src.rb, (__attribute__((address_space(3))) void*)d, 16,
+          vb[j & 1] * 2, (u32)(k + j * 8 * K) * 2, 0, 0);
   };
 
-  int kad[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk)
-    kad[kk] = ln * 128 + (((kk * 2 + hi) ^ ((ln >> 1) & 7)) << 4);
+  const int kad = ln * 128 + ((quad ^ ((ln >> 1) & 7)) << 4);
   const int arow = wm * 128 * 128;
-  const int brow0 = (GATED ? wn * 32 : wn * 64) * 128 + TILE;
-  const int brow1 = (GATED ? 128 + wn * 32 : wn * 64 + 32) * 128 + TILE;
+  const int brow = wn * (GATED ? 64 : 128) * 128;
+  f32x4 acc[8][8];                // gated: columns 0 to 3 gate, 4 to 7 up
+  bf16x8 fa[2][8], fb[2][8];
+  auto load_a = [&](int i, int slot, int kk) {
+    fa[kk][i] = *(const bf16x8*)(gw_smem + slot + arow + i * 2048 +
+                                 (kad ^ (kk << 6)));
+  };
+  auto load_b = [&](int j, int slot, int kk) {
+    const int o = GATED ? (j >> 2) * 16384 + (j & 3) * 2048 : j * 2048;
+    fb[kk][j] = *(const bf16x8*)(gw_smem + slot + brow + o + (kad ^ (kk << 6)));
+  };
+  auto wrap = [](int o) { return o >= GW_LDS ? o - GW_LDS : o; };
 
-  f32x16 acc[4][2];
+  // The sums are transposed (B rows first), so a lane has four columns of a row;
+  // lanes of neighbouring column tiles swap halves: 16 bytes a lane and store.
+  auto store_tile = [&](const GwTile& g) {
+    const u32 off = (u32)(ln * n_cols + (quad & 1) * 16 + (quad >> 1) * 8) * 2;
+    const long row = g.seg + wm * 128;
+    char* at = (char*)(out + row * n_cols + g.n0 + wn * (GATED ? 64 : 128));
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i, at += (long)n_cols * 32) {
+      const float rw = MODE == 4 ? row_w[row + i * 16 + ln] : 1.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x16)(0.f);
+      for (int j = 0; j < (GATED ? 4 : 8); j += 2) {
+        // the sums stay where the products left them until here: read all at
+        // once they would need more registers than there are
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          asm volatile("" : "+a"(acc[i][j + q]));
+          if (GATED) asm volatile("" : "+a"(acc[i][(j + q + 4) & 7]));
+        }
+        u32 p[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float x[2];
+#pragma unroll
+          for (int z = 0; z < 2; ++z) {
+            const int jj = j + (q >> 1), r = (q & 1) * 2 + z;
+            x[z] = gg_unit<MODE>(acc[i][jj][r],
+                                 GATED ? acc[i][(jj + 4) & 7][r] : 0.f, limit,
+                                 rw);
+          }
+          p[q] = gw_pack(x[0], x[1]);
+        }
+        const auto s0 =
+            __builtin_amdgcn_permlane16_swap(p[0], p[2], false, false);
+        const auto s1 =
+            __builtin_amdgcn_permlane16_swap(p[1], p[3], false, false);
+        const u32x4 pk = {s0[0], s1[0], s0[1], s1[1]};
+        u16* o = (u16*)(at + off) + j * 16;
+        if (ANY) {
+#pragma unroll
+          for (int z = 0; z < 8; ++z)
+            o[z] = (u16)(pk[z >> 1] >> ((z & 1) * 16));
+        } else {
+          *(u32x4*)o = pk;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  int sa = 0;   // LDS offset of the step's A rows; its B rows are one unit further
+  // FIRST: the sums begin at zero. AHEAD: copies of A and B two steps on, at k2 of
+  // the source. MORE: another step follows, whose operands are read at the end.
+  auto step = [&](int k2, auto first_c, auto ahead_c, auto more_c) {
+    constexpr bool FIRST = decltype(first_c)::v, AHEAD = decltype(ahead_c)::v,
+                   MORE = decltype(more_c)::v;
+    const int sb = wrap(sa + GW_UNIT), na = wrap(sa + 2 * GW_UNIT),
+              nbs = wrap(sa + 3 * GW_UNIT), ca = wrap(sa + 4 * GW_UNIT);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      if (kk == 1 && MORE) {
+        // All reads of this step are done and the next step's operands are there
+        // (behind them only the A rows of two steps on), for all four waves:
+        // copies may overwrite this step's, reads may go on to the next one's.
+        __builtin_amdgcn_sched_barrier(0);
+        if (AHEAD)
+          asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int x = 0; x < 64; ++x) {
+        const int i = x >> 3, j = x & 7;
+        acc[i][j] = mfma16g(fb[kk][j], fa[kk][i],
+                            FIRST && kk == 0 ? (f32x4)(0.f) : acc[i][j]);
+        // reads behind every third product, copies behind every fourth: the LDS
+        // takes both beside each other
+        if (x % 3 == 0 && x / 3 < 16 && (kk == 0 || MORE)) {
+          const int y = x / 3;
+          if (y < 8) load_b(y, kk ? nbs : sb, kk ^ 1);
+          else load_a(y - 8, kk ? na : sa, kk ^ 1);
+        }
+        if (AHEAD && x % 4 == 1 && x / 4 < 8) {
+          if (kk == 0) copy_a(ca, x / 4, k2);
+          else copy_b(sa, x / 4, k2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    sa = na;
+  };
+  constexpr GwFlag<0> no{};
+  constexpr GwFlag<1> yes{};
 
   const int KT = (int)(K >> 6);
-  stage(0, 0);
-  for (int kt = 0; kt < KT; ++kt) {
-    __syncthreads();
-    if (kt + 1 < KT) stage((kt + 1) & 1, (long)(kt + 1) * 64);
-    const char* at = gw_smem + (kt & 1) * 2 * TILE;
+  const int lead = min(KT, 2);
+  // the first two steps of a tile, and the operands of its first products
+  auto open = [&]() {
+    for (int s = 0; s < lead; ++s) {
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const bf16x8 b0 = *(const bf16x8*)(at + brow0 + kad[kk]);
-      const bf16x8 b1 = *(const bf16x8*)(at + brow1 + kad[kk]);
+      for (int j = 0; j < 8; ++j) copy_a(2 * s * GW_UNIT, j, s * 64);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bf16x8 af = *(const bf16x8*)(at + arow + i * 4096 + kad[kk]);
-        acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, b0, acc[i][0],
-                                                            0, 0, 0);
-        acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, b1, acc[i][1],
-                                                            0, 0, 0);
-      }
+      for (int j = 0; j < 8; ++j) copy_b((2 * s + 1) * GW_UNIT, j, s * 64);
     }
-    // ten fragments ahead of the products, then one behind each
-    __builtin_amdgcn_sched_group_barrier(0x100, 10, 0);
+    if (lead == 2)
+      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    sa = 0;
 #pragma unroll
-    for (int i = 0; i < 14; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    for (int j = 0; j < 8; ++j) {
+      load_b(j, GW_UNIT, 0);
+      load_a(j, 0, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x8, 18, 0);
-  }
+  };
 
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const long row =
-          seg + wm * 128 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-      u16* o = out + row * n_cols + n0;
-      const float rw = MODE == 4 ? row_w[row] : 1.f;
-      if (GATED) {
-        o[wn * 32 + ln] = f2bf(
-            gg_unit<MODE>(acc[i][0][r], acc[i][1][r], limit, rw));
+  point(cur, src);
+  if (KT < 3) {       // too short to run across tiles
+    for (;;) {
+      open();
+      if (KT == 2) {
+        step(0, yes, no, yes);
+        step(0, no, no, no);
       } else {
-        o[wn * 64 + ln] = f2bf(gg_unit<MODE>(acc[i][0][r], 0.f, limit, rw));
-        o[wn * 64 + 32 + ln] =
-            f2bf(gg_unit<MODE>(acc[i][1][r], 0.f, limit, rw));
+        step(0, yes, no, no);
       }
+      store_tile(cur);
+      if (!next(cur)) return;
+      point(cur, src);
+      __syncthreads();        // the reads of this tile's operands are done
     }
+  }
+  open();
+  for (;;) {
+    step(128, yes, yes, yes);
+    GwTile nxt;
+    Source after;
+    const bool more = next(nxt);
+    if (more) point(nxt, after);
+    const int last = more ? KT : KT - 2;
+    int k2 = 192;
+    for (int s = 1; s < last; ++s, k2 += 64) {
+      if (s == KT - 2) {      // from here on the copies are the next tile's
+        src = after;
+        k2 = 0;
+      }
+      step(k2, no, yes, yes);
+    }
+    if (!more) {
+      step(0, no, no, yes);
+      step(0, no, no, no);
+    }
+    store_tile(cur);
+    if (!more) return;
+    cur = nxt;
+  }
 }
 
-static void grouped_gemm_launch(void* out, const void* a, const void* w,
+template <int MODE, bool ANY>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+gw_kernel(u16* __restrict__ out, const u16* __restrict__ a,
+          const u16* __restrict__ w, const int* __restrict__ row_tok,
+          const int* __restrict__ tile_off, const int* __restrict__ counts,
+          int n_experts, int n_cols, long K, float limit,
+          const float* __restrict__ row_w) {
+  gw_body<MODE, ANY>(out, a, w, row_tok, tile_off, counts, n_experts, n_cols, K,
+                     limit, row_w);
+}
+
+static void grouped_gemm_launch(void* out, const void* a, long a_rows,
+                                const void* w,
                                 const int* row_tok, const int* tile_off,
                                 const int* counts, int n_experts,
                                 int max_tiles, int n_cols, long K,
@@ -427,16 +648,23 @@ static void grouped_gemm_launch(void* out, const void* a, const void* w,
       n_experts, n_cols, K, limit, row_w
   const bool gated = gate_silu == 1 || gate_silu >= 3;
   if (bm == 256) {
-    const int nb = n_cols / (gated ? 128 : 256);
     const unsigned groups = (unsigned)((max_tiles + 8 * GW_ROWS - 1) /
                                        (8 * GW_ROWS));
-    const dim3 grid(groups * 8 * GW_ROWS * nb);
-#define GG_WIDE(M)                                                          \
+    const unsigned work = groups * 8 * GW_ROWS * (n_cols / (gated ? 128 : 256));
+    const dim3 grid(work < GW_CUS ? work : GW_CUS);
+    const bool any = (gate_silu && a_rows >= (0xf0000000l / 2) / K) ||
+                     (((size_t)out | (size_t)a | (size_t)w) & 15);
+#define GG_WIDE_AS(M, ANY)                                                  \
   {                                                                         \
     static std::atomic<unsigned long long> asked{0};                        \
-    lds_limit((const void*)gg_wide_kernel<M>, 4 * 256 * 128, asked);        \
-    hipLaunchKernelGGL(gg_wide_kernel<M>, grid, dim3(512), 4 * 256 * 128,   \
+    lds_limit((const void*)gw_kernel<M, ANY>, GW_LDS, asked);               \
+    hipLaunchKernelGGL((gw_kernel<M, ANY>), grid, dim3(256), GW_LDS,        \
                        stream, GG_ARGS);                                    \
+  }
+#define GG_WIDE(M)                                                          \
+  {                                                                         \
+    if (any) GG_WIDE_AS(M, true)                                            \
+    else GG_WIDE_AS(M, false)                                               \
   }
     GG_MODES(GG_WIDE)
     return;
@@ -472,34 +700,34 @@ static void grouped_gemm_launch(void* out, const void* a, const void* w,
 #undef GG_LAUNCH
 }
 
-extern "C" void sutro_grouped_gemm(void* out, const void* a, const void* w,
-                                   const int* row_tok, const int* tile_off,
+extern "C" void sutro_grouped_gemm(void* out, const void* a, long a_rows,
+                                   const void* w, const int* row_tok, const int* tile_off,
                                    const int* counts, int n_experts,
                                    int max_tiles, int n_cols, long K,
                                    int gate_silu, int bm,
                                    hipStream_t stream) {
-  grouped_gemm_launch(out, a, w, row_tok, tile_off, counts, n_experts,
+  grouped_gemm_launch(out, a, a_rows, w, row_tok, tile_off, counts, n_experts,
                       max_tiles, n_cols, K, gate_silu, bm, 0.f, nullptr,
                       stream);
 }
 
 // the clamped gated unit (mode 3) with its limit
-extern "C" void sutro_grouped_gemm_glu(void* out, const void* a, const void* w,
-                                       const int* row_tok, const int* tile_off,
+extern "C" void sutro_grouped_gemm_glu(void* out, const void* a, long a_rows,
+                                       const void* w, const int* row_tok, const int* tile_off,
                                        const int* counts, int n_experts,
                                        int max_tiles, int n_cols, long K,
                                        int bm, float limit,
                                        hipStream_t stream) {
-  grouped_gemm_launch(out, a, w, row_tok, tile_off, counts, n_experts,
+  grouped_gemm_launch(out, a, a_rows, w, row_tok, tile_off, counts, n_experts,
                       max_tiles, n_cols, K, 3, bm, limit, nullptr, stream);
 }
 
 // the silu unit over weighted rows (mode 4)
 extern "C" void sutro_grouped_gemm_weighted(
-    void* out, const void* a, const void* w, const int* row_tok,
+    void* out, const void* a, long a_rows, const void* w, const int* row_tok,
     const int* tile_off, const int* counts, int n_experts, int max_tiles,
     int n_cols, long K, int bm, const float* row_w, hipStream_t stream) {
-  grouped_gemm_launch(out, a, w, row_tok, tile_off, counts, n_experts,
+  grouped_gemm_launch(out, a, a_rows, w, row_tok, tile_off, counts, n_experts,
                       max_tiles, n_cols, K, 4, bm, 0.f, row_w, stream);
 }
 

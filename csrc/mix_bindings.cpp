@@ -89,16 +89,16 @@ long mix_moe_dispatch_scratch(long, int);
 void mix_expert_gemm_plain(void*, const void*, const void*, const int*,
                            const int*, const int*, int, int, int, int, long,
                            int, float, const float*, int, hipStream_t);
-void sutro_grouped_gemm_weighted(void*, const void*, const void*, const int*,
-                                 const int*, const int*, int, int, int, long,
-                                 int, const float*, hipStream_t);
+void sutro_grouped_gemm_weighted(void*, const void*, long, const void*,
+                                 const int*, const int*, const int*, int, int,
+                                 int, long, int, const float*, hipStream_t);
 long mix_hyper_lds(int, int);
 int mix_hyper_rmsnorm(float*, const float*, const void*, const void*,
                       const int*, const float*, float, int, const void*,
                       const float*, const float*, const float*, const float*,
                       float, void*, int, long, int, int, int, hipStream_t);
 void mix_relu_sq(void*, long, int, hipStream_t);
-void sutro_grouped_gemm_glu(void*, const void*, const void*, const int*,
+void sutro_grouped_gemm_glu(void*, const void*, long, const void*, const int*,
                             const int*, const int*, int, int, int, long, int,
                             float, hipStream_t);
 void mix_add_rmsnorm(float*, const float*, const float*, const void*,
@@ -132,7 +132,7 @@ int mix_decay_scan(float*, const float*, long, const float*, long,
                    const float*, float*, const int*, const int*, const int*,
                    int, int, int, int, int, hipStream_t);
 void mix_softcap(float*, const void*, float, long, int, hipStream_t);
-void sutro_grouped_gemm(void*, const void*, const void*, const int*,
+void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
                         int, hipStream_t);
 void mix_weighted_rmsnorm(void*, const float*, const float*, float, long, int,
@@ -1032,19 +1032,19 @@ void expert_gemm(torch::Tensor out, torch::Tensor a, torch::Tensor w,
   if (mfma) {
     if (rw)
       sutro_grouped_gemm_weighted(
-          out.data_ptr(), a.data_ptr(), w.data_ptr(), rt,
+          out.data_ptr(), a.data_ptr(), a.size(0), w.data_ptr(), rt,
           tile_off.data_ptr<int>(), counts.data_ptr<int>(), (int)E,
           (int)(n_rows / bm), (int)N, K, (int)bm, rw, cur_stream());
     else if (act == 3)
-      sutro_grouped_gemm_glu(out.data_ptr(), a.data_ptr(), w.data_ptr(), rt,
-                             tile_off.data_ptr<int>(), counts.data_ptr<int>(),
-                             (int)E, (int)(n_rows / bm), (int)N, K, (int)bm,
-                             (float)limit, cur_stream());
+      sutro_grouped_gemm_glu(out.data_ptr(), a.data_ptr(), a.size(0),
+                             w.data_ptr(), rt, tile_off.data_ptr<int>(),
+                             counts.data_ptr<int>(), (int)E, (int)(n_rows / bm),
+                             (int)N, K, (int)bm, (float)limit, cur_stream());
     else
-      sutro_grouped_gemm(out.data_ptr(), a.data_ptr(), w.data_ptr(), rt,
-                         tile_off.data_ptr<int>(), counts.data_ptr<int>(),
-                         (int)E, (int)(n_rows / bm), (int)N, K, (int)act,
-                         (int)bm, cur_stream());
+      sutro_grouped_gemm(out.data_ptr(), a.data_ptr(), a.size(0),
+                         w.data_ptr(), rt, tile_off.data_ptr<int>(),
+                         counts.data_ptr<int>(), (int)E, (int)(n_rows / bm),
+                         (int)N, K, (int)act, (int)bm, cur_stream());
     return;
   }
   mix_expert_gemm_plain(out.data_ptr(), a.data_ptr(), w.data_ptr(), rt,

@@ -266,15 +266,15 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
     for `n_rows` (token, expert) pairs in bf16 on the matrix cores (K and N
     multiples of 64), by the rows an expert gets on average. Taller tiles do
     more work per byte but pad more; both products together, at 32 experts of
-    2048 x 2048: at 96 rows 302 / 230 / 249 us on tiles of 64 / 128 / 256, at
-    192 rows 523 / 373 / 258, at 384 rows 1050 / 650 / 415.
+    2048 x 2048: at 96 rows 281 / 213 / 233 us on tiles of 64 / 128 / 256, at
+    192 rows 393 / 340 / 232, at 384 rows 952 / 511 / 360.
 
     They also leave fewer workgroups: one of 256 rows takes 128 columns of the
     gated product or 256 of the other, and below 128 of them in either product
     the chip idles. 8 experts of 1024 x 512, 192 / 512 / 1024 rows an expert (24 /
-    64 / 128 of either) 35 / 52 / 76 us on 64, 41 / 47 / 78 on 128, 55 / 56 / 61 on
-    256; 8 of 2048 x 2048 at 384 / 512 rows (96 / 128 of the second) 223 / 263 on
-    64, 147 / 208 on 128, 180 / 183 on 256. Tiles of 128 want 96.
+    64 / 128 of either) 26 / 40 / 63 us on 64, 33 / 37 / 47 on 128, 45 / 44 / 43 on
+    256; 8 of 2048 x 2048 at 384 / 512 rows (96 / 128 of the second) 183 / 245 on
+    64, 132 / 146 on 128, 148 / 147 on 256. Tiles of 128 want 96.
 
     Up to 16 rows, where the weights are all there is to read, tiles of 32: four
     workgroups of the gated product fit a CU instead of three. They are taken

@@ -1,0 +1,67 @@
+"""The expert GEMMs on tiles of 256 rows where a workgroup goes through several
+tiles: more tiles than workgroups, one to several steps of k, few and many experts
+(their table in lanes, or searched), operands off 16-byte boundaries."""
+
+import pytest
+import torch
+
+from sutro_amd.ops import hybrid as hops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _run(counts, K, ff, act, shift=0):
+    g = torch.Generator(device=DEV).manual_seed(K + len(counts))
+
+    def rnd(*shape):
+        n = 1
+        for s in shape:
+            n *= s
+        flat = torch.randn(n + shift, generator=g, device=DEV).bfloat16()
+        return flat[shift:].view(*shape)
+
+    gated = act == hops.ACT_SILU_GATE
+    tiles = [(c + 255) // 256 for c in counts]
+    off = torch.tensor([0] + tiles, device=DEV).cumsum(0).int()
+    cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
+    rows = sum(tiles) * 256
+    w = rnd(len(counts), 2 * ff if gated else ff, K).mul_(K ** -0.5)
+    T = 300
+    x = rnd(T, K) if gated else rnd(rows, K)
+    tok = None
+    if gated:
+        tok = torch.full((rows,), -1, device=DEV, dtype=torch.int32)
+        for e, c in enumerate(counts):
+            a = int(off[e]) * 256
+            tok[a:a + c] = torch.randint(T, (c,), generator=g,
+                                         device=DEV).int()
+    out = rnd(rows, ff)
+    hops.expert_gemm(out, x, w, tok, off, cnt, act, 256, 0.0, None)
+    for e, c in enumerate(counts):
+        a = int(off[e]) * 256
+        xe = (x[tok[a:a + c].long()] if gated else x[a:a + c]).float()
+        y = xe @ w[e].float().T
+        if gated:
+            y = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+        # one rounding to bf16 (2^-9) over fp32 sums of K products
+        torch.testing.assert_close(out[a:a + c].float(), y, rtol=2 ** -7,
+                                   atol=2 ** -7)
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 448])
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
+def test_more_tiles_than_workgroups(K, act):
+    # 8 tiles of a group, 5 column blocks (gated: 10) and a last group in part
+    _run([300, 0, 1, 256, 257, 9000, 2500], K, 1280, act)
+
+
+@pytest.mark.parametrize("experts", [63, 64, 130])
+def test_many_experts(experts):
+    _run([(i * 37) % 300 for i in range(experts)], 192, 256,
+         hops.ACT_SILU_GATE)
+
+
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
+def test_operands_off_boundaries(act):
+    _run([600, 5, 300], 320, 512, act, shift=8 + 2)
