@@ -163,6 +163,21 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   const int b_off = BM * 64;
   const int b2_off = (BM + BN) * 64;
 
+  // Workgroups start at different steps of k where weight rows are multiples of
+  // 4 KB apart: all in step they read the same few 128-byte columns of a hundred
+  // thousand rows at a time, which lie on few memory channels. 32 experts of 2048
+  // x 2048, 128 tokens of 4: gate and up 132 -> 95 us, down 67 -> 48 (4.0 -> 5.6
+  // TB/s); 16 tokens 100 -> 79 and 61 -> 49; K of 4096 and 8192 1 to 10 % less. Rows
+  // of 6 KB spread by themselves (160 us, rotated 172). All tiles of an expert and
+  // column block share a start, as they share weights; tiles of 128 rows share
+  // rows of x between column blocks and stay in step (71 us, rotated 80).
+  const int KT = (int)(K >> 6);
+  const int start =
+      BM <= 64 && K % 2048 == 0 ? (int)(e * 5u + blockIdx.y * 3u) % KT : 0;
+  auto k_of = [&](int kt) {
+    const int z = kt + start;
+    return (long)(z < KT ? z : z - KT) * 64;
+  };
   const long Kb = K * 2;
   const u16* wa = w + (long)e * (GATED ? 2 : 1) * n_cols * K;
   const u16* wg = wa + (long)n0 * K;
@@ -180,25 +195,27 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
     }
 
   // prologue
+  const long k_first = k_of(0);
   if (GATHER)
-    gg_stage<BM, WAVES, true>(smem[0], aa, Kb, rt, m0, rows_valid, wave, lane);
+    gg_stage<BM, WAVES, true>(smem[0], aa + k_first, Kb, rt, m0, rows_valid,
+                              wave, lane);
   else
-    gg_stage<BM, WAVES, false>(smem[0], aa, Kb, nullptr, m0, BM, wave, lane);
-  gg_stage<BN, WAVES, false>(smem[0] + b_off, wg, Kb, nullptr, 0, BN, wave,
-                             lane);
-  if (GATED)
-    gg_stage<BN, WAVES, false>(smem[0] + b2_off, wu, Kb, nullptr, 0, BN, wave,
+    gg_stage<BM, WAVES, false>(smem[0], aa + k_first, Kb, nullptr, m0, BM, wave,
                                lane);
+  gg_stage<BN, WAVES, false>(smem[0] + b_off, wg + k_first, Kb, nullptr, 0, BN,
+                             wave, lane);
+  if (GATED)
+    gg_stage<BN, WAVES, false>(smem[0] + b2_off, wu + k_first, Kb, nullptr, 0,
+                               BN, wave, lane);
   __syncthreads();
 
-  const int KT = (int)(K >> 6);
   for (int kt = 0; kt < KT; ++kt) {
     const int p = kt & 1;
     u16* aT = smem[p];
     u16* bgT = smem[p] + b_off;
     u16* buT = smem[p] + b2_off;
     if (kt + 1 < KT) {
-      const long ko = (long)(kt + 1) * 64;
+      const long ko = k_of(kt + 1);
       if (GATHER)
         gg_stage<BM, WAVES, true>(smem[p ^ 1], aa + ko, Kb, rt, m0,
                                   rows_valid, wave, lane);
@@ -542,13 +559,23 @@ __device__ __forceinline__ void gw_body(
 
   const int KT = (int)(K >> 6);
   const int lead = min(KT, 2);
+  // XCDs start an eighth of k apart where rows are multiples of 4 KB long (see the
+  // kernel above; within an XCD workgroups share operands and stay in step): gate
+  // and up / down of 32 experts of 2048 x 2048 at 375 rows 257 / 120 -> 229 / 115 us,
+  // at 4096 rows 1736 / 891 -> 1718 / 858; rows of 2 KB 244 -> 257, so not there
+  int kc = K % 2048 == 0 ? (int)(blockIdx.x & 7) * KT / 8 * 64 : 0;
+  auto advance = [&]() {        // after KT steps it is where it began
+    kc += 64;
+    if (kc == (int)K) kc = 0;
+  };
   // the first two steps of a tile, and the operands of its first products
   auto open = [&]() {
     for (int s = 0; s < lead; ++s) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) copy_a(2 * s * GW_UNIT, j, s * 64);
+      for (int j = 0; j < 8; ++j) copy_a(2 * s * GW_UNIT, j, kc);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) copy_b((2 * s + 1) * GW_UNIT, j, s * 64);
+      for (int j = 0; j < 8; ++j) copy_b((2 * s + 1) * GW_UNIT, j, kc);
+      advance();
     }
     if (lead == 2)
       asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
@@ -582,19 +609,17 @@ __device__ __forceinline__ void gw_body(
   }
   open();
   for (;;) {
-    step(128, yes, yes, yes);
+    step(kc, yes, yes, yes);
+    advance();
     GwTile nxt;
     Source after;
     const bool more = next(nxt);
     if (more) point(nxt, after);
     const int last = more ? KT : KT - 2;
-    int k2 = 192;
-    for (int s = 1; s < last; ++s, k2 += 64) {
-      if (s == KT - 2) {      // from here on the copies are the next tile's
-        src = after;
-        k2 = 0;
-      }
-      step(k2, no, yes, yes);
+    for (int s = 1; s < last; ++s) {
+      if (s == KT - 2) src = after;   // the copies are the next tile's now
+      step(kc, no, yes, yes);
+      advance();
     }
     if (!more) {
       step(0, no, no, yes);
