@@ -50,6 +50,8 @@ void sutro_sampler_fused(const void*, int, const float*, const float*,
 void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
                         int, hipStream_t);
+void sutro_linear_silu_mul(void*, const void*, const void*, int, int, long,
+                           hipStream_t);
 void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
                        int, int, hipStream_t);
 void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
@@ -348,6 +350,26 @@ torch::Tensor linear_skinny(torch::Tensor x, torch::Tensor w,
   return out;
 }
 
+// silu of x [M, K] times the first N rows of w [2 N, K], times x and the others
+torch::Tensor linear_silu_mul(torch::Tensor x, torch::Tensor w) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device(),
+              "operands on one GPU");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16, "bf16 operands");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.is_contiguous() &&
+              w.is_contiguous(), "contiguous matrices");
+  const long M = x.size(0), K = x.size(1), N = w.size(0) / 2;
+  TORCH_CHECK(w.size(1) == K && w.size(0) == 2 * N && K > 0 && K % 64 == 0 &&
+              N > 0 && N % 128 == 0 && M >= 1 && M * K < (1l << 30) &&
+              K < (1l << 21) && N < (1l << 24), "unsupported sizes");
+  TORCH_CHECK((size_t)x.data_ptr() % 16 == 0 && (size_t)w.data_ptr() % 16 == 0,
+              "16-byte rows");
+  auto out = torch::empty({M, N}, x.options());
+  sutro_linear_silu_mul(out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M,
+                        (int)N, K, cur_stream());
+  return out;
+}
+
 void sampler_fused(torch::Tensor logits, torch::Tensor temps,
                    torch::Tensor topps, torch::Tensor topks, torch::Tensor us,
                    c10::optional<torch::Tensor> mask, long vl,
@@ -392,6 +414,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma16_probe", &mfma16_probe, "16x16 MFMA fragment-layout probe");
   m.def("moe_combine", &moe_combine, "fused MoE weighted gather-combine");
   m.def("linear_skinny", &linear_skinny, "linear layer over few rows");
+  m.def("linear_silu_mul", &linear_silu_mul,
+        "linear layer with the silu gate behind it, many rows");
   m.def("moe_layout", &moe_layout, "softmax top-k router + expert segments");
   m.def("grouped_gemm", &grouped_gemm,
         "dropless MoE grouped GEMM (padded segments, static grid)");

@@ -98,7 +98,7 @@ __device__ __forceinline__ float gg_unit(float v, float u, float limit,
     v *= rw;
     u *= rw;
   }
-  if (MODE == 1 || MODE == 4) return v / (1.0f + __expf(-v)) * u;
+  if (MODE == 1 || MODE >= 4) return v / (1.0f + __expf(-v)) * u;
   if (MODE == 3) {
     const float g = fminf(v, limit);
     u = fminf(fmaxf(u, -limit), limit);
@@ -166,14 +166,17 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   // Workgroups start at different steps of k where weight rows are multiples of
   // 4 KB apart: all in step they read the same few 128-byte columns of a hundred
   // thousand rows at a time, which lie on few memory channels. 32 experts of 2048
-  // x 2048, 128 tokens of 4: gate and up 132 -> 95 us, down 67 -> 48 (4.0 -> 5.6
-  // TB/s); 16 tokens 100 -> 79 and 61 -> 49; K of 4096 and 8192 1 to 10 % less. Rows
-  // of 6 KB spread by themselves (160 us, rotated 172). All tiles of an expert and
-  // column block share a start, as they share weights; tiles of 128 rows share
-  // rows of x between column blocks and stay in step (71 us, rotated 80).
+  // x 2048, 128 tokens of 4 on tiles of 32: gate and up 132 -> 95 us, down 67 -> 48
+  // (4.0 -> 5.6 TB/s); 16 tokens 100 -> 79 and 61 -> 49; 256 tokens on tiles of 64
+  // 154 -> 129 and 75 -> 53. Rows of 6 KB spread by themselves (160 us, rotated 172).
+  // Tiles of one expert share its weights and stay in step (70 rows an expert on
+  // tiles of 64: down 115 us, 134 with starts of their own), and so do tiles of 128
+  // rows, whose column blocks share rows of x (71, rotated 80).
   const int KT = (int)(K >> 6);
-  const int start =
-      BM <= 64 && K % 2048 == 0 ? (int)(e * 5u + blockIdx.y * 3u) % KT : 0;
+  const int start = BM <= 64 && K % 2048 == 0 && tile_off[e + 1] == t + 1 &&
+                            tile_off[e] == t
+                        ? (int)(e * 5u + blockIdx.y * 3u) % KT
+                        : 0;
   auto k_of = [&](int kt) {
     const int z = kt + start;
     return (long)(z < KT ? z : z - KT) * 64;
@@ -291,9 +294,16 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
 //   scalar) into a ring of five units of 32 KB: three of A rows and B rows ahead
 //   of those in use, A two steps and B one step before they are needed.
 // At 32 experts of 2048 x 2048, gate and up / down, against eight waves of 128 x
-// 64 with two buffers: 4096 rows an expert 2081 / 1086 -> 1604 / 835 us (1057 /
-// 1013 -> 1371 / 1317 TFLOP/s), 384 rows 277 / 145 -> 242 / 118. A large product of
+// 64 with two buffers: 4096 rows an expert 2081 / 1086 -> 1630 / 840 us (1057 /
+// 1013 -> 1350 / 1309 TFLOP/s), 384 rows 277 / 145 -> 225 / 112. A large product of
 // the library reaches 1.6 PFLOP/s on the same card (8192^3: 675 us).
+//
+// DENSE (mode 5) is a gated linear layer of its own, one matrix over m_rows rows,
+// against the library's product and a pass of silu over its result (2 N columns
+// written and read again): 2 x 3072 x 1024 at 24,000 rows 363 -> 256 us, 2 x 8192 x
+// 2048 at 32,768 rows 1827 -> 1605, 2 x 12288 x 4096 4734 -> 4613, 2 x 25600 x 5120
+// at 8192 rows 3356 -> 2925; the unit's inputs stay in fp32 (error against 64 bits
+// 3.1e-3 -> 1.7e-3).
 //
 // An XCD (workgroup id % 8) takes GW_ROWS neighbouring row tiles and goes through
 // all column blocks with them: its 32 workgroups share 4 row tiles and 8 column
@@ -314,41 +324,75 @@ struct GwTile {
   int n0, e, live;
 };
 
-// where a workgroup is: first row tile of its XCD's group, place in the group
+// where a workgroup is: first row tile of the group, place among its XCD's share
 struct GwWalk {
-  int t0, r8;
+  int t0, place;
 };
 
-// next tile of the walk; lanes hold tile_off and counts where experts are few
-template <int BN>
+// Next tile of the walk. Groups of 8 * GW_ROWS row tiles go through all column
+// blocks, GW_ROWS rows an XCD. The rows that are left go GW_ROWS at a time, every
+// eighth column block an XCD (or, of fewer than 8 column blocks, tile by tile):
+// with rows of their own 1024 x 16384 x 2048 would run on one XCD of eight.
+// Lanes hold tile_off and counts where experts are few; DENSE: one matrix for
+// m_rows rows.
+template <int BN, bool DENSE>
 __device__ __forceinline__ bool gw_next(GwWalk& k, int nb, int total,
-                                        int n_experts, int loff, int lcnt,
-                                        const int* tile_off, const int* counts,
-                                        GwTile& g) {
-  for (; k.t0 < total; k.r8 += gridDim.x >> 3) {
-    while (k.r8 >= GW_ROWS * nb) {
-      k.r8 -= GW_ROWS * nb;
+                                        int n_experts, int m_rows, int loff,
+                                        int lcnt, const int* tile_off,
+                                        const int* counts, GwTile& g) {
+  const int xcd = blockIdx.x & 7;
+  int t, col;
+  for (;;) {
+    const int left = total - k.t0;
+    if (left >= 8 * GW_ROWS) {
+      if (k.place < GW_ROWS * nb) {
+        t = k.t0 + xcd * GW_ROWS + k.place % GW_ROWS;
+        col = k.place / GW_ROWS;
+        break;
+      }
+      k.place -= GW_ROWS * nb;
       k.t0 += 8 * GW_ROWS;
-    }
-    const int t = k.t0 + k.r8 % GW_ROWS;
-    if (t >= total) continue;
-    int first, rows;
-    if (n_experts < 64) {
-      g.e = __builtin_popcountll(__ballot(loff <= t)) - 1;
-      first = __builtin_amdgcn_readlane(loff, g.e);
-      rows = __builtin_amdgcn_readlane(lcnt, g.e);
+    } else if (left <= 0) {
+      return false;
+    } else if (nb >= 8) {
+      const int rows = min(left, GW_ROWS);
+      const int x = (xcd + k.t0 / GW_ROWS) & 7;   // who gets one more varies
+      const int size = rows * ((nb - x + 7) >> 3);
+      if (k.place < size) {
+        col = k.place / rows;
+        t = k.t0 + k.place - col * rows;
+        col = col * 8 + x;
+        break;
+      }
+      k.place -= size;
+      k.t0 += rows;
     } else {
-      g.e = gg_expert(tile_off, n_experts, t);
-      first = tile_off[g.e];
-      rows = counts[g.e];
+      const int item = k.place * 8 + xcd;
+      if (item >= left * nb) return false;
+      t = item / nb;
+      col = item - t * nb;
+      t += k.t0;
+      break;
     }
-    g.n0 = k.r8 / GW_ROWS * BN;
-    g.seg = (long)t * 256;
-    g.live = rows - (t - first) * 256;
-    k.r8 += gridDim.x >> 3;
-    return true;
   }
-  return false;
+  k.place += gridDim.x >> 3;
+  int first, rows;
+  if (DENSE) {
+    g.e = first = 0;
+    rows = m_rows;
+  } else if (n_experts < 64) {
+    g.e = __builtin_popcountll(__ballot(loff <= t)) - 1;
+    first = __builtin_amdgcn_readlane(loff, g.e);
+    rows = __builtin_amdgcn_readlane(lcnt, g.e);
+  } else {
+    g.e = gg_expert(tile_off, n_experts, t);
+    first = tile_off[g.e];
+    rows = counts[g.e];
+  }
+  g.n0 = col * BN;
+  g.seg = (long)t * 256;
+  g.live = rows - (t - first) * 256;
+  return true;
 }
 
 // two floats to bf16 (round to nearest even), the first in the low half
@@ -360,7 +404,7 @@ __device__ __forceinline__ u32 gw_pack(float x, float y) {
   return __builtin_bit_cast(u32, p);
 }
 
-// ANY: gathered rows of 4 GB or more in all, or operands that do not begin at
+// DENSE: see above. ANY: gathered rows of 4 GB or more in all, or operands that do not begin at
 // multiples of 16 bytes; 64-bit addresses and narrow stores then.
 template <int MODE, bool ANY>
 __device__ __forceinline__ void gw_body(
@@ -368,25 +412,27 @@ __device__ __forceinline__ void gw_body(
     const u16* __restrict__ w, const int* __restrict__ row_tok,
     const int* __restrict__ tile_off, const int* __restrict__ counts,
     int n_experts, int n_cols, long K, float limit,
-    const float* __restrict__ row_w) {
+    const float* __restrict__ row_w, int m_rows) {
   constexpr bool GATED = MODE == 1 || MODE >= 3;
-  constexpr bool GATHER = MODE != 0;
+  constexpr bool DENSE = MODE == 5;
+  constexpr bool GATHER = MODE != 0 && !DENSE;
   constexpr int BN = GATED ? 128 : 256;   // output columns
   const int nb = n_cols / BN;
-  const int total = tile_off[n_experts];
+  const int total = DENSE ? (m_rows + 255) / 256 : tile_off[n_experts];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 15, quad = lane >> 4;
   const int wm = wave >> 1, wn = wave & 1;
   extern __shared__ __attribute__((aligned(16))) char gw_smem[];
 
-  const int loff = lane <= n_experts ? tile_off[lane] : 0x7fffffff;
-  const int lcnt = lane < n_experts ? counts[lane] : 0;
-  GwWalk walk = {(int)(blockIdx.x & 7) * GW_ROWS, (int)(blockIdx.x >> 3)};
+  const int loff =
+      !DENSE && lane <= n_experts ? tile_off[lane] : 0x7fffffff;
+  const int lcnt = !DENSE && lane < n_experts ? counts[lane] : 0;
+  GwWalk walk = {0, (int)(blockIdx.x >> 3)};
   GwTile cur;
   auto next = [&](GwTile& g) {
-    return gw_next<BN>(walk, nb, total, n_experts, loff, lcnt, tile_off, counts,
-                       g);
+    return gw_next<BN, DENSE>(walk, nb, total, n_experts, m_rows, loff, lcnt,
+                              tile_off, counts, g);
   };
   if (!next(cur)) return;
 
@@ -407,7 +453,7 @@ __device__ __forceinline__ void gw_body(
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int r = (wave * 8 + j) * 8 + pr;
-      int row = r;
+      int row = DENSE ? min(r, g.live - 1) : r;
       if (GATHER)        // padding rows repeat the last
         row = max(row_tok[g.seg + min(r, g.live - 1)], 0);
       if (ANY)
@@ -450,6 +496,10 @@ __device__ __forceinline__ void gw_body(
   const int arow = wm * 128 * 128;
   const int brow = wn * (GATED ? 64 : 128) * 128;
   f32x4 acc[8][8];                // gated: columns 0 to 3 gate, 4 to 7 up
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = (f32x4)(0.f);
   bf16x8 fa[2][8], fb[2][8];
   auto load_a = [&](int i, int slot, int kk) {
     fa[kk][i] = *(const bf16x8*)(gw_smem + slot + arow + i * 2048 +
@@ -492,13 +542,19 @@ __device__ __forceinline__ void gw_body(
           }
           p[q] = gw_pack(x[0], x[1]);
         }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {       // for the next tile
+          acc[i][j + q] = (f32x4)(0.f);
+          if (GATED) acc[i][(j + q + 4) & 7] = (f32x4)(0.f);
+        }
         const auto s0 =
             __builtin_amdgcn_permlane16_swap(p[0], p[2], false, false);
         const auto s1 =
             __builtin_amdgcn_permlane16_swap(p[1], p[3], false, false);
         const u32x4 pk = {s0[0], s1[0], s0[1], s1[1]};
         u16* o = (u16*)(at + off) + j * 16;
-        if (ANY) {
+        if (DENSE && wm * 128 + i * 16 + ln >= g.live) {
+        } else if (ANY) {
 #pragma unroll
           for (int z = 0; z < 8; ++z)
             o[z] = (u16)(pk[z >> 1] >> ((z & 1) * 16));
@@ -511,11 +567,10 @@ __device__ __forceinline__ void gw_body(
   };
 
   int sa = 0;   // LDS offset of the step's A rows; its B rows are one unit further
-  // FIRST: the sums begin at zero. AHEAD: copies of A and B two steps on, at k2 of
-  // the source. MORE: another step follows, whose operands are read at the end.
-  auto step = [&](int k2, auto first_c, auto ahead_c, auto more_c) {
-    constexpr bool FIRST = decltype(first_c)::v, AHEAD = decltype(ahead_c)::v,
-                   MORE = decltype(more_c)::v;
+  // AHEAD: copies of A and B two steps on, at k2 of the source. MORE: another step
+  // follows, whose operands are read at the end.
+  auto step = [&](int k2, auto ahead_c, auto more_c) {
+    constexpr bool AHEAD = decltype(ahead_c)::v, MORE = decltype(more_c)::v;
     const int sb = wrap(sa + GW_UNIT), na = wrap(sa + 2 * GW_UNIT),
               nbs = wrap(sa + 3 * GW_UNIT), ca = wrap(sa + 4 * GW_UNIT);
 #pragma unroll
@@ -536,8 +591,7 @@ __device__ __forceinline__ void gw_body(
 #pragma unroll
       for (int x = 0; x < 64; ++x) {
         const int i = x >> 3, j = x & 7;
-        acc[i][j] = mfma16g(fb[kk][j], fa[kk][i],
-                            FIRST && kk == 0 ? (f32x4)(0.f) : acc[i][j]);
+        acc[i][j] = mfma16g(fb[kk][j], fa[kk][i], acc[i][j]);
         // reads behind every third product, copies behind every fourth: the LDS
         // takes both beside each other
         if (x % 3 == 0 && x / 3 < 16 && (kk == 0 || MORE)) {
@@ -553,6 +607,16 @@ __device__ __forceinline__ void gw_body(
       }
     }
     sa = na;
+  };
+  // Sums in one half of the registers, operands in the other, wherever steps meet:
+  // the two mixed cost a move in every second instruction.
+  auto keep = [&]() {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
+      asm volatile("" : "+v"(fa[0][i]), "+v"(fb[0][i]));
+    }
   };
   constexpr GwFlag<0> no{};
   constexpr GwFlag<1> yes{};
@@ -596,10 +660,10 @@ __device__ __forceinline__ void gw_body(
     for (;;) {
       open();
       if (KT == 2) {
-        step(0, yes, no, yes);
-        step(0, no, no, no);
+        step(0, no, yes);
+        step(0, no, no);
       } else {
-        step(0, yes, no, no);
+        step(0, no, no);
       }
       store_tile(cur);
       if (!next(cur)) return;
@@ -609,21 +673,21 @@ __device__ __forceinline__ void gw_body(
   }
   open();
   for (;;) {
-    step(kc, yes, yes, yes);
-    advance();
     GwTile nxt;
     Source after;
     const bool more = next(nxt);
     if (more) point(nxt, after);
     const int last = more ? KT : KT - 2;
-    for (int s = 1; s < last; ++s) {
+    keep();
+    for (int s = 0; s < last; ++s) {
       if (s == KT - 2) src = after;   // the copies are the next tile's now
-      step(kc, no, yes, yes);
+      step(kc, yes, yes);
+      keep();
       advance();
     }
     if (!more) {
-      step(0, no, no, yes);
-      step(0, no, no, no);
+      step(0, no, yes);
+      step(0, no, no);
     }
     store_tile(cur);
     if (!more) return;
@@ -637,9 +701,15 @@ gw_kernel(u16* __restrict__ out, const u16* __restrict__ a,
           const u16* __restrict__ w, const int* __restrict__ row_tok,
           const int* __restrict__ tile_off, const int* __restrict__ counts,
           int n_experts, int n_cols, long K, float limit,
-          const float* __restrict__ row_w) {
+          const float* __restrict__ row_w, int m_rows) {
   gw_body<MODE, ANY>(out, a, w, row_tok, tile_off, counts, n_experts, n_cols, K,
-                     limit, row_w);
+                     limit, row_w, m_rows);
+}
+
+// a workgroup a CU, a multiple of 8 of them
+static unsigned gw_grid(long tiles, int blocks) {
+  const long work = (tiles * blocks + 7) / 8 * 8;
+  return (unsigned)(work < GW_CUS ? work : GW_CUS);
 }
 
 static void grouped_gemm_launch(void* out, const void* a, long a_rows,
@@ -673,10 +743,7 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
       n_experts, n_cols, K, limit, row_w
   const bool gated = gate_silu == 1 || gate_silu >= 3;
   if (bm == 256) {
-    const unsigned groups = (unsigned)((max_tiles + 8 * GW_ROWS - 1) /
-                                       (8 * GW_ROWS));
-    const unsigned work = groups * 8 * GW_ROWS * (n_cols / (gated ? 128 : 256));
-    const dim3 grid(work < GW_CUS ? work : GW_CUS);
+    const dim3 grid(gw_grid(max_tiles, n_cols / (gated ? 128 : 256)));
     const bool any = (gate_silu && a_rows >= (0xf0000000l / 2) / K) ||
                      (((size_t)out | (size_t)a | (size_t)w) & 15);
 #define GG_WIDE_AS(M, ANY)                                                  \
@@ -684,7 +751,7 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
     static std::atomic<unsigned long long> asked{0};                        \
     lds_limit((const void*)gw_kernel<M, ANY>, GW_LDS, asked);               \
     hipLaunchKernelGGL((gw_kernel<M, ANY>), grid, dim3(256), GW_LDS,        \
-                       stream, GG_ARGS);                                    \
+                       stream, GG_ARGS, 0);                                 \
   }
 #define GG_WIDE(M)                                                          \
   {                                                                         \
@@ -723,6 +790,20 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
   else if (gate_silu == 2) GG_LAUNCH(2, 64, 64, 2, 2)
   else GG_LAUNCH(0, 64, 64, 2, 2)
 #undef GG_LAUNCH
+}
+
+// out [M, N] = silu(x Wg^T) * (x Wu^T): w [2 N, K], the gate's rows first. x and
+// w at multiples of 16 bytes, K a multiple of 64, N of 128, M K below 2 G.
+extern "C" void sutro_linear_silu_mul(void* out, const void* x, const void* w,
+                                      int M, int N, long K,
+                                      hipStream_t stream) {
+  static std::atomic<unsigned long long> asked{0};
+  lds_limit((const void*)gw_kernel<5, false>, GW_LDS, asked);
+  hipLaunchKernelGGL((gw_kernel<5, false>),
+                     dim3(gw_grid(((long)M + 255) / 256, N / 128)), dim3(256),
+                     GW_LDS, stream, (u16*)out, (const u16*)x,
+                     (const u16*)w, nullptr, nullptr, nullptr, 0, N, K, 0.f,
+                     nullptr, M);
 }
 
 extern "C" void sutro_grouped_gemm(void* out, const void* a, long a_rows,

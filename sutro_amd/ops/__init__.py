@@ -253,10 +253,41 @@ def linear(x, w, bias=None):
     return F.linear(x, w, bias)
 
 
+def _many_rows(x, w) -> bool:
+    """Whether csrc/grouped_gemm.hip makes silu_mul(x w^T) in one launch. Its
+    tiles are 256 rows by 128 columns of the result, one a CU at a time: below
+    256 of them the library's smaller tiles are ahead (us of both, tiles):
+      2 x 3072 x 1024    1024 rows  25.1 /  26.7 ( 96)   2048   36.2 / 29.2 (192)
+      2 x 6144 x 2048     512 rows  33.4 /  42.6 ( 96)   1024   53.6 / 48.9 (192)
+      2 x 8192 x 2048     512 rows  39.7 /  45.5 (128)   1024   66.5 / 54.2 (256)
+      2 x 9728 x 2560     512 rows  58.7 /  96.8 (152)   1024    107 /  108 (304)
+      2 x 12288 x 4096   1024 rows   173 /   170 (384)   1500    257 /  258 (576)
+    and from there on it is 2 to 45 % faster, or as fast (the figures at many
+    rows stand beside the kernel)."""
+    if (type(x) is not torch.Tensor or _tracing()
+            or type(w) not in (torch.Tensor, torch.nn.Parameter)):
+        return False
+    if x.dim() != 2 or w.dim() != 2 or not _use_hip(x):
+        return False
+    M, K = x.shape
+    rows = w.shape[0]
+    return (rows % 256 == 0 and -(-M // 256) * (rows // 256) >= 256
+            and K % 64 == 0 and 0 < K < 1 << 21 and M * K < 1 << 30
+            and rows < 1 << 24 and w.shape[1] == K and _unwatched()
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and w.device == x.device and x.is_contiguous()
+            and w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
 def linear_silu_mul(x, w):
     """silu_mul(x w^T), w the gate's rows and then the up's."""
     if _few_rows(x, w, gated=True):
         return _require_hip().linear_skinny(x, w, None, True)
+    if _many_rows(x, w):
+        return _require_hip().linear_silu_mul(x, w)
     return silu_mul(F.linear(x, w))
 
 
@@ -266,20 +297,21 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
     for `n_rows` (token, expert) pairs in bf16 on the matrix cores (K and N
     multiples of 64), by the rows an expert gets on average. Taller tiles do
     more work per byte but pad more; both products together, at 32 experts of
-    2048 x 2048: at 96 rows 281 / 213 / 233 us on tiles of 64 / 128 / 256, at
-    192 rows 393 / 340 / 232, at 384 rows 952 / 511 / 360.
+    2048 x 2048: at 96 rows 281 / 213 / 219 us on tiles of 64 / 128 / 256, at
+    192 rows 393 / 340 / 218, at 384 rows 952 / 510 / 340.
 
     They also leave fewer workgroups: one of 256 rows takes 128 columns of the
     gated product or 256 of the other, and below 128 of them in either product
     the chip idles. 8 experts of 1024 x 512, 192 / 512 / 1024 rows an expert (24 /
-    64 / 128 of either) 26 / 40 / 63 us on 64, 33 / 37 / 47 on 128, 45 / 44 / 43 on
-    256; 8 of 2048 x 2048 at 384 / 512 rows (96 / 128 of the second) 183 / 245 on
-    64, 132 / 146 on 128, 148 / 147 on 256. Tiles of 128 want 96.
+    64 / 128 of either) 26 / 40 / 63 us on 64, 33 / 37 / 47 on 128, 41 / 42 / 44 on
+    256. (8 of 2048 x 2048 would already gain with 64 to 96 of the second, 192 /
+    384 rows: 81 / 131 us on 128, 83 / 99 on 256; the line is the one that holds
+    for both.) Tiles of 128 want 96.
 
     Up to 16 rows, where the weights are all there is to read, tiles of 32: four
     workgroups of the gated product fit a CU instead of three. They are taken
     unless their number then fills the rounds worse: 1024 workgroups (2048 wide)
-    222 -> 200 us, 1536 (3072 wide, K 4096) 431 -> 445.
+    167 -> 140 us, 1536 (3072 wide, K 4096) 438 -> 445.
 
     `local`: the experts whose products this rank makes (all by default); its
     workgroups are counted."""
