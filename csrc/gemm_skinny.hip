@@ -5,11 +5,13 @@
 // Bound by the weights, which are read once, and for the small matrices of a
 // step by the time to get enough loads in flight. A workgroup owns 16 or 32
 // rows of W (gated: 16 and 16) and its waves split k, each with a batch of
-// fragments ahead of its products (gemm_stream.h); their sums meet in LDS. The
-// split is as fine as leaves every wave four k-steps, so that also a 2048 x
-// 2048 matrix keeps 2000 waves of loads in flight. Against the library: 2048 x
-// 2048 at 16 rows 11.0 -> 6.5 us, 4096 x 4096 15.5 -> 12.5; at more rows or
-// longer k the waves read too much of x, which nothing shares.
+// fragments ahead of its products (gemm_stream.h); their sums meet in LDS. Two
+// waves with long runs are the faster ones (a wave that ends after a batch or two
+// has nothing in flight while its workgroup adds up): 16 rows, 6144 x 4096 on 8
+// waves of 16 rows of W 22.1 -> 14.9 us on 2 of 32, 18432 x 2048 28.0 -> 22.9,
+// 5120 x 25600 111 -> 72. Only where a CU has no more than one workgroup do more
+// waves pay: 2048 x 2048 6.5 on 2, 6.3 on 16 (a batch each); 4096 x 4096 at 8 rows
+// 10.3 on 2, 9.4 on 4.
 #include "common.h"
 #include "gemm_stream.h"
 
@@ -23,7 +25,7 @@ struct SkinnyArgs {
   int act;           // 0 none, 1 silu(gate) up (W has 2 N rows)
 };
 
-template <int NF, int MB, int WAVES, bool GATED>
+template <int NF, int MB, int WAVES, bool GATED, bool SPREAD>
 __global__ void __launch_bounds__(WAVES * 64) skinny_kernel(SkinnyArgs A) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -50,7 +52,10 @@ __global__ void __launch_bounds__(WAVES * 64) skinny_kernel(SkinnyArgs A) {
   for (int i = 0; i < NF; ++i)
 #pragma unroll
     for (int m = 0; m < MB; ++m) acc[i][m] = (f32x4)(0.f);
-  if (s1 > s0) gs_dot<NF, MB>(wp, ap, s1 - s0, acc);
+  const int n = s1 - s0;
+  if (n > 0)
+    gs_dot<NF, MB, SPREAD>(wp, ap, n, SPREAD ? (int)(blockIdx.x * 4u) % n : 0,
+                           acc);
 
   __shared__ f32x4 red[WAVES][NF][MB][64];
 #pragma unroll
@@ -187,14 +192,21 @@ static void skinny_launch(const SkinnyArgs& A, hipStream_t s) {
   const unsigned blocks = (A.N + (GATED ? 16 : NF * 16) - 1) /
                           (GATED ? 16 : NF * 16);
   const int steps = A.K / GS_STEP;
-#define LAUNCH_SK(WW)                                                        \
-  hipLaunchKernelGGL((skinny_kernel<NF, MB, WW, GATED>), dim3(blocks),       \
-                     dim3(WW * 64), 0, s, A)
-  // waves that split k: toward 2048 in all, at least four k-steps each
-  if (blocks >= 1024 || steps < 16) LAUNCH_SK(2);
-  else if (blocks >= 512 || steps < 32) LAUNCH_SK(4);
-  else if (blocks >= 256 || steps < 64) LAUNCH_SK(8);
-  else LAUNCH_SK(16);
+#define LAUNCH_SK(WW, SPREAD)                                                \
+  hipLaunchKernelGGL((skinny_kernel<NF, MB, WW, GATED, SPREAD>),             \
+                     dim3(blocks), dim3(WW * 64), 0, s, A)
+  // Weight rows 8 KB apart lie on few memory channels where all workgroups read
+  // the same columns of them: starts are spread. 32768 x 4096 at 3 rows 62 -> 51 us,
+  // 8192 x 4096 16.2 -> 14.2; rows of 4 KB or fewer than 8192 of them 0 to 10 % more.
+  // Waves: see the top.
+  const bool spread = A.K % 4096 == 0 && (GATED ? 2 : 1) * A.N >= 8192;
+  if (spread) LAUNCH_SK(2, true);
+  else if ((NF == 2 && !GATED) || blocks > 256 ||
+           (steps > 64 && A.M > 8))
+    LAUNCH_SK(2, false);
+  else if (steps > 64) LAUNCH_SK(4, false);
+  else if (steps > 32) LAUNCH_SK(16, false);
+  else LAUNCH_SK(8, false);
 #undef LAUNCH_SK
 }
 
@@ -221,8 +233,13 @@ extern "C" void sutro_linear_skinny(void* out, long ldo, const void* x,
     if (mb == 1) skinny_launch<NF, 1, GG>(A, s);                             \
     else skinny_launch<NF, 2, GG>(A, s);                                     \
   } while (0)
+  // 32 rows of W a workgroup read half as much of x, but where they take more
+  // rounds of the chip than 16 do: 10304 x 4096 at 16 rows 30.6 and 27.0 us, 6144 x
+  // 4096 14.9 and 18.3
+  const int rounds16 = (N + 16 * 256 - 1) / (16 * 256);
+  const int rounds32 = (N + 32 * 256 - 1) / (32 * 256);
   if (act == 1) SK_MB(2, true);
-  else if (N >= 8192) SK_MB(2, false);
+  else if (2 * rounds32 <= rounds16) SK_MB(2, false);
   else SK_MB(1, false);
 #undef SK_MB
 }

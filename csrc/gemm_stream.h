@@ -21,17 +21,21 @@ __device__ __forceinline__ u32x2 gs_pack4(f32x4 v) {
   return __builtin_bit_cast(u32x2, __builtin_convertvector(v, gs_bf16x4));
 }
 
-// acc[i][m] += sum over k-steps [0, steps) of W_i (16 rows) x A_m (16 rows);
-// wp / ap: this lane's row of every block at its k chunk, steps >= 1
-template <int NF, int MB>
+// acc[i][m] += sum over k-steps [0, steps) of W_i (16 rows) x A_m (16 rows), ROUND:
+// from step `first` (0 <= first < steps) on and round; wp / ap: this lane's row of
+// every block at its k chunk, steps >= 1
+template <int NF, int MB, bool ROUND>
 __device__ __forceinline__ void gs_dot(const u16* const (&wp)[NF],
                                        const u16* const (&ap)[MB], int steps,
+                                       int first,
                                        f32x4 (&acc)[NF][MB]) {
   s16x8 w[2][GS_BATCH][NF], a[2][GS_BATCH][MB];
   auto load = [&](int buf, int s0) {
 #pragma unroll
     for (int u = 0; u < GS_BATCH; ++u) {
-      const int s = min(s0 + u, steps - 1);  // the tail repeats (not used)
+      int s = min(s0 + u, steps - 1);  // the tail repeats (not used)
+      if (ROUND) s += first;
+      if (ROUND && s >= steps) s -= steps;
 #pragma unroll
       for (int i = 0; i < NF; ++i)
         w[buf][u][i] = *(const s16x8*)(wp[i] + s * GS_STEP);

@@ -197,28 +197,51 @@ def _two_rows(rows: int, K: int, gated: bool) -> bool:
             or (rows > 8192 and K <= 5120) or (rows < 8192 and K >= 16384))
 
 
+def _long_weights(M: int, rows: int, K: int) -> bool:
+    """Larger matrices over 3 to 32 rows (both sides in `_few_rows`)."""
+    if 16384 < rows <= 24576 and rows * K < 96 << 20 and K <= 4096:
+        return M <= 16                    # the library has no good tile there
+    if rows <= 8192 and K <= 4096:
+        return M <= 12
+    if K <= 2048 or K == 4096:
+        return M <= (8 if rows * K <= 1 << 28 else 6) and (
+            rows <= 24576 or K >= 2048)
+    return rows <= 5120 and K >= 16384 and K % 4096 != 0    # nor there
+
+
 def _few_rows(x, w, gated: bool = False) -> bool:
     """Whether csrc/gemm_skinny.hip is the faster one for x [M, K] w^T. The
-    library takes 11 us or more for any product; us by it and by the kernel,
+    library takes 11 us or more for most products; us by it and by the kernel,
     weights from memory:
-      rows of w x K    M = 1          2             3             16            32
-      2048 x 2048      11.0 /  4.8    10.7 /  5.9   10.7 /  5.2   10.7 /  6.4   10.9 /  8.6
-      3072 x 2048      11.5 /  5.1    11.1 /  6.5   11.1 /  5.6   11.0 /  6.7   11.2 /  9.0
-      2048 x 3072      12.1 /  5.2    11.9 /  6.3   11.9 /  7.1   11.8 /  9.3   10.1 / 13.9
-      4096 x 4096      15.4 /  7.8    15.2 / 10.0   15.2 /  9.7   15.4 / 12.4   13.0 / 17.3
-      2048 x 8192      12.6 /  8.2    12.5 / 10.2   12.4 / 15.4   13.0 / 21.8
-      6144 x 4096      15.6 / 10.9    15.3 / 13.0   14.3 / 16.0   14.3 / 22.1
-      5120 x 5120      13.6 / 12.0    13.9 / 14.8   13.7 / 17.4   15.2 / 24.9
-      8192 x 4096      17.1 / 14.7    16.5 / 18.3
+      rows of w x K    M = 1          2             3             8             16            32
+      2048 x 2048      11.0 /  4.8    10.7 /  5.9   11.1 /  5.3   11.0 /  5.6   11.0 /  6.3   11.2 /  8.5
+      4096 x 2048                                   11.6 /  6.3   11.6 /  6.4   11.6 /  7.1   11.8 /  9.2
+      6144 x 2048                                   13.0 /  8.9   12.7 /  9.4   12.5 /  9.0   12.6 / 11.8
+      10240 x 2048                                  16.2 / 11.9   16.0 / 13.6   14.2 / 15.3   14.2 / 21.6
+      18432 x 2048                                  57.6 / 19.2   57.4 / 20.3   57.4 / 24.5   20.6 / 34.7
+      32768 x 2048                                  34.0 / 30.3   31.8 / 30.2   31.7 / 33.3   34.0 / 41.1
+      151936 x 2048                                  205 / 126     204 / 137     202 / 155     145 / 193
+      8192 x 3072                                   19.3 / 12.7   17.2 / 12.3   17.2 / 12.9   17.3 / 17.5
+      16384 x 3072                                  22.5 / 22.9   21.4 / 23.4   21.5 / 26.5   21.6 / 35.1
+      4096 x 4096      15.4 /  7.8    15.2 / 10.0   15.7 /  9.1   15.5 /  9.4   15.4 / 10.9   13.0 / 14.0
+      6144 x 4096      15.6 / 10.9    15.3 / 13.0   15.6 / 14.5   14.5 / 13.9   14.4 / 14.8   15.2 / 20.2
+      8192 x 4096      17.1 / 14.7    16.5 / 18.3   16.7 / 15.2   15.8 / 14.6   15.8 / 15.5   16.4 / 20.3
+      12288 x 4096                                  27.8 / 21.5   26.7 / 23.1   26.5 / 28.5   23.1 / 39.7
+      20000 x 4096                                  67.2 / 34.5   67.0 / 37.6   67.1 / 46.0   38.7 / 64.9
+      32768 x 4096     63.2 / 49.5    62.9 / 56.1   61.3 / 53.6   58.9 / 54.9   59.0 / 61.9   63.0 / 74.8
+      65536 x 4096                                   122 / 104     120 / 107     120 / 121     122 / 178
+      5120 x 5120      13.6 / 12.0    13.9 / 14.8   13.9 / 15.3   14.2 / 16.6   15.4 / 19.1   18.0 / 27.8
       12288 x 5120     26.8 / 23.9    25.9 / 25.7
       12288 x 12288    61.0 / 60.6    60.7 / 64.9
-      5120 x 25600      135 / 51       136 / 57      136 / 79      139 / 116
-      32768 x 4096     63.2 / 49.5    62.9 / 56.1   63.1 / 67.0   60.9 / 69.1
+      4096 x 16384                                  30.8 / 31.3   29.8 / 31.1   29.8 / 36.6   33.7 / 46.0
+      5120 x 17408                                   111 / 43      112 / 46      114 / 52      121 / 77
+      5120 x 25600      135 / 51       136 / 57      134 / 60      135 / 64      137 / 72      145 / 108
     and with silu_mul behind it (rows of both halves)
-      4096 x 2048      13.8 /  5.6    13.6 /  7.0   13.6 /  8.4   13.9 /  9.7   13.9 / 13.4
-      16384 x 2048     20.8 / 14.0    20.3 / 17.6   20.4 / 17.5   20.6 / 21.1   19.3 / 24.1
+      4096 x 2048      13.8 /  5.6    13.6 /  7.0   14.2 /  8.5   14.2 /  9.1   14.1 /  9.8   14.3 / 14.0
+      16384 x 2048     20.8 / 14.0    20.3 / 17.6   20.7 / 15.8   19.5 / 16.1   19.5 / 18.0   19.7 / 22.9
+      24576 x 4096                                  46.7 / 41.6   45.3 / 42.0   45.6 / 46.4   46.0 / 58.1
       12288 x 8192     43.9 / 42.4    43.8 / 47.5
-      51200 x 5120     98.8 / 92.3    99.1 / 95.9   99.3 / 143
+      51200 x 5120     98.8 / 92.3    99.1 / 95.9   95.6 / 134    92.3 / 139    92.8 / 158    95.8 / 196
     Two rows lose where the library has a good tile (24 to 64 M weights of long
     rows) and one load a weight row is no longer the whole cost."""
     if (type(x) is not torch.Tensor or _tracing()
@@ -230,7 +253,8 @@ def _few_rows(x, w, gated: bool = False) -> bool:
     rows = w.shape[0]
     fits = (M == 1 or (M == 2 and _two_rows(rows, K, gated))
             or (M <= 16 and K <= 4096 and rows * K <= 1 << 24)
-            or (K <= 2048 and rows * K <= 1 << 23))
+            or (K <= 2048 and rows * K <= 1 << 23)
+            or (M > 2 and _long_weights(M, rows, K)))
     return (fits and _unwatched() and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.device == x.device
             and w.dim() == 2 and w.shape[1] == K and K % 32 == 0 and K > 0
