@@ -6,7 +6,8 @@
 // kept first keys, a logarithmic distance bias, sinks, output gates and an
 // output section.
 //
-// Both kernels make S^T = K Q^T, so a lane holds the scores of ONE query row:
+// Both kernels make S^T = K Q^T, so a lane holds scores of ONE query row (a prompt's
+// waves of 32 rows: of two, each in registers of its own):
 // softmax is lane-local, the weights are already in the B layout of
 // O^T += V^T P^T (with the contraction index permuted alike on both sides) and
 // never pass through LDS, and rescaling O is one multiplication by a lane's own
@@ -16,8 +17,6 @@
 // weights hold without loss of relative precision.
 //
 // Fragment layouts (gfx950), lane l:
-//   mfma_f32_32x32x16_bf16: A[l%32][(l/32)*8 + j], B[(l/32)*8 + j][l%32],
-//     D[(r&3) + 8*(r>>2) + 4*(l/32)][l%32], r = 0..15
 //   mfma_f32_16x16x32_bf16: A[l%16][(l/16)*8 + j], B[(l/16)*8 + j][l%16],
 //     D[(l/16)*4 + r][l%16], r = 0..3
 //   ds_read_tr16_b64: in a group of 16 lanes lane i addresses the 4 columns
@@ -77,9 +76,6 @@ struct PagedArgs {
   float out_scale;
 };
 
-__device__ __forceinline__ f32x16 pa_mfma32(pa_frag a, pa_frag b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
 __device__ __forceinline__ f32x4 pa_mfma16(pa_frag a, pa_frag b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
@@ -105,18 +101,27 @@ __device__ __forceinline__ pa_frag pa_tr(const char* a, const char* b) {
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 // Issue order of a run of LDS reads feeding matrix products: AHEAD reads first,
-// then EACH reads behind every product (left alone, the compiler waits for
-// every fragment in front of its product).
-template <int READS, int MFMAS, int AHEAD, int EACH>
+// then EACH reads behind every PER products of MFMAS times PER (left alone, the
+// compiler waits for every fragment in front of its product).
+template <int READS, int MFMAS, int AHEAD, int EACH, int PER = 1>
 __device__ __forceinline__ void pa_order() {
   constexpr int STEPS = (READS - AHEAD) / EACH;
   __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, PER, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);
   }
-  __builtin_amdgcn_sched_group_barrier(0x8, MFMAS - STEPS, 0);
+  __builtin_amdgcn_sched_group_barrier(0x8, (MFMAS - STEPS) * PER, 0);
+}
+// maximum over the four lanes of equal lane % 16
+__device__ __forceinline__ float pa_max4(float v) {
+  const u32 x = __float_as_uint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  const u32 y = __float_as_uint(
+      fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+  const auto b = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 // 8 cached elements as they are stored, and as bf16
 template <bool KV8> struct PaRaw { typedef u16x8 type; };
@@ -168,6 +173,12 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 // 0.22 ms on 160 short ones (24 k tokens). Two workgroups a CU (64 KB of LDS,
 // up to 256 registers a lane) are what both limits allow.
 //
+// Products are of 16 x 16 x 32: those of 32 x 32 x 16 do as much a cycle but read
+// and write every sum twice as often, which the power limit takes off the clock.
+// 32 k prompt (16 heads, 4 kv heads, 128) 4.59 -> 4.19 ms (958 -> 1050 TFLOP/s), 16 of
+// 2 k 359 -> 338 us, 7 of 3 k with 32 heads over e4m3 605 -> 560, 2 of 20 k with 16
+// heads of 64 2.19 -> 2.05 ms, 16 of 2 k in chunks of 1024 251 -> 243 us.
+//
 // BLOCKS: more than one block of rows in a workgroup.
 //
 // Entries of the tile map that continue each other (same sequence, 32 rows on)
@@ -183,7 +194,7 @@ paged_prefill_kernel(PagedArgs A) {
   constexpr int PER = TILE / 1024;          // 1 KB pieces per tile
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ln = lane & 31, hi = lane >> 5;
+  const int ln = lane & 15, g = lane >> 4;
   // heads vary fastest: workgroup id i runs on XCD i % 8, so an XCD works on
   // few kv heads and the tiles that share their pages meet in its L2; long
   // contexts first. Entries rpb apart follow each other, the rest comes after
@@ -214,42 +225,46 @@ paged_prefill_kernel(PagedArgs A) {
   const int L = pa_same(A.seq_lens[s]);
   const int p0 = L - nq_total + q0;         // position of the first row
   const int kv_end = p0 + rows;             // causal bound (exclusive)
-  const int my_r = rb * 32 + ln;            // this lane's row of the workgroup
-  const int my_p = p0 + my_r;
+  // this lane's rows of the workgroup, one of each sixteen, and their positions
+  const int my_r[2] = {rb * 32 + ln, rb * 32 + 16 + ln};
+  const int my_p[2] = {p0 + my_r[0], p0 + my_r[1]};
   const bool live = rb * 32 < rows && head < A.G;     // this wave has work
   const int w_end = min(kv_end, p0 + rb * 32 + 32);
 
   extern __shared__ __attribute__((aligned(16))) char pa_smem[];
 
-  pa_frag qb[D / 16];
-  {
-    const u16* qp =
-        A.q + ((long)(row_base + min(my_r, rows - 1)) * A.Hq + hq) * D + hi * 8;
+  pa_frag qb[2][D / 32];
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
-      qb[kk] = *(const s16x8*)(qp + kk * 16);
+  for (int u = 0; u < 2; ++u) {
+    const u16* qp =
+        A.q + ((long)(row_base + min(my_r[u], rows - 1)) * A.Hq + hq) * D +
+        g * 8;
+#pragma unroll
+    for (int kk = 0; kk < D / 32; ++kk) {
+      qb[u][kk] = *(const s16x8*)(qp + kk * 32);
       // scores are compared before they are scaled: by a positive number
-      if (A.scale < 0.f) qb[kk] ^= (short)0x8000;
+      if (A.scale < 0.f) qb[u][kk] ^= (short)0x8000;
     }
   }
   const float scale = fabsf(A.scale);
-  f32x16 acc[D / 32];
+  f32x4 acc[D / 16][2];
 #pragma unroll
-  for (int b = 0; b < D / 32; ++b) acc[b] = (f32x16)(0.f);
-  float m_run = PA_NONE, l_run = 0.f;
+  for (int b = 0; b < D / 16; ++b) acc[b][0] = acc[b][1] = (f32x4)(0.f);
+  float m_run[2] = {PA_NONE, PA_NONE}, l_run[2] = {0.f, 0.f};
   if (LOCAL && A.sink) {
-    m_run = A.sink_w ? A.sink_w[hq] * PA_LOG2E : 0.f;
-    l_run = hi == 0 ? 1.f : 0.f;            // the lane pair's sums are added
+    m_run[0] = m_run[1] = A.sink_w ? A.sink_w[hq] * PA_LOG2E : 0.f;
+    l_run[0] = l_run[1] = g == 0 ? 1.f : 0.f;   // four lanes' sums are added
   }
   const float r1 = LOCAL && A.r1 ? A.r1[hq] : 0.f;
   const float r2 = LOCAL && A.r1 ? A.r2[hq] : 0.f;
   // lower key bounds: of this lane's row, of the workgroup's first row, and of
   // this wave's last row (above which a step needs no mask)
-  int lo_row = 0, c_row = 0, kt0 = 0, kf0 = 0, n_kept = 0, lo_last = 0;
+  int lo_row[2] = {0, 0}, c_row[2] = {0, 0}, kt0 = 0, kf0 = 0, n_kept = 0, lo_last = 0;
   int lo_first = 0, c_first = 0, w_lo = 0, w_c = 0;  // w: this wave's first row
   if (LOCAL) {
     int c_last;
-    lo_row = pa_lower(A, my_p, c_row);
+    lo_row[0] = pa_lower(A, my_p[0], c_row[0]);
+    lo_row[1] = pa_lower(A, my_p[1], c_row[1]);
     lo_first = pa_lower(A, p0, c_first);
     lo_last = pa_lower(A, w_end - 1, c_last);
     w_lo = pa_lower(A, p0 + rb * 32, w_c);
@@ -257,7 +272,8 @@ paged_prefill_kernel(PagedArgs A) {
     kf0 = c_first / PA_KEYS;
     n_kept = max(min(kt0, (A.keep_first + PA_KEYS - 1) / PA_KEYS) - kf0, 0);
   }
-  const u32 kept_n = max(A.keep_first - c_row, 0);
+  const u32 kept_n[2] = {(u32)max(A.keep_first - c_row[0], 0),
+                         (u32)max(A.keep_first - c_row[1], 0)};
   const int kt1 = (kv_end + PA_KEYS - 1) / PA_KEYS;
   const int steps = n_kept + kt1 - kt0;
   const int last_page = (kv_end - 1) / PA_PG;
@@ -318,20 +334,18 @@ paged_prefill_kernel(PagedArgs A) {
       *(u16x8*)(buf + (j * 4 + w) * 1024 + lane * 16) = pa_widen<KV8>(st[j]);
   };
 
-  // fragment addresses: keys row ln (+32), chunk kk*2 + hi; values rows
-  // 4*hi + ti/4 (+8), columns of 32-block b
-  int kad[4];
+  // fragment addresses: keys row ln (+16 a tile), chunk kk*4 + g; values rows
+  // 4*g + ti/4 (+16), columns of 16-block b
+  int kad[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    kad[j] = ln * (2 * D) + pa_kchunk(ln, j * 2 + hi) * 16;
+  for (int j = 0; j < 2; ++j)
+    kad[j] = ln * (2 * D) + pa_kchunk(ln, j * 4 + g) * 16;
   const int ti = lane & 15;
-  int vad[2];
+  int vad[4];
 #pragma unroll
-  for (int o = 0; o < 2; ++o)
-    vad[o] = (4 * hi + (ti >> 2)) * (2 * D) +
-             pa_vchunk(ti >> 2,
-                       o * 4 + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) * 16 +
-             (ti & 1) * 8;
+  for (int o = 0; o < 4; ++o)
+    vad[o] = (4 * g + (ti >> 2)) * (2 * D) +
+             pa_vchunk(ti >> 2, o * 2 + ((ti & 3) >> 1)) * 16 + (ti & 1) * 8;
 
   pages(step_tile(0));
   load();
@@ -364,114 +378,140 @@ paged_prefill_kernel(PagedArgs A) {
     const char* kb = pa_smem + (it & 1) * 2 * TILE;
     const char* vb = kb + TILE;
 
-    f32x16 d[2];
+    f32x4 d[2][4];      // scores: row u, keys kv0 + t*16 + 4*g + r
 #pragma unroll
-    for (int h = 0; h < 2; ++h) d[h] = (f32x16)(0.f);
+    for (int t = 0; t < 4; ++t) d[0][t] = d[1][t] = (f32x4)(0.f);
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk)
+    for (int kk = 0; kk < D / 32; ++kk)
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        d[h] = pa_mfma32(*(const s16x8*)(kb + kad[kk & 3] + (kk >> 2) * 128 +
-                                         h * 32 * 2 * D),
-                         qb[kk], d[h]);
-    pa_order<D / 8, D / 8, 6, 1>();
-    // ---- scores: this lane's row, keys kv0 + h*32 + (r&3) + 8*(r>>2) + 4*hi;
-    // without a distance bias they stay unscaled until the exponential
-    float tmax = PA_NONE;
+      for (int t = 0; t < 4; ++t) {
+        const pa_frag ka = *(const s16x8*)(kb + kad[kk & 1] + (kk >> 1) * 128 +
+                                           t * 16 * 2 * D);
+        d[0][t] = pa_mfma16(ka, qb[0][kk], d[0][t]);
+        d[1][t] = pa_mfma16(ka, qb[1][kk], d[1][t]);
+      }
+    pa_order<D / 8, D / 8, 6, 1, 2>();
+    // without a distance bias scores stay unscaled until the exponential
     const bool whole = kv0 + PA_KEYS <= p0 + rb * 32 + 1 &&
                        (!LOCAL || kv0 >= lo_last);
     const bool biased = (LOCAL && A.r1) || scale < 1e-20f;
     if (biased) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kp = kv0 + h * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          d[h][r] = d[h][r] * scale -
-                    r1 * __builtin_amdgcn_logf(
-                             1.f + r2 * (float)max(my_p - kp, 0));
-        }
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kp = kv0 + t * 16 + 4 * g + r;
+            d[u][t][r] =
+                d[u][t][r] * scale -
+                r1 * __builtin_amdgcn_logf(
+                         1.f + r2 * (float)max(my_p[u] - kp, 0));
+          }
     }
     const float mul = biased ? 1.f : scale;
     if (!whole) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kp = kv0 + h * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          bool vis = kp <= my_p;
-          if (LOCAL)  // no short circuits: 32 selects, not 32 branches
-            vis &= (kp >= lo_row) | ((u32)(kp - c_row) < kept_n);
-          d[h][r] = vis ? d[h][r] : -INFINITY;
-        }
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kp = kv0 + t * 16 + 4 * g + r;
+            bool vis = kp <= my_p[u];
+            if (LOCAL)  // no short circuits: 32 selects, not 32 branches
+              vis &= (kp >= lo_row[u]) | ((u32)(kp - c_row[u]) < kept_n[u]);
+            d[u][t][r] = vis ? d[u][t][r] : -INFINITY;
+          }
     }
+    float tmax[2];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, fmaxf(d[0][r], d[1][r]));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * mul;
-    const bool up = tmax > m_run + PA_SLACK;
-    if (__any(up)) {
-      const float m_new = up ? tmax : m_run;
-      const float al = __builtin_amdgcn_exp2f(m_run - m_new);
-      m_run = m_new;
-      l_run *= al;
+    for (int u = 0; u < 2; ++u) {
+      float m = PA_NONE;
 #pragma unroll
-      for (int b = 0; b < D / 32; ++b)
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[b][r] *= al;
+        for (int r = 0; r < 4; ++r) m = fmaxf(m, d[u][t][r]);
+      tmax[u] = pa_max4(m) * mul;
+    }
+    const bool up0 = tmax[0] > m_run[0] + PA_SLACK,
+               up1 = tmax[1] > m_run[1] + PA_SLACK;
+    if (__any(up0 | up1)) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float m_new = (u ? up1 : up0) ? tmax[u] : m_run[u];
+        const float al = __builtin_amdgcn_exp2f(m_run[u] - m_new);
+        m_run[u] = m_new;
+        l_run[u] *= al;
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b) acc[b][u] *= al;
+      }
     }
     // a row that has seen no key yet: every weight is exp2(-inf) = 0
-    const float m_sub = LOCAL && m_run < 0.1f * PA_NONE ? 0.f : m_run;
+    float m_sub[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      m_sub[u] = LOCAL && m_run[u] < 0.1f * PA_NONE ? 0.f : m_run[u];
     // a step's weights are summed by themselves: added one by one to the sum of
     // 20,000 they would each lose bits (0.7 at 14,000: 3e-4 of the sum)
-    float sum = 0.f;
+    float sum[2] = {0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      pa_f32x8 p;
-      const int h = ks >> 1;
+    for (int ks = 0; ks < 2; ++ks) {
+      pa_frag pb[2];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        p[j] = __builtin_amdgcn_exp2f(
-            __builtin_fmaf(d[h][(ks & 1) * 8 + j], mul, -m_sub));
-        sum += p[j];
+      for (int u = 0; u < 2; ++u) {
+        pa_f32x8 p;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          p[j] = __builtin_amdgcn_exp2f(
+              __builtin_fmaf(d[u][2 * ks + (j >> 2)][j & 3], mul, -m_sub[u]));
+          sum[u] += p[j];
+        }
+        pb[u] = pa_pack8(p);
       }
-      const pa_frag pb = pa_pack8(p);
-      const char* vk = vb + ks * 16 * 2 * D;
-      if (BLOCKS) vk = seen & (1u << ks) ? vk : pa_smem + 4 * TILE;
+      const char* v0 = vb + ks * 32 * 2 * D;
+      const char* v1 = v0 + 16 * 2 * D;
+      if (BLOCKS) {
+        v0 = seen & (1u << 2 * ks) ? v0 : pa_smem + 4 * TILE;
+        v1 = seen & (2u << 2 * ks) ? v1 : pa_smem + 4 * TILE;
+      }
 #pragma unroll
-      for (int b = 0; b < D / 32; ++b) {
-        const char* at = vk + vad[b & 1] + (b >> 1) * 128;
-        acc[b] = pa_mfma32(pa_tr(at, at + 8 * 2 * D), pb, acc[b]);
+      for (int b = 0; b < D / 16; ++b) {
+        const int at = vad[b & 3] + (b >> 2) * 128;
+        const pa_frag va = pa_tr(v0 + at, v1 + at);
+        acc[b][0] = pa_mfma16(va, pb[0], acc[b][0]);
+        acc[b][1] = pa_mfma16(va, pb[1], acc[b][1]);
       }
     }
-    pa_order<D / 4, D / 8, 8, 2>();
-    l_run += sum;
+    pa_order<D / 4, D / 8, 8, 2, 2>();
+    l_run[0] += sum[0];
+    l_run[1] += sum[1];
     }
     if (more)
       store(pa_smem + ((it + 1) & 1) * 2 * TILE, step_tile(it + 1) * PA_KEYS);
   }
 
   if (!live) return;
-  const float l = l_run + __shfl_xor(l_run, 32, 64);
-  float f = l > 0.f ? 1.0f / l : 0.f;
-  const long row = row_base + my_r;
-  if (my_r >= rows) return;
-  const u16* gp = nullptr;
-  if (LOCAL) {
-    f *= A.out_scale;
-    if (A.gate_off >= 0) {
-      gp = A.proj + row * A.ld + A.gate_off + (long)hq * A.gate_n;
-      if (A.gate_n == 1) f *= 1.f / (1.f + expf(-bf2f(gp[0])));
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    float l = l_run[u] + __shfl_xor(l_run[u], 32, 64);
+    l += __shfl_xor(l, 16, 64);
+    float f = l > 0.f ? 1.0f / l : 0.f;
+    const long row = row_base + my_r[u];
+    if (my_r[u] >= rows) continue;
+    const u16* gp = nullptr;
+    if (LOCAL) {
+      f *= A.out_scale;
+      if (A.gate_off >= 0) {
+        gp = A.proj + row * A.ld + A.gate_off + (long)hq * A.gate_n;
+        if (A.gate_n == 1) f *= 1.f / (1.f + expf(-bf2f(gp[0])));
+      }
     }
-  }
-  u16* op = A.out + row * A.ldo + A.out_off + (long)hq * D;
+    u16* op = A.out + row * A.ldo + A.out_off + (long)hq * D;
 #pragma unroll
-  for (int b = 0; b < D / 32; ++b)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int col = b * 32 + 8 * g + 4 * hi;
-      f32x4 o;
-#pragma unroll
-      for (int e2 = 0; e2 < 4; ++e2) o[e2] = acc[b][4 * g + e2] * f;
+    for (int b = 0; b < D / 16; ++b) {
+      const int col = b * 16 + 4 * g;
+      f32x4 o = acc[b][u] * f;
       if (LOCAL && gp && A.gate_n > 1) {
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2)
@@ -479,6 +519,7 @@ paged_prefill_kernel(PagedArgs A) {
       }
       *(u32x2*)(op + col) = pa_pack4(o);
     }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -955,16 +996,15 @@ static inline void pa_launch_prefill(PagedArgs A, int n_seqs, hipStream_t s) {
   A.per = (A.G + A.hpb - 1) / A.hpb;
   A.groups = A.Hk * A.per;
   A.leads = (A.n_tiles + A.rpb - 1) / A.rpb;
-  // Heads of 64 leave room for four workgroups a CU in 128 registers. Many short
+  // Heads of 64 leave room for three workgroups a CU in 168 registers. Many short
   // prompts, a few steps each with nothing to overlap them, are faster that way:
-  // 128 of 100 tokens, 8 heads and kv heads 19 -> 16 us, 160 of 150, 14 and 2
-  // heads, 60 -> 45, 500 of 30, 16 and 8, 38 -> 26; long ones (2000 tokens 38 ->
-  // 40) and few are not. (Layer lists would spill registers: 32 prompts of 200
-  // tokens, 8 heads and kv heads, 19 -> 24 us.)
+  // 128 of 100 tokens, 8 heads and kv heads 18.3 -> 15.9 us, 160 of 150, 14 and 2
+  // heads, 60 -> 49, 500 of 30, 16 and 8, 37 -> 29, 256 of 200 117 -> 99; long ones
+  // and few are not. (Four in 128 registers spill: 17.7 us for the first.)
   if constexpr (D == 64 && !LOCAL) {
     if ((long)A.n_tiles * A.groups >= 512 && A.n_tiles <= 8 * n_seqs) {
-      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 4>(A, s);
-      else pa_start_prefill<D, KV8, LOCAL, true, 4>(A, s);
+      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 3>(A, s);
+      else pa_start_prefill<D, KV8, LOCAL, true, 3>(A, s);
       return;
     }
   }
