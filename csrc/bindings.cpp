@@ -50,6 +50,8 @@ void sutro_sampler_fused(const void*, int, const float*, const float*,
 void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
                         int, hipStream_t);
+void sutro_norm_linear(void*, const void*, const void*, void*, const void*,
+                       float, const void*, int, int, int, hipStream_t);
 void sutro_linear_silu_mul(void*, const void*, const void*, int, int, long,
                            hipStream_t);
 void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
@@ -350,6 +352,30 @@ torch::Tensor linear_skinny(torch::Tensor x, torch::Tensor w,
   return out;
 }
 
+// (y w^T or, `gated`, its silu unit; x + residual), y the RMSNorm of x + residual,
+// one row
+std::vector<torch::Tensor> norm_linear(torch::Tensor x, torch::Tensor residual,
+                                       torch::Tensor norm_w, double eps,
+                                       torch::Tensor w, bool gated) {
+  for (const auto& t : {x, residual, norm_w, w})
+    TORCH_CHECK(t.is_cuda() && t.device() == x.device() &&
+                t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
+                (size_t)t.data_ptr() % 16 == 0,
+                "contiguous bf16 operands on one GPU, 16-byte rows");
+  TORCH_CHECK(x.dim() == 2 && x.size(0) == 1 && x.sizes() == residual.sizes() &&
+              w.dim() == 2, "one row");
+  const long K = x.size(1), rows = w.size(0), N = gated ? rows / 2 : rows;
+  TORCH_CHECK(norm_w.numel() == K && w.size(1) == K && K >= 32 &&
+              K <= 4096 && K % 32 == 0 && N >= 1 && N < (1l << 30) &&
+              rows == (gated ? 2 * N : N), "unsupported sizes");
+  auto out = torch::empty({1, N}, x.options());
+  auto sum = torch::empty_like(residual);
+  sutro_norm_linear(out.data_ptr(), x.data_ptr(), residual.data_ptr(),
+                    sum.data_ptr(), norm_w.data_ptr(), (float)eps, w.data_ptr(),
+                    (int)N, (int)K, gated ? 1 : 0, cur_stream());
+  return {out, sum};
+}
+
 // silu of x [M, K] times the first N rows of w [2 N, K], times x and the others
 torch::Tensor linear_silu_mul(torch::Tensor x, torch::Tensor w) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device(),
@@ -414,6 +440,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma16_probe", &mfma16_probe, "16x16 MFMA fragment-layout probe");
   m.def("moe_combine", &moe_combine, "fused MoE weighted gather-combine");
   m.def("linear_skinny", &linear_skinny, "linear layer over few rows");
+  m.def("norm_linear", &norm_linear,
+        "linear layer of one row behind an addition and RMSNorm");
   m.def("linear_silu_mul", &linear_silu_mul,
         "linear layer with the silu gate behind it, many rows");
   m.def("moe_layout", &moe_layout, "softmax top-k router + expert segments");

@@ -15,6 +15,8 @@
 #include "common.h"
 #include "gemm_stream.h"
 
+#define NG_BLOCKS 1024   // most workgroups of the product with a norm in front
+
 struct SkinnyArgs {
   u16* out;
   const u16* x;
@@ -23,6 +25,11 @@ struct SkinnyArgs {
   long ldx, ldo;
   int M, N, K;
   int act;           // 0 none, 1 silu(gate) up (W has 2 N rows)
+  // a norm in front (one row): x is norm(x + residual) * norm_w
+  const u16* residual;
+  u16* residual_out; // x + residual
+  const u16* norm_w;
+  float eps;
 };
 
 template <int NF, int MB, int WAVES, bool GATED, bool SPREAD>
@@ -174,6 +181,149 @@ __global__ void __launch_bounds__(WAVES * 64) gemv_kernel(SkinnyArgs A) {
   A.out[(long)m * A.ldo + n0 + c] = f2bf(y);
 }
 
+// One row with the addition and RMSNorm in front of it. In a launch of its own the
+// norm takes 2 to 3 us before each product of a step, all of it latency; here every
+// workgroup makes the row again (three reads of it out of the L2), behind the loads
+// of its first weights. So that it is not made too often, workgroups go through
+// several sets of weight rows, the next one's on their way while a set's sums meet:
+// 1024 of them, 512 are 0.1 to 0.8 us slower, one a set 0 to 2. In a graph, two
+// launches and this one: 3072 x 2048 7.6 and 6.0 us, 6144 x 4096 14.2 and 12.2; with
+// the unit behind it 2 x 8192 x 2048 17.2 and 14.9, 2 x 12288 x 4096 40.9 and 34.9.
+// All of a row of weights is loaded at once: K up to WAVES * 1024.
+template <int WAVES, bool GATED>
+__global__ void __launch_bounds__(WAVES * 64) norm_gemv_kernel(SkinnyArgs A) {
+  constexpr int R = 4, COLS = GATED ? R / 2 : R, T = WAVES * 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int groups = (A.N + COLS - 1) / COLS;
+  __shared__ __attribute__((aligned(16))) u16 xs[WAVES * 1024];
+  __shared__ float red[WAVES][R];
+  u16x8 w[2][R];
+  auto load = [&](int g) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int n = g * COLS + (GATED ? i & 1 : i);
+        const long row = min(n, A.N - 1) + (GATED ? (i >> 1) * (long)A.N : 0);
+        w[b][i] =
+            *(const u16x8*)(A.w + row * A.K + min((b * T + tid) * 8, A.K - 8));
+      }
+  };
+  load(blockIdx.x);
+
+  float xf[2][8], ssq = 0.f;
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int k = (b * T + tid) * 8;
+    if (k >= A.K) continue;
+    const u16x8 xv = *(const u16x8*)(A.x + k);
+    const u16x8 rv = *(const u16x8*)(A.residual + k);
+    u16x8 sum;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      xf[b][e] = bf2f(xv[e]) + bf2f(rv[e]);
+      ssq += xf[b][e] * xf[b][e];
+      sum[e] = f2bf(xf[b][e]);
+    }
+    if (blockIdx.x == 0) *(u16x8*)(A.residual_out + k) = sum;
+  }
+  ssq = wave_sum_f32(ssq);
+  if (lane == 0) red[wave][0] = ssq;
+  __syncthreads();
+  ssq = red[0][0];
+#pragma unroll
+  for (int i = 1; i < WAVES; ++i) ssq += red[i][0];
+  const float inv = rsqrtf(ssq / (float)A.K + A.eps);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int k = (b * T + tid) * 8;
+    if (k >= A.K) continue;
+    const u16x8 nv = *(const u16x8*)(A.norm_w + k);
+    u16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = f2bf(xf[b][e] * inv * bf2f(nv[e]));
+    *(u16x8*)(xs + k) = o;    // read by the same thread only
+  }
+
+  for (int g = blockIdx.x; g < groups; g += gridDim.x) {
+    float acc[R] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int k = (b * T + tid) * 8;
+      if (k >= A.K) continue;
+      const u16x8 xv = *(const u16x8*)(xs + k);
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          acc[i] = fmaf(bf2f(w[b][i][e]), bf2f(xv[e]), acc[i]);
+    }
+    if (g + (int)gridDim.x < groups) load(g + gridDim.x);
+    // the lanes of 16 neighbours end with the sum of one value
+    int v0 = 0;
+#pragma unroll
+    for (int half = R / 2, bit = 32; half >= 1; half /= 2, bit /= 2) {
+      const bool up = lane & bit;
+#pragma unroll
+      for (int v = 0; v < R / 2; ++v)
+        if (v < half) {
+          const float give = up ? acc[v] : acc[v + half];
+          const float keep = up ? acc[v + half] : acc[v];
+          acc[v] = keep + __shfl_xor(give, bit, 64);
+        }
+      v0 += up ? half : 0;
+    }
+#pragma unroll
+    for (int bit = 8; bit >= 1; bit /= 2)
+      acc[0] += __shfl_xor(acc[0], bit, 64);
+    __syncthreads();          // the sums before these have been read
+    if ((lane & 15) == 0) red[wave][v0] = acc[0];
+    __syncthreads();
+    const int n = g * COLS + tid;
+    if (tid < COLS && n < A.N) {
+      auto total = [&](int i) {
+        float y = red[0][i];
+#pragma unroll
+        for (int z = 1; z < WAVES; ++z) y += red[z][i];
+        return y;
+      };
+      float y = total(tid);
+      if (GATED) y = y / (1.f + __expf(-y)) * total(tid + 2);
+      A.out[n] = f2bf(y);
+    }
+  }
+}
+
+// one row, K % 32 == 0, K <= 4096; residual and residual_out differ
+extern "C" void sutro_norm_linear(void* out, const void* x,
+                                  const void* residual, void* residual_out,
+                                  const void* norm_w, float eps, const void* w,
+                                  int N, int K, int act, hipStream_t s) {
+  SkinnyArgs A = {};
+  A.out = (u16*)out;
+  A.x = (const u16*)x;
+  A.w = (const u16*)w;
+  A.M = 1;
+  A.N = N;
+  A.K = K;
+  A.residual = (const u16*)residual;
+  A.residual_out = (u16*)residual_out;
+  A.norm_w = (const u16*)norm_w;
+  A.eps = eps;
+  const int groups = (N + (act ? 1 : 3)) / (act ? 2 : 4);
+  const dim3 grid(groups < NG_BLOCKS ? groups : NG_BLOCKS);
+#define LAUNCH_NG(WW, GG)                                                    \
+  hipLaunchKernelGGL((norm_gemv_kernel<WW, GG>), grid, dim3(WW * 64), 0, s, A)
+  if (K <= 2048) {
+    if (act) LAUNCH_NG(2, true);
+    else LAUNCH_NG(2, false);
+  } else {
+    if (act) LAUNCH_NG(4, true);
+    else LAUNCH_NG(4, false);
+  }
+#undef LAUNCH_NG
+}
+
 template <int MR, bool GATED>
 static void gemv_launch(const SkinnyArgs& A, hipStream_t s) {
   const unsigned blocks = A.N / (GATED ? 2 : 4);
@@ -217,7 +367,7 @@ extern "C" void sutro_linear_skinny(void* out, long ldo, const void* x,
                                     int M, int N, int K, int act,
                                     hipStream_t s) {
   SkinnyArgs A = {(u16*)out, (const u16*)x, (const u16*)w, (const u16*)bias,
-                  ldx, ldo, M, N, K, act};
+                  ldx, ldo, M, N, K, act, nullptr, nullptr, nullptr, 0.f};
   const int mb = (M + 15) / 16;
 #define SK_GEMV(MR)                                                          \
   do {                                                                       \

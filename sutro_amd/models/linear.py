@@ -22,3 +22,10 @@ def bare(layer: nn.Module) -> bool:
             and not layer._forward_hooks and not layer._forward_pre_hooks
             and not module._has_any_global_hook()
             and "forward" not in layer.__dict__)
+
+
+def unhooked(block: nn.Module) -> bool:
+    """Whether nothing sees a block's input but the block."""
+    return (not block._forward_hooks and not block._forward_pre_hooks
+            and not module._has_any_global_hook()
+            and "forward" not in block.__dict__)

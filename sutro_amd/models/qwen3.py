@@ -22,7 +22,7 @@ from ..engine.batch import ForwardBatch
 from ..engine.kv_cache import PagedKVCache
 from ..ops import torch_ref
 from ..parallel.tp import TPContext
-from .linear import Linear, bare
+from .linear import Linear, bare, unhooked
 from .registry import ModelSpec
 
 
@@ -89,10 +89,13 @@ class Qwen3Attention(nn.Module):
             self.q_norm = RMSNorm(self.head_dim, spec.rms_eps, dtype)
             self.k_norm = RMSNorm(self.head_dim, spec.rms_eps, dtype)
 
-    def forward(self, x: torch.Tensor, fb: ForwardBatch, kv: PagedKVCache,
-                cos_sin: torch.Tensor) -> torch.Tensor:
-        T = x.shape[0]
-        qkv = self.qkv_proj(x)
+    def forward(self, x: Optional[torch.Tensor], fb: ForwardBatch,
+                kv: PagedKVCache, cos_sin: torch.Tensor,
+                qkv: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """`qkv`: the projection of x, where the caller has made it."""
+        if qkv is None:
+            qkv = self.qkv_proj(x)
+        T = qkv.shape[0]
         q = ops.fused_qkv_prep(
             qkv, self.num_heads, self.num_kv_heads, self.head_dim,
             fb.positions, fb.slot_mapping,
@@ -123,8 +126,13 @@ class Qwen3MLP(nn.Module):
         self.down_proj = Linear(inter_l, hidden, bias=False, dtype=dtype)
         _mark_shard(self.down_proj.weight, (hidden, intermediate), 1, tp)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if bare(self.gate_up_proj):
+    def forward(self, x: Optional[torch.Tensor],
+                act: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """`act`: what goes into the down projection, where the caller has made
+        it."""
+        if act is not None:
+            pass
+        elif bare(self.gate_up_proj):
             act = ops.linear_silu_mul(x, self.gate_up_proj.weight)
         else:
             act = ops.silu_mul(self.gate_up_proj(x))
@@ -498,19 +506,26 @@ class Qwen3Block(nn.Module):
             self.mlp = Qwen3MLP(spec.hidden_size, spec.intermediate_size, dtype, tp)
 
     def forward(self, x, residual, fb: ForwardBatch, kv, cos_sin):
+        attn, mlp = self.self_attn, self.mlp
+        norm = self.input_layernorm
         if residual is None:
             residual = x
-            x = self.input_layernorm(x)
+            x = attn(norm(x), fb, kv, cos_sin)
+        elif bare(attn.qkv_proj) and unhooked(attn):
+            qkv, residual = ops.norm_linear(x, residual, norm.weight, norm.eps,
+                                            attn.qkv_proj.weight)
+            x = attn(None, fb, kv, cos_sin, qkv)
         else:
-            x, residual = ops.fused_add_rmsnorm(x, residual,
-                                                self.input_layernorm.weight,
-                                                self.input_layernorm.eps)
-        x = self.self_attn(x, fb, kv, cos_sin)
-        x, residual = ops.fused_add_rmsnorm(x, residual,
-                                            self.post_attention_layernorm.weight,
-                                            self.post_attention_layernorm.eps)
-        x = self.mlp(x)
-        return x, residual
+            x, residual = ops.fused_add_rmsnorm(x, residual, norm.weight,
+                                                norm.eps)
+            x = attn(x, fb, kv, cos_sin)
+        norm = self.post_attention_layernorm
+        if type(mlp) is Qwen3MLP and bare(mlp.gate_up_proj) and unhooked(mlp):
+            act, residual = ops.norm_linear(x, residual, norm.weight, norm.eps,
+                                            mlp.gate_up_proj.weight, gated=True)
+            return mlp(None, act), residual
+        x, residual = ops.fused_add_rmsnorm(x, residual, norm.weight, norm.eps)
+        return mlp(x), residual
 
 
 class Qwen3Model(nn.Module):

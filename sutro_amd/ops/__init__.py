@@ -315,6 +315,33 @@ def linear_silu_mul(x, w):
     return silu_mul(F.linear(x, w))
 
 
+def _one_row(x, residual, norm_w, w, gated: bool) -> bool:
+    """Whether csrc/gemm_skinny.hip makes the norm of one row inside the product
+    behind it."""
+    return (_few_rows(x, w, gated) and x.shape[0] == 1 and x.shape[1] <= 4096
+            and x.is_contiguous()
+            and type(residual) is torch.Tensor
+            and type(norm_w) in (torch.Tensor, torch.nn.Parameter)
+            and residual.shape == x.shape and norm_w.shape == x.shape[1:]
+            and residual.dtype == torch.bfloat16
+            and norm_w.dtype == torch.bfloat16
+            and residual.device == x.device and norm_w.device == x.device
+            and residual.is_contiguous() and norm_w.is_contiguous()
+            and residual.data_ptr() % 16 == 0
+            and norm_w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (residual.requires_grad or norm_w.requires_grad)))
+
+
+def norm_linear(x, residual, norm_w, eps: float, w, gated: bool = False):
+    """(y w^T, r) for r = x + residual and y = rmsnorm(r), `gated`: (silu_mul(y
+    w^T), r). x and residual may be overwritten."""
+    if _one_row(x, residual, norm_w, w, gated):
+        return _require_hip().norm_linear(x, residual, norm_w, eps, w, gated)
+    x, residual = fused_add_rmsnorm(x, residual, norm_w, eps)
+    return (linear_silu_mul(x, w) if gated else linear(x, w)), residual
+
+
 def expert_tile(n_rows: int, experts: int, inner: int, width: int,
                 gated: bool = True, local: Optional[int] = None) -> int:
     """Rows that the segments of both expert GEMMs of a layer are padded to,
