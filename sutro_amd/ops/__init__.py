@@ -280,14 +280,18 @@ def linear(x, w, bias=None):
 def _many_rows(x, w) -> bool:
     """Whether csrc/grouped_gemm.hip makes silu_mul(x w^T) in one launch. Its
     tiles are 256 rows by 128 columns of the result, one a CU at a time: below
-    256 of them the library's smaller tiles are ahead (us of both, tiles):
+    256 of them the library's smaller tiles are ahead, and where the last round
+    leaves a quarter of all places empty (us of both, tiles):
       2 x 3072 x 1024    1024 rows  25.1 /  26.7 ( 96)   2048   36.2 / 29.2 (192)
+                         2600 rows  51.6 /  54.3 (264)   3328   58.6 / 53.6 (312)
       2 x 6144 x 2048     512 rows  33.4 /  42.6 ( 96)   1024   53.6 / 48.9 (192)
+                         2816 rows   138 /   141 (528)   3328    156 /  145 (624)
       2 x 8192 x 2048     512 rows  39.7 /  45.5 (128)   1024   66.5 / 54.2 (256)
-      2 x 9728 x 2560     512 rows  58.7 /  96.8 (152)   1024    107 /  108 (304)
-      2 x 12288 x 4096   1024 rows   173 /   170 (384)   1500    257 /  258 (576)
-    and from there on it is 2 to 45 % faster, or as fast (the figures at many
-    rows stand beside the kernel)."""
+                         1280 rows  86.9 /  89.4 (320)   1536   96.7 / 93.1 (384)
+      2 x 12288 x 4096    768 rows   150 /   161 (288)   1024    173 /  170 (384)
+    Otherwise it is 2 to 45 % faster, or as fast (the figures at many rows stand
+    beside the kernel). Short k, which the library does worst at, still gains
+    with two fifths empty."""
     if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False
@@ -295,7 +299,10 @@ def _many_rows(x, w) -> bool:
         return False
     M, K = x.shape
     rows = w.shape[0]
-    return (rows % 256 == 0 and -(-M // 256) * (rows // 256) >= 256
+    tiles = -(-M // 256) * (rows // 256)
+    places = -(-tiles // 256) * 256
+    return (rows % 256 == 0 and tiles >= 256
+            and tiles >= places * (0.6 if K <= 1024 else 0.75)
             and K % 64 == 0 and 0 < K < 1 << 21 and M * K < 1 << 30
             and rows < 1 << 24 and w.shape[1] == K and _unwatched()
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16

@@ -48,6 +48,9 @@ def test_route():
     assert err[0] <= err[1]
     assert not ops._many_rows(x[:, :192], w[:, :192])     # strided
     assert not ops._many_rows(x[:3000], w)                # too few tiles
+    more = x.repeat(3, 1)
+    assert ops._many_rows(more[:5632], w)                 # 352 of 512 places
+    assert not ops._many_rows(more[:4608], w)             # 288
     assert not ops._many_rows(x.float(), w.float())
     wide = torch.empty(2, 4096, 256, device=DEV, dtype=torch.bfloat16)
     assert not ops._many_rows(wide, w)
