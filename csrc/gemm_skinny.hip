@@ -15,7 +15,7 @@
 #include "common.h"
 #include "gemm_stream.h"
 
-#define NG_BLOCKS 1024   // most workgroups of the product with a norm in front
+#define SETS_WAVES 4096   // most waves of a product that goes through sets of rows
 
 struct SkinnyArgs {
   u16* out;
@@ -181,21 +181,26 @@ __global__ void __launch_bounds__(WAVES * 64) gemv_kernel(SkinnyArgs A) {
   A.out[(long)m * A.ldo + n0 + c] = f2bf(y);
 }
 
-// One row with the addition and RMSNorm in front of it. In a launch of its own the
+// One row again, K up to WAVES * 1024: all of a weight row is loaded at once, and a
+// workgroup goes through several sets of weight rows, the next one's on their way
+// while a set's sums meet. Against a workgroup a set (us in a graph): 8192 x 2048
+// 9.4 -> 8.4, 32768 x 2048 26.0 -> 23.9, 32768 x 4096 48.5 -> 46.0; with the unit behind
+// it 2 x 8192 x 2048 14.4 -> 13.6, 2 x 12288 x 4096 37.1 -> 35.3; below 2048 sets there
+// is nothing to go through, and 151936 rows lose 1 to 2 %. Twice as few or as many
+// workgroups are 5 to 10 % slower, one way or the other.
+//
+// NORM: with the addition and RMSNorm in front of it. In a launch of its own the
 // norm takes 2 to 3 us before each product of a step, all of it latency; here every
 // workgroup makes the row again (three reads of it out of the L2), behind the loads
-// of its first weights. So that it is not made too often, workgroups go through
-// several sets of weight rows, the next one's on their way while a set's sums meet:
-// 1024 of them, 512 are 0.1 to 0.8 us slower, one a set 0 to 2. In a graph, two
-// launches and this one: 3072 x 2048 7.6 and 6.0 us, 6144 x 4096 14.2 and 12.2; with
-// the unit behind it 2 x 8192 x 2048 17.2 and 14.9, 2 x 12288 x 4096 40.9 and 34.9.
-// All of a row of weights is loaded at once: K up to WAVES * 1024.
-template <int WAVES, bool GATED>
-__global__ void __launch_bounds__(WAVES * 64) norm_gemv_kernel(SkinnyArgs A) {
+// of its first weights. Two launches and this one: 3072 x 2048 7.6 and 6.0 us, 6144 x
+// 4096 14.2 and 12.2; with the unit 2 x 8192 x 2048 17.2 and 14.5, 2 x 12288 x 4096 40.9
+// and 34.9.
+template <int WAVES, bool GATED, bool NORM>
+__global__ void __launch_bounds__(WAVES * 64) sets_gemv_kernel(SkinnyArgs A) {
   constexpr int R = 4, COLS = GATED ? R / 2 : R, T = WAVES * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int groups = (A.N + COLS - 1) / COLS;
-  __shared__ __attribute__((aligned(16))) u16 xs[WAVES * 1024];
+  __shared__ __attribute__((aligned(16))) u16 xs[NORM ? WAVES * 1024 : 8];
   __shared__ float red[WAVES][R];
   u16x8 w[2][R];
   auto load = [&](int g) {
@@ -211,38 +216,45 @@ __global__ void __launch_bounds__(WAVES * 64) norm_gemv_kernel(SkinnyArgs A) {
   };
   load(blockIdx.x);
 
-  float xf[2][8], ssq = 0.f;
+  if (NORM) {
+    // the squares are added in the order of the norm's own kernel (four waves a
+    // row, a piece or two a lane): the two agree to the bit
+    float xf[2][8], sq[2] = {0.f, 0.f};
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int k = (b * T + tid) * 8;
-    if (k >= A.K) continue;
-    const u16x8 xv = *(const u16x8*)(A.x + k);
-    const u16x8 rv = *(const u16x8*)(A.residual + k);
-    u16x8 sum;
+    for (int b = 0; b < 2; ++b) {
+      const int k = (b * T + tid) * 8;
+      if (k >= A.K) continue;
+      const u16x8 xv = *(const u16x8*)(A.x + k);
+      const u16x8 rv = *(const u16x8*)(A.residual + k);
+      u16x8 sum;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      xf[b][e] = bf2f(xv[e]) + bf2f(rv[e]);
-      ssq += xf[b][e] * xf[b][e];
-      sum[e] = f2bf(xf[b][e]);
+      for (int e = 0; e < 8; ++e) {
+        xf[b][e] = bf2f(xv[e]) + bf2f(rv[e]);
+        sq[WAVES == 2 ? b : 0] += xf[b][e] * xf[b][e];
+        sum[e] = f2bf(xf[b][e]);
+      }
+      if (blockIdx.x == 0) *(u16x8*)(A.residual_out + k) = sum;
     }
-    if (blockIdx.x == 0) *(u16x8*)(A.residual_out + k) = sum;
-  }
-  ssq = wave_sum_f32(ssq);
-  if (lane == 0) red[wave][0] = ssq;
-  __syncthreads();
-  ssq = red[0][0];
 #pragma unroll
-  for (int i = 1; i < WAVES; ++i) ssq += red[i][0];
-  const float inv = rsqrtf(ssq / (float)A.K + A.eps);
+    for (int b = 0; b < (WAVES == 2 ? 2 : 1); ++b) {
+      sq[b] = wave_sum_f32(sq[b]);
+      if (lane == 0) red[wave][b] = sq[b];
+    }
+    __syncthreads();
+    float ssq = red[0][0];
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int k = (b * T + tid) * 8;
-    if (k >= A.K) continue;
-    const u16x8 nv = *(const u16x8*)(A.norm_w + k);
-    u16x8 o;
+    for (int i = 1; i < 4; ++i) ssq += red[i % WAVES][i / WAVES];
+    const float inv = rsqrtf(ssq / (float)A.K + A.eps);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = f2bf(xf[b][e] * inv * bf2f(nv[e]));
-    *(u16x8*)(xs + k) = o;    // read by the same thread only
+    for (int b = 0; b < 2; ++b) {
+      const int k = (b * T + tid) * 8;
+      if (k >= A.K) continue;
+      const u16x8 nv = *(const u16x8*)(A.norm_w + k);
+      u16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = f2bf(xf[b][e] * inv * bf2f(nv[e]));
+      *(u16x8*)(xs + k) = o;    // read by the same thread only
+    }
   }
 
   for (int g = blockIdx.x; g < groups; g += gridDim.x) {
@@ -251,7 +263,7 @@ __global__ void __launch_bounds__(WAVES * 64) norm_gemv_kernel(SkinnyArgs A) {
     for (int b = 0; b < 2; ++b) {
       const int k = (b * T + tid) * 8;
       if (k >= A.K) continue;
-      const u16x8 xv = *(const u16x8*)(xs + k);
+      const u16x8 xv = *(const u16x8*)((NORM ? xs : A.x) + k);
 #pragma unroll
       for (int i = 0; i < R; ++i)
 #pragma unroll
@@ -311,9 +323,10 @@ extern "C" void sutro_norm_linear(void* out, const void* x,
   A.norm_w = (const u16*)norm_w;
   A.eps = eps;
   const int groups = (N + (act ? 1 : 3)) / (act ? 2 : 4);
-  const dim3 grid(groups < NG_BLOCKS ? groups : NG_BLOCKS);
+  const int most = SETS_WAVES / (K <= 2048 ? 2 : 4);
+  const dim3 grid(groups < most ? groups : most);
 #define LAUNCH_NG(WW, GG)                                                    \
-  hipLaunchKernelGGL((norm_gemv_kernel<WW, GG>), grid, dim3(WW * 64), 0, s, A)
+  hipLaunchKernelGGL((sets_gemv_kernel<WW, GG, true>), grid, dim3(WW * 64), 0, s, A)
   if (K <= 2048) {
     if (act) LAUNCH_NG(2, true);
     else LAUNCH_NG(2, false);
@@ -327,6 +340,18 @@ extern "C" void sutro_norm_linear(void* out, const void* x,
 template <int MR, bool GATED>
 static void gemv_launch(const SkinnyArgs& A, hipStream_t s) {
   const unsigned blocks = A.N / (GATED ? 2 : 4);
+  // From 2048 sets of rows on (one row, no bias), up to the largest output layers,
+  // which have the same 4096 waves busy either way: see sets_gemv_kernel.
+  if (MR == 1 && !A.bias && A.K > 1024 && A.K <= 4096 && blocks >= 2048 &&
+      blocks < 32768) {
+    if (A.K <= 2048)
+      hipLaunchKernelGGL((sets_gemv_kernel<2, GATED, false>),
+                         dim3(SETS_WAVES / 2), dim3(128), 0, s, A);
+    else
+      hipLaunchKernelGGL((sets_gemv_kernel<4, GATED, false>),
+                         dim3(SETS_WAVES / 4), dim3(256), 0, s, A);
+    return;
+  }
 #define LAUNCH_GV(WW)                                                        \
   hipLaunchKernelGGL((gemv_kernel<MR, WW, GATED>), dim3(blocks),             \
                      dim3(WW * 64), 0, s, A)

@@ -57,3 +57,31 @@ def test_route():
     assert not ops._one_row(x, res, p, w, False)
     with torch.no_grad():
         assert ops._one_row(x, res, p, w, False)
+
+
+@pytest.mark.parametrize("K", [512, 1024, 2048, 2560, 4096])
+def test_norm_to_the_bit(K):
+    """Through the unit matrix: the row the norm's own kernel makes."""
+    eye = torch.eye(K, device=DEV).bfloat16()
+    for seed in range(20):
+        torch.manual_seed(seed)
+        x, res = (torch.randn(1, K, device=DEV).bfloat16() for _ in range(2))
+        nw = (1 + 0.1 * torch.randn(K, device=DEV)).bfloat16()
+        got, total = ops._require_hip().norm_linear(x, res, nw, 1e-6, eye,
+                                                    False)
+        want, r2 = ops.fused_add_rmsnorm(x.clone(), res.clone(), nw, 1e-6)
+        assert torch.equal(got, want) and torch.equal(total, r2)
+
+
+@pytest.mark.parametrize("N,K,gated", [
+    (8188, 2048, False), (8200, 2080, False), (20000, 4096, False),
+    (4100, 2048, True), (12288, 3104, True)])
+def test_one_row_through_sets(N, K, gated):
+    """2047 and more sets of weight rows, without a norm."""
+    x, _, _, w = _operands(N, K, gated)
+    got = ops._require_hip().linear_skinny(x, w, None, gated).double()
+    y = x.double() @ w.double().T
+    if gated:
+        y = F.silu(y[:, :N]) * y[:, N:]
+    # fp32 sums of K products of size 1, one rounding to bf16 at the end
+    torch.testing.assert_close(got, y, rtol=2 ** -8, atol=2 ** -12)
