@@ -313,8 +313,8 @@ class Qwen3MoE(nn.Module):
         The big per-forward transients (act / out_sorted / gather+combine
         buffers) must not be allocated inside a captured decode step: every
         capture would own its own copy per layer per batch bucket — measured
-        ~277 GB of graph-pool memory on qwen-3-30b-a3b before this fix
-        (gpurun call 9). The workspace is module-level (one set per
+        ~277 GB of graph-pool memory on qwen-3-30b-a3b before this fix.
+        The workspace is module-level (one set per
         (device, dtype, h, m_l) — all 48 layers share it: execution is
         sequential) and grow-only."""
         dev = next(self.parameters()).device
