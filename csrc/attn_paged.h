@@ -292,6 +292,8 @@ paged_prefill_kernel(PagedArgs A) {
   const int st_row = lane / CPR;
   const u32 koff = (st_row * D + pa_kchunk(st_row, lane % CPR) * 8) * ES;
   const u32 voff = (st_row * D + pa_vchunk(st_row, lane % CPR) * 8) * ES;
+  // LATE: four workgroups a CU, no registers to hold them while a step is computed
+  constexpr bool LATE = WAVES_PER_SIMD == 4;
   typename PaRaw<KV8>::type st[PER / 2];
   int pa = 0, pb = 0;    // pages of the next step to load
   auto pages = [&](int kt) {
@@ -360,8 +362,8 @@ paged_prefill_kernel(PagedArgs A) {
     __syncthreads();
     const int kv0 = step_tile(it) * PA_KEYS;
     const bool more = it + 1 < steps;
-    if (more) load();
-    if (it + 2 < steps) pages(step_tile(it + 2));
+    if (more && !LATE) load();
+    if (!LATE && it + 2 < steps) pages(step_tile(it + 2));
     // With several row blocks in the workgroup a step may be for the rows of
     // others: which of its four times 16 keys does a row of this wave see?
     u32 seen = 15;
@@ -390,7 +392,7 @@ paged_prefill_kernel(PagedArgs A) {
         d[0][t] = pa_mfma16(ka, qb[0][kk], d[0][t]);
         d[1][t] = pa_mfma16(ka, qb[1][kk], d[1][t]);
       }
-    pa_order<D / 8, D / 8, 6, 1, 2>();
+    pa_order<D / 8, D / 8, LATE ? 2 : 6, 1, 2>();
     // without a distance bias scores stay unscaled until the exponential
     const bool whole = kv0 + PA_KEYS <= p0 + rb * 32 + 1 &&
                        (!LOCAL || kv0 >= lo_last);
@@ -483,12 +485,15 @@ paged_prefill_kernel(PagedArgs A) {
         acc[b][1] = pa_mfma16(va, pb[1], acc[b][1]);
       }
     }
-    pa_order<D / 4, D / 8, 8, 2, 2>();
+    pa_order<D / 4, D / 8, LATE ? 4 : 8, 2, 2>();
     l_run[0] += sum[0];
     l_run[1] += sum[1];
     }
-    if (more)
+    if (more) {
+      if (LATE) load();
+      if (LATE && it + 2 < steps) pages(step_tile(it + 2));
       store(pa_smem + ((it + 1) & 1) * 2 * TILE, step_tile(it + 1) * PA_KEYS);
+    }
   }
 
   if (!live) return;
@@ -996,15 +1001,17 @@ static inline void pa_launch_prefill(PagedArgs A, int n_seqs, hipStream_t s) {
   A.per = (A.G + A.hpb - 1) / A.hpb;
   A.groups = A.Hk * A.per;
   A.leads = (A.n_tiles + A.rpb - 1) / A.rpb;
-  // Heads of 64 leave room for three workgroups a CU in 168 registers. Many short
-  // prompts, a few steps each with nothing to overlap them, are faster that way:
-  // 128 of 100 tokens, 8 heads and kv heads 18.3 -> 15.9 us, 160 of 150, 14 and 2
-  // heads, 60 -> 49, 500 of 30, 16 and 8, 37 -> 29, 256 of 200 117 -> 99; long ones
-  // and few are not. (Four in 128 registers spill: 17.7 us for the first.)
+  // Heads of 64 leave room for four workgroups a CU in 128 registers, if a step's
+  // keys and values are loaded behind the one before it (LATE). Many short prompts, a
+  // few steps each with nothing to overlap them, are faster that way: 128 of 100
+  // tokens, 8 heads and kv heads 18.3 -> 15.1 us, 160 of 150, 14 and 2 heads, 60 -> 44,
+  // 500 of 30, 16 and 8, 37 -> 25, 256 of 200 117 -> 94 (three workgroups in 168
+  // registers 16.0, 47.6, 28.3 and 97.7); long ones and few are not. (Layer lists would
+  // spill registers: 32 prompts of 200 tokens, 8 heads and kv heads, 19 -> 24 us.)
   if constexpr (D == 64 && !LOCAL) {
     if ((long)A.n_tiles * A.groups >= 512 && A.n_tiles <= 8 * n_seqs) {
-      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 3>(A, s);
-      else pa_start_prefill<D, KV8, LOCAL, true, 3>(A, s);
+      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 4>(A, s);
+      else pa_start_prefill<D, KV8, LOCAL, true, 4>(A, s);
       return;
     }
   }
