@@ -511,7 +511,8 @@ class Qwen3Block(nn.Module):
         if residual is None:
             residual = x
             x = attn(norm(x), fb, kv, cos_sin)
-        elif bare(attn.qkv_proj) and unhooked(attn):
+        elif (type(attn) is Qwen3Attention and bare(attn.qkv_proj)
+              and unhooked(attn)):
             qkv, residual = ops.norm_linear(x, residual, norm.weight, norm.eps,
                                             attn.qkv_proj.weight)
             x = attn(None, fb, kv, cos_sin, qkv)
