@@ -622,12 +622,19 @@ __device__ __forceinline__ void gw_body(
 
   const int KT = (int)(K >> 6);
   const int lead = min(KT, 2);
-  // XCDs start an eighth of k apart where rows are multiples of 4 KB long (see the
-  // kernel above; within an XCD workgroups share operands and stay in step): gate
-  // and up / down of 32 experts of 2048 x 2048 at 375 rows 257 / 120 -> 229 / 115 us,
-  // at 4096 rows 1736 / 891 -> 1718 / 858; rows of 2 KB 244 -> 257, so not there
-  int kc = K % 2048 == 0 ? (int)(blockIdx.x & 7) * KT / 8 * 64 : 0;
-  auto advance = [&]() {        // after KT steps it is where it began
+  // Experts start at different eighths of k where rows are multiples of 4 KB long
+  // (see the kernel above): gate and up / down of 32 experts of 2048 x 2048 at 187
+  // rows 151 / 81 -> 129 / 67 us, at 375 rows 251 / 120 -> 224 / 117, at 4096 rows
+  // 1634 / 844 and 1637 / 850. The tile's rows have no part in it: the dispatch puts
+  // a token where its counter happens to stand, and the token's sums have to come
+  // out the same in every place. By column blocks as well, which takes workgroups of
+  // an XCD out of step: 144 / 85, 233 / 125, 1704 / 842. One matrix (DENSE) has one
+  // start, 0.
+  auto first = [&](const GwTile& g) {
+    return !DENSE && K % 2048 == 0 ? (g.e * 5 & 7) * KT / 8 * 64 : 0;
+  };
+  int kc = first(cur);
+  auto advance = [&]() {
     kc += 64;
     if (kc == (int)K) kc = 0;
   };
@@ -667,6 +674,7 @@ __device__ __forceinline__ void gw_body(
       store_tile(cur);
       if (!next(cur)) return;
       point(cur, src);
+      kc = first(cur);
       __syncthreads();        // the reads of this tile's operands are done
     }
   }
@@ -679,7 +687,10 @@ __device__ __forceinline__ void gw_body(
     const int last = more ? KT : KT - 2;
     keep();
     for (int s = 0; s < last; ++s) {
-      if (s == KT - 2) src = after;   // the copies are the next tile's now
+      if (s == KT - 2) {      // the copies are the next tile's now
+        src = after;
+        kc = first(nxt);
+      }
       step(kc, yes, yes);
       keep();
       advance();

@@ -65,3 +65,31 @@ def test_many_experts(experts):
 @pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
 def test_operands_off_boundaries(act):
     _run([600, 5, 300], 320, 512, act, shift=8 + 2)
+
+
+@pytest.mark.parametrize("K", [1024, 2048, 4096])
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
+def test_place_of_a_row(K, act):
+    """The dispatch puts tokens where its counters stand: a token's result is the
+    same to the bit in every tile of its expert, on every XCD."""
+    g = torch.Generator(device=DEV).manual_seed(K)
+    gated = act == hops.ACT_SILU_GATE
+    counts, ff, T = [9000, 300, 5000], 512, 7
+    tiles = [(c + 255) // 256 for c in counts]
+    off = torch.tensor([0] + tiles, device=DEV).cumsum(0).int()
+    cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
+    rows = sum(tiles) * 256
+    x = torch.randn(T, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(3, 2 * ff if gated else ff, K, generator=g, device=DEV)
+         * K ** -0.5).bfloat16()
+    which = torch.arange(rows, device=DEV) * 5 % T
+    out = torch.empty(rows, ff, device=DEV, dtype=torch.bfloat16)
+    if gated:
+        hops.expert_gemm(out, x, w, which.int(), off, cnt, act, 256, 0.0, None)
+    else:
+        hops.expert_gemm(out, x[which], w, None, off, cnt, act, 256, 0.0, None)
+    for e, c in enumerate(counts):
+        a = int(off[e]) * 256
+        for t in range(T):
+            same = out[a:a + c][which[a:a + c] == t]
+            assert torch.equal(same, same[:1].expand_as(same)), (e, t)

@@ -60,3 +60,14 @@ def test_route():
         assert ops._many_rows(x, p)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert not ops._many_rows(x, w)
+
+
+@pytest.mark.parametrize("K", [1024, 2048, 4096])
+def test_place_of_a_row(K):
+    """Equal rows of a batch have equal results, in whichever tile they are."""
+    x, w = _operands(5, 1024, K)
+    which = torch.arange(9000, device=DEV) * 3 % 5
+    got = ops._require_hip().linear_silu_mul(x[which], w)
+    for t in range(5):
+        same = got[which == t]
+        assert torch.equal(same, same[:1].expand_as(same)), t
