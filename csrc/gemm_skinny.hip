@@ -5,13 +5,18 @@
 // Bound by the weights, which are read once, and for the small matrices of a
 // step by the time to get enough loads in flight. A workgroup owns 16 or 32
 // rows of W (gated: 16 and 16) and its waves split k, each with a batch of
-// fragments ahead of its products (gemm_stream.h); their sums meet in LDS. Two
-// waves with long runs are the faster ones (a wave that ends after a batch or two
-// has nothing in flight while its workgroup adds up): 16 rows, 6144 x 4096 on 8
-// waves of 16 rows of W 22.1 -> 14.9 us on 2 of 32, 18432 x 2048 28.0 -> 22.9,
-// 5120 x 25600 111 -> 72. Only where a CU has no more than one workgroup do more
-// waves pay: 2048 x 2048 6.5 on 2, 6.3 on 16 (a batch each); 4096 x 4096 at 8 rows
-// 10.3 on 2, 9.4 on 4.
+// fragments ahead of its products (gemm_stream.h); their sums meet in LDS.
+//
+// Waves, by the k-steps of a row (a batch is four). Where 4, 8 or 16 waves have
+// exactly a batch each, all loads of a workgroup are in flight at once: 2048 x 512
+// at 16 rows 3.4 / 3.2 / 3.7 us on 2 / 4 / 8 waves, 4104 x 1024 6.0 / 6.8 / 5.4. Else
+// few waves with long runs are ahead, as one that ends after a batch or two has
+// nothing in flight while its workgroup adds up: 16 rows, 6144 x 4096 on 8 waves of
+// 16 rows of W 22.1 -> 14.9 us on 2 of 32, 18432 x 2048 28.0 -> 22.9, 5120 x 25600
+// 111 -> 72; a router of 32 x 4096 12.0 on 16 waves, 9.2 on 2. Four of them pay up to
+// 12 rows of x while a CU has no more than one workgroup (4096 x 3072 at 8 rows 8.7 on
+// 2, 8.2 on 4; at 16 rows 9.1 and 9.9), not with a unit behind them, whose workgroup
+// reads two blocks of weights (2 x 4096 x 3072 at 8 rows 12.2, 14.9).
 #include "common.h"
 #include "gemm_stream.h"
 
@@ -375,13 +380,14 @@ static void skinny_launch(const SkinnyArgs& A, hipStream_t s) {
   // 8192 x 4096 16.2 -> 14.2; rows of 4 KB or fewer than 8192 of them 0 to 10 % more.
   // Waves: see the top.
   const bool spread = A.K % 4096 == 0 && (GATED ? 2 : 1) * A.N >= 8192;
+  const bool few = blocks <= 256 && !(NF == 2 && !GATED);
   if (spread) LAUNCH_SK(2, true);
-  else if ((NF == 2 && !GATED) || blocks > 256 ||
-           (steps > 64 && A.M > 8))
-    LAUNCH_SK(2, false);
-  else if (steps > 64) LAUNCH_SK(4, false);
-  else if (steps > 32) LAUNCH_SK(16, false);
-  else LAUNCH_SK(8, false);
+  else if (steps == 16) LAUNCH_SK(4, false);
+  else if (steps == 32) LAUNCH_SK(8, false);
+  else if (GATED || !few || steps < 16) LAUNCH_SK(2, false);
+  else if (steps == 64) LAUNCH_SK(16, false);
+  else if (A.M <= 12) LAUNCH_SK(4, false);
+  else LAUNCH_SK(2, false);
 #undef LAUNCH_SK
 }
 
@@ -410,11 +416,12 @@ extern "C" void sutro_linear_skinny(void* out, long ldo, const void* x,
   } while (0)
   // 32 rows of W a workgroup read half as much of x, but where they take more
   // rounds of the chip than 16 do: 10304 x 4096 at 16 rows 30.6 and 27.0 us, 6144 x
-  // 4096 14.9 and 18.3
+  // 4096 14.9 and 18.3. A few workgroups more than one round are none: 4104 x 3072 at
+  // 3 rows 10.6 and 9.4, 4608 x 3072 10.8 and 10.8, at 16 rows 12.1 and 15.4.
   const int rounds16 = (N + 16 * 256 - 1) / (16 * 256);
   const int rounds32 = (N + 32 * 256 - 1) / (32 * 256);
   if (act == 1) SK_MB(2, true);
-  else if (2 * rounds32 <= rounds16) SK_MB(2, false);
+  else if (2 * rounds32 <= rounds16 && N >= 4352) SK_MB(2, false);
   else SK_MB(1, false);
 #undef SK_MB
 }

@@ -29,6 +29,19 @@ def test_kernel(N, K, gated, M):
     torch.testing.assert_close(got, y, rtol=2 ** -8, atol=2 ** -12)
 
 
+@pytest.mark.parametrize("M", [3, 12, 13, 17])
+@pytest.mark.parametrize("N,K,gated", [
+    (64, 448, False), (4096, 512, False), (9216, 512, False),
+    (12, 1024, False), (8272, 1024, False), (2048, 1056, False),
+    (4096, 2048, False), (4112, 2048, False), (4348, 640, False),
+    (4352, 640, False), (4096, 2080, False), (40, 512, True), (8208, 512, True),
+    (1024, 1024, True), (256, 2048, True), (8192, 1536, True)])
+def test_waves(N, K, gated, M):
+    """A batch each for 4, 8 and 16 waves, one k-step less and more; a round of
+    workgroups and some more."""
+    test_kernel(N, K, gated, M)
+
+
 @pytest.mark.parametrize("M,rows,K,want", [
     (3, 20000, 2048, True), (16, 24576, 2048, True), (16, 24576, 4096, False),
     (17, 20000, 2048, False), (12, 8192, 4096, True), (13, 8192, 4096, False),
