@@ -206,7 +206,9 @@ def _long_weights(M: int, rows: int, K: int) -> bool:
     if K <= 2048 or K == 4096:
         return M <= (8 if rows * K <= 1 << 28 else 6) and (
             rows <= 24576 or K >= 2048)
-    return rows <= 5120 and K >= 16384 and K % 4096 != 0    # nor there
+    # nor there; of fewer than 2048 rows it has one for more than 16 of x
+    return ((64 if M <= 16 else 2048) <= rows <= 5120 and K >= 16384
+            and K % 4096 != 0)
 
 
 def _few_rows(x, w, gated: bool = False) -> bool:
@@ -214,6 +216,8 @@ def _few_rows(x, w, gated: bool = False) -> bool:
     library takes 11 us or more for most products; us by it and by the kernel,
     weights from memory:
       rows of w x K    M = 1          2             3             8             16            32
+      2048 x 512                                     4.6 /  2.9     4.6 /  3.0     4.6 /  3.2     6.7 /  3.6
+      2048 x 1024                                    5.8 /  3.6     5.8 /  3.8     5.8 /  4.1     8.1 /  5.0
       2048 x 2048      11.0 /  4.8    10.7 /  5.9   11.1 /  5.3   11.0 /  5.6   11.0 /  6.3   11.2 /  8.5
       4096 x 2048                                   11.6 /  6.3   11.6 /  6.4   11.6 /  7.1   11.8 /  9.2
       6144 x 2048                                   13.0 /  8.9   12.7 /  9.4   12.5 /  9.0   12.6 / 11.8
@@ -221,8 +225,12 @@ def _few_rows(x, w, gated: bool = False) -> bool:
       18432 x 2048                                  57.6 / 19.2   57.4 / 20.3   57.4 / 24.5   20.6 / 34.7
       32768 x 2048                                  34.0 / 30.3   31.8 / 30.2   31.7 / 33.3   34.0 / 41.1
       151936 x 2048                                  205 / 126     204 / 137     202 / 155     145 / 193
+      32 x 3072                                      7.1 /  5.6     7.0 /  6.3     8.3 /  7.2     7.0 / 10.0
+      2048 x 3072      12.1 /  5.2    11.9 /  6.3   12.3 /  6.8    12.3 /  7.6    12.2 /  8.6    10.3 / 11.3
       8192 x 3072                                   19.3 / 12.7   17.2 / 12.3   17.2 / 12.9   17.3 / 17.5
       16384 x 3072                                  22.5 / 22.9   21.4 / 23.4   21.5 / 26.5   21.6 / 35.1
+      32 x 4096                                      8.0 /  7.1     8.1 /  7.9    10.7 /  9.0     8.4 / 12.7
+      512 x 4096                                    11.0 /  7.4    11.1 /  8.3    11.1 /  9.4     8.6 / 13.0
       4096 x 4096      15.4 /  7.8    15.2 / 10.0   15.7 /  9.1   15.5 /  9.4   15.4 / 10.9   13.0 / 14.0
       6144 x 4096      15.6 / 10.9    15.3 / 13.0   15.6 / 14.5   14.5 / 13.9   14.4 / 14.8   15.2 / 20.2
       8192 x 4096      17.1 / 14.7    16.5 / 18.3   16.7 / 15.2   15.8 / 14.6   15.8 / 15.5   16.4 / 20.3
@@ -234,6 +242,11 @@ def _few_rows(x, w, gated: bool = False) -> bool:
       12288 x 5120     26.8 / 23.9    25.9 / 25.7
       12288 x 12288    61.0 / 60.6    60.7 / 64.9
       4096 x 16384                                  30.8 / 31.3   29.8 / 31.1   29.8 / 36.6   33.7 / 46.0
+      32 x 17408                                                   22.7 / 26.3    36.7 / 31.4    43.1 / 46.2
+      64 x 25600                                    53.3 / 32.1    53.4 / 37.5    53.3 / 45.3    40.6 / 66.9
+      1024 x 25600                                  67.0 / 32.9    67.5 / 38.9    67.2 / 46.9    65.1 / 68.6
+      2048 x 25600                                  70.1 / 33.4    70.1 / 39.5    70.0 / 47.7    94.0 / 69.1
+      5120 x 20000                                  70.6 / 47.5    68.9 / 50.3    69.0 / 56.8    72.4 / 75.8
       5120 x 17408                                   111 / 43      112 / 46      114 / 52      121 / 77
       5120 x 25600      135 / 51       136 / 57      134 / 60      135 / 64      137 / 72      145 / 108
     and with silu_mul behind it (rows of both halves)
