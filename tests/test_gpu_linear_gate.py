@@ -36,6 +36,14 @@ def test_kernel(M, N, K):
     torch.testing.assert_close(got, want, rtol=2 ** -8, atol=2 ** -12)
 
 
+@pytest.mark.parametrize("M", [1025, 2900, 8193 + 1800])
+@pytest.mark.parametrize("blocks", [9, 12, 15])
+def test_leftover_row_tiles(M, blocks):
+    """Row tiles past the last group of 32, four at a time on all XCDs, with
+    column blocks that do not divide among these."""
+    test_kernel(M, blocks * 128, 192)
+
+
 def test_route():
     """The one launch and the library's two passes agree, and what torch has to
     see still goes through torch."""
