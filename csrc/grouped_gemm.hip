@@ -163,24 +163,18 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   const int b_off = BM * 64;
   const int b2_off = (BM + BN) * 64;
 
-  // Workgroups start at different steps of k where weight rows are multiples of
-  // 4 KB apart: all in step they read the same few 128-byte columns of a hundred
-  // thousand rows at a time, which lie on few memory channels. 32 experts of 2048
-  // x 2048, 128 tokens of 4 on tiles of 32: gate and up 132 -> 95 us, down 67 -> 48
-  // (4.0 -> 5.6 TB/s); 16 tokens 100 -> 79 and 61 -> 49; 256 tokens on tiles of 64
-  // 154 -> 129 and 75 -> 53. Rows of 6 KB spread by themselves (160 us, rotated 172).
-  // Tiles of one expert share its weights and stay in step (70 rows an expert on
-  // tiles of 64: down 115 us, 134 with starts of their own), and so do tiles of 128
-  // rows, whose column blocks share rows of x (71, rotated 80).
+  // Experts start at different steps of k where weight rows are multiples of 4 KB
+  // apart: all in step, workgroups read the same few 128-byte columns of a hundred
+  // thousand rows at a time, which lie on few memory channels. 32 experts of
+  // 2048 x 2048, 128 tokens of 4 on tiles of 32: gate and up 130 -> 91 us, down 72 ->
+  // 54 (5.9 TB/s and 5.0); 16 tokens 137 -> 95 and 74 -> 56; 256 tokens on tiles of 64
+  // 160 -> 133 and 77 -> 55. Rows of 6 KB spread by themselves. All workgroups of an
+  // expert stay in step: its column blocks share rows of x (a start for each of them
+  // 65 us instead of 54, 78 instead of 55, and 12 to 27 % more than none for 60
+  // experts), its tiles weights, and a row's sums come out the same in every tile.
+  // Tiles of 128 rows all start at 0.
   const int KT = (int)(K >> 6);
-  const int start = BM <= 64 && K % 2048 == 0 && tile_off[e + 1] == t + 1 &&
-                            tile_off[e] == t
-                        ? (int)(e * 5u + blockIdx.y * 3u) % KT
-                        : 0;
-  auto k_of = [&](int kt) {
-    const int z = kt + start;
-    return (long)(z < KT ? z : z - KT) * 64;
-  };
+  int ko = BM <= 64 && K % 2048 == 0 ? (int)(e * 5u) % KT * 64 : 0;
   const long Kb = K * 2;
   const u16* wa = w + (long)e * (GATED ? 2 : 1) * n_cols * K;
   const u16* wg = wa + (long)n0 * K;
@@ -198,18 +192,17 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
     }
 
   // prologue
-  const long k_first = k_of(0);
   if (GATHER)
-    gg_stage<BM, WAVES, true>(smem[0], aa + k_first, Kb, rt, m0, rows_valid,
-                              wave, lane);
+    gg_stage<BM, WAVES, true>(smem[0], aa + ko, Kb, rt, m0, rows_valid, wave,
+                              lane);
   else
-    gg_stage<BM, WAVES, false>(smem[0], aa + k_first, Kb, nullptr, m0, BM, wave,
+    gg_stage<BM, WAVES, false>(smem[0], aa + ko, Kb, nullptr, m0, BM, wave,
                                lane);
-  gg_stage<BN, WAVES, false>(smem[0] + b_off, wg + k_first, Kb, nullptr, 0, BN,
-                             wave, lane);
+  gg_stage<BN, WAVES, false>(smem[0] + b_off, wg + ko, Kb, nullptr, 0, BN, wave,
+                             lane);
   if (GATED)
-    gg_stage<BN, WAVES, false>(smem[0] + b2_off, wu + k_first, Kb, nullptr, 0,
-                               BN, wave, lane);
+    gg_stage<BN, WAVES, false>(smem[0] + b2_off, wu + ko, Kb, nullptr, 0, BN,
+                               wave, lane);
   __syncthreads();
 
   for (int kt = 0; kt < KT; ++kt) {
@@ -218,7 +211,8 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
     u16* bgT = smem[p] + b_off;
     u16* buT = smem[p] + b2_off;
     if (kt + 1 < KT) {
-      const long ko = k_of(kt + 1);
+      ko += 64;
+      if (ko == (int)K) ko = 0;
       if (GATHER)
         gg_stage<BM, WAVES, true>(smem[p ^ 1], aa + ko, Kb, rt, m0,
                                   rows_valid, wave, lane);

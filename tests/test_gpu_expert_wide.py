@@ -69,27 +69,61 @@ def test_operands_off_boundaries(act):
 
 @pytest.mark.parametrize("K", [1024, 2048, 4096])
 @pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
-def test_place_of_a_row(K, act):
+@pytest.mark.parametrize("bm", [32, 64, 128, 256])
+def test_place_of_a_row(K, act, bm):
     """The dispatch puts tokens where its counters stand: a token's result is the
     same to the bit in every tile of its expert, on every XCD."""
     g = torch.Generator(device=DEV).manual_seed(K)
     gated = act == hops.ACT_SILU_GATE
     counts, ff, T = [9000, 300, 5000], 512, 7
-    tiles = [(c + 255) // 256 for c in counts]
+    tiles = [(c + bm - 1) // bm for c in counts]
     off = torch.tensor([0] + tiles, device=DEV).cumsum(0).int()
     cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
-    rows = sum(tiles) * 256
+    rows = sum(tiles) * bm
     x = torch.randn(T, K, generator=g, device=DEV).bfloat16()
     w = (torch.randn(3, 2 * ff if gated else ff, K, generator=g, device=DEV)
          * K ** -0.5).bfloat16()
     which = torch.arange(rows, device=DEV) * 5 % T
     out = torch.empty(rows, ff, device=DEV, dtype=torch.bfloat16)
     if gated:
-        hops.expert_gemm(out, x, w, which.int(), off, cnt, act, 256, 0.0, None)
+        hops.expert_gemm(out, x, w, which.int(), off, cnt, act, bm, 0.0, None)
     else:
-        hops.expert_gemm(out, x[which], w, None, off, cnt, act, 256, 0.0, None)
+        hops.expert_gemm(out, x[which], w, None, off, cnt, act, bm, 0.0, None)
     for e, c in enumerate(counts):
-        a = int(off[e]) * 256
+        a = int(off[e]) * bm
         for t in range(T):
             same = out[a:a + c][which[a:a + c] == t]
             assert torch.equal(same, same[:1].expand_as(same)), (e, t)
+
+
+@pytest.mark.parametrize("bm", [32, 64])
+@pytest.mark.parametrize("K", [2048, 4096])
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
+def test_starts_of_small_tiles(bm, K, act):
+    """Rows of 4 KB: experts that begin at all steps of k, some without rows,
+    some with several tiles, against 64 bits."""
+    g = torch.Generator(device=DEV).manual_seed(K + bm)
+    counts = [(i * 23) % 70 for i in range(40)]
+    gated = act == hops.ACT_SILU_GATE
+    ff, T = 128, 50
+    tiles = [(c + bm - 1) // bm for c in counts]
+    off = torch.tensor([0] + tiles, device=DEV).cumsum(0).int()
+    cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
+    rows = sum(tiles) * bm
+    w = (torch.randn(40, 2 * ff if gated else ff, K, generator=g, device=DEV)
+         * K ** -0.5).bfloat16()
+    x = torch.randn(T, K, generator=g, device=DEV).bfloat16()
+    which = torch.arange(rows, device=DEV) * 7 % T
+    out = torch.empty(rows, ff, device=DEV, dtype=torch.bfloat16)
+    if gated:
+        hops.expert_gemm(out, x, w, which.int(), off, cnt, act, bm, 0.0, None)
+    else:
+        hops.expert_gemm(out, x[which], w, None, off, cnt, act, bm, 0.0, None)
+    for e, c in enumerate(counts):
+        a = int(off[e]) * bm
+        y = x[which[a:a + c]].double() @ w[e].double().T
+        if gated:
+            y = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+        # fp32 sums of K products of size K^-1/2, one rounding to bf16
+        torch.testing.assert_close(out[a:a + c].double(), y, rtol=2 ** -8,
+                                   atol=2 ** -12)
