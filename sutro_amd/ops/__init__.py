@@ -292,9 +292,10 @@ def linear(x, w, bias=None):
 
 def _many_rows(x, w) -> bool:
     """Whether csrc/grouped_gemm.hip makes silu_mul(x w^T) in one launch. Its
-    tiles are 256 rows by 128 columns of the result, one a CU at a time: below
-    256 of them the library's smaller tiles are ahead, and where the last round
-    leaves a quarter of all places empty (us of both, tiles):
+    tiles are 256 rows by 128 columns of the result, one a CU at a time. Far
+    below 256 of them the library's smaller tiles are ahead, and from there on
+    where the last round leaves a quarter of all places empty (us of both,
+    tiles):
       2 x 3072 x 1024    1024 rows  25.1 /  26.7 ( 96)   2048   36.2 / 29.2 (192)
                          2600 rows  51.6 /  54.3 (264)   3328   58.6 / 53.6 (312)
       2 x 6144 x 2048     512 rows  33.4 /  42.6 ( 96)   1024   53.6 / 48.9 (192)
@@ -302,22 +303,33 @@ def _many_rows(x, w) -> bool:
       2 x 8192 x 2048     512 rows  39.7 /  45.5 (128)   1024   66.5 / 54.2 (256)
                          1280 rows  86.9 /  89.4 (320)   1536   96.7 / 93.1 (384)
       2 x 12288 x 4096    768 rows   150 /   161 (288)   1024    173 /  170 (384)
-    Otherwise it is 2 to 45 % faster, or as fast (the figures at many rows stand
+    or where a row tile that is nearly empty does (of all rows that the places
+    have, those of x):
+      2 x 25344 x 2048    274 rows  77.4 /  93.4 (0.41)
+      2 x 26496 x 5120    363 rows   224 /   239 (0.57)
+      2 x 21248 x 4096   1027 rows   339 /   364 (0.65)
+      2 x 23168 x 512     775 rows  83.2 /  51.2 (0.71)
+      2 x 12544 x 256     938 rows  36.8 /  25.8 (0.70)
+    Otherwise it is 2 to 50 % faster, or as fast (the figures at many rows stand
     beside the kernel). Short k, which the library does worst at, still gains
-    with two fifths empty."""
+    with two fifths of the places empty. (192 to 255 tiles would gain where they
+    were tried; they stay with the library.)"""
     if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False
-    if x.dim() != 2 or w.dim() != 2 or not _use_hip(x):
+    if x.dim() != 2 or w.dim() != 2:
         return False
     M, K = x.shape
     rows = w.shape[0]
     tiles = -(-M // 256) * (rows // 256)
+    if tiles < 256:
+        return False
     places = -(-tiles // 256) * 256
-    return (rows % 256 == 0 and tiles >= 256
-            and tiles >= places * (0.6 if K <= 1024 else 0.75)
-            and K % 64 == 0 and 0 < K < 1 << 21 and M * K < 1 << 30
-            and rows < 1 << 24 and w.shape[1] == K and _unwatched()
+    filled, live = (0.6, 0.5) if K <= 1024 else (0.75, 0.67)
+    return (tiles >= places * filled and M * (rows // 256) >= 256 * places * live
+            and rows % 256 == 0 and K % 64 == 0 and 0 < K < 1 << 21
+            and M * K < 1 << 30 and rows < 1 << 24 and w.shape[1] == K
+            and _use_hip(x) and _unwatched()
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.device == x.device and x.is_contiguous()
             and w.is_contiguous()

@@ -159,3 +159,14 @@ def test_long_rows_of_few(kernels, rows, k, n, kernel):
     w = torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
     assert ops._few_rows(torch.empty(rows, k, dtype=torch.bfloat16),
                          w) == bool(kernel)
+
+
+@pytest.mark.parametrize("rows,k,n,kernel", [
+    (274, 2048, 50688, 0), (363, 5120, 52992, 0), (512, 2048, 50688, 1),
+    (1027, 4096, 42496, 0), (1280, 4096, 42496, 1), (775, 512, 46336, 1),
+    (300, 1024, 34816, 0), (2048, 1024, 8192, 1), (2047, 1024, 7936, 0)])
+def test_gated_layers_of_many_rows(kernels, rows, k, n, kernel):
+    """A row tile with few rows in it counts by its rows."""
+    x = torch.empty(rows, k, dtype=torch.bfloat16)
+    w = torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
+    assert ops._many_rows(x, w) == bool(kernel)
