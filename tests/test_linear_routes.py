@@ -170,3 +170,14 @@ def test_gated_layers_of_many_rows(kernels, rows, k, n, kernel):
     x = torch.empty(rows, k, dtype=torch.bfloat16)
     w = torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
     assert ops._many_rows(x, w) == bool(kernel)
+
+
+@pytest.mark.parametrize("k,n,inside", [
+    (128, 12288, 1), (128, 35296, 0), (640, 16384, 0), (672, 65536, 1),
+    (2048, 65536, 1), (2048, 131072, 0), (4096, 24576, 1), (4128, 4096, 0)])
+def test_norm_in_front_of_one_row(kernels, k, n, inside):
+    """Many short rows of weights: the norm has a launch of its own."""
+    def bf(*shape):
+        return torch.empty(*shape, dtype=torch.bfloat16)
+    assert ops._one_row(bf(1, k), bf(1, k), bf(k), bf(n, k),
+                        False) == bool(inside)
