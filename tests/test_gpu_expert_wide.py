@@ -127,3 +127,37 @@ def test_starts_of_small_tiles(bm, K, act):
         # fp32 sums of K products of size K^-1/2, one rounding to bf16
         torch.testing.assert_close(out[a:a + c].double(), y, rtol=2 ** -8,
                                    atol=2 ** -12)
+
+
+@pytest.mark.parametrize("K", [2048, 4096])
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
+@pytest.mark.parametrize("shift", [0, 8 + 2])
+def test_rows_of_4_kb(K, act, shift):
+    """Experts start at steps of their own, and a workgroup goes from a tile of
+    one to a tile of the next: more tiles than workgroups, 64-bit addresses too."""
+    _run([3000, 0, 257, 2900, 1, 520, 256, 700], K, 2304, act, shift)
+
+
+def test_gathered_rows_past_4_gb():
+    """1,100,000 rows of 4 KB: more than 32-bit offsets reach."""
+    K, ff, R = 2048, 256, 1_100_000
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.zeros(R, K, device=DEV, dtype=torch.bfloat16)
+    used = torch.cat([torch.arange(0, 40), torch.arange(1048576 - 40, 1048576 + 40),
+                      torch.arange(R - 40, R)]).to(DEV)
+    x[used] = torch.randn(len(used), K, generator=g, device=DEV).bfloat16()
+    counts = [300, 70]
+    off = torch.tensor([0, 2, 3], device=DEV, dtype=torch.int32)
+    cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
+    tok = used[torch.arange(768, device=DEV) * 7 % len(used)]
+    w = (torch.randn(2, 2 * ff, K, generator=g, device=DEV)
+         * K ** -0.5).bfloat16()
+    out = torch.empty(768, ff, device=DEV, dtype=torch.bfloat16)
+    hops.expert_gemm(out, x, w, tok.int(), off, cnt, hops.ACT_SILU_GATE, 256,
+                     0.0, None)
+    for e, a, c in ((0, 0, 300), (1, 512, 70)):
+        y = x[tok[a:a + c]].double() @ w[e].double().T
+        y = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+        # fp32 sums of K products, one rounding to bf16
+        torch.testing.assert_close(out[a:a + c].double(), y, rtol=2 ** -8,
+                                   atol=2 ** -12)

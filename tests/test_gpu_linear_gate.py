@@ -36,6 +36,12 @@ def test_kernel(M, N, K):
     torch.testing.assert_close(got, want, rtol=2 ** -8, atol=2 ** -12)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (9000, 1024, 2048), (8500, 1152, 4096), (2300, 4096, 2048)])
+def test_more_tiles_than_workgroups(M, N, K):
+    test_kernel(M, N, K)
+
+
 @pytest.mark.parametrize("M", [1025, 2900, 8193 + 1800])
 @pytest.mark.parametrize("blocks", [9, 12, 15])
 def test_leftover_row_tiles(M, blocks):

@@ -150,6 +150,19 @@ def test_many_short_prompts(Hq, Hk, D, longest):
     _check(args, _prefill(args, D, _tiles(new)))
 
 
+# heads of 64, several steps a prompt: four workgroups a CU
+@pytest.mark.parametrize("Hq,Hk", [(8, 8), (14, 2), (16, 8), (16, 4)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_many_prompts_of_several_steps(Hq, Hk, fp8):
+    g = torch.Generator().manual_seed(Hq)
+    new = torch.randint(90, 257, (130,), generator=g).tolist()
+    ctx = torch.randint(0, 150, (130,), generator=g).tolist()
+    args = _paged([a + b for a, b in zip(new, ctx)], new, Hq, Hk, 64, fp8, seed=3)
+    tiles = _tiles(new)
+    assert 512 <= len(tiles[0]) <= 8 * 130
+    _check(args, _prefill(args, 64, tiles))
+
+
 @pytest.mark.parametrize("Hq,Hk", [(2, 2), (4, 2), (4, 1)])
 def test_prompt_tiles_in_any_order(Hq, Hk):
     # a tile map need not list a sequence's tiles in order, nor at all
