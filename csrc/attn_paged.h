@@ -175,9 +175,14 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 //
 // Products are of 16 x 16 x 32: those of 32 x 32 x 16 do as much a cycle but read
 // and write every sum twice as often, which the power limit takes off the clock.
-// 32 k prompt (16 heads, 4 kv heads, 128) 4.59 -> 4.19 ms (958 -> 1050 TFLOP/s), 16 of
-// 2 k 359 -> 338 us, 7 of 3 k with 32 heads over e4m3 605 -> 560, 2 of 20 k with 16
-// heads of 64 2.19 -> 2.05 ms, 16 of 2 k in chunks of 1024 251 -> 243 us.
+// In turn on one card: 32 k prompt (16 heads, 4 kv heads, 128) 4.41 -> 4.04 ms (998 ->
+// 1088 TFLOP/s, the clock 1.99 -> 2.11 GHz, the matrix cores as busy as before), 40 k
+// 6.55 -> 6.03, 16 of 2 k 358 -> 335 us, 7 of 3 k with 32 heads over e4m3 609 -> 550, 2
+// of 20 k with 16 heads of 64 2.15 -> 2.02 ms; 16 of 2 k in chunks of 1024 231 -> 230 us.
+// Where the power limit is out of reach a step takes as long as before or a little
+// longer: one prompt of 3000 tokens with 16 heads and 8 kv heads 76.2 and 76.5 us, of
+// 3850 with one head 86.2 and 88.8. Four keys' fragments are read ahead for it (six,
+// which the larger products wanted: 78.6 and 91.4; two 79.0 and 92.1; all 84.3 and 99.5).
 //
 // BLOCKS: more than one block of rows in a workgroup.
 //
@@ -392,7 +397,7 @@ paged_prefill_kernel(PagedArgs A) {
         d[0][t] = pa_mfma16(ka, qb[0][kk], d[0][t]);
         d[1][t] = pa_mfma16(ka, qb[1][kk], d[1][t]);
       }
-    pa_order<D / 8, D / 8, LATE ? 2 : 6, 1, 2>();
+    pa_order<D / 8, D / 8, LATE ? 2 : 4, 1, 2>();
     // without a distance bias scores stay unscaled until the exponential
     const bool whole = kv0 + PA_KEYS <= p0 + rb * 32 + 1 &&
                        (!LOCAL || kv0 >= lo_last);
