@@ -277,8 +277,9 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
 // sums, and a wave reads 32 KB of LDS for 2.1 MFLOP. One workgroup a CU stays for
 // the whole launch and goes from tile to tile; its copies run across the tiles.
 //
-// Bound by the power limit and by the copies' share of the LDS: the matrix cores
-// are busy 65 to 77 % at 1.75 to 1.85 GHz. What that took:
+// Bound by the power limit and by the copies' share of the LDS: by the counters the
+// matrix cores are busy 65 to 79 %, and the clock falls from 2.7 GHz in a launch of
+// 44 us to 1.8 in one of 4.7 ms. What that took:
 // - mfma 16x16x32 instead of 32x32x16. Both do as much a cycle, but a sum is read
 //   and written half as often, and the clock the power limit leaves is higher:
 //   8192^3 785 -> 727 us, the rest alike.
@@ -288,15 +289,16 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
 //   scalar) into a ring of five units of 32 KB: three of A rows and B rows ahead
 //   of those in use, A two steps and B one step before they are needed.
 // At 32 experts of 2048 x 2048, gate and up / down, against eight waves of 128 x
-// 64 with two buffers: 4096 rows an expert 2081 / 1086 -> 1630 / 840 us (1057 /
-// 1013 -> 1350 / 1309 TFLOP/s), 384 rows 277 / 145 -> 225 / 112. A large product of
-// the library reaches 1.6 PFLOP/s on the same card (8192^3: 675 us).
+// 64 with two buffers, in turn on one card: 4096 rows an expert 1910 / 977 -> 1595 /
+// 808 us (1151 / 1125 -> 1379 / 1361 TFLOP/s), 384 rows 276 / 135 -> 224 / 117, 187
+// rows 163 / 82 -> 140 / 70. A large product of the library reaches 1.65 PFLOP/s
+// there (8192^3: 668 us). Cards differ by 5 to 15 % in what their power limit leaves.
 //
 // DENSE (mode 5) is a gated linear layer of its own, one matrix over m_rows rows,
 // against the library's product and a pass of silu over its result (2 N columns
-// written and read again): 2 x 3072 x 1024 at 24,000 rows 363 -> 256 us, 2 x 8192 x
-// 2048 at 32,768 rows 1827 -> 1605, 2 x 12288 x 4096 4734 -> 4613, 2 x 25600 x 5120
-// at 8192 rows 3356 -> 2925; the unit's inputs stay in fp32 (error against 64 bits
+// written and read again): 2 x 3072 x 1024 at 24,000 rows 357 -> 259 us, 2 x 8192 x
+// 2048 at 32,768 rows 1775 -> 1555, 2 x 12288 x 4096 4597 -> 4413, 2 x 25600 x 5120
+// at 8192 rows 3280 -> 2829; the unit's inputs stay in fp32 (error against 64 bits
 // 3.1e-3 -> 1.7e-3).
 //
 // An XCD (workgroup id % 8) takes GW_ROWS neighbouring row tiles and goes through
@@ -402,8 +404,8 @@ __device__ __forceinline__ u32 gw_pack(float x, float y) {
   return __builtin_bit_cast(u32, p);
 }
 
-// DENSE: see above. ANY: gathered rows of 4 GB or more in all, or operands that do not begin at
-// multiples of 16 bytes; 64-bit addresses and narrow stores then.
+// DENSE: see above. ANY: gathered rows of 4 GB or more in all, or operands that do
+// not begin at multiples of 16 bytes; 64-bit addresses and narrow stores then.
 template <int MODE, bool ANY>
 __device__ __forceinline__ void gw_body(
     u16* __restrict__ out, const u16* __restrict__ a,
@@ -592,7 +594,7 @@ __device__ __forceinline__ void gw_body(
         acc[i][j] = mfma16g(fb[kk][j], fa[kk][i], acc[i][j]);
         // reads behind every third product, copies behind every eighth: the LDS
         // takes both beside each other, and the cache the copies of four waves
-        // (eight within the first half: down of 32 experts 843 us, now 812)
+        // (eight within the first half: down of 32 experts at 4096 rows 4 % more)
         if (x % 3 == 0 && x / 3 < 16 && (kk == 0 || MORE)) {
           const int y = x / 3;
           if (y < 8) load_b(y, kk ? nbs : sb, kk ^ 1);
@@ -627,7 +629,8 @@ __device__ __forceinline__ void gw_body(
   // a token where its counter happens to stand, and the token's sums have to come
   // out the same in every place. By column blocks as well, which takes workgroups of
   // an XCD out of step: 144 / 85, 233 / 125, 1704 / 842. One matrix (DENSE) has one
-  // start, 0.
+  // start, 0 (whole prompts were 0 to 1.5 % faster with one for each XCD, but equal
+  // rows of a batch differed).
   auto first = [&](const GwTile& g) {
     return !DENSE && K % 2048 == 0 ? (g.e * 5 & 7) * KT / 8 * 64 : 0;
   };
@@ -801,7 +804,8 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
 }
 
 // out [M, N] = silu(x Wg^T) * (x Wu^T): w [2 N, K], the gate's rows first. x and
-// w at multiples of 16 bytes, K a multiple of 64, N of 128, M K below 2 G.
+// w at multiples of 16 bytes, K a multiple of 64 and below 2^21 (a tile's offsets
+// are of 32 bits, where it begins of 64), N a multiple of 128.
 extern "C" void sutro_linear_silu_mul(void* out, const void* x, const void* w,
                                       int M, int N, long K,
                                       hipStream_t stream) {

@@ -212,9 +212,8 @@ def _long_weights(M: int, rows: int, K: int) -> bool:
 
 
 def _few_rows(x, w, gated: bool = False) -> bool:
-    """Whether csrc/gemm_skinny.hip is the faster one for x [M, K] w^T. The
-    library takes 11 us or more for most products; us by it and by the kernel,
-    weights from memory:
+    """Whether x [M, K] w^T goes to csrc/gemm_skinny.hip. The library takes 11 us
+    or more for most products; us by it and by the kernel, weights from memory:
       rows of w x K    M = 1          2             3             8             16            32
       2048 x 512                                     4.6 /  2.9     4.6 /  3.0     4.6 /  3.2     6.7 /  3.6
       2048 x 1024                                    5.8 /  3.6     5.8 /  3.8     5.8 /  4.1     8.1 /  5.0
@@ -256,7 +255,10 @@ def _few_rows(x, w, gated: bool = False) -> bool:
       12288 x 8192     43.9 / 42.4    43.8 / 47.5
       51200 x 5120     98.8 / 92.3    99.1 / 95.9   95.6 / 134    92.3 / 139    92.8 / 158    95.8 / 196
     Two rows lose where the library has a good tile (24 to 64 M weights of long
-    rows) and one load a weight row is no longer the whole cost."""
+    rows) and one load a weight row is no longer the whole cost. The line is on
+    the library's side of some sizes at which the kernel is ahead: 7 to 16 rows
+    over 151936 x 2048, 13 to 16 over 8192 x 3072 or, with the unit, 16384 x
+    2048 (the sizes between them have not been tried)."""
     if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False
@@ -384,21 +386,23 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
     for `n_rows` (token, expert) pairs in bf16 on the matrix cores (K and N
     multiples of 64), by the rows an expert gets on average. Taller tiles do
     more work per byte but pad more; both products together, at 32 experts of
-    2048 x 2048: at 96 rows 281 / 213 / 219 us on tiles of 64 / 128 / 256, at
-    192 rows 393 / 340 / 218, at 384 rows 952 / 510 / 340.
+    2048 x 2048: at 72 rows 261 / 215 / 200 us on tiles of 64 / 128 / 256, at 96
+    rows 261 / 212 / 197, at 192 rows 370 / 341 / 198, at 384 rows 877 / 511 /
+    337. (So tiles of 256 would already pay at 72 rows there, and the lines below
+    were drawn when their kernel was a slower one; they have not been moved.)
 
     They also leave fewer workgroups: one of 256 rows takes 128 columns of the
-    gated product or 256 of the other, and below 128 of them in either product
-    the chip idles. 8 experts of 1024 x 512, 192 / 512 / 1024 rows an expert (24 /
-    64 / 128 of either) 26 / 40 / 63 us on 64, 33 / 37 / 47 on 128, 41 / 42 / 44 on
-    256. (8 of 2048 x 2048 would already gain with 64 to 96 of the second, 192 /
-    384 rows: 81 / 131 us on 128, 83 / 99 on 256; the line is the one that holds
-    for both.) Tiles of 128 want 96.
+    gated product or 256 of the other, and with few of them in either product
+    the chip idles: the rule wants 128. 8 experts of 1024 x 512, 192 / 512 / 1024
+    rows an expert (24 / 64 / 128 of either) 26 / 42 / 64 us on 64, 33 / 37 / 47 on
+    128, 41 / 42 / 44 on 256. 8 of 2048 x 2048 are past the crossing with 64 to 96
+    of the second, 192 / 384 / 512 rows: 82 / 133 / 147 us on 128, 83 / 100 / 99 on
+    256. Tiles of 128 want 96.
 
     Up to 16 rows, where the weights are all there is to read, tiles of 32: four
     workgroups of the gated product fit a CU instead of three. They are taken
     unless their number then fills the rounds worse: 1024 workgroups (2048 wide)
-    167 -> 140 us, 1536 (3072 wide, K 4096) 438 -> 445.
+    171 -> 133 us, 1536 (3072 wide, K 4096) 448 and 448.
 
     `local`: the experts whose products this rank makes (all by default); its
     workgroups are counted."""

@@ -88,8 +88,8 @@ def test_tile_rule(n_rows, want):
     (8, 2048, 2048, 512, 256), (8, 1024, 512, 1024, 128),
     (4, 512, 512, 512, 64), (32, 2048, 2048, 192, 256)])
 def test_tiles_that_leave_the_chip_busy(experts, inner, width, avg, want):
-    """Few experts of small matrices: the tile that was measured as the faster
-    one."""
+    """Few experts of small matrices: tiles by the workgroups they leave (the
+    figures, and sizes past the crossing, stand with the rule)."""
     from sutro_amd.ops import expert_tile
 
     n = avg * experts
