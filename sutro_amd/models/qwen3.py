@@ -508,10 +508,11 @@ class Qwen3Block(nn.Module):
     def forward(self, x, residual, fb: ForwardBatch, kv, cos_sin):
         attn, mlp = self.self_attn, self.mlp
         norm = self.input_layernorm
+        one = x.shape[0] == 1   # others have no kernel with the norm inside
         if residual is None:
             residual = x
             x = attn(norm(x), fb, kv, cos_sin)
-        elif (type(attn) is Qwen3Attention and bare(attn.qkv_proj)
+        elif (one and type(attn) is Qwen3Attention and bare(attn.qkv_proj)
               and unhooked(attn)):
             qkv, residual = ops.norm_linear(x, residual, norm.weight, norm.eps,
                                             attn.qkv_proj.weight)
@@ -521,7 +522,8 @@ class Qwen3Block(nn.Module):
                                                 norm.eps)
             x = attn(x, fb, kv, cos_sin)
         norm = self.post_attention_layernorm
-        if type(mlp) is Qwen3MLP and bare(mlp.gate_up_proj) and unhooked(mlp):
+        if (one and type(mlp) is Qwen3MLP and bare(mlp.gate_up_proj)
+                and unhooked(mlp)):
             act, residual = ops.norm_linear(x, residual, norm.weight, norm.eps,
                                             mlp.gate_up_proj.weight, gated=True)
             return mlp(None, act), residual

@@ -355,7 +355,7 @@ def _one_row(x, residual, norm_w, w, gated: bool) -> bool:
     rows most of their lanes have no weights to read meanwhile: of two launches
     it takes 0.65 to 0.95 up to 12288 rows of weights; at 65536 0.92 to 0.98 from
     a k of 768 on, 1.00 at 640, 1.2 to 1.4 at 512 and less; at 131072 1.0 to 1.7."""
-    return (_few_rows(x, w, gated) and x.shape[0] == 1 and x.shape[1] <= 4096
+    return (x.shape[0] == 1 and _few_rows(x, w, gated) and x.shape[1] <= 4096
             and w.shape[0] <= (65536 if x.shape[1] > 640 else 12288)
             and x.is_contiguous()
             and type(residual) is torch.Tensor

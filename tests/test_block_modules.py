@@ -105,3 +105,16 @@ def test_backward_hook_of_the_feed_forward(inner):
     (gin, gout), = seen
     assert [tuple(g.shape) for g in gin] == [(1, WIDTH)]
     assert gout[0].shape == (1, module.weight.shape[0] if inner else WIDTH)
+
+
+@pytest.mark.parametrize("rows,calls", [(1, 1), (2, 0), (18, 0)])
+def test_only_one_row_asks_for_the_norm_inside(monkeypatch, rows, calls):
+    """The checks of that call cost small eager batches 5 us a layer."""
+    block, seen = _block(Plain), []
+    whole = ops.norm_linear
+    monkeypatch.setattr(ops, "norm_linear",
+                        lambda *a, **k: seen.append(1) or whole(*a, **k))
+    with torch.no_grad():
+        block(torch.randn(rows, WIDTH), torch.randn(rows, WIDTH), None, None,
+              None)
+    assert len(seen) == calls
