@@ -175,10 +175,12 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 //
 // Products are of 16 x 16 x 32: those of 32 x 32 x 16 do as much a cycle but read
 // and write every sum twice as often, which the power limit takes off the clock.
-// In turn on one card: 32 k prompt (16 heads, 4 kv heads, 128) 4.41 -> 4.04 ms (998 ->
-// 1088 TFLOP/s, the clock 1.99 -> 2.11 GHz, the matrix cores as busy as before), 40 k
-// 6.55 -> 6.03, 16 of 2 k 358 -> 335 us, 7 of 3 k with 32 heads over e4m3 609 -> 550, 2
-// of 20 k with 16 heads of 64 2.15 -> 2.02 ms; 16 of 2 k in chunks of 1024 231 -> 230 us.
+// In turn on one card: 32 k prompt (16 heads, 4 kv heads, 128) 4.42 -> 4.18 ms (996 ->
+// 1052 TFLOP/s, the clock 1.99 -> 2.08 GHz, the matrix cores as busy as before), 40 k
+// 6.63 -> 6.19, 16 of 2 k 361 -> 339 us, 7 of 3 k with 32 heads over e4m3 603 -> 552, 2
+// of 20 k with 16 heads of 64 2.18 -> 2.04 ms, 16 of 2 k in chunks of 1024 235 -> 225 us.
+// Between a decoder's other kernels: the 40 k prompt 31.6 -> 29.6 ms for four layers
+// (0.83 -> 0.89 PFLOP/s), 16 ragged ones of 2 k 443 and 446 us.
 // Where the power limit is out of reach a step takes as long as before or a little
 // longer: one prompt of 3000 tokens with 16 heads and 8 kv heads 76.2 and 76.5 us, of
 // 3850 with one head 86.2 and 88.8. Four keys' fragments are read ahead for it (six,
