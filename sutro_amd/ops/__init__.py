@@ -199,13 +199,19 @@ def _two_rows(rows: int, K: int, gated: bool) -> bool:
 
 def _long_weights(M: int, rows: int, K: int) -> bool:
     """Larger matrices over 3 to 32 rows (both sides in `_few_rows`)."""
-    if 16384 < rows <= 24576 and rows * K < 96 << 20 and K <= 4096:
+    if 16384 < rows <= 24576 and rows * K <= 80 << 20 and K <= 4096:
         return M <= 16                    # the library has no good tile there
     if rows <= 8192 and K <= 4096:
         return M <= 12
     if K <= 2048 or K == 4096:
-        return M <= (8 if rows * K <= 1 << 28 else 6) and (
-            rows <= 24576 or K >= 2048)
+        most = 8
+        # a last round of workgroups (of 32 weight rows) with many CUs idle
+        if (rows > 40960 and 0 < rows % 8192 < 7782) or (
+                K == 4096 and 12288 < rows < 16384):
+            most = 6
+        if rows * K > 1 << 28:
+            most = 6 if K <= 2048 else 4
+        return M <= most and (rows <= 24576 or K >= 2048)
     # nor there; of fewer than 2048 rows it has one for more than 16 of x
     return ((64 if M <= 16 else 2048) <= rows <= 5120 and K >= 16384
             and K % 4096 != 0)
@@ -234,8 +240,13 @@ def _few_rows(x, w, gated: bool = False) -> bool:
       6144 x 4096      15.6 / 10.9    15.3 / 13.0   15.6 / 14.5   14.5 / 13.9   14.4 / 14.8   15.2 / 20.2
       8192 x 4096      17.1 / 14.7    16.5 / 18.3   16.7 / 15.2   15.8 / 14.6   15.8 / 15.5   16.4 / 20.3
       12288 x 4096                                  27.8 / 21.5   26.7 / 23.1   26.5 / 28.5   23.1 / 39.7
+      14336 x 4096                                  27.9 / 25.6    28.4 / 29.0
       20000 x 4096                                  67.2 / 34.5   67.0 / 37.6   67.1 / 46.0   38.7 / 64.9
       32768 x 4096     63.2 / 49.5    62.9 / 56.1   61.3 / 53.6   58.9 / 54.9   59.0 / 61.9   63.0 / 74.8
+      21200 x 4096                                  41.6 / 38.2    40.3 / 41.0    40.6 / 45.4
+      42624 x 4096                                  72.0 / 67.3    72.3 / 78.4
+      59344 x 4096                                   101 / 94      96.9 / 110
+      62592 x 4096                                   117 / 98       116 / 107
       65536 x 4096                                   122 / 104     120 / 107     120 / 121     122 / 178
       5120 x 5120      13.6 / 12.0    13.9 / 14.8   13.9 / 15.3   14.2 / 16.6   15.4 / 19.1   18.0 / 27.8
       12288 x 5120     26.8 / 23.9    25.9 / 25.7

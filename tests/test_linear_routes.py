@@ -181,3 +181,16 @@ def test_norm_in_front_of_one_row(kernels, k, n, inside):
         return torch.empty(*shape, dtype=torch.bfloat16)
     assert ops._one_row(bf(1, k), bf(1, k), bf(k), bf(n, k),
                         False) == bool(inside)
+
+
+@pytest.mark.parametrize("rows,k,n,kernel", [
+    (16, 4096, 20480, 1), (16, 4096, 20720, 0), (8, 4096, 20720, 1),
+    (8, 4096, 14336, 0), (6, 4096, 14336, 1), (8, 4096, 40960, 1),
+    (8, 4096, 59344, 0), (6, 4096, 59344, 1), (8, 4096, 65536, 1),
+    (5, 4096, 113184, 0), (6, 2048, 151936, 1), (8, 2048, 59424, 0)])
+def test_larger_matrices(kernels, rows, k, n, kernel):
+    """Where the library has a good tile, or the last round of workgroups leaves
+    CUs idle, for as many rows as the kernel is still ahead."""
+    w = torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
+    assert ops._few_rows(torch.empty(rows, k, dtype=torch.bfloat16),
+                         w) == bool(kernel)
