@@ -130,7 +130,7 @@ void mix_ssd_prep(float*, float*, float*, const void*, long, int, int,
 int mix_decay_scan(float*, const float*, long, const float*, long,
                    const float*, long, const float*, long, const float*,
                    const float*, float*, const int*, const int*, const int*,
-                   int, int, int, int, int, hipStream_t);
+                   long, int, int, int, int, int, hipStream_t);
 void mix_softcap(float*, const void*, float, long, int, hipStream_t);
 void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
@@ -152,8 +152,8 @@ void mix_sigmoid_gate_mul(void*, long, const void*, long, int, long, int, int,
                           hipStream_t);
 void mix_mlstm_scan(float*, float*, float*, float*, const void*, long, int,
                     int, int, int, int, const float*, const float*, float,
-                    float*, float*, const int*, const int*, const int*, int,
-                    int, int, int, int, hipStream_t);
+                    float*, float*, const int*, const int*, const int*, long,
+                    int, int, int, int, int, hipStream_t);
 void mix_mlstm_out(void*, long, int, const float*, const float*, const float*,
                    const void*, long, int, float, long, int, int, int,
                    hipStream_t);
@@ -789,7 +789,7 @@ void mlstm_scan(torch::Tensor o, torch::Tensor em, torch::Tensor proj,
                  (int)v_off, (int)i_off, (int)f_off, i_bias.data_ptr<float>(),
                  f_bias.data_ptr<float>(), (float)cap, mem.data_ptr<float>(),
                  mstate.data_ptr<float>(), state_slots.data_ptr<int>(),
-                 qlocs.data_ptr<int>(), seq_lens.data_ptr<int>(), (int)S,
+                 qlocs.data_ptr<int>(), seq_lens.data_ptr<int>(), T, (int)S,
                  (int)H, (int)dk, (int)dv, act_kind(proj), cur_stream());
 }
 
@@ -1465,7 +1465,7 @@ void decay_scan(torch::Tensor o, torch::Tensor q, torch::Tensor k,
       k.data_ptr<float>(), k.stride(0), v.data_ptr<float>(), v.stride(0),
       decay.data_ptr<float>(), lda, gp, sp, state.data_ptr<float>(),
       state_slots.data_ptr<int>(), qlocs.data_ptr<int>(),
-      seq_lens.data_ptr<int>(), (int)S, (int)H, (int)G, (int)dk, (int)dv,
+      seq_lens.data_ptr<int>(), T, (int)S, (int)H, (int)G, (int)dk, (int)dv,
       cur_stream());
   TORCH_CHECK(ok, "decay_scan: key size above 256 is unsupported");
 }

@@ -19,7 +19,9 @@
 // interact, so a column is owned by R adjacent lanes holding RPT rows each in
 // registers; one token costs one R-lane sum (DPP moves) and broadcast reads
 // of the staged k and q rows. Blocks cover (sequence, head, group of columns).
-#include "mix_common.h"
+#include <climits>
+
+#include "mix_chunk.h"
 
 template <typename A>
 __global__ void __launch_bounds__(256) ssd_prep_kernel(
@@ -295,7 +297,8 @@ extern "C" void mix_rotary_sections(float* out, const void* proj, long ld,
 // global loads of tile s+1 are issued before the arithmetic of tile s and
 // parked in registers. With this row mapping the R lanes of a column read
 // consecutive float4s of a staged row, and all columns read the same
-// addresses (LDS broadcast).
+// addresses (LDS broadcast). Sequences of `below` or more new tokens are left to the
+// chunks.
 template <int R, int RPT>
 __global__ void __launch_bounds__(256) decay_scan_kernel(
     float* __restrict__ o, const float* __restrict__ q, long ldq,
@@ -304,7 +307,7 @@ __global__ void __launch_bounds__(256) decay_scan_kernel(
     const float* __restrict__ gain, const float* __restrict__ skip,
     float* __restrict__ state, const int* __restrict__ state_slots,
     const int* __restrict__ qlocs, const int* __restrict__ seq_lens, int H,
-    int G, int dk, int dv, int col_groups) {
+    int G, int dk, int dv, int col_groups, int below) {
   constexpr int DKP = R * RPT;
   constexpr int CPB = 256 / R;             // columns per block
   constexpr int NK = 2 * DTB * DKP / 256;  // staged k|q floats per lane
@@ -318,7 +321,7 @@ __global__ void __launch_bounds__(256) decay_scan_kernel(
   const int h = b % H;
   const int s = b / H;
   const int q0 = qlocs[s], n = qlocs[s + 1] - q0;
-  if (n <= 0) return;
+  if (n <= 0 || n >= below) return;
   const int start = seq_lens[s] - n;
   const int g = h / (H / G);
   const int tid = threadIdx.x;
@@ -428,16 +431,30 @@ extern "C" int mix_decay_scan(float* o, const float* q, long ldq,
                               long ldv, const float* decay, long lda,
                               const float* gain, const float* skip,
                               float* state, const int* state_slots,
-                              const int* qlocs, const int* seq_lens, int S,
-                              int H, int G, int dk, int dv, hipStream_t s) {
+                              const int* qlocs, const int* seq_lens, long T,
+                              int S, int H, int G, int dk, int dv,
+                              hipStream_t s) {
   if (S == 0) return 1;
+  const int least =
+      chunk_scan_least(dk, ldq, ldk, ldv, (long)H * dv, q, k, 16, false, T, S);
+  if (least) {
+    ChunkArgs a = {};
+    a.o = o; a.q = q; a.k = k; a.v = v;
+    a.ldq = ldq; a.ldk = ldk; a.ldv = ldv;
+    a.a = decay; a.lda = lda; a.b = gain; a.skip = skip;
+    a.state = state; a.state_slots = state_slots;
+    a.qlocs = qlocs; a.seq_lens = seq_lens;
+    a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.ov = dv;
+    chunk_scan_launch<false>(a, S, least, s);
+  }
+  const int below = least ? least : INT_MAX;
 #define LAUNCH_DS(RR, PP)                                                    \
   do {                                                                       \
     const int cgs = (dv + 256 / RR - 1) / (256 / RR);                        \
     hipLaunchKernelGGL((decay_scan_kernel<RR, PP>), dim3(S * H * cgs),       \
                        dim3(256), 0, s, o, q, ldq, k, ldk, v, ldv, decay,    \
                        lda, gain, skip, state, state_slots, qlocs, seq_lens, \
-                       H, G, dk, dv, cgs);                                   \
+                       H, G, dk, dv, cgs, below);                            \
   } while (0)
   if (dk <= 16) LAUNCH_DS(4, 4);
   else if (dk <= 32) LAUNCH_DS(4, 8);

@@ -21,7 +21,9 @@
 // columns); a fifth wave of the first group's block carries the normaliser. A sequence whose first token (position 0) is in the batch starts
 // from zero, whatever its slot held. Everything is fp32 except the
 // projection sections, which arrive in the activation type.
-#include "mix_common.h"
+#include <climits>
+
+#include "mix_chunk.h"
 
 #define MTB 8   // tokens staged per step
 
@@ -84,7 +86,8 @@ __global__ void __launch_bounds__(320) mlstm_scan_kernel(
     int k_off, int v_off, const float* __restrict__ fa,
     const float* __restrict__ ib, float* __restrict__ mem,
     const int* __restrict__ state_slots, const int* __restrict__ qlocs,
-    const int* __restrict__ seq_lens, int H, int dk, int dv, int col_groups) {
+    const int* __restrict__ seq_lens, int H, int dk, int dv, int col_groups,
+    int below) {
   constexpr int DKP = R * RPT;
   constexpr int CPB = 256 / R;             // value columns per block
   constexpr int NK = 2 * MTB * DKP / 256;  // staged k|q floats per lane
@@ -109,7 +112,7 @@ __global__ void __launch_bounds__(320) mlstm_scan_kernel(
   const int col = extra ? dv : cg * CPB + cl;
   const bool cv = extra ? (cg == 0 && tid - 256 < R) : col < dv;
   const int q0 = qlocs[s], q1 = qlocs[s + 1];
-  if (q1 <= q0) return;
+  if (q1 <= q0 || q1 - q0 >= below) return;
   const int start = seq_lens[s] - (q1 - q0);
   float* Cg = mem + (((long)state_slots[s] * H + h) * dk) * dv1;
   const float qscale = 1.f / sqrtf((float)dk);
@@ -241,8 +244,8 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
                                const float* i_bias, const float* f_bias,
                                float cap, float* mem, float* mstate,
                                const int* state_slots, const int* qlocs,
-                               const int* seq_lens, int S, int H, int dk,
-                               int dv, int f32, hipStream_t s) {
+                               const int* seq_lens, long T, int S, int H,
+                               int dk, int dv, int f32, hipStream_t s) {
   if (S == 0) return;
   {
     const int waves = S * H;
@@ -258,6 +261,22 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
                          f_bias, cap, mstate, state_slots, qlocs, seq_lens, S,
                          H);
   }
+  const u16* p = (const u16*)proj;
+  const int least =
+      f32 ? 0 : chunk_scan_least(dk, ld, ld, ld, (long)H * (dv + 1), p + q_off,
+                                 p + k_off, 8, true, T, S);
+  if (least) {
+    ChunkArgs a = {};
+    a.o = o; a.q = p + q_off; a.k = p + k_off; a.v = p + v_off;
+    a.ldq = a.ldk = a.ldv = ld;
+    a.a = fa; a.lda = H; a.b = ib;
+    a.state = mem; a.state_slots = state_slots;
+    a.qlocs = qlocs; a.seq_lens = seq_lens;
+    a.H = H; a.G = H; a.dk = dk; a.dv = dv; a.ov = dv + 1;
+    a.qscale = 1.f / sqrtf((float)dk);
+    chunk_scan_launch<true>(a, S, least, s);
+  }
+  const int below = least ? least : INT_MAX;
   int R = 1;
   while (R * 32 < dk) R <<= 1;  // dk <= 256 -> R <= 8 at 32 rows a lane
   int rpt = 32;
@@ -277,7 +296,7 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
   hipLaunchKernelGGL((mlstm_scan_kernel<AA, RR, PP>), dim3((unsigned)grid),   \
                      dim3(320), 0, s, o, (const AA*)proj, ld, q_off, k_off,   \
                      v_off, fa, ib, mem, state_slots, qlocs, seq_lens, H, dk, \
-                     dv, col_groups)
+                     dv, col_groups, below)
 #define PICK_MS(AA)                                                      \
   if (rpt == 32) {                                                       \
     if (R == 1) LAUNCH_MS(AA, 1, 32);                                    \

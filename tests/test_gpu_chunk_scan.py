@@ -1,0 +1,154 @@
+"""Recurrences with one decay per head in chunks of 32 tokens, beside sequences too
+short for them, against the recurrence in float64: sizes around the chunk, the key and
+value tiles and the last column group, grouped keys, strided rows, old and new states."""
+
+import pytest
+import torch
+
+from sutro_amd.ops import hybrid as hops
+from sutro_amd.ops import torch_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+LENS = [33, 1, 95, 0, 32, 31, 64, 200, 7]
+OLD = [0, 5, 3, 2, 0, 9, 40, 0, 0]       # tokens a sequence had before
+
+
+def _batch():
+    q = torch.tensor([0] + LENS).cumsum(0).int()
+    total = torch.tensor([n + o for n, o in zip(LENS, OLD)], dtype=torch.int32)
+    slots = torch.tensor([4, 9, 0, 7, 2, 1, 8, 3, 6], dtype=torch.int32)
+    return q, total, slots
+
+
+def _recur(q, k, v, a, b, skip, state, qlocs, total, slots):
+    """In float64: [T, G, dk], [T, H, dv], [T, H] -> o, states by slot."""
+    rep = v.shape[1] // k.shape[1]
+    q, k = (x.double().repeat_interleave(rep, 1) for x in (q, k))
+    v, a, b, state = v.double(), a.double(), b.double(), state.double().clone()
+    o = torch.zeros(v.shape, dtype=torch.float64)
+    for s in range(len(total)):
+        lo, hi = int(qlocs[s]), int(qlocs[s + 1])
+        if lo == hi:
+            continue
+        S = state[slots[s]] * (1.0 if int(total[s]) > hi - lo else 0.0)
+        for t in range(lo, hi):
+            S = (S * a[t][:, None, None]
+                 + k[t][:, :, None] * (b[t][:, None] * v[t])[:, None, :])
+            o[t] = (S * q[t][:, :, None]).sum(1) + skip.double()[:, None] * v[t]
+        state[slots[s]] = S
+    return o, state
+
+
+def _off(got, want):
+    return float((got.double().cpu() - want).norm() / want.norm())
+
+
+# fp32 sums of up to dk + 32 products, a few roundings each: below 32 units of 2^-24
+TOL = 32 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("H,G,dk,dv,kind", [
+    (2, 2, 128, 128, "constant"), (4, 2, 128, 130, "token"),
+    (2, 1, 100, 20, "token"), (3, 3, 64, 256, "constant"), (2, 2, 36, 72, "token"),
+    (2, 2, 8, 300, "constant"), (2, 2, 128, 16, "zero")])
+def test_decay_chunks(H, G, dk, dv, kind):
+    g = torch.Generator().manual_seed(dk + dv)
+    qlocs, total, slots = _batch()
+    T = int(qlocs[-1])
+    # rows of one buffer, as the mixers hand them over
+    buf = torch.randn(T, 2 * G * dk + H * dv + 4, generator=g)
+    q = buf[:, :G * dk].view(T, G, dk)
+    k = buf[:, G * dk:2 * G * dk].view(T, G, dk)
+    v = buf[:, 2 * G * dk:2 * G * dk + H * dv].view(T, H, dv)
+    state = torch.randn(11, H, dk, dv, generator=g)
+    if kind == "constant":
+        a = 1.0 - 2.0 ** torch.linspace(-2.0, -9.0, H)
+        gain = skip = None
+    else:
+        a = torch.rand(T, H, generator=g)
+        if kind == "zero":              # decays that forget everything, and growth
+            a[::5] = 0.0
+            a[3::7] = 1.25
+        gain, skip = torch.rand(T, H, generator=g), torch.randn(H, generator=g)
+    want, end = _recur(
+        q, k, v, a.expand(T, H) if a.dim() == 1 else a,
+        torch.ones(T, H) if gain is None else gain,
+        torch.zeros(H) if skip is None else skip, state, qlocs, total, slots)
+    d = buf.to(DEV)
+    st = state.to(DEV)
+    o = hops.decay_scan(
+        d[:, :G * dk].unflatten(1, (G, dk)),
+        d[:, G * dk:2 * G * dk].unflatten(1, (G, dk)),
+        d[:, 2 * G * dk:2 * G * dk + H * dv].unflatten(1, (H, dv)), a.to(DEV),
+        None if gain is None else gain.to(DEV),
+        None if skip is None else skip.to(DEV), st, slots.to(DEV),
+        qlocs.to(DEV), total.to(DEV))
+    assert _off(o, want) < TOL
+    assert _off(st, end) < TOL
+    for s in (5, 10):                   # slots of no sequence, and of an empty one
+        assert torch.equal(st[s].cpu(), state[s])
+    assert torch.equal(st[7].cpu(), state[7])
+
+
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 128), (3, 64, 40), (1, 12, 144),
+                                     (2, 100, 143)])
+def test_mlstm_chunks(H, dk, dv):
+    g = torch.Generator().manual_seed(dk + dv)
+    qlocs, total, slots = _batch()
+    T = int(qlocs[-1])
+    cols = 2 * H * dk + H * dv
+    cols += -cols % 4
+    proj = torch.randn(T, cols + 2 * H + 8, generator=g)
+    proj = proj[:, :(cols + 2 * H + 3) // 4 * 4].contiguous().bfloat16()
+    offs = (0, H * dk, 2 * H * dk, cols, cols + H)
+    ib, fb = torch.randn(H, generator=g), torch.randn(H, generator=g) + 2
+    mem = torch.randn(11, H, dk, dv + 1, generator=g)
+    m0 = torch.randn(11, H, generator=g)
+    args = (H, dk, dv, ib, fb, 5.0)
+    want_m, want_ms = mem.clone(), m0.clone()
+    want, em = ref.mlstm_scan(proj, *offs, *args, want_m, want_ms, slots, qlocs,
+                              total)
+    md, ms = mem.to(DEV), m0.to(DEV)
+    o, got_em = hops.mlstm_scan(proj.to(DEV), *offs, H, dk, dv, ib.to(DEV),
+                                fb.to(DEV), 5.0, md, ms, slots.to(DEV),
+                                qlocs.to(DEV), total.to(DEV))
+    # the reference is fp32 as well: its roundings and its gates' beside the kernel's
+    assert _off(o, want.double()) < 4 * TOL
+    assert _off(md, want_m.double()) < 4 * TOL
+    assert _off(got_em, em.double()) < 4 * TOL
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
+@pytest.mark.parametrize("which", ["q", "k", "v", "decay", "state"])
+def test_numbers_that_are_not_finite(bad, which):
+    """They reach what the recurrence lets them reach: no earlier token, no other
+    sequence, and in a value no other column."""
+    g = torch.Generator().manual_seed(3)
+    H, dk, dv = 2, 64, 48
+    lens, old = [70, 40], [4, 4]
+    qlocs = torch.tensor([0, 70, 110], dtype=torch.int32)
+    total = torch.tensor([74, 44], dtype=torch.int32)
+    slots = torch.tensor([1, 0], dtype=torch.int32)
+    T = 110
+    q, k = (torch.randn(T, H, dk, generator=g) for _ in "qk")
+    v = torch.randn(T, H, dv, generator=g)
+    a = torch.rand(T, H, generator=g) * 0.5 + 0.5
+    state = torch.randn(2, H, dk, dv, generator=g)
+    where = {"q": q, "k": k, "v": v}
+    if which == "decay":
+        a[41, 1] = bad
+    elif which == "state":
+        state[1, 0, 5, 7] = bad
+    else:
+        where[which][41, 1, 9] = bad
+    want_s = state.clone()
+    want = ref.decay_scan(q, k, v, a, None, None, want_s, slots, qlocs, total)
+    st = state.to(DEV)
+    got = hops.decay_scan(q.to(DEV), k.to(DEV), v.to(DEV), a.to(DEV), None, None,
+                          st, slots.to(DEV), qlocs.to(DEV), total.to(DEV)).cpu()
+    for x, y in ((got, want), (st.cpu(), want_s)):
+        fine = torch.isfinite(y)
+        assert torch.equal(torch.isfinite(x), fine)
+        torch.testing.assert_close(x[fine], y[fine], rtol=2e-4, atol=2e-4)
