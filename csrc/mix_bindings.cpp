@@ -163,9 +163,13 @@ void mix_delta_prep(float*, float*, float*, float*, float*, const void*, long,
                     int, const float*, const float*, float*, const int*,
                     const int*, const int*, const int*, long, int, int, int,
                     int, int, int, hipStream_t);
+int mix_delta_least(const float*, const float*, const float*, int, long, int,
+                    int, int, int);
+long mix_delta_pairs_floats(long, int, int);
 void mix_delta_scan(float*, const float*, const float*, const float*,
                     const float*, int, const float*, float*, const int*, const int*,
-                    const int*, int, int, int, int, int, hipStream_t);
+                    const int*, float*, int, long, int, int, int, int, int,
+                    hipStream_t);
 void mix_delta_out(void*, long, int, const float*, const float*, const void*,
                    long, int, const float*, int, float, float, long, int, int,
                    int, hipStream_t);
@@ -550,11 +554,19 @@ void delta_scan(torch::Tensor o, torch::Tensor qn, torch::Tensor kn,
                (decay.dim() == 2 && decay.numel() == T * H)) &&
               beta.numel() == T * H && qlocs.numel() == S + 1 &&
               state_slots.numel() == S, "operand sizes");
+  const int head = decay.dim() == 2 ? 1 : 0;
+  const int least = mix_delta_least(qn.data_ptr<float>(), kn.data_ptr<float>(),
+                                    decay.data_ptr<float>(), head, T, (int)S,
+                                    (int)H, (int)dk, (int)dv);
+  torch::Tensor pairs;
+  if (least)
+    pairs = torch::empty({mix_delta_pairs_floats(T, (int)S, (int)H)}, o.options());
   mix_delta_scan(o.data_ptr<float>(), qn.data_ptr<float>(),
                  kn.data_ptr<float>(), v.data_ptr<float>(),
-                 decay.data_ptr<float>(), decay.dim() == 2 ? 1 : 0,
-                 beta.data_ptr<float>(), ssm.data_ptr<float>(), state_slots.data_ptr<int>(),
-                 qlocs.data_ptr<int>(), seq_lens.data_ptr<int>(), (int)S,
+                 decay.data_ptr<float>(), head, beta.data_ptr<float>(),
+                 ssm.data_ptr<float>(), state_slots.data_ptr<int>(),
+                 qlocs.data_ptr<int>(), seq_lens.data_ptr<int>(),
+                 least ? pairs.data_ptr<float>() : nullptr, least, T, (int)S,
                  (int)H, (int)G, (int)dk, (int)dv, cur_stream());
 }
 

@@ -15,7 +15,8 @@
 // sequence in which any read-out or state is not finite is done once more, token
 // by token (chunk_serial), from the state that is still in memory.
 //
-// A wave owns 16 columns of S in registers, laid out as the products leave them (row dk = 16 m + 4 (lane / 16) + r of tile m, column lane % 16).
+// A wave owns 16 columns of S in registers, laid out as the products leave them (row
+// dk = 16 m + 4 (lane / 16) + r of tile m, column lane % 16).
 // The contraction over dk is permuted alike in q, k (in LDS, 32 at a time:
 // place 8 g + 4 hi + r holds 16 hi + 4 g + r) and S, and the one over tokens in v,
 // so neither S nor v passes through LDS; k^T comes from the rows of k through the
@@ -113,6 +114,23 @@ struct ChSum {
         if (i < NA && o - i < NB) c[o] = ch_mfma(a[i], b[o - i], c[o]);
   }
   __device__ __forceinline__ f32x4 total() const { return c[0] + (c[1] + c[2]); }
+};
+
+// the same with the two small orders in one sum
+struct ChSum2 {
+  f32x4 c[2];
+  __device__ __forceinline__ ChSum2() { c[0] = c[1] = (f32x4)(0.f); }
+  template <int NA, int NB>
+  __device__ __forceinline__ void mul(const s16x8 (&a)[NA],
+                                      const s16x8 (&b)[NB]) {
+#pragma unroll
+    for (int o = 2; o >= 0; --o)
+#pragma unroll
+      for (int i = 0; i <= o; ++i)
+        if (i < NA && o - i < NB)
+          c[o > 0] = ch_mfma(a[i], b[o - i], c[o > 0]);
+  }
+  __device__ __forceinline__ f32x4 total() const { return c[0] + c[1]; }
 };
 
 // lane n of a row of 16 <- lane n - N (shr) or n + N (shl), 1 from outside

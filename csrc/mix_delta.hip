@@ -23,8 +23,11 @@
 // interact, so a column is owned by R adjacent lanes holding dk/R rows each
 // in registers; one token costs two R-lane sums (DPP moves) and broadcast
 // reads of the staged k, q and decay rows. Blocks cover (sequence, head,
-// group of columns).
-#include "mix_common.h"
+// group of columns). Longer pieces of prompts go through chunks instead
+// (mix_delta_chunk.h).
+#include <climits>
+
+#include "mix_delta_chunk.h"
 
 #define WPB 4
 #define PT 8   // tokens per wave in delta_prep
@@ -461,6 +464,7 @@ __global__ void conv_state_update_kernel(
 // this row mapping the R lanes of a column read consecutive float4s of a
 // staged row, and all columns read the same addresses (LDS broadcast).
 // HEAD: decay [T, H], one number a token and head (staged beside beta).
+// Sequences of `below` or more new tokens are left to the chunks.
 template <int R, int RPT, bool HEAD>
 __global__ void __launch_bounds__(256) delta_scan_kernel(
     float* __restrict__ o, const float* __restrict__ qn,
@@ -468,7 +472,7 @@ __global__ void __launch_bounds__(256) delta_scan_kernel(
     const float* __restrict__ decay, const float* __restrict__ beta,
     float* __restrict__ ssm, const int* __restrict__ state_slots,
     const int* __restrict__ qlocs, const int* __restrict__ seq_lens, int H,
-    int G, int dk, int dv, int col_groups) {
+    int G, int dk, int dv, int col_groups, int below) {
   constexpr int DKP = R * RPT;
   constexpr int CPB = 256 / R;            // columns per block
   constexpr int KQD = HEAD ? 2 : 3;       // rows of DKP floats a token
@@ -489,7 +493,7 @@ __global__ void __launch_bounds__(256) delta_scan_kernel(
   const bool cv = col < dv;
   const int g = h / (H / G);
   const int q0 = qlocs[s], q1 = qlocs[s + 1];
-  if (q1 <= q0) return;
+  if (q1 <= q0 || q1 - q0 >= below) return;
   const int start = seq_lens[s] - (q1 - q0);
   float* Sg = ssm + (((long)state_slots[s] * H + h) * dk) * dv;
 
@@ -907,12 +911,40 @@ extern "C" void mix_delta_prep(
   }
 }
 
+// New tokens from which a sequence goes through chunks (mix_delta_chunk.h), 0 if none
+// of the batch can be that long or rows are not in whole 16-byte pieces
+extern "C" int mix_delta_least(const float* qn, const float* kn,
+                               const float* decay, int head_decay, long T, int S,
+                               int H, int dk, int dv) {
+  return delta_chunks_least(qn, kn, decay, head_decay, T, S, H, dk, dv);
+}
+extern "C" long mix_delta_pairs_floats(long T, int S, int H) {
+  return (T / CH_T + S) * H * (long)DC_PAIRS;
+}
+
+// pairs: mix_delta_pairs_floats(T, S, H) floats of scratch if least is not 0
 extern "C" void mix_delta_scan(float* o, const float* qn, const float* kn,
                                const float* vv, const float* decay,
                                int head_decay, const float* beta, float* ssm,
                                const int* state_slots, const int* qlocs,
-                               const int* seq_lens, int S, int H, int G, int dk,
-                               int dv, hipStream_t s) {
+                               const int* seq_lens, float* pairs, int least,
+                               long T, int S, int H, int G, int dk, int dv,
+                               hipStream_t s) {
+  if (least) {
+    DeltaChunkArgs a = {};
+    a.o = o; a.q = qn; a.k = kn; a.v = vv; a.d = decay; a.beta = beta;
+    a.state = ssm; a.state_slots = state_slots;
+    a.qlocs = qlocs; a.seq_lens = seq_lens; a.pairs = pairs;
+    a.S = S; a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.least = least;
+    if (head_decay) {
+      if (dk <= 64) delta_chunks_launch<64, true>(a, T, s);
+      else delta_chunks_launch<128, true>(a, T, s);
+    } else {
+      if (dk <= 64) delta_chunks_launch<64, false>(a, T, s);
+      else delta_chunks_launch<128, false>(a, T, s);
+    }
+  }
+  const int below = least ? least : INT_MAX;
   int R = 1;
   while (R * 32 < dk) R <<= 1;  // dk <= 256 -> R <= 8 at 32 rows a lane
   int rpt = 32;
@@ -932,7 +964,8 @@ extern "C" void mix_delta_scan(float* o, const float* qn, const float* kn,
 #define LAUNCH_SCAN_D(RR, PP, HD)                                            \
   hipLaunchKernelGGL((delta_scan_kernel<RR, PP, HD>), dim3((unsigned)grid),  \
                      dim3(256), 0, s, o, qn, kn, vv, decay, beta, ssm,       \
-                     state_slots, qlocs, seq_lens, H, G, dk, dv, col_groups)
+                     state_slots, qlocs, seq_lens, H, G, dk, dv, col_groups, \
+                     below)
 #define LAUNCH_SCAN(RR, PP)                                                  \
   do {                                                                       \
     if (head_decay) LAUNCH_SCAN_D(RR, PP, true);                             \

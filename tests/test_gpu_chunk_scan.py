@@ -1,5 +1,5 @@
-"""Recurrences with one decay per head in chunks of 32 tokens, beside sequences too
-short for them, against the recurrence in float64: sizes around the chunk, the key and
+"""Recurrences with one decay per head, and the gated delta rule, in chunks of 32
+tokens, beside sequences too short for them, against the recurrence in float64: sizes around the chunk, the key and
 value tiles and the last column group, grouped keys, strided rows, old and new states."""
 
 import pytest
@@ -118,6 +118,100 @@ def test_mlstm_chunks(H, dk, dv):
     assert _off(o, want.double()) < 4 * TOL
     assert _off(md, want_m.double()) < 4 * TOL
     assert _off(got_em, em.double()) < 4 * TOL
+
+
+def _delta(q, k, v, d, beta, state, qlocs, total, slots):
+    """The gated delta rule in float64; d [T, H, dk]."""
+    rep = v.shape[1] // k.shape[1]
+    q, k = (x.double().repeat_interleave(rep, 1) for x in (q, k))
+    v, d, beta = v.double(), d.double(), beta.double()
+    state = state.double().clone()
+    o = torch.zeros(v.shape, dtype=torch.float64)
+    for s in range(len(total)):
+        lo, hi = int(qlocs[s]), int(qlocs[s + 1])
+        if lo == hi:
+            continue
+        S = state[slots[s]] * (1.0 if int(total[s]) > hi - lo else 0.0)
+        for t in range(lo, hi):
+            S = S * d[t][:, :, None]
+            u = beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1))
+            S = S + k[t][:, :, None] * u[:, None, :]
+            o[t] = (S * q[t][:, :, None]).sum(1)
+        state[slots[s]] = S
+    return o, state
+
+
+@pytest.mark.parametrize("H,G,dk,dv,kind", [
+    (2, 2, 128, 128, "channel"), (4, 2, 128, 130, "head"), (2, 1, 100, 20, "channel"),
+    (3, 3, 64, 72, "head"), (2, 2, 36, 144, "channel"), (2, 2, 8, 16, "head"),
+    (2, 2, 128, 48, "zero"), (2, 2, 128, 128, "one"), (17, 17, 64, 128, "channel")])
+def test_delta_chunks(H, G, dk, dv, kind):
+    g = torch.Generator().manual_seed(dk + dv + H)
+    lens = [65, 1, 95, 0, 64, 63, 96, 200, 7]
+    if H == 17:                         # more heads and sequences than CUs
+        lens = [64 + i for i in range(9)]
+    qlocs = torch.tensor([0] + lens).cumsum(0).int()
+    total = torch.tensor([n + o for n, o in zip(lens, OLD)], dtype=torch.int32)
+    _, _, slots = _batch()
+    T = int(qlocs[-1])
+    unit = torch.nn.functional.normalize
+    q = unit(torch.randn(T, G, dk, generator=g), dim=-1) * dk ** -0.5
+    k = unit(torch.randn(T, G, dk, generator=g) + 0.2, dim=-1)
+    v = torch.randn(T, H, dv, generator=g)
+    shape = (T, H) if kind == "head" else (T, H, dk)
+    d = torch.exp(-0.5 * torch.nn.functional.softplus(
+        torch.randn(shape, generator=g) * 2))
+    if kind == "zero":                  # memory that ends, and strong decays
+        d[::5] = 0.0
+        d[3::7, :, ::2] = 1e-30
+    if kind == "one":                   # no decay at all
+        d[:] = 1.0
+    beta = torch.sigmoid(torch.randn(T, H, generator=g))
+    state = torch.randn(11, H, dk, dv, generator=g)
+    want, end = _delta(q, k, v, d[..., None].expand(T, H, dk) if kind == "head" else d,
+                       beta, state, qlocs, total, slots)
+    st = state.to(DEV)
+    o = hops.delta_scan(*(x.to(DEV) for x in (q, k, v, d, beta)), st, slots.to(DEV),
+                        qlocs.to(DEV), total.to(DEV))
+    assert _off(o, want) < TOL
+    assert _off(st, end) < TOL
+    for s in (5, 10) + ((7,) if H != 17 else ()):
+        assert torch.equal(st[s].cpu(), state[s])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
+@pytest.mark.parametrize("which", ["q", "k", "v", "d", "beta", "state"])
+def test_delta_numbers_that_are_not_finite(bad, which):
+    g = torch.Generator().manual_seed(5)
+    H, dk, dv, T = 2, 64, 48, 170
+    qlocs = torch.tensor([0, 90, 170], dtype=torch.int32)
+    total = torch.tensor([94, 84], dtype=torch.int32)
+    slots = torch.tensor([1, 0], dtype=torch.int32)
+    x = {"q": torch.randn(T, H, dk, generator=g) * dk ** -0.5,
+         "k": torch.nn.functional.normalize(torch.randn(T, H, dk, generator=g), dim=-1),
+         "v": torch.randn(T, H, dv, generator=g),
+         "d": torch.rand(T, H, dk, generator=g) * 0.5 + 0.5,
+         "beta": torch.rand(T, H, generator=g)}
+    state = torch.randn(2, H, dk, dv, generator=g)
+    if which == "state":
+        state[1, 0, 5, 7] = bad
+    elif which == "beta":
+        x["beta"][41, 1] = bad
+    else:
+        x[which][41, 1, 9] = bad
+    want_s = state.clone()
+    want = ref.delta_scan(*x.values(), want_s, slots, qlocs, total)
+    st = state.to(DEV)
+    got = hops.delta_scan(*(y.to(DEV) for y in x.values()), st, slots.to(DEV),
+                          qlocs.to(DEV), total.to(DEV)).cpu()
+    # every other head and sequence is as it was, and so are the tokens before
+    mine = torch.zeros_like(want, dtype=torch.bool)
+    head = 0 if which == "state" else 1
+    mine[0 if which == "state" else 41:90, head] = True
+    torch.testing.assert_close(got[~mine], want[~mine], rtol=2e-4, atol=2e-4)
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    fine = torch.isfinite(want_s)
+    assert torch.equal(torch.isfinite(st.cpu()), fine)
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
