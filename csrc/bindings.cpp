@@ -58,6 +58,8 @@ void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
                        int, int, hipStream_t);
 void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
                     hipStream_t);
+void sutro_linear_mid(void*, const void*, long, const void*, const void*, int, int,
+                      int, int, hipStream_t);
 void sutro_linear_skinny(void*, long, const void*, long, const void*,
                          const void*, int, int, int, int, hipStream_t);
 long mix_moe_dispatch_scratch(long, int);
@@ -352,6 +354,35 @@ torch::Tensor linear_skinny(torch::Tensor x, torch::Tensor w,
   return out;
 }
 
+// linear layer over 2 to 256 rows (csrc/gemm_mid.hip), `gated` with silu_mul
+torch::Tensor linear_mid(torch::Tensor x, torch::Tensor w,
+                         c10::optional<torch::Tensor> bias, bool gated) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device(),
+              "operands on one GPU");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16, "bf16 operands");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.is_contiguous() &&
+              x.stride(1) == 1, "matrix operands, rows contiguous");
+  const long M = x.size(0), K = x.size(1), rows = w.size(0), ld = x.stride(0);
+  const long N = gated ? rows / 2 : rows;
+  TORCH_CHECK(w.size(1) == K && K >= 256 && K % 256 == 0 && N >= 4 && N % 4 == 0 &&
+              (!gated || rows == 2 * N) && M >= 1 && M <= 256 && K < (1l << 20) &&
+              rows < (1l << 24) && ld >= K && M * ld < (1l << 30) &&
+              (N + 128) * K < (gated ? 1l << 30 : 1l << 44), "unsupported sizes");
+  TORCH_CHECK(ld % 8 == 0 && (size_t)x.data_ptr() % 16 == 0 &&
+              (size_t)w.data_ptr() % 16 == 0, "16-byte rows");
+  const void* b = nullptr;
+  if (bias.has_value()) {
+    TORCH_CHECK(!gated && bias->is_cuda() && bias->scalar_type() == at::kBFloat16 &&
+                bias->is_contiguous() && bias->numel() == rows, "bias");
+    b = bias->data_ptr();
+  }
+  auto out = torch::empty({M, N}, x.options());
+  sutro_linear_mid(out.data_ptr(), x.data_ptr(), ld, w.data_ptr(), b, (int)M, (int)N,
+                   (int)K, gated ? 1 : 0, cur_stream());
+  return out;
+}
+
 // (y w^T or, `gated`, its silu unit; x + residual), y the RMSNorm of x + residual,
 // one row
 std::vector<torch::Tensor> norm_linear(torch::Tensor x, torch::Tensor residual,
@@ -440,6 +471,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma16_probe", &mfma16_probe, "16x16 MFMA fragment-layout probe");
   m.def("moe_combine", &moe_combine, "fused MoE weighted gather-combine");
   m.def("linear_skinny", &linear_skinny, "linear layer over few rows");
+  m.def("linear_mid", &linear_mid, "linear layer over 2 to 256 rows");
   m.def("norm_linear", &norm_linear,
         "linear layer of one row behind an addition and RMSNorm");
   m.def("linear_silu_mul", &linear_silu_mul,

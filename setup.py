@@ -25,6 +25,7 @@ SOURCES = [
     "csrc/grouped_gemm.hip",
     "csrc/moe_topk.hip",
     "csrc/gemm_skinny.hip",
+    "csrc/gemm_mid.hip",
     "csrc/moe_dispatch.hip",
 ]
 

@@ -292,13 +292,108 @@ def _few_rows(x, w, gated: bool = False) -> bool:
                      and (x.requires_grad or w.requires_grad)))
 
 
+def _mid_sizes(M: int, rows: int, K: int, gated: bool) -> bool:
+    """The sizes of `_mid_rows` at which csrc/gemm_mid.hip is ahead."""
+    if K <= 4096:
+        if M == 2:
+            if K <= 1024:
+                return rows >= (4096 if gated else 32) and rows <= 65536
+            return 6144 <= rows <= 65536 and (
+                K <= 2048 or (not gated and rows <= 32768))
+        if M <= 12:                       # from 513 to 1024 of k: short chains
+            if K <= 1024:
+                return K > 512 and rows >= 10240
+            if K > 3072 and (rows <= 5120 or (gated and 12288 < rows <= 20480)):
+                return False
+            return rows >= 4096
+        if M <= 16:
+            return rows >= (10240 if K <= 512 else 2048 if K <= 1024 else 32)
+        if rows < 512 and K > 2048:
+            return False
+        if M <= 64:
+            return rows <= 36864 or K % 2048 == 0
+        if M <= 128:
+            return rows <= 16384 or (M >= 96 and 28672 <= rows <= 32768
+                                     and K % 2048 == 0)
+        if M <= 192:
+            return rows <= 10240 or (gated and 15360 <= rows <= 16384
+                                     and K <= 2048)
+        return rows <= 8192 or (gated and 12800 <= rows <= 16384)
+    if K <= 5120:
+        if M <= 16:
+            return M > 3 and (
+                ((512 if M <= 8 else 4096) <= rows <= 6144 and not gated)
+                or 16384 <= rows <= 40960)
+        if M <= 64:
+            return 512 <= rows <= 8192 or 16384 <= rows <= 32768
+        return 2048 <= rows <= (10240 if 128 < M <= 192 else 8192)
+    if K <= 6144:
+        return 16 < M <= 128 and 4096 <= rows <= 8192
+    if K >= 16384 and M > 32:
+        return 2048 <= rows <= 6144
+    return 64 < M <= 192 and (
+        4096 if gated or K > 8192 else 2048) <= rows <= 6144 and not (
+        gated and K > 8192)
+
+
+def _mid_rows(x, w, gated: bool = False) -> bool:
+    """Whether x [M, K] w^T goes to csrc/gemm_mid.hip, 2 to 256 rows. Against what
+    it went to before (the library, or csrc/gemm_skinny.hip up to 32 rows; gated:
+    and silu_mul behind it), in a graph, weights from memory, it takes this part
+    of the time (the figures in us stand beside the kernel):
+      rows of w x K     M = 2     4     8    16    32    64   128   192   256
+      2048 x 1024       0.85  1.07  1.05  0.97  0.86  0.57  0.60  0.64  0.63
+      16384 x 1024      0.82  0.89  0.84  0.77  0.61  0.69  0.77  1.09  1.06
+      51200 x 1024      0.96  0.95  0.95  0.95  0.97  1.03  1.28  2.0   1.9
+      2048 x 2048       1.03  1.02  0.98  0.90  0.73  0.71  0.74  0.81  0.77
+      6144 x 2048       0.80  0.89  0.89  0.80  0.58  0.80  0.79  0.75  0.67
+      16384 x 2048 g    0.77  0.85  0.82  0.67  0.69  0.71  0.75  0.92  0.85
+      32768 x 2048      0.87  0.87  0.82  0.81  0.78  0.80  0.89  1.43  1.35
+      4096 x 4096       1.00  1.10  1.02  0.89  0.80  0.85  0.64  0.63  0.91
+      6144 x 4096       0.90  0.83  0.81  0.81  0.85  0.93  0.88  0.91  0.71
+      16384 x 4096 g    1.07  1.12  1.05  0.92  0.93  0.95  0.92  1.01  0.88
+      24576 x 4096 g    0.95  0.94  0.89  0.80  0.76  0.80  1.03  1.41  1.34
+      2048 x 5120       1.23  0.66  0.67  1.23  0.96  0.85  0.91  0.84  0.86
+      10240 x 5120      1.07  1.06  1.05  1.05  1.03  0.96  1.01  0.84  1.00
+      4096 x 8192       1.05  1.05  1.07  1.09  0.99  0.88  0.64  0.60  1.03
+      4096 x 12288      1.26  1.25  1.32  1.28  1.10  0.95  0.65  0.65  1.08
+      4096 x 25600      1.25  1.23  1.13  0.98  0.74  0.44  0.64  0.77  0.66
+    It loses where few weights are long rows (one workgroup has all of k), where
+    128 x 128 tiles of many rows leave more than one round, and to the kernel for
+    few rows where that one is quickest."""
+    if (type(x) is not torch.Tensor or _tracing()
+            or type(w) not in (torch.Tensor, torch.nn.Parameter)):
+        return False
+    if x.dim() != 2 or not 2 <= x.shape[0] <= 256 or not _use_hip(x):
+        return False
+    M, K = x.shape
+    rows = w.shape[0]
+    return (K % 256 == 0 and K >= 512 and _mid_sizes(M, rows, K, gated)
+            and _unwatched() and x.dtype == torch.bfloat16
+            and w.dtype == torch.bfloat16 and w.device == x.device
+            and w.dim() == 2 and w.shape[1] == K
+            and rows % (16 if gated else 4) == 0 and rows < 1 << 24
+            and (not gated or (rows // 2 + 128) * K < 1 << 30)
+            and w.is_contiguous() and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 22
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
+def _plain_bias(bias, x, w) -> bool:
+    return bias is None or (
+        bias.dtype == torch.bfloat16 and bias.device == x.device
+        and bias.shape == w.shape[:1] and bias.is_contiguous()
+        and not (torch.is_grad_enabled() and bias.requires_grad))
+
+
 def linear(x, w, bias=None):
-    """x w^T (+ bias): the library's product, or over few rows (decode steps)
-    csrc/gemm_skinny.hip."""
-    if _few_rows(x, w) and (bias is None or (
-            bias.dtype == torch.bfloat16 and bias.device == x.device
-            and bias.shape == w.shape[:1] and bias.is_contiguous()
-            and not (torch.is_grad_enabled() and bias.requires_grad))):
+    """x w^T (+ bias): the library's product, or over up to 256 rows (decode
+    steps, short prompts) csrc/gemm_mid.hip or csrc/gemm_skinny.hip."""
+    if _mid_rows(x, w) and _plain_bias(bias, x, w):
+        return _require_hip().linear_mid(x, w, bias, False)
+    if _few_rows(x, w) and _plain_bias(bias, x, w):
         return _require_hip().linear_skinny(x, w, bias, False)
     return F.linear(x, w, bias)
 
@@ -353,6 +448,8 @@ def _many_rows(x, w) -> bool:
 
 def linear_silu_mul(x, w):
     """silu_mul(x w^T), w the gate's rows and then the up's."""
+    if _mid_rows(x, w, gated=True):
+        return _require_hip().linear_mid(x, w, None, True)
     if _few_rows(x, w, gated=True):
         return _require_hip().linear_skinny(x, w, None, True)
     if _many_rows(x, w):
