@@ -8,8 +8,8 @@
 // decoded tokens run the same kernel and every cached row is fetched once for
 // 64 query rows. A workgroup of 4 waves owns a tile and walks the visible keys
 // 64 at a time (double-buffered in LDS, 16-byte chunks XOR-swizzled by row; the
-// next tile's pages travel through registers, one during the scores, one during
-// the values):
+// next tile's pages are copied straight there meanwhile, their places in the block
+// table looked up a step before):
 //   scores   wave (a, b) makes the 32 x 32 block of row half a and key half b,
 //            S^T = mfma(A = K, B = Q^T), Q in registers; soft-max statistics
 //            meet in LDS
@@ -25,6 +25,13 @@
 // XCDs work through the same sequence and its pages stay in their L2.
 // When there are too few tiles for the chip the keys are also cut into
 // `nsplit` runs whose partial results a second kernel joins.
+//
+// Times: 16 prompts of 1024 tokens, 32 heads of 576 and 512, 1343 -> 990 us; 61 prompts
+// of 490, 16 heads of 256 and 256, window 1024, 441 -> 246 (590 and 480 TFLOP/s). Pages
+// through registers waited for two memory latencies (table, page) twice a step; 64 rows
+// of queries read and of results written in pieces of 8 to 32 bytes were 17 K cycles a
+// tile. A step now takes 5.6 K cycles (products 2.2 K, the softmax between them 1.5 K,
+// one wave a SIMD), a tile's begin and end 15 K.
 //
 // Fragment layouts (gfx950 v_mfma_f32_32x32x16_bf16): lane l holds
 //   A[l%32][(l/32)*8 + j], B[(l/32)*8 + j][l%32], j = 0..7;
@@ -59,7 +66,7 @@ __device__ __forceinline__ f32x16 mfma32l(bfrag a, bfrag b, f32x16 c) {
 // addresses and reaches the rest by constant offsets.
 
 struct LatentArgs {
-  u16* out;             // rows [t][out_off + h * dv ..]
+  u16* out;             // rows [t][out_off + h * dv ..], multiples of 16 bytes
   long ldo;
   int out_off;
   const u16* q;         // [T, H, dk]
@@ -118,8 +125,7 @@ __device__ __forceinline__ void lt_scale(f32x16& v, int r, float f) {
 }
 
 template <int DK, int DV>
-__global__ void __launch_bounds__(256, 1)
-latent_attention_kernel(LatentArgs A) {
+__device__ __forceinline__ void latent_body(const LatentArgs& A) {
   constexpr int CPR = DK / 8;             // chunks per row
   constexpr int CPT = LT_KEYS * CPR / 256;  // staged chunks per thread
   constexpr int NC = DV / 128;            // 32-column blocks per wave
@@ -178,15 +184,6 @@ latent_attention_kernel(LatentArgs A) {
   float* mx = (float*)(lt_smem + 2 * TILE + LT_ROWS * LT_PP * 2);  // [2][64]
   float* alpha_lds = mx + 2 * LT_ROWS;               // [64]
 
-  bfrag qb[QF];
-  {
-    const u16* qp = A.q + ((long)tok0 * H + row0 + my_row) * dk;
-#pragma unroll
-    for (int kk = 0; kk < QF; ++kk) {
-      const int c = kk * 16 + hi * 8;
-      qb[kk] = c < dk ? *(const s16x8*)(qp + c) : (s16x8)(0);
-    }
-  }
   f32x16 acc[2][NC];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -197,28 +194,32 @@ latent_attention_kernel(LatentArgs A) {
 
   const int* table = A.bt + (long)s * A.bt_stride;
   const int last_page = (kv_end - 1) / LT_PG;
-  // One page at a time: a thread's chunks of either page sit at the same
-  // places of the page. Columns past the row end are fetched from its start:
+  // Pages go straight to LDS, 16 bytes a lane; a thread's chunks of either page sit at
+  // the same places of the page. Columns past the row end are fetched from its start:
   // the query is zero there, so any finite value does.
   constexpr int HC = CPT / 2;
-  u16x8 st[HC];
-  int src[HC];
+  u32 src[HC];
 #pragma unroll
   for (int i = 0; i < HC; ++i) {
     const int L = i * 256 + tid, row = L / CPR, pc = L % CPR;
     int c = ((pc & ~7) | ((pc ^ row) & 7)) * 8;
     if (c >= dk) c = 0;
-    src[i] = row * dk + c;
+    src[i] = (u32)(row * dk + c) * 2;
   }
-  auto load = [&](int page) {
-    const u16* pg = A.cache + (long)table[min(page, last_page)] * LT_PG * dk;
-#pragma unroll
-    for (int i = 0; i < HC; ++i) st[i] = *(const u16x8*)(pg + src[i]);
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  // entries of the block table through the scalar cache (no kernel writes it)
+  auto page = [&](int i) {
+    return ((const __attribute__((address_space(4))) int*)table)[min(i, last_page)];
   };
-  auto store = [&](int buf, int half) {
-    char* dst = lt_smem + buf * TILE + half * (TILE / 2) + tid * 16;
+  auto copy = [&](int buf, int half, int pg) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(A.cache + (long)pg * LT_PG * dk), 0, 0xffffffffu, 0x00027000);
+    char* dst = lt_smem + buf * TILE + half * (TILE / 2) + wu * 1024;
 #pragma unroll
-    for (int i = 0; i < HC; ++i) *(u16x8*)(dst + i * 4096) = st[i];
+    for (int i = 0; i < HC; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          r, (__attribute__((address_space(3))) void*)(dst + i * 4096), 16, src[i],
+          0, 0, 0);
   };
 
   // key fragments: row wk*32 + ln, logical chunks kk*2 + hi
@@ -239,16 +240,53 @@ latent_attention_kernel(LatentArgs A) {
       vad[h][o] = row * (2 * DK) + (c & ~7) * 16 + ((c ^ row) & 7) * 16 +
                   (ti & 1) * 8;
     }
-  load(2 * kt0);
-  store(0, 0);
-  load(2 * kt0 + 1);
-  store(0, 1);
+  copy(0, 0, page(2 * kt0));
+  copy(0, 1, page(2 * kt0 + 1));
+  int pg0 = page(2 * kt0 + 2), pg1 = page(2 * kt0 + 3);
+  // The queries come through the second buffer, laid out like 64 keys (read where the
+  // products want them, a load touched 32 rows of 32 bytes: 8 K cycles a tile), and
+  // through registers: copies straight to LDS do some 28 bytes a cycle.
+  {
+    const u16* qp = A.q + ((long)tok0 * H + row0) * dk;
+    u16x8 v[CPT];
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int L = i * 256 + tid, row = L / CPR, pc = L % CPR;
+      int c = ((pc & ~7) | ((pc ^ row) & 7)) * 8;
+      if (c >= dk) c = 0;
+      v[i] = *(const u16x8*)(qp + min(row, nrow - 1) * dk + c);
+    }
+#pragma unroll
+    for (int i = 0; i < CPT; ++i)
+      *(u16x8*)(lt_smem + TILE + i * 4096 + tid * 16) = v[i];
+  }
   __syncthreads();
+  bfrag qb[QF];
+  {
+    const int row = wr * 32 + ln;
+    int qad[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      qad[j] = TILE + row * (2 * DK) + (((j * 2 + hi) ^ row) & 7) * 16;
+#pragma unroll
+    for (int kk = 0; kk < QF; ++kk) {
+      qb[kk] = *(const s16x8*)(lt_smem + qad[kk & 3] + (kk >> 2) * 128);
+      if (kk * 16 + hi * 8 >= dk) qb[kk] = (s16x8)(0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  // each step's end waits for the next one's pages and sends for those of the step
+  // behind it
+  if (kt0 + 1 < kt1) {
+    copy(1, 0, pg0);
+    copy(1, 1, pg1);
+    pg0 = page(2 * kt0 + 4);
+    pg1 = page(2 * kt0 + 5);
+  }
   int buf = 0;
   for (int kt = kt0; kt < kt1; ++kt, buf ^= 1) {
-    const bool more = kt + 1 < kt1;
     lt_pin<NC>(acc);
-    if (more) load(2 * kt + 2);
     const char* tile = lt_smem + buf * TILE;
     // ---- scores: keys wk*32.., rows wr*32..
     f32x16 d = (f32x16)(0.f), d2 = (f32x16)(0.f);  // two independent chains
@@ -261,11 +299,22 @@ latent_attention_kernel(LatentArgs A) {
     }
     const int kv0 = kt * LT_KEYS + wk * 32;
     float tmax = -1e30f;
+    // (uniform) every row of the tile sees all keys of the step
+    const bool all = kt * LT_KEYS + LT_KEYS - 1 <= pf &&
+                     (A.window <= 0 || kt * LT_KEYS >= kv_end - A.window);
+    if (all) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kp = kv0 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-      d[r] = kp <= my_p && kp >= my_lo ? (d[r] + d2[r]) * A.scale : -1e30f;
-      tmax = fmaxf(tmax, d[r]);
+      for (int r = 0; r < 16; ++r) {
+        d[r] = (d[r] + d2[r]) * A.scale;
+        tmax = fmaxf(tmax, d[r]);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int kp = kv0 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+        d[r] = kp <= my_p && kp >= my_lo ? (d[r] + d2[r]) * A.scale : -1e30f;
+        tmax = fmaxf(tmax, d[r]);
+      }
     }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
     if (hi == 0) mx[wk * LT_ROWS + wr * 32 + ln] = tmax;
@@ -290,10 +339,6 @@ latent_attention_kernel(LatentArgs A) {
     }
     l_run = l_run * al + psum;  // this lane's share of this wave's keys
     if (wk == 0 && hi == 0) alpha_lds[wr * 32 + ln] = al;
-    if (more) {
-      store(buf ^ 1, 0);
-      load(2 * kt + 3);
-    }
     __syncthreads();
     // ---- values: columns w * NC * 32.. of all rows
     const float al0 = alpha_lds[ln], al1 = alpha_lds[32 + ln];
@@ -328,8 +373,14 @@ latent_attention_kernel(LatentArgs A) {
     }
     lt_sched<4 * (2 + 2 * NC), 8 * NC, 4 + 2 * NC>();
     lt_pin<NC>(acc);
-    if (more) store(buf ^ 1, 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if (kt + 2 < kt1) {
+      copy(buf, 0, pg0);
+      copy(buf, 1, pg1);
+      pg0 = page(2 * kt + 6);
+      pg1 = page(2 * kt + 7);
+    }
   }
 
   // ---- epilogue: the row sums meet in LDS
@@ -341,35 +392,62 @@ latent_attention_kernel(LatentArgs A) {
     pml[tid * 2] = alpha_lds[tid];
     pml[tid * 2 + 1] = mx[tid] + mx[LT_ROWS + tid];
   }
+  if (A.nsplit > 1) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const int row = a * 32 + ln;
+      if (row >= nrow) continue;
+      float* pp = A.part_o + ((long)blockIdx.y * A.rows + prow + row) * dv;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int col = (w * NC + c) * 32 + g * 8 + hi * 4;
+          f32x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = acc[a][c][g * 4 + e];
+          if (col < dv) *(f32x4*)(pp + col) = o;
+        }
+    }
+    return;
+  }
+  // Results go through the key buffers, so that lanes write neighbouring places of a
+  // row (8 bytes of 32 rows a store took 9 K cycles a tile).
+  constexpr int OS = DV * 2 + 16;
+  static_assert(LT_ROWS * OS <= 2 * TILE, "results fit the key buffers");
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
     const int row = a * 32 + ln;
-    if (row >= nrow) continue;
     const float l = mx[row] + mx[LT_ROWS + row];
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int rr = row0 + row;
-    u16* op = A.out + (long)(tok0 + rr / H) * A.ldo + A.out_off +
-              (long)(rr % H) * dv;
-    float* pp = A.part_o + ((long)blockIdx.y * A.rows + prow + row) * dv;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int col = (w * NC + c) * 32 + g * 8 + hi * 4;
-        if (col >= dv) continue;
-        if (A.nsplit > 1) {
-          f32x4 o;
+        f32x4 o;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = acc[a][c][g * 4 + e];
-          *(f32x4*)(pp + col) = o;
-        } else {
-          f32x4 o;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = acc[a][c][g * 4 + e] * inv;
-          *(u16x4l*)(op + col) = pack_bf4(o);
-        }
+        for (int e = 0; e < 4; ++e) o[e] = acc[a][c][g * 4 + e] * inv;
+        *(u16x4l*)(lt_smem + row * OS +
+                   ((w * NC + c) * 32 + g * 8 + hi * 4) * 2) = pack_bf4(o);
       }
   }
+  __syncthreads();
+  constexpr int PER = DV / 8;              // 16-byte pieces of a row
+  const int c8 = tid % PER * 8;
+  int row = tid / PER, t = (row0 + row) / H, h = row0 + row - t * H;
+#pragma unroll 4
+  for (; row < nrow; row += 256 / PER) {
+    const u16x8 v = *(const u16x8*)(lt_smem + row * OS + c8 * 2);
+    u16* op = A.out + (long)(tok0 + t) * A.ldo + A.out_off + (long)h * dv + c8;
+    for (h += 256 / PER; h >= H; h -= H) ++t;
+    if (c8 < dv) *(u16x8*)op = v;
+  }
+}
+
+template <int DK, int DV>
+__global__ void __launch_bounds__(256, 1)
+latent_attention_kernel(const LatentArgs A) {
+  latent_body<DK, DV>(A);
 }
 
 // one 128-thread block a (token, head) row: joins the partial results
@@ -440,7 +518,7 @@ extern "C" int mix_latent_attention(
     int nsplit, float* part_o, float* part_ml, hipStream_t s) {
   int DV = 0;
   const int DK = latent_pad(dk, dv, page, &DV);
-  if (!DK) return 0;
+  if (!DK || ldo % 8 || out_off % 8 || (size_t)out % 16) return 0;
   if (T == 0) return 1;
   LatentArgs A;
   A.out = (u16*)out; A.ldo = ldo; A.out_off = out_off;
