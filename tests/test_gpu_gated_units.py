@@ -1,0 +1,83 @@
+"""The gated units of the products on tiles of 256 rows, for sums chosen one by one:
+steep and flat parts, both ends of the exponential, infinities and NaN."""
+
+import math
+
+import pytest
+import torch
+
+from sutro_amd import ops
+from sutro_amd.ops import hybrid as hops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+K, N, M = 64, 128, 256
+GATES = [0.0, -0.0, 1e-30, 1e-3, 0.5, 1.0, 1.5, 3.0, 7.0, 11.0, 20.0, 87.0, 100.0,
+         1e4, 1e30, 3e38, math.inf, math.nan]
+UPS = [0.0, 1.0, -1.0, 0.3, 7.5, -9.0, 1e-20, 1e20]
+
+
+def _operands():
+    """x [M, K], w [2 N, K] whose product has gate GATES (either sign) and up UPS
+    in all pairs: a row of x is one column of w."""
+    g = torch.tensor(GATES + [-v for v in GATES])
+    pairs = torch.cartesian_prod(g, torch.tensor(UPS)).bfloat16()
+    w = torch.zeros(2 * N, K, dtype=torch.bfloat16)
+    n = len(pairs)
+    cols = -(-n // N)
+    for c in range(cols):
+        part = pairs[c * N:(c + 1) * N]
+        w[:len(part), c], w[N:N + len(part), c] = part[:, 0], part[:, 1]
+    x = torch.zeros(M, K, dtype=torch.bfloat16)
+    x[torch.arange(M), torch.arange(M) % cols] = 1
+    return x, w
+
+
+def _want(x, w, unit):
+    y = x.double() @ w.double().T
+    return unit(y[:, :N], y[:, N:])
+
+
+def _check(got, want):
+    """One rounding to bf16 (2^-9), the unit in fp32 far below it; where exp(-gate)
+    is past 2^126 the quotient, under 2^-119 of the up's, may be 0."""
+    got, want = got.double().cpu(), want
+    assert torch.equal(got.isnan(), want.isnan())
+    ok = ~want.isnan()
+    big = want.abs() > 3.4e38                       # past bf16's largest: infinite
+    assert torch.equal(got[ok & big], want[ok & big].sign() * math.inf)
+    ok &= ~big
+    err = (got[ok] - want[ok]).abs()
+    assert (err <= want[ok].abs() * 2 ** -8 + 2.0 ** -119 * 1e20).all()
+
+
+def silu(g, u):
+    return g / (1 + torch.exp(-g)) * u
+
+
+def clamped(g, u, limit=7.0):
+    lim = torch.tensor(limit, dtype=g.dtype)        # (of a NaN the limit)
+    g, u = torch.fmin(g, lim), torch.fmin(torch.fmax(u, -lim), lim)
+    return g / (1 + torch.exp(-1.702 * g)) * (u + 1)
+
+
+def test_one_matrix():
+    x, w = _operands()
+    got = ops._require_hip().linear_silu_mul(x.to(DEV), w.to(DEV))
+    _check(got, _want(x, w, silu))
+
+
+@pytest.mark.parametrize("kind", ["silu", "clamped", "weighted"])
+def test_experts(kind):
+    x, w = _operands()
+    off = torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+    cnt = torch.tensor([M], dtype=torch.int32, device=DEV)
+    tok = torch.arange(M, dtype=torch.int32, device=DEV)
+    out = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+    rw = torch.rand(M, generator=torch.Generator().manual_seed(1)) * 0.5 + 0.25
+    act = hops.ACT_GLU_CLAMPED if kind == "clamped" else hops.ACT_SILU_GATE
+    hops.expert_gemm(out, x.to(DEV), w.to(DEV)[None], tok, off, cnt, act, 256, 7.0,
+                     rw.to(DEV) if kind == "weighted" else None)
+    y = rw[:, None].double() if kind == "weighted" else 1.0
+    unit = clamped if kind == "clamped" else silu
+    _check(out, _want(x, w, lambda g, u: unit(g * y, u * y)))
