@@ -54,6 +54,8 @@ void sutro_norm_linear(void*, const void*, const void*, void*, const void*,
                        float, const void*, int, int, int, hipStream_t);
 void sutro_linear_silu_mul(void*, const void*, const void*, int, int, long,
                            hipStream_t);
+void sutro_linear_gelu_mul(void*, void*, const void*, const void*, const void*, int,
+                           int, int, long, hipStream_t);
 void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
                        int, int, hipStream_t);
 void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
@@ -407,24 +409,51 @@ std::vector<torch::Tensor> norm_linear(torch::Tensor x, torch::Tensor residual,
   return {out, sum};
 }
 
-// silu of x [M, K] times the first N rows of w [2 N, K], times x and the others
-torch::Tensor linear_silu_mul(torch::Tensor x, torch::Tensor w) {
+static void check_gated(const torch::Tensor& x, const torch::Tensor& w, long N) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device(),
               "operands on one GPU");
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 &&
               w.scalar_type() == at::kBFloat16, "bf16 operands");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.is_contiguous() &&
               w.is_contiguous(), "contiguous matrices");
-  const long M = x.size(0), K = x.size(1), N = w.size(0) / 2;
-  TORCH_CHECK(w.size(1) == K && w.size(0) == 2 * N && K > 0 && K % 64 == 0 &&
+  const long M = x.size(0), K = x.size(1);
+  TORCH_CHECK(w.size(1) == K && w.size(0) >= 2 * N && K > 0 && K % 64 == 0 &&
               N > 0 && N % 128 == 0 && M >= 1 && M * K < (1l << 30) &&
-              K < (1l << 21) && N < (1l << 24), "unsupported sizes");
+              K < (1l << 21) && w.size(0) < (1l << 25), "unsupported sizes");
   TORCH_CHECK((size_t)x.data_ptr() % 16 == 0 && (size_t)w.data_ptr() % 16 == 0,
               "16-byte rows");
-  auto out = torch::empty({M, N}, x.options());
-  sutro_linear_silu_mul(out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)M,
-                        (int)N, K, cur_stream());
+}
+
+// silu of x [M, K] times the first N rows of w [2 N, K], times x and the others
+torch::Tensor linear_silu_mul(torch::Tensor x, torch::Tensor w) {
+  const long N = w.size(0) / 2;
+  check_gated(x, w, N);
+  TORCH_CHECK(w.size(0) == 2 * N, "gate and up rows");
+  auto out = torch::empty({x.size(0), N}, x.options());
+  sutro_linear_silu_mul(out.data_ptr(), x.data_ptr(), w.data_ptr(),
+                        (int)x.size(0), (int)N, x.size(1), cur_stream());
   return out;
+}
+
+// GELU by tanh of the first N columns of x w^T + bias times the next N, and the rest
+std::vector<torch::Tensor> linear_gelu_mul(torch::Tensor x, torch::Tensor w,
+                                           c10::optional<torch::Tensor> bias,
+                                           long N) {
+  check_gated(x, w, N);
+  const long more = w.size(0) - 2 * N;
+  TORCH_CHECK(more % 256 == 0, "unsupported sizes");
+  if (bias.has_value())
+    TORCH_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+                bias->dim() == 1 && bias->size(0) == w.size(0) &&
+                bias->device() == x.device() &&
+                (size_t)bias->data_ptr() % 8 == 0, "bias");
+  auto out = torch::empty({x.size(0), N}, x.options());
+  auto rest = torch::empty({x.size(0), more}, x.options());
+  sutro_linear_gelu_mul(out.data_ptr(), rest.data_ptr(), x.data_ptr(),
+                        w.data_ptr(),
+                        bias.has_value() ? bias->data_ptr() : nullptr,
+                        (int)x.size(0), (int)N, (int)more, x.size(1), cur_stream());
+  return {out, rest};
 }
 
 void sampler_fused(torch::Tensor logits, torch::Tensor temps,
@@ -474,6 +503,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_mid", &linear_mid, "linear layer over 2 to 256 rows");
   m.def("norm_linear", &norm_linear,
         "linear layer of one row behind an addition and RMSNorm");
+  m.def("linear_gelu_mul", &linear_gelu_mul,
+        "linear layer with the GELU gate behind its first columns, many rows");
   m.def("linear_silu_mul", &linear_silu_mul,
         "linear layer with the silu gate behind it, many rows");
   m.def("moe_layout", &moe_layout, "softmax top-k router + expert segments");

@@ -300,12 +300,16 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
 // rows 163 / 82 -> 140 / 70. A large product of the library reaches 1.65 PFLOP/s
 // there (8192^3: 668 us). Cards differ by 5 to 15 % in what their power limit leaves.
 //
-// DENSE (mode 5) is a gated linear layer of its own, one matrix over m_rows rows,
+// DENSE (modes 5 and 6) is a gated linear layer of its own, one matrix over m_rows rows,
 // against the library's product and a pass of silu over its result (2 N columns
 // written and read again): 2 x 3072 x 1024 at 24,000 rows 357 -> 259 us, 2 x 8192 x
 // 2048 at 32,768 rows 1775 -> 1555, 2 x 12288 x 4096 4597 -> 4413, 2 x 25600 x 5120
 // at 8192 rows 3280 -> 2829; the unit's inputs stay in fp32 (error against 64 bits
-// 3.1e-3 -> 1.7e-3).
+// 3.1e-3 -> 1.7e-3). Mode 6 is the unit with GELU by tanh; column blocks behind its own
+// are 256 plain columns each, of the same input (a residual gate), so that these need no
+// launch that fills the chip for itself: 2 x 8192 and 2048 columns of 2048 at 32,768
+// rows 2011 -> 1814 us, at 1532 rows 112 -> 103 (119 with the product of the 2048 by the
+// library); error against 64 bits 6.6e-3 -> 3.7e-3.
 //
 // An XCD (workgroup id % 8) takes GW_ROWS neighbouring row tiles and goes through
 // all column blocks with them: its 32 workgroups share 4 row tiles and 8 column
@@ -429,7 +433,11 @@ __device__ __forceinline__ void gw_unit8(float (&v)[8], float (&u)[8], float lim
     GW_EACH(v[i] *= rw)
     GW_EACH(u[i] *= rw)
   }
-  if (MODE == 3) {
+  if (MODE == 6) {     // 0.5 (1 + tanh z) = 1 / (1 + exp(-2 z))
+    GW_EACH(d[i] = v[i] * v[i])
+    GW_EACH(d[i] = fmaf(d[i], -2.302208198f * 0.044715f, -2.302208198f))
+    GW_EACH(d[i] = d[i] * v[i])
+  } else if (MODE == 3) {
     GW_EACH(v[i] = fminf(v[i], limit))
     GW_EACH(u[i] = fminf(fmaxf(u[i], -limit), limit) + 1.0f)
     GW_EACH(d[i] = v[i] * -1.702f)
@@ -456,12 +464,13 @@ __device__ __forceinline__ void gw_body(
     const u16* __restrict__ w, const int* __restrict__ row_tok,
     const int* __restrict__ tile_off, const int* __restrict__ counts,
     int n_experts, int n_cols, long K, float limit,
-    const float* __restrict__ row_w, int m_rows) {
+    const float* __restrict__ row_w, int m_rows, const u16* __restrict__ bias,
+    u16* __restrict__ rest, int n_rest) {
   constexpr bool GATED = MODE == 1 || MODE >= 3;
-  constexpr bool DENSE = MODE == 5;
+  constexpr bool DENSE = MODE >= 5, REST = MODE == 6;
   constexpr bool GATHER = MODE != 0 && !DENSE;
   constexpr int BN = GATED ? 128 : 256;   // output columns
-  const int nb = n_cols / BN;
+  const int nb = n_cols / BN + (REST ? n_rest / 256 : 0);
   const int total = DENSE ? (m_rows + 255) / 256 : tile_off[n_experts];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -506,8 +515,8 @@ __device__ __forceinline__ void gw_body(
         s.va[ANY ? 0 : j] = (u32)row * (u32)(K * 2) + ch[j & 1] * 2;
     }
     const int br = wave * 64;                  // first of this wave's B rows
-    const long brow =
-        (GATED && br >= 128) ? n_cols + g.n0 + br - 128 : g.n0 + br;
+    long brow = (GATED && br >= 128) ? n_cols + g.n0 + br - 128 : g.n0 + br;
+    if (REST && g.n0 >= n_cols) brow = 2 * g.n0 + br;   // 256 rows behind the up's
     s.pb = w + ((long)g.e * (GATED ? 2 : 1) * n_cols + brow) * K;
     s.ra = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu,
                                              0x00027000);
@@ -561,6 +570,27 @@ __device__ __forceinline__ void gw_body(
     const u32 off = (u32)(ln * n_cols + (quad & 1) * 16 + (quad >> 1) * 8) * 2;
     const long row = g.seg + wm * 128;
     char* at = (char*)(out + row * n_cols + g.n0 + wn * (GATED ? 64 : 128));
+    const bool gate = !REST || g.n0 < n_cols;    // else plain sums, 256 columns
+    u16x4 bs[REST ? 8 : 1];
+    char* more = nullptr;
+    if (REST) {
+      const u16* bp = bias + (gate ? g.n0 : 2 * g.n0) + wn * 64 + quad * 4;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        bs[j] = bias ? *(const u16x4*)(bp + (j & 3) * 16 +
+                                       (j < 4 ? 0 : gate ? n_cols : 128))
+                     : (u16x4)(0);
+      more = (char*)(rest + row * n_rest + 2 * (g.n0 - n_cols) + wn * 64 +
+                     (long)ln * n_rest + (quad & 1) * 16 + (quad >> 1) * 8);
+    }
+    auto pack = [](const float (&x)[8]) {
+      u32 p[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) p[q] = gw_pack(x[2 * q], x[2 * q + 1]);
+      const auto s0 = __builtin_amdgcn_permlane16_swap(p[0], p[2], false, false);
+      const auto s1 = __builtin_amdgcn_permlane16_swap(p[1], p[3], false, false);
+      return u32x4{s0[0], s1[0], s0[1], s1[1]};
+    };
 #pragma unroll
     for (int i = 0; i < 8; ++i, at += (long)n_cols * 32) {
       const float rw = MODE == 4 ? row_w[row + i * 16 + ln] : 1.f;
@@ -580,20 +610,30 @@ __device__ __forceinline__ void gw_body(
           if (GATED) up[q] = acc[i][(j + (q >> 2) + 4) & 7][q & 3];
           else x[q] = gg_unit<MODE>(x[q], 0.f, limit, rw);
         }
-        if (GATED) gw_unit8<MODE>(x, up, limit, rw);
-        u32 p[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) p[q] = gw_pack(x[2 * q], x[2 * q + 1]);
 #pragma unroll
         for (int q = 0; q < 2; ++q) {       // for the next tile
           acc[i][j + q] = (f32x4)(0.f);
           if (GATED) acc[i][(j + q + 4) & 7] = (f32x4)(0.f);
         }
-        const auto s0 =
-            __builtin_amdgcn_permlane16_swap(p[0], p[2], false, false);
-        const auto s1 =
-            __builtin_amdgcn_permlane16_swap(p[1], p[3], false, false);
-        const u32x4 pk = {s0[0], s1[0], s0[1], s1[1]};
+        if (REST) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            x[q] += bf2f(bs[j + (q >> 2)][q & 3]);
+            up[q] += bf2f(bs[j + 4 + (q >> 2)][q & 3]);
+          }
+          if (!gate) {
+            u16* o = (u16*)(more + (long)i * n_rest * 32) + j * 16;
+            const u32x4 pa = pack(x), pb = pack(up);
+            if (wm * 128 + i * 16 + ln < g.live) {
+              *(u32x4*)o = pa;
+              *(u32x4*)(o + 128) = pb;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            continue;
+          }
+        }
+        if (GATED) gw_unit8<MODE>(x, up, limit, rw);
+        const u32x4 pk = pack(x);
         u16* o = (u16*)(at + off) + j * 16;
         if (DENSE && wm * 128 + i * 16 + ln >= g.live) {
         } else if (ANY) {
@@ -754,9 +794,10 @@ gw_kernel(u16* __restrict__ out, const u16* __restrict__ a,
           const u16* __restrict__ w, const int* __restrict__ row_tok,
           const int* __restrict__ tile_off, const int* __restrict__ counts,
           int n_experts, int n_cols, long K, float limit,
-          const float* __restrict__ row_w, int m_rows) {
+          const float* __restrict__ row_w, int m_rows,
+          const u16* __restrict__ bias, u16* __restrict__ rest, int n_rest) {
   gw_body<MODE, ANY>(out, a, w, row_tok, tile_off, counts, n_experts, n_cols, K,
-                     limit, row_w, m_rows);
+                     limit, row_w, m_rows, bias, rest, n_rest);
 }
 
 // a workgroup a CU, a multiple of 8 of them
@@ -804,7 +845,7 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
     static std::atomic<unsigned long long> asked{0};                        \
     lds_limit((const void*)gw_kernel<M, ANY>, GW_LDS, asked);               \
     hipLaunchKernelGGL((gw_kernel<M, ANY>), grid, dim3(256), GW_LDS,        \
-                       stream, GG_ARGS, 0);                                 \
+                       stream, GG_ARGS, 0, nullptr, nullptr, 0);                             \
   }
 #define GG_WIDE(M)                                                          \
   {                                                                         \
@@ -845,19 +886,34 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
 #undef GG_LAUNCH
 }
 
-// out [M, N] = silu(x Wg^T) * (x Wu^T): w [2 N, K], the gate's rows first. x and
-// w at multiples of 16 bytes, K a multiple of 64 and below 2^21 (a tile's offsets
-// are of 32 bits, where it begins of 64), N a multiple of 128.
+template <int MODE>
+static void gw_dense(void* out, void* rest, const void* x, const void* w,
+                     const void* bias, int M, int N, int n_rest, long K,
+                     hipStream_t stream) {
+  static std::atomic<unsigned long long> asked{0};
+  lds_limit((const void*)gw_kernel<MODE, false>, GW_LDS, asked);
+  hipLaunchKernelGGL((gw_kernel<MODE, false>),
+                     dim3(gw_grid(((long)M + 255) / 256, N / 128 + n_rest / 256)),
+                     dim3(256), GW_LDS, stream, (u16*)out, (const u16*)x,
+                     (const u16*)w, nullptr, nullptr, nullptr, 0, N, K, 0.f,
+                     nullptr, M, (const u16*)bias, (u16*)rest, n_rest);
+}
+
+// out [M, N] = silu(x Wg^T) * (x Wu^T): w [2 N, K], the gate's rows first. x and w at
+// multiples of 16 bytes, K a multiple of 64 and below 2^21 (a tile's offsets are of 32
+// bits, where it begins of 64), N a multiple of 128.
 extern "C" void sutro_linear_silu_mul(void* out, const void* x, const void* w,
                                       int M, int N, long K,
                                       hipStream_t stream) {
-  static std::atomic<unsigned long long> asked{0};
-  lds_limit((const void*)gw_kernel<5, false>, GW_LDS, asked);
-  hipLaunchKernelGGL((gw_kernel<5, false>),
-                     dim3(gw_grid(((long)M + 255) / 256, N / 128)), dim3(256),
-                     GW_LDS, stream, (u16*)out, (const u16*)x,
-                     (const u16*)w, nullptr, nullptr, nullptr, 0, N, K, 0.f,
-                     nullptr, M);
+  gw_dense<5>(out, nullptr, x, w, nullptr, M, N, 0, K, stream);
+}
+
+// The same with GELU by tanh, a bias (null or at multiples of 8 bytes) and more columns
+// behind them: rest [M, n_rest] = x Wr^T, w [2 N + n_rest, K], n_rest a multiple of 256.
+extern "C" void sutro_linear_gelu_mul(void* out, void* rest, const void* x,
+                                      const void* w, const void* bias, int M, int N,
+                                      int n_rest, long K, hipStream_t stream) {
+  gw_dense<6>(out, rest, x, w, bias, M, N, n_rest, K, stream);
 }
 
 extern "C" void sutro_grouped_gemm(void* out, const void* a, long a_rows,

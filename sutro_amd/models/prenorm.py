@@ -43,7 +43,7 @@ from .hybrid_spec import (AttnMixerSpec, DecayAttnMixerSpec, DeltaMixerSpec,
 from .layers import (DecayAttention, GatedDeltaRule, HyperConnection,
                      LatentAttention, LocalAttention, RoutedExperts,
                      SectionedLinear, SSDMixer, _pad)
-from .linear import Linear
+from .linear import Linear, unhooked
 
 
 class PreNormBlock(nn.Module):
@@ -189,11 +189,18 @@ class PreNormBlock(nn.Module):
         self._join(x, h, self.hc1, self.norm2,
                    self.hc2.w_in if self.streams else None, x_in, y=y)
         if self.ff:
-            proj = self.ff_in(h)
             off = self.ff_in.offsets
-            if self.relu2:
-                act = hops.relu_sq(proj)[:, :self.ff]
+            act = None
+            if (type(self.ff_in) is SectionedLinear and not self.relu2
+                    and off["up"] == self.ff and self.ff_in.bias is None
+                    and unhooked(self.ff_in)):
+                act = ops.linear_silu_rows(h, self.ff_in.weight)
+            if act is not None:
+                pass
+            elif self.relu2:
+                act = hops.relu_sq(self.ff_in(h))[:, :self.ff]
             else:
+                proj = self.ff_in(h)
                 act = hops.glu_mul(proj, off["gate"], off["up"], self.ff,
                                    hops.GLU_SILU)
             self._join(x, h, self.hc2, next_norm, next_in, None, extra, write,

@@ -24,6 +24,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import ops
 from ..engine.batch import ForwardBatch
 from ..engine.kv_cache import PagedKVCache
 from ..ops import hybrid as hops
@@ -31,7 +32,7 @@ from ..parallel.tp import TPContext
 from .hybrid_spec import (AttnMixerSpec, DeltaMixerSpec, HybridLayerSpec,
                           HybridSpec, ParallelMixerSpec)
 from .layers import GatedDeltaRule, LocalAttention, SectionedLinear, _pad
-from .linear import Linear
+from .linear import Linear, unhooked
 
 
 class HybridBlock(nn.Module):
@@ -150,11 +151,18 @@ class HybridBlock(nn.Module):
         hops.gated_norm_residual(x, y, proj, off["rg"], self.norm1, self.eps,
                                  self.mult, h_out)
         if self.ff:
-            proj = self.ff_in(h)
             off = self.ff_in.offsets
-            act = hops.gelu_tanh_mul(proj, off["gate"], off["up"], self.ff)
+            made, rg, lin = None, 0, self.ff_in
+            if (type(lin) is SectionedLinear and off["up"] == self.ff
+                    and off["rg"] == 2 * self.ff and unhooked(lin)):
+                made = ops.linear_gelu_mul(h, lin.weight, lin.bias, self.ff)
+            if made is not None:
+                act, proj = made
+            else:
+                proj, rg = lin(h), off["rg"]
+                act = hops.gelu_tanh_mul(proj, off["gate"], off["up"], self.ff)
             y = self.ff_out(act)
-            hops.gated_norm_residual(x, y, proj, off["rg"], self.norm2,
+            hops.gated_norm_residual(x, y, proj, rg, self.norm2,
                                      self.eps, self.mult, h_out)
 
 

@@ -457,6 +457,34 @@ def linear_silu_mul(x, w):
     return silu_mul(F.linear(x, w))
 
 
+def linear_gelu_mul(x, w, bias, ff: int):
+    """(gelu_tanh(gate) * up, the rest) of x w^T + bias, whose first 2 ff columns are
+    gate and up: where one launch makes all of it (prompts), else None. us of the
+    library and the unit's launch, and of this one, columns 2 ff + the rest:
+      16384 + 2048 x 2048   32768 rows  2011 / 1814    8192   529 / 464
+      17408 + 2048 x 2048    1532 rows   112 /  103
+      20992 + 4096 x 4096    5298 rows   878 /  801
+       6144 + 1024 x 1024   26243 rows   444 /  333
+       2560 +  512 x  512   11279 rows    97 /   58
+      12288 + 4096 x 4096   26526 rows  2437 / 2471
+    With a long k and few gated columns the unit's pass is small beside the product,
+    which the library makes 2 % faster."""
+    if not (_many_rows(x, w) and ff % 128 == 0 and 0 < 2 * ff <= w.shape[0]
+            and w.shape[0] % 256 == 0
+            and (x.shape[1] < 4096 or 2 * ff * 5 >= w.shape[0] * 4)
+            and _plain_bias(bias, x, w)
+            and (bias is None or bias.data_ptr() % 8 == 0)):
+        return None
+    return _require_hip().linear_gelu_mul(x, w, bias, ff)
+
+
+def linear_silu_rows(x, w):
+    """silu_mul(x w^T) where one launch makes it (prompts), else None. Against the
+    library and the unit's launch 0.86 to 0.95 of the time at 16384 x 2048 and 24576
+    x 4096, 0.45 to 0.8 with a k of 1024 and less."""
+    return _require_hip().linear_silu_mul(x, w) if _many_rows(x, w) else None
+
+
 def _one_row(x, residual, norm_w, w, gated: bool) -> bool:
     """Whether csrc/gemm_skinny.hip makes the norm of one row inside the product
     behind it. Up to 4096 waves make it, each workgroup for itself, and with short

@@ -39,7 +39,7 @@ def _want(x, w, unit):
 
 
 def _check(got, want):
-    """One rounding to bf16 (2^-9), the unit in fp32 far below it; where exp(-gate)
+    """One rounding to bf16 (2^-8 / (1 + 2^-8)), the unit in fp32 far below it; where exp(-gate)
     is past 2^126 the quotient, under 2^-119 of the up's, may be 0."""
     got, want = got.double().cpu(), want
     assert torch.equal(got.isnan(), want.isnan())
@@ -55,6 +55,11 @@ def silu(g, u):
     return g / (1 + torch.exp(-g)) * u
 
 
+def gelu(g, u):
+    z = 2 * math.sqrt(2 / math.pi) * (g + 0.044715 * g ** 3)
+    return torch.where(g.abs() > 1e4, g * (g > 0), g / (1 + torch.exp(-z))) * u
+
+
 def clamped(g, u, limit=7.0):
     lim = torch.tensor(limit, dtype=g.dtype)        # (of a NaN the limit)
     g, u = torch.fmin(g, lim), torch.fmin(torch.fmax(u, -lim), lim)
@@ -65,6 +70,39 @@ def test_one_matrix():
     x, w = _operands()
     got = ops._require_hip().linear_silu_mul(x.to(DEV), w.to(DEV))
     _check(got, _want(x, w, silu))
+
+
+def test_gelu():
+    x, w = _operands()
+    x, w = x[:, :3], w[:, :3]           # (an infinite gate: 0 or the gate itself)
+    w[w.isinf()] = 0
+    x, w = (torch.nn.functional.pad(t, (0, K - 3)) for t in (x, w))
+    got = ops._require_hip().linear_gelu_mul(x.to(DEV), w.to(DEV), None, N)[0]
+    _check(got, _want(x, w, gelu))
+
+
+@pytest.mark.parametrize("biased", [True, False])
+@pytest.mark.parametrize("rows,ff,k,more", [(1, 128, 64, 0), (255, 256, 192, 256),
+                                            (257, 384, 1024, 2048),
+                                            (3000, 1152, 320, 512)])
+def test_columns_behind(rows, ff, k, more, biased):
+    """GELU with a bias, and plain columns behind gate and up: the fp32 sum (and
+    unit) rounded once, 2^-8, and the sum's own error of k products in fp32."""
+    g = torch.Generator().manual_seed(rows + k)
+    x = torch.randn(rows, k, generator=g).bfloat16()
+    w = (torch.randn(2 * ff + more, k, generator=g) * 2 * k ** -0.5).bfloat16()
+    b = torch.randn(2 * ff + more, generator=g).bfloat16() if biased else None
+    act, rest = ops._require_hip().linear_gelu_mul(
+        x.to(DEV), w.to(DEV), None if b is None else b.to(DEV), ff)
+    y = x.double() @ w.double().T + (0 if b is None else b.double())
+    gate, up, more_y = y[:, :ff], y[:, ff:2 * ff], y[:, 2 * ff:]
+    sums = k * 2.0 ** -22
+    want = gelu(gate, up)
+    assert ((act.double().cpu() - want).abs() <= want.abs() * 2 ** -8
+            + sums * (1 + gate.abs()) * (1 + up.abs())).all()
+    assert rest.shape == more_y.shape
+    assert ((rest.double().cpu() - more_y).abs() <= more_y.abs() * 2 ** -8
+            + sums).all()
 
 
 @pytest.mark.parametrize("kind", ["silu", "clamped", "weighted"])

@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 def test_uneven_sequences(H, dk, dv, window):
     """Sequences of one key to seven steps of 64, with and without cached tokens
     in front, tiles with fewer than 64 rows, and decoded tokens whose keys may be
-    cut into runs. A weight is rounded to 2^-9 of itself and so is the result:
-    2^-8 of the largest value, and 2^-12 more for scores in 32 bits."""
+    cut into runs. A weight is rounded to bf16, at most 2^-8 of itself, and so is
+    the result: 2^-7 of the largest value, and 2^-12 more for scores in 32 bits."""
     dev = "cuda"
     g = torch.Generator().manual_seed(dk * H + window)
     new = [1, 63, 64, 65, 33, 2, 130, 200]       # prompt pieces
@@ -65,4 +65,4 @@ def test_uneven_sequences(H, dk, dv, window):
         s.masked_fill_(~seen, float("-inf"))
         want = torch.einsum("htk,kd->thd", s.softmax(-1), kv[:, :dv])
         err = (got[locs[i]:locs[i + 1]] - want).abs().max()
-        assert err <= (2 ** -8 + 2 ** -12) * float(kv[:, :dv].abs().max())
+        assert err <= (2 ** -7 + 2 ** -12) * float(kv[:, :dv].abs().max())
