@@ -58,28 +58,17 @@ __device__ __forceinline__ u32 gswz(u32 byte) {
 
 // Stage a ROWS x 64 bf16 tile (ROWS rows of 128B) with WAVES waves; each
 // wave issues ROWS/(8*WAVES) x 1KB chunks.
-template <int ROWS, int WAVES, bool GATHER>
-__device__ __forceinline__ void gg_stage(
-    u16* lds, const u16* gsrc, long row_stride_b, const int* row_tok,
-    int m0, int rows_valid, int wave, int lane) {
+template <int ROWS, int WAVES>
+__device__ __forceinline__ void gg_stage(u16* lds, const u16* gsrc,
+                                         long row_stride_b, int wave, int lane) {
   constexpr int CH = ROWS / (8 * WAVES);
   static_assert(CH >= 1, "tile too small for wave count");
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
-    const int c = wave * CH + j;
-    const u32 b = (u32)c * 1024u + (u32)lane * 16u;  // lane-linear LDS byte
-    const u32 lb = gswz(b);                          // pre-swizzled source
-    int row = (int)(lb >> 7);
-    long grow;
-    if (GATHER) {
-      int r = m0 + row;
-      int tok = (row < rows_valid) ? row_tok[r] : 0;
-      if (tok < 0) tok = 0;  // padding: deterministic garbage, discarded
-      grow = (long)tok;
-    } else {
-      grow = (long)(m0 + min(row, rows_valid - 1));
-    }
-    glds16g((const u32*)((const char*)gsrc + grow * row_stride_b + (lb & 127u)),
+    const u32 b = (u32)(wave * CH + j) * 1024u + (u32)lane * 16u;
+    const u32 lb = gswz(b);      // lane-linear LDS byte, pre-swizzled source
+    glds16g((const u32*)((const char*)gsrc + (long)(lb >> 7) * row_stride_b +
+                         (lb & 127u)),
             (u32*)((char*)lds + b));
   }
 }
@@ -156,7 +145,7 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   const int rows_valid = counts[e] - m0;              // live rows this tile
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WCOLS, wn = wave % WCOLS;
 
   __shared__ u16 smem[2][(BM + (GATED ? 2 : 1) * BN) * 64];
@@ -196,20 +185,54 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   // rows each 53.9 us, carried 47.5); tiles of 32 are 1 % faster without.
   constexpr bool CARRY = BM == 64;
   const u16 *pa = aa + ko, *pg = wg + ko, *pu = wu + ko;
-  auto stage = [&](u16* to) {
-    const u16* sa = CARRY ? pa : aa + ko;
-    const u16* sg = CARRY ? pg : wg + ko;
-    const u16* su = CARRY ? pu : wu + ko;
-    if (GATHER)
-      gg_stage<BM, WAVES, true>(to, sa, Kb, rt, m0, rows_valid, wave, lane);
-    else
-      gg_stage<BM, WAVES, false>(to, sa, Kb, nullptr, m0, BM, wave, lane);
-    gg_stage<BN, WAVES, false>(to + b_off, sg, Kb, nullptr, 0, BN, wave, lane);
+  auto stage_w = [&](u16* to) {
+    gg_stage<BN, WAVES>(to + b_off, CARRY ? pg : wg + ko, Kb, wave, lane);
     if (GATED)
-      gg_stage<BN, WAVES, false>(to + b2_off, su, Kb, nullptr, 0, BN, wave,
-                                 lane);
+      gg_stage<BN, WAVES>(to + b2_off, CARRY ? pu : wu + ko, Kb, wave, lane);
   };
-  stage(smem[0]);
+  stage_w(smem[0]);     // (while the rows are looked up)
+
+  // The tile's rows, 8 a chunk; chunks of rows past the live ones are left out (what the
+  // LDS holds there is multiplied for rows that nobody reads: a branch around those
+  // products costs 20 cycles a step). Where experts get two rows, tiles of 64 fetched
+  // as much of rows as of weights: down of 28 experts of 4096 x 3072 158 -> 126 us, of
+  // 2048 x 2048 on tiles of 32 50.7 -> 44.5. Rows are looked up once: at each step, the
+  // wait for the table stood before the copies (16 rows an expert of 2048 x 2048 on
+  // tiles of 64 139 -> 119 us, 64 of 3072 x 4096 530 -> 432, 112 of 2048 x 2048 on 128
+  // 198 -> 169). Only with 2.5 workgroups a CU or more on tiles of 32 that wait does
+  // good, it seems by taking them out of step: 28 experts 70.9 us without and 68.0 with
+  // it, 32 at 16 rows 96.2 and 94.0, 660 workgroups of 2 x 768 columns 72.1 and 69.3;
+  // 640 of 2 x 2048 59.4 and 60.7, 352 of them 38.7 and 46.3; with a k of 4096 (960
+  // workgroups) 216 and 230.
+  constexpr int CHA = BM / (8 * WAVES);
+  static_assert(CHA >= 1, "tile too small for wave count");
+  // (from the last wave on: the first ones have the products of few rows)
+  auto a_chunk = [&](int j) { return j * WAVES + WAVES - 1 - wave; };
+  auto a_row = [&](int j) {
+    const u32 lb = gswz((u32)a_chunk(j) * 1024u + (u32)lane * 16u);
+    int row = m0 + min((int)(lb >> 7), rows_valid - 1);
+    asm volatile("" : "+v"(row));       // (a look-up at a step stays there)
+    return (long)(GATHER ? max(rt[row], 0) : row) * Kb + (lb & 127u);
+  };
+  long a_at[CHA];
+#pragma unroll
+  for (int j = 0; j < CHA; ++j) a_at[j] = a_row(j);
+  constexpr bool AGAIN = BM == 32 && GATHER;
+  const bool again = K < 4096 && tile_off[n_experts] * gridDim.y > 640;
+
+  auto stage_a = [&](u16* to) {
+    const char* sa = (const char*)(CARRY ? pa : aa + ko);
+#pragma unroll
+    for (int j = 0; j < CHA; ++j) {
+      const int c = a_chunk(j);
+      if (c * 8 < rows_valid) {
+        if (AGAIN && again) a_at[j] = a_row(j);
+        glds16g((const u32*)(sa + a_at[j]),
+                (u32*)((char*)to + c * 1024 + lane * 16));
+      }
+    }
+  };
+  stage_a(smem[0]);
   __syncthreads();
 
   for (int kt = 0; kt < KT; ++kt) {
@@ -229,7 +252,8 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
         pg += step;
         if (GATED) pu += step;
       }
-      stage(smem[p ^ 1]);
+      stage_a(smem[p ^ 1]);
+      stage_w(smem[p ^ 1]);
     }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -260,6 +284,7 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   const int dcol = lane & 15;
 #pragma unroll
   for (int i = 0; i < MF; ++i) {
+    if (wm * WM + i * 16 >= rows_valid) break;
 #pragma unroll
     for (int j = 0; j < NF; ++j) {
       const int gn = n0 + wn * WN + j * 16 + dcol;
@@ -267,6 +292,10 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int grow = grow0 + r;
+        // Padding rows are left as they are: those of a workspace that keeps zeros or
+        // results may be gathered with weight 0, and what was multiplied for them
+        // need not be finite.
+        if (grow >= rows_valid) continue;
         const long o = (long)(seg0 + m0 + grow) * n_cols + gn;
         const float v = gg_unit<MODE>(
             accg[i][j][r], GATED ? accu[GATED ? i : 0][GATED ? j : 0][r] : 0.f,

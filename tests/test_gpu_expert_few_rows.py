@@ -1,0 +1,53 @@
+"""The expert GEMMs on tiles of 32 to 128 rows where the last tile of an expert has few
+rows: what lies in padding rows is not seen in the others, and nothing is put there."""
+
+import pytest
+import torch
+
+from sutro_amd.ops import hybrid as hops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("bm", [32, 64, 128])
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE, hops.ACT_RELU2])
+@pytest.mark.parametrize("K,ff", [(64, 64), (320, 192), (2048, 1024), (4096, 1024)])
+def test_live_rows(K, ff, act, bm):
+    """Counts around chunks of 8 rows and blocks of 16; with 1024 columns more than
+    640 workgroups (tiles of 32 look their rows up at each step), with fewer not."""
+    counts = [1, 0, 7, 8, 9, 15, 16, 17, 31, 32, 33, 2, 63, 65, 127, 129, 0, 3]
+    counts += [5] * (24 if ff == 1024 else 0)
+    g = torch.Generator(device=DEV).manual_seed(K + bm)
+    gated, gather = act == hops.ACT_SILU_GATE, act != hops.ACT_NONE
+    tiles = [(c + bm - 1) // bm for c in counts]
+    off = torch.tensor([0] + tiles, device=DEV).cumsum(0).int()
+    cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
+    rows, T = sum(tiles) * bm, 50
+    w = torch.randn(len(counts), 2 * ff if gated else ff, K, generator=g, device=DEV)
+    w = (w * K ** -0.5).bfloat16()
+    x = torch.randn(T if gather else rows, K, generator=g, device=DEV).bfloat16()
+    live = torch.zeros(rows, dtype=torch.bool, device=DEV)
+    tok = torch.full((rows,), -1, device=DEV, dtype=torch.int32)
+    for e, c in enumerate(counts):
+        a = int(off[e]) * bm
+        live[a:a + c] = True
+        tok[a:a + c] = torch.randint(1, T, (c,), generator=g, device=DEV).int()
+    if gather:
+        x[0] = float("nan")            # what a row without a token would read
+    else:
+        x[~live] = float("nan")
+    out = torch.zeros(rows, ff, device=DEV, dtype=torch.bfloat16)
+    hops.expert_gemm(out, x, w, tok if gather else None, off, cnt, act, bm, 0.0, None)
+    assert (out[~live] == 0).all()
+    for e, c in enumerate(counts):
+        a = int(off[e]) * bm
+        xe = (x[tok[a:a + c].long()] if gather else x[a:a + c]).float()
+        y = xe @ w[e].float().T
+        if gated:
+            y = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+        elif act == hops.ACT_RELU2:
+            y = y.relu() ** 2
+        # one rounding to bf16 (2^-8) and fp32 sums of K products in other orders
+        torch.testing.assert_close(out[a:a + c].float(), y, rtol=2 ** -7,
+                                   atol=2 ** -7)
