@@ -388,13 +388,20 @@ def _plain_bias(bias, x, w) -> bool:
         and not (torch.is_grad_enabled() and bias.requires_grad))
 
 
+def _up_to_256(x) -> bool:
+    """(One look for the two kernels: eager calls on more rows pay for it.)"""
+    return (type(x) is torch.Tensor and not _tracing() and x.dim() == 2
+            and x.shape[0] <= 256)
+
+
 def linear(x, w, bias=None):
     """x w^T (+ bias): the library's product, or over up to 256 rows (decode
     steps, short prompts) csrc/gemm_mid.hip or csrc/gemm_skinny.hip."""
-    if _mid_rows(x, w) and _plain_bias(bias, x, w):
-        return _require_hip().linear_mid(x, w, bias, False)
-    if _few_rows(x, w) and _plain_bias(bias, x, w):
-        return _require_hip().linear_skinny(x, w, bias, False)
+    if _up_to_256(x):
+        if _mid_rows(x, w) and _plain_bias(bias, x, w):
+            return _require_hip().linear_mid(x, w, bias, False)
+        if _few_rows(x, w) and _plain_bias(bias, x, w):
+            return _require_hip().linear_skinny(x, w, bias, False)
     return F.linear(x, w, bias)
 
 
@@ -448,10 +455,11 @@ def _many_rows(x, w) -> bool:
 
 def linear_silu_mul(x, w):
     """silu_mul(x w^T), w the gate's rows and then the up's."""
-    if _mid_rows(x, w, gated=True):
-        return _require_hip().linear_mid(x, w, None, True)
-    if _few_rows(x, w, gated=True):
-        return _require_hip().linear_skinny(x, w, None, True)
+    if _up_to_256(x):
+        if _mid_rows(x, w, gated=True):
+            return _require_hip().linear_mid(x, w, None, True)
+        if _few_rows(x, w, gated=True):
+            return _require_hip().linear_skinny(x, w, None, True)
     if _many_rows(x, w):
         return _require_hip().linear_silu_mul(x, w)
     return silu_mul(F.linear(x, w))
