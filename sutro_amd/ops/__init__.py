@@ -530,23 +530,23 @@ def expert_tile(n_rows: int, experts: int, inner: int, width: int,
     for `n_rows` (token, expert) pairs in bf16 on the matrix cores (K and N
     multiples of 64), by the rows an expert gets on average. Taller tiles do
     more work per byte but pad more; both products together, at 32 experts of
-    2048 x 2048: at 72 rows 261 / 215 / 200 us on tiles of 64 / 128 / 256, at 96
-    rows 261 / 212 / 197, at 192 rows 370 / 341 / 198, at 384 rows 877 / 511 /
-    337. (So tiles of 256 would already pay at 72 rows there, and the lines below
+    2048 x 2048: at 72 rows 240 / 221 / 208 us on tiles of 64 / 128 / 256, at 96
+    rows 243 / 226 / 209, at 192 rows 366 / 314 / 204, at 384 rows 890 / 465 /
+    332. (So tiles of 256 would already pay at 72 rows there, and the lines below
     were drawn when their kernel was a slower one; they have not been moved.)
 
     They also leave fewer workgroups: one of 256 rows takes 128 columns of the
     gated product or 256 of the other, and with few of them in either product
     the chip idles: the rule wants 128. 8 experts of 1024 x 512, 192 / 512 / 1024
-    rows an expert (24 / 64 / 128 of either) 26 / 42 / 64 us on 64, 33 / 37 / 47 on
-    128, 41 / 42 / 44 on 256. 8 of 2048 x 2048 are past the crossing with 64 to 96
-    of the second, 192 / 384 / 512 rows: 82 / 133 / 147 us on 128, 83 / 100 / 99 on
+    rows an expert (24 / 64 / 128 of either) 28 / 43 / 52 us on 64, 29 / 35 / 53 on
+    128, 43 / 46 / 48 on 256. 8 of 2048 x 2048 are past the crossing with 64 to 96
+    of the second, 192 / 384 / 512 rows: 74 / 115 / 136 us on 128, 85 / 101 / 102 on
     256. Tiles of 128 want 96.
 
     Up to 16 rows, where the weights are all there is to read, tiles of 32: four
     workgroups of the gated product fit a CU instead of three. They are taken
     unless their number then fills the rounds worse: 1024 workgroups (2048 wide)
-    171 -> 133 us, 1536 (3072 wide, K 4096) 448 and 448.
+    156 -> 144 us, 1536 (3072 wide, K 4096) 427 -> 447.
 
     `local`: the experts whose products this rank makes (all by default); its
     workgroups are counted."""
