@@ -368,8 +368,8 @@ def _mid_rows(x, w, gated: bool = False) -> bool:
         return False
     M, K = x.shape
     rows = w.shape[0]
-    return (K % 256 == 0 and K >= 512 and _mid_sizes(M, rows, K, gated)
-            and _unwatched() and x.dtype == torch.bfloat16
+    return (K % 256 == 0 and 512 <= K < 1 << 20 and rows > 0
+            and _mid_sizes(M, rows, K, gated) and _unwatched() and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.device == x.device
             and w.dim() == 2 and w.shape[1] == K
             and rows % (16 if gated else 4) == 0 and rows < 1 << 24

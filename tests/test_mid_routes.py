@@ -52,3 +52,15 @@ def test_operands(on_gpu):
         seen = []
         torch.func.vmap(lambda v: seen.append(ops._mid_rows(v, w)) or v)(x[None])
     assert seen == [False]
+
+
+@pytest.mark.parametrize("M,K,rows,gated", [
+    (20, 2048, 0, False), (100, 2048, 0, False), (256, 2048, 0, False),
+    (20, 2048, 0, True), (100, 2048, 0, True), (48, 1 << 20, 2048, False),
+    (100, 1 << 20, 4096, True)])
+def test_sizes_the_kernel_refuses(on_gpu, M, K, rows, gated):
+    """No weights at all, and rows of a million numbers: the library's. (Meta tensors
+    stand in for them: the rule does not read.)"""
+    x = torch.empty(M, K, dtype=torch.bfloat16, device="meta")
+    w = torch.empty(rows, K, dtype=torch.bfloat16, device="meta")
+    assert not ops._mid_rows(x, w, gated)
