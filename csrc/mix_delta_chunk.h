@@ -105,6 +105,7 @@ delta_pairs_kernel(const DeltaChunkArgs A) {
     const int i = b + lane;
     s += __popcll(__ballot(i < A.S && dc_slot(A.qlocs[i < A.S ? i : 0], i) <= slot));
   }
+  if (s < 0) return;       // tokens in front of the first sequence
   const int q0 = A.qlocs[s], n = A.qlocs[s + 1] - q0;
   const int base = (slot - dc_slot(q0, s)) * CH_T;
   if (n < A.least || base >= n) return;

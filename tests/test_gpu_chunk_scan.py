@@ -246,3 +246,34 @@ def test_numbers_that_are_not_finite(bad, which):
         fine = torch.isfinite(y)
         assert torch.equal(torch.isfinite(x), fine)
         torch.testing.assert_close(x[fine], y[fine], rtol=2e-4, atol=2e-4)
+
+
+@pytest.mark.parametrize("front", [31, 100, 1000])
+@pytest.mark.parametrize("delta", [False, True])
+def test_tokens_in_front_of_the_first_sequence(front, delta):
+    """Rows that no sequence has, before the first one: the same results to the bit as
+    without them."""
+    g = torch.Generator().manual_seed(front)
+    H, dk, dv, T = 2, 64, 48, 170
+    qlocs = torch.tensor([0, 90, 170], dtype=torch.int32)
+    total = torch.tensor([94, 80], dtype=torch.int32).to(DEV)
+    slots = torch.tensor([1, 0], dtype=torch.int32).to(DEV)
+    n = front + T
+    q, k = (torch.nn.functional.normalize(torch.randn(n, H, dk, generator=g), dim=-1)
+            for _ in "qk")
+    v = torch.randn(n, H, dv, generator=g)
+    a = torch.rand(n, H, generator=g) * 0.5 + 0.5
+    b = torch.rand(n, H, generator=g)
+    state = torch.randn(2, H, dk, dv, generator=g)
+
+    def run(lo, locs):
+        x = [y[lo:].contiguous().to(DEV) for y in (q, k, v, a, b)]
+        st = state.to(DEV)
+        f = hops.delta_scan if delta else hops.decay_scan
+        more = () if delta else (None,)
+        return f(*x, *more, st, slots, locs.to(DEV), total), st
+
+    got, st = run(0, qlocs + front)
+    want, end = run(front, qlocs)
+    assert torch.equal(got[front:], want)
+    assert torch.equal(st, end)
