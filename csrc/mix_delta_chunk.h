@@ -29,7 +29,13 @@
 // in delta_pairs: adding the halves of a product with LDS atomics (328 instead of 235
 // us), two channels of eight tokens a lane; in delta_chunks: loading the next chunk's
 // rows at once (443 us instead of 380 for 16 heads), K- through the transposed read.
-// Errors against 64 bits at those sizes: read-out 1.3e-7 and 9.8e-8, state 6.8e-8 both.
+// Errors against 64 bits, scan and chunks: at those sizes read-out 1.3e-7 and 9.8e-8,
+// state 6.8e-8 both; 4096 tokens of the same decay, 0.9987654 or 0.99987, beta 0.02 to
+// 0.98, independent keys, keys behind silu, keys that resemble each other, keys that
+// leave half of the channels alone: read-out 2.7e-7 to 1.4e-6 and 1.2e-7 to 3.2e-7,
+// state 2.1e-7 to 2.2e-6 and 9.7e-8 to 2.9e-7. Larger than the scan's are those of keys
+// that resemble each other (cosine 0.9) with beta 0.98 and decays that change, 1.4e-7
+// and 2.1e-7: there u_t is the small difference of large numbers of S0.
 #pragma once
 
 #include "mix_chunk.h"
@@ -63,6 +69,22 @@ template <int PLANE>
 __device__ __forceinline__ void dc_put(char* p, float x, float y) {
 #pragma unroll
   for (int n = 0; n < 3; ++n) *(u32*)(p + n * PLANE) = ch_term(x, y);
+}
+
+// A product of decays times one more, and what its roundings left out (of first
+// order). The state is multiplied by a product in every chunk, and where the decays
+// stay the same, so does its rounding: over 4096 tokens of 0.9987654 errors were 2 to 9
+// times the scan's (beta 0.02, keys that resemble each other: state 8.2e-6 and 9.4e-7).
+// So what the product of a chunk lacks is handed on to that of the next (2.3e-7). It
+// costs nothing where the chip is full and 1 % for one row of 4000 tokens; a second
+// factor in the consumers took 5 % there.
+__device__ __forceinline__ void dc_times(f32x2& p, f32x2& lost, f32x2 d) {
+#pragma clang fp contract(off)    // (the product is the rounded one also behind this)
+  const f32x2 x = p * d;
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    lost[e] = fmaf(lost[e], d[e], fmaf(p[e], d[e], -x[e]));
+  p = x;
 }
 
 // ---- pairs of tokens -----------------------------------------------------------
@@ -396,7 +418,7 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
   struct Lds {
     char kp[3 * PLANE], qp[3 * PLANE], km[3 * PLANE];
     char m[3 * WPLANE], b[3 * WPLANE];
-    float tot8[2][4][DK], all[DK], beta[CH_T];
+    float tot8[2][2][4][DK], all[DK], beta[CH_T];   // (products over 8: hi, lo)
   };
   extern __shared__ __attribute__((aligned(16))) char dc_lds[];
   Lds& L = *(Lds*)dc_lds;
@@ -433,6 +455,7 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
     const u32 off = in ? ch * 4u : CH_OUT;
     f32x2 rk[8], rq[8], rd[8], rm[8];    // loaded rows; K- on its way
     f32x4 rp[2];                         // pairs on their way
+    f32x2 owed = (f32x2)(0.f);           // by the last chunk's product, as a part of it
     float rb = 0.f;                      // and beta (wave 2)
     auto fetch_d = [&](int c) {
       const long row = ch_plain(q0 + c * CH_T);
@@ -487,13 +510,21 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
 #pragma unroll
       for (int r = 0; r < 8; ++r)
         if (r >= left) rd[r] = (f32x2)(1.f);
+      // what the products behind the first lose (see dc_times)
+      f32x2 lost = (f32x2)(0.f);
       pre[0] = rd[0];
 #pragma unroll
-      for (int r = 1; r < 8; ++r) pre[r] = pre[r - 1] * rd[r];
+      for (int r = 1; r < 8; ++r) {
+        pre[r] = pre[r - 1];
+        dc_times(pre[r], lost, rd[r]);
+      }
       suf[7] = (f32x2)(1.f);
 #pragma unroll
       for (int r = 6; r >= 0; --r) suf[r] = suf[r + 1] * rd[r + 1];
-      if (DK == 128 || lane < 32) *(f32x2*)&L.tot8[c & 1][pw][ch] = pre[7];
+      if (DK == 128 || lane < 32) {
+        *(f32x2*)&L.tot8[c & 1][0][pw][ch] = pre[7];
+        *(f32x2*)&L.tot8[c & 1][1][pw][ch] = lost;
+      }
     };
     // K+ and Q+ into LDS, K- into registers; rows of the next chunk take the place of
     // those that are done (loads all at once would wait for the memory)
@@ -503,7 +534,7 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const f32x2 t = DK == 128 || lane < 32
-                            ? *(const f32x2*)&L.tot8[c & 1][i][ch] : (f32x2)(1.f);
+                            ? *(const f32x2*)&L.tot8[c & 1][0][i][ch] : (f32x2)(1.f);
         if (i < pw) before *= t;
         if (i > pw) behind *= t;
       }
@@ -557,9 +588,22 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
       if (pw < 2) put_pairs(pw + 4, rp[1]);
       if (pw == 2 && lane < 32) L.beta[lane] = rb;
       if (pw == 3 && (DK == 128 || lane < 32)) {
-        f32x2 t = (f32x2)(1.f);
+        f32x2 t = *(const f32x2*)&L.tot8[c & 1][0][0][ch];
+        f32x2 lost = *(const f32x2*)&L.tot8[c & 1][1][0][ch];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) t *= *(const f32x2*)&L.tot8[c & 1][i][ch];
+        for (int i = 1; i < 4; ++i) {
+          const f32x2 y = t * *(const f32x2*)&L.tot8[c & 1][1][i][ch];
+          dc_times(t, lost, *(const f32x2*)&L.tot8[c & 1][0][i][ch]);
+          lost += y;
+        }
+        // what this product lacks goes into the next chunk's
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float more = fmaf(t[e], owed[e], lost[e]), all = t[e] + more;
+          owed[e] = fabsf(all) > 1e-30f
+                        ? (t[e] - all + more) * __builtin_amdgcn_rcpf(all) : 0.f;
+          t[e] = all;
+        }
         *(f32x2*)&L.all[ch] = t;
       }
       if (c + 1 < steps) {
@@ -729,7 +773,7 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
 template <int DK, bool HEAD, int NC>
 static void delta_chunks_go(DeltaChunkArgs A, hipStream_t s) {
   constexpr int bytes =
-      9 * CH_T * DK * 2 + 6 * CH_T * CH_T * 2 + (2 * 4 + 1) * DK * 4 + CH_T * 4;
+      9 * CH_T * DK * 2 + 6 * CH_T * CH_T * 2 + (2 * 2 * 4 + 1) * DK * 4 + CH_T * 4;
   static std::atomic<unsigned long long> asked{0};
   const auto fn = delta_chunks_kernel<DK, HEAD, NC>;
   lds_limit((const void*)fn, bytes, asked);

@@ -277,3 +277,49 @@ def test_tokens_in_front_of_the_first_sequence(front, delta):
     want, end = run(front, qlocs)
     assert torch.equal(got[front:], want)
     assert torch.equal(st, end)
+
+
+@pytest.mark.parametrize("head", [False, True])
+def test_delta_decays_that_stay_the_same(head):
+    """The rounding of a product of decays is the same in every chunk then, and must not
+    add up: 128 chunks whose products are off by a third of 2^-24 each, one way, are
+    8e-6 off for keys that resemble each other and a small beta. Roundings both ways
+    stay below TOL."""
+    g = torch.Generator().manual_seed(8)
+    H, dk, dv, T = 2, 64, 16, 4096
+    unit = torch.nn.functional.normalize
+    q = unit(torch.randn(T, H, dk, generator=g), dim=-1) * dk ** -0.5
+    k = unit(torch.randn(1, H, dk, generator=g)
+             + 0.3 * torch.randn(T, H, dk, generator=g), dim=-1)
+    v = torch.randn(T, H, dv, generator=g)
+    d = torch.full((T, H) if head else (T, H, dk), 0.9987654)
+    beta = torch.full((T, H), 0.02)
+    state = torch.randn(1, H, dk, dv, generator=g)
+    qlocs = torch.tensor([0, T], dtype=torch.int32)
+    total, slots = torch.tensor([T + 1]).int(), torch.tensor([0]).int()
+    want, end = _delta(q, k, v, d[..., None].expand(T, H, dk) if head else d, beta,
+                       state, qlocs, total, slots)
+    st = state.to(DEV)
+    o = hops.delta_scan(*(x.to(DEV) for x in (q, k, v, d, beta)), st, slots.to(DEV),
+                        qlocs.to(DEV), total.to(DEV))
+    assert _off(o, want) < TOL
+    assert _off(st, end) < TOL
+
+
+@pytest.mark.parametrize("decay", [0.9987654, 0.99987])
+def test_decays_that_stay_the_same(decay):
+    g = torch.Generator().manual_seed(9)
+    H, dk, dv, T = 2, 64, 16, 8192
+    q, k = (torch.randn(T, H, dk, generator=g) * dk ** -0.5 for _ in "qk")
+    v = torch.randn(T, H, dv, generator=g)
+    a = torch.full((H,), decay)
+    state = torch.randn(1, H, dk, dv, generator=g)
+    qlocs = torch.tensor([0, T], dtype=torch.int32)
+    total, slots = torch.tensor([T + 1]).int(), torch.tensor([0]).int()
+    want, end = _recur(q, k, v, a.expand(T, H), torch.ones(T, H), torch.zeros(H), state,
+                       qlocs, total, slots)
+    st = state.to(DEV)
+    o = hops.decay_scan(q.to(DEV), k.to(DEV), v.to(DEV), a.to(DEV), None, None, st,
+                        slots.to(DEV), qlocs.to(DEV), total.to(DEV))
+    assert _off(o, want) < TOL
+    assert _off(st, end) < TOL
