@@ -56,7 +56,10 @@ def test_kernel(M, N, K):
 @pytest.mark.parametrize("M,N,K", [
     (9, 4100, 4096), (16, 8200, 2048), (30, 16400, 512), (32, 33000, 256),
     (40, 8300, 1024), (64, 16500, 768), (50, 33000, 512), (100, 8300, 1024),
-    (128, 16600, 512), (90, 33000, 256), (180, 12000, 512), (250, 16000, 512)])
+    (128, 16600, 512), (90, 33000, 256), (180, 12000, 512), (250, 16000, 512),
+    # starts at eighths of k
+    (20, 16400, 2048), (31, 33000, 2048), (60, 9000, 4096), (64, 33000, 2048),
+    (100, 9000, 2048), (128, 16600, 2048), (128, 33000, 4096)])
 def test_larger_tiles(M, N, K):
     check(M, K, N, False)
     check(M, K, N // 8 * 4, True)
