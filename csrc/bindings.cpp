@@ -62,6 +62,7 @@ void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
                     hipStream_t);
 void sutro_linear_mid(void*, const void*, long, const void*, const void*, int, int,
                       int, int, hipStream_t);
+void sutro_mid_tile(int*, int, int, int, int);
 void sutro_linear_skinny(void*, long, const void*, long, const void*,
                          const void*, int, int, int, int, hipStream_t);
 long mix_moe_dispatch_scratch(long, int);
@@ -385,6 +386,13 @@ torch::Tensor linear_mid(torch::Tensor x, torch::Tensor w,
   return out;
 }
 
+// rows of x and of w (`rows` in all) in a tile of linear_mid
+std::vector<long> mid_tile(long M, long rows, long K, bool gated) {
+  int t[2];
+  sutro_mid_tile(t, (int)M, (int)(gated ? rows / 2 : rows), (int)K, gated ? 1 : 0);
+  return {t[0], t[1]};
+}
+
 // (y w^T or, `gated`, its silu unit; x + residual), y the RMSNorm of x + residual,
 // one row
 std::vector<torch::Tensor> norm_linear(torch::Tensor x, torch::Tensor residual,
@@ -500,6 +508,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma16_probe", &mfma16_probe, "16x16 MFMA fragment-layout probe");
   m.def("moe_combine", &moe_combine, "fused MoE weighted gather-combine");
   m.def("linear_skinny", &linear_skinny, "linear layer over few rows");
+  m.def("mid_tile", &mid_tile, "tile of linear_mid");
   m.def("linear_mid", &linear_mid, "linear layer over 2 to 256 rows");
   m.def("norm_linear", &norm_linear,
         "linear layer of one row behind an addition and RMSNorm");

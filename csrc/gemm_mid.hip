@@ -232,38 +232,57 @@ static void mid_go(MidArgs A, hipStream_t s) {
                      dim3(256 * KG), bytes, s, A);
 }
 
-// the smallest tile of which 256 or fewer make M rows by `rows` of w; of more weight
-// rows than that, tiles of 128 that leave two workgroups a CU
-template <bool GATED>
-static void mid_pick(const MidArgs& A, hipStream_t s) {
-  const long rows = GATED ? 2L * A.N : A.N;
+// The smallest tile of which 256 or fewer make M rows by `rows` of w; of more weight
+// rows than that, tiles of 128. (ops._mid_tile is the same choice: the sizes that come
+// here depend on it.)
+template <bool GATED, typename GO>
+static void mid_pick(int M, int N, int K, GO go) {
+  const long rows = GATED ? 2L * N : N;
   auto fit = [&](int bm, int bn) {
-    return ((A.M + bm - 1) / bm) * ((rows + bn - 1) / bn) <= 256;
+    return ((M + bm - 1) / bm) * ((rows + bn - 1) / bn) <= 256;
   };
   if constexpr (!GATED) {
     // (long rows of few weights: 4096 x 4096 at 16 rows 11.2 us on 64 x 16, 11.7)
-    if (A.M <= 32 && !(A.M > 8 && A.K >= 4096 && fit(64, 16)) && fit(32, 32))
-      return mid_go<32, 32, 256, 4, 2, 2, false>(A, s);
-    if (fit(64, 16)) return mid_go<64, 16, 256, 4, 4, 2, false>(A, s);
+    if (M <= 32 && !(M > 8 && K >= 4096 && fit(64, 16)) && fit(32, 32))
+      return go.template tile<32, 32, 256, 4, 2, 2, false>();
+    if (fit(64, 16)) return go.template tile<64, 16, 256, 4, 4, 2, false>();
   }
-  if (fit(64, 32) && (GATED || A.M > 32))
-    return mid_go<64, 32, 256, 3, 4, 2, GATED>(A, s);
-  if (A.M <= 32) {
-    if (fit(32, 64)) return mid_go<32, 64, 128, 3, 2, 1, GATED>(A, s);
-    if (fit(32, 128)) return mid_go<32, 128, 128, 4, 2, 2, GATED>(A, s);
-    return mid_go<32, 128, 128, 2, 2, 1, GATED>(A, s);
+  if (fit(64, 32) && (GATED || M > 32))
+    return go.template tile<64, 32, 256, 3, 4, 2, GATED>();
+  if (M <= 32) {
+    if (fit(32, 64)) return go.template tile<32, 64, 128, 3, 2, 1, GATED>();
+    if (fit(32, 128)) return go.template tile<32, 128, 128, 4, 2, 2, GATED>();
+    return go.template tile<32, 128, 128, 2, 2, 1, GATED>();       // two a CU
   }
-  if (fit(64, 64)) return mid_go<64, 64, 128, 5, 2, 2, GATED>(A, s);
-  if (A.M <= 64) {
-    if (fit(64, 128)) return mid_go<64, 128, 128, 3, 2, 2, GATED>(A, s);
-    return mid_go<64, 128, 64, 3, 2, 1, GATED>(A, s);
+  if (fit(64, 64)) return go.template tile<64, 64, 128, 5, 2, 2, GATED>();
+  if (M <= 64) {
+    if (fit(64, 128)) return go.template tile<64, 128, 128, 3, 2, 2, GATED>();
+    return go.template tile<64, 128, 64, 3, 2, 1, GATED>();        // two a CU
   }
-  if (A.M <= 128 || A.M > 192) {
-    if (fit(128, 64)) return mid_go<128, 64, 128, 3, 2, 2, GATED>(A, s);
+  if (M <= 128 || M > 192) {
+    if (fit(128, 64)) return go.template tile<128, 64, 128, 3, 2, 2, GATED>();
   } else if (fit(64, 128)) {
-    return mid_go<64, 128, 128, 3, 2, 2, GATED>(A, s);
+    return go.template tile<64, 128, 128, 3, 2, 2, GATED>();
   }
-  mid_go<128, 128, 64, 5, 2, 1, GATED>(A, s);
+  go.template tile<128, 128, 64, 5, 2, 1, GATED>();
+}
+
+struct MidLaunch {
+  const MidArgs& A;
+  hipStream_t s;
+  template <int BM, int BN, int BK, int ST, int WR, int KG, bool GATED>
+  void tile() const { mid_go<BM, BN, BK, ST, WR, KG, GATED>(A, s); }
+};
+struct MidSize {
+  int* out;
+  template <int BM, int BN, int BK, int ST, int WR, int KG, bool GATED>
+  void tile() const { out[0] = BM; out[1] = BN; }
+};
+
+// rows of x and of w in a tile
+extern "C" void sutro_mid_tile(int* out, int M, int N, int K, int gated) {
+  if (gated) mid_pick<true>(M, N, K, MidSize{out});
+  else mid_pick<false>(M, N, K, MidSize{out});
 }
 
 // x and w at multiples of 16 bytes, ldx a multiple of 8, K of 256, N of 4; offsets within
@@ -273,6 +292,6 @@ extern "C" void sutro_linear_mid(void* out, const void* x, long ldx, const void*
                                  hipStream_t stream) {
   const MidArgs A = {(u16*)out, (const u16*)x, (const u16*)w, (const u16*)bias,
                      M, N, K, ldx, 0, 0, 0};
-  if (gated) mid_pick<true>(A, stream);
-  else mid_pick<false>(A, stream);
+  if (gated) mid_pick<true>(M, N, K, MidLaunch{A, stream});
+  else mid_pick<false>(M, N, K, MidLaunch{A, stream});
 }

@@ -8,6 +8,7 @@ hot path.
 
 from __future__ import annotations
 
+import functools
 import os
 from typing import Optional
 
@@ -292,48 +293,161 @@ def _few_rows(x, w, gated: bool = False) -> bool:
                      and (x.requires_grad or w.requires_grad)))
 
 
+def _mid_tile(M: int, rows: int, K: int, gated: bool):
+    """Rows of x and of w in a tile of csrc/gemm_mid.hip (its mid_pick), and how many
+    tiles there are."""
+    def tiles(m, n):
+        return -(-M // m) * -(-rows // n)
+    if M <= 32:
+        if not gated:
+            t = tiles(64, 16)
+            if tiles(32, 32) <= 256 and not (M > 8 and K >= 4096 and t <= 256):
+                return 32, 32, tiles(32, 32)
+            if t <= 256:
+                return 64, 16, t
+        sizes = ((64, 32), (32, 64)) if gated else ((32, 64),)
+        last = 32, 128
+    else:
+        sizes = ((64, 32), (64, 64)) if gated else ((64, 16), (64, 32), (64, 64))
+        last = (64, 128) if M <= 64 else (128, 128)
+        if M > 64:
+            sizes += ((64, 128),) if 128 < M <= 192 else ((128, 64),)
+    for m, n in sizes:
+        if tiles(m, n) <= 256:
+            return m, n, tiles(m, n)
+    return *last, tiles(*last)
+
+
+@functools.lru_cache(maxsize=4096)
 def _mid_sizes(M: int, rows: int, K: int, gated: bool) -> bool:
-    """The sizes of `_mid_rows` at which csrc/gemm_mid.hip is ahead."""
-    if K <= 4096:
-        if M == 2:
-            if K <= 1024:
-                return rows >= (4096 if gated else 32) and rows <= 65536
-            return 6144 <= rows <= 65536 and (
-                K <= 2048 or (not gated and rows <= 32768))
-        if M <= 12:                       # from 513 to 1024 of k: short chains
-            if K <= 1024:
-                return K > 512 and rows >= 10240
-            if K > 3072 and (rows <= 5120 or (gated and 12288 < rows <= 20480)):
-                return False
-            return rows >= 4096
-        if M <= 16:
-            return rows >= (10240 if K <= 512 else 2048 if K <= 1024 else 32)
-        if rows < 512 and K > 2048:
+    """The sizes of `_mid_rows` at which csrc/gemm_mid.hip is ahead: ranges of k and of
+    weight rows, as the table there shows, and by the round: not where tiles of 128
+    weight rows are a few more than the 256 CUs (or 512, two a CU), and not where larger
+    tiles leave a third of the CUs without one while the library's smaller ones fit. us
+    of the other side and of the kernel there:
+      30 x 36512 x 3072        49.7 / 52.5      54 x 36224 x 3584        57.1 / 66.2
+      48 x 39952 x 4096        70.8 / 74.9       9 x 44368 x 3584        58.2 / 61.3
+       8 x 71840 x  768        26.0 / 28.0       3 x 66672 x 2048        53.4 / 58.9
+      87 x  2432 x 4096        11.0 / 11.8     141 x  1472 x 3584        10.0 / 10.8
+     122 x  9440 x 3072        24.1 / 25.1     240 x  4544 x 3840        25.7 / 28.5
+     186 x  6224 x 3584        24.3 / 28.2     213 x 16336 x 3840 gated  48.5 / 54.0
+       4 x  6528 x 3584 gated  12.3 / 12.9       6 x  2400 x 5120         8.2 /  9.7
+    Of 7500 sizes drawn from those left 6 were 3 to 5 % slower than without the kernel.
+    The largest output layers: 151936 x 2048 at 7 to 16 rows 204 / 112, at 32 rows 147 /
+    114; 151936 x 4096 at 3 to 64 rows 244 to 266 / 217 to 229; 151936 x 1024 at 3 to 16
+    rows 59 to 61 / 58 to 61."""
+    bm, bn, n = _mid_tile(M, rows, K, gated)
+    if K > 4096:
+        return _mid_long(M, rows, K, gated, bm, bn, n)
+    if M <= 16:
+        return _mid_16(M, rows, K, gated, bn, n)
+    if rows < 512 and K > 2048:
+        return False
+    if M <= 64:
+        if bn < 128 or n <= 256:
+            return True
+        if M <= 32:                       # (two tiles a CU)
+            if n <= (304 if K > 2048 else 288) and K >= 1024 and K != 2048:
+                return gated and (K <= 2048 or K == 4096)
+            return n <= 288 or K % 2048 == 0
+        if K == 4096:
+            return n > (288 if gated else 352)
+        return K == 2048 or (n <= 288 and K <= (2048 if gated else 512))
+    if bm == bn == 128:
+        if n > 256 or K > 3072 or (K > 2560 and M > 192):
             return False
-        if M <= 64:
-            return rows <= 36864 or K % 2048 == 0
         if M <= 128:
-            return rows <= 16384 or (M >= 96 and 28672 <= rows <= 32768
-                                     and K % 2048 == 0)
-        if M <= 192:
-            return rows <= 10240 or (gated and 15360 <= rows <= 16384
-                                     and K <= 2048)
-        return rows <= 8192 or (gated and 12800 <= rows <= 16384)
+            return M >= 96 and n >= 224 and K % 2048 == 0
+        return gated and n >= (200 if M > 192 else 240) and (M > 192 or K <= 2048)
+    if bn == 128 and n > 240:
+        return False
+    return gated or _mid_beside(M, rows, K, bm, bn, n)
+
+
+def _mid_beside(M, rows, K, bm, bn, n) -> bool:
+    """More than 64 rows, one round: beside the library's tiles, of which one of 32 x 32
+    also takes 65 to 96, 129 to 160 or 193 to 224 rows without padding."""
+    if bn == 32:
+        return K <= 2560 or -(-M // 32) * -(-rows // 32) > 256
+    if bm == 128:
+        return K <= 2048 or n >= 192 or (M <= 96 if M <= 128 else
+                                         M <= 224 and n <= 144)
+    if bn == 128:
+        return K <= 1536 or n >= 204 or (M <= 160 and n <= 147)
+    return True
+
+
+def _mid_16(M, rows, K, gated, bn, n) -> bool:
+    """2 to 16 rows, a k of up to 4096."""
+    if bn == 128:                         # two a CU: the beginning of a round
+        if M == 2 and 256 < n <= 320 and K > 1024:
+            return False
+        if M > 8 and 256 < n <= 288 and 1024 <= K < 2048 and not gated:
+            return False
+        if M > 2 and 320 < n <= 384 and 3072 <= K < 4096 and not gated:
+            return False
+        if M > 2 and 512 < n <= 592 and (
+                (K == 768 and not gated) or (n <= 544 and M <= 8 and (
+                    K == 1024 or K > 3328 or (K == 2048 and M <= 4)))):
+            return False
+        if 2 < M <= 5 and n <= 160 and K <= 1280 and not gated:
+            return False
+    if M == 2:
+        if K <= 1024:
+            return rows >= (4096 if gated else 32) and rows <= 65536
+        return 6144 <= rows <= 65536 and (
+            K <= 2048 or (not gated and rows <= 32768 and not 8192 < rows <= 9216))
+    if M <= 12:
+        if gated and bn == 32 and K > 1024 and n > (
+                128 if M <= 8 else 192 if K <= 1536 else 256):
+            return False                  # (the other kernel for few rows)
+        if K <= 1024:                     # from 513 to 1024 of k: short chains
+            return K > 512 and rows >= 10240
+        if K <= 1280 and 7168 < rows <= 8192:
+            return False
+        if K > 3072 and (rows <= 5120 or (gated and 12288 < rows <= 20480)):
+            return False
+        return rows >= 4096 + (K > 2048)
+    if K <= 1280 and M <= 14 and rows <= 2560:
+        return False
+    return rows >= (10240 if K <= 512 else 8208 if K < 1024
+                    else 2048 if K <= 1024 else 32)
+
+
+def _mid_long(M, rows, K, gated, bm, bn, n) -> bool:
+    """A k of more than 4096: one workgroup has all of it."""
     if K <= 5120:
         if M <= 16:
-            return M > 3 and (
-                ((512 if M <= 8 else 4096) <= rows <= 6144 and not gated)
-                or 16384 <= rows <= 40960)
+            if M <= 3:
+                return False
+            if gated or rows > 6144:
+                return 16384 <= rows <= 32768
+            return rows > 4096 or (M <= 8 and 512 <= rows < 2304)
         if M <= 64:
             return 512 <= rows <= 8192 or 16384 <= rows <= 32768
-        return 2048 <= rows <= (10240 if 128 < M <= 192 else 8192)
-    if K <= 6144:
-        return 16 < M <= 128 and 4096 <= rows <= 8192
-    if K >= 16384 and M > 32:
+        if not 2048 <= rows <= (10240 if 128 < M <= 192 else 8192):
+            return False
+        if gated:
+            return bm < 128 or n >= 192
+    elif K <= 6144:
+        if not (16 < M <= 128 and 4096 <= rows <= 8192):
+            return False
+    elif K >= 16384 and M > 32:
         return 2048 <= rows <= 6144
-    return 64 < M <= 192 and (
-        4096 if gated or K > 8192 else 2048) <= rows <= 6144 and not (
-        gated and K > 8192)
+    else:
+        if not (64 < M <= 192 and rows <= 6144) or (gated and K > 8192):
+            return False
+        if rows < (4096 if gated or K > 8192 else 2048):
+            return False
+        if bn == 128:
+            return M <= 160 and (gated or n <= 147)
+        if bn == 64 and (n < 176 or (K == 10240 and M > 160)):
+            return False
+    if gated or M <= 64:
+        return True
+    if bm == bn == 64 and K <= 6144 and -(-M // 32) % 2:
+        return n >= (160 if M <= 96 else 145)
+    return _mid_beside(M, rows, K, bm, bn, n)
 
 
 def _mid_rows(x, w, gated: bool = False) -> bool:
@@ -358,9 +472,9 @@ def _mid_rows(x, w, gated: bool = False) -> bool:
       4096 x 8192       1.05  1.05  1.07  1.09  0.99  0.88  0.64  0.60  1.03
       4096 x 12288      1.26  1.25  1.32  1.28  1.10  0.95  0.65  0.65  1.08
       4096 x 25600      1.25  1.23  1.13  0.98  0.74  0.44  0.64  0.77  0.66
-    It loses where few weights are long rows (one workgroup has all of k), where
-    128 x 128 tiles of many rows leave more than one round, and to the kernel for
-    few rows where that one is quickest."""
+    It loses where few weights are long rows (one workgroup has all of k), where a
+    round is filled badly (`_mid_sizes`), and to the kernel for few rows where that
+    one is quickest."""
     if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False
@@ -369,7 +483,8 @@ def _mid_rows(x, w, gated: bool = False) -> bool:
     M, K = x.shape
     rows = w.shape[0]
     return (K % 256 == 0 and 512 <= K < 1 << 20 and rows > 0
-            and _mid_sizes(M, rows, K, gated) and _unwatched() and x.dtype == torch.bfloat16
+            and _mid_sizes(M, rows, K, gated) and _unwatched()
+            and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.device == x.device
             and w.dim() == 2 and w.shape[1] == K
             and rows % (16 if gated else 4) == 0 and rows < 1 << 24

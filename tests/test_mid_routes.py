@@ -64,3 +64,36 @@ def test_sizes_the_kernel_refuses(on_gpu, M, K, rows, gated):
     x = torch.empty(M, K, dtype=torch.bfloat16, device="meta")
     w = torch.empty(rows, K, dtype=torch.bfloat16, device="meta")
     assert not ops._mid_rows(x, w, gated)
+
+
+def test_the_rule_knows_the_kernels_tiles():
+    if ops._C is None:
+        pytest.skip("extension not built")
+    for M in (2, 8, 9, 16, 31, 32, 33, 64, 65, 96, 128, 129, 150, 192, 193, 256):
+        for K in (512, 2048, 4096, 5120):
+            for rows in (16, 1024, 1040, 2048, 2064, 4096, 4112, 5456, 5472, 8192,
+                         8208, 10880, 10896, 16384, 16400, 32768, 32784, 151936):
+                for gated in (False, True):
+                    m, n, tiles = ops._mid_tile(M, rows, K, gated)
+                    assert [m, n] == ops._C.mid_tile(M, rows, K, gated)
+                    assert tiles == -(-M // m) * -(-rows // n)
+
+
+@pytest.mark.parametrize("M,K,rows,gated,kernel", [
+    (30, 3072, 36512, False, 0), (30, 3072, 32768, False, 1),
+    (54, 3584, 36224, False, 0), (54, 3584, 32768, False, 1),
+    (48, 4096, 39952, False, 0), (48, 4096, 51200, False, 1),
+    (9, 3584, 44368, False, 0), (9, 4096, 44368, False, 1),
+    (8, 768, 71840, False, 0), (8, 768, 65536, False, 1), (3, 2048, 66672, False, 0),
+    (87, 4096, 2432, False, 0), (87, 4096, 2752, False, 1), (87, 4096, 2432, True, 1),
+    (97, 4096, 2432, False, 1), (171, 3584, 1472, False, 1), (141, 3584, 1472, False, 0),
+    (122, 3072, 9440, False, 0), (122, 3072, 12288, False, 1), (90, 3072, 9440, False, 1),
+    (240, 3840, 4544, False, 0), (240, 3840, 6144, False, 1), (186, 3584, 6224, False, 0),
+    (150, 3584, 6224, False, 1), (186, 3584, 6224, True, 1),
+    (213, 3840, 16336, True, 0), (213, 2048, 16336, True, 1),
+    (6, 5120, 2288, False, 1), (6, 5120, 4096, False, 0), (14, 768, 4096, False, 0),
+    (4, 3584, 6528, True, 0), (80, 8192, 5056, False, 0), (80, 8192, 5696, False, 1)])
+def test_rounds(on_gpu, M, K, rows, gated, kernel):
+    """Tiles that begin a round with few of them, or leave a third of the CUs without
+    one, where the library's tiles fit."""
+    assert ops._mid_rows(bf(M, K), bf(rows, K), gated) == bool(kernel)
