@@ -199,7 +199,9 @@ def _two_rows(rows: int, K: int, gated: bool) -> bool:
 
 
 def _long_weights(M: int, rows: int, K: int) -> bool:
-    """Larger matrices over 3 to 32 rows (both sides in `_few_rows`)."""
+    """Larger matrices over 3 to 32 rows (both sides in `_few_rows`). Nearly all with a
+    k that is a multiple of 256 and not above 4096 go to csrc/gemm_mid.hip before they
+    come here; this decides for the others."""
     if 16384 < rows <= 24576 and rows * K <= 80 << 20 and K <= 4096:
         return M <= 16                    # the library has no good tile there
     if rows <= 8192 and K <= 4096:
@@ -267,10 +269,14 @@ def _few_rows(x, w, gated: bool = False) -> bool:
       12288 x 8192     43.9 / 42.4    43.8 / 47.5
       51200 x 5120     98.8 / 92.3    99.1 / 95.9   95.6 / 134    92.3 / 139    92.8 / 158    95.8 / 196
     Two rows lose where the library has a good tile (24 to 64 M weights of long
-    rows) and one load a weight row is no longer the whole cost. The line is on
-    the library's side of some sizes at which the kernel is ahead: 7 to 16 rows
-    over 151936 x 2048, 13 to 16 over 8192 x 3072 or, with the unit, 16384 x
-    2048 (the sizes between them have not been tried)."""
+    rows) and one load a weight row is no longer the whole cost.
+
+    `linear` asks `_mid_rows` first. Of the sizes above csrc/gemm_mid.hip takes those
+    with a k of 512 to 4096 at 32 rows and of 1024 to 4096 at 16 (few weight rows apart),
+    and at 2, 3 and 8 rows most from 4096 or 6144 weight rows on; the figures there are
+    what it was measured against. With a k that is no multiple of 256 such sizes still
+    come here. For those the line is on the library's side of some: beside 7 to 16 rows
+    over 151936 x 2048 and 13 to 16 over 8192 x 3072."""
     if (type(x) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)):
         return False

@@ -194,3 +194,37 @@ def test_larger_matrices(kernels, rows, k, n, kernel):
     w = torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
     assert ops._few_rows(torch.empty(rows, k, dtype=torch.bfloat16),
                          w) == bool(kernel)
+
+
+class _Names(_Kernels):
+    """The same, with the name of the kernel instead of its result."""
+
+    def linear_skinny(self, x, w, bias, gated):
+        return "few"
+
+    def linear_mid(self, x, w, bias, gated):
+        return "mid"
+
+
+@pytest.mark.parametrize("rows,k,n,kernel", [
+    # the sizes above
+    (16, 4096, 20480, "mid"), (16, 4096, 20720, "mid"), (8, 4096, 20720, "mid"),
+    (8, 4096, 14336, "mid"), (6, 4096, 14336, "mid"), (8, 4096, 40960, "mid"),
+    (8, 4096, 59344, "mid"), (6, 4096, 59344, "mid"), (8, 4096, 65536, "mid"),
+    (5, 4096, 113184, "mid"), (6, 2048, 151936, "mid"), (8, 2048, 59424, "mid"),
+    (2, 5120, 10240, "few"), (2, 4096, 6144, "mid"), (3, 25600, 5120, "few"),
+    (32, 25600, 2048, "few"), (32, 17408, 128, "lib"), (16, 25600, 64, "few"),
+    # where the first kernel is not ahead, and a k that it does not take
+    (8, 4096, 66560, "lib"), (6, 4096, 66560, "lib"), (4, 4096, 66560, "few"),
+    (8, 2048, 4080, "few"), (8, 4096, 4096, "few"), (32, 4096, 32, "lib"),
+    (12, 4064, 4096, "few"), (13, 4064, 4096, "few"), (13, 4064, 8192, "lib"),
+    (8, 1600, 59424, "lib"), (8, 2016, 20000, "few"), (8, 2016, 151936, "lib"),
+    (33, 4064, 4096, "lib"), (33, 4096, 4096, "mid"), (257, 4096, 4096, "lib")])
+def test_the_kernel_that_is_called(monkeypatch, rows, k, n, kernel):
+    """Both rules one behind the other, as ops.linear asks them."""
+    monkeypatch.setattr(ops, "_use_hip", lambda t: True)
+    monkeypatch.setattr(ops, "_require_hip", _Names)
+    monkeypatch.setattr(F, "linear", lambda x, w, bias=None: "lib")
+    with torch.no_grad():
+        assert ops.linear(torch.empty(rows, k, dtype=torch.bfloat16),
+                          torch.empty(n, k, dtype=torch.bfloat16)) == kernel
