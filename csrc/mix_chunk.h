@@ -620,19 +620,21 @@ __global__ void __launch_bounds__(768, 3) chunk_scan_kernel(const ChunkArgs A) {
 
 // New tokens from which a sequence goes through chunks; the scans keep the shorter
 // ones of the same batch (single tokens among them: state in, state out, for which
-// one workgroup a CU is too few). 0: no sequence of the batch can be long enough, or
-// rows that are not in whole 16-byte (8-byte) pieces. Measured, scan and chunks, us:
+// one workgroup a CU is too few). 0: no sequence of the batch can be long enough,
+// rows that are not in whole 16-byte (8-byte) pieces, or rows less than a head apart
+// (one row for all tokens): what a chunk may read ends a row's distance behind its last
+// row. Measured, scan and chunks, us:
 // dk 128, 16 heads x 256 rows of 10 tokens 185 and 268, 64 rows of 10 49 and 67, 1
 // row of 40 22 and 20, 4 rows of 100 44 and 30; dk 64, 4 rows of 16 9 to 14 and 8 to
 // 10, 64 of 10 12 and 14; MLSTM, 64 rows of 10 47 and 35, 256 rows of 1 91 and 115.
 static inline int chunk_scan_least(int dk, long ldq, long ldk, long ldv, long ldo,
-                                   const void* q, const void* k, int align,
-                                   bool mlstm, long T, int S) {
+                                   const void* q, const void* k, int dv,
+                                   int align, bool mlstm, long T, int S) {
   const int least = mlstm ? 8 : (dk <= 64 ? 16 : 32);
   const long most = 1 << 23;               // 32 rows within 2^31 bytes
   if (dk > 128 || dk % 4 || ldq % 4 || ldk % 4 || (size_t)q % align ||
       (size_t)k % align || ldq >= most || ldk >= most || ldv >= most ||
-      ldo >= most || T < S + least - 1)
+      ldo >= most || ldq < dk || ldk < dk || ldv < dv || T < S + least - 1)
     return 0;
   return least;
 }

@@ -436,7 +436,8 @@ extern "C" int mix_decay_scan(float* o, const float* q, long ldq,
                               hipStream_t s) {
   if (S == 0) return 1;
   const int least =
-      chunk_scan_least(dk, ldq, ldk, ldv, (long)H * dv, q, k, 16, false, T, S);
+      chunk_scan_least(dk, ldq, ldk, ldv, (long)H * dv, q, k, dv, 16, false, T,
+                       S);
   if (least) {
     ChunkArgs a = {};
     a.o = o; a.q = q; a.k = k; a.v = v;

@@ -264,7 +264,7 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
   const u16* p = (const u16*)proj;
   const int least =
       f32 ? 0 : chunk_scan_least(dk, ld, ld, ld, (long)H * (dv + 1), p + q_off,
-                                 p + k_off, 8, true, T, S);
+                                 p + k_off, dv, 8, true, T, S);
   if (least) {
     ChunkArgs a = {};
     a.o = o; a.q = p + q_off; a.k = p + k_off; a.v = p + v_off;

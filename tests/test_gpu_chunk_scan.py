@@ -92,6 +92,33 @@ def test_decay_chunks(H, G, dk, dv, kind):
     assert torch.equal(st[7].cpu(), state[7])
 
 
+@pytest.mark.parametrize("which", ["q", "k", "v", "windows"])
+def test_rows_less_than_a_head_apart(which):
+    """One row for all tokens, and rows that overlap: token by token, as ever."""
+    g = torch.Generator().manual_seed(12)
+    H, dk, dv = 2, 64, 48
+    qlocs, total, slots = _batch()
+    T = int(qlocs[-1])
+    x = {"q": torch.randn(T, 1, dk, generator=g), "k": torch.randn(T, 1, dk, generator=g),
+         "v": torch.randn(T, H, dv, generator=g)}
+    dev = {n: t.to(DEV) for n, t in x.items()}
+    if which == "windows":
+        buf = torch.randn(4 * T + dk, generator=g)
+        x["k"] = buf.as_strided((T, 1, dk), (4, dk, 1))
+        dev["k"] = buf.to(DEV).as_strided((T, 1, dk), (4, dk, 1))
+    else:
+        x[which], dev[which] = (t[which][:1].expand(T, -1, -1) for t in (x, dev))
+    a = torch.rand(T, H, generator=g)
+    state = torch.randn(11, H, dk, dv, generator=g)
+    want, end = _recur(*x.values(), a, torch.ones(T, H), torch.zeros(H), state, qlocs,
+                       total, slots)
+    st = state.to(DEV)
+    o = hops.decay_scan(*dev.values(), a.to(DEV), None, None, st, slots.to(DEV),
+                        qlocs.to(DEV), total.to(DEV))
+    assert _off(o, want) < TOL
+    assert _off(st, end) < TOL
+
+
 @pytest.mark.parametrize("H,dk,dv", [(2, 128, 128), (3, 64, 40), (1, 12, 144),
                                      (2, 100, 143)])
 def test_mlstm_chunks(H, dk, dv):
