@@ -518,7 +518,9 @@ extern "C" int mix_latent_attention(
     int nsplit, float* part_o, float* part_ml, hipStream_t s) {
   int DV = 0;
   const int DK = latent_pad(dk, dv, page, &DV);
-  if (!DK || ldo % 8 || out_off % 8 || (size_t)out % 16) return 0;
+  // (pages that do not begin at multiples of 16 bytes are not copied straight to LDS)
+  if (!DK || ldo % 8 || out_off % 8 || (size_t)out % 16 || (size_t)cache % 16)
+    return 0;
   if (T == 0) return 1;
   LatentArgs A;
   A.out = (u16*)out; A.ldo = ldo; A.out_off = out_off;

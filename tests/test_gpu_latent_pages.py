@@ -66,3 +66,27 @@ def test_uneven_sequences(H, dk, dv, window):
         want = torch.einsum("htk,kd->thd", s.softmax(-1), kv[:, :dv])
         err = (got[locs[i]:locs[i + 1]] - want).abs().max()
         assert err <= (2 ** -7 + 2 ** -12) * float(kv[:, :dv].abs().max())
+
+
+@pytest.mark.parametrize("start", [1, 4])
+def test_pages_at_other_places(start):
+    """Pages that begin at 2 or 8 bytes past a multiple of 16 (a part of a larger
+    buffer): the general kernel's, one rounding of weights and results from the other."""
+    dev = "cuda"
+    H, dk, dv, S = 4, 72, 64, 3
+    g = torch.Generator().manual_seed(start)
+    flat = torch.randn(start + 5 * 32 * dk, generator=g).bfloat16().to(dev)
+    cache = flat[start:].view(5, 1, 32, dk)
+    q = torch.randn(S, H, dk, generator=g).bfloat16().to(dev)
+    i32 = dict(dtype=torch.int32, device=dev)
+    table = torch.tensor([[1, 2], [3, 0], [4, 0]], **i32)
+    lens, locs = torch.tensor([50, 32, 3], **i32), torch.arange(S + 1, **i32)
+    rest = (table, lens, locs, dk ** -0.5, 0, 0,
+            torch.empty(S, 8, dtype=torch.bfloat16, device=dev), -1)
+    outs = []
+    for c in (cache, cache.clone()):
+        out = torch.zeros(S, H * dv, dtype=torch.bfloat16, device=dev)
+        hops.local_attention(q, c, c[..., :dv], *rest, out, 0, 1.0,
+                             token_seq=torch.arange(S, **i32))
+        outs.append(out.double())
+    assert (outs[0] - outs[1]).abs().max() <= 2 ** -6 * float(cache.abs().max())
