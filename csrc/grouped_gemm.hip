@@ -446,20 +446,25 @@ __device__ __forceinline__ u32 gw_pack(float x, float y) {
 // The gated unit of 8 sums at a time. Its operations run beside no products, with one
 // wave a SIMD: a tile's 128 units a lane were a quarter of its time at a k of 1024. So
 // each operation is issued for all 8 before the next, which waits for none of them
-// then, and the quotient v / d is v times the reciprocal, corrected by its remainder: d
-// is 1 or more, nothing has to be scaled: 9 operations a unit instead of 15. 2 x
-// 3072 x 1024 at 24,000 rows 260 -> 251 us, 2 x 8192 x 2048 at 32,768 1582 -> 1530, 2 x
-// 12288 x 4096 4533 -> 4469, 32 experts of 2048 x 2048 at 4096 rows 1661 -> 1604, 187
-// rows 126.5 -> 123.3, in turn on one card. 1.3e9 results were the same to the bit.
+// then, and the quotient v / d is v times the reciprocal, corrected by its remainder: 10
+// operations a unit instead of 15. 2 x 3072 x 1024 at 24,000 rows 260 -> 251 us, 2 x 8192 x
+// 2048 at 32,768 1582 -> 1530, 2 x 12288 x 4096 4533 -> 4469, 32 experts of 2048 x 2048 at
+// 4096 rows 1661 -> 1604, 187 rows 126.5 -> 123.3, in turn on one card, with 9. 1.3e9
+// results were the same to the bit.
+// d = 1 + exp(-v) passes 2^126 for v below -87.3, and its reciprocal, too small a number,
+// is 0 then (-5e-37 for v = -88 was). So v and d are taken as quarters, the tenth
+// operation (0.3 %: 24,000 rows 234.7 and 236.0, 32,768 1519.5 and 1523.5), which changes
+// no other bit, but of v below 2^-124. GELU by tanh has long been 0 there.
 template <int MODE>
 __device__ __forceinline__ void gw_unit8(float (&v)[8], float (&u)[8], float limit,
                                          float rw) {
   float g[8], d[8], r[8], e[8];
+  constexpr float Q = MODE == 6 ? 1.f : 0.25f;
 #define GW_EACH(X)                                                          \
   _Pragma("unroll") for (int i = 0; i < 8; ++i) { X; }                      \
   __builtin_amdgcn_sched_barrier(0);
   if (MODE == 4) {
-    GW_EACH(v[i] *= rw)
+    GW_EACH(v[i] *= rw * Q)
     GW_EACH(u[i] *= rw)
   }
   if (MODE == 6) {     // 0.5 (1 + tanh z) = 1 / (1 + exp(-2 z))
@@ -472,10 +477,11 @@ __device__ __forceinline__ void gw_unit8(float (&v)[8], float (&u)[8], float lim
     GW_EACH(d[i] = v[i] * -1.702f)
     GW_EACH(d[i] = d[i] * 1.4426950408889634f)
   } else {
-    GW_EACH(d[i] = v[i] * -1.4426950408889634f)
+    GW_EACH(d[i] = v[i] * (-1.4426950408889634f / (MODE == 4 ? Q : 1.f)))
   }
+  if (MODE != 4 && MODE != 6) { GW_EACH(v[i] *= Q) }
   GW_EACH(d[i] = __builtin_amdgcn_exp2f(d[i]))
-  GW_EACH(d[i] = 1.0f + d[i])
+  GW_EACH(d[i] = fmaf(d[i], Q, Q))
   GW_EACH(r[i] = __builtin_amdgcn_rcpf(d[i]))
   GW_EACH(g[i] = v[i] * r[i])
   GW_EACH(e[i] = fmaf(-d[i], g[i], v[i]))

@@ -12,8 +12,8 @@ from sutro_amd.ops import hybrid as hops
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 K, N, M = 64, 128, 256
-GATES = [0.0, -0.0, 1e-30, 1e-3, 0.5, 1.0, 1.5, 3.0, 7.0, 11.0, 20.0, 87.0, 100.0,
-         1e4, 1e30, 3e38, math.inf, math.nan]
+GATES = [0.0, -0.0, 1e-30, 1e-3, 0.5, 1.0, 1.5, 3.0, 7.0, 11.0, 52.0, 87.0, 88.0, 88.5,
+         20.0, 100.0, 1e4, 1e30, 3e38, math.inf, math.nan]
 UPS = [0.0, 1.0, -1.0, 0.3, 7.5, -9.0, 1e-20, 1e20]
 
 
@@ -38,17 +38,19 @@ def _want(x, w, unit):
     return unit(y[:, :N], y[:, N:])
 
 
-def _check(got, want):
-    """One rounding to bf16 (2^-8 / (1 + 2^-8)), the unit in fp32 far below it; where exp(-gate)
-    is past 2^126 the quotient, under 2^-119 of the up's, may be 0."""
-    got, want = got.double().cpu(), want
+def _check(got, want, power):
+    """One rounding to bf16 (2^-8 / (1 + 2^-8), below 2^-126 half of 2^-133), the unit in
+    fp32 far below it; where e^power is infinite in fp32 (2^128) the quotient, under
+    2^-121 of the up's 1e20, is 0."""
+    got, past = got.double().cpu(), torch.exp(power.float()).isinf()
     assert torch.equal(got.isnan(), want.isnan())
     ok = ~want.isnan()
     big = want.abs() > 3.4e38                       # past bf16's largest: infinite
     assert torch.equal(got[ok & big], want[ok & big].sign() * math.inf)
     ok &= ~big
     err = (got[ok] - want[ok]).abs()
-    assert (err <= want[ok].abs() * 2 ** -8 + 2.0 ** -119 * 1e20).all()
+    lost = past[ok].double() * 2.0 ** -121 * 1e20
+    assert (err <= want[ok].abs() * 2 ** -8 + 2.0 ** -134 + lost).all()
 
 
 def silu(g, u):
@@ -69,7 +71,7 @@ def clamped(g, u, limit=7.0):
 def test_one_matrix():
     x, w = _operands()
     got = ops._require_hip().linear_silu_mul(x.to(DEV), w.to(DEV))
-    _check(got, _want(x, w, silu))
+    _check(got, _want(x, w, silu), _want(x, w, lambda g, u: -g))
 
 
 def test_gelu():
@@ -78,7 +80,7 @@ def test_gelu():
     w[w.isinf()] = 0
     x, w = (torch.nn.functional.pad(t, (0, K - 3)) for t in (x, w))
     got = ops._require_hip().linear_gelu_mul(x.to(DEV), w.to(DEV), None, N)[0]
-    _check(got, _want(x, w, gelu))
+    _check(got, _want(x, w, gelu), torch.full_like(got.double().cpu(), math.inf))
 
 
 @pytest.mark.parametrize("biased", [True, False])
@@ -113,9 +115,11 @@ def test_experts(kind):
     tok = torch.arange(M, dtype=torch.int32, device=DEV)
     out = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
     rw = torch.rand(M, generator=torch.Generator().manual_seed(1)) * 0.5 + 0.25
+    rw[::7] = 1.0
     act = hops.ACT_GLU_CLAMPED if kind == "clamped" else hops.ACT_SILU_GATE
     hops.expert_gemm(out, x.to(DEV), w.to(DEV)[None], tok, off, cnt, act, 256, 7.0,
                      rw.to(DEV) if kind == "weighted" else None)
     y = rw[:, None].double() if kind == "weighted" else 1.0
-    unit = clamped if kind == "clamped" else silu
-    _check(out, _want(x, w, lambda g, u: unit(g * y, u * y)))
+    unit, c = (clamped, 1.702) if kind == "clamped" else (silu, 1.0)
+    _check(out, _want(x, w, lambda g, u: unit(g * y, u * y)),
+           _want(x, w, lambda g, u: -c * y * g))
