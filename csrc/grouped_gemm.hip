@@ -143,6 +143,7 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   const int m0 = (t - tile_off[e]) * BM;              // within-segment row
   const int seg0 = tile_off[e] * BM;                  // segment global base
   const int rows_valid = counts[e] - m0;              // live rows this tile
+  if (rows_valid <= 0) return;       // a segment longer than its rows need
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -542,8 +543,8 @@ __device__ __forceinline__ void gw_body(
     for (int j = 0; j < 8; ++j) {
       const int r = (wave * 8 + j) * 8 + pr;
       int row = DENSE ? min(r, g.live - 1) : r;
-      if (GATHER)        // padding rows repeat the last
-        row = max(row_tok[g.seg + min(r, g.live - 1)], 0);
+      if (GATHER)        // padding rows repeat the last (a tile may have none)
+        row = max(row_tok[g.seg + min(r, max(g.live, 1) - 1)], 0);
       if (ANY)
         s.pa[ANY ? j : 0] = base + row * K + ch[j & 1];
       else

@@ -51,3 +51,32 @@ def test_live_rows(K, ff, act, bm):
         # one rounding to bf16 (2^-8) and fp32 sums of K products in other orders
         torch.testing.assert_close(out[a:a + c].float(), y, rtol=2 ** -7,
                                    atol=2 ** -7)
+
+
+@pytest.mark.parametrize("bm", [32, 64, 128, 256])
+@pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE])
+def test_segments_longer_than_their_rows(act, bm):
+    """Two tiles for every expert, however many rows it has: none, a few, one more than
+    a tile. Tiles without rows are not asked for the row in front of them."""
+    counts = [0, 3, bm + 1, 0, bm, 2 * bm]
+    g = torch.Generator(device=DEV).manual_seed(bm)
+    gated, gather = act == hops.ACT_SILU_GATE, act != hops.ACT_NONE
+    K, ff, E = 128, 256, len(counts)
+    off = torch.arange(E + 1, device=DEV, dtype=torch.int32) * 2
+    cnt = torch.tensor(counts, device=DEV, dtype=torch.int32)
+    w = torch.randn(E, 2 * ff if gated else ff, K, generator=g, device=DEV)
+    w = (w * K ** -0.5).bfloat16()
+    rows, T = 2 * E * bm, 40
+    x = torch.randn(T if gather else rows, K, generator=g, device=DEV).bfloat16()
+    tok = torch.randint(0, T, (rows,), generator=g, device=DEV).int()
+    for e, c in enumerate(counts):
+        tok[2 * e * bm + c:2 * (e + 1) * bm] = -1
+    out = torch.zeros(rows, ff, device=DEV, dtype=torch.bfloat16)
+    hops.expert_gemm(out, x, w, tok if gather else None, off, cnt, act, bm, 0.0, None)
+    for e, c in enumerate(counts):
+        a = 2 * e * bm
+        y = (x[tok[a:a + c].long()] if gather else x[a:a + c]).float() @ w[e].float().T
+        if gated:
+            y = torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]
+        torch.testing.assert_close(out[a:a + c].float(), y, rtol=2 ** -7,
+                                   atol=2 ** -7)
