@@ -200,11 +200,15 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   // 2048 x 2048 on tiles of 32 50.7 -> 44.5. Rows are looked up once: at each step, the
   // wait for the table stood before the copies (16 rows an expert of 2048 x 2048 on
   // tiles of 64 139 -> 119 us, 64 of 3072 x 4096 530 -> 432, 112 of 2048 x 2048 on 128
-  // 198 -> 169). Only with 2.5 workgroups a CU or more on tiles of 32 that wait does
-  // good, it seems by taking them out of step: 28 experts 70.9 us without and 68.0 with
-  // it, 32 at 16 rows 96.2 and 94.0, 660 workgroups of 2 x 768 columns 72.1 and 69.3;
-  // 640 of 2 x 2048 59.4 and 60.7, 352 of them 38.7 and 46.3; with a k of 4096 (960
-  // workgroups) 216 and 230.
+  // 198 -> 169).
+  // Only on gated tiles of 32 that wait does good where it is hidden: with all four
+  // workgroups that a CU's LDS holds it takes them out of step. With fewer it is in the
+  // way. So it goes by whether the last round of workgroups is over three quarters full.
+  // Once and by this rule, us: 2848 workgroups of 2 x 2048 x 2048 (0.78 of a round) 267 and
+  // 257, 1932 of 2 x 768 x 6144 (0.89) 545 and 529, 992 of 2 x 2048 x 2048 (0.97) 93.7 and
+  // 91.6; at each step against once, 396 of 2 x 2816 x 6144 (0.39) 144 and 117, 1216 of 2 x
+  // 1024 x 2880 (0.19) 202 and 174, 736 of 2 x 2048 x 6144 (0.72) 206 and 202. To ask costs
+  // 0.4 us at most; the other units (six a CU) would pay 4 % for it and gain 1 to 3.
   constexpr int CHA = BM / (8 * WAVES);
   static_assert(CHA >= 1, "tile too small for wave count");
   // (from the last wave on: the first ones have the products of few rows)
@@ -218,8 +222,10 @@ __global__ __launch_bounds__(WROWS* WCOLS * 64) void grouped_gemm_kernel(
   long a_at[CHA];
 #pragma unroll
   for (int j = 0; j < CHA; ++j) a_at[j] = a_row(j);
-  constexpr bool AGAIN = BM == 32 && GATHER;
-  const bool again = K < 4096 && tile_off[n_experts] * gridDim.y > 640;
+  constexpr bool AGAIN = BM == 32 && GATED;
+  constexpr u32 ROUND = 256 * (160 * 1024 / sizeof(smem));
+  const u32 last = (tile_off[n_experts] * gridDim.y - 1) % ROUND + 1;
+  const bool again = last * 4 > ROUND * 3;
 
   auto stage_a = [&](u16* to) {
     const char* sa = (const char*)(CARRY ? pa : aa + ko);

@@ -12,12 +12,14 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("bm", [32, 64, 128])
 @pytest.mark.parametrize("act", [hops.ACT_NONE, hops.ACT_SILU_GATE, hops.ACT_RELU2])
-@pytest.mark.parametrize("K,ff", [(64, 64), (320, 192), (2048, 1024), (4096, 1024)])
-def test_live_rows(K, ff, act, bm):
-    """Counts around chunks of 8 rows and blocks of 16; with 1024 columns more than
-    640 workgroups (tiles of 32 look their rows up at each step), with fewer not."""
+@pytest.mark.parametrize("K,ff,more", [(64, 64, 0), (320, 192, 0), (2048, 1024, 24),
+                                       (4096, 1024, 24), (1024, 1024, 55)])
+def test_live_rows(K, ff, more, act, bm):
+    """Counts around chunks of 8 rows and blocks of 16; with 24 experts more 816
+    workgroups of tiles of 32, a round nearly full (gated ones look their rows up at each
+    step then), with 55 more a second round of few."""
     counts = [1, 0, 7, 8, 9, 15, 16, 17, 31, 32, 33, 2, 63, 65, 127, 129, 0, 3]
-    counts += [5] * (24 if ff == 1024 else 0)
+    counts += [5] * more
     g = torch.Generator(device=DEV).manual_seed(K + bm)
     gated, gather = act == hops.ACT_SILU_GATE, act != hops.ACT_NONE
     tiles = [(c + bm - 1) // bm for c in counts]
