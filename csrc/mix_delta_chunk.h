@@ -18,7 +18,8 @@
 // that from i to the middle, and both are shared by all pairs of the 2h tokens; one
 // tile of 16 x 16 holds the pairs of a level. fp32 operands are split into three bf16
 // terms as in mix_chunk.h, whose layouts are used here as well; sequences with
-// numbers that are not finite are done once more token by token.
+// numbers that are not finite are done once more token by token (as there; 16 rows of
+// 1024 tokens of 32 heads 763 us, with a NaN in one of them 2993, in all 7551).
 //
 // Times for 16 rows of 2048 tokens with a decay a channel, heads of 128 x 128, scan and
 // both kernels: 16 heads 1530 and 619 us (pairs 235), 8 heads 1000 and 354 (pairs 133);
