@@ -560,7 +560,7 @@ void delta_scan(torch::Tensor o, torch::Tensor qn, torch::Tensor kn,
                                     (int)H, (int)dk, (int)dv);
   torch::Tensor pairs;
   if (least)
-    pairs = torch::empty({mix_delta_pairs_floats(T, (int)S, (int)H)}, o.options());
+    pairs = torch::empty({mix_delta_pairs_floats(T, least, (int)H)}, o.options());
   mix_delta_scan(o.data_ptr<float>(), qn.data_ptr<float>(),
                  kn.data_ptr<float>(), v.data_ptr<float>(),
                  decay.data_ptr<float>(), head, beta.data_ptr<float>(),

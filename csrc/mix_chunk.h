@@ -19,8 +19,8 @@
 // Infinities and NaN do not survive a split: a sequence in which any read-out or state is
 // not finite is done once more, token by token (chunk_serial), from the state that is
 // still in memory, by each wave with such a column and without LDS: 16 rows of 1024 tokens
-// of 32 heads 498 us, with a NaN in one of them 1675, in all 4138; 1 row of 4000 of 16
-// heads 564, 5808 and 6825.
+// of 32 heads 441 us, with a NaN in one of them 1824, in all 4517; 1 row of 4000 of 16
+// heads 526, 6464 and 7397.
 //
 // A wave owns 16 columns of S in registers, laid out as the products leave them (row
 // dk = 16 m + 4 (lane / 16) + r of tile m, column lane % 16).
@@ -32,9 +32,9 @@
 // The scan does four fp32 operations an element of S and token, at 70 % of the VALU's
 // rate, one token behind the other; here they are 80,000 operations a token of a head
 // of 128 x 128 on the matrix cores, six times over. Times, scan and chunks: 13 rows of
-// 30,001 tokens in all, 16 heads of 128 x 128, 1367 and 455 us; 16 rows of 1024, 32
-// heads, 1128 and 346; 1 row of 4000, 16 heads, 1234 and 526; MLSTM, 61 rows of 30,000
-// in all, 8 heads, 834 and 168. What bounds it: a chunk takes 9950 cycles of a CU, its
+// 30,001 tokens in all, 16 heads of 128 x 128, 1280 and 495 us; 16 rows of 1024, 32
+// heads, 990 and 375; 1 row of 4000, 16 heads, 1240 and 532; MLSTM with its gates, 61 rows
+// of 30,000 in all, 8 heads, 891 and 237. What bounds it: a chunk takes 9950 cycles of a CU, its
 // SIMDs issue VALU instructions in 5900 of them (the splits above all) and are at
 // products in 3750, and the two overlap little. Slower: waves of 32 columns (half the
 // reads of LDS, but half the waves: 620 instead of 350 us), workgroups without
@@ -65,10 +65,10 @@ struct ChunkArgs {
   const int* state_slots;
   const int* qlocs;
   const int* seq_lens;
-  int H, G, dk, dv;
+  int S, H, G, dk, dv;
   int ov;               // dv; MLSTM dv + 1: the last column's value is 1
   int cgs;              // column groups of a head
-  int n_wg;             // S * H * cgs
+  int n_wg, run;        // see ch_wg
   float qscale;         // of the read-out
   int least;            // new tokens from which a sequence is done here
 };
@@ -277,6 +277,36 @@ __device__ __forceinline__ double ch_scan64(double v) {
   return v;
 }
 
+// Workgroups are numbered by the rank of their sequence among those of `least` or more
+// new tokens, of which there are no more than T / least: single tokens beside a few
+// prompts need none that way. Runs of up to four go to one XCD (k and q are shared where
+// heads share them), the next run to the next XCD. All sequences, an eighth of them for
+// each XCD, left the prompts of a batch to few XCDs: 3 of 1200 tokens beside 48 single
+// ones, 32 heads of 128 x 128, 617 us (the scan 418) and 236 now, the delta rule 636
+// (730) and 275; 16 rows of 2048, 16 heads, 385 and 347.
+__device__ __forceinline__ int ch_wg(int run) {
+  const int x = blockIdx.x % 8, j = blockIdx.x / 8;
+  return (j / run * 8 + x) * run + j % run;
+}
+static inline int ch_run(int n_wg) { return n_wg < 32 ? (n_wg + 7) / 8 : 4; }
+static inline unsigned ch_grid(int n_wg, int run) {
+  return (unsigned)((n_wg + 8 * run - 1) / (8 * run) * (8 * run));
+}
+// the sequence of rank k, or -1
+__device__ __forceinline__ int ch_sequence(const int* qlocs, int S, int least, int k) {
+  const int lane = threadIdx.x & 63;
+  for (int b = 0; b < S; b += 64) {
+    const int i = b + lane < S ? b + lane : S - 1;
+    const bool is = b + lane < S && qlocs[i + 1] - qlocs[i] >= least;
+    const u64 all = __ballot(is);
+    if (k < __popcll(all))
+      return b + __builtin_ctzll(
+                     __ballot(is && __popcll(all & ((1ull << lane) - 1)) == k));
+    k -= __popcll(all);
+  }
+  return -1;
+}
+
 // One workgroup: a sequence, a head and NC tiles of 16 columns. NC consumer waves
 // hold a tile each; four (MLSTM: three) producer waves bring k, q and the weights of
 // the next chunk into the other half of LDS meanwhile. Two barriers a chunk:
@@ -306,17 +336,13 @@ __global__ void __launch_bounds__(768, 3) chunk_scan_kernel(const ChunkArgs A) {
   extern __shared__ __attribute__((aligned(16))) char ch_lds[];
   Buf* const buf = (Buf*)ch_lds;
 
-  // heads that share k and q are neighbours: one XCD has them
-  int wg;
-  {
-    const int per = A.n_wg / 8, left = A.n_wg % 8, x = blockIdx.x % 8;
-    wg = x * per + (x < left ? x : left) + blockIdx.x / 8;
-  }
+  int wg = ch_wg(A.run);
+  if (wg >= A.n_wg) return;
   const int cg = wg % A.cgs;
   wg /= A.cgs;
-  const int h = wg % A.H, s = wg / A.H;
+  const int h = wg % A.H, s = ch_sequence(A.qlocs, A.S, A.least, wg / A.H);
+  if (s < 0) return;
   const int q0 = A.qlocs[s], n = A.qlocs[s + 1] - q0;
-  if (n < A.least) return;
   const bool old = A.seq_lens[s] > n;
   const int tid = threadIdx.x;
   const int lane = tid & 63, lr = lane & 15, lg = lane >> 4;
@@ -654,13 +680,15 @@ static void chunk_scan_go(const ChunkArgs& A, hipStream_t s) {
   static std::atomic<unsigned long long> asked{0};
   const auto fn = chunk_scan_kernel<DK, MLSTM>;
   lds_limit((const void*)fn, bytes, asked);
-  hipLaunchKernelGGL(fn, dim3(A.n_wg), dim3(768), bytes, s, A);
+  hipLaunchKernelGGL(fn, dim3(ch_grid(A.n_wg, A.run)), dim3(768), bytes, s, A);
 }
 template <bool MLSTM>
-static void chunk_scan_launch(ChunkArgs A, int S, int least, hipStream_t s) {
+static void chunk_scan_launch(ChunkArgs A, long T, int S, int least, hipStream_t s) {
   const int per = ChunkWaves<MLSTM>::NC * 16;
   A.cgs = (A.ov + per - 1) / per;
-  A.n_wg = S * A.H * A.cgs;
+  A.S = S;
+  A.n_wg = (int)(T / least < S ? T / least : S) * A.H * A.cgs;
+  A.run = ch_run(A.n_wg);
   A.least = least;
   if (A.dk <= 64) chunk_scan_go<64, MLSTM>(A, s);
   else chunk_scan_go<128, MLSTM>(A, s);

@@ -446,7 +446,7 @@ extern "C" int mix_decay_scan(float* o, const float* q, long ldq,
     a.state = state; a.state_slots = state_slots;
     a.qlocs = qlocs; a.seq_lens = seq_lens;
     a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.ov = dv;
-    chunk_scan_launch<false>(a, S, least, s);
+    chunk_scan_launch<false>(a, T, S, least, s);
   }
   const int below = least ? least : INT_MAX;
 #define LAUNCH_DS(RR, PP)                                                    \

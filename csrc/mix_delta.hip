@@ -918,11 +918,11 @@ extern "C" int mix_delta_least(const float* qn, const float* kn,
                                int H, int dk, int dv) {
   return delta_chunks_least(qn, kn, decay, head_decay, T, S, H, dk, dv);
 }
-extern "C" long mix_delta_pairs_floats(long T, int S, int H) {
-  return (T / CH_T + S) * H * (long)DC_PAIRS;
+extern "C" long mix_delta_pairs_floats(long T, int least, int H) {
+  return dc_slots(T, least) * H * (long)DC_PAIRS;
 }
 
-// pairs: mix_delta_pairs_floats(T, S, H) floats of scratch if least is not 0
+// pairs: mix_delta_pairs_floats(T, least, H) floats of scratch if least is not 0
 extern "C" void mix_delta_scan(float* o, const float* qn, const float* kn,
                                const float* vv, const float* decay,
                                int head_decay, const float* beta, float* ssm,

@@ -19,7 +19,8 @@
 // tile of 16 x 16 holds the pairs of a level. fp32 operands are split into three bf16
 // terms as in mix_chunk.h, whose layouts are used here as well; sequences with
 // numbers that are not finite are done once more token by token (as there; 16 rows of
-// 1024 tokens of 32 heads 763 us, with a NaN in one of them 2993, in all 7551).
+// 1024 tokens of 32 heads 727 us, with a NaN in one of them 3640, in all 8629; 1 row of
+// 4000 of 16 heads 399 and 12,300).
 //
 // Times for 16 rows of 2048 tokens with a decay a channel, heads of 128 x 128, scan and
 // both kernels: 16 heads 1530 and 619 us (pairs 235), 8 heads 1000 and 354 (pairs 133);
@@ -52,18 +53,18 @@ struct DeltaChunkArgs {
   const int* state_slots;
   const int* qlocs;
   const int* seq_lens;
-  float* pairs;         // [T / 32 + S, H, DC_PAIRS]
+  float* pairs;         // [T / 32 + T / least, H, DC_PAIRS]
   int S, H, G, dk, dv;
-  int cgs, n_wg;        // as in ChunkArgs
+  int cgs, n_wg, run;   // as in ChunkArgs
   int least;
 };
 
 // tiles (0, 0), (1, 0), (1, 1) of 16 x 16: M, then the read-out's sums
 #define DC_PAIRS (2 * 3 * 256)
 
-// chunks of a sequence are numbered from this on: no two have the same number, and
-// all are below T / 32 + S
-__device__ __forceinline__ int dc_slot(int q0, int s) { return (q0 >> 5) + s; }
+// chunks of the sequence of rank k (see ch_wg) are numbered from this on: no two have
+// the same number, and all are below T / 32 + T / least
+__device__ __forceinline__ int dc_slot(int q0, int k) { return (q0 >> 5) + k; }
 
 // two channels of a row -> three terms at `p`, PLANE bytes apart
 template <int PLANE>
@@ -123,15 +124,24 @@ delta_pairs_kernel(const DeltaChunkArgs A) {
   const int lr = lane & 15, lg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = blockIdx.x % A.H, slot = blockIdx.x / A.H;
-  int s = -1;
-  for (int b = 0; b < A.S; b += 64) {
-    const int i = b + lane;
-    s += __popcll(__ballot(i < A.S && dc_slot(A.qlocs[i < A.S ? i : 0], i) <= slot));
+  int s = -1, rank = 0;    // the last sequence that begins at or in front of the slot
+  for (int b = 0, before = 0; b < A.S; b += 64) {
+    const int i = b + lane < A.S ? b + lane : A.S - 1, q = A.qlocs[i];
+    const bool is = b + lane < A.S && A.qlocs[i + 1] - q >= A.least;
+    const u64 all = __ballot(is);
+    const int k = before + __popcll(all & ((1ull << lane) - 1));
+    const u64 hit = __ballot(is && dc_slot(q, k) <= slot);
+    if (hit) {
+      const int last = 63 - __builtin_clzll(hit);
+      s = b + last;
+      rank = before + __popcll(all & ((1ull << last) - 1));
+    }
+    before += __popcll(all);
   }
-  if (s < 0) return;       // tokens in front of the first sequence
+  if (s < 0) return;       // none
   const int q0 = A.qlocs[s], n = A.qlocs[s + 1] - q0;
-  const int base = (slot - dc_slot(q0, s)) * CH_T;
-  if (n < A.least || base >= n) return;
+  const int base = (slot - dc_slot(q0, rank)) * CH_T;
+  if (base >= n) return;
   const int left = n - base < CH_T ? n - base : CH_T;
   const int dk = A.dk, g = h / (A.H / A.G);
   const int ch = lr * 8, r0 = w * 8 + lg * 2;   // channels and tokens of this lane
@@ -424,16 +434,14 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
   extern __shared__ __attribute__((aligned(16))) char dc_lds[];
   Lds& L = *(Lds*)dc_lds;
 
-  int wg;
-  {
-    const int per = A.n_wg / 8, left = A.n_wg % 8, x = blockIdx.x % 8;
-    wg = x * per + (x < left ? x : left) + blockIdx.x / 8;
-  }
+  int wg = ch_wg(A.run);
+  if (wg >= A.n_wg) return;
   const int cg = wg % A.cgs;
   wg /= A.cgs;
-  const int h = wg % A.H, s = wg / A.H;
+  const int h = wg % A.H, rank = wg / A.H;
+  const int s = ch_sequence(A.qlocs, A.S, A.least, rank);
+  if (s < 0) return;
   const int q0 = A.qlocs[s], n = A.qlocs[s + 1] - q0;
-  if (n < A.least) return;
   const bool old = A.seq_lens[s] > n;
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -476,7 +484,7 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
                      left > 0 ? left * ldk : 0u);
     };
     // tiles pw and (waves 0, 1) 4 + pw of the chunk's six
-    const int slot0 = dc_slot(q0, s);
+    const int slot0 = dc_slot(q0, rank);
     auto fetch_pairs = [&](int c) {
       const float* p = A.pairs + ((long)(slot0 + c) * A.H + h) * DC_PAIRS + lane * 4;
       rp[0] = *(const f32x4*)(p + pw * 256);
@@ -772,23 +780,27 @@ delta_chunks_kernel(const DeltaChunkArgs A) {
 }
 
 template <int DK, bool HEAD, int NC>
-static void delta_chunks_go(DeltaChunkArgs A, hipStream_t s) {
+static void delta_chunks_go(DeltaChunkArgs A, int seqs, hipStream_t s) {
   constexpr int bytes =
       9 * CH_T * DK * 2 + 6 * CH_T * CH_T * 2 + (2 * 2 * 4 + 1) * DK * 4 + CH_T * 4;
   static std::atomic<unsigned long long> asked{0};
   const auto fn = delta_chunks_kernel<DK, HEAD, NC>;
   lds_limit((const void*)fn, bytes, asked);
   A.cgs = (A.dv + 16 * NC - 1) / (16 * NC);
-  A.n_wg = A.S * A.H * A.cgs;
-  hipLaunchKernelGGL(fn, dim3(A.n_wg), dim3((NC + 4) * 64), bytes, s, A);
+  A.n_wg = seqs * A.H * A.cgs;
+  A.run = ch_run(A.n_wg);
+  hipLaunchKernelGGL(fn, dim3(ch_grid(A.n_wg, A.run)), dim3((NC + 4) * 64), bytes, s, A);
 }
+static inline long dc_slots(long T, int least) { return T / CH_T + T / least; }
+
 template <int DK, bool HEAD>
 static void delta_chunks_launch(const DeltaChunkArgs& A, long T, hipStream_t s) {
   hipLaunchKernelGGL((delta_pairs_kernel<DK, HEAD>),
-                     dim3((unsigned)((T / 32 + A.S) * A.H)), dim3(256), 0, s, A);
-  const long wgs = (long)A.S * A.H * ((A.dv + 127) / 128);
-  if (A.dv > 64 && wgs > 128) delta_chunks_go<DK, HEAD, 8>(A, s);
-  else delta_chunks_go<DK, HEAD, 4>(A, s);
+                     dim3((unsigned)(dc_slots(T, A.least) * A.H)), dim3(256), 0, s, A);
+  const int seqs = (int)(T / A.least < A.S ? T / A.least : A.S);
+  const long wgs = (long)seqs * A.H * ((A.dv + 127) / 128);
+  if (A.dv > 64 && wgs > 128) delta_chunks_go<DK, HEAD, 8>(A, seqs, s);
+  else delta_chunks_go<DK, HEAD, 4>(A, seqs, s);
 }
 
 // New tokens from which a sequence goes through chunks; the scan keeps the shorter

@@ -274,7 +274,7 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
     a.qlocs = qlocs; a.seq_lens = seq_lens;
     a.H = H; a.G = H; a.dk = dk; a.dv = dv; a.ov = dv + 1;
     a.qscale = 1.f / sqrtf((float)dk);
-    chunk_scan_launch<true>(a, S, least, s);
+    chunk_scan_launch<true>(a, T, S, least, s);
   }
   const int below = least ? least : INT_MAX;
   int R = 1;

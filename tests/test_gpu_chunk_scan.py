@@ -417,3 +417,54 @@ def test_decays_that_stay_the_same(decay):
                         slots.to(DEV), qlocs.to(DEV), total.to(DEV))
     assert _off(o, want) < TOL
     assert _off(st, end) < TOL
+
+
+@pytest.mark.parametrize("front", [0, 75])
+@pytest.mark.parametrize("kind", ["decay", "delta", "deltah", "mlstm"])
+def test_long_sequences_among_many(kind, front):
+    """150 sequences, a few of them long: the chunks find those by their rank, 64
+    sequences at a time, whatever lies between them (none, one token, pieces)."""
+    g = torch.Generator().manual_seed(front + 1)
+    H, dk, dv = 2, 64, 48
+    lens = [(0, 1, 1, 3, 1)[i % 5] for i in range(150)]
+    for i, n in {0: 70, 62: 97, 63: 64, 64: 131, 65: 65, 127: 66, 128: 96, 149: 100}.items():
+        lens[i] = n
+    qlocs = torch.tensor([0] + lens).cumsum(0).int() + front
+    T = int(qlocs[-1])
+    total = torch.tensor([n + i % 2 for i, n in enumerate(lens)], dtype=torch.int32)
+    slots = torch.randperm(151, generator=g)[:150].int()
+    meta = (slots.to(DEV), qlocs.to(DEV), total.to(DEV))
+    if kind == "mlstm":
+        cols = 2 * H * dk + H * dv
+        offs = (0, H * dk, 2 * H * dk, cols, cols + H)
+        proj = torch.randn(T, cols + 2 * H, generator=g).bfloat16()
+        ib, fb = torch.randn(H, generator=g), torch.randn(H, generator=g) + 2
+        state, m0 = torch.randn(151, H, dk, dv + 1, generator=g), torch.randn(151, H, generator=g)
+        end, want_m = state.clone(), m0.clone()
+        want, _ = ref.mlstm_scan(proj, *offs, H, dk, dv, ib, fb, 5.0, end, want_m, slots,
+                                 qlocs, total)
+        st = state.to(DEV)
+        o, _ = hops.mlstm_scan(proj.to(DEV), *offs, H, dk, dv, ib.to(DEV), fb.to(DEV),
+                               5.0, st, m0.to(DEV), *meta)
+        tol = 4 * TOL                   # the reference is fp32 as well
+    else:
+        unit = torch.nn.functional.normalize
+        q, k = (unit(torch.randn(T, H, dk, generator=g), dim=-1) for _ in "qk")
+        v = torch.randn(T, H, dv, generator=g)
+        a, b = torch.rand(T, H, generator=g), torch.rand(T, H, generator=g)
+        state = torch.randn(151, H, dk, dv, generator=g)
+        st = state.to(DEV)
+        if kind == "decay":
+            want, end = _recur(q, k, v, a, b, torch.zeros(H), state, qlocs, total, slots)
+            o = hops.decay_scan(*(x.to(DEV) for x in (q, k, v, a, b)), None, st, *meta)
+        else:
+            d = a if kind == "deltah" else torch.rand(T, H, dk, generator=g)
+            want, end = _delta(q, k, v, d[..., None].expand(T, H, dk)
+                               if kind == "deltah" else d, b, state, qlocs, total, slots)
+            o = hops.delta_scan(*(x.to(DEV) for x in (q, k, v, d, b)), st, *meta)
+        tol = TOL
+    assert _off(o[front:], want[front:].double()) < tol
+    assert _off(st, end.double()) < tol
+    for s, n in zip(slots.tolist(), lens):
+        if not n:
+            assert torch.equal(st[s].cpu(), state[s])
