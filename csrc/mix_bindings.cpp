@@ -130,7 +130,7 @@ void mix_ssd_prep(float*, float*, float*, const void*, long, int, int,
 int mix_decay_scan(float*, const float*, long, const float*, long,
                    const float*, long, const float*, long, const float*,
                    const float*, float*, const int*, const int*, const int*,
-                   long, int, int, int, int, int, hipStream_t);
+                   long, long, int, int, int, int, int, hipStream_t);
 void mix_softcap(float*, const void*, float, long, int, hipStream_t);
 void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
@@ -152,7 +152,7 @@ void mix_sigmoid_gate_mul(void*, long, const void*, long, int, long, int, int,
                           hipStream_t);
 void mix_mlstm_scan(float*, float*, float*, float*, const void*, long, int,
                     int, int, int, int, const float*, const float*, float,
-                    float*, float*, const int*, const int*, const int*, long,
+                    float*, float*, const int*, const int*, const int*, long, long,
                     int, int, int, int, int, hipStream_t);
 void mix_mlstm_out(void*, long, int, const float*, const float*, const float*,
                    const void*, long, int, float, long, int, int, int,
@@ -163,8 +163,8 @@ void mix_delta_prep(float*, float*, float*, float*, float*, const void*, long,
                     int, const float*, const float*, float*, const int*,
                     const int*, const int*, const int*, long, int, int, int,
                     int, int, int, hipStream_t);
-int mix_delta_least(const float*, const float*, const float*, int, long, int,
-                    int, int, int);
+int mix_delta_least(const float*, const float*, const float*, int, long, long,
+                    int, int, int, int);
 long mix_delta_pairs_floats(long, int, int);
 void mix_delta_scan(float*, const float*, const float*, const float*,
                     const float*, int, const float*, float*, const int*, const int*,
@@ -535,7 +535,7 @@ void delta_prep(torch::Tensor qn, torch::Tensor kn, torch::Tensor v,
 void delta_scan(torch::Tensor o, torch::Tensor qn, torch::Tensor kn,
                 torch::Tensor v, torch::Tensor decay, torch::Tensor beta,
                 torch::Tensor ssm, torch::Tensor state_slots,
-                torch::Tensor qlocs, torch::Tensor seq_lens) {
+                torch::Tensor qlocs, torch::Tensor seq_lens, long longest) {
   CHECK_GPU(v); CHECK_F32(o); CHECK_F32(qn); CHECK_F32(kn); CHECK_F32(v);
   CHECK_F32(decay); CHECK_F32(beta); CHECK_F32(ssm);
   CHECK_CONTIG(o); CHECK_CONTIG(qn); CHECK_CONTIG(kn); CHECK_CONTIG(v);
@@ -556,8 +556,8 @@ void delta_scan(torch::Tensor o, torch::Tensor qn, torch::Tensor kn,
               state_slots.numel() == S, "operand sizes");
   const int head = decay.dim() == 2 ? 1 : 0;
   const int least = mix_delta_least(qn.data_ptr<float>(), kn.data_ptr<float>(),
-                                    decay.data_ptr<float>(), head, T, (int)S,
-                                    (int)H, (int)dk, (int)dv);
+                                    decay.data_ptr<float>(), head, T, longest,
+                                    (int)S, (int)H, (int)dk, (int)dv);
   torch::Tensor pairs;
   if (least)
     pairs = torch::empty({mix_delta_pairs_floats(T, least, (int)H)}, o.options());
@@ -772,7 +772,7 @@ void mlstm_scan(torch::Tensor o, torch::Tensor em, torch::Tensor proj,
                 torch::Tensor i_bias, torch::Tensor f_bias, double cap,
                 torch::Tensor mem, torch::Tensor mstate,
                 torch::Tensor state_slots, torch::Tensor qlocs,
-                torch::Tensor seq_lens) {
+                torch::Tensor seq_lens, long longest) {
   CHECK_GPU(proj); CHECK_GPU(o); CHECK_F32(o); CHECK_CONTIG(o);
   CHECK_GPU(em); CHECK_F32(em); CHECK_CONTIG(em);
   CHECK_GPU(mem); CHECK_F32(mem); CHECK_CONTIG(mem);
@@ -801,7 +801,7 @@ void mlstm_scan(torch::Tensor o, torch::Tensor em, torch::Tensor proj,
                  (int)v_off, (int)i_off, (int)f_off, i_bias.data_ptr<float>(),
                  f_bias.data_ptr<float>(), (float)cap, mem.data_ptr<float>(),
                  mstate.data_ptr<float>(), state_slots.data_ptr<int>(),
-                 qlocs.data_ptr<int>(), seq_lens.data_ptr<int>(), T, (int)S,
+                 qlocs.data_ptr<int>(), seq_lens.data_ptr<int>(), T, longest, (int)S,
                  (int)H, (int)dk, (int)dv, act_kind(proj), cur_stream());
 }
 
@@ -1431,7 +1431,7 @@ void decay_scan(torch::Tensor o, torch::Tensor q, torch::Tensor k,
                 c10::optional<torch::Tensor> gain,
                 c10::optional<torch::Tensor> skip, torch::Tensor state,
                 torch::Tensor state_slots, torch::Tensor qlocs,
-                torch::Tensor seq_lens) {
+                torch::Tensor seq_lens, long longest) {
   CHECK_GPU(o); CHECK_F32(o); CHECK_CONTIG(o);
   CHECK_GPU(q); CHECK_F32(q); CHECK_GPU(k); CHECK_F32(k);
   CHECK_GPU(v); CHECK_F32(v); CHECK_GPU(decay); CHECK_F32(decay);
@@ -1477,8 +1477,8 @@ void decay_scan(torch::Tensor o, torch::Tensor q, torch::Tensor k,
       k.data_ptr<float>(), k.stride(0), v.data_ptr<float>(), v.stride(0),
       decay.data_ptr<float>(), lda, gp, sp, state.data_ptr<float>(),
       state_slots.data_ptr<int>(), qlocs.data_ptr<int>(),
-      seq_lens.data_ptr<int>(), T, (int)S, (int)H, (int)G, (int)dk, (int)dv,
-      cur_stream());
+      seq_lens.data_ptr<int>(), T, longest, (int)S, (int)H, (int)G, (int)dk,
+      (int)dv, cur_stream());
   TORCH_CHECK(ok, "decay_scan: key size above 256 is unsupported");
 }
 

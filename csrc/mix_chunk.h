@@ -651,25 +651,78 @@ __global__ void __launch_bounds__(768, 3) chunk_scan_kernel(const ChunkArgs A) {
   }
 }
 
-// New tokens from which a sequence goes through chunks; the scans keep the shorter
-// ones of the same batch (single tokens among them: state in, state out, for which
-// one workgroup a CU is too few). 0: no sequence of the batch can be long enough,
-// rows that are not in whole 16-byte (8-byte) pieces, or rows less than a head apart
-// (one row for all tokens): what a chunk may read ends a row's distance behind its last
-// row. Measured, scan and chunks, us:
-// dk 128, 16 heads x 256 rows of 10 tokens 185 and 268, 64 rows of 10 49 and 67, 1
-// row of 40 22 and 20, 4 rows of 100 44 and 30; dk 64, 4 rows of 16 9 to 14 and 8 to
-// 10, 64 of 10 12 and 14; MLSTM, 64 rows of 10 47 and 35, 256 rows of 1 91 and 115.
+// New tokens from which a sequence goes through chunks (0: none of the batch does); the
+// scans keep the shorter ones (single tokens among them: state in, state out). A chunk
+// takes a CU as long whatever its columns, and one workgroup is on a CU; the scan takes
+// what its rows and columns cost, several workgroups a CU. So where more than a round of
+// workgroups is at work, small heads stay with the scan for long, or always: `few`, `mid`
+// and `many` for up to 256 workgroups, up to 512, and more. But only T / n sequences can
+// have n tokens: longer ones may be few where shorter ones were many.
+// One kernel runs behind the other, so that sequences on both sides of the line take
+// the time of both: not where the longest (`longest` new tokens; 0: not known) has less than
+// twice the line and the mean is below 5/4 of it.
+struct ChunkNeed { int few, mid, many; };
+#define CH_NEVER (1 << 30)
+static inline int chunk_least(ChunkNeed need, long T, long longest, int S, long wgs) {
+  long least = need.many;
+  const long caps[2] = {256, 512}, needs[2] = {need.few, need.mid};
+  for (int i = 0; i < 2; ++i) {
+    const long seqs = caps[i] / wgs;          // sequences within `caps`
+    if (!seqs) continue;
+    long n = S > seqs ? T / (seqs + 1) + 1 : 0;
+    if (n < needs[i]) n = needs[i];
+    if (n < least) least = n;
+  }
+  if (longest <= 0) longest = T - S + 1;     // (a token for each of the others)
+  if (S < 1 || least > T || least > longest || (longest < 2 * least && 4 * T < 5 * S * least))
+    return 0;
+  return (int)least;
+}
+
+// Measured, tokens from which chunks are ahead in batches of equal sequences, 32 to 256
+// workgroups, 512, and 1024 to 4096 (keys x values of a head):
+//   decay  16 x 64    24        96   never     MLSTM  16 x 64     8    16   24 to 32
+//          16 x 128   32        96   192, 256         64 x 64    16    16    4 to 8
+//          32 x 64    24        64   192, 256         64 x 128   16    16    8
+//          64 x 16    24        48   96 to 192       128 x 16    24    32   32
+//          64 x 64    24        24   48              128 x 64    24    48   32 to 48
+//          64 x 128   24        16   24              128 x 128   32    16   16 to 24
+//         128 x 16    48       192   never
+//         128 x 64    64       128   128 to 256
+//         128 x 128   64        64   48 to 96
+// (128 x 32, 256 sequences of 64 tokens, 16 heads: 170 and 440 us; 128 x 128, 1024 workgroups
+// of 40 111 and 127, of 64 157 and 132; 1 row of 40 18.5 and 26, of 96 36 and 31.)
+static inline ChunkNeed chunk_need(bool mlstm, int dk, int columns) {
+  if (mlstm) {
+    if (dk > 64) return columns > 80 ? ChunkNeed{28, 24, 24} : ChunkNeed{28, 48, 48};
+    return dk > 32 ? ChunkNeed{12, 12, 12} : ChunkNeed{12, 32, 32};
+  }
+  if (dk > 64) {
+    if (columns > 80) return {64, 64, columns > 112 ? 80 : 96};
+    return columns > 48 ? ChunkNeed{64, 128, 256} : ChunkNeed{64, 192, CH_NEVER};
+  }
+  if (dk > 32) {
+    if (columns > 96) return {24, 24, 24};
+    return {24, 48, columns > 48 ? 48 : columns > 24 ? 128 : 192};
+  }
+  if (columns > 96) return {24, 96, dk > 16 ? 96 : 256};
+  return {24, 96, dk > 16 ? 256 : CH_NEVER};
+}
+
+// 0 also where rows are not in whole 16-byte (8-byte) pieces, or less than a head apart
+// (one row for all tokens): what a chunk may read ends a row's distance behind its last.
 static inline int chunk_scan_least(int dk, long ldq, long ldk, long ldv, long ldo,
                                    const void* q, const void* k, int dv,
-                                   int align, bool mlstm, long T, int S) {
-  const int least = mlstm ? 8 : (dk <= 64 ? 16 : 32);
+                                   int align, bool mlstm, long T, long longest,
+                                   int S, int H) {
   const long most = 1 << 23;               // 32 rows within 2^31 bytes
   if (dk > 128 || dk % 4 || ldq % 4 || ldk % 4 || (size_t)q % align ||
       (size_t)k % align || ldq >= most || ldk >= most || ldv >= most ||
-      ldo >= most || ldq < dk || ldk < dk || ldv < dv || T < S + least - 1)
+      ldo >= most || ldq < dk || ldk < dk || ldv < dv)
     return 0;
-  return least;
+  const int ov = mlstm ? dv + 1 : dv, per = mlstm ? 144 : 128;
+  const int cgs = (ov + per - 1) / per;
+  return chunk_least(chunk_need(mlstm, dk, dv / cgs), T, longest, S, (long)H * cgs);
 }
 
 template <int DK, bool MLSTM>

@@ -432,12 +432,12 @@ extern "C" int mix_decay_scan(float* o, const float* q, long ldq,
                               const float* gain, const float* skip,
                               float* state, const int* state_slots,
                               const int* qlocs, const int* seq_lens, long T,
-                              int S, int H, int G, int dk, int dv,
+                              long longest, int S, int H, int G, int dk, int dv,
                               hipStream_t s) {
   if (S == 0) return 1;
   const int least =
       chunk_scan_least(dk, ldq, ldk, ldv, (long)H * dv, q, k, dv, 16, false, T,
-                       S);
+                       longest, S, H);
   if (least) {
     ChunkArgs a = {};
     a.o = o; a.q = q; a.k = k; a.v = v;

@@ -914,9 +914,9 @@ extern "C" void mix_delta_prep(
 // New tokens from which a sequence goes through chunks (mix_delta_chunk.h), 0 if none
 // of the batch can be that long or rows are not in whole 16-byte pieces
 extern "C" int mix_delta_least(const float* qn, const float* kn,
-                               const float* decay, int head_decay, long T, int S,
-                               int H, int dk, int dv) {
-  return delta_chunks_least(qn, kn, decay, head_decay, T, S, H, dk, dv);
+                               const float* decay, int head_decay, long T,
+                               long longest, int S, int H, int dk, int dv) {
+  return delta_chunks_least(qn, kn, decay, head_decay, T, longest, S, H, dk, dv);
 }
 extern "C" long mix_delta_pairs_floats(long T, int least, int H) {
   return dc_slots(T, least) * H * (long)DC_PAIRS;

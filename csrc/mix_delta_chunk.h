@@ -803,20 +803,33 @@ static void delta_chunks_launch(const DeltaChunkArgs& A, long T, hipStream_t s) 
   else delta_chunks_go<DK, HEAD, 4>(A, seqs, s);
 }
 
-// New tokens from which a sequence goes through chunks; the scan keeps the shorter
-// ones of a batch. Measured, scan and chunks (per-channel decays, heads of 128 x 128),
-// us: 16 heads x 256 rows of 32 tokens 426 and 468, of 48 612 and 548, of 64 758 and
-// 570; 4 rows of 32 21 and 23, of 64 36 and 27; 4 heads of 64 x 64, 64 rows of 48 25
-// and 28, 256 of 64 96 and 84. 0: no sequence of the batch can be long enough, or rows
-// that are not whole 16-byte pieces.
+// New tokens from which a sequence goes through chunks (0: none of the batch does), as in
+// chunk_scan_least. Measured, 32 to 256 workgroups, 512, and 1024 to 4096:
+//            a decay a channel                 a decay a head
+//   16 x 64    24, 32   64   128 to never       32        64   never
+//   32 x 128   48, 64   64   never              48, 64   128   never
+//   64 x 16    48, 64   64    48                48, 64    64    64 to 192
+//   64 x 64    48, 64   64    64                48, 64    96    64 to 128
+//   64 x 128   48, 64   96    64                48, 64    96    96 to never
+//  128 x 16    48, 96   96    64 to 128         64, 128  128   128
+//  128 x 64    48, 64  128    96 to 128         64, 96   128   128 to 192
+//  128 x 128   48, 64   48    48                64        64    48 to 64
+// (16 heads of 32 x 64 with a decay a head, 256 sequences of 128 tokens: 370 and 481 us; of
+// 64 x 128, 32 heads, 128 of 64: 306 and 389; of 128 x 128, 256 of 64: 663 and 560.)
 static inline int delta_chunks_least(const float* q, const float* k,
-                                     const float* d, bool head, long T, int S,
-                                     int H, int dk, int dv) {
-  const int least = 64;
+                                     const float* d, bool head, long T,
+                                     long longest, int S, int H, int dk, int dv) {
   const long most = 1 << 23;               // 32 rows within 2^31 bytes
   if (dk > 128 || dk % 4 || (size_t)q % 16 || (size_t)k % 16 ||
-      (!head && (size_t)d % 16) || (long)H * dk >= most || (long)H * dv >= most ||
-      T < S + least - 1)
+      (!head && (size_t)d % 16) || (long)H * dk >= most || (long)H * dv >= most)
     return 0;
-  return least;
+  const int cgs = (dv + 127) / 128, columns = dv / cgs;
+  ChunkNeed need;
+  if (dk > 64)
+    need = columns > 80 ? ChunkNeed{64, 64, 64} : ChunkNeed{96, 128, head ? 192 : 128};
+  else if (dk > 32)
+    need = head ? ChunkNeed{64, 96, 192} : ChunkNeed{64, 96, 64};
+  else
+    need = ChunkNeed{64, 192, CH_NEVER};   // (ragged, 480 workgroups, from 128: 148 -> 166)
+  return chunk_least(need, T, longest, S, (long)H * cgs);
 }

@@ -244,8 +244,8 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
                                const float* i_bias, const float* f_bias,
                                float cap, float* mem, float* mstate,
                                const int* state_slots, const int* qlocs,
-                               const int* seq_lens, long T, int S, int H,
-                               int dk, int dv, int f32, hipStream_t s) {
+                               const int* seq_lens, long T, long longest,
+                               int S, int H, int dk, int dv, int f32, hipStream_t s) {
   if (S == 0) return;
   {
     const int waves = S * H;
@@ -264,7 +264,8 @@ extern "C" void mix_mlstm_scan(float* o, float* em, float* fa, float* ib,
   const u16* p = (const u16*)proj;
   const int least =
       f32 ? 0 : chunk_scan_least(dk, ld, ld, ld, (long)H * (dv + 1), p + q_off,
-                                 p + k_off, dv, 8, true, T, S);
+                                 p + k_off, dv, 8, true, T, longest,
+                                 S, H);
   if (least) {
     ChunkArgs a = {};
     a.o = o; a.q = p + q_off; a.k = p + k_off; a.v = p + v_off;

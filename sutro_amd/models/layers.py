@@ -297,7 +297,8 @@ class GatedDeltaRule(nn.Module):
             fb.seq_lens, token_seq=fb.token_seq, a2_t=self._t[0],
             conv_w_t=self._t[2])
         o = hops.delta_scan(qn, kn, v, decay, beta, st.ssm[ci],
-                            fb.state_slots, fb.query_start_locs, fb.seq_lens)
+                            fb.state_slots, fb.query_start_locs, fb.seq_lens,
+                            fb.max_query_len)
         if g2 is None:
             hops.gated_group_norm(o, proj, off[tag + "g"], self.norm_w,
                                   self.eps, s.heads, False, out, out_off,
@@ -576,7 +577,7 @@ class MLSTM(nn.Module):
             proj, off[tag + "q"], off[tag + "k"], off[tag + "v"],
             off[tag + "i"], off[tag + "f"], s.heads, s.dim, s.vdim,
             self.i_bias, self.f_bias, s.gate_cap, st["mem"], st["m"],
-            fb.state_slots, fb.query_start_locs, fb.seq_lens)
+            fb.state_slots, fb.query_start_locs, fb.seq_lens, fb.max_query_len)
         hops.mlstm_out(o, em, self.norm_w, proj, off[tag + "g"], self.eps,
                        out, out_off)
 
@@ -662,7 +663,7 @@ class DecayAttention(nn.Module):
             q.unflatten(1, (s.heads, s.dim)), k.unflatten(1, (s.heads, s.dim)),
             v.unflatten(1, (s.heads, s.vdim)), self.decay, None, None,
             kv.state.named[ci]["mem"], fb.state_slots,
-            fb.query_start_locs, fb.seq_lens)
+            fb.query_start_locs, fb.seq_lens, fb.max_query_len)
         per_head = s.norm == "head"
         hops.gated_group_norm(o, proj, off[tag + "g"],
                               None if per_head else self.norm_w, self.eps,
@@ -738,7 +739,7 @@ class SSDMixer(nn.Module):
             conv_w_t=self._t)
         y = hops.decay_scan(C, B, x, decay, dt, self.skip,
                             st.ssm[self.layer_idx], fb.state_slots,
-                            fb.query_start_locs, fb.seq_lens)
+                            fb.query_start_locs, fb.seq_lens, fb.max_query_len)
         hops.gated_group_norm(y, proj, base, self.norm_w, self.eps,
                               s.norm_groups, True, out, out_off)
 

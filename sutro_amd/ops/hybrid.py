@@ -194,11 +194,13 @@ def delta_prep(proj, q_off, k_off, v_off, b_off, a1_off, H, G, dk, dv,
 
 
 def delta_scan(qn, kn, v, decay, beta, ssm_state, state_slots,
-               query_start_locs, seq_lens):
+               query_start_locs, seq_lens, longest: int = 0):
+    """`longest`: new tokens of the longest sequence if the caller knows them. It decides
+    about the kernels only."""
     if v.is_cuda:
         o = torch.empty_like(v)
         _mix().delta_scan(o, qn, kn, v, decay, beta, ssm_state, state_slots,
-                          query_start_locs, seq_lens)
+                          query_start_locs, seq_lens, longest)
         return o
     return torch_ref.delta_scan(qn, kn, v, decay, beta, ssm_state,
                                 state_slots, query_start_locs, seq_lens)
@@ -301,7 +303,8 @@ def sigmoid_gate_mul(v, proj, g_off: int) -> None:
 
 def mlstm_scan(proj, q_off, k_off, v_off, i_off, f_off, H, dk, dv, i_bias,
                f_bias, cap: float, mem, mstate, state_slots, query_start_locs,
-               seq_lens):
+               seq_lens, longest: int = 0):
+    """`longest`: as in delta_scan."""
     if proj.is_cuda:
         T = proj.shape[0]
         o = torch.empty((T, H, dv + 1), dtype=torch.float32,
@@ -309,7 +312,7 @@ def mlstm_scan(proj, q_off, k_off, v_off, i_off, f_off, H, dk, dv, i_bias,
         em = torch.empty((T, H), dtype=torch.float32, device=proj.device)
         _mix().mlstm_scan(o, em, proj, q_off, k_off, v_off, i_off, f_off,
                           i_bias, f_bias, cap, mem, mstate, state_slots,
-                          query_start_locs, seq_lens)
+                          query_start_locs, seq_lens, longest)
         return o, em
     return torch_ref.mlstm_scan(proj, q_off, k_off, v_off, i_off, f_off, H,
                                 dk, dv, i_bias, f_bias, cap, mem, mstate,
@@ -533,16 +536,17 @@ def ssd_prep(proj, xbc_off: int, dt_off: int, H: int, dv: int, G: int, N: int,
 
 
 def decay_scan(q, k, v, decay, gain, skip, state, state_slots,
-               query_start_locs, seq_lens):
+               query_start_locs, seq_lens, longest: int = 0):
     """S <- decay S + gain k v^T, o = S^T q + skip v per sequence and head
     over the new tokens; q, k [T, G, dk], v [T, H, dv] fp32 (row-strided views
     are fine), decay [T, H] or [H], gain [T, H] or None, skip [H] or None,
-    state [slots, H, dk, dv] fp32. Returns o [T, H, dv] fp32."""
+    state [slots, H, dk, dv] fp32; `longest` as in delta_scan. Returns o [T, H, dv]
+    fp32."""
     if v.is_cuda:
         T, H, dv = v.shape
         o = torch.empty((T, H, dv), dtype=torch.float32, device=v.device)
         _mix().decay_scan(o, q, k, v, decay, gain, skip, state, state_slots,
-                          query_start_locs, seq_lens)
+                          query_start_locs, seq_lens, longest)
         return o
     return torch_ref.decay_scan(q, k, v, decay, gain, skip, state,
                                 state_slots, query_start_locs, seq_lens)

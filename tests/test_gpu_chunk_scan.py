@@ -465,6 +465,57 @@ def test_long_sequences_among_many(kind, front):
         tol = TOL
     assert _off(o[front:], want[front:].double()) < tol
     assert _off(st, end.double()) < tol
+    # the longest of them makes no difference but to the kernels that are taken
+    for longest in (131, 1):
+        again = state.to(DEV)
+        if kind == "mlstm":
+            o, _ = hops.mlstm_scan(proj.to(DEV), *offs, H, dk, dv, ib.to(DEV), fb.to(DEV),
+                                   5.0, again, m0.to(DEV), *meta, longest)
+        elif kind == "decay":
+            o = hops.decay_scan(*(x.to(DEV) for x in (q, k, v, a, b)), None, again, *meta,
+                                longest)
+        else:
+            o = hops.delta_scan(*(x.to(DEV) for x in (q, k, v, d, b)), again, *meta, longest)
+        assert _off(o[front:], want[front:].double()) < tol
+        assert _off(again, end.double()) < tol
     for s, n in zip(slots.tolist(), lens):
         if not n:
             assert torch.equal(st[s].cpu(), state[s])
+
+
+@pytest.mark.parametrize("dk,dv,H,S,n", [
+    (128, 32, 16, 40, 70), (128, 32, 16, 4, 200), (16, 64, 16, 80, 40), (16, 16, 4, 3, 40),
+    (64, 64, 16, 33, 50), (64, 128, 16, 33, 26), (128, 128, 16, 17, 66), (96, 96, 16, 40, 97)])
+def test_both_sides_of_the_rule(dk, dv, H, S, n):
+    """A round of workgroups and more of them: sequences of n tokens on either side, and
+    one that is longer than all others can be."""
+    g = torch.Generator().manual_seed(n)
+    lens = [n] * (S - 1) + [n * 3]
+    qlocs = torch.tensor([0] + lens).cumsum(0).int()
+    T = int(qlocs[-1])
+    total, slots = torch.tensor(lens).int() + 1, torch.arange(S).int()
+    unit = torch.nn.functional.normalize
+    q, k = (unit(torch.randn(T, H, dk, generator=g), dim=-1) for _ in "qk")
+    v = torch.randn(T, H, dv, generator=g)
+    a, b = torch.rand(T, H, generator=g), torch.rand(T, H, generator=g)
+    state = torch.randn(S, H, dk, dv, generator=g)
+    meta = [x.to(DEV) for x in (slots, qlocs, total)]
+    x = [y.to(DEV) for y in (q, k, v, a, b)]
+    for delta in (False, True):
+        st = state.to(DEV)
+        want = torch.zeros(T, H, dv, dtype=torch.float64, device=DEV)
+        end = state.to(DEV).double()
+        for t in range(3 * n):          # all sequences side by side, on the GPU
+            live = [s for s in range(S) if t < lens[s]]
+            at = (qlocs[:-1][live].long() + t).to(DEV)
+            live = torch.tensor(live, device=DEV)
+            P = end[live] * a.to(DEV).double()[at][:, :, None, None]
+            kk, vv, bb = (y.double()[at] for y in (x[1], x[2], x[4]))
+            u = vv - (P * kk[..., None]).sum(2) if delta else vv
+            P = P + kk[..., None] * (bb[..., None] * u)[:, :, None, :]
+            want[at] = (P * x[0].double()[at][..., None]).sum(2)
+            end[live] = P
+        f = hops.delta_scan if delta else hops.decay_scan
+        o = f(*x, *(() if delta else (None,)), st, *meta)
+        assert float((o.double() - want).norm() / want.norm()) < TOL
+        assert float((st.double() - end).norm() / end.norm()) < TOL
