@@ -123,3 +123,28 @@ def test_experts(kind):
     unit, c = (clamped, 1.702) if kind == "clamped" else (silu, 1.0)
     _check(out, _want(x, w, lambda g, u: unit(g * y, u * y)),
            _want(x, w, lambda g, u: -c * y * g))
+
+
+@pytest.mark.parametrize("tiles,blocks", [
+    (5, 8), (5, 9), (5, 15), (6, 9), (11, 46), (13, 39), (9, 29), (35, 11), (33, 60), (7, 8)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_every_tile_once(tiles, blocks, gated):
+    """Row tiles by column blocks at which the last rows go to the XCDs by single tiles, or
+    not: whole numbers come out as they are."""
+    M, N, K = tiles * 256 - 5, blocks * (128 if gated else 256), 64
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randint(-2, 3, (M, K), generator=g, device=DEV).bfloat16()
+    w = torch.randint(-2, 3, (2 * N if gated else N, K), generator=g, device=DEV).bfloat16()
+    y = x.float() @ w.float().T
+    if gated:
+        got = ops._require_hip().linear_silu_mul(x, w)
+        want = torch.nn.functional.silu(y[:, :N]) * y[:, N:]
+        assert ((got.float() - want).abs() <= want.abs() * 2 ** -8).all()
+        return
+    off = torch.tensor([0, tiles], dtype=torch.int32, device=DEV)
+    cnt = torch.tensor([M], dtype=torch.int32, device=DEV)
+    a = torch.zeros(tiles * 256, K, dtype=torch.bfloat16, device=DEV)
+    a[:M] = x
+    out = torch.zeros(tiles * 256, N, dtype=torch.bfloat16, device=DEV)
+    hops.expert_gemm(out, a, w[None], None, off, cnt, hops.ACT_NONE, 256)
+    assert torch.equal(out[:M].float(), y.bfloat16().float())
