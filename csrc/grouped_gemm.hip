@@ -477,9 +477,11 @@ __device__ __forceinline__ u32 gw_pack(float x, float y) {
 // 4096 rows 1661 -> 1604, 187 rows 126.5 -> 123.3, in turn on one card, with 9. 1.3e9
 // results were the same to the bit.
 // d = 1 + exp(-v) passes 2^126 for v below -87.3, and its reciprocal, too small a number,
-// is 0 then (-5e-37 for v = -88 was). So v and d are taken as quarters, the tenth
-// operation (0.3 %: 24,000 rows 234.7 and 236.0, 32,768 1519.5 and 1523.5), which changes
-// no other bit, but of v below 2^-124. GELU by tanh has long been 0 there.
+// is 0 then (-5e-37 for v = -88 was). So v and d are taken as quarters, which changes no
+// other bit, but of v below 2^-124; it is the tenth operation (24,000 rows of k 1024 236.0
+// us instead of 234.7, 32,768 of 2048 1523.5 and 1519.5, 2688 of 2 x 8064 x 320 35.8 and
+// 34.5), but where the row's weight or the clamped up takes the quarter. GELU by tanh has
+// long been 0 there.
 template <int MODE>
 __device__ __forceinline__ void gw_unit8(float (&v)[8], float (&u)[8], float limit,
                                          float rw) {
@@ -498,13 +500,13 @@ __device__ __forceinline__ void gw_unit8(float (&v)[8], float (&u)[8], float lim
     GW_EACH(d[i] = d[i] * v[i])
   } else if (MODE == 3) {
     GW_EACH(v[i] = fminf(v[i], limit))
-    GW_EACH(u[i] = fminf(fmaxf(u[i], -limit), limit) + 1.0f)
+    GW_EACH(u[i] = fmaf(fminf(fmaxf(u[i], -limit), limit), Q, Q))   // (v stays)
     GW_EACH(d[i] = v[i] * -1.702f)
     GW_EACH(d[i] = d[i] * 1.4426950408889634f)
   } else {
     GW_EACH(d[i] = v[i] * (-1.4426950408889634f / (MODE == 4 ? Q : 1.f)))
   }
-  if (MODE != 4 && MODE != 6) { GW_EACH(v[i] *= Q) }
+  if (MODE != 3 && MODE != 4 && MODE != 6) { GW_EACH(v[i] *= Q) }
   GW_EACH(d[i] = __builtin_amdgcn_exp2f(d[i]))
   GW_EACH(d[i] = fmaf(d[i], Q, Q))
   GW_EACH(r[i] = __builtin_amdgcn_rcpf(d[i]))
