@@ -56,6 +56,9 @@ void sutro_linear_silu_mul(void*, const void*, const void*, int, int, long,
                            hipStream_t);
 void sutro_linear_gelu_mul(void*, void*, const void*, const void*, const void*, int,
                            int, int, long, hipStream_t);
+void sutro_linear_heads(void*, void*, void*, const void*, const void*, const long*,
+                        const long*, const float*, const void*, const void*, float,
+                        int, int, int, int, long, hipStream_t);
 void sutro_moe_combine(void*, const void*, const void*, int, const float*, int,
                        int, int, hipStream_t);
 void sutro_moe_topk(int*, float*, const void*, long, int, int, int, int,
@@ -464,6 +467,42 @@ std::vector<torch::Tensor> linear_gelu_mul(torch::Tensor x, torch::Tensor w,
   return {out, rest};
 }
 
+// heads of 128 of x w^T: query heads normed and rotated (returned), key heads likewise
+// and value heads as they are to the tokens' slots
+torch::Tensor linear_heads(torch::Tensor x, torch::Tensor w, torch::Tensor k_cache,
+                           torch::Tensor v_cache, torch::Tensor positions,
+                           torch::Tensor slot_mapping, torch::Tensor cos_sin,
+                           c10::optional<torch::Tensor> q_norm_w,
+                           c10::optional<torch::Tensor> k_norm_w, double eps) {
+  CHECK_CONTIG(k_cache); CHECK_CONTIG(v_cache); CHECK_CONTIG(cos_sin);
+  CHECK_BF16(k_cache); CHECK_BF16(v_cache);
+  CHECK_CONTIG(positions); CHECK_CONTIG(slot_mapping);
+  check_gated(x, w, 128);
+  const long M = x.size(0), K = x.size(1), bs = k_cache.size(2);
+  const long Hk = k_cache.size(1), Hq = w.size(0) / 128 - 2 * Hk;
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(3) == 128 &&
+              v_cache.sizes() == k_cache.sizes() && bs > 0 && (bs & (bs - 1)) == 0 &&
+              k_cache.numel() >> 7 < (1l << 32) && Hk > 0 && Hq > 0 && Hq % 2 == 0 &&
+              w.size(0) == (Hq + 2 * Hk) * 128 && K >= 192, "unsupported sizes");
+  TORCH_CHECK(positions.numel() == M && slot_mapping.numel() == M &&
+              cos_sin.dim() == 2 && cos_sin.size(1) == 128, "tokens");
+  for (const auto& n : {q_norm_w, k_norm_w})
+    TORCH_CHECK(!n || (n->scalar_type() == at::kBFloat16 && n->is_contiguous() &&
+                       n->numel() == 128 && (size_t)n->data_ptr() % 8 == 0), "norm");
+  for (const auto& t : {k_cache, v_cache, cos_sin})
+    TORCH_CHECK((size_t)t.data_ptr() % 16 == 0, "16-byte rows");
+  auto q = torch::empty({M, Hq, 128}, x.options());
+  int shift = 0;
+  while (1l << shift < bs) ++shift;
+  sutro_linear_heads(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                     x.data_ptr(), w.data_ptr(), positions.data_ptr<long>(),
+                     slot_mapping.data_ptr<long>(), cos_sin.data_ptr<float>(),
+                     q_norm_w ? q_norm_w->data_ptr() : nullptr,
+                     k_norm_w ? k_norm_w->data_ptr() : nullptr, (float)eps, (int)M,
+                     (int)Hq, (int)Hk, shift, K, cur_stream());
+  return q;
+}
+
 void sampler_fused(torch::Tensor logits, torch::Tensor temps,
                    torch::Tensor topps, torch::Tensor topks, torch::Tensor us,
                    c10::optional<torch::Tensor> mask, long vl,
@@ -514,6 +553,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "linear layer of one row behind an addition and RMSNorm");
   m.def("linear_gelu_mul", &linear_gelu_mul,
         "linear layer with the GELU gate behind its first columns, many rows");
+  m.def("linear_heads", &linear_heads,
+        "QKV projection with qk-norm, RoPE and KV write behind it, many rows");
   m.def("linear_silu_mul", &linear_silu_mul,
         "linear layer with the silu gate behind it, many rows");
   m.def("moe_layout", &moe_layout, "softmax top-k router + expert segments");

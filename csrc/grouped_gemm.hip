@@ -360,6 +360,20 @@ struct GwFlag {
   static constexpr bool v = V != 0;
 };
 
+// What mode 7 makes of the products: columns of 128 are heads, hq of queries, hk of
+// keys, hk of values (see store_heads).
+struct GwHeads {
+  u16* kc;                 // pages [blocks, hk, 1 << shift, 128], fewer than 2^32 tokens
+  u16* vc;
+  const long* pos;         // [M]
+  const long* slots;       // [M]
+  const float* cos_sin;    // [positions, 128]
+  const u16* qw;           // [128] or null
+  const u16* kw;
+  float eps;
+  int hq, hk, shift;
+};
+
 // an output tile: first row, first column, expert, live rows from the first on
 struct GwTile {
   long seg;
@@ -545,9 +559,9 @@ __device__ __forceinline__ void gw_body(
     const int* __restrict__ tile_off, const int* __restrict__ counts,
     int n_experts, int n_cols, long K, float limit,
     const float* __restrict__ row_w, int m_rows, const u16* __restrict__ bias,
-    u16* __restrict__ rest, int n_rest) {
-  constexpr bool GATED = MODE == 1 || MODE >= 3;
-  constexpr bool DENSE = MODE >= 5, REST = MODE == 6;
+    u16* __restrict__ rest, int n_rest, const GwHeads& H) {
+  constexpr bool GATED = MODE == 1 || (MODE >= 3 && MODE < 7);
+  constexpr bool DENSE = MODE >= 5, REST = MODE == 6, HEADS = MODE == 7;
   constexpr bool GATHER = MODE != 0 && !DENSE;
   constexpr int BN = GATED ? 128 : 256;   // output columns
   const int nb = n_cols / BN + (REST ? n_rest / 256 : 0);
@@ -646,6 +660,14 @@ __device__ __forceinline__ void gw_body(
 
   // The sums are transposed (B rows first), so a lane has four columns of a row;
   // lanes of neighbouring column tiles swap halves: 16 bytes a lane and store.
+  auto pack8 = [](const float (&x)[8]) {
+    u32 p[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = gw_pack(x[2 * q], x[2 * q + 1]);
+    const auto s0 = __builtin_amdgcn_permlane16_swap(p[0], p[2], false, false);
+    const auto s1 = __builtin_amdgcn_permlane16_swap(p[1], p[3], false, false);
+    return u32x4{s0[0], s1[0], s0[1], s1[1]};
+  };
   auto store_tile = [&](const GwTile& g) {
     const u32 off = (u32)(ln * n_cols + (quad & 1) * 16 + (quad >> 1) * 8) * 2;
     const long row = g.seg + wm * 128;
@@ -663,14 +685,6 @@ __device__ __forceinline__ void gw_body(
       more = (char*)(rest + row * n_rest + 2 * (g.n0 - n_cols) + wn * 64 +
                      (long)ln * n_rest + (quad & 1) * 16 + (quad >> 1) * 8);
     }
-    auto pack = [](const float (&x)[8]) {
-      u32 p[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) p[q] = gw_pack(x[2 * q], x[2 * q + 1]);
-      const auto s0 = __builtin_amdgcn_permlane16_swap(p[0], p[2], false, false);
-      const auto s1 = __builtin_amdgcn_permlane16_swap(p[1], p[3], false, false);
-      return u32x4{s0[0], s1[0], s0[1], s1[1]};
-    };
 #pragma unroll
     for (int i = 0; i < 8; ++i, at += (long)n_cols * 32) {
       const float rw = MODE == 4 ? row_w[row + i * 16 + ln] : 1.f;
@@ -703,7 +717,7 @@ __device__ __forceinline__ void gw_body(
           }
           if (!gate) {
             u16* o = (u16*)(more + (long)i * n_rest * 32) + j * 16;
-            const u32x4 pa = pack(x), pb = pack(up);
+            const u32x4 pa = pack8(x), pb = pack8(up);
             if (wm * 128 + i * 16 + ln < g.live) {
               *(u32x4*)o = pa;
               *(u32x4*)(o + 128) = pb;
@@ -713,7 +727,7 @@ __device__ __forceinline__ void gw_body(
           }
         }
         if (GATED) gw_unit8<MODE>(x, up, limit, rw);
-        const u32x4 pk = pack(x);
+        const u32x4 pk = pack8(x);
         u16* o = (u16*)(at + off) + j * 16;
         if (DENSE && wm * 128 + i * 16 + ln >= g.live) {
         } else if (ANY) {
@@ -725,6 +739,120 @@ __device__ __forceinline__ void gw_body(
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+    }
+  };
+
+  // Mode 7: a wave's 128 columns are one head, of which a lane has 32 columns of a row
+  // and the lanes of equal ln the others: RMS norm (sums in registers and across four
+  // lanes), rotation (columns d and d + 64 in the same lane) and the store to the
+  // queries or to the token's slot, on fp32 products. By itself that pass reads and
+  // writes all heads once more, at the rate of memory (78 us for 24,000 tokens of 32
+  // heads, with the library's product of k 1024 267; here 198, of which 165 are the
+  // product's; 32,768 of 24 heads, k 2048 383 -> 340; of 48, k 4096 1245 -> 1222).
+  // Positions and slots of all rows are asked for first and each row's cosines while
+  // the row before is computed, as no other wave hides them.
+  auto store_heads = [&](const GwTile& g, auto plain_c) {
+    constexpr bool PLAIN = decltype(plain_c)::v;
+    const int hd = (g.n0 >> 7) + wn;
+    const bool isq = hd < H.hq;
+    const int kh = hd - H.hq - (PLAIN ? H.hk : 0);
+    const long row0 = g.seg + wm * 128;
+    const int live = g.live - wm * 128;     // of this wave's rows
+    u32 pos[PLAIN ? 1 : 8], slot[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      // (a wave may have no live row: then the tile's last)
+      const long row = g.seg + min(wm * 128 + i * 16 + ln, g.live - 1);
+      if (!PLAIN) pos[PLAIN ? 0 : i] = (u32)H.pos[row];
+      slot[i] = isq ? 0 : (u32)H.slots[row];
+    }
+    u16x4 nw[PLAIN ? 1 : 8];
+    f32x4 cs[4], sn[4];
+    const u16* wv = isq ? H.qw : H.kw;
+    auto turn = [&](int i, int j) {
+      const float* t = H.cos_sin + (long)pos[PLAIN ? 0 : i] * 128 + j * 16 + quad * 4;
+      cs[j] = *(const f32x4*)t;
+      sn[j] = *(const f32x4*)(t + 64);
+    };
+    if (!PLAIN) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) turn(0, j);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        nw[PLAIN ? 0 : j] =
+            wv ? *(const u16x4*)(wv + j * 16 + quad * 4) : (u16x4)(0x3f80);
+    }
+    const int off = (quad & 1) * 16 + (quad >> 1) * 8;
+    u16* const to = !PLAIN && isq ? out : PLAIN ? H.vc : H.kc;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x[8][4];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        asm volatile("" : "+a"(acc[i][j]));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[j][e] = acc[i][j][e];
+        acc[i][j] = (f32x4)(0.f);
+      }
+      const u32 page = (slot[i] >> H.shift) * H.hk + kh;
+      long at = (((long)page << H.shift) + (slot[i] & ((1u << H.shift) - 1))) * 128;
+      if (!PLAIN && isq) at = ((row0 + i * 16 + ln) * H.hq + hd) * 128;
+      at += off;
+      float inv = 1.f;
+      if (!PLAIN) {
+        float q[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = x[j][0] * x[j][0];
+#pragma unroll
+        for (int e = 1; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) q[j] = fmaf(x[j][e], x[j][e], q[j]);
+        const float sum =
+            ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+        const u32 b = __float_as_uint(sum);
+        const auto h = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        const u32 c =
+            __float_as_uint(__uint_as_float(h[0]) + __uint_as_float(h[1]));
+        const auto f = __builtin_amdgcn_permlane16_swap(c, c, false, false);
+        inv = rsqrtf((__uint_as_float(f[0]) + __uint_as_float(f[1])) * (1.f / 128) +
+                     H.eps);
+        if (!wv) inv = 1.f;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        float lo[8], hi[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int t = j + (q >> 2), e = q & 3;
+          lo[q] = x[t][e];
+          hi[q] = x[t + 4][e];
+          if (!PLAIN) {
+            const float a = lo[q] * (inv * bf2f(nw[PLAIN ? 0 : t][e]));
+            const float b = hi[q] * (inv * bf2f(nw[PLAIN ? 0 : t + 4][e]));
+            lo[q] = a * cs[t][e] - b * sn[t][e];
+            hi[q] = b * cs[t][e] + a * sn[t][e];
+          }
+        }
+        if (!PLAIN && i < 7) {
+          turn(i + 1, j);
+          turn(i + 1, j + 1);
+        }
+        const u32x4 first = pack8(lo), second = pack8(hi);
+        if (i * 16 + ln < live) {
+          *(u32x4*)(to + at + j * 16) = first;
+          *(u32x4*)(to + at + j * 16 + 64) = second;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  auto finish = [&](const GwTile& g) {
+    if constexpr (HEADS) {
+      if ((g.n0 >> 7) + wn >= H.hq + H.hk) store_heads(g, GwFlag<1>{});
+      else store_heads(g, GwFlag<0>{});
+    } else {
+      store_tile(g);
     }
   };
 
@@ -825,7 +953,7 @@ __device__ __forceinline__ void gw_body(
   };
 
   point(cur, src);
-  if (KT < 3) {       // too short to run across tiles
+  if (!HEADS && KT < 3) {       // too short to run across tiles
     for (;;) {
       open();
       if (KT == 2) {
@@ -834,7 +962,7 @@ __device__ __forceinline__ void gw_body(
       } else {
         step(0, no, no);
       }
-      store_tile(cur);
+      finish(cur);
       if (!next(cur)) return;
       point(cur, src);
       kc = first(cur);
@@ -862,7 +990,7 @@ __device__ __forceinline__ void gw_body(
       step(0, no, yes);
       step(0, no, no);
     }
-    store_tile(cur);
+    finish(cur);
     if (!more) return;
     cur = nxt;
   }
@@ -875,9 +1003,10 @@ gw_kernel(u16* __restrict__ out, const u16* __restrict__ a,
           const int* __restrict__ tile_off, const int* __restrict__ counts,
           int n_experts, int n_cols, long K, float limit,
           const float* __restrict__ row_w, int m_rows,
-          const u16* __restrict__ bias, u16* __restrict__ rest, int n_rest) {
+          const u16* __restrict__ bias, u16* __restrict__ rest, int n_rest,
+          GwHeads heads) {
   gw_body<MODE, ANY>(out, a, w, row_tok, tile_off, counts, n_experts, n_cols, K,
-                     limit, row_w, m_rows, bias, rest, n_rest);
+                     limit, row_w, m_rows, bias, rest, n_rest, heads);
 }
 
 // a workgroup a CU, a multiple of 8 of them
@@ -925,7 +1054,7 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
     static std::atomic<unsigned long long> asked{0};                        \
     lds_limit((const void*)gw_kernel<M, ANY>, GW_LDS, asked);               \
     hipLaunchKernelGGL((gw_kernel<M, ANY>), grid, dim3(256), GW_LDS,        \
-                       stream, GG_ARGS, 0, nullptr, nullptr, 0);                             \
+                       stream, GG_ARGS, 0, nullptr, nullptr, 0, GwHeads{});  \
   }
 #define GG_WIDE(M)                                                          \
   {                                                                         \
@@ -969,14 +1098,15 @@ static void grouped_gemm_launch(void* out, const void* a, long a_rows,
 template <int MODE>
 static void gw_dense(void* out, void* rest, const void* x, const void* w,
                      const void* bias, int M, int N, int n_rest, long K,
-                     hipStream_t stream) {
+                     hipStream_t stream, const GwHeads& heads = GwHeads{}) {
+  const int blocks = N / (MODE == 7 ? 256 : 128) + n_rest / 256;
   static std::atomic<unsigned long long> asked{0};
   lds_limit((const void*)gw_kernel<MODE, false>, GW_LDS, asked);
   hipLaunchKernelGGL((gw_kernel<MODE, false>),
-                     dim3(gw_grid(((long)M + 255) / 256, N / 128 + n_rest / 256)),
+                     dim3(gw_grid(((long)M + 255) / 256, blocks)),
                      dim3(256), GW_LDS, stream, (u16*)out, (const u16*)x,
                      (const u16*)w, nullptr, nullptr, nullptr, 0, N, K, 0.f,
-                     nullptr, M, (const u16*)bias, (u16*)rest, n_rest);
+                     nullptr, M, (const u16*)bias, (u16*)rest, n_rest, heads);
 }
 
 // out [M, N] = silu(x Wg^T) * (x Wu^T): w [2 N, K], the gate's rows first. x and w at
@@ -994,6 +1124,20 @@ extern "C" void sutro_linear_gelu_mul(void* out, void* rest, const void* x,
                                       const void* w, const void* bias, int M, int N,
                                       int n_rest, long K, hipStream_t stream) {
   gw_dense<6>(out, rest, x, w, bias, M, N, n_rest, K, stream);
+}
+
+// x w^T as heads of 128, w [(hq + 2 hk) 128, K] with hq even: query heads normed and
+// rotated to q [M, hq, 128], key heads likewise and value heads as they are to their
+// tokens' slots in pages of 1 << shift tokens, bf16. Operands at multiples of
+// 16 bytes, K as above and 192 or more.
+extern "C" void sutro_linear_heads(void* q, void* kc, void* vc, const void* x,
+                                   const void* w, const long* pos, const long* slots,
+                                   const float* cos_sin, const void* qw,
+                                   const void* kw, float eps, int M, int hq, int hk,
+                                   int shift, long K, hipStream_t stream) {
+  const GwHeads heads = {(u16*)kc, (u16*)vc, pos, slots, cos_sin, (const u16*)qw,
+                         (const u16*)kw, eps, hq, hk, shift};
+  gw_dense<7>(q, nullptr, x, w, nullptr, M, (hq + 2 * hk) * 128, 0, K, stream, heads);
 }
 
 extern "C" void sutro_grouped_gemm(void* out, const void* a, long a_rows,

@@ -93,17 +93,20 @@ class Qwen3Attention(nn.Module):
                 kv: PagedKVCache, cos_sin: torch.Tensor,
                 qkv: Optional[torch.Tensor] = None) -> torch.Tensor:
         """`qkv`: the projection of x, where the caller has made it."""
-        if qkv is None:
-            qkv = self.qkv_proj(x)
-        T = qkv.shape[0]
-        q = ops.fused_qkv_prep(
-            qkv, self.num_heads, self.num_kv_heads, self.head_dim,
-            fb.positions, fb.slot_mapping,
-            kv.k_cache[self.layer_idx], kv.v_cache[self.layer_idx], cos_sin,
-            self.q_norm.weight if self.qk_norm else None,
-            self.k_norm.weight if self.qk_norm else None,
-            self.q_norm.eps if self.qk_norm else 1e-6,
-        )
+        heads = (self.num_heads, self.num_kv_heads, self.head_dim,
+                 fb.positions, fb.slot_mapping,
+                 kv.k_cache[self.layer_idx], kv.v_cache[self.layer_idx], cos_sin,
+                 self.q_norm.weight if self.qk_norm else None,
+                 self.k_norm.weight if self.qk_norm else None,
+                 self.q_norm.eps if self.qk_norm else 1e-6)
+        q = None
+        if qkv is None and bare(self.qkv_proj):
+            q = ops.linear_qkv_prep(x, self.qkv_proj.weight, *heads)
+        if q is None:
+            if qkv is None:
+                qkv = self.qkv_proj(x)
+            q = ops.fused_qkv_prep(qkv, *heads)
+        T = q.shape[0]
         o = ops.paged_attention(q, kv.k_cache[self.layer_idx],
                                 kv.v_cache[self.layer_idx], fb.block_tables,
                                 fb.seq_lens, fb.query_start_locs, self.scale,

@@ -614,6 +614,45 @@ def linear_silu_rows(x, w):
     return _require_hip().linear_silu_mul(x, w) if _many_rows(x, w) else None
 
 
+def _last_round(x, w) -> float:
+    """Of all places in the rounds of 256 tiles of 256 x 256, those that are taken."""
+    tiles = -(-x.shape[0] // 256) * (w.shape[0] // 256)
+    return tiles / (-(-tiles // 256) * 256)
+
+
+def linear_qkv_prep(x, w, num_heads: int, num_kv_heads: int, head_dim: int,
+                    positions, slot_mapping, k_cache, v_cache, cos_sin,
+                    q_norm_w=None, k_norm_w=None, eps: float = 1e-6):
+    """fused_qkv_prep of x w^T where one launch makes it (prompts), else None. us of the
+    library's product with the pass over its result, and of this one, by rows:
+       4096 x  512    4096   35.5 /  27.9     6000   62.5 /  46.1    24000  203 / 136
+       4096 x 1024    3000   36.3 /  34.3     4096   44.6 /  38.0    24000  267 / 198
+       3072 x 2048    6000   99.1 / 101.3     8192  108.7 / 106.6    32768  383 / 340
+       6144 x 4096    6000    257 /  281      8192    310 /  304     32768 1245 / 1222
+      10240 x 5120    3000    241 /  246      6000    517 /  481     16384 1290 / 1244
+    From a k of 2048 on the library's product is 4 to 7 % faster than the one here and
+    the pass small beside it: then where the last round is nearly full."""
+    caches = (k_cache, v_cache)
+    if not (head_dim == 128 and num_heads % 2 == 0 and _many_rows(x, w)
+            and x.shape[1] >= 192
+            and (x.shape[1] <= 2048 or _last_round(x, w) >= 0.95)
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in caches)
+            and k_cache.shape == v_cache.shape
+            and k_cache.shape[2] & (k_cache.shape[2] - 1) == 0
+            and k_cache.numel() >> 7 < 1 << 32
+            and cos_sin.is_contiguous() and cos_sin.data_ptr() % 16 == 0
+            and cos_sin.dtype == torch.float32 and cos_sin.shape[1:] == (128,)
+            and positions.is_contiguous() and slot_mapping.is_contiguous()
+            and all(n is None or (n.dtype == torch.bfloat16 and n.is_contiguous()
+                                  and n.data_ptr() % 8 == 0)
+                    for n in (q_norm_w, k_norm_w))):
+        return None
+    return _require_hip().linear_heads(x, w, k_cache, v_cache, positions,
+                                       slot_mapping, cos_sin, q_norm_w, k_norm_w,
+                                       eps)
+
+
 def _one_row(x, residual, norm_w, w, gated: bool) -> bool:
     """Whether csrc/gemm_skinny.hip makes the norm of one row inside the product
     behind it. Up to 4096 waves make it, each workgroup for itself, and with short
