@@ -46,7 +46,7 @@ void sutro_qkv_prep(const void*, void*, void*, void*, const long*, const long*,
                     int, int, int, int, int, hipStream_t);
 void sutro_sampler_fused(const void*, int, const float*, const float*,
                          const int*, const float*, const unsigned int*, int,
-                         long, int, int, int*, float*, hipStream_t);
+                         long, int, int, int*, float*, int, hipStream_t);
 void sutro_grouped_gemm(void*, const void*, long, const void*, const int*,
                         const int*, const int*, int, int, int, long, int,
                         int, hipStream_t);
@@ -506,7 +506,7 @@ torch::Tensor linear_heads(torch::Tensor x, torch::Tensor w, torch::Tensor k_cac
 void sampler_fused(torch::Tensor logits, torch::Tensor temps,
                    torch::Tensor topps, torch::Tensor topks, torch::Tensor us,
                    c10::optional<torch::Tensor> mask, long vl,
-                   torch::Tensor out_tok, torch::Tensor out_lp) {
+                   torch::Tensor out_tok, torch::Tensor out_lp, bool greedy) {
   CHECK_CUDA(logits); CHECK_CONTIG(logits);
   const bool f32 = logits.scalar_type() == at::kFloat;
   TORCH_CHECK(f32 || logits.scalar_type() == at::kBFloat16,
@@ -532,7 +532,7 @@ void sampler_fused(torch::Tensor logits, torch::Tensor temps,
                       topks.data_ptr<int>(), us.data_ptr<float>(), mptr,
                       (int)n, v_row, (int)vl, w_words,
                       out_tok.data_ptr<int>(), out_lp.data_ptr<float>(),
-                      cur_stream());
+                      greedy ? 1 : 0, cur_stream());
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -561,7 +561,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("grouped_gemm", &grouped_gemm,
         "dropless MoE grouped GEMM (padded segments, static grid)");
   m.def("sampler_fused", &sampler_fused,
-        "fused mask+temp+topk/topp+sample+logprob (radix descent, no sort)");
+        "fused mask+temp+topk/topp+sample+logprob (no sort)", py::arg("logits"),
+        py::arg("temps"), py::arg("topps"), py::arg("topks"), py::arg("us"),
+        py::arg("mask"), py::arg("vl"), py::arg("out_tok"), py::arg("out_lp"),
+        py::arg("greedy") = false);
   m.def("gemm_tn", &gemm_tn, "bf16 TN GEMM (MFMA, glds dbuf)",
         py::arg("x"), py::arg("w"), py::arg("res") = c10::nullopt,
         py::arg("bm") = 256, py::arg("bn") = 256, py::arg("swz") = 2,

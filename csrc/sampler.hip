@@ -37,6 +37,7 @@
 
 #define SMP_THREADS 256
 #define HREP 8  // level-0 histogram replicas
+#define SMP_LEFT -2  // token of a row that another kernel has to sample
 
 struct SmpArgs {
   const void* logits;
@@ -46,9 +47,10 @@ struct SmpArgs {
   const float* us;
   const u32* mask;
   long v_row;
-  int vl, w_words;
+  int n, vl, w_words;
   int* out_tok;
   float* out_lp;
+  bool left;            // only rows whose token is SMP_LEFT
 };
 
 // monotonic u32 key: key(a) < key(b)  <=>  a < b (floats, no NaN)
@@ -559,7 +561,8 @@ __global__ void __launch_bounds__(SMP_THREADS) sampler_kernel(SmpArgs A) {
 // 1024 x 151,936 by the general kernel and here: 1382 -> 197 us (top_p 0.95 at
 // temperature 0.8), 1393 -> 151 with top_k 20, 1338 -> 250
 // with a mask; one row 636 -> 41 us. Of the 50 us that a row takes its
-// workgroup 16 are fixed, clearing and scanning 128 KB of counters.
+// workgroup 16 are fixed, clearing and scanning 128 KB of counters. Greedy rows, those
+// of more than 155,648 logits and what sampler_fast_kernel leaves come here.
 #define CNT_MIN 2048
 #define CNT_THREADS 1024
 #define CNT_WAVES (CNT_THREADS / 64)
@@ -627,6 +630,7 @@ sampler_count_kernel(SmpArgs A) {
   extern __shared__ __attribute__((aligned(16))) char cnt_lds[];
   CountShared& sm = *(CountShared*)cnt_lds;
   const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  if (A.left && A.out_tok[row] != SMP_LEFT) return;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const u16* lrow = (const u16*)A.logits + (long)row * A.v_row;
   const u8* mrow = MASKED ? (const u8*)(A.mask + (long)row * A.w_words)
@@ -1112,30 +1116,548 @@ sampler_count_kernel(SmpArgs A) {
   }
 }
 
+// ---- bf16 rows, most of them: counts of fewer values, by quarters of the row ----
+//
+// The counts above are of 65,536 values, so that a CU has room for one row's, and what
+// selects has to go through the whole row again, a dozen instructions a logit. Here a
+// logit is counted under its sign and its magnitude between 2^-24 and 255, 8192 values
+// in 32 bits, in four tables, one for each quarter of the row. They tell the kept mass of
+// every quarter, and only the one that u falls into is read again. What lies outside is
+// counted at the ends. That is exact where the largest logit is from 2 to 254 (a magnitude
+// of 2^-24 or less then vanishes in the difference to it) and where nothing lies below
+// -255 or all of it is 0 as a weight; other rows, with NaN or +inf among them, and
+// greedy ones are left to the kernel above, which runs behind this one.
+//
+// One workgroup a CU stays for all of its rows: where a piece of the row has been counted,
+// the same piece of the next row is asked for, so that the copies run on beside the
+// counting, the thresholds and the selection.
+// Bound by instruction issue and LDS additions while it counts (four instructions and an
+// addition a logit, 9 of 20 us a row), the chain of eight barriers behind it (7 us), and
+// the quarter (4). 1024 / 256 / 1 rows of 151,936, top_p 0.95 at temperature 0.8: 193 /
+// 49 / 41 us by the kernel above, 109 / 29 / 24 here; top_k 20 150 -> 105, with a mask
+// 248 -> 136, at temperature 3 194 -> 113; 1024 of 32,000 92 -> 53, of 2048 69 -> 39. Of
+// these 3 us are the launch that finds nothing left to do.
+#define FAST_PARTS 4
+#define FAST_BASE 0x3380        // bits of 2^-24
+#define FAST_TOP 4095           // 255, and what is larger
+#define FAST_SIGN 4096
+#define FAST_CODES 8192
+#define FAST_DEAD 0xc37fc37fu   // -255 twice
+#define FAST_BLK (FAST_PARTS * CNT_CHUNKS)
+#define FAST_RING 8             // pieces of a wave that are asked for ahead
+
+struct FastShared {
+  u32 cnt[FAST_PARTS][FAST_CODES];
+  u64 part[FAST_PARTS];         // kept mass
+  u64 blk[128];                 // of 512 logits of the quarter that u falls into
+  u64 wave_mass[CNT_WAVES];
+  u32 wave_cnt[CNT_WAVES];
+  float wave_z[CNT_WAVES];
+  int first, code;              // of the largest value: its thread, its magnitude
+  int one;                      // lowest value with p = 1, as bits
+  int low;                      // lowest kept value: magnitude, or -1 - magnitude
+  u32 odd, tau[2];
+  int token, last;
+};
+
+// v of the lane that CTRL names, `none` where there is none or ROWS leaves it out
+template <int CTRL, int ROWS = 15>
+__device__ __forceinline__ u32 dpp(u32 none, u32 v) {
+  return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 15, false);
+}
+template <int CTRL, int ROWS = 15>
+__device__ __forceinline__ u64 dpp(u64 none, u64 v) {
+  return (u64)dpp<CTRL, ROWS>((u32)(none >> 32), (u32)(v >> 32)) << 32 |
+         dpp<CTRL, ROWS>((u32)none, (u32)v);
+}
+template <int CTRL, int ROWS = 15>
+__device__ __forceinline__ float dpp(float none, float v) {
+  return __uint_as_float(
+      dpp<CTRL, ROWS>(__float_as_uint(none), __float_as_uint(v)));
+}
+// Inclusive scans over rows of 16 lanes and over the wave, without the LDS: of 16 waves
+// one may be alone with this.
+template <class T, class Op>
+__device__ __forceinline__ T row_scan(T v, T none, Op op) {
+  v = op(v, dpp<0x111>(none, v));    // from 1, 2, 4, 8 lanes below
+  v = op(v, dpp<0x112>(none, v));
+  v = op(v, dpp<0x114>(none, v));
+  return op(v, dpp<0x118>(none, v));
+}
+template <class T, class Op>
+__device__ __forceinline__ T lane_scan(T v, T none, Op op) {
+  v = row_scan(v, none, op);
+  v = op(v, dpp<0x142, 0xa>(none, v));   // lane 15 to the next row's, then 31
+  return op(v, dpp<0x143, 0xc>(none, v));
+}
+__device__ __forceinline__ u32 from_lane(u32 v, int l) {
+  return __builtin_amdgcn_readlane(v, l);
+}
+__device__ __forceinline__ u64 from_lane(u64 v, int l) {
+  return (u64)from_lane((u32)(v >> 32), l) << 32 | from_lane((u32)v, l);
+}
+struct AddOp {
+  template <class T>
+  __device__ T operator()(T a, T b) const { return a + b; }
+};
+struct MinOp {
+  __device__ u32 operator()(u32 a, u32 b) const { return min(a, b); }
+};
+
+// The first pieces of 512 logits of each wave's part of a row, and their masks.
+template <bool MASKED>
+struct FastRing {
+  u32x4 w[FAST_RING];
+  u32 bits[MASKED ? FAST_RING : 1];
+  __device__ __forceinline__ void load(const SmpArgs& A, int row, int slot, int i0) {
+    const int i = min(i0, (A.vl - 1) & ~7);
+    w[slot] = *(const u32x4*)((const u16*)A.logits + (long)row * A.v_row + i);
+    if (MASKED)
+      bits[MASKED ? slot : 0] =
+          ((const u8*)(A.mask + (long)row * A.w_words))[i >> 3];
+  }
+};
+
+// Samples the row that begins in r, and leaves the beginning of row `ahead` there, if that
+// is not negative. False: nothing was done.
+template <bool MASKED>
+__device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
+                                         char* lds, FastRing<MASKED>& r) {
+  FastShared& sm = *(FastShared*)lds;
+  // (what follows from these is made for each row: kept for all of them it took more
+  // registers than there are)
+  int tid = threadIdx.x, vl = A.vl;
+  asm volatile("" : "+v"(tid), "+s"(vl));
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const u16* lrow = (const u16*)A.logits + (long)row * A.v_row;
+  const u8* mrow = MASKED ? (const u8*)(A.mask + (long)row * A.w_words)
+                          : nullptr;
+  const int last8 = (vl - 1) & ~7;
+  const int part = (vl + CNT_CHUNK - 1) / CNT_CHUNK;   // pieces of a wave
+  // weight of a difference to the largest logit, and its whole part of 2^32 (of which
+  // those of 1 lack one: the conversion stops at 2^32 - 1)
+  const float inv_t = 1.0f / A.temps[row];
+  auto weight = [&](float d) { return __expf(d * inv_t); };
+  auto q32 = [&](float p) { return to_u32(p * 4294967296.0f); };
+
+  // logits that are not alive become `dead` (twice 16 bits)
+  auto patch = [&](u32x4& w, u32 bits, int i0, u32 dead) {
+    const int left = vl - i0;
+    if (left < 8) bits &= left > 0 ? (1u << left) - 1 : 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u32 keep = ((bits >> (2 * j)) & 1u) * 0xffffu |
+                       ((bits >> (2 * j + 1)) & 1u) * 0xffff0000u;
+      w[j] = (w[j] & keep) | (dead & ~keep);
+    }
+  };
+
+  {
+    u32x4* z = (u32x4*)sm.cnt;
+#pragma unroll
+    for (int i = 0; i < FAST_PARTS * FAST_CODES / 4 / CNT_THREADS; ++i)
+      z[i * CNT_THREADS + tid] = (u32x4)(0u);
+    if (tid < FAST_PARTS) sm.part[tid] = 0;
+    if (tid == 0) {
+      sm.first = CNT_THREADS;
+      sm.code = -1;
+      sm.one = 0x7f800000;
+      sm.low = FAST_CODES;
+      sm.odd = sm.tau[0] = sm.tau[1] = 0;
+      sm.token = sm.last = -1;
+    }
+  }
+  __syncthreads();
+
+  // ---- count ----
+  u16x2 most = (u16x2)(0);
+  {
+    typedef __attribute__((address_space(3))) u32 lds_u32;
+    lds_u32* const table = (lds_u32*)sm.cnt[wave * FAST_PARTS / CNT_WAVES];
+    const u32 base = (u32)(size_t)table;
+#pragma unroll
+    for (int c = 0; c < CNT_CHUNKS; ++c) {
+      const int i0 = (wave * part + c) * 512;
+      if (c < part) {
+        if (i0 < vl) {
+          u32x4 w = r.w[c % FAST_RING];
+          if (MASKED || i0 + 512 > vl) {
+            patch(w, MASKED ? r.bits[MASKED ? c % FAST_RING : 0] : 0xffu, i0 + lane * 8,
+                  FAST_DEAD);
+            if (!MASKED && lane == 0)      // they are not to be counted
+              atomicSub(&sm.cnt[wave * FAST_PARTS / CNT_WAVES][FAST_SIGN | FAST_TOP],
+                        (u32)(i0 + 512 - vl));
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const u16x2 mag = __builtin_bit_cast(u16x2, w[j] & 0x7fff7fffu);
+            most = __builtin_elementwise_max(most, mag);
+            u16x2 d = __builtin_elementwise_sub_sat(mag, (u16x2)(FAST_BASE));
+            d = __builtin_elementwise_min(d, (u16x2)(FAST_TOP));
+            const u32 a = ((w[j] >> 3) & (FAST_SIGN * 0x10001u)) |
+                          __builtin_bit_cast(u32, d);
+            u32 lo, hi;
+            asm("v_mad_u32_u16 %0, %1, 4, %2" : "=v"(lo) : "v"(a), "v"(base));
+            asm("v_mad_u32_u16 %0, %1, 4, %2 op_sel:[1,0,0,0]"
+                : "=v"(hi) : "v"(a), "v"(base));
+            // (under a mask -255 is not counted: all that are not alive would add there)
+            if (!MASKED || (a & 0xffffu) != (FAST_SIGN | FAST_TOP))
+              __hip_atomic_fetch_add((lds_u32*)(size_t)lo, 1u, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (!MASKED || a >> 16 != (FAST_SIGN | FAST_TOP))
+              __hip_atomic_fetch_add((lds_u32*)(size_t)hi, 1u, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+        }
+        if (c + FAST_RING < part)
+          r.load(A, row, c % FAST_RING, i0 + FAST_RING * 512 + lane * 8);
+        else if (ahead >= 0)
+          r.load(A, ahead, c % FAST_RING,
+                 (wave * part + c % FAST_RING) * 512 + lane * 8);
+      }
+    }
+  }
+  {
+    const u32 mag = max((u32)most[0], (u32)most[1]);
+    const u32 nan = __any(mag > 0x7f80u) ? 1u : 0u;
+    const u32 far = __any(mag > FAST_BASE + FAST_TOP) ? 2u : 0u;
+    if (lane == 0 && (nan | far)) atomicOr(&sm.odd, nan | far);
+  }
+  __syncthreads();
+
+  // ---- a thread has eight values, from the largest (thread 0) down ----
+  const bool up = wave < CNT_WAVES / 2;
+  const int mag0 = up ? (CNT_THREADS / 2 - 1 - tid) * 8 : (tid - CNT_THREADS / 2) * 8;
+  const int at0 = up ? mag0 : FAST_SIGN + mag0;
+  auto mag_of = [&](int j) { return up ? mag0 + 7 - j : mag0 + j; };
+  auto value = [&](int j) {
+    const int mag = mag_of(j);
+    const float v = mag ? bf2f((u16)(FAST_BASE + mag)) : 0.f;
+    return up ? v : -v;
+  };
+  auto counts = [&](int p, u32 (&c)[8]) {
+    const u32x4 a = *(const u32x4*)&sm.cnt[p][at0];
+    const u32x4 b = *(const u32x4*)&sm.cnt[p][at0 + 4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      c[j] = up ? b[3 - j] : a[j];
+      c[4 + j] = up ? a[3 - j] : b[j];
+    }
+  };
+  u32 tot[8], my_cnt = 0;
+  counts(0, tot);
+#pragma unroll
+  for (int p = 1; p < FAST_PARTS; ++p) {
+    u32 c[8];
+    counts(p, c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tot[j] += c[j];
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) my_cnt += tot[j];
+  {
+    const u64 any = __ballot(my_cnt != 0);
+    if (lane == 0 && any)
+      atomicMin(&sm.first, wave * 64 + __ffsll((unsigned long long)any) - 1);
+  }
+  __syncthreads();
+  if (tid == sm.first && up) {
+    int code = -1;
+#pragma unroll
+    for (int j = 7; j >= 0; --j)
+      if (tot[j]) code = mag_of(j);
+    sm.code = code;
+  }
+  __syncthreads();
+  const int code = sm.code;
+  const float m = bf2f((u16)(FAST_BASE + max(code, 0)));
+  const u32 odd = sm.odd;
+  const float range = (255.f + m) * inv_t;
+  if (code >= FAST_TOP || !(m >= 2.f) || (odd & 1) || ((odd & 2) && !(range > 104.f)) ||
+      (MASKED && !(range > 40.f)))
+    return false;
+
+  // ---- Z, and running count and mass ----
+  const AddOp add;
+  u64 mass = 0, my_mass = 0;
+  u32 cnt = 0, q[8];
+  float z = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q[j] = 0;
+  u32 ones = 0;            // which values have a weight of 1
+  if (__any(my_cnt != 0)) {
+    u32 one = 0x7f800000;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float v = value(j);
+      // (no value above m has a count, but its exponential may be infinite)
+      const float p = weight(fminf(v, m) - m);
+      z += (float)tot[j] * p;
+      q[j] = q32(p);
+      my_mass += (u64)q[j] * tot[j];
+      if (p >= 1.f) {
+        ones |= 1u << j;
+        my_mass += tot[j];
+        if (tot[j]) one = min(one, __float_as_uint(v));
+      }
+    }
+    if (__any(one != 0x7f800000)) {
+      one = lane_scan(one, 0x7f800000u, MinOp());
+      if (lane == 63) atomicMin(&sm.one, (int)one);
+    }
+    mass = lane_scan(my_mass, (u64)0, add);
+    cnt = lane_scan(my_cnt, 0u, add);
+    z = lane_scan(z, 0.f, add);
+  }
+  if (lane == 63) {
+    sm.wave_mass[wave] = mass;
+    sm.wave_cnt[wave] = cnt;
+    sm.wave_z[wave] = z;
+  }
+  __syncthreads();
+  const int l16 = lane & (CNT_WAVES - 1);
+  const u64 wm = row_scan(sm.wave_mass[l16], (u64)0, add);
+  const u32 wc = row_scan(sm.wave_cnt[l16], 0u, add);
+  float zf = row_scan(sm.wave_z[l16], 0.f, add);
+  zf = __uint_as_float(from_lane(__float_as_uint(zf), CNT_WAVES - 1));
+  const u64 zfix = from_lane(wm, CNT_WAVES - 1);
+  if (wave) {
+    mass += from_lane(wm, wave - 1);
+    cnt += from_lane(wc, wave - 1);
+  }
+  const u32 k_thr = (u32)max(1, A.topks[row]);
+  const double pd = (double)A.topps[row] * (double)zfix;
+  u64 p_thr = (pd >= (double)zfix) ? zfix : (u64)pd;
+  if (p_thr == 0) p_thr = 1;   // top_p ~ 0: keep at least the max token
+  if (cnt >= k_thr && cnt - my_cnt < k_thr) {
+    u32 run = cnt - my_cnt;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (run < k_thr && run + tot[j] >= k_thr)
+        sm.tau[0] = f32key((value(j) - m) * inv_t);
+      run += tot[j];
+    }
+  }
+  if (mass >= p_thr && mass - my_mass < p_thr) {
+    u64 run = mass - my_mass;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const u64 own = ((u64)q[j] + ((ones >> j) & 1u)) * tot[j];
+      if (run < p_thr && run + own >= p_thr)
+        sm.tau[1] = f32key((value(j) - m) * inv_t);
+      run += own;
+    }
+  }
+  __syncthreads();
+
+  // ---- kept mass of the quarters, and the lowest kept value ----
+  const u32 tau = max(sm.tau[0], sm.tau[1]);
+  {
+    u32 kept = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      kept |= (tot[j] && f32key((value(j) - m) * inv_t) >= tau) ? 1u << j : 0u;
+    if (__any(kept)) {
+      u32 low = 2 * FAST_CODES;          // FAST_CODES for the magnitude 0
+      u64 sum[FAST_PARTS] = {};
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if ((kept >> j) & 1u)
+          low = up ? FAST_CODES + mag_of(j) : FAST_CODES - 1 - mag_of(j);
+#pragma unroll
+      for (int p = 0; p < FAST_PARTS; ++p) {
+        u32 c[8];
+        counts(p, c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if ((kept >> j) & 1u) {
+            sum[p] += (u64)q[j] * c[j];
+            if ((ones >> j) & 1u) sum[p] += c[j];
+          }
+      }
+#pragma unroll
+      for (int p = 0; p < FAST_PARTS; ++p) sum[p] = lane_scan(sum[p], (u64)0, add);
+      low = lane_scan(low, (u32)2 * FAST_CODES, MinOp());
+      if (lane == 63) {
+#pragma unroll
+        for (int p = 0; p < FAST_PARTS; ++p)
+          atomicAdd((unsigned long long*)&sm.part[p], (unsigned long long)sum[p]);
+        atomicMin(&sm.low, (int)low - FAST_CODES);
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- selection, in order of index ----
+  u64 total = 0;
+#pragma unroll
+  for (int p = 0; p < FAST_PARTS; ++p) total += sm.part[p];
+  const u64 target = (u64)((double)A.us[row] * (double)total);
+  u64 at = 0;
+  int own = 0;
+#pragma unroll
+  for (int p = 0; p < FAST_PARTS - 1; ++p)
+    if (own == p && at + sm.part[p] <= target) {
+      at += sm.part[p];
+      own = p + 1;
+    }
+  const int lc = sm.low;
+  const int lm = lc >= 0 ? lc : -1 - lc;
+  // (what is counted as 0 is kept together)
+  const float low = lm == 0 ? -bf2f(FAST_BASE)
+                            : bf2f((u16)((lc < 0 ? 0x8000 : 0) | (FAST_BASE + lm)));
+  const float top = fmaxf(__uint_as_float((u32)sm.one), low);
+  auto mass_of = [&](float v) { return v >= low ? q32(weight(v - m)) : 0u; };
+  auto half = [](u32 w, int j) {
+    return __uint_as_float(j & 1 ? w & 0xffff0000u : w << 16);
+  };
+  const int first = own * (CNT_WAVES / FAST_PARTS) * part;   // piece of 512
+  const int pieces = CNT_WAVES / FAST_PARTS * part;
+  constexpr int TURNS = (FAST_BLK + CNT_WAVES - 1) / CNT_WAVES;
+  {
+    u32x4 w[TURNS];
+    u32 alive[TURNS];
+#pragma unroll
+    for (int k = 0; k < TURNS; ++k) {
+      const int i = min((first + wave + k * CNT_WAVES) * 512 + lane * 8, last8);
+      w[k] = *(const u32x4*)(lrow + i);
+      alive[k] = MASKED ? mrow[i >> 3] : 0xffu;
+    }
+#pragma unroll
+    for (int k = 0; k < TURNS; ++k) {
+      const int c = wave + k * CNT_WAVES;
+      if (c >= pieces) break;
+      const int i0 = (first + c) * 512;
+      if (MASKED || i0 + 512 > vl) patch(w[k], alive[k], i0 + lane * 8, 0xffffffffu);
+      u64 sum = 0;
+      float best = half(w[k][0], 0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = half(w[k][j >> 1], j);
+        sum += mass_of(v);
+        best = fmaxf(best, v);
+      }
+      if (__any(best >= top))
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum += half(w[k][j >> 1], j) >= top;
+      sum = lane_scan(sum, (u64)0, add);
+      if (lane == 63) sm.blk[c] = sum;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const u64 a = 2 * lane < pieces ? sm.blk[2 * lane] : 0;
+    const u64 b = 2 * lane + 1 < pieces ? sm.blk[2 * lane + 1] : 0;
+    const u64 to = lane_scan(a + b, (u64)0, add) + at, from = to - a - b;
+    const u64 mine = __ballot(to > target && from <= target);
+    if (mine) {
+      const int src = __ffsll((unsigned long long)mine) - 1;
+      const bool second = from + a <= target;
+      const int c = (int)from_lane((u32)(2 * lane + second), src);
+      const u64 begin = from_lane(second ? from + a : from, src);
+      const int i0 = (first + c) * 512 + lane * 8;
+      u32x4 w = *(const u32x4*)(lrow + min(i0, last8));
+      if (MASKED || i0 + 8 > vl)
+        patch(w, MASKED ? mrow[min(i0, last8) >> 3] : 0xffu, i0, 0xffffffffu);
+      u64 q[8], sum = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = half(w[j >> 1], j);
+        q[j] = (u64)mass_of(v) + (v >= top);
+        sum += q[j];
+      }
+      const u64 end = lane_scan(sum, (u64)0, add) + begin;
+      u64 run = end - sum;
+      if (end > target && run <= target) {
+        int tok = i0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if (run <= target) tok = i0 + j;
+          run += q[j];
+        }
+        sm.token = tok;
+      }
+    }
+  }
+  __syncthreads();
+  if (sm.token < 0) {   // u at the upper edge: the last kept token
+    for (int i = tid; i < vl; i += CNT_THREADS)
+      if ((!MASKED || ((mrow[i >> 3] >> (i & 7)) & 1u)) && bf2f(lrow[i]) >= low)
+        atomicMax(&sm.last, i);
+    __syncthreads();
+    if (tid == 0) sm.token = sm.last;
+    __syncthreads();
+  }
+  if (tid == 0) {
+    const int tok = sm.token;
+    A.out_tok[row] = tok;
+    A.out_lp[row] = (bf2f(lrow[tok]) - m) * inv_t - logf(zf);
+  }
+  return true;
+}
+
+template <bool MASKED>
+__global__ void __launch_bounds__(CNT_THREADS)
+sampler_fast_kernel(SmpArgs A) {
+  extern __shared__ __attribute__((aligned(16))) char fast_lds[];
+  FastRing<MASKED> r;
+  bool have = false;       // r is this row's
+  for (int row = blockIdx.x; row < A.n; row += gridDim.x) {
+    const int next = row + gridDim.x;
+    bool done = false;
+    if (!(A.temps[row] < 1e-5f)) {
+      if (!have) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int part = (A.vl + CNT_CHUNK - 1) / CNT_CHUNK;
+#pragma unroll
+        for (int c = 0; c < FAST_RING; ++c)
+          if (c < part)
+            r.load(A, row, c, ((tid >> 6) * part + c) * 512 + (tid & 63) * 8);
+      }
+      have = next < A.n;
+      done = fast_row<MASKED>(A, row, have ? next : -1, fast_lds, r);
+      __syncthreads();
+    } else {
+      have = false;
+    }
+    if (!done && threadIdx.x == 0) A.out_tok[row] = SMP_LEFT;
+  }
+}
+
 extern "C" void sutro_sampler_fused(const void* logits, int logits_f32,
                                     const float* temps, const float* topps,
                                     const int* topks, const float* us,
                                     const unsigned int* mask, int n,
                                     long v_row, int vl, int w_words,
-                                    int* out_tok, float* out_lp,
+                                    int* out_tok, float* out_lp, int greedy,
                                     hipStream_t stream) {
   if (n == 0) return;
-  const SmpArgs A = {logits, temps, topps, topks, us, mask, v_row, vl, w_words,
-                     out_tok, out_lp};
+  SmpArgs A = {logits, temps, topps, topks, us, mask, v_row, n, vl, w_words,
+               out_tok, out_lp, false};
   dim3 grid((unsigned)n), block(SMP_THREADS);
   // counting: rows of whole, aligned 16-byte pieces, from 2048 logits on (there
   // 124 -> 67 us for 1024 rows and 91 -> 17 us for one; below that no
   // vocabulary in use, and the general kernel has no 128 KB to clear)
   if (!logits_f32 && vl >= CNT_MIN && v_row % 8 == 0 &&
       (size_t)logits % 16 == 0) {
-    const auto fn = mask ? sampler_count_kernel<true>
-                         : sampler_count_kernel<false>;
-    constexpr int lds = sizeof(CountShared) > sizeof(SmpShared<CNT_WAVES>)
-                            ? sizeof(CountShared)
-                            : sizeof(SmpShared<CNT_WAVES>);
-    (void)hipFuncSetAttribute((const void*)fn,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    hipLaunchKernelGGL(fn, grid, dim3(CNT_THREADS), lds, stream, A);
+    auto run = [&](void (*fn)(SmpArgs), unsigned groups, int lds) {
+      (void)hipFuncSetAttribute((const void*)fn,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      hipLaunchKernelGGL(fn, dim3(groups), dim3(CNT_THREADS), lds, stream, A);
+    };
+    if (vl <= CNT_TILE && !greedy) {
+      run(mask ? sampler_fast_kernel<true> : sampler_fast_kernel<false>,
+          n < 256 ? n : 256, sizeof(FastShared));
+      A.left = true;
+    }
+    // (a workgroup a row: in a loop over four rows each, the kernel needs more registers
+    // than there are, 109 -> 113 us for 1024 rows of which none is left)
+    run(mask ? sampler_count_kernel<true> : sampler_count_kernel<false>, n,
+        sizeof(CountShared) > sizeof(SmpShared<CNT_WAVES>)
+            ? sizeof(CountShared)
+            : sizeof(SmpShared<CNT_WAVES>));
   } else if (logits_f32) {
     hipLaunchKernelGGL((sampler_kernel<false>), grid, block, 0,
                        stream, A);

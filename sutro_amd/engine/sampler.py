@@ -126,6 +126,7 @@ class Sampler:
         # three H2D param uploads + index lists amortize to ~nothing
         self._param_key: Optional[tuple] = None
         self._params: Optional[tuple] = None
+        self._greedy = False      # all rows of the batch are
         # pinned ping-pong staging for the per-step uniforms: a pageable
         # .to(device) is a stream-ordered BLOCKING copy (it would serialize
         # the async-decode path behind the whole replay). Two buffers: the
@@ -155,6 +156,7 @@ class Sampler:
         seeded = [i for i, r in enumerate(reqs) if r.sampling.seed is not None]
         seeds = np.array([reqs[i].sampling.seed for i in seeded], dtype=np.uint64)
         self._param_key = key
+        self._greedy = all(r.sampling.temperature < _GREEDY_EPS for r in reqs)
         self._params = (temps, top_ps, top_ks, unseeded, seeded, seeds)
         return self._params
 
@@ -236,5 +238,6 @@ class Sampler:
             self._out_bufs = bufs
         tokens32, lp = bufs[0][:n], bufs[1][:n]
         ops.sampler_fused(logits, temps, top_ps, top_ks, u, fsm_mask,
-                          min(self.vocab_limit, logits.shape[1]), tokens32, lp)
+                          min(self.vocab_limit, logits.shape[1]), tokens32, lp,
+                          self._greedy)
         return tokens32.long(), lp

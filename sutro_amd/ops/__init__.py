@@ -167,11 +167,13 @@ def mean_pool_normalize(hidden: torch.Tensor, query_start_locs: torch.Tensor) ->
 
 
 def sampler_fused(logits, temps, top_ps, top_ks, u, packed_mask, vocab_limit,
-                  out_tok, out_lp):
+                  out_tok, out_lp, greedy: bool = False):
     """Fused mask+temperature+top-k/top-p+sample+logprob (csrc/sampler.hip).
-    GPU-only: logits must be CUDA; raises if the extension is missing."""
+    GPU-only: logits must be CUDA; raises if the extension is missing. `greedy`:
+    all rows have a temperature of 0 (the result is the same, in one launch)."""
     _require_hip().sampler_fused(logits, temps, top_ps, top_ks, u,
-                                 packed_mask, vocab_limit, out_tok, out_lp)
+                                 packed_mask, vocab_limit, out_tok, out_lp,
+                                 greedy)
 
 
 _functions, _dispatches = (torch._C._len_torch_function_stack,

@@ -193,3 +193,29 @@ def test_infinities_and_nans(temp, top_p, top_k):
     bits[3, 5], bits[3, 4000] = -1, -1            # the NaN of all bits
     same_as_general(bits.view(torch.bfloat16).to(DEV), temp, top_p, top_k,
                     (0.0, 0.4, 0.999))
+
+
+@pytest.mark.parametrize("temp,top_p,top_k", [
+    (0.8, 0.95, 0), (1.0, 1.0, 5), (2.0, 0.5, 0), (3.0, 1.0, 0), (30.0, 0.9, 0)])
+def test_ends_of_the_short_range(temp, top_p, top_k):
+    """Rows at the edges of what is counted by magnitudes from 2^-24 to 255, among
+    more rows than there are workgroups, and greedy rows between them."""
+    v = 4096
+    rows = torch.randn(600, v, generator=torch.Generator().manual_seed(7)) * 3
+    rows[0] = rows[0].clamp(max=1.5)              # below 2
+    rows[1] = rows[1].clamp(max=2.0)
+    rows[2, 9], rows[3, 9], rows[4, 9], rows[5, 9] = 254., 255., 256., 1e30
+    rows[6, ::3], rows[7, ::3], rows[8, ::3] = -255., -256., -1e30
+    rows[9, ::2], rows[10, ::2] = -float("inf"), 0.
+    tiny = 2.0 ** -torch.arange(20, 30).repeat_interleave(2)
+    tiny[::2] *= -1
+    rows[11, :20], rows[12, :20], rows[12, 20:] = tiny, tiny, 3.
+    rows[13, :], rows[13, :20] = -5., tiny
+    rows[14, :] = 2.5
+    rows[15, :], rows[15, 4000] = -300., 100.
+    lg = rows.to(torch.bfloat16).to(DEV)
+    same_as_general(lg, temp, top_p, top_k, (0.0, 0.3, 0.999))
+    # the last of several pieces of 512 is not full, and not all of a wave's have one
+    wide = torch.randn(3, 70008, generator=torch.Generator().manual_seed(8)) * 2.5
+    same_as_general(wide.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
+                    (0.0, 0.5, 0.999))
