@@ -29,12 +29,16 @@ composition.
 
 from __future__ import annotations
 
+from operator import attrgetter
 from typing import List, Optional
 
 import numpy as np
 import torch
 
+from .. import ops
 from .request import Request
+
+_REQ_ID = attrgetter("req_id")
 
 # below this, a temperature is treated as greedy (the reference cloud's
 # sampling_params pass through verbatim, so defend against denormals)
@@ -133,14 +137,17 @@ class Sampler:
         # async engine's consume() of step N-1 (inside step N) synchronizes
         # that step's stream work, so buffer (N+1)%2 == (N-1)%2 is free by
         # the time step N+1 reuses it.
+        # A caller that looks at no result may be further ahead than that:
+        # then it waits for the buffer's copy.
         self._u_pinned = [None, None]
+        self._u_copied = [None, None]
         self._u_flip = 0
         self._out_bufs: Optional[tuple] = None
 
     def _param_tensors(self, reqs: List[Request], device) -> tuple:
         # req_ids are unique for the engine's lifetime and a request's sampling
         # params are immutable, so this key is collision-free (unlike id())
-        key = tuple(r.req_id for r in reqs)
+        key = tuple(map(_REQ_ID, reqs))
         if key == self._param_key:
             return self._params
         vl = self.vocab_limit
@@ -155,25 +162,15 @@ class Sampler:
         unseeded = [i for i, r in enumerate(reqs) if r.sampling.seed is None]
         seeded = [i for i, r in enumerate(reqs) if r.sampling.seed is not None]
         seeds = np.array([reqs[i].sampling.seed for i in seeded], dtype=np.uint64)
+        seeded = np.array(seeded, dtype=np.int64)
         self._param_key = key
         self._greedy = all(r.sampling.temperature < _GREEDY_EPS for r in reqs)
         self._params = (temps, top_ps, top_ks, unseeded, seeded, seeds)
         return self._params
 
     def _uniforms(self, reqs, unseeded, seeded, seeds, steps_override, device, n):
-        u = torch.empty(n, dtype=torch.float64)
-        if unseeded:
-            u[unseeded] = torch.rand(len(unseeded), generator=self.generator,
-                                     dtype=torch.float64)
-        if seeded:
-            if steps_override is not None:
-                steps = steps_override[seeded].astype(np.uint64)
-            else:
-                steps = np.fromiter((reqs[i].total_len for i in seeded),
-                                    np.uint64, len(seeded))
-            u[seeded] = torch.from_numpy(seeded_uniform(seeds, steps).copy())
-        u = u.float()
-        if device.type == "cuda":
+        cuda = device.type == "cuda"
+        if cuda:
             i = self._u_flip
             self._u_flip ^= 1
             buf = self._u_pinned[i]
@@ -181,8 +178,29 @@ class Sampler:
                 buf = torch.empty(max(n, 256), dtype=torch.float32,
                                   pin_memory=True)
                 self._u_pinned[i] = buf
-            buf[:n].copy_(u)
-            return buf[:n].to(device, non_blocking=True)
+                self._u_copied[i] = torch.cuda.Event()
+            else:
+                self._u_copied[i].synchronize()
+            u = buf[:n]
+        else:
+            u = torch.empty(n, dtype=torch.float32)
+        if unseeded:
+            u[unseeded] = torch.rand(len(unseeded), generator=self.generator,
+                                     dtype=torch.float64).float()
+        if len(seeded) and not ops.seeded_uniforms(
+                u, reqs, seeded, seeds,
+                None if steps_override is None
+                else np.asarray(steps_override, np.int64), Request):
+            if steps_override is not None:
+                steps = steps_override[seeded].astype(np.uint64)
+            else:
+                steps = np.fromiter((reqs[j].total_len for j in seeded),
+                                    np.uint64, len(seeded))
+            u[torch.from_numpy(seeded)] = torch.from_numpy(
+                seeded_uniform(seeds, steps)).float()
+        if cuda:
+            u = u.to(device, non_blocking=True)
+            self._u_copied[i].record(torch.cuda.current_stream(device))
         return u
 
     @torch.no_grad()
@@ -226,8 +244,6 @@ class Sampler:
     def _sample_hip(self, logits, temps, top_ps, top_ks, u, fsm_mask):
         """Fused CDNA4 mask+sample kernel; the torch reference is only a CPU
         fallback — on a GPU box a missing extension is a hard error."""
-        from .. import ops
-
         n = logits.shape[0]
         bufs = self._out_bufs
         if bufs is None or bufs[0].numel() < n or bufs[0].device != logits.device:

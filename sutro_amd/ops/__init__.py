@@ -166,6 +166,15 @@ def mean_pool_normalize(hidden: torch.Tensor, query_start_locs: torch.Tensor) ->
     return torch_ref.mean_pool_normalize(hidden, query_start_locs)
 
 
+def seeded_uniforms(out, reqs, rows, seeds, steps, plain) -> bool:
+    """out[i] = the uniform of (seed, step) of request i, for i in `rows`
+    (engine/sampler.py); False where there is no native code for it."""
+    if _C is None:
+        return False
+    _C.seeded_uniforms(out, reqs, rows, seeds, steps, plain)
+    return True
+
+
 def sampler_fused(logits, temps, top_ps, top_ks, u, packed_mask, vocab_limit,
                   out_tok, out_lp, greedy: bool = False):
     """Fused mask+temperature+top-k/top-p+sample+logprob (csrc/sampler.hip).
