@@ -139,10 +139,18 @@ __device__ __forceinline__ u16x8 pa_widen(typename PaRaw<KV8>::type raw) {
                                  f[7]}));
   }
 }
-// Tiles in LDS are row-major; 16-byte chunks are XOR-swizzled by the row so
-// that 8 rows of one chunk (keys, read in 16-byte fragments) and 4 rows of two
-// neighbouring chunks (values, read transposed) lie on different banks.
-__device__ __forceinline__ int pa_kchunk(int row, int c) { return c ^ (row & 7); }
+// Tiles in LDS are row-major; 16-byte chunks are XOR-swizzled by the row. Of a
+// prompt's tiles 256 bytes are read in a cycle: 16 rows of one chunk (keys) or 8 rows
+// of two neighbouring ones (values, read transposed), which cover all 64 banks.
+template <int D>
+__device__ __forceinline__ int pa_kswz(int row, int c) {
+  return c ^ (D == 128 ? row & 15 : row >> 1 & 7);
+}
+template <int D>
+__device__ __forceinline__ int pa_vswz(int row, int c) {
+  return c ^ (D == 128 ? row & 7 : row >> 1 & 3) << 1;
+}
+// single tokens: 4 rows of two chunks
 __device__ __forceinline__ int pa_vchunk(int row, int c) {
   return c ^ ((row & 3) << 1);
 }
@@ -158,13 +166,22 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 // ---------------------------------------------------------------------------
 // Prompt pieces. A workgroup owns (up to) hpb query heads of one kv head times
 // rpb blocks of 32 rows, one wave each (hpb * rpb = 4), and walks the visible keys
-// 64 at a time: K and V of the next step are on their way in registers while
-// this step is computed and then go to the other half of a double-buffered LDS
-// tile, one barrier a step. (Straight copies into LDS are no use here: the
-// transposed reads wait for every one of them in flight.)
+// 64 at a time: K and V of the next step go to the other half of a double-buffered
+// LDS tile while this step is computed, straight from memory (e4m3: through
+// registers, where they are widened), one barrier a step. Through registers that way
+// took a fifth of the time: without any copies at all, on one tile over and over, the
+// 40 k prompt below was at 0.79 of it. Now, in turn on one card: 40 k 6549 -> 6079 us
+// (1.01 -> 1.09 PFLOP/s), 16 of 2 k 356 -> 334, one of 3000 with 16 heads and 8 kv heads
+// 76.7 -> 71.9, of 3850 with one head 88.8 -> 82.8, 256 of 200 with 8 heads of 64 49.0 ->
+// 46.7, 160 of 150 with 16 and 8 heads 82 and 82.
 //
-// Bound by LDS reads (every wave reads the whole K and V tile for its 32 rows:
-// as many cycles as its products take) and by the exponentials beside them. The
+// Bound by the products (0.47 of the matrix cores' cycles), the exponentials and the
+// other operations of the softmax (0.5 of the vector unit's): the two waves of a SIMD
+// cover each other's by little. Mixing them within a wave as well, a run of 32 keys'
+// weights among the next one's scores and its values among the next one's maximum, is
+// slower (40 k without copies 4.86 and 6.11 ms: more branches, one wave's order fixed).
+// LDS reads are 0.35 of its cycles; with two rows on the same banks, as it was, 0.58, at
+// the same time. The
 // form before, 32 keys a step, two barriers, V scattered into a transposed tile
 // two bytes at a time and weights passed through LDS, ran at 337 TFLOP/s on a
 // 32 k prompt (16 heads, 4 kv heads, 128; useful flops) and 250 on prompts of
@@ -297,29 +314,28 @@ paged_prefill_kernel(PagedArgs A) {
   constexpr int ES = KV8 ? 1 : 2;
   constexpr int RPP = 64 / CPR;             // rows per piece
   const int st_row = lane / CPR;
-  const u32 koff = (st_row * D + pa_kchunk(st_row, lane % CPR) * 8) * ES;
-  const u32 voff = (st_row * D + pa_vchunk(st_row, lane % CPR) * 8) * ES;
+  const int t_row = w * RPP + st_row;       // of the tile, modulo 4 * RPP
+  const u32 koff = (st_row * D + pa_kswz<D>(t_row, lane % CPR) * 8) * ES;
+  const u32 voff = (st_row * D + pa_vswz<D>(t_row, lane % CPR) * 8) * ES;
   // LATE: four workgroups a CU, no registers to hold them while a step is computed
-  constexpr bool LATE = WAVES_PER_SIMD == 4;
-  typename PaRaw<KV8>::type st[PER / 2];
+  constexpr bool LATE = KV8 && WAVES_PER_SIMD == 4;
+  typename PaRaw<KV8>::type st[KV8 ? PER / 2 : 1];
   int pa = 0, pb = 0;    // pages of the next step to load
   auto pages = [&](int kt) {
     pa = pa_entry(table, min(2 * kt, last_page));
     pb = pa_entry(table, min(2 * kt + 1, last_page));
   };
+  // e4m3: the pieces in registers, to be widened on their way to LDS
   auto load = [&]() {
 #pragma unroll
-    for (int j = 0; j < PER / 2; ++j) {
+    for (int j = 0; KV8 && j < PER / 2; ++j) {
       const bool isv = j >= PER / 4;
       const int piece = (isv ? j - PER / 4 : j) * 4 + w;
       const long blk = j % (PER / 4) >= PER / 8 ? pb : pa;
       const u8* base = (isv ? A.vc : A.kc) +
                        ((blk * A.Hk + kh) * PA_PG + piece % (PER / 2) * RPP) *
                            (D * ES);
-      // rows of odd pieces of 4 rows swizzle keys with row bit 2 set
-      const u32 off =
-          isv ? voff : (RPP == 4 && (w & 1) ? koff ^ (4 * 8 * ES) : koff);
-      st[j] = *(const typename PaRaw<KV8>::type*)(base + off);
+      st[j] = *(const typename PaRaw<KV8>::type*)(base + (isv ? voff : koff));
     }
   };
   // Keys that a row does not see have weight 0, but their values may be infinite
@@ -328,38 +344,73 @@ paged_prefill_kernel(PagedArgs A) {
   // stored as zeros, and a wave takes 16 keys that none of its own rows see from
   // a tile of zeros.
   const u32 g_kept = max(A.keep_first - c_first, 0);
+  auto edge = [&](int kv) {
+    return kv + PA_KEYS > kv_end || (LOCAL && kv < lo_first);
+  };
+  auto any_sees = [&](int kp) {
+    bool any = kp < kv_end;
+    if (LOCAL) any &= (kp >= lo_first) | ((u32)(kp - c_first) < g_kept);
+    return any;
+  };
   auto store = [&](char* buf, int kv) {
-    const bool edge = kv + PA_KEYS > kv_end || (LOCAL && kv < lo_first);
-    if (edge)
+    if (edge(kv))
 #pragma unroll
-      for (int j = PER / 4; j < PER / 2; ++j) {
-        const int kp = kv + ((j - PER / 4) * 4 + w) * RPP + st_row;
-        bool any = kp < kv_end;
-        if (LOCAL) any &= (kp >= lo_first) | ((u32)(kp - c_first) < g_kept);
-        if (!any) st[j] = typename PaRaw<KV8>::type(0);
-      }
+      for (int j = PER / 4; KV8 && j < PER / 2; ++j)
+        if (!any_sees(kv + ((j - PER / 4) * 4 + w) * RPP + st_row))
+          st[j] = typename PaRaw<KV8>::type(0);
 #pragma unroll
-    for (int j = 0; j < PER / 2; ++j)
+    for (int j = 0; KV8 && j < PER / 2; ++j)
       *(u16x8*)(buf + (j * 4 + w) * 1024 + lane * 16) = pa_widen<KV8>(st[j]);
   };
 
+  // bf16: straight to LDS, a page (of one kv head) a buffer, past whose end a lane of an
+  // unseen value reads zeros. Written as assembly, since the compiler would wait for all
+  // of them in front of every transposed read; without results, so that it has
+  // nothing to wait for: the end of the step does.
+  auto copy = [&](char* buf, int kv) {
+    const bool e = edge(kv);
+#pragma unroll
+    for (int j = 0; j < PER / 2; ++j) {
+      const bool isv = j >= PER / 4;
+      const int piece = (isv ? j - PER / 4 : j) * 4 + w;
+      const long blk = j % (PER / 4) >= PER / 8 ? pb : pa;
+      const u64 base =
+          (u64)(isv ? A.vc : A.kc) + (u64)(blk * A.Hk + kh) * (PA_PG * D * 2);
+      const u32x4 page = {(u32)base, (u32)(base >> 32) & 0xffffu, PA_PG * D * 2,
+                          0x00027000u};
+      u32 off = isv ? voff : koff;
+      if (isv && e && !any_sees(kv + piece * RPP + st_row)) off = 1u << 30;
+      const u32 to = (u32)(size_t)(__attribute__((address_space(3))) char*)(
+          buf + (j * 4 + w) * 1024);
+      asm volatile(
+          "s_mov_b32 m0, %0\n\ts_nop 3\n\t"
+          "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(to),
+          "v"(off), "s"(page), "s"(piece % (PER / 2) * RPP * (D * 2))
+          : "m0", "memory");
+    }
+  };
+  auto landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+
   // fragment addresses: keys row ln (+16 a tile), chunk kk*4 + g; values rows
   // 4*g + ti/4 (+16), columns of 16-block b
-  int kad[2];
+  int kad[D / 32];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-    kad[j] = ln * (2 * D) + pa_kchunk(ln, j * 4 + g) * 16;
+  for (int kk = 0; kk < D / 32; ++kk)
+    kad[kk] = ln * (2 * D) + pa_kswz<D>(ln, kk * 4 + g) * 16;
   const int ti = lane & 15;
-  int vad[4];
+  int vad[D / 16];
 #pragma unroll
-  for (int o = 0; o < 4; ++o)
-    vad[o] = (4 * g + (ti >> 2)) * (2 * D) +
-             pa_vchunk(ti >> 2, o * 2 + ((ti & 3) >> 1)) * 16 + (ti & 1) * 8;
+  for (int b = 0; b < D / 16; ++b)
+    vad[b] = (4 * g + (ti >> 2)) * (2 * D) +
+             pa_vswz<D>(4 * g + (ti >> 2), b * 2 + ((ti & 3) >> 1)) * 16 +
+             (ti & 1) * 8;
 
   pages(step_tile(0));
-  load();
+  if (KV8) load();
+  else copy(pa_smem, step_tile(0) * PA_KEYS);
   if (steps > 1) pages(step_tile(1));
-  store(pa_smem, step_tile(0) * PA_KEYS);
+  if (KV8) store(pa_smem, step_tile(0) * PA_KEYS);
+  else landed();
   if (BLOCKS)
 #pragma unroll
     for (int z = 0; z < D / 64; ++z)
@@ -369,7 +420,9 @@ paged_prefill_kernel(PagedArgs A) {
     __syncthreads();
     const int kv0 = step_tile(it) * PA_KEYS;
     const bool more = it + 1 < steps;
-    if (more && !LATE) load();
+    char* const other = pa_smem + ((it + 1) & 1) * 2 * TILE;
+    if (more && !KV8) copy(other, step_tile(it + 1) * PA_KEYS);
+    if (more && KV8 && !LATE) load();
     if (!LATE && it + 2 < steps) pages(step_tile(it + 2));
     // With several row blocks in the workgroup a step may be for the rows of
     // others: which of its four times 16 keys does a row of this wave see?
@@ -394,12 +447,12 @@ paged_prefill_kernel(PagedArgs A) {
     for (int kk = 0; kk < D / 32; ++kk)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const pa_frag ka = *(const s16x8*)(kb + kad[kk & 1] + (kk >> 1) * 128 +
-                                           t * 16 * 2 * D);
-        d[0][t] = pa_mfma16(ka, qb[0][kk], d[0][t]);
-        d[1][t] = pa_mfma16(ka, qb[1][kk], d[1][t]);
+        const pa_frag ka = *(const s16x8*)(kb + kad[kk] + t * 16 * 2 * D);
+        const int f = t & 1;        // (one new operand a product)
+        d[f][t] = pa_mfma16(ka, qb[f][kk], d[f][t]);
+        d[1 - f][t] = pa_mfma16(ka, qb[1 - f][kk], d[1 - f][t]);
       }
-    pa_order<D / 8, D / 8, LATE ? 2 : 4, 1, 2>();
+    pa_order<D / 8, D / 8, WAVES_PER_SIMD == 4 ? 2 : 4, 1, 2>();
     // without a distance bias scores stay unscaled until the exponential
     const bool whole = kv0 + PA_KEYS <= p0 + rb * 32 + 1 &&
                        (!LOCAL || kv0 >= lo_last);
@@ -486,21 +539,22 @@ paged_prefill_kernel(PagedArgs A) {
       }
 #pragma unroll
       for (int b = 0; b < D / 16; ++b) {
-        const int at = vad[b & 3] + (b >> 2) * 128;
-        const pa_frag va = pa_tr(v0 + at, v1 + at);
-        acc[b][0] = pa_mfma16(va, pb[0], acc[b][0]);
-        acc[b][1] = pa_mfma16(va, pb[1], acc[b][1]);
+        const pa_frag va = pa_tr(v0 + vad[b], v1 + vad[b]);
+        const int f = b & 1;
+        acc[b][f] = pa_mfma16(va, pb[f], acc[b][f]);
+        acc[b][1 - f] = pa_mfma16(va, pb[1 - f], acc[b][1 - f]);
       }
     }
-    pa_order<D / 4, D / 8, LATE ? 4 : 8, 2, 2>();
+    pa_order<D / 4, D / 8, WAVES_PER_SIMD == 4 ? 4 : 8, 2, 2>();
     l_run[0] += sum[0];
     l_run[1] += sum[1];
     }
-    if (more) {
+    if (more && KV8) {
       if (LATE) load();
       if (LATE && it + 2 < steps) pages(step_tile(it + 2));
-      store(pa_smem + ((it + 1) & 1) * 2 * TILE, step_tile(it + 1) * PA_KEYS);
+      store(other, step_tile(it + 1) * PA_KEYS);
     }
+    if (!KV8) landed();
   }
 
   if (!live) return;
