@@ -880,7 +880,17 @@ __device__ __forceinline__ void gw_body(
       }
 #pragma unroll
       for (int x = 0; x < 64; ++x) {
-        const int i = x >> 3, j = x & 7;
+        // In squares of squares, one operand of two new at a product: what changes
+        // at the matrix core's inputs is part of the power that sets the clock. Row
+        // by row (the same sums): 2 x 12288 x 4096 at 32,768 rows 4458 -> 4355 us, 2
+        // x 8192 x 2048 1532 -> 1512, 2 x 3072 x 1024 at 24,000 240 -> 238; with
+        // zeros in all operands, far from the limit, 3572 and 3572. By columns 4421,
+        // rows and columns there and back 4368 and 4376. Heads take rows there and
+        // back: in squares their step has 180 moves between the sums' registers.
+        const int i = HEADS ? x >> 3
+                            : (x >> 1 & 1) | (x >> 3 & 1) << 1 | (x >> 5) << 2;
+        const int j = HEADS ? (x & 7) ^ (x >> 3 & 1 ? 7 : 0)
+                            : ((x ^ x >> 1) & 1) | (x >> 2 & 1) << 1 | (x >> 4 & 1) << 2;
         acc[i][j] = mfma16g(fb[kk][j], fa[kk][i], acc[i][j]);
         // reads behind every third product, copies behind every eighth: the LDS
         // takes both beside each other, and the cache the copies of four waves
