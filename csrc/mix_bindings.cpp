@@ -75,7 +75,7 @@ int mix_latent_attention(void*, long, int, const void*, const void*,
                          hipStream_t);
 void mix_token_embed(float*, const long*, const long*, const long*,
                      const void*, const void*, long, long, long, const float*,
-                     float, long, int, int, hipStream_t);
+                     float, const float*, float, void*, long, int, int, hipStream_t);
 void mix_dyt_residual(float*, const void*, const float*, const void*,
                       const float*, const void*, const int*, const float*, int,
                       const float*, const float*, const float*, void*, long,
@@ -596,7 +596,9 @@ void token_embed(torch::Tensor out, torch::Tensor ids,
                  c10::optional<torch::Tensor> prev, torch::Tensor pos,
                  torch::Tensor embed, c10::optional<torch::Tensor> bigram,
                  long buckets, long mul_prev, long mul_cur,
-                 c10::optional<torch::Tensor> inv_freq, double scale) {
+                 c10::optional<torch::Tensor> inv_freq, double scale,
+                 c10::optional<torch::Tensor> norm_w, double eps,
+                 c10::optional<torch::Tensor> h_out) {
   CHECK_GPU(out); CHECK_F32(out); CHECK_CONTIG(out); CHECK_GPU(ids);
   CHECK_I64(ids); CHECK_I64(pos); CHECK_CONTIG(ids); CHECK_CONTIG(pos);
   CHECK_GPU(embed); CHECK_CONTIG(embed);
@@ -619,10 +621,19 @@ void token_embed(torch::Tensor out, torch::Tensor ids,
     TORCH_CHECK(inv_freq->numel() == (W + 1) / 2, "sinusoid table");
     fp = inv_freq->data_ptr<float>();
   }
+  const float* np = nullptr; void* hp = nullptr;
+  if (norm_w.has_value()) {
+    TORCH_CHECK(h_out.has_value(), "a norm needs its output");
+    CHECK_GPU(*norm_w); CHECK_F32(*norm_w); CHECK_CONTIG(*norm_w);
+    CHECK_GPU(*h_out); CHECK_CONTIG(*h_out);
+    TORCH_CHECK(norm_w->numel() == W && h_out->numel() == T * W &&
+                h_out->scalar_type() == embed.scalar_type(), "norm shapes");
+    np = norm_w->data_ptr<float>(); hp = h_out->data_ptr();
+  }
   mix_token_embed(out.data_ptr<float>(), ids.data_ptr<long>(), pp,
                   pos.data_ptr<long>(), embed.data_ptr(), bp, buckets,
-                  mul_prev, mul_cur, fp, (float)scale, T, (int)W,
-                  act_kind(embed), cur_stream());
+                  mul_prev, mul_cur, fp, (float)scale, np, (float)eps, hp, T,
+                  (int)W, act_kind(embed), cur_stream());
 }
 
 void weighted_rmsnorm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -1562,7 +1573,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("out"), py::arg("ids"), py::arg("prev"), py::arg("pos"),
         py::arg("embed"), py::arg("bigram"), py::arg("buckets"),
         py::arg("mul_prev"), py::arg("mul_cur"), py::arg("inv_freq"),
-        py::arg("scale") = 1.0);
+        py::arg("scale") = 1.0, py::arg("norm_w") = py::none(),
+        py::arg("eps") = 0.0, py::arg("h_out") = py::none());
   m.def("weighted_rmsnorm", &weighted_rmsnorm, "RMS norm with a weight vector");
   m.def("norm_residual", &norm_residual,
         "post-norm + residual (+ depth-weighted sum) (+ next pre-norm)");

@@ -211,7 +211,10 @@ __global__ void __launch_bounds__(320) mlstm_scan_kernel(
 }
 
 // one wave per (token, head)
-template <typename A>
+// NV > 0: dv is at most 64 * NV, and all of a head's values, gates and weights are asked
+// for before its norm is known: one wait for memory instead of three (30,000 tokens of 8
+// heads of 128: 117 -> 101 us).
+template <typename A, int NV>
 __global__ void mlstm_out_kernel(A* __restrict__ out, long ldo, int out_off,
                                  const float* __restrict__ o,
                                  const float* __restrict__ em,
@@ -224,6 +227,34 @@ __global__ void mlstm_out_kernel(A* __restrict__ out, long ldo, int out_off,
   const long t = u / H;
   const int h = (int)(u - t * H);
   const float* orow = o + u * (long)(dv + 1);
+  if constexpr (NV > 0) {
+    float x[NV], w[NV];
+    A gate[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int c = lane + k * (int)WAVE;
+      const bool in = c < dv;
+      x[k] = in ? orow[c] : 0.f;
+      w[k] = in ? norm_w[h * dv + c] : 0.f;
+      gate[k] = in ? proj[t * ld + g_off + h * dv + c] : A(0);
+    }
+    const float den = fmaxf(fabsf(orow[dv]), em[u]) + 1e-6f;
+    float ssq = 0.f;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      x[k] /= den;
+      if (lane + k * (int)WAVE < dv) ssq += x[k] * x[k];
+    }
+    const float inv = 1.f / sqrtf(wave_sum_f32(ssq) / (float)dv + eps);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int c = lane + k * (int)WAVE;
+      if (c < dv)
+        stf<A>(out + t * ldo + out_off + h * dv + c,
+               x[k] * inv * w[k] * sigmoid_f(ldf<A>(&gate[k])));
+    }
+    return;
+  }
   const float den = fmaxf(fabsf(orow[dv]), em[u]) + 1e-6f;
   float ssq = 0.f;
   for (int c = lane; c < dv; c += WAVE) {
@@ -322,12 +353,15 @@ extern "C" void mix_mlstm_out(void* out, long ldo, int out_off, const float* o,
   const long units = T * H;
   if (units == 0) return;
   const int grid = (int)((units + 3) / 4);
-  if (f32)
-    hipLaunchKernelGGL(mlstm_out_kernel<float>, dim3(grid), dim3(256), 0, s,
-                       (float*)out, ldo, out_off, o, em, norm_w,
-                       (const float*)proj, ld, g_off, eps, T, H, dv);
-  else
-    hipLaunchKernelGGL(mlstm_out_kernel<u16>, dim3(grid), dim3(256), 0, s,
-                       (u16*)out, ldo, out_off, o, em, norm_w,
-                       (const u16*)proj, ld, g_off, eps, T, H, dv);
+#define LAUNCH_MO(AA, NN)                                                     \
+  hipLaunchKernelGGL((mlstm_out_kernel<AA, NN>), dim3(grid), dim3(256), 0, s, \
+                     (AA*)out, ldo, out_off, o, em, norm_w, (const AA*)proj,  \
+                     ld, g_off, eps, T, H, dv)
+#define PICK_MO(AA)                                \
+  if (dv <= 128) LAUNCH_MO(AA, 2);                 \
+  else if (dv <= 256) LAUNCH_MO(AA, 4);            \
+  else LAUNCH_MO(AA, 0);
+  if (f32) { PICK_MO(float) } else { PICK_MO(u16) }
+#undef PICK_MO
+#undef LAUNCH_MO
 }

@@ -183,12 +183,12 @@ class RuludraModel(nn.Module):
         X = torch.empty((L + 1, T, s.hidden_size), dtype=torch.float32,
                         device=dev)
         big = s.bigram or (0, 0, 0)
+        h = torch.empty((T, s.hidden_size), dtype=self.act_dtype, device=dev)
         hops.token_embed(
             fb.input_ids, fb.prev_ids, fb.positions, self.embed_tokens.weight,
             self.bigram.weight if s.bigram else None, big[0], big[1], big[2],
-            self.pos_inv_freq if s.pos_base else None, out=X[0])
-        h = hops.weighted_rmsnorm(X[0], self.layers[0].norm1, s.norm_eps,
-                                  self.act_dtype)
+            self.pos_inv_freq if s.pos_base else None, out=X[0],
+            norm_w=self.layers[0].norm1, eps=s.norm_eps, h_out=h)
         xw = torch.empty((T, s.hidden_size), dtype=torch.float32, device=dev)
         for i, blk in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < L else self.final_norm

@@ -226,19 +226,24 @@ sinusoid_inv_freq = torch_ref.sinusoid_inv_freq
 
 def token_embed(ids, prev_ids, positions, embed_w, bigram_w, buckets: int,
                 mul_prev: int, mul_cur: int, inv_freq, out=None,
-                scale: float = 1.0):
+                scale: float = 1.0, norm_w=None, eps: float = 0.0, h_out=None):
     """fp32 [T, W] sum of `scale` times the token row, the hashed bigram row
-    (row `buckets` where prev_ids < 0) and the sinusoid of the position."""
+    (row `buckets` where prev_ids < 0) and the sinusoid of the position; with
+    `norm_w` also its RMS norm into h_out (of the embeddings' type)."""
     if out is None:
         out = torch.empty((ids.shape[0], embed_w.shape[1]),
                           dtype=torch.float32, device=ids.device)
     if ids.is_cuda:
         _mix().token_embed(out, ids, prev_ids, positions, embed_w, bigram_w,
-                           buckets, mul_prev, mul_cur, inv_freq, scale)
+                           buckets, mul_prev, mul_cur, inv_freq, scale, norm_w,
+                           eps, h_out)
     else:
         out.copy_(torch_ref.token_embed(ids, prev_ids, positions, embed_w,
                                         bigram_w, buckets, mul_prev, mul_cur,
                                         inv_freq, scale))
+        if norm_w is not None:
+            h_out.copy_(torch_ref.weighted_rmsnorm(out, norm_w, eps,
+                                                   h_out.dtype))
     return out
 
 

@@ -1,0 +1,107 @@
+"""Embedding sums with their norm, queries and keys of tied attention and the read-out
+of the mLSTM against float64, at the widths where their vector forms begin, end and
+change the number of vectors a thread (others take the general kernels).
+
+Rounding to bf16 (8 significant bits) is off by up to 2**-8 of a value, sums of n
+squares in any order by fewer than n 2**-24 of themselves and by half as much below a
+root; ten more operations of 2**-24 each are allowed for."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from sutro_amd.ops import hybrid as hops
+    from sutro_amd.ops import torch_ref
+
+TYPES = [torch.bfloat16, torch.float32]
+
+
+def rand(*shape, seed=0):
+    g = torch.Generator().manual_seed(seed + sum(shape))
+    return torch.randn(*shape, generator=g)
+
+
+def close(got, want, n, extra=0.0):
+    rel = (n / 2 + 10) * 2.0 ** -24
+    if got.dtype == torch.bfloat16:
+        rel += 2.0 ** -8
+    err = (got.double().cpu() - want).abs()
+    assert bool((err <= rel * want.abs() + extra).all()), float(err.max())
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("W", [4, 15, 1020, 1024, 1028, 2048, 4100, 8192, 8196])
+@pytest.mark.parametrize("bigram,sine", [(True, True), (False, True), (False, False)])
+def test_token_embed_norm(dtype, W, bigram, sine):
+    T, V, buckets = 9, 33, 7
+    emb, big = rand(V, W).to(dtype), rand(buckets + 1, W, seed=1).to(dtype)
+    g = torch.Generator().manual_seed(W)
+    ids = torch.randint(0, V, (T,), generator=g)
+    prev = torch.cat([torch.tensor([-1]), ids[:-1]])
+    pos = torch.arange(T) * 1000 + 3
+    w = 1 + rand(W, seed=2) / 10
+    freq = hops.sinusoid_inv_freq(W, 10000.0) if sine else None
+    want = 0.5 * emb[ids].double()
+    size = want.abs()
+    if bigram:
+        row = torch.where(prev < 0, buckets, (prev * 5 + ids * 9) % buckets)
+        want = want + big[row].double()
+        size = size + big[row].double().abs()
+    if sine:
+        ang = (pos.float()[:, None] * freq[None]).double()
+        want = want + torch.stack([ang.sin(), ang.cos()], -1).reshape(T, -1)[:, :W]
+        size = size + 1
+    dev = lambda t: None if t is None else t.cuda()
+    h = torch.empty(T, W, dtype=dtype, device="cuda")
+    x = hops.token_embed(ids.cuda(), dev(prev), pos.cuda(), emb.cuda(),
+                         big.cuda() if bigram else None, buckets if bigram else 0,
+                         5, 9, dev(freq), scale=0.5, norm_w=w.cuda(), eps=1e-5, h_out=h)
+    # (a sine is good to four units of its last place)
+    err = (x.double().cpu() - want).abs()
+    assert bool((err <= 6 * 2.0 ** -23 * size).all()), float(err.max())
+    plain = hops.token_embed(ids.cuda(), dev(prev), pos.cuda(), emb.cuda(),
+                             big.cuda() if bigram else None, buckets if bigram else 0,
+                             5, 9, dev(freq), scale=0.5)
+    assert torch.equal(x, plain)
+    x = x.double().cpu()
+    close(h, x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt() * w.double(), W)
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("H,G,dk", [(16, 4, 128), (3, 1, 8), (1, 2, 12), (17, 1, 128),
+                                    (32, 2, 128), (33, 3, 128), (8, 8, 256), (2, 2, 7)])
+def test_tied_attn_prep(dtype, H, G, dk):
+    T, page, temp = 5, 4, 3
+    q0, k0 = 8, 8 + H * dk
+    proj = rand(T, k0 + G * dk + (-(G + H) * dk) % 8).to(dtype)
+    qw, kw = 1 + rand(H * dk, seed=1) / 10, 1 + rand(G * dk, seed=2) / 10
+    pos, slots = torch.tensor([0, 1, 2, 7, 500]), torch.tensor([3, 4, 11, 0, 9])
+    kc = torch.zeros(3, G, page, dk, dtype=dtype, device="cuda")
+    vc = torch.zeros_like(kc)
+    q = hops.tied_attn_prep(proj.cuda(), q0, k0, H, G, dk, qw.cuda(), kw.cuda(), 1e-5,
+                            pos.cuda(), 0.2, temp, slots.cuda(), kc, vc)
+    p = proj.double()
+    unit = lambda v: v / (v.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    grow = 1 + 0.2 * torch.log(((pos + 1) // temp).double() + 1)
+    close(q.reshape(T, -1), unit(p[:, q0:k0]) * qw.double() * grow[:, None], H * dk)
+    raw = proj[:, k0:k0 + G * dk]
+    close(kc[slots // page, :, slots % page].reshape(T, -1),
+          unit(raw.double()) * kw.double(), G * dk)
+    assert torch.equal(vc[slots // page, :, slots % page].reshape(T, -1).cpu(), raw)
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("H,dv", [(8, 128), (3, 1), (2, 65), (1, 129), (2, 256), (2, 257)])
+def test_mlstm_out(dtype, H, dv):
+    T = 7
+    o, em = rand(T, H, dv + 1), rand(T, H, seed=1).exp()
+    proj, w = rand(T, H * dv + 3, seed=2).to(dtype), 1 + rand(H * dv, seed=3) / 10
+    out = torch.zeros(T, H * dv + 5, dtype=dtype, device="cuda")
+    hops.mlstm_out(o.cuda(), em.cuda(), w.cuda(), proj.cuda(), 3, 1e-5, out, 2)
+    x = o.double()
+    h = x[..., :dv] / (torch.maximum(x[..., dv].abs(), em.double()) + 1e-6)[..., None]
+    h = (h / (h.square().mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(T, -1)
+    want = h * w.double() * torch.sigmoid(proj[:, 3:].double())
+    close(out[:, 2:2 + H * dv], want, dv)
+    assert not out[:, :2].any() and not out[:, 2 + H * dv:].any()
