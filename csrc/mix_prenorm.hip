@@ -449,6 +449,64 @@ __global__ void __launch_bounds__(256) gated_head_norm_kernel(
   *(vec_t*)(out + t * ldo + out_off + part * m + c) = r;
 }
 
+// Long parts: a block owns a (token, part), NCH runs of V values a thread, which stay in
+// registers: every number is read once, 16 bytes a load, and its gate computed once.
+// Same needs as above, parts of up to 256 * V * NCH values. Bound by memory: 30,001
+// tokens of one part of 2048 210 -> 145 us, 13 tokens 5.8 -> 3.9.
+template <typename A, int V, int NCH>
+__global__ void __launch_bounds__(256) gated_row_norm_kernel(
+    A* __restrict__ out, long ldo, int out_off, const float* __restrict__ o,
+    const A* __restrict__ proj, long ld, int g_off,
+    const float* __restrict__ nw, int wstride, float eps, int m, int parts,
+    int mode) {
+  typedef A vec_t __attribute__((ext_vector_type(V)));
+  __shared__ float red[4];
+  const long t = blockIdx.x / parts;
+  const int part = blockIdx.x % parts;
+  f32x4 v[NCH][V / 4];
+  vec_t g[NCH];
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    const int c = (threadIdx.x + 256 * k) * V;
+    if (c >= m) continue;
+#pragma unroll
+    for (int b = 0; b < V / 4; ++b)
+      v[k][b] = *(const f32x4*)(o + (long)blockIdx.x * m + c + b * 4);
+    g[k] = *(const vec_t*)(proj + t * ld + g_off + part * m + c);
+  }
+  float ssq = 0.f, z[NCH][V];          // the gates
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    if ((threadIdx.x + 256 * k) * V >= m) continue;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      A ge = g[k][e];
+      const float y = ldf<A>(&ge), sg = sigmoid_f(y);
+      z[k][e] = mode & (GGN_FIRST | GGN_SILU) ? y * sg : sg;
+      float x = v[k][e >> 2][e & 3];
+      if (mode & GGN_FIRST) x *= z[k][e];
+      v[k][e >> 2][e & 3] = x;
+      ssq += x * x;
+    }
+  }
+  const float inv = 1.f / sqrtf(block_sum_256(ssq, red) / (float)m + eps);
+#pragma unroll
+  for (int k = 0; k < NCH; ++k) {
+    const int c = (threadIdx.x + 256 * k) * V;
+    if (c >= m) continue;
+    vec_t r;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      float y = v[k][e >> 2][e & 3] * (inv * (nw ? nw[part * wstride + c + e] : 1.f));
+      if (!(mode & GGN_FIRST)) y *= z[k][e];
+      A re;
+      stf<A>(&re, y);
+      r[e] = re;
+    }
+    *(vec_t*)(out + t * ldo + out_off + part * m + c) = r;
+  }
+}
+
 extern "C" void mix_gated_group_norm(void* out, long ldo, int out_off,
                                      const float* o, const void* proj, long ld,
                                      int g_off, const float* nw, int wstride,
@@ -483,6 +541,21 @@ extern "C" void mix_gated_group_norm(void* out, long ldo, int out_off,
     return;
   }
   const unsigned grid = (unsigned)(T * parts);
+  if (m % V == 0 && m <= 256 * V * 2 && ldo % V == 0 && ld % V == 0 &&
+      out_off % V == 0 && g_off % V == 0 && (size_t)out % 16 == 0 &&
+      (size_t)proj % 16 == 0 && (size_t)o % 16 == 0) {
+#define LAUNCH_RN(AA, VV, NN)                                                 \
+  hipLaunchKernelGGL((gated_row_norm_kernel<AA, VV, NN>), dim3(grid),         \
+                     dim3(256), 0, s, (AA*)out, ldo, out_off, o,              \
+                     (const AA*)proj, ld, g_off, nw, wstride, eps, m, parts,  \
+                     mode)
+    if (f32 && m <= 256 * V) LAUNCH_RN(float, 4, 1);
+    else if (f32) LAUNCH_RN(float, 4, 2);
+    else if (m <= 256 * V) LAUNCH_RN(u16, 8, 1);
+    else LAUNCH_RN(u16, 8, 2);
+#undef LAUNCH_RN
+    return;
+  }
   if (f32)
     hipLaunchKernelGGL(gated_group_norm_kernel<float>, dim3(grid), dim3(256), 0,
                        s, (float*)out, ldo, out_off, o, (const float*)proj, ld,

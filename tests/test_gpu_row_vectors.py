@@ -105,3 +105,24 @@ def test_mlstm_out(dtype, H, dv):
     want = h * w.double() * torch.sigmoid(proj[:, 3:].double())
     close(out[:, 2:2 + H * dv], want, dv)
     assert not out[:, :2].any() and not out[:, 2 + H * dv:].any()
+
+
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("m", [260, 520, 1024, 1028, 2048, 2052, 2056, 4096, 4104])
+@pytest.mark.parametrize("parts,shared", [(1, False), (3, True), (2, None)])
+def test_gated_norm_of_long_parts(dtype, m, parts, shared):
+    T, n = 3, m * parts
+    o, proj = rand(T, n), rand(T, n + 16, seed=1).to(dtype)
+    w = None if shared is None else 1 + rand(m if shared else n, seed=2) / 10
+    z = proj[:, 8:8 + n].double()
+    for first, silu in ((True, False), (False, True), (False, False)):
+        out = torch.zeros(T, n + 16, dtype=dtype, device="cuda")
+        hops.gated_group_norm(o.cuda(), proj.cuda(), 8, None if w is None else w.cuda(),
+                              1e-5, parts, first, out, 8, silu)
+        gate = torch.sigmoid(z) * (z if first or silu else 1)
+        y = (o.double() * gate if first else o.double()).reshape(T, parts, m)
+        y = (y / (y.square().mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(T, n)
+        if w is not None:
+            y = y * (w.double().repeat(parts) if shared else w.double())
+        close(out[:, 8:8 + n], y if first else y * gate, m)
+        assert not out[:, :8].any() and not out[:, 8 + n:].any()
