@@ -80,6 +80,7 @@ void mix_dyt_residual(float*, const void*, const float*, const void*,
                       const float*, const void*, const int*, const float*, int,
                       const float*, const float*, const float*, void*, long,
                       int, int, hipStream_t);
+void mix_router_scores(float*, const void*, const float*, int, int, int, hipStream_t);
 void mix_moe_route(int*, float*, const float*, long, int, int, int, int, int,
                    int, hipStream_t);
 void mix_moe_dispatch(int*, int*, int*, int*, const int*, const long*, long,
@@ -591,6 +592,20 @@ void delta_out(torch::Tensor out, long out_off, torch::Tensor o,
 }
 
 // ---- embedding, sandwich norms with depth-weighted sums, PolyNorm ----
+
+torch::Tensor router_scores(torch::Tensor h, torch::Tensor w) {
+  CHECK_GPU(h); CHECK_CONTIG(h); CHECK_GPU(w); CHECK_F32(w); CHECK_CONTIG(w);
+  TORCH_CHECK(h.dim() == 2 && w.dim() == 2 && h.size(1) == w.size(1) &&
+              h.scalar_type() == torch::kBFloat16, "router operands");
+  const long T = h.size(0), E = w.size(0), W = h.size(1);
+  TORCH_CHECK(W > 0 && W % 32 == 0 && W < (1L << 30) && T < (1L << 30) &&
+              E <= 1024 && ((size_t)h.data_ptr() & 15) == 0 &&
+              ((size_t)w.data_ptr() & 15) == 0, "router sizes");
+  auto out = torch::empty({T, E}, w.options());
+  mix_router_scores(out.data_ptr<float>(), h.data_ptr(), w.data_ptr<float>(), (int)T,
+                    (int)E, (int)W, cur_stream());
+  return out;
+}
 
 void token_embed(torch::Tensor out, torch::Tensor ids,
                  c10::optional<torch::Tensor> prev, torch::Tensor pos,
@@ -1589,6 +1604,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dyt_residual", &dyt_residual,
         "layer-scaled parallel residual (second branch dense or gathered "
         "expert rows) + Dynamic-Tanh norm of the result");
+  m.def("router_scores", &router_scores, "bf16 rows times fp32 weights, in fp32");
   m.def("moe_route", &moe_route,
         "sigmoid router with group-limited choice; the weights are the scores, "
         "normalised or as they are",

@@ -841,7 +841,7 @@ class RoutedExperts(nn.Module):
     def route(self, h: torch.Tensor):
         """(idx, weights, identity weight or None)."""
         s = self.spec
-        logits = F.linear(h.float(), self.router)
+        logits = hops.router_scores(h, self.router)
         if s.router == "softmax":
             return hops.moe_route_softmax(
                 logits, self.correction if s.correction else None, s.top,

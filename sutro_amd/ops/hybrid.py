@@ -24,8 +24,9 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+import torch.nn.functional as F
 
-from . import expert_tile, torch_ref
+from . import _tracing, _unwatched, expert_tile, torch_ref
 
 _M = None
 _M_ERR: Optional[str] = None
@@ -351,6 +352,40 @@ def dyt_residual(x, y1=None, ls1=None, y2=None, ls2=None, rows=None,
         return
     torch_ref.dyt_residual(x, y1, ls1, y2, ls2, rows, padpos, wts, alpha, nw,
                            nb, h_out if norm is not None else None)
+
+
+def _router_kernel(h, w) -> bool:
+    """Whether csrc/mix_moe.hip makes a router's scores. It reads the rows once for 16
+    experts, so many rows and experts are the library's (us of its product with the
+    conversion, and of this one; calls below 26 us are the host's there):
+      experts of        8        32        64       160       256
+      512,    256 rows  26/5.1   25/4.9    37/5.0    83/4.8   121/4.7
+      512,  30001       33/7.7   32/15     40/27     65/59     86/90
+      2048,    13       25/5.4   25/6.8    25/7.4    25/7.0    26/7.2
+      2048,  1024       25/7.1   25/7.6    25/8.1    26/19     25/24
+      2048, 30001      125/22   105/47    127/94    208/210   288/327
+      4096,   256       25/10    25/13     26/13     25/13     25/14
+      4096, 30001      249/41   246/90    260/184   403/439   565/692"""
+    if (type(h) is not torch.Tensor or _tracing()
+            or type(w) not in (torch.Tensor, torch.nn.Parameter)):
+        return False
+    return (h.is_cuda and h.dim() == 2 and w.dim() == 2 and _unwatched()
+            and h.dtype == torch.bfloat16 and w.dtype == torch.float32
+            and w.device == h.device and w.shape[1] == h.shape[1]
+            and 0 < h.shape[1] < 1 << 30 and h.shape[1] % 32 == 0
+            and 0 < h.shape[0] < 1 << 30
+            and 0 < w.shape[0] <= (256 if h.shape[0] <= 256 else 64)
+            and h.is_contiguous() and w.is_contiguous()
+            and h.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (h.requires_grad or w.requires_grad)))
+
+
+def router_scores(h, w):
+    """fp32 [T, E]: h w^T of fp32 weights."""
+    if _router_kernel(h, w):
+        return _mix().router_scores(h, w)
+    return F.linear(h.float(), w)
 
 
 def moe_route(logits, top: int, groups: int, keep: int, group_rank: int = 2,

@@ -126,3 +126,37 @@ def test_gated_norm_of_long_parts(dtype, m, parts, shared):
             y = y * (w.double().repeat(parts) if shared else w.double())
         close(out[:, 8:8 + n], y if first else y * gate, m)
         assert not out[:, :8].any() and not out[:, 8 + n:].any()
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 2048, 2049, 2117])
+@pytest.mark.parametrize("E,W", [(1, 32), (4, 64), (15, 544), (28, 2048), (65, 96), (256, 512)])
+def test_router_scores(T, E, W):
+    """Exact products of three terms a weight, fp32 sums: off by at most 3 W 2**-24 of
+    the sum of the magnitudes; sums that are not finite as one product a number has them."""
+    h, w = rand(T, W).to(torch.bfloat16), rand(E, W, seed=1)
+    scores = hops._mix().router_scores      # (also where a rule prefers the library)
+    got = scores(h.cuda(), w.cuda()).double().cpu()
+    want = h.double() @ w.double().T
+    size = h.double().abs() @ w.double().abs().T
+    assert bool(((got - want).abs() <= 3 * W * 2.0 ** -24 * size).all())
+    h[0, 1], h[-1, W - 1], w[E - 1, 2] = float("inf"), float("nan"), 3.4e38
+    w[0, 1] = abs(w[0, 1]) + 1
+    got = scores(h.cuda(), w.cuda()).cpu()
+    assert torch.equal(torch.isnan(got[-1]), torch.ones(E, dtype=torch.bool))
+    if T > 1:
+        assert float(got[0, 0]) == float("inf") and not torch.isnan(got[0]).any()
+        assert torch.isfinite(got[1:-1, :E - 1]).all()
+        near = 3.4e38 * h[1:-1, 2].double().abs() < 3e38
+        assert torch.isfinite(got[1:-1, E - 1][near]).all()
+
+
+@pytest.mark.parametrize("make", [lambda h, w: (h.float(), w), lambda h, w: (h[:, 8:], w[:, 8:]),
+                                  lambda h, w: (h[:, :40], w[:, :40]),
+                                  lambda h, w: (h[:, 1:33], w[:, 1:33]),
+                                  lambda h, w: (h.t()[:9].t(), w.t()[:9].t())])
+def test_router_scores_elsewhere(make):
+    h, w = make(rand(70, 96).to(torch.bfloat16).cuda(), rand(300, 96, seed=1)[:20].cuda())
+    want = h.double() @ w.double().T
+    got = hops.router_scores(h, w).double()
+    size = h.double().abs() @ w.double().abs().T
+    assert bool(((got - want).abs() <= 3 * 96 * 2.0 ** -24 * size).all())
