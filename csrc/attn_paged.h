@@ -167,8 +167,8 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 // Prompt pieces. A workgroup owns (up to) hpb query heads of one kv head times
 // rpb blocks of 32 rows, one wave each (hpb * rpb = 4), and walks the visible keys
 // 64 at a time: K and V of the next step go to the other half of a double-buffered
-// LDS tile while this step is computed, straight from memory (e4m3: through
-// registers, where they are widened), one barrier a step. Through registers that way
+// LDS tile while this step is computed, straight from memory (REGS: through
+// registers), one barrier a step. Through registers that way
 // took a fifth of the time: without any copies at all, on one tile over and over, the
 // 40 k prompt below was at 0.79 of it. Now, in turn on one card: 40 k 6549 -> 6079 us
 // (1.01 -> 1.09 PFLOP/s), 16 of 2 k 356 -> 334, one of 3000 with 16 heads and 8 kv heads
@@ -203,13 +203,14 @@ __device__ __forceinline__ int pa_lower(const PagedArgs& A, int p, int& kept) {
 // 3850 with one head 86.2 and 88.8. Four keys' fragments are read ahead for it (six,
 // which the larger products wanted: 78.6 and 91.4; two 79.0 and 92.1; all 84.3 and 99.5).
 //
-// BLOCKS: more than one block of rows in a workgroup.
+// BLOCKS: more than one block of rows in a workgroup. REGS: keys and values through
+// registers, where they are widened or begin elsewhere than at 16 bytes.
 //
 // Entries of the tile map that continue each other (same sequence, 32 rows on)
 // share a workgroup; the entry at a multiple of rpb, or one that continues
 // nothing, leads.
 // ---------------------------------------------------------------------------
-template <int D, bool KV8, bool LOCAL, bool BLOCKS, int WAVES_PER_SIMD>
+template <int D, bool KV8, bool LOCAL, bool BLOCKS, int WAVES_PER_SIMD, bool REGS>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(WAVES_PER_SIMD, WAVES_PER_SIMD)))
 paged_prefill_kernel(PagedArgs A) {
@@ -318,24 +319,26 @@ paged_prefill_kernel(PagedArgs A) {
   const u32 koff = (st_row * D + pa_kswz<D>(t_row, lane % CPR) * 8) * ES;
   const u32 voff = (st_row * D + pa_vswz<D>(t_row, lane % CPR) * 8) * ES;
   // LATE: four workgroups a CU, no registers to hold them while a step is computed
-  constexpr bool LATE = KV8 && WAVES_PER_SIMD == 4;
-  typename PaRaw<KV8>::type st[KV8 ? PER / 2 : 1];
+  constexpr bool LATE = REGS && WAVES_PER_SIMD == 4;
+  typedef typename PaRaw<KV8>::type raw_t;
+  typedef raw_t page_t __attribute__((aligned(KV8 ? 8 : 2)));   // as it lies in a page
+  raw_t st[REGS ? PER / 2 : 1];
   int pa = 0, pb = 0;    // pages of the next step to load
   auto pages = [&](int kt) {
     pa = pa_entry(table, min(2 * kt, last_page));
     pb = pa_entry(table, min(2 * kt + 1, last_page));
   };
-  // e4m3: the pieces in registers, to be widened on their way to LDS
+  // REGS: the pieces in registers, on their way to LDS
   auto load = [&]() {
 #pragma unroll
-    for (int j = 0; KV8 && j < PER / 2; ++j) {
+    for (int j = 0; REGS && j < PER / 2; ++j) {
       const bool isv = j >= PER / 4;
       const int piece = (isv ? j - PER / 4 : j) * 4 + w;
       const long blk = j % (PER / 4) >= PER / 8 ? pb : pa;
       const u8* base = (isv ? A.vc : A.kc) +
                        ((blk * A.Hk + kh) * PA_PG + piece % (PER / 2) * RPP) *
                            (D * ES);
-      st[j] = *(const typename PaRaw<KV8>::type*)(base + (isv ? voff : koff));
+      st[j] = *(const page_t*)(base + (isv ? voff : koff));
     }
   };
   // Keys that a row does not see have weight 0, but their values may be infinite
@@ -355,15 +358,15 @@ paged_prefill_kernel(PagedArgs A) {
   auto store = [&](char* buf, int kv) {
     if (edge(kv))
 #pragma unroll
-      for (int j = PER / 4; KV8 && j < PER / 2; ++j)
+      for (int j = PER / 4; REGS && j < PER / 2; ++j)
         if (!any_sees(kv + ((j - PER / 4) * 4 + w) * RPP + st_row))
-          st[j] = typename PaRaw<KV8>::type(0);
+          st[j] = raw_t(0);
 #pragma unroll
-    for (int j = 0; KV8 && j < PER / 2; ++j)
+    for (int j = 0; REGS && j < PER / 2; ++j)
       *(u16x8*)(buf + (j * 4 + w) * 1024 + lane * 16) = pa_widen<KV8>(st[j]);
   };
 
-  // bf16: straight to LDS, a page (of one kv head) a buffer, past whose end a lane of an
+  // Otherwise straight to LDS, a page (of one kv head) a buffer, past whose end a lane of an
   // unseen value reads zeros. Written as assembly, since the compiler would wait for all
   // of them in front of every transposed read; without results, so that it has
   // nothing to wait for: the end of the step does.
@@ -406,10 +409,10 @@ paged_prefill_kernel(PagedArgs A) {
              (ti & 1) * 8;
 
   pages(step_tile(0));
-  if (KV8) load();
+  if (REGS) load();
   else copy(pa_smem, step_tile(0) * PA_KEYS);
   if (steps > 1) pages(step_tile(1));
-  if (KV8) store(pa_smem, step_tile(0) * PA_KEYS);
+  if (REGS) store(pa_smem, step_tile(0) * PA_KEYS);
   else landed();
   if (BLOCKS)
 #pragma unroll
@@ -421,8 +424,8 @@ paged_prefill_kernel(PagedArgs A) {
     const int kv0 = step_tile(it) * PA_KEYS;
     const bool more = it + 1 < steps;
     char* const other = pa_smem + ((it + 1) & 1) * 2 * TILE;
-    if (more && !KV8) copy(other, step_tile(it + 1) * PA_KEYS);
-    if (more && KV8 && !LATE) load();
+    if (more && !REGS) copy(other, step_tile(it + 1) * PA_KEYS);
+    if (more && REGS && !LATE) load();
     if (!LATE && it + 2 < steps) pages(step_tile(it + 2));
     // With several row blocks in the workgroup a step may be for the rows of
     // others: which of its four times 16 keys does a row of this wave see?
@@ -549,12 +552,12 @@ paged_prefill_kernel(PagedArgs A) {
     l_run[0] += sum[0];
     l_run[1] += sum[1];
     }
-    if (more && KV8) {
+    if (more && REGS) {
       if (LATE) load();
       if (LATE && it + 2 < steps) pages(step_tile(it + 2));
       store(other, step_tile(it + 1) * PA_KEYS);
     }
-    if (!KV8) landed();
+    if (!REGS) landed();
   }
 
   if (!live) return;
@@ -1031,13 +1034,13 @@ static inline int pa_splits(long rows, int Hk, int max_pages) {
   return n < 1 ? 1 : (int)n;
 }
 
-template <int D, bool KV8, bool LOCAL, bool BLOCKS, int WAVES_PER_SIMD>
+template <int D, bool KV8, bool LOCAL, bool BLOCKS, int WAVES_PER_SIMD, bool REGS>
 static inline void pa_start_prefill(const PagedArgs& A, hipStream_t s) {
   // K and V twice, and zeros for 16 keys
   const size_t smem =
       2 * 2 * (size_t)PA_KEYS * D * 2 + (BLOCKS ? 16 * D * 2 : 0);
   const auto kernel =
-      paged_prefill_kernel<D, KV8, LOCAL, BLOCKS, WAVES_PER_SIMD>;
+      paged_prefill_kernel<D, KV8, LOCAL, BLOCKS, WAVES_PER_SIMD, REGS>;
   static std::atomic<unsigned long long> asked{0};
   if (smem > 65536) lds_limit((const void*)kernel, (int)smem, asked);
   hipLaunchKernelGGL(kernel, dim3((unsigned)A.leads * A.groups, 1, A.rpb),
@@ -1045,8 +1048,15 @@ static inline void pa_start_prefill(const PagedArgs& A, hipStream_t s) {
 }
 
 // n_seqs: prompts that the tile map is of
-template <int D, bool KV8, bool LOCAL>
+template <int D, bool KV8, bool LOCAL, bool REGS = KV8>
 static inline void pa_launch_prefill(PagedArgs A, int n_seqs, hipStream_t s) {
+  // The copies to LDS take 16 bytes from multiples of 16. Pages that are a part of a
+  // larger buffer may begin at any number (of layer lists they go to another kernel):
+  // 16 of 2048 tokens, 16 and 4 heads of 128, 400 us from an odd one, as before, and
+  // 317 straight from multiples of 16.
+  if constexpr (!REGS && !LOCAL)
+    if (((size_t)A.kc | (size_t)A.vc) % 16)
+      return pa_launch_prefill<D, KV8, LOCAL, true>(A, n_seqs, s);
   // K and V are read once for 128 rows: 4, 2 or 1 query heads (what divides
   // their group) times 1, 2 or 4 row blocks. Prompts of one or two blocks have no
   // more of them: where workgroups are many they take 4 or 2 heads of any group,
@@ -1071,13 +1081,13 @@ static inline void pa_launch_prefill(PagedArgs A, int n_seqs, hipStream_t s) {
   // spill registers: 32 prompts of 200 tokens, 8 heads and kv heads, 19 -> 24 us.)
   if constexpr (D == 64 && !LOCAL) {
     if ((long)A.n_tiles * A.groups >= 512 && A.n_tiles <= 8 * n_seqs) {
-      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 4>(A, s);
-      else pa_start_prefill<D, KV8, LOCAL, true, 4>(A, s);
+      if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 4, REGS>(A, s);
+      else pa_start_prefill<D, KV8, LOCAL, true, 4, REGS>(A, s);
       return;
     }
   }
-  if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 2>(A, s);
-  else pa_start_prefill<D, KV8, LOCAL, true, 2>(A, s);
+  if (A.rpb == 1) pa_start_prefill<D, KV8, LOCAL, false, 2, REGS>(A, s);
+  else pa_start_prefill<D, KV8, LOCAL, true, 2, REGS>(A, s);
 }
 
 // max_pages: of a row at most (by the table, the window or the chunk)

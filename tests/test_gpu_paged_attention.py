@@ -163,6 +163,39 @@ def test_many_prompts_of_several_steps(Hq, Hk, fp8):
     _check(args, _prefill(args, 64, tiles))
 
 
+# one block and several a workgroup, two workgroups a CU and four
+@pytest.mark.parametrize("Hq,Hk,D,prompts", [
+    (8, 2, 128, 1), (5, 1, 128, 1), (4, 1, 64, 1), (3, 3, 64, 1), (8, 8, 64, 30),
+    (16, 4, 64, 60)])
+@pytest.mark.parametrize("k_at,v_at", [(1, 0), (0, 4), (3, 7)])
+def test_pages_at_other_places(Hq, Hk, D, prompts, k_at, v_at):
+    """Pages that begin elsewhere than at multiples of 16 bytes (a part of a larger
+    buffer): the same results to the bit, values behind the context not a number."""
+    new = [1, 33, 63, 64, 65, 130, 40] * prompts
+    ctx = [0, 0, 70, 0, 5, 31, 352] * prompts
+    lens = [a + b for a, b in zip(new, ctx)]
+    args = _paged(lens, new, Hq, Hk, D, False, seed=Hq)
+    q, kc, vc, bt, sl, ql = args
+    tiles = _tiles(new)
+    assert prompts == 1 or 512 <= len(tiles[0]) * Hk <= 8 * len(new) * Hk
+    want = _prefill(args, D, tiles)
+    if prompts == 1:
+        _check(args, want)
+    for s, n in enumerate(lens):
+        if n % 32:
+            vc[int(bt[s, n // 32]), :, n % 32:] = float("nan")
+
+    def shifted(c, at):
+        flat = torch.empty(c.numel() + at, dtype=c.dtype, device=DEV)
+        part = flat[at:].view(c.shape)
+        part.copy_(c)
+        assert part.data_ptr() % 16 == at * 2
+        return part
+
+    moved = (q, shifted(kc, k_at), shifted(vc, v_at), bt, sl, ql)
+    assert torch.equal(_prefill(moved, D, tiles), want)
+
+
 @pytest.mark.parametrize("Hq,Hk", [(2, 2), (4, 2), (4, 1)])
 def test_prompt_tiles_in_any_order(Hq, Hk):
     # a tile map need not list a sequence's tiles in order, nor at all
