@@ -135,6 +135,7 @@ void paged_attention(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                      int64_t num_decodes, torch::Tensor tile_seq,
                      torch::Tensor tile_q0, int64_t prefill_token_count) {
   CHECK_CUDA(q); CHECK_CONTIG(q); CHECK_BF16(q); CHECK_CONTIG(k_cache);
+  CHECK_CONTIG(v_cache);
   const int Hq = q.size(1), D = q.size(2);
   const int Hk = k_cache.size(1);
   const int bs = k_cache.size(2);

@@ -196,6 +196,15 @@ def test_pages_at_other_places(Hq, Hk, D, prompts, k_at, v_at):
     assert torch.equal(_prefill(moved, D, tiles), want)
 
 
+@pytest.mark.parametrize("which", [1, 2])
+def test_pages_with_gaps_are_refused(which):
+    args = list(_paged([40], [40], 2, 1, 64, False))
+    c = args[which]
+    args[which] = torch.cat([c, c], -1).to(DEV)[..., :64]
+    with pytest.raises(RuntimeError, match="contiguous"):
+        _prefill(args, 64, _tiles([40]))
+
+
 @pytest.mark.parametrize("Hq,Hk", [(2, 2), (4, 2), (4, 1)])
 def test_prompt_tiles_in_any_order(Hq, Hk):
     # a tile map need not list a sequence's tiles in order, nor at all
