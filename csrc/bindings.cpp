@@ -185,6 +185,11 @@ void qkv_prep(torch::Tensor qkv, torch::Tensor q_out, torch::Tensor k_cache,
               c10::optional<torch::Tensor> k_norm_w, double eps) {
   CHECK_CUDA(qkv); CHECK_CONTIG(qkv); CHECK_BF16(qkv);
   CHECK_CONTIG(q_out); CHECK_CONTIG(k_cache); CHECK_CONTIG(v_cache);
+  // (pinned host memory can be read, and written, from the GPU)
+  for (const auto& t : {q_out, k_cache, v_cache, positions, slot_mapping, cos_sin})
+    TORCH_CHECK(t.is_cuda() || t.is_pinned(), "operands on the GPU");
+  for (const auto& n : {q_norm_w, k_norm_w})
+    TORCH_CHECK(!n || n->is_cuda() || n->is_pinned(), "norm weights on the GPU");
   const int T = qkv.size(0);
   const int Hq = q_out.size(1), D = q_out.size(2);
   const int Hk = k_cache.size(1);
@@ -480,6 +485,10 @@ torch::Tensor linear_heads(torch::Tensor x, torch::Tensor w, torch::Tensor k_cac
   CHECK_BF16(k_cache); CHECK_BF16(v_cache);
   CHECK_CONTIG(positions); CHECK_CONTIG(slot_mapping);
   check_gated(x, w, 128);
+  for (const auto& t : {k_cache, v_cache, positions, slot_mapping, cos_sin})
+    TORCH_CHECK(t.device() == x.device(), "operands on one GPU");
+  for (const auto& n : {q_norm_w, k_norm_w})
+    TORCH_CHECK(!n || n->device() == x.device(), "norm weights on one GPU");
   const long M = x.size(0), K = x.size(1), bs = k_cache.size(2);
   const long Hk = k_cache.size(1), Hq = w.size(0) / 128 - 2 * Hk;
   TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(3) == 128 &&

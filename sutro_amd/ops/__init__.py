@@ -644,6 +644,7 @@ def linear_qkv_prep(x, w, num_heads: int, num_kv_heads: int, head_dim: int,
     From a k of 2048 on the library's product is 4 to 7 % faster than the one here and
     the pass small beside it: then where the last round is nearly full."""
     caches = (k_cache, v_cache)
+    norms = tuple(n for n in (q_norm_w, k_norm_w) if n is not None)
     if not (head_dim == 128 and num_heads % 2 == 0 and _many_rows(x, w)
             and x.shape[1] >= 192
             and (x.shape[1] <= 2048 or _last_round(x, w) >= 0.95)
@@ -655,9 +656,10 @@ def linear_qkv_prep(x, w, num_heads: int, num_kv_heads: int, head_dim: int,
             and cos_sin.is_contiguous() and cos_sin.data_ptr() % 16 == 0
             and cos_sin.dtype == torch.float32 and cos_sin.shape[1:] == (128,)
             and positions.is_contiguous() and slot_mapping.is_contiguous()
-            and all(n is None or (n.dtype == torch.bfloat16 and n.is_contiguous()
-                                  and n.data_ptr() % 8 == 0)
-                    for n in (q_norm_w, k_norm_w))):
+            and all(n.dtype == torch.bfloat16 and n.is_contiguous()
+                    and n.data_ptr() % 8 == 0 for n in norms)
+            and all(t.device == x.device for t in
+                    caches + norms + (positions, slot_mapping, cos_sin))):
         return None
     return _require_hip().linear_heads(x, w, k_cache, v_cache, positions,
                                        slot_mapping, cos_sin, q_norm_w, k_norm_w,

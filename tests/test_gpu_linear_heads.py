@@ -77,3 +77,18 @@ def test_route():
         assert ops.linear_qkv_prep(x, w, *a, k, v, cos_sin, qw, kw, 1e-6) is None
     assert ops.linear_qkv_prep(x[:64], w, *args, kc, vc, cos_sin, qw, kw,
                                1e-6) is None
+
+
+@pytest.mark.parametrize("which", range(2, 9))
+def test_operands_on_the_host(which):
+    """An error, by either way, and not an address of the host's on the GPU."""
+    M, Hq, Hk, K = 4096, 16, 8, 512
+    host = list(_case(M, Hq, Hk, K))
+    host[which] = host[which].cpu()
+    x, w, kc, vc, pos, slots, cos_sin, qw, kw = host
+    args = (Hq, Hk, 128, pos, slots, kc, vc, cos_sin, qw, kw, 1e-6)
+    assert ops.linear_qkv_prep(x, w, *args) is None
+    with pytest.raises(RuntimeError, match="GPU"):
+        ops._require_hip().linear_heads(*host, 1e-6)
+    with pytest.raises(RuntimeError, match="GPU"):
+        ops.fused_qkv_prep(ops.linear(x, w), *args)

@@ -1,0 +1,56 @@
+"""Where the QKV projection of a prompt may make queries, keys and values in one launch:
+what that launch cannot read goes to the product and the pass behind it."""
+
+import pytest
+import torch
+
+from sutro_amd import ops
+
+M, HQ, HK, K = 4096, 16, 8, 512
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """Stands in for the extension: counts the calls that reach it."""
+    class Kernels:
+        calls = 0
+
+        def linear_heads(self, *args):
+            self.calls += 1
+            return args[0]
+
+    k = Kernels()
+    monkeypatch.setattr(ops, "_use_hip", lambda t: True)
+    monkeypatch.setattr(ops, "_require_hip", lambda: k)
+    return k
+
+
+def _operands():
+    bf = dict(dtype=torch.bfloat16)              # (never read)
+    return dict(
+        x=torch.empty(M, K, **bf), w=torch.empty((HQ + 2 * HK) * 128, K, **bf),
+        num_heads=HQ, num_kv_heads=HK, head_dim=128,
+        positions=torch.zeros(M, dtype=torch.int64),
+        slot_mapping=torch.zeros(M, dtype=torch.int64),
+        k_cache=torch.empty(4, HK, 32, 128, **bf),
+        v_cache=torch.empty(4, HK, 32, 128, **bf),
+        cos_sin=torch.empty(9, 128), q_norm_w=torch.empty(128, **bf),
+        k_norm_w=torch.empty(128, **bf))
+
+
+def _calls(kernels, **other):
+    got = ops.linear_qkv_prep(**{**_operands(), **other})
+    assert (got is not None) == kernels.calls
+    return kernels.calls
+
+
+@pytest.mark.parametrize("norm", [True, False])
+def test_taken(kernels, norm):
+    assert _calls(kernels, **({} if norm else dict(q_norm_w=None, k_norm_w=None))) == 1
+
+
+@pytest.mark.parametrize("name", ["positions", "slot_mapping", "k_cache", "v_cache",
+                                  "cos_sin", "q_norm_w", "k_norm_w"])
+def test_operands_elsewhere(kernels, name):
+    """On another device than the rows."""
+    assert _calls(kernels, **{name: _operands()[name].to("meta")}) == 0
