@@ -650,14 +650,17 @@ def linear_qkv_prep(x, w, num_heads: int, num_kv_heads: int, head_dim: int,
             and (x.shape[1] <= 2048 or _last_round(x, w) >= 0.95)
             and all(t.dtype == torch.bfloat16 and t.is_contiguous()
                     and t.data_ptr() % 16 == 0 for t in caches)
-            and k_cache.shape == v_cache.shape
+            and w.shape[0] == (num_heads + 2 * num_kv_heads) * 128
+            and k_cache.dim() == 4 and k_cache.shape == v_cache.shape
+            and k_cache.shape[1] == num_kv_heads and k_cache.shape[3] == 128
             and k_cache.shape[2] & (k_cache.shape[2] - 1) == 0
             and k_cache.numel() >> 7 < 1 << 32
             and cos_sin.is_contiguous() and cos_sin.data_ptr() % 16 == 0
             and cos_sin.dtype == torch.float32 and cos_sin.shape[1:] == (128,)
-            and positions.is_contiguous() and slot_mapping.is_contiguous()
+            and all(t.is_contiguous() and t.numel() == x.shape[0]
+                    for t in (positions, slot_mapping))
             and all(n.dtype == torch.bfloat16 and n.is_contiguous()
-                    and n.data_ptr() % 8 == 0 for n in norms)
+                    and n.numel() == 128 and n.data_ptr() % 8 == 0 for n in norms)
             and all(t.device == x.device for t in
                     caches + norms + (positions, slot_mapping, cos_sin))):
         return None

@@ -92,3 +92,17 @@ def test_operands_on_the_host(which):
         ops._require_hip().linear_heads(*host, 1e-6)
     with pytest.raises(RuntimeError, match="GPU"):
         ops.fused_qkv_prep(ops.linear(x, w), *args)
+
+
+def test_longer_positions():
+    """Positions and slots of the largest batch, of which the first are used."""
+    M, Hq, Hk, K = 4096, 16, 8, 512
+    x, w, kc, vc, pos, slots, cos_sin, qw, kw = _case(M, Hq, Hk, K)
+    qkv, outs = ops.linear(x, w), []
+    for p, s in ((pos, slots), (pos.repeat(2), slots.repeat(2))):
+        k, v = kc.clone(), vc.clone()
+        args = (Hq, Hk, 128, p, s, k, v, cos_sin, qw, kw, 1e-6)
+        assert (ops.linear_qkv_prep(x, w, *args) is None) == (p is not pos)
+        outs.append((ops.fused_qkv_prep(qkv, *args), k, v))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

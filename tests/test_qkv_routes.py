@@ -54,3 +54,18 @@ def test_taken(kernels, norm):
 def test_operands_elsewhere(kernels, name):
     """On another device than the rows."""
     assert _calls(kernels, **{name: _operands()[name].to("meta")}) == 0
+
+
+@pytest.mark.parametrize("name,make", [
+    # as many positions and slots as the largest batch, of which the first are used
+    ("positions", lambda t: torch.zeros(M + 64, dtype=torch.int64)),
+    ("slot_mapping", lambda t: torch.zeros(M + 64, dtype=torch.int64)),
+    ("q_norm_w", lambda t: torch.cat([t, t])), ("k_norm_w", lambda t: torch.cat([t, t])),
+    # (the pass refuses these)
+    ("num_heads", lambda n: n + 2), ("num_kv_heads", lambda n: n + 1),
+    ("k_cache", lambda t: t[:, :4].contiguous()), ("k_cache", lambda t: t.flatten(2))])
+def test_sizes_that_differ(kernels, name, make):
+    other = {name: make(_operands()[name])}
+    if name == "k_cache":
+        other["v_cache"] = other[name]
+    assert _calls(kernels, **other) == 0
