@@ -100,7 +100,8 @@ class Qwen3Attention(nn.Module):
                  self.k_norm.weight if self.qk_norm else None,
                  self.q_norm.eps if self.qk_norm else 1e-6)
         q = None
-        if qkv is None and bare(self.qkv_proj):
+        # (a look at the rows first: eager steps of few are bound by what is asked here)
+        if qkv is None and x.shape[0] > 256 and bare(self.qkv_proj):
             q = ops.linear_qkv_prep(x, self.qkv_proj.weight, *heads)
         if q is None:
             if qkv is None:

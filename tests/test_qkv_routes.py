@@ -1,10 +1,13 @@
 """Where the QKV projection of a prompt may make queries, keys and values in one launch:
 what that launch cannot read goes to the product and the pass behind it."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
 from sutro_amd import ops
+from sutro_amd.models.qwen3 import Qwen3Attention
 
 M, HQ, HK, K = 4096, 16, 8, 512
 
@@ -69,3 +72,22 @@ def test_sizes_that_differ(kernels, name, make):
     if name == "k_cache":
         other["v_cache"] = other[name]
     assert _calls(kernels, **other) == 0
+
+
+@pytest.mark.parametrize("rows,asked", [(1, 0), (21, 0), (256, 0), (257, 1)])
+def test_few_rows_are_not_asked(monkeypatch, rows, asked):
+    """Eager steps of few rows are bound by what is asked on the host."""
+    spec = SimpleNamespace(num_heads=2, num_kv_heads=1, head_dim=8, hidden_size=16,
+                           qk_norm=True, rms_eps=1e-6)
+    attn = Qwen3Attention(spec, torch.float32, 0)
+    calls = []
+    monkeypatch.setattr(ops, "linear_qkv_prep", lambda *a: calls.append(1))
+    monkeypatch.setattr(ops, "fused_qkv_prep",
+                        lambda qkv, *a: qkv[:, :16].reshape(-1, 2, 8))
+    monkeypatch.setattr(ops, "paged_attention", lambda q, *a: q)
+    fb = SimpleNamespace(**dict.fromkeys((
+        "positions", "slot_mapping", "block_tables", "seq_lens", "query_start_locs",
+        "num_decodes_tail", "tile_seq", "tile_q0", "prefill_token_count")))
+    kv = SimpleNamespace(k_cache=[None], v_cache=[None])
+    assert attn(torch.zeros(rows, 16), fb, kv, None).shape == (rows, 16)
+    assert len(calls) == asked
