@@ -58,6 +58,10 @@ __device__ __forceinline__ u32 f32key(float s) {
   u32 b = __float_as_uint(s);
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
+// and back
+__device__ __forceinline__ float f32val(u32 k) {
+  return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
+}
 
 struct Boundary {
   u32 pref;        // resolved key prefix (eventually the exact 32-bit key)
@@ -1123,10 +1127,11 @@ sampler_count_kernel(SmpArgs A) {
 // logit is counted under its sign and its magnitude between 2^-24 and 255, 8192 values
 // in 32 bits, in four tables, one for each quarter of the row. They tell the kept mass of
 // every quarter, and only the one that u falls into is read again. What lies outside is
-// counted at the ends. That is exact where the largest logit is from 2 to 254 (a magnitude
-// of 2^-24 or less then vanishes in the difference to it) and where nothing lies below
-// -255 or all of it is 0 as a weight; other rows, with NaN or +inf among them, and
-// greedy ones are left to the kernel above, which runs behind this one.
+// counted at the ends. That is exact where the largest logit is above 1 (a magnitude of
+// 2^-24 or less then vanishes in the difference to it) or no magnitude is as small, and
+// where none is above 254, or those are negative and 0 as weights; other rows, with NaN
+// or +inf among them, and greedy ones are left to the kernel above, which runs behind
+// this one.
 //
 // One workgroup a CU stays for all of its rows: where a piece of the row has been counted,
 // the same piece of the next row is asked for, so that the copies run on beside the
@@ -1136,7 +1141,12 @@ sampler_count_kernel(SmpArgs A) {
 // the quarter (4). 1024 / 256 / 1 rows of 151,936, top_p 0.95 at temperature 0.8: 193 /
 // 49 / 41 us by the kernel above, 109 / 29 / 24 here; top_k 20 150 -> 105, with a mask
 // 248 -> 136, at temperature 3 194 -> 113; 1024 of 32,000 92 -> 53, of 2048 69 -> 39. Of
-// these 3 us are the launch that finds nothing left to do.
+// these 4.7 us are the launch that finds nothing left to do. Flat rows (normal, 0.3) 198 ->
+// 115, log-probabilities 185 -> 117, all at -20 and less 185 -> 119.
+// That a row is left is known when it has been counted, which is then lost: 1024 / 64 /
+// 1 rows of 151,936 with logits above 254 152 / 33 / 31 us by the kernel above alone and
+// 219 / 46 / 44 with this one in front, with NaN 1693 / 418 / 411 and 1885 / 467 / 458,
+// with a largest logit of 0 1716 / 415 / 363 and 1999 / 485 / 433.
 #define FAST_PARTS 4
 #define FAST_BASE 0x3380        // bits of 2^-24
 #define FAST_TOP 4095           // 255, and what is larger
@@ -1153,9 +1163,9 @@ struct FastShared {
   u64 wave_mass[CNT_WAVES];
   u32 wave_cnt[CNT_WAVES];
   float wave_z[CNT_WAVES];
-  int first, code;              // of the largest value: its thread, its magnitude
-  int one;                      // lowest value with p = 1, as bits
-  int low;                      // lowest kept value: magnitude, or -1 - magnitude
+  int first, code;              // of the largest value: its thread and what it is,
+  int low;                      // and the lowest kept one: magnitude, or -1 - magnitude
+  u32 one;                      // lowest value with p = 1, by its key
   u32 odd, tau[2];
   int token, last;
 };
@@ -1261,8 +1271,8 @@ __device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
     if (tid < FAST_PARTS) sm.part[tid] = 0;
     if (tid == 0) {
       sm.first = CNT_THREADS;
-      sm.code = -1;
-      sm.one = 0x7f800000;
+      sm.code = -FAST_CODES;
+      sm.one = f32key(INFINITY);
       sm.low = FAST_CODES;
       sm.odd = sm.tau[0] = sm.tau[1] = 0;
       sm.token = sm.last = -1;
@@ -1360,22 +1370,24 @@ __device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
     const u64 any = __ballot(my_cnt != 0);
     if (lane == 0 && any)
       atomicMin(&sm.first, wave * 64 + __ffsll((unsigned long long)any) - 1);
+    if (mag0 == 0 && (up ? tot[7] : tot[0])) atomicOr(&sm.odd, 4u);
   }
   __syncthreads();
-  if (tid == sm.first && up) {
-    int code = -1;
+  if (tid == sm.first) {
+    int code = 0;
 #pragma unroll
     for (int j = 7; j >= 0; --j)
-      if (tot[j]) code = mag_of(j);
+      if (tot[j]) code = up ? mag_of(j) : -1 - mag_of(j);
     sm.code = code;
   }
   __syncthreads();
   const int code = sm.code;
-  const float m = bf2f((u16)(FAST_BASE + max(code, 0)));
+  const int mag = code >= 0 ? code : -1 - code;
+  const float size = bf2f((u16)(FAST_BASE + mag)), m = code >= 0 ? size : -size;
   const u32 odd = sm.odd;
   const float range = (255.f + m) * inv_t;
-  if (code >= FAST_TOP || !(m >= 2.f) || (odd & 1) || ((odd & 2) && !(range > 104.f)) ||
-      (MASKED && !(range > 40.f)))
+  if (mag >= FAST_TOP || (size <= 1.f && (odd & 4)) || (odd & 1) ||
+      ((odd & 2) && !(range > 104.f)) || (MASKED && !(range > 40.f)))
     return false;
 
   // ---- Z, and running count and mass ----
@@ -1387,7 +1399,7 @@ __device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
   for (int j = 0; j < 8; ++j) q[j] = 0;
   u32 ones = 0;            // which values have a weight of 1
   if (__any(my_cnt != 0)) {
-    u32 one = 0x7f800000;
+    u32 one = f32key(INFINITY);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float v = value(j);
@@ -1399,12 +1411,13 @@ __device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
       if (p >= 1.f) {
         ones |= 1u << j;
         my_mass += tot[j];
-        if (tot[j]) one = min(one, __float_as_uint(v));
+        // (what is counted as 0 is kept together)
+        if (tot[j]) one = min(one, f32key(mag_of(j) ? v : -bf2f(FAST_BASE)));
       }
     }
-    if (__any(one != 0x7f800000)) {
-      one = lane_scan(one, 0x7f800000u, MinOp());
-      if (lane == 63) atomicMin(&sm.one, (int)one);
+    if (__any(one != f32key(INFINITY))) {
+      one = lane_scan(one, f32key(INFINITY), MinOp());
+      if (lane == 63) atomicMin(&sm.one, one);
     }
     mass = lane_scan(my_mass, (u64)0, add);
     cnt = lane_scan(my_cnt, 0u, add);
@@ -1504,10 +1517,9 @@ __device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
     }
   const int lc = sm.low;
   const int lm = lc >= 0 ? lc : -1 - lc;
-  // (what is counted as 0 is kept together)
   const float low = lm == 0 ? -bf2f(FAST_BASE)
                             : bf2f((u16)((lc < 0 ? 0x8000 : 0) | (FAST_BASE + lm)));
-  const float top = fmaxf(__uint_as_float((u32)sm.one), low);
+  const float top = fmaxf(f32val(sm.one), low);
   auto mass_of = [&](float v) { return v >= low ? q32(weight(v - m)) : 0u; };
   auto half = [](u32 w, int j) {
     return __uint_as_float(j & 1 ? w & 0xffff0000u : w << 16);

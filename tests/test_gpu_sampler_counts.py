@@ -134,10 +134,11 @@ def test_extreme_rows():
         assert tok.item() == 0 and lp.item() == ninf
 
 
-def same_as_general(logits, temp, top_p, top_k, us):
+def same_as_general(logits, temp, top_p, top_k, us, keep=None):
     """bf16 rows against the same values in float32, which the kernel without
     counters samples: the tokens are equal, as both sum whole numbers."""
     v = logits.shape[1]
+    mask = None if keep is None else pack(keep)
     for u in us:
         res = []
         for lg in (logits, logits.float()):
@@ -148,7 +149,7 @@ def same_as_general(logits, temp, top_p, top_k, us):
                 lg, torch.full((n,), temp, device=DEV),
                 torch.full((n,), top_p, device=DEV),
                 torch.full((n,), top_k or v, dtype=torch.int32, device=DEV),
-                torch.full((n,), u, device=DEV), None, v, tok, lp)
+                torch.full((n,), u, device=DEV), mask, v, tok, lp)
             res.append((tok.cpu(), lp.cpu()))
         assert torch.equal(res[0][0], res[1][0]), (temp, top_p, top_k, u)
         torch.testing.assert_close(res[0][1], res[1][1], rtol=0, atol=1e-5,
@@ -219,3 +220,34 @@ def test_ends_of_the_short_range(temp, top_p, top_k):
     wide = torch.randn(3, 70008, generator=torch.Generator().manual_seed(8)) * 2.5
     same_as_general(wide.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
                     (0.0, 0.5, 0.999))
+
+
+@pytest.mark.parametrize("temp,top_p,top_k", [
+    (0.8, 0.95, 0), (1.0, 1.0, 5), (3.0, 1.0, 0), (30.0, 0.9, 0), (1e9, 1.0, 0)])
+def test_rows_that_are_small_or_negative(temp, top_p, top_k):
+    """Flat rows and log-probabilities: a largest logit of 2 and less, with and
+    without others of 2^-24 and less, zeros and negative zeros, and all of them negative."""
+    v = 4096
+    rows = torch.randn(28, v, generator=torch.Generator().manual_seed(9)) * 0.2
+    tiny = 2.0 ** -torch.arange(20, 30).repeat_interleave(2)
+    tiny[::2] *= -1
+    rows[1, 50], rows[2, 50], rows[3, 50] = 0.0, -0.0, 1e-9
+    rows[4:8] -= torch.tensor([0.5, 2.0, 20.0, 253.0])[:, None]
+    rows[8] = rows[8].clamp(max=0.0)
+    rows[9], rows[10] = -rows[9].abs() - 2.0 ** -24, -rows[10].abs() - 2.0 ** -23
+    rows[11] = torch.log_softmax(rows[11] * 10, -1)
+    rows[12] = torch.log_softmax(rows[12] * 100, -1)
+    rows[13], rows[13, 7] = -30.0, 0.0
+    rows[14], rows[14, 7] = -30.0, -1e-3
+    rows[15, :20], rows[15, 20:] = tiny, -3.0
+    rows[16, :20], rows[16, 20:] = -tiny.abs(), -3.0
+    rows[17, :20], rows[17, 20] = tiny, 1.9921875
+    rows[24:, :20] = tiny
+    rows[24:, 20] = torch.tensor([1.0078125, 1.0, 0.99609375, 2.0])
+    rows[18], rows[18, ::3], rows[18, 5] = -200.0, -255.0, -254.0
+    rows[19], rows[19, ::3], rows[19, 5] = -254.0, -256.0, -255.0
+    rows[20], rows[21] = -255.0, -300.0
+    rows[22, ::2] = -float("inf")
+    rows[23], rows[23, ::2] = -float("inf"), -2.0
+    same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
+                    (0.0, 0.3, 0.999))
