@@ -251,3 +251,38 @@ def test_rows_that_are_small_or_negative(temp, top_p, top_k):
     rows[23], rows[23, ::2] = -float("inf"), -2.0
     same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
                     (0.0, 0.3, 0.999))
+
+
+@pytest.mark.parametrize("temp,top_p,top_k", [
+    (0.8, 0.95, 0), (1.0, 1.0, 5), (6.0, 1.0, 0), (6.5, 1.0, 0), (9.0, 0.9, 3000),
+    (30.0, 0.9, 0)])
+def test_masked_ends_of_the_short_range(temp, top_p, top_k):
+    """Under a mask what lies at -255 and below is not counted, and rows are left
+    where (255 + the largest) / temperature is 40 or less: from a temperature of 6.4 on
+    at a largest of 1.5, of 8.9 at 100. What is masked is no number, infinite, or larger."""
+    v = 4096
+    g = torch.Generator().manual_seed(11)
+    rows = torch.randn(300, v, generator=g) * 3
+    keep = torch.rand(300, v, generator=g) < 0.5
+    rows[0] = rows[0].clamp(max=1.5)
+    rows[1, 9], rows[2, 9], rows[3, 9] = 100.0, 254.0, 255.0
+    for r, low in ((4, -254.0), (5, -255.0), (6, -256.0), (7, -1e30),
+                   (8, -float("inf"))):
+        rows[r, ::3] = low
+        rows[r + 5, ::3] = low
+        rows[r + 5, 9] = 100.0
+    rows[14] = rows[14] / 20 - 20.0
+    rows[15] = torch.log_softmax(rows[15], -1)
+    rows[16] /= 10
+    rows[17, 5:], rows[17, 5] = -255.0, 1.5
+    rows[18], rows[18, 5:8] = -300.0, 2.5
+    rows[19] = -255.0
+    for r in (1, 2, 3, *range(9, 14)):
+        keep[r, 9] = True
+    keep[17, :], keep[18, 5:8], keep[18, 100:] = True, True, True
+    for i, odd in enumerate((float("nan"), float("inf"), 250.0, 300.0)):
+        rows[20 + i] = torch.where(keep[20 + i], rows[20 + i], odd)
+    keep[24, :] = False
+    keep[24, 4000] = True
+    same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
+                    (0.0, 0.3, 0.999), keep)
