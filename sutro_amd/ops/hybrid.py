@@ -230,14 +230,18 @@ def token_embed(ids, prev_ids, positions, embed_w, bigram_w, buckets: int,
                 scale: float = 1.0, norm_w=None, eps: float = 0.0, h_out=None):
     """fp32 [T, W] sum of `scale` times the token row, the hashed bigram row
     (row `buckets` where prev_ids < 0) and the sinusoid of the position; with
-    `norm_w` also its RMS norm into h_out (of the embeddings' type)."""
+    `norm_w` also its RMS norm into h_out (in the same launch where that is of the
+    embeddings' type)."""
     if out is None:
         out = torch.empty((ids.shape[0], embed_w.shape[1]),
                           dtype=torch.float32, device=ids.device)
     if ids.is_cuda:
+        one = norm_w is not None and h_out.dtype == embed_w.dtype
         _mix().token_embed(out, ids, prev_ids, positions, embed_w, bigram_w,
-                           buckets, mul_prev, mul_cur, inv_freq, scale, norm_w,
-                           eps, h_out)
+                           buckets, mul_prev, mul_cur, inv_freq, scale,
+                           norm_w if one else None, eps, h_out if one else None)
+        if norm_w is not None and not one:
+            _mix().weighted_rmsnorm(h_out, out, norm_w, eps)
     else:
         out.copy_(torch_ref.token_embed(ids, prev_ids, positions, embed_w,
                                         bigram_w, buckets, mul_prev, mul_cur,

@@ -68,6 +68,18 @@ def test_token_embed_norm(dtype, W, bigram, sine):
     close(h, x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt() * w.double(), W)
 
 
+@pytest.mark.parametrize("dtype,other", [TYPES, TYPES[::-1]])
+def test_token_embed_norm_of_another_type(dtype, other):
+    """Activations need not be of the embeddings' type."""
+    emb, w = rand(33, 64).to(dtype).cuda(), (1 + rand(64, seed=2) / 10).cuda()
+    ids = torch.arange(9, device="cuda")
+    h = torch.empty(9, 64, dtype=other, device="cuda")
+    x = hops.token_embed(ids, None, ids, emb, None, 0, 0, 0, None, norm_w=w, eps=1e-5,
+                         h_out=h)
+    assert torch.equal(x, emb[:9].float())
+    assert torch.equal(h, hops.weighted_rmsnorm(x, w, 1e-5, other))
+
+
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("H,G,dk", [(16, 4, 128), (3, 1, 8), (1, 2, 12), (17, 1, 128),
                                     (32, 2, 128), (33, 3, 128), (8, 8, 256), (2, 2, 7)])
