@@ -172,3 +172,21 @@ def test_router_scores_elsewhere(make):
     got = hops.router_scores(h, w).double()
     size = h.double().abs() @ w.double().abs().T
     assert bool(((got - want).abs() <= 3 * 96 * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("T", [13, 2117])
+@pytest.mark.parametrize("E,W", [(4, 32), (28, 544), (32, 2048)])
+def test_router_scores_beyond_bf16(T, E, W):
+    """Weights whose first bf16 number is infinite, and sums of which a part is: what
+    64 bits give, rounded once."""
+    h, w = rand(T, W).to(torch.bfloat16), rand(E, W, seed=1)
+    h[:, 0], h[:, 1], h[:, W - 1] = 2.0, -1.5, -0.25
+    w[:, 0], w[:, 1], w[1, W - 1] = 3.4e38, 3.4e38, float("inf")
+    h[T // 2, 2:] = float("nan")
+    got = hops._mix().router_scores(h.cuda(), w.cuda()).double().cpu()
+    assert torch.isnan(got[T // 2]).all()
+    sure = torch.arange(T) != T // 2
+    assert (got[sure, 1] == -float("inf")).all()
+    cols = torch.arange(E) != 1
+    got, want = (x[sure][:, cols] for x in (got, h.double() @ w.double().T))
+    assert bool(((got - want).abs() <= 2.0 ** -24 * want.abs()).all())
