@@ -625,29 +625,41 @@ def linear_silu_rows(x, w):
     return _require_hip().linear_silu_mul(x, w) if _many_rows(x, w) else None
 
 
-def _last_round(x, w) -> float:
-    """Of all places in the rounds of 256 tiles of 256 x 256, those that are taken."""
-    tiles = -(-x.shape[0] // 256) * (w.shape[0] // 256)
-    return tiles / (-(-tiles // 256) * 256)
+def _heads_pay(M: int, K: int, rows: int) -> bool:
+    """Whether the QKV projection of M rows pays in one launch, of the sizes that
+    `_many_rows` takes. Up to a k of 2048 by the share that x's rows are of all rows in
+    its rounds of 256 tiles of 256 x 256; lowest quotient of the library's time with
+    the pass by the launch's from a share on, 700 sizes:
+      share         0.58   0.62   0.66   0.70   0.72   0.74   0.76   0.80
+      k up to 512   1.28   1.19   1.19   1.24   1.26   1.26   1.22
+      640 .. 1024   0.89   0.93   0.92   0.96   1.03   0.99   1.10
+      .. 2048                            0.97   0.95   0.96   1.00   1.01
+    Above, where the library's product is 4 to 7 % faster than this one and the pass small
+    beside it, where 0.95 of the places have a tile: 0.99 up to a k of 6144, 0.96 at
+    8192 (200 sizes)."""
+    tiles = -(-M // 256) * (rows // 256)
+    places = -(-tiles // 256) * 256
+    if K > 2048:
+        return K <= 6144 and tiles >= 0.95 * places
+    return K <= 512 or M * (rows // 256) >= 256 * places * (0.72 if K <= 1024 else 0.76)
 
 
 def linear_qkv_prep(x, w, num_heads: int, num_kv_heads: int, head_dim: int,
                     positions, slot_mapping, k_cache, v_cache, cos_sin,
                     q_norm_w=None, k_norm_w=None, eps: float = 1e-6):
     """fused_qkv_prep of x w^T where one launch makes it (prompts), else None. us of the
-    library's product with the pass over its result, and of this one, by rows:
+    library's product with the pass over its result, and of this one, by rows (* not
+    taken: fewer than 256 tiles, or by `_heads_pay`):
        4096 x  512    4096   35.5 /  27.9     6000   62.5 /  46.1    24000  203 / 136
-       4096 x 1024    3000   36.3 /  34.3     4096   44.6 /  38.0    24000  267 / 198
-       3072 x 2048    6000   99.1 / 101.3     8192  108.7 / 106.6    32768  383 / 340
-       6144 x 4096    6000    257 /  281      8192    310 /  304     32768 1245 / 1222
-      10240 x 5120    3000    241 /  246      6000    517 /  481     16384 1290 / 1244
-    From a k of 2048 on the library's product is 4 to 7 % faster than the one here and
-    the pass small beside it: then where the last round is nearly full."""
+       4096 x 1024   *3000   36.3 /  34.3     4096   44.6 /  38.0    24000  267 / 198
+       3072 x 2048   *6000   99.1 / 101.3    *8192  108.7 / 106.6    32768  383 / 340
+       6144 x 4096   *6000    257 /  281      8192    310 /  304     32768 1245 / 1222
+      10240 x 5120   *3000    241 /  246     *6000    517 /  481     16384 1290 / 1244
+    e4m3 pages keep the pass: nothing here rounds to them."""
     caches = (k_cache, v_cache)
     norms = tuple(n for n in (q_norm_w, k_norm_w) if n is not None)
     if not (head_dim == 128 and num_heads % 2 == 0 and _many_rows(x, w)
-            and x.shape[1] >= 192
-            and (x.shape[1] <= 2048 or _last_round(x, w) >= 0.95)
+            and x.shape[1] >= 192 and _heads_pay(*x.shape, w.shape[0])
             and all(t.dtype == torch.bfloat16 and t.is_contiguous()
                     and t.data_ptr() % 16 == 0 for t in caches)
             and w.shape[0] == (num_heads + 2 * num_kv_heads) * 128

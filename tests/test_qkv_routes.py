@@ -74,6 +74,25 @@ def test_sizes_that_differ(kernels, name, make):
     assert _calls(kernels, **other) == 0
 
 
+@pytest.mark.parametrize("rows,k,wide,one", [
+    # few places taken: a short k gains all the same
+    (5045, 512, 4096, 1), (5045, 576, 4096, 0), (5045, 1024, 4096, 0),
+    (3336, 1024, 6144, 0), (7138, 1024, 3072, 0), (6438, 768, 3072, 0),
+    (6000, 1024, 4096, 1), (4096, 1024, 4096, 1), (24000, 1024, 4096, 1),
+    (9130, 2048, 4096, 0), (6048, 2048, 6144, 0), (9400, 2048, 4096, 1),
+    (32768, 2048, 3072, 1), (8192, 4096, 6144, 1), (7600, 4096, 6144, 0),
+    (16384, 8192, 4096, 0)])
+def test_sizes(kernels, rows, k, wide, one):
+    bf = dict(dtype=torch.bfloat16, device="meta")
+    heads = wide // 128 // 4
+    i64 = torch.zeros(rows, dtype=torch.int64, device="meta")
+    norm, pages = torch.empty(128, **bf), torch.empty(4, heads, 32, 128, **bf)
+    assert _calls(kernels, x=torch.empty(rows, k, **bf), w=torch.empty(wide, k, **bf),
+                  num_heads=2 * heads, num_kv_heads=heads, positions=i64,
+                  slot_mapping=i64, k_cache=pages, v_cache=pages, q_norm_w=norm,
+                  k_norm_w=norm, cos_sin=torch.empty(9, 128, device="meta")) == one
+
+
 @pytest.mark.parametrize("rows,asked", [(1, 0), (21, 0), (256, 0), (257, 1)])
 def test_few_rows_are_not_asked(monkeypatch, rows, asked):
     """Eager steps of few rows are bound by what is asked on the host."""
