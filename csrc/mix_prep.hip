@@ -414,7 +414,10 @@ extern "C" void mix_tied_attn_prep(void* q_out, const void* proj, long ld,
   if (T == 0) return;
   const dim3 grid((unsigned)T, 2);
   const int V = f32 ? 4 : 8, n = (H > G ? H : G) * dk;
-  if (dk % V == 0 && q_off % V == 0 && k_off % V == 0 && ld % V == 0 &&
+  // Short sections leave most threads of the vector form without one: 30,000 tokens, one
+  // head of 32 each 39 by the general kernel and 48 us by this one, 8 and 2 of 32 46 and
+  // 51, 2 and 1 of 128 51 and 52, 4 and 4 of 64 58 and 54.
+  if ((H + G) * dk >= 448 && dk % V == 0 && q_off % V == 0 && k_off % V == 0 && ld % V == 0 &&
       n <= 256 * V * 2 &&
       (((size_t)q_out | (size_t)proj | (size_t)q_w | (size_t)k_w |
         (size_t)k_cache | (size_t)v_cache) & 15) == 0) {

@@ -82,7 +82,8 @@ def test_token_embed_norm_of_another_type(dtype, other):
 
 @pytest.mark.parametrize("dtype", TYPES)
 @pytest.mark.parametrize("H,G,dk", [(16, 4, 128), (3, 1, 8), (1, 2, 12), (17, 1, 128),
-                                    (32, 2, 128), (33, 3, 128), (8, 8, 256), (2, 2, 7)])
+                                    (32, 2, 128), (33, 3, 128), (8, 8, 256), (2, 2, 7),
+                                    (4, 3, 64), (13, 1, 32), (55, 1, 8)])
 def test_tied_attn_prep(dtype, H, G, dk):
     T, page, temp = 5, 4, 3
     q0, k0 = 8, 8 + H * dk
