@@ -31,7 +31,7 @@ def close(got, want, n, extra=0.0):
 
 
 @pytest.mark.parametrize("dtype", TYPES)
-@pytest.mark.parametrize("W", [4, 15, 1020, 1024, 1028, 2048, 4100, 8192, 8196])
+@pytest.mark.parametrize("W", [4, 15, 124, 128, 1020, 1024, 1028, 2048, 4100, 8192, 8196])
 @pytest.mark.parametrize("bigram,sine", [(True, True), (False, True), (False, False)])
 def test_token_embed_norm(dtype, W, bigram, sine):
     T, V, buckets = 9, 33, 7
