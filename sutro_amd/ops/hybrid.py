@@ -371,14 +371,14 @@ def _router_kernel(h, w) -> bool:
       4096,   256       25/10    25/13     26/13     25/13     25/14
       4096, 30001      249/41   246/90    260/184   403/439   565/692"""
     if (type(h) is not torch.Tensor or _tracing()
-            or type(w) not in (torch.Tensor, torch.nn.Parameter)):
+            or type(w) not in (torch.Tensor, torch.nn.Parameter)
+            or w.shape[0] > (256 if h.shape[0] <= 256 else 64)):
         return False
     return (h.is_cuda and h.dim() == 2 and w.dim() == 2 and _unwatched()
             and h.dtype == torch.bfloat16 and w.dtype == torch.float32
             and w.device == h.device and w.shape[1] == h.shape[1]
             and 0 < h.shape[1] < 1 << 30 and h.shape[1] % 32 == 0
-            and 0 < h.shape[0] < 1 << 30
-            and 0 < w.shape[0] <= (256 if h.shape[0] <= 256 else 64)
+            and 0 < h.shape[0] < 1 << 30 and w.shape[0] > 0
             and h.is_contiguous() and w.is_contiguous()
             and h.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled()
