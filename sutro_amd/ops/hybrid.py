@@ -369,7 +369,10 @@ def _router_kernel(h, w) -> bool:
       2048,  1024       25/7.1   25/7.6    25/8.1    26/19     25/24
       2048, 30001      125/22   105/47    127/94    208/210   288/327
       4096,   256       25/10    25/13     26/13     25/13     25/14
-      4096, 30001      249/41   246/90    260/184   403/439   565/692"""
+      4096, 30001      249/41   246/90    260/184   403/439   565/692
+    and long rows of which there are too few workgroups to hide its loads (by 48 experts):
+      7168,   768      30/20    1536  36/39    2049  36/38    3000  52/39
+      8192,   768      30/23    1536  38/44    2049  39/44    3000  58/45"""
     if (type(h) is not torch.Tensor or _tracing()
             or type(w) not in (torch.Tensor, torch.nn.Parameter)
             or w.shape[0] > (256 if h.shape[0] <= 256 else 64)):
@@ -379,6 +382,7 @@ def _router_kernel(h, w) -> bool:
             and w.device == h.device and w.shape[1] == h.shape[1]
             and 0 < h.shape[1] < 1 << 30 and h.shape[1] % 32 == 0
             and 0 < h.shape[0] < 1 << 30 and w.shape[0] > 0
+            and (h.shape[1] <= 5120 or not 1024 < h.shape[0] < 3000)
             and h.is_contiguous() and w.is_contiguous()
             and h.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled()

@@ -191,3 +191,12 @@ def test_router_scores_beyond_bf16(T, E, W):
     cols = torch.arange(E) != 1
     got, want = (x[sure][:, cols] for x in (got, h.double() @ w.double().T))
     assert bool(((got - want).abs() <= 2.0 ** -24 * want.abs()).all())
+
+
+@pytest.mark.parametrize("T,E,W,kernel", [
+    (13, 256, 2048, 1), (256, 256, 2048, 1), (257, 65, 2048, 0), (257, 64, 2048, 1),
+    (30001, 64, 2048, 1), (13, 257, 2048, 0), (1024, 48, 8192, 1), (1025, 48, 8192, 0),
+    (1536, 48, 5120, 1), (2999, 16, 6144, 0), (3000, 16, 6144, 1), (13, 32, 2040, 0)])
+def test_router_rule(T, E, W, kernel):
+    h = torch.empty(T, W, dtype=torch.bfloat16, device="cuda")      # (never read)
+    assert hops._router_kernel(h, torch.empty(E, W, device="cuda")) == bool(kernel)
