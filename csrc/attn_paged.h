@@ -141,14 +141,18 @@ __device__ __forceinline__ u16x8 pa_widen(typename PaRaw<KV8>::type raw) {
 }
 // Tiles in LDS are row-major; 16-byte chunks are XOR-swizzled by the row. Of a
 // prompt's tiles 256 bytes are read in a cycle: 16 rows of one chunk (keys) or 8 rows
-// of two neighbouring ones (values, read transposed), which cover all 64 banks.
-template <int D>
+// of two neighbouring ones (values, read transposed), which cover all 64 banks. That
+// takes twice the addresses, which tiles that come through registers (REGS) have no
+// registers for: with e4m3 pages and heads of 128 it was 2 % slower in the median of 55
+// sizes and up to 5 (34 prompts of 120 behind 1500 keys, 20 and 4 heads, 101 -> 106 us), as
+// was one new operand a product. They cover half of the banks.
+template <int D, bool REGS>
 __device__ __forceinline__ int pa_kswz(int row, int c) {
-  return c ^ (D == 128 ? row & 15 : row >> 1 & 7);
+  return c ^ (REGS ? row & 7 : D == 128 ? row & 15 : row >> 1 & 7);
 }
-template <int D>
+template <int D, bool REGS>
 __device__ __forceinline__ int pa_vswz(int row, int c) {
-  return c ^ (D == 128 ? row & 7 : row >> 1 & 3) << 1;
+  return c ^ (REGS ? row & 3 : D == 128 ? row & 7 : row >> 1 & 3) << 1;
 }
 // single tokens: 4 rows of two chunks
 __device__ __forceinline__ int pa_vchunk(int row, int c) {
@@ -316,8 +320,8 @@ paged_prefill_kernel(PagedArgs A) {
   constexpr int RPP = 64 / CPR;             // rows per piece
   const int st_row = lane / CPR;
   const int t_row = w * RPP + st_row;       // of the tile, modulo 4 * RPP
-  const u32 koff = (st_row * D + pa_kswz<D>(t_row, lane % CPR) * 8) * ES;
-  const u32 voff = (st_row * D + pa_vswz<D>(t_row, lane % CPR) * 8) * ES;
+  const u32 koff = (st_row * D + pa_kswz<D, REGS>(t_row, lane % CPR) * 8) * ES;
+  const u32 voff = (st_row * D + pa_vswz<D, REGS>(t_row, lane % CPR) * 8) * ES;
   // LATE: four workgroups a CU, no registers to hold them while a step is computed
   constexpr bool LATE = REGS && WAVES_PER_SIMD == 4;
   typedef typename PaRaw<KV8>::type raw_t;
@@ -396,16 +400,17 @@ paged_prefill_kernel(PagedArgs A) {
 
   // fragment addresses: keys row ln (+16 a tile), chunk kk*4 + g; values rows
   // 4*g + ti/4 (+16), columns of 16-block b
-  int kad[D / 32];
+  constexpr int KA = REGS ? 2 : D / 32, VA = REGS ? 4 : D / 16;
+  int kad[KA];
 #pragma unroll
-  for (int kk = 0; kk < D / 32; ++kk)
-    kad[kk] = ln * (2 * D) + pa_kswz<D>(ln, kk * 4 + g) * 16;
+  for (int kk = 0; kk < KA; ++kk)
+    kad[kk] = ln * (2 * D) + pa_kswz<D, REGS>(ln, kk * 4 + g) * 16;
   const int ti = lane & 15;
-  int vad[D / 16];
+  int vad[VA];
 #pragma unroll
-  for (int b = 0; b < D / 16; ++b)
+  for (int b = 0; b < VA; ++b)
     vad[b] = (4 * g + (ti >> 2)) * (2 * D) +
-             pa_vswz<D>(4 * g + (ti >> 2), b * 2 + ((ti & 3) >> 1)) * 16 +
+             pa_vswz<D, REGS>(4 * g + (ti >> 2), b * 2 + ((ti & 3) >> 1)) * 16 +
              (ti & 1) * 8;
 
   pages(step_tile(0));
@@ -450,8 +455,9 @@ paged_prefill_kernel(PagedArgs A) {
     for (int kk = 0; kk < D / 32; ++kk)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const pa_frag ka = *(const s16x8*)(kb + kad[kk] + t * 16 * 2 * D);
-        const int f = t & 1;        // (one new operand a product)
+        const pa_frag ka = *(const s16x8*)(kb + kad[kk % KA] + kk / KA * 128 +
+                                           t * 16 * 2 * D);
+        const int f = REGS ? 0 : t & 1;     // (one new operand a product)
         d[f][t] = pa_mfma16(ka, qb[f][kk], d[f][t]);
         d[1 - f][t] = pa_mfma16(ka, qb[1 - f][kk], d[1 - f][t]);
       }
@@ -542,8 +548,9 @@ paged_prefill_kernel(PagedArgs A) {
       }
 #pragma unroll
       for (int b = 0; b < D / 16; ++b) {
-        const pa_frag va = pa_tr(v0 + vad[b], v1 + vad[b]);
-        const int f = b & 1;
+        const int at = vad[b % VA] + b / VA * 128;
+        const pa_frag va = pa_tr(v0 + at, v1 + at);
+        const int f = REGS ? 0 : b & 1;
         acc[b][f] = pa_mfma16(va, pb[f], acc[b][f]);
         acc[b][1 - f] = pa_mfma16(va, pb[1 - f], acc[b][1 - f]);
       }
