@@ -565,7 +565,7 @@ __global__ void __launch_bounds__(SMP_THREADS) sampler_kernel(SmpArgs A) {
 // 1024 x 151,936 by the general kernel and here: 1382 -> 197 us (top_p 0.95 at
 // temperature 0.8), 1393 -> 151 with top_k 20, 1338 -> 250
 // with a mask; one row 636 -> 41 us. Of the 50 us that a row takes its
-// workgroup 16 are fixed, clearing and scanning 128 KB of counters. Greedy rows, those
+// workgroup 16 are fixed, clearing and scanning 128 KB of counters. Greedy batches, rows
 // of more than 155,648 logits and what sampler_fast_kernel leaves come here.
 #define CNT_MIN 2048
 #define CNT_THREADS 1024
@@ -1130,8 +1130,7 @@ sampler_count_kernel(SmpArgs A) {
 // counted at the ends. That is exact where the largest logit is above 1 (a magnitude of
 // 2^-24 or less then vanishes in the difference to it) or no magnitude is as small, and
 // where none is above 254, or those are negative and 0 as weights; other rows, with NaN
-// or +inf among them, and greedy ones are left to the kernel above, which runs behind
-// this one.
+// or +inf among them, are left to the kernel above, which runs behind this one.
 //
 // One workgroup a CU stays for all of its rows: where a piece of the row has been counted,
 // the same piece of the next row is asked for, so that the copies run on beside the
@@ -1609,6 +1608,110 @@ __device__ __forceinline__ bool fast_row(const SmpArgs& A, int row, int ahead,
   return true;
 }
 
+// A greedy row among others: the same sums as the kernel above makes of it, in the same
+// order, but the row is read twice, eight pieces a wave and turn, for want of registers.
+// Left to the kernel above, which runs behind, one greedy row in three made a batch wait
+// for it: 3 / 116 / 378 rows of 151,936 43 / 45 / 93 us, now 30 / 30 / 76 (by the kernel
+// above alone 32 / 35 / 90). False: nothing was done (the NaN that stands for logits that are not alive is one).
+template <bool MASKED>
+__device__ __forceinline__ bool fast_greedy(const SmpArgs& A, int row, char* lds) {
+  u32* red = (u32*)lds;
+  int tid = threadIdx.x, vl = A.vl;
+  asm volatile("" : "+v"(tid), "+s"(vl));
+  const int lane = tid & 63, l16 = lane & (CNT_WAVES - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const u16* lrow = (const u16*)A.logits + (long)row * A.v_row;
+  const u8* mrow = MASKED ? (const u8*)(A.mask + (long)row * A.w_words)
+                          : nullptr;
+  const int last8 = (vl - 1) & ~7;
+  const int part = (vl + CNT_CHUNK - 1) / CNT_CHUNK, t0 = wave * part * 512 + lane * 8;
+  // f(logits, how many of them are not alive, index); those are 0xffff
+  auto pieces = [&](auto f) {
+#pragma unroll 1
+    for (int c = 0; c < part; c += FAST_RING) {
+      u32x4 w[FAST_RING];
+      u32 bits[FAST_RING];
+#pragma unroll
+      for (int k = 0; k < FAST_RING; ++k) {
+        const int i = min(t0 + (c + k) * 512, last8);
+        w[k] = *(const u32x4*)(lrow + i);
+        bits[k] = MASKED ? mrow[i >> 3] : 0xffu;
+      }
+#pragma unroll
+      for (int k = 0; k < FAST_RING; ++k) {
+        const int i = t0 + (c + k) * 512, left = c + k < part ? vl - i : 0;
+        if (left < 8) bits[k] &= left > 0 ? (1u << left) - 1 : 0u;
+        if (MASKED || left < 8)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            w[k][j] |= ((~bits[k] >> (2 * j)) & 1u) * 0xffffu |
+                       ((~bits[k] >> (2 * j + 1)) & 1u) * 0xffff0000u;
+        f(w[k], 8 - __popc(bits[k]), i);
+      }
+    }
+  };
+  float best = -INFINITY;
+  int ones = 0;
+  pieces([&](const u32x4& w, int dead, int) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ones += ((w[j] & 0xffffu) == 0xffffu) + (w[j] >= 0xffff0000u);
+      best = fmaxf(best, fmaxf(__uint_as_float(w[j] << 16),
+                               __uint_as_float(w[j] & 0xffff0000u)));
+    }
+    ones -= dead;
+  });
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    best = fmaxf(best, __shfl_xor(best, off, 64));
+  const bool odd = __any(ones != 0);
+  if (lane == 0) {
+    red[wave] = __float_as_uint(best);
+    red[CNT_WAVES + wave] = odd;
+  }
+  __syncthreads();
+  best = __uint_as_float(red[l16]);
+  u32 any = red[CNT_WAVES + l16];
+#pragma unroll
+  for (int off = 1; off < CNT_WAVES; off <<= 1) {
+    best = fmaxf(best, __shfl_xor(best, off, CNT_WAVES));
+    any |= __shfl_xor(any, off, CNT_WAVES);
+  }
+  if (any) return false;
+  float z = 0.f;
+  int first = 0x7fffffff;
+  pieces([&](const u32x4& w, int, int i) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const u32 h = j & 1 ? w[j >> 1] & 0xffff0000u : w[j >> 1] << 16;
+      const float v = __uint_as_float(h);
+      z += h == 0xffff0000u ? 0.f : __expf(v - best);
+      if (v == best) first = min(first, i + j);
+    }
+  });
+  z = wave_sum(z);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    first = min(first, __shfl_xor(first, off, 64));
+  red += 2 * CNT_WAVES;
+  if (lane == 0) {
+    red[wave] = (u32)first;
+    red[CNT_WAVES + wave] = __float_as_uint(z);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    z = 0.f;
+    for (int w = 0; w < CNT_WAVES; ++w) {
+      first = min(first, (int)red[w]);
+      z += __uint_as_float(red[CNT_WAVES + w]);
+    }
+    const bool none = best == -INFINITY;
+    A.out_tok[row] = none ? 0 : first;
+    A.out_lp[row] = none ? -INFINITY : -logf(z);
+  }
+  return true;
+}
+
 template <bool MASKED>
 __global__ void __launch_bounds__(CNT_THREADS)
 sampler_fast_kernel(SmpArgs A) {
@@ -1630,10 +1733,12 @@ sampler_fast_kernel(SmpArgs A) {
       }
       have = next < A.n;
       done = fast_row<MASKED>(A, row, have ? next : -1, fast_lds, r);
-      __syncthreads();
     } else {
       have = false;
+      done = fast_greedy<MASKED>(A, row, fast_lds);
+      r = {};                // (not kept meanwhile)
     }
+    __syncthreads();
     if (!done && threadIdx.x == 0) A.out_tok[row] = SMP_LEFT;
   }
 }

@@ -286,3 +286,46 @@ def test_masked_ends_of_the_short_range(temp, top_p, top_k):
     keep[24, 4000] = True
     same_as_general(rows.to(torch.bfloat16).to(DEV), temp, top_p, top_k,
                     (0.0, 0.3, 0.999), keep)
+
+
+@pytest.mark.parametrize("row,vl", [(2048, 2048), (8200, 8193), (70008, 70005),
+                                    (155648, 155648)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_greedy_rows_among_others(row, vl, masked):
+    """More rows than workgroups, every third of them greedy: to the bit what two calls
+    make of them, ties, numbers that are none and rows without a live logit among them."""
+    n = 300
+    g = torch.Generator().manual_seed(vl)
+    lg = (torch.randn(n, row, generator=g) * 3).to(torch.bfloat16)
+    inf, nan = float("inf"), float("nan")
+    lg[0, 40], lg[0, vl - 1] = 30.0, 30.0
+    lg[3, vl - 1], lg[6, :], lg[9, 5], lg[12, 7] = 30.0, -inf, inf, nan
+    lg[15, ::2], lg[18, 3] = nan, -inf
+    lg[0:n:3, vl:] = 100.0
+    bits = lg.view(torch.int16)
+    bits[21, 5] = -1                              # the NaN of all bits
+    keep = torch.rand(n, row, generator=g) < 0.3
+    keep[[0, 3], vl - 1], keep[24, :], keep[27, :] = True, False, False
+    keep[27, vl - 1] = True
+    lg, mask = lg.to(DEV), pack(keep) if masked else None
+    temps = torch.full((n,), 0.8, device=DEV)
+    temps[::3] = 0.0
+    rest = (torch.full((n,), 0.9, device=DEV),
+            torch.full((n,), vl, dtype=torch.int32, device=DEV),
+            torch.rand(n, generator=g).to(DEV))
+
+    def sample(rows, **kw):
+        k = len(range(n)[rows])
+        tok, lp = torch.empty(k, dtype=torch.int32, device=DEV), torch.empty(k, device=DEV)
+        ops.sampler_fused(lg[rows].contiguous(), temps[rows].contiguous(),
+                          *(t[rows].contiguous() for t in rest),
+                          None if mask is None else mask[rows].contiguous(), vl, tok, lp,
+                          **kw)
+        return tok, lp.view(torch.int32)
+
+    tok, lp = sample(slice(None))
+    for rows, kw in ((slice(0, n, 3), dict(greedy=True)), (slice(1, n, 3), {}),
+                     (slice(2, n, 3), {})):
+        one = sample(rows, **kw)
+        assert torch.equal(tok[rows], one[0])
+        assert torch.equal(lp[rows], one[1])
