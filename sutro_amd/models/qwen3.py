@@ -100,8 +100,11 @@ class Qwen3Attention(nn.Module):
                  self.k_norm.weight if self.qk_norm else None,
                  self.q_norm.eps if self.qk_norm else 1e-6)
         q = None
-        # (a look at the rows first: eager steps of few are bound by what is asked here)
-        if qkv is None and x.shape[0] > 256 and bare(self.qkv_proj):
+        # (that launch wants 256 tiles of 256 x 256: looked at first, as steps of fewer
+        # rows are bound by what is asked here)
+        if (qkv is None
+                and (x.shape[0] + 255) * (self.q_size + 2 * self.kv_size) >= 1 << 24
+                and bare(self.qkv_proj)):
             q = ops.linear_qkv_prep(x, self.qkv_proj.weight, *heads)
         if q is None:
             if qkv is None:

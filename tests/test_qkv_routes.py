@@ -93,20 +93,20 @@ def test_sizes(kernels, rows, k, wide, one):
                   k_norm_w=norm, cos_sin=torch.empty(9, 128, device="meta")) == one
 
 
-@pytest.mark.parametrize("rows,asked", [(1, 0), (21, 0), (256, 0), (257, 1)])
+@pytest.mark.parametrize("rows,asked", [(1, 0), (21, 0), (1000, 0), (3840, 0), (3841, 1)])
 def test_few_rows_are_not_asked(monkeypatch, rows, asked):
     """Eager steps of few rows are bound by what is asked on the host."""
-    spec = SimpleNamespace(num_heads=2, num_kv_heads=1, head_dim=8, hidden_size=16,
+    spec = SimpleNamespace(num_heads=30, num_kv_heads=1, head_dim=128, hidden_size=4,
                            qk_norm=True, rms_eps=1e-6)
     attn = Qwen3Attention(spec, torch.float32, 0)
     calls = []
     monkeypatch.setattr(ops, "linear_qkv_prep", lambda *a: calls.append(1))
     monkeypatch.setattr(ops, "fused_qkv_prep",
-                        lambda qkv, *a: qkv[:, :16].reshape(-1, 2, 8))
+                        lambda qkv, *a: qkv[:, :3840].reshape(-1, 30, 128))
     monkeypatch.setattr(ops, "paged_attention", lambda q, *a: q)
     fb = SimpleNamespace(**dict.fromkeys((
         "positions", "slot_mapping", "block_tables", "seq_lens", "query_start_locs",
         "num_decodes_tail", "tile_seq", "tile_q0", "prefill_token_count")))
     kv = SimpleNamespace(k_cache=[None], v_cache=[None])
-    assert attn(torch.zeros(rows, 16), fb, kv, None).shape == (rows, 16)
+    assert attn(torch.zeros(rows, 4), fb, kv, None).shape == (rows, 4)
     assert len(calls) == asked
